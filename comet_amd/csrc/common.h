@@ -44,6 +44,19 @@ void forget_pending_product();     // ciface.hip: SpGEMM "sizes" call -> "fill" 
             return rc_;                \
     } while (0)
 
+// Device memory of the library and of its callers (comet_hip_malloc).  hipMalloc and hipFree cost tens of
+// microseconds for a small array, tens of milliseconds for one of gigabytes, and hipFree drains the device, so freed
+// blocks are kept for the next request of about their size: at most POOL_SHARE of the device's memory, oldest given
+// back first, all of it when an allocation fails or the library is finalized.  A freed block may still be in use by
+// work launched on any stream, so it is handed out again only after the device has been drained since
+// (stream_wait and dev_malloc see to that).  Safe to call from several threads.
+constexpr size_t POOL_SHARE = 16;          // a sixteenth of the device
+hipError_t dev_malloc(void **p, size_t bytes);
+hipError_t dev_free(void *p);
+void dev_pool_release();
+// waits for stream(); the place where blocks freed before it become free to hand out again
+int stream_wait();
+
 // Grow-only device scratch buffer.  `zeroed` buffers are cleared when they are
 // (re)allocated and their users must leave them all-zero on return.
 struct Workspace {

@@ -249,7 +249,7 @@ int csr_entry_rows(Csr *a, const int32_t **rows)
     if (!a->entry_row && a->nnz > 0) {
         if (a->nrows >= (1ll << 31))
             return set_error(COMET_HIP_ERR_SIZE, "row ids of %lld rows do not fit 32 bits", (long long)a->nrows);
-        COMET_HIPCHK(hipMalloc((void **)&a->entry_row, sizeof(int32_t) * (size_t)a->nnz));
+        COMET_HIPCHK(dev_malloc((void **)&a->entry_row, sizeof(int32_t) * (size_t)a->nnz));
         KernelTimer t("csr_expand_rows");
         csr_expand_rows<<<dim3((unsigned)ceil_div(a->nnz, 256)), dim3(256), 0, stream()>>>(a->nrows, a->nnz, a->pos,
                                                                                            a->entry_row);
@@ -288,10 +288,10 @@ __global__ void dcsr_compact_rows(int64_t nrows, const int64_t *__restrict__ pos
 
 struct DevBuf {
     void *p = nullptr;
-    ~DevBuf() { if (p) (void)hipFree(p); }
+    ~DevBuf() { if (p) (void)dev_free(p); }
     int alloc(size_t bytes)
     {
-        COMET_HIPCHK(hipMalloc(&p, bytes ? bytes : 1));
+        COMET_HIPCHK(dev_malloc(&p, bytes ? bytes : 1));
         return COMET_HIP_OK;
     }
     template <typename T> T *as() { return (T *)p; }
@@ -349,13 +349,13 @@ static Csr *coo_device_to_csr_struct(int64_t nrows, int64_t ncols, int64_t n, co
     c->ncols = ncols;
     c->owns = true;
     auto fail = [&]() -> Csr * {
-        (void)hipFree(c->pos);
-        (void)hipFree(c->crd);
-        (void)hipFree(c->val);
+        (void)dev_free(c->pos);
+        (void)dev_free(c->crd);
+        (void)dev_free(c->val);
         delete c;
         return nullptr;
     };
-    if (hipMalloc((void **)&c->pos, sizeof(int64_t) * (size_t)(nrows + 1)) != hipSuccess) {
+    if (dev_malloc((void **)&c->pos, sizeof(int64_t) * (size_t)(nrows + 1)) != hipSuccess) {
         set_error(COMET_HIP_ERR_HIP, "row pointer allocation failed");
         return fail();
     }
@@ -408,8 +408,8 @@ static Csr *coo_device_to_csr_struct(int64_t nrows, int64_t ncols, int64_t n, co
         }
     }
     c->nnz = kept;
-    if (hipMalloc((void **)&c->crd, sizeof(int32_t) * (size_t)(kept > 0 ? kept : 1)) != hipSuccess ||
-        hipMalloc((void **)&c->val, sizeof(double) * (size_t)(kept > 0 ? kept : 1)) != hipSuccess ||
+    if (dev_malloc((void **)&c->crd, sizeof(int32_t) * (size_t)(kept > 0 ? kept : 1)) != hipSuccess ||
+        dev_malloc((void **)&c->val, sizeof(double) * (size_t)(kept > 0 ? kept : 1)) != hipSuccess ||
         crow.alloc(4 * (size_t)(kept > 0 ? kept : 1))) {
         set_error(COMET_HIP_ERR_HIP, "allocation of %lld entries failed", (long long)kept);
         return fail();

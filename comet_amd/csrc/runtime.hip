@@ -7,9 +7,12 @@
 #include <stdlib.h>
 #include <string.h>
 
-#include <map>
+#include <algorithm>
 #include <atomic>
+#include <list>
+#include <map>
 #include <mutex>
+#include <unordered_map>
 #include <unordered_set>
 
 #include "common.h"
@@ -96,6 +99,146 @@ int ensure_init()
     return do_init(0);
 }
 
+// ------------------------------------------------------------------ device memory
+struct PoolBlock {
+    size_t bytes;
+    bool live;
+    std::list<void *>::iterator age;         // of a free block: its place in g_pool_age
+};
+constexpr size_t POOL_BLOCKS = 512;                                  // free blocks kept at most: the lists stay short
+static std::mutex g_pool_mu;
+static std::unordered_map<void *, PoolBlock> g_pool_blocks;          // every block that came from hipMalloc here
+static std::multimap<size_t, void *> g_pool_clean;                   // free, and the device was drained since
+static std::vector<std::pair<size_t, void *>> g_pool_pending;        // free, possibly still in use by launched work
+static std::list<void *> g_pool_age;                                 // the free blocks, longest free first
+static size_t g_pool_free_bytes = 0, g_pool_cap = 0;
+
+// Sizes in eighths of a power of two: requests of about the same size find each other's blocks.
+static size_t pool_size(size_t bytes)
+{
+    size_t step = 512;
+    while (step * 16 <= bytes)
+        step *= 2;
+    return bytes > 0 ? (bytes + step - 1) / step * step : step;
+}
+
+static void pool_promote()
+{
+    g_pool_clean.insert(g_pool_pending.begin(), g_pool_pending.end());
+    g_pool_pending.clear();
+}
+
+static void pool_leave(PoolBlock &b)         // a block leaves the free ones
+{
+    g_pool_age.erase(b.age);
+    g_pool_free_bytes -= b.bytes;
+}
+
+static void pool_trim(size_t keep_bytes, size_t keep_blocks)         // hipFree itself waits for the device
+{
+    while (!g_pool_age.empty() && (g_pool_free_bytes > keep_bytes || g_pool_age.size() > keep_blocks)) {
+        void *p = g_pool_age.front();
+        PoolBlock &b = g_pool_blocks[p];
+        const std::pair<size_t, void *> entry(b.bytes, p);
+        auto range = g_pool_clean.equal_range(b.bytes);
+        for (auto it = range.first; it != range.second; ++it)
+            if (it->second == p) {
+                g_pool_clean.erase(it);
+                break;
+            }
+        g_pool_pending.erase(std::remove(g_pool_pending.begin(), g_pool_pending.end(), entry), g_pool_pending.end());
+        pool_leave(b);
+        g_pool_blocks.erase(p);
+        (void)hipFree(p);
+    }
+}
+
+// a clean block of at least `bytes` that wastes at most a quarter of the request
+static void *pool_take(size_t bytes)
+{
+    auto it = g_pool_clean.lower_bound(bytes);
+    if (it == g_pool_clean.end() || it->first > bytes + bytes / 4)
+        return nullptr;
+    void *p = it->second;
+    g_pool_clean.erase(it);
+    PoolBlock &b = g_pool_blocks[p];
+    pool_leave(b);
+    b.live = true;
+    return p;
+}
+
+hipError_t dev_malloc(void **out, size_t need)
+{
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    const size_t bytes = pool_size(need);
+    void *p = pool_take(bytes);
+    if (!p) {
+        for (const auto &q : g_pool_pending) {
+            if (q.first < bytes || q.first > bytes + bytes / 4)
+                continue;
+            const hipError_t e = hipDeviceSynchronize();
+            if (e != hipSuccess)
+                return e;
+            pool_promote();
+            p = pool_take(bytes);
+            break;
+        }
+    }
+    if (!p) {
+        hipError_t e = hipMalloc(&p, bytes);
+        if (e != hipSuccess && g_pool_free_bytes > 0) {
+            (void)hipGetLastError();
+            pool_trim(0, 0);
+            e = hipMalloc(&p, bytes);
+        }
+        if (e != hipSuccess)
+            return e;
+        g_pool_blocks[p] = PoolBlock{bytes, true, g_pool_age.end()};
+    }
+    *out = p;
+    return hipSuccess;
+}
+
+hipError_t dev_free(void *p)
+{
+    if (!p)
+        return hipSuccess;
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    auto it = g_pool_blocks.find(p);
+    if (it == g_pool_blocks.end())           // not one of ours
+        return hipFree(p);
+    if (!it->second.live)
+        return hipErrorInvalidValue;         // freed twice
+    if (g_pool_cap == 0) {
+        size_t f = 0, t = 0;
+        g_pool_cap = hipMemGetInfo(&f, &t) == hipSuccess && t >= POOL_SHARE ? t / POOL_SHARE : 1;
+    }
+    it->second.live = false;
+    it->second.age = g_pool_age.insert(g_pool_age.end(), p);
+    g_pool_pending.emplace_back(it->second.bytes, p);
+    g_pool_free_bytes += it->second.bytes;
+    pool_trim(g_pool_cap, POOL_BLOCKS);
+    return hipSuccess;
+}
+
+void dev_pool_release()
+{
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    pool_trim(0, 0);
+}
+
+int stream_wait()
+{
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    if (g_pool_pending.empty()) {
+        COMET_HIPCHK(hipStreamSynchronize(stream()));
+        return COMET_HIP_OK;
+    }
+    COMET_HIPCHK(hipDeviceSynchronize());
+    pool_promote();
+    return COMET_HIP_OK;
+}
+
 // every workspace that ever held memory, so that comet_hip_finalize can give all of it back
 static std::vector<Workspace *> g_workspaces;
 
@@ -108,12 +251,11 @@ int Workspace::ensure(size_t need, bool zeroed)
         listed = true;
     }
     if (ptr) {
-        COMET_HIPCHK(hipStreamSynchronize(stream()));
-        COMET_HIPCHK(hipFree(ptr));
+        COMET_HIPCHK(dev_free(ptr));
         ptr = nullptr;
         bytes = 0;
     }
-    COMET_HIPCHK(hipMalloc(&ptr, need));
+    COMET_HIPCHK(dev_malloc(&ptr, need));
     bytes = need;
     if (zeroed)
         COMET_HIPCHK(hipMemsetAsync(ptr, 0, need, stream()));
@@ -123,7 +265,7 @@ int Workspace::ensure(size_t need, bool zeroed)
 void Workspace::release()
 {
     if (ptr)
-        (void)hipFree(ptr);
+        (void)dev_free(ptr);
     ptr = nullptr;
     bytes = 0;
 }
@@ -158,9 +300,9 @@ int csr_alloc(Csr *c, int64_t nrows, int64_t ncols, int64_t nnz)
     c->ncols = ncols;
     c->nnz = nnz;
     c->owns = true;
-    COMET_HIPCHK(hipMalloc((void **)&c->pos, sizeof(int64_t) * (size_t)(nrows + 1)));
-    COMET_HIPCHK(hipMalloc((void **)&c->crd, sizeof(int32_t) * (size_t)(nnz > 0 ? nnz : 1)));
-    COMET_HIPCHK(hipMalloc((void **)&c->val, sizeof(double) * (size_t)(nnz > 0 ? nnz : 1)));
+    COMET_HIPCHK(dev_malloc((void **)&c->pos, sizeof(int64_t) * (size_t)(nrows + 1)));
+    COMET_HIPCHK(dev_malloc((void **)&c->crd, sizeof(int32_t) * (size_t)(nnz > 0 ? nnz : 1)));
+    COMET_HIPCHK(dev_malloc((void **)&c->val, sizeof(double) * (size_t)(nnz > 0 ? nnz : 1)));
     return COMET_HIP_OK;
 }
 
@@ -180,8 +322,8 @@ static void csr_drop_plans(Csr *c)
 {
     c->uid = next_csr_uid();
     for (auto &e : c->row_lists) {
-        (void)hipFree(e.rows);
-        (void)hipFree(e.bounds);
+        (void)dev_free(e.rows);
+        (void)dev_free(e.bounds);
     }
     c->row_lists.clear();
     if (c->light)
@@ -193,17 +335,17 @@ static void csr_drop_plans(Csr *c)
     c->light = c->transposed = c->transposed_index = nullptr;
     c->dup_state = 0;
     c->iso_state = 0;
-    (void)hipFree(c->entry_row);
+    (void)dev_free(c->entry_row);
     c->entry_row = nullptr;
-    (void)hipFree(c->rowmap);
-    (void)hipFree(c->empty_rows);
+    (void)dev_free(c->rowmap);
+    (void)dev_free(c->empty_rows);
     c->rowmap = c->empty_rows = nullptr;
     c->nempty = 0;
-    (void)hipFree(c->heavy_seg);
-    (void)hipFree(c->heavy_ent);
-    (void)hipFree(c->heavy_row);
-    (void)hipFree(c->heavy_code);
-    (void)hipFree(c->medium_row);
+    (void)dev_free(c->heavy_seg);
+    (void)dev_free(c->heavy_ent);
+    (void)dev_free(c->heavy_row);
+    (void)dev_free(c->heavy_code);
+    (void)dev_free(c->medium_row);
     c->medium_row = nullptr;
     c->medium_rows = 0;
     c->heavy_seg = nullptr;
@@ -212,19 +354,19 @@ static void csr_drop_plans(Csr *c)
     c->heavy_state = 0;
     c->spmm_uses = c->spmv_uses = 0;
     c->heavy_nnz = c->heavy_rows = 0;
-    (void)hipFree(c->spmm_chunk_row);
+    (void)dev_free(c->spmm_chunk_row);
     c->spmm_chunk_row = nullptr;
     c->spmm_nchunks = 0;
-    (void)hipFree(c->sg_blkptr);
-    (void)hipFree(c->sg_crd16);
+    (void)dev_free(c->sg_blkptr);
+    (void)dev_free(c->sg_crd16);
     c->sg_blkptr = nullptr;
     c->sg_crd16 = nullptr;
     c->sg_nblk = 0;
-    (void)hipFree(c->spmv_bpos);
-    (void)hipFree(c->spmv_bpos32);
+    (void)dev_free(c->spmv_bpos);
+    (void)dev_free(c->spmv_bpos32);
     c->spmv_bpos32 = nullptr;
-    (void)hipFree(c->spmv_bcrd);
-    (void)hipFree(c->spmv_bval);
+    (void)dev_free(c->spmv_bcrd);
+    (void)dev_free(c->spmv_bval);
     c->spmv_bpos = nullptr;
     c->spmv_bcrd = nullptr;
     c->spmv_bval = nullptr;
@@ -236,9 +378,9 @@ void csr_release(Csr *c)
 {
     csr_drop_plans(c);
     if (c->owns) {
-        (void)hipFree(c->pos);
-        (void)hipFree(c->crd);
-        (void)hipFree(c->val);
+        (void)dev_free(c->pos);
+        (void)dev_free(c->crd);
+        (void)dev_free(c->val);
     }
     delete c;
 }
@@ -548,8 +690,7 @@ int reduce_sum_device(const double *v, int64_t n, double *out_host)
     }
     COMET_HIPCHK(hipGetLastError());
     COMET_HIPCHK(hipMemcpyAsync(out_host, partial + nb, sizeof(double), hipMemcpyDeviceToHost, stream()));
-    COMET_HIPCHK(hipStreamSynchronize(stream()));
-    return COMET_HIP_OK;
+    return stream_wait();
 }
 
 }  // namespace comet
@@ -662,6 +803,7 @@ int comet_hip_finalize(void)
     g_live.clear();
     for (Workspace *w : g_workspaces)
         w->release();
+    dev_pool_release();
     (void)hipStreamSynchronize(g_aux);
     (void)hipEventDestroy(g_fork);
     (void)hipEventDestroy(g_join);
@@ -695,7 +837,7 @@ int64_t comet_hip_malloc(int64_t bytes)
         return 0;
     }
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, (size_t)(bytes > 0 ? bytes : 1));
+    hipError_t e = dev_malloc(&p, (size_t)(bytes > 0 ? bytes : 1));
     if (e != hipSuccess) {
         set_error(COMET_HIP_ERR_HIP, "hipMalloc(%lld) failed: %s", (long long)bytes, hipGetErrorString(e));
         return 0;
@@ -708,8 +850,7 @@ int comet_hip_free(int64_t dptr)
     COMET_CHK(ensure_init());
     if (!dptr)
         return COMET_HIP_OK;
-    COMET_HIPCHK(hipStreamSynchronize(stream()));
-    COMET_HIPCHK(hipFree((void *)dptr));
+    COMET_HIPCHK(dev_free((void *)dptr));
     return COMET_HIP_OK;
 }
 
@@ -724,8 +865,7 @@ int comet_hip_memcpy(int64_t dptr, void *host, int64_t bytes, int64_t direction)
         COMET_HIPCHK(hipMemcpyAsync((void *)dptr, host, (size_t)bytes, hipMemcpyHostToDevice, stream()));
     else
         COMET_HIPCHK(hipMemcpyAsync(host, (void *)dptr, (size_t)bytes, hipMemcpyDeviceToHost, stream()));
-    COMET_HIPCHK(hipStreamSynchronize(stream()));
-    return COMET_HIP_OK;
+    return stream_wait();
 }
 
 int comet_hip_memset(int64_t dptr, int byte_value, int64_t bytes)
@@ -781,7 +921,7 @@ int64_t comet_hip_csr_upload_i64(int64_t nrows, int64_t ncols, const int64_t *po
     int64_t *tmp = nullptr;
     auto fail = [&]() -> int64_t {
         if (tmp)
-            (void)hipFree(tmp);
+            (void)dev_free(tmp);
         csr_release(c);
         return 0;
     };
@@ -791,7 +931,7 @@ int64_t comet_hip_csr_upload_i64(int64_t nrows, int64_t ncols, const int64_t *po
     if (hipMemcpyAsync(c->pos, pos, sizeof(int64_t) * (size_t)(nrows + 1), hipMemcpyHostToDevice, s) != hipSuccess)
         return set_error(COMET_HIP_ERR_HIP, "pos upload failed"), fail();
     if (nnz > 0) {
-        if (hipMalloc((void **)&tmp, sizeof(int64_t) * (size_t)nnz) != hipSuccess)
+        if (dev_malloc((void **)&tmp, sizeof(int64_t) * (size_t)nnz) != hipSuccess)
             return set_error(COMET_HIP_ERR_HIP, "staging allocation failed"), fail();
         if (hipMemcpyAsync(tmp, crd, sizeof(int64_t) * (size_t)nnz, hipMemcpyHostToDevice, s) != hipSuccess ||
             hipMemcpyAsync(c->val, val, sizeof(double) * (size_t)nnz, hipMemcpyHostToDevice, s) != hipSuccess)
@@ -802,7 +942,7 @@ int64_t comet_hip_csr_upload_i64(int64_t nrows, int64_t ncols, const int64_t *po
     if (hipStreamSynchronize(s) != hipSuccess)
         return set_error(COMET_HIP_ERR_HIP, "upload synchronisation failed"), fail();
     if (tmp)
-        (void)hipFree(tmp);
+        (void)dev_free(tmp);
     return csr_register(c);
 }
 
@@ -818,14 +958,14 @@ int64_t comet_hip_csr_upload_i32(int64_t nrows, int64_t ncols, const int32_t *po
     int32_t *tmp = nullptr;
     auto fail = [&]() -> int64_t {
         if (tmp)
-            (void)hipFree(tmp);
+            (void)dev_free(tmp);
         csr_release(c);
         return 0;
     };
     if (csr_alloc(c, nrows, ncols, nnz) != COMET_HIP_OK)
         return fail();
     hipStream_t s = stream();
-    if (hipMalloc((void **)&tmp, sizeof(int32_t) * (size_t)(nrows + 1)) != hipSuccess)
+    if (dev_malloc((void **)&tmp, sizeof(int32_t) * (size_t)(nrows + 1)) != hipSuccess)
         return set_error(COMET_HIP_ERR_HIP, "staging allocation failed"), fail();
     if (hipMemcpyAsync(tmp, pos, sizeof(int32_t) * (size_t)(nrows + 1), hipMemcpyHostToDevice, s) != hipSuccess)
         return set_error(COMET_HIP_ERR_HIP, "pos upload failed"), fail();
@@ -838,7 +978,7 @@ int64_t comet_hip_csr_upload_i32(int64_t nrows, int64_t ncols, const int32_t *po
     }
     if (hipStreamSynchronize(s) != hipSuccess)
         return set_error(COMET_HIP_ERR_HIP, "upload synchronisation failed"), fail();
-    (void)hipFree(tmp);
+    (void)dev_free(tmp);
     return csr_register(c);
 }
 
@@ -902,12 +1042,12 @@ int comet_hip_csr_download_i64(int64_t csr, int64_t *pos, int64_t *crd, double *
         COMET_HIPCHK(hipMemcpyAsync(val, c->val, sizeof(double) * (size_t)c->nnz, hipMemcpyDeviceToHost, s));
     if (crd && c->nnz) {
         int64_t *tmp = nullptr;
-        COMET_HIPCHK(hipMalloc((void **)&tmp, sizeof(int64_t) * (size_t)c->nnz));
+        COMET_HIPCHK(dev_malloc((void **)&tmp, sizeof(int64_t) * (size_t)c->nnz));
         unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(c->nnz, 256), 65536);
         widen_i32_to_i64<<<dim3(blocks), dim3(256), 0, s>>>(c->crd, tmp, c->nnz);
         hipError_t e = hipMemcpyAsync(crd, tmp, sizeof(int64_t) * (size_t)c->nnz, hipMemcpyDeviceToHost, s);
         hipError_t e2 = hipStreamSynchronize(s);
-        (void)hipFree(tmp);
+        (void)dev_free(tmp);
         COMET_HIPCHK(e);
         COMET_HIPCHK(e2);
     }
@@ -925,12 +1065,12 @@ int comet_hip_csr_download_i32(int64_t csr, int32_t *pos, int32_t *crd, double *
     hipStream_t s = stream();
     if (pos) {
         int32_t *tmp = nullptr;
-        COMET_HIPCHK(hipMalloc((void **)&tmp, sizeof(int32_t) * (size_t)(c->nrows + 1)));
+        COMET_HIPCHK(dev_malloc((void **)&tmp, sizeof(int32_t) * (size_t)(c->nrows + 1)));
         unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(c->nrows + 1, 256), 65536);
         narrow_i64_to_i32<<<dim3(blocks), dim3(256), 0, s>>>(c->pos, tmp, c->nrows + 1);
         hipError_t e = hipMemcpyAsync(pos, tmp, sizeof(int32_t) * (size_t)(c->nrows + 1), hipMemcpyDeviceToHost, s);
         hipError_t e2 = hipStreamSynchronize(s);
-        (void)hipFree(tmp);
+        (void)dev_free(tmp);
         COMET_HIPCHK(e);
         COMET_HIPCHK(e2);
     }
@@ -961,7 +1101,8 @@ int comet_hip_csr_destroy(int64_t csr)
     Csr *c = csr_from_handle(csr, true);
     if (!c)
         return COMET_HIP_ERR_HANDLE;
-    COMET_HIPCHK(hipStreamSynchronize(stream()));
+    if (!c->owns)          // the caller may free or rewrite the arrays as soon as this returns
+        COMET_HIPCHK(hipStreamSynchronize(stream()));
     {
         std::lock_guard<std::mutex> lk(g_mu);
         g_live.erase(c);

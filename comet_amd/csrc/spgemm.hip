@@ -3309,15 +3309,15 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
     if (keep && n > 0) {
         // a copy of its own; failing to get the memory only means that the list is built again next time
         if (owner->row_lists.size() >= SG_ROW_LISTS_KEPT) {
-            COMET_HIPCHK(hipStreamSynchronize(stream()));        // a kernel may still be reading the oldest one
-            (void)hipFree(owner->row_lists.front().rows);
-            (void)hipFree(owner->row_lists.front().bounds);
+            COMET_CHK(stream_wait());        // a kernel may still be reading the oldest one
+            (void)dev_free(owner->row_lists.front().rows);
+            (void)dev_free(owner->row_lists.front().bounds);
             owner->row_lists.erase(owner->row_lists.begin());
         }
-        if (hipMalloc((void **)&key.rows, 4 * (size_t)n) != hipSuccess ||
-            hipMalloc((void **)&key.bounds, 24) != hipSuccess) {
+        if (dev_malloc((void **)&key.rows, 4 * (size_t)n) != hipSuccess ||
+            dev_malloc((void **)&key.bounds, 24) != hipSuccess) {
             (void)hipGetLastError();
-            (void)hipFree(key.rows);
+            (void)dev_free(key.rows);
             return COMET_HIP_OK;
         }
         COMET_HIPCHK(hipMemcpyAsync(key.rows, g_rl.idx_out.ptr, 4 * (size_t)n, hipMemcpyDeviceToDevice, stream()));
@@ -3405,14 +3405,14 @@ static int sg_plan_blocks(Csr *b)
     if (b->sg_blkptr && b->sg_nblk == nblk)
         return COMET_HIP_OK;
     if (b->sg_blkptr) {
-        COMET_HIPCHK(hipStreamSynchronize(stream()));
-        COMET_HIPCHK(hipFree(b->sg_blkptr));
-        (void)hipFree(b->sg_crd16);
+        COMET_CHK(stream_wait());
+        COMET_HIPCHK(dev_free(b->sg_blkptr));
+        (void)dev_free(b->sg_crd16);
         b->sg_blkptr = nullptr;
         b->sg_crd16 = nullptr;
     }
     static_assert(SG_CB <= 65536, "a column inside its block fits 16 bits");
-    if (hipMalloc((void **)&b->sg_crd16, sizeof(uint16_t) * (size_t)(b->nnz > 0 ? b->nnz : 1)) != hipSuccess) {
+    if (dev_malloc((void **)&b->sg_crd16, sizeof(uint16_t) * (size_t)(b->nnz > 0 ? b->nnz : 1)) != hipSuccess) {
         (void)hipGetLastError();        // an allocation that may fail: its error must not reach the next check
         b->sg_crd16 = nullptr;          // the kernel then reads the 32-bit columns
     } else if (b->nnz > 0) {
@@ -3420,7 +3420,7 @@ static int sg_plan_blocks(Csr *b)
                                                                                                  b->sg_crd16);
         COMET_HIPCHK(hipGetLastError());
     }
-    COMET_HIPCHK(hipMalloc((void **)&b->sg_blkptr,
+    COMET_HIPCHK(dev_malloc((void **)&b->sg_blkptr,
                            sizeof(int64_t) * (size_t)(nblk + 1) * (size_t)(b->nrows > 0 ? b->nrows : 1)));
     b->sg_nblk = nblk;
     if (b->nrows > 0) {
@@ -3453,7 +3453,7 @@ static int dot_transposed_index(const Csr *x, Csr **out)
     Csr *m = const_cast<Csr *>(x);
     if (!m->transposed_index) {
         double *iota = nullptr;
-        COMET_HIPCHK(hipMalloc((void **)&iota, sizeof(double) * (size_t)(m->nnz > 0 ? m->nnz : 1)));
+        COMET_HIPCHK(dev_malloc((void **)&iota, sizeof(double) * (size_t)(m->nnz > 0 ? m->nnz : 1)));
         if (m->nnz > 0)
             fill_iota_f64<<<dim3((unsigned)ceil_div(m->nnz, 256)), dim3(256), 0, stream()>>>(m->nnz, iota);
         Csr view;
@@ -3465,7 +3465,7 @@ static int dot_transposed_index(const Csr *x, Csr **out)
         view.val = iota;
         m->transposed_index = csr_transposed_copy(&view);
         const hipError_t e = hipStreamSynchronize(stream());
-        (void)hipFree(iota);
+        (void)dev_free(iota);
         if (!m->transposed_index || e != hipSuccess)
             return set_error(COMET_HIP_ERR_HIP, "transposing the mask failed");
     }
@@ -3485,7 +3485,7 @@ static int dot_no_duplicates(const Csr *x, bool *ok)
                                                                                                    (int *)g_dot_flag.ptr);
         int flag = 0;
         COMET_HIPCHK(hipMemcpyAsync(&flag, g_dot_flag.ptr, sizeof(int), hipMemcpyDeviceToHost, stream()));
-        COMET_HIPCHK(hipStreamSynchronize(stream()));
+        COMET_CHK(stream_wait());
         m->dup_state = flag ? 2 : 1;
     }
     *ok = m->dup_state == 1;
@@ -3519,7 +3519,7 @@ static int dot_pairs(const Csr *a, const Csr *b, const Csr *m, int64_t rb, int64
     int64_t ends[2] = {0, 0};
     COMET_HIPCHK(hipMemcpyAsync(&ends[0], m->pos + rb, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
     COMET_HIPCHK(hipMemcpyAsync(&ends[1], m->pos + re, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
-    COMET_HIPCHK(hipStreamSynchronize(stream()));
+    COMET_CHK(stream_wait());
     const int64_t out0 = ends[0], npairs = ends[1] - ends[0];
     COMET_CHK(g_dot_hit.ensure((size_t)(npairs > 0 ? npairs : 1), false));
     COMET_CHK(g_dot_val.ensure(sizeof(double) * (size_t)(npairs > 0 ? npairs : 1), false));
@@ -3652,7 +3652,7 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     if (by_blocks) {
         int64_t nd = 0;
         COMET_HIPCHK(hipMemcpyAsync(&nd, list.bounds + 2, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
-        COMET_HIPCHK(hipStreamSynchronize(stream()));
+        COMET_CHK(stream_wait());
         if (nd > 0) {
             ran_blocks = true;
             COMET_CHK(g_sg.dense_rows.ensure(sizeof(DenseRow) * (size_t)nd, false));
@@ -3738,7 +3738,7 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     if (ran_blocks) {           // did a workgroup stop waiting for the block before its own
         int gave_up = 0;
         COMET_HIPCHK(hipMemcpyAsync(&gave_up, g_sg.gave_up.ptr, sizeof(int), hipMemcpyDeviceToHost, stream()));
-        COMET_HIPCHK(hipStreamSynchronize(stream()));
+        COMET_CHK(stream_wait());
         if (gave_up) {
             COMET_HIPCHK(hipMemsetAsync(g_sg.gave_up.ptr, 0, sizeof(int), stream()));
             return set_error(COMET_HIP_ERR_HIP, "spgemm numeric: a column block's place in its row never arrived");
@@ -3768,7 +3768,7 @@ extern "C" int comet_hip_spgemm_csr_symbolic(int64_t ah, int64_t bh, int64_t mh,
     COMET_CHK(exclusive_scan_i64((const int64_t *)g_sg.rowcount.ptr, a->nrows, pos));
     if (nnz_out) {
         COMET_HIPCHK(hipMemcpyAsync(nnz_out, pos + a->nrows, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
-        COMET_HIPCHK(hipStreamSynchronize(stream()));
+        COMET_CHK(stream_wait());
     }
     return COMET_HIP_OK;
 }
@@ -3831,7 +3831,7 @@ static int64_t masked_product_one_pass(const Csr *a, const Csr *b, const Csr *m,
         csr_release(c);
         return 0;
     };
-    if (hipMalloc((void **)&c->pos, sizeof(int64_t) * (size_t)(a->nrows + 1)) != hipSuccess)
+    if (dev_malloc((void **)&c->pos, sizeof(int64_t) * (size_t)(a->nrows + 1)) != hipSuccess)
         return fail("row pointer allocation failed");
     {
         KernelTimer t("spgemm_symbolic_dot_count");
@@ -3841,10 +3841,10 @@ static int64_t masked_product_one_pass(const Csr *a, const Csr *b, const Csr *m,
     if (exclusive_scan_i64((const int64_t *)g_sg.rowcount.ptr, a->nrows, c->pos) != COMET_HIP_OK)
         return fail(nullptr);
     if (hipMemcpyAsync(&c->nnz, c->pos + a->nrows, sizeof(int64_t), hipMemcpyDeviceToHost, stream()) != hipSuccess ||
-        hipStreamSynchronize(stream()) != hipSuccess)
+        stream_wait() != COMET_HIP_OK)
         return fail("reading the size of the product failed");
-    if (hipMalloc((void **)&c->crd, sizeof(int32_t) * (size_t)(c->nnz > 0 ? c->nnz : 1)) != hipSuccess ||
-        hipMalloc((void **)&c->val, sizeof(double) * (size_t)(c->nnz > 0 ? c->nnz : 1)) != hipSuccess)
+    if (dev_malloc((void **)&c->crd, sizeof(int32_t) * (size_t)(c->nnz > 0 ? c->nnz : 1)) != hipSuccess ||
+        dev_malloc((void **)&c->val, sizeof(double) * (size_t)(c->nnz > 0 ? c->nnz : 1)) != hipSuccess)
         return fail("output allocation failed");
     {
         KernelTimer t("spgemm_numeric_dot_compact");
@@ -3872,13 +3872,13 @@ extern "C" int64_t comet_hip_spgemm_csr_semiring(int64_t ah, int64_t bh, int64_t
             return h;
     }
     int64_t *pos = nullptr;
-    if (hipMalloc((void **)&pos, sizeof(int64_t) * (size_t)(a->nrows + 1)) != hipSuccess) {
+    if (dev_malloc((void **)&pos, sizeof(int64_t) * (size_t)(a->nrows + 1)) != hipSuccess) {
         set_error(COMET_HIP_ERR_HIP, "row pointer allocation failed");
         return 0;
     }
     int64_t nnz = 0;
     if (comet_hip_spgemm_csr_symbolic(ah, bh, mh, (int64_t)pos, &nnz) != COMET_HIP_OK) {
-        (void)hipFree(pos);
+        (void)dev_free(pos);
         return 0;
     }
     Csr *c = new Csr();
@@ -3887,18 +3887,18 @@ extern "C" int64_t comet_hip_spgemm_csr_semiring(int64_t ah, int64_t bh, int64_t
     c->nnz = nnz;
     c->pos = pos;
     c->owns = true;
-    if (hipMalloc((void **)&c->crd, sizeof(int32_t) * (size_t)(nnz > 0 ? nnz : 1)) != hipSuccess ||
-        hipMalloc((void **)&c->val, sizeof(double) * (size_t)(nnz > 0 ? nnz : 1)) != hipSuccess) {
+    if (dev_malloc((void **)&c->crd, sizeof(int32_t) * (size_t)(nnz > 0 ? nnz : 1)) != hipSuccess ||
+        dev_malloc((void **)&c->val, sizeof(double) * (size_t)(nnz > 0 ? nnz : 1)) != hipSuccess) {
         set_error(COMET_HIP_ERR_HIP, "output allocation of %lld entries failed", (long long)nnz);
-        (void)hipFree(c->crd);
-        (void)hipFree(pos);
+        (void)dev_free(c->crd);
+        (void)dev_free(pos);
         delete c;
         return 0;
     }
     if (nnz > 0 && numeric_rows(a, b, m, pos, 0, a->nrows, c->crd, c->val, reduce_op, mult_op) != COMET_HIP_OK) {
-        (void)hipFree(c->crd);
-        (void)hipFree(c->val);
-        (void)hipFree(pos);
+        (void)dev_free(c->crd);
+        (void)dev_free(c->val);
+        (void)dev_free(pos);
         delete c;
         return 0;
     }
@@ -3918,7 +3918,7 @@ static int csr_is_iso(const Csr *x, bool *iso)
             COMET_HIPCHK(hipGetLastError());
             COMET_HIPCHK(hipMemcpyAsync(&flag, g_dot_flag.ptr, sizeof(int), hipMemcpyDeviceToHost, stream()));
             COMET_HIPCHK(hipMemcpyAsync(&m->iso_value, m->val, sizeof(double), hipMemcpyDeviceToHost, stream()));
-            COMET_HIPCHK(hipStreamSynchronize(stream()));
+            COMET_CHK(stream_wait());
         }
         m->iso_state = flag ? 2 : 1;
     }
@@ -4030,17 +4030,17 @@ extern "C" int64_t comet_hip_eltwise_mult_csr(int64_t ah, int64_t bh)
     }
     const int64_t n = a->nrows;
     int64_t *pos = nullptr;
-    if (hipMalloc((void **)&pos, sizeof(int64_t) * (size_t)(n + 1)) != hipSuccess) {
+    if (dev_malloc((void **)&pos, sizeof(int64_t) * (size_t)(n + 1)) != hipSuccess) {
         set_error(COMET_HIP_ERR_HIP, "row pointer allocation failed");
         return 0;
     }
     auto fail = [&](Csr *c) -> int64_t {
         if (c) {
-            (void)hipFree(c->crd);
-            (void)hipFree(c->val);
+            (void)dev_free(c->crd);
+            (void)dev_free(c->val);
             delete c;
         }
-        (void)hipFree(pos);
+        (void)dev_free(pos);
         return 0;
     };
     if (g_sg.rowcount.ensure(sizeof(int64_t) * (size_t)(n > 0 ? n : 1), false) != COMET_HIP_OK)
@@ -4056,7 +4056,7 @@ extern "C" int64_t comet_hip_eltwise_mult_csr(int64_t ah, int64_t bh)
         return fail(nullptr);
     int64_t nnz = 0;
     if (hipMemcpyAsync(&nnz, pos + n, sizeof(int64_t), hipMemcpyDeviceToHost, stream()) != hipSuccess ||
-        hipStreamSynchronize(stream()) != hipSuccess) {
+        stream_wait() != COMET_HIP_OK) {
         set_error(COMET_HIP_ERR_HIP, "reading nnz failed");
         return fail(nullptr);
     }
@@ -4066,8 +4066,8 @@ extern "C" int64_t comet_hip_eltwise_mult_csr(int64_t ah, int64_t bh)
     c->nnz = nnz;
     c->pos = pos;
     c->owns = true;
-    if (hipMalloc((void **)&c->crd, sizeof(int32_t) * (size_t)(nnz > 0 ? nnz : 1)) != hipSuccess ||
-        hipMalloc((void **)&c->val, sizeof(double) * (size_t)(nnz > 0 ? nnz : 1)) != hipSuccess) {
+    if (dev_malloc((void **)&c->crd, sizeof(int32_t) * (size_t)(nnz > 0 ? nnz : 1)) != hipSuccess ||
+        dev_malloc((void **)&c->val, sizeof(double) * (size_t)(nnz > 0 ? nnz : 1)) != hipSuccess) {
         set_error(COMET_HIP_ERR_HIP, "output allocation failed");
         return fail(c);
     }

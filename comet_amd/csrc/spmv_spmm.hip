@@ -278,11 +278,11 @@ static int spmv_plan(Csr *a)
     int64_t *bpos = nullptr;
     int32_t *bcrd = nullptr;
     double *bval = nullptr;
-    COMET_HIPCHK(hipMalloc((void **)&bpos, sizeof(int64_t) * (size_t)nb * (size_t)(n + 1)));
+    COMET_HIPCHK(dev_malloc((void **)&bpos, sizeof(int64_t) * (size_t)nb * (size_t)(n + 1)));
     auto cleanup = [&]() {
-        (void)hipFree(bpos);
-        (void)hipFree(bcrd);
-        (void)hipFree(bval);
+        (void)dev_free(bpos);
+        (void)dev_free(bcrd);
+        (void)dev_free(bval);
     };
     const dim3 grid((unsigned)ceil_div(n, 256)), block(256);
     {
@@ -317,8 +317,8 @@ static int spmv_plan(Csr *a)
         run += totals[b];
     }
     // the blocks cut every row into consecutive segments, so they always hold all nonzeros, in order
-    if (hipMalloc((void **)&bcrd, sizeof(int32_t) * (size_t)a->nnz) != hipSuccess ||
-        hipMalloc((void **)&bval, sizeof(double) * (size_t)a->nnz) != hipSuccess) {
+    if (dev_malloc((void **)&bcrd, sizeof(int32_t) * (size_t)a->nnz) != hipSuccess ||
+        dev_malloc((void **)&bval, sizeof(double) * (size_t)a->nnz) != hipSuccess) {
         cleanup();
         return set_error(COMET_HIP_ERR_HIP, "allocating the column-blocked copy failed");
     }
@@ -338,14 +338,14 @@ static int spmv_plan(Csr *a)
     if (narrow) {
         int32_t *bpos32 = nullptr;
         const int64_t count = (int64_t)nb * (n + 1);
-        if (hipMalloc((void **)&bpos32, sizeof(int32_t) * (size_t)count) == hipSuccess) {
+        if (dev_malloc((void **)&bpos32, sizeof(int32_t) * (size_t)count) == hipSuccess) {
             spmv_narrow_pos<<<dim3((unsigned)ceil_div(count, 256)), dim3(256), 0, stream()>>>(bpos, bpos32, count);
             if (hipStreamSynchronize(stream()) == hipSuccess) {
                 a->spmv_bpos32 = bpos32;
-                (void)hipFree(bpos);
+                (void)dev_free(bpos);
                 bpos = nullptr;
             } else {
-                (void)hipFree(bpos32);
+                (void)dev_free(bpos32);
             }
         } else {
             (void)hipGetLastError();        // an allocation that may fail: the 64-bit pointers stay in use
@@ -880,10 +880,10 @@ static int spmm_plan(Csr *a)
     if (a->spmm_chunk_row && a->spmm_nchunks == nchunks)
         return COMET_HIP_OK;
     if (a->spmm_chunk_row) {
-        COMET_HIPCHK(hipFree(a->spmm_chunk_row));
+        COMET_HIPCHK(dev_free(a->spmm_chunk_row));
         a->spmm_chunk_row = nullptr;
     }
-    COMET_HIPCHK(hipMalloc((void **)&a->spmm_chunk_row, sizeof(int32_t) * (size_t)(nchunks > 0 ? nchunks : 1)));
+    COMET_HIPCHK(dev_malloc((void **)&a->spmm_chunk_row, sizeof(int32_t) * (size_t)(nchunks > 0 ? nchunks : 1)));
     a->spmm_nchunks = nchunks;
     if (nchunks > 0) {
         KernelTimer t("spmm_chunk_rows");
@@ -1237,15 +1237,15 @@ static int spmm_heavy_plan(Csr *a)
     Csr *light = new Csr();
     char *scratch = nullptr;        // everything that does not outlive the planning, in one allocation
     auto cleanup = [&](bool failed) {
-        (void)hipFree(scratch);
+        (void)dev_free(scratch);
         if (failed) {
-            (void)hipFree(a->heavy_seg);
-            (void)hipFree(a->heavy_ent);
-            (void)hipFree(a->heavy_row);
-            (void)hipFree(a->heavy_code);
-            (void)hipFree(a->medium_row);
+            (void)dev_free(a->heavy_seg);
+            (void)dev_free(a->heavy_ent);
+            (void)dev_free(a->heavy_row);
+            (void)dev_free(a->heavy_code);
+            (void)dev_free(a->medium_row);
             a->medium_row = nullptr;
-            (void)hipFree(a->empty_rows);
+            (void)dev_free(a->empty_rows);
             a->heavy_seg = nullptr;
             a->heavy_ent = nullptr;
             a->heavy_row = a->heavy_code = a->empty_rows = nullptr;
@@ -1276,7 +1276,7 @@ static int spmm_heavy_plan(Csr *a)
                      o_iin = room(4 * (size_t)nent), o_iout = room(4 * (size_t)nent), o_first = room(8 * (size_t)nent),
                      o_runs = room(8 * (size_t)(nent + 1)), o_start = room(8 * (size_t)(nent + 1)),
                      o_odd = room(8 * (size_t)nent), o_pads = room(8 * (size_t)(nent + 1));
-        HEAVY_TRY(hipMalloc((void **)&scratch, total));
+        HEAVY_TRY(dev_malloc((void **)&scratch, total));
         d_cnt = (int32_t *)(scratch + o_cnt);
         d_srow = (int32_t *)(scratch + o_srow);
         d_hstart = (int64_t *)(scratch + o_hstart);
@@ -1292,15 +1292,15 @@ static int spmm_heavy_plan(Csr *a)
         d_odd = (int64_t *)(scratch + o_odd);
         d_pads = (int64_t *)(scratch + o_pads);
     }
-    HEAVY_TRY(hipMalloc((void **)&a->medium_row, 4 * at_least_one(M)));
+    HEAVY_TRY(dev_malloc((void **)&a->medium_row, 4 * at_least_one(M)));
     if (M > 0)
         HEAVY_TRY(hipMemcpyAsync(a->medium_row, mrow.data(), 4 * (size_t)M, hipMemcpyHostToDevice, stream()));
     HEAVY_TRY(hipMemcpyAsync(d_mstart, mstart.data(), 8 * (size_t)(M + 1), hipMemcpyHostToDevice, stream()));
-    HEAVY_TRY(hipMalloc((void **)&a->heavy_seg, 8 * (size_t)(8 * hbins + 1)));
-    HEAVY_TRY(hipMalloc((void **)&a->heavy_row, 4 * (size_t)H));
-    HEAVY_TRY(hipMalloc((void **)&a->heavy_code, 4 * (size_t)(8 * H)));
-    HEAVY_TRY(hipMalloc((void **)&a->empty_rows, 4 * at_least_one(E)));
-    HEAVY_TRY(hipMalloc((void **)&light->rowmap, 4 * at_least_one(L)));
+    HEAVY_TRY(dev_malloc((void **)&a->heavy_seg, 8 * (size_t)(8 * hbins + 1)));
+    HEAVY_TRY(dev_malloc((void **)&a->heavy_row, 4 * (size_t)H));
+    HEAVY_TRY(dev_malloc((void **)&a->heavy_code, 4 * (size_t)(8 * H)));
+    HEAVY_TRY(dev_malloc((void **)&a->empty_rows, 4 * at_least_one(E)));
+    HEAVY_TRY(dev_malloc((void **)&light->rowmap, 4 * at_least_one(L)));
     HEAVY_TRY(hipMemcpyAsync(a->heavy_row, hrow.data(), 4 * (size_t)H, hipMemcpyHostToDevice, stream()));
     if (S > 0)
         HEAVY_TRY(hipMemcpyAsync(d_srow, srow.data(), 4 * (size_t)S, hipMemcpyHostToDevice, stream()));
@@ -1376,7 +1376,7 @@ static int spmm_heavy_plan(Csr *a)
     }
     HEAVY_TRY(hipMemcpyAsync(&npads, d_pads + nruns, 8, hipMemcpyDeviceToHost, stream()));
     HEAVY_TRY(hipStreamSynchronize(stream()));
-    HEAVY_TRY(hipMalloc((void **)&a->heavy_ent, sizeof(HeavyEnt) * (size_t)(nent + npads)));
+    HEAVY_TRY(dev_malloc((void **)&a->heavy_ent, sizeof(HeavyEnt) * (size_t)(nent + npads)));
     {
         KernelTimer t("heavy_fill");
         heavy_fill<<<dim3((unsigned)ceil_div(nent, 256)), dim3(256), 0, stream()>>>(
@@ -1390,9 +1390,9 @@ static int spmm_heavy_plan(Csr *a)
     light->ncols = a->ncols;
     light->nnz = a->nnz - hnnz - S - mnnz;
     light->owns = true;
-    HEAVY_TRY(hipMalloc((void **)&light->pos, 8 * (size_t)(L + 1)));
-    HEAVY_TRY(hipMalloc((void **)&light->crd, 4 * at_least_one(light->nnz)));
-    HEAVY_TRY(hipMalloc((void **)&light->val, 8 * at_least_one(light->nnz)));
+    HEAVY_TRY(dev_malloc((void **)&light->pos, 8 * (size_t)(L + 1)));
+    HEAVY_TRY(dev_malloc((void **)&light->crd, 4 * at_least_one(light->nnz)));
+    HEAVY_TRY(dev_malloc((void **)&light->val, 8 * at_least_one(light->nnz)));
     if (L > 0) {
         light_lengths<<<dim3((unsigned)ceil_div(L, 256)), dim3(256), 0, stream()>>>(L, light->rowmap, a->pos, d_len);
         if (exclusive_scan_i64(d_len, L, light->pos) != COMET_HIP_OK) {
