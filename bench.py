@@ -306,7 +306,7 @@ def bench_ttgt(rt, orc, gen, args):
     kt = kernel_times(rt, step, args.steps)
     M = N = K = e * e
     flops = 2.0 * M * N * K
-    dom = "dgemm_mfma_kernel"
+    dom = "gett_mfma_kernel"
     dom_ms = kt[dom]["avg_ms"]
     # parity on a slab of the output: C[a0,b0,:,:] against the checker's GEMM order is too slow at e = 64,
     # so compare with numpy's einsum on a few (a,b) pairs, tolerance relative to sum |a||b|
@@ -336,7 +336,7 @@ def bench_ttgt(rt, orc, gen, args):
     peak = C.c_double(float("nan"))
     if not args.no_peak:        # the yardstick kernel; left out of a profiled run so that the trace holds the workload only
         rt._check(rt.lib().comet_hip_mfma_f64_peak(20000, C.byref(peak)), "comet_hip_mfma_f64_peak")
-    perm_bytes = 2 * 8 * e ** 4 * (plan.transA + plan.transB + plan.transC)
+    perm_bytes = 2 * 8 * e ** 4        # both operands are contiguous along k in different dimensions: one is turned
     return {
         "metric": "TTGT contraction TFLOP/s (fp64 MFMA GEMM + LDS-tiled transposes) on 1 MI355X",
         "value": flops / (dev_ms * 1e-3) / 1e12, "unit": "TFLOP/s", "ms_per_step": dev_ms, "dtype": "f64",

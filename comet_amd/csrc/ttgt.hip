@@ -9,6 +9,9 @@
 // (linalg.matmul -> loops, frontends/comet_dsl/comet.cpp:594-595, or the BLIS
 // micro-kernel of lib/ExecutionEngine/blis_interface.cpp:143-181) replaced by
 // v_mfma_f64_16x16x4_f64 tiles.
+#include <stdio.h>
+#include <stdlib.h>
+
 #include <algorithm>
 #include <cstring>
 
@@ -206,157 +209,604 @@ static int transpose_device(int rank, const int64_t *in_shape, const int32_t *pe
 }
 
 // ============================================================================
-// DGEMM, row-major, C[M,N] = beta*C + A[M,K]*B[K,N].
-// Workgroup tile 128 x 128, four wavefronts in a 2 x 2 arrangement, each
-// wavefront 64 x 64 as 4 x 4 MFMA tiles (16 accumulators of 4 doubles per
-// lane).  K advances 16 at a time through double-buffered LDS: A is stored
-// k-major (so a 16 x 4 operand is read with one ds_read_b64 per lane), B as in
-// memory.  Operand layout of v_mfma_f64_16x16x4_f64: lane l supplies
-// A[l%16][l/16] and B[l/16][l%16] and receives D[4*v + l/16][l%16], v = 0..3
-// (measured on gfx950 with one-hot operands).
+// Contraction on strided operands: C[m,n] (+)= sum_k A[m,k] * B[k,n], where m, n
+// and k are multi-indices and the address of an element is the sum of an offset
+// that depends on m (or n) alone and one that depends on k alone.  A tensor in
+// any index order is such a matrix, so nothing is transposed: the loads that
+// bring a tile to LDS follow the tensor's own layout.  DGEMM is the case of one
+// index each.
+//
+// A workgroup (four wavefronts) makes a BM x BN tile of C, each wavefront
+// TM x TN MFMA tiles of 16 x 16.  K advances 16 at a time through
+// double-buffered LDS, both operands stored k-major (a 16 x 4 operand is one
+// ds_read_b64 per lane).  Offsets of the rows and columns are worked out once
+// per tile of C, those of the 16 k of a turn by sixteen lanes two turns ahead.
+// A thread takes its elements along whichever index is contiguous in memory
+// (A_M / B_N: the outer one, else along k).  Operand layout of
+// v_mfma_f64_16x16x4_f64: lane l supplies A[l%16][l/16] and B[l/16][l%16] and
+// receives D[4*v + l/16][l%16], v = 0..3 (measured with one-hot operands).
+//
+// Rows and columns beyond the matrix repeat the last one and are not stored; k
+// beyond the end reads the last k and counts as zero.
+//
+// The sum over k may be shared out over gridDim.y workgroups per tile, which
+// leave partial tiles that gett_reduce adds in order: a contraction with few
+// outputs and a long sum otherwise runs on a handful of CUs (30 x 61 outputs
+// over 54,900 products: 8.7 ms on the one workgroup that a 128 x 128 tile gave it).
 // ============================================================================
-#ifndef COMET_GM_BK
-#define COMET_GM_BK 16
-#endif
-#ifndef COMET_GM_PAD
-#define COMET_GM_PAD 4
-#endif
 #ifndef COMET_GM_OCC
 #define COMET_GM_OCC 2
 #endif
-// Measured on the 4096^3 product: 2 wavefronts per SIMD (register budget 256) lifts the kernel from 62 % to
-// 90 % of the fp64 MFMA peak; a deeper K tile (32) does not fit two workgroups' LDS and falls back to 59 %.
-constexpr int GM_BM = 128, GM_BN = 128, GM_BK = COMET_GM_BK;
-constexpr int GM_LDA = GM_BM + COMET_GM_PAD;   // padded leading dimensions (doubles)
-constexpr int GM_LDB = GM_BN + COMET_GM_PAD;
-constexpr int GM_EA = GM_BM * GM_BK / 256;     // doubles each lane stages per tile of A (along k)
-constexpr int GM_EB = GM_BK * GM_BN / 256;     // ... and of B (along n)
+constexpr int GM_BK = 16, GM_PAD = 4;
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
-template <bool GUARD>
-__global__ __launch_bounds__(256, COMET_GM_OCC) void dgemm_mfma_kernel(int64_t M, int64_t N, int64_t K,
-                                                         const double *__restrict__ A,
-                                                         const double *__restrict__ B, double *__restrict__ C,
-                                                         int use_c)
+// A multi-index: extents (outermost first) and the strides of its dimensions in the two tensors it appears in.
+struct GettIndex {
+    int nd;
+    uint32_t ext[TR_MAXRANK];
+    int64_t s0[TR_MAXRANK], s1[TR_MAXRANK];
+};
+struct GettArgs {
+    GettIndex m, n, k;           // m: A, C   n: B, C   k: A, B
+    uint32_t M, N, K;
+    uint32_t turns;              // turns of 16 k per split
+};
+
+// an element by its byte offset from a pointer that is the same for the whole wavefront
+template <typename OFF>
+__device__ __forceinline__ double gett_load(const double *base, OFF bytes)
 {
-    __shared__ double As[2][GM_BK][GM_LDA];
-    __shared__ double Bs[2][GM_BK][GM_LDB];
+    return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(base) + bytes);
+}
+
+// The same with the wavefront's part of the offset in a scalar register: a buffer load, whose address needs no vector
+// arithmetic (the compiler turns pointer + offset into a 64-bit add per load inside the loop).
+typedef double double2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t gett_buffer(const double *p)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(p), 0, -1, 0x00027000);
+}
+__device__ __forceinline__ double gett_fetch(__amdgpu_buffer_rsrc_t p, uint32_t bytes, uint32_t scalar_bytes)
+{
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(p, bytes, scalar_bytes, 0));
+}
+__device__ __forceinline__ double2_t gett_fetch2(__amdgpu_buffer_rsrc_t p, uint32_t bytes, uint32_t scalar_bytes)
+{
+    return __builtin_bit_cast(double2_t, __builtin_amdgcn_raw_buffer_load_b128(p, bytes, scalar_bytes, 0));
+}
+
+template <typename OFF>
+__device__ __forceinline__ void gett_offsets(const GettIndex &g, uint32_t i, OFF *o0, OFF *o1)
+{
+    OFF a = 0, b = 0;
+    for (int d = g.nd - 1; d > 0; --d) {
+        const uint32_t q = i / g.ext[d], r = i - q * g.ext[d];
+        a += (OFF)r * (OFF)g.s0[d];
+        b += (OFF)r * (OFF)g.s1[d];
+        i = q;
+    }
+    *o0 = a + (OFF)i * (OFF)g.s0[0];
+    *o1 = b + (OFF)i * (OFF)g.s1[0];
+}
+
+template <int BM, int BN, int WM, int OCC, bool A_M, bool B_N, bool REG, bool RUN, typename OFF>
+__global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const double *__restrict__ A,
+                                                             const double *__restrict__ B, double *__restrict__ C,
+                                                             double *__restrict__ partial, int use_c)
+{
+    constexpr int WN = 4 / WM, TM = BM / WM / 16, TN = BN / WN / 16;
+    constexpr int EA = BM / 16, EB = BN / 16;               // elements a thread stages per turn
+    constexpr int LDA = BM + GM_PAD, LDB = BN + GM_PAD;
+    constexpr int KSA = 256 / BM, KSB = 256 / BN;
+    __shared__ double As[2][GM_BK][LDA];
+    __shared__ double Bs[2][GM_BK][LDB];
+    // offsets in bytes of the rows (A), the columns (B) and, unless they are regular, of the k of two turns
+    __shared__ OFF rowA[BM], colB[BN], kA[2][GM_BK], kB[2][GM_BK];
+    __shared__ int64_t rowC[BM], colC[BN];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    // neighbouring workgroups share a block row of A: walk N fastest inside groups of 8 block rows
-    const int64_t bm = blockIdx.y, bn = blockIdx.x;
-    const int64_t m0 = bm * GM_BM, n0 = bn * GM_BN;
+    const int wm = wave / WN, wn = wave % WN;
+    const uint32_t tiles_n = (g.N + BN - 1) / BN;
+    const uint32_t m0 = blockIdx.x / tiles_n * BM, n0 = blockIdx.x % tiles_n * BN;
+    const uint32_t k_begin = blockIdx.y * g.turns * GM_BK;
+    const uint32_t k_end = k_begin + g.turns * GM_BK < g.K ? k_begin + g.turns * GM_BK : g.K;
+    const int nt = (int)((k_end - k_begin + GM_BK - 1) / GM_BK);
 
-    // global -> register staging: A tile 128 x BK (two lanes per row, GM_EA consecutive k each),
-    // B tile BK x 128 (GM_EB consecutive columns per lane)
-    const int a_row = tid / (GM_BK / GM_EA), a_k = (tid % (GM_BK / GM_EA)) * GM_EA;
-    const int b_k = tid / (GM_BN / GM_EB), b_col = (tid % (GM_BN / GM_EB)) * GM_EB;
-    double ra[GM_EA], rb[GM_EB];
-
-    auto load_tiles = [&](int64_t k0) {
-        const int64_t gm = m0 + a_row;
-        const double *ap = A + gm * K + k0 + a_k;
-#pragma unroll
-        for (int e = 0; e < GM_EA; ++e) {
-            if (GUARD)
-                ra[e] = (gm < M && k0 + a_k + e < K) ? ap[e] : 0.0;
-            else
-                ra[e] = ap[e];
-        }
-        const int64_t gk = k0 + b_k;
-        const double *bp = B + gk * N + n0 + b_col;
-#pragma unroll
-        for (int e = 0; e < GM_EB; ++e) {
-            if (GUARD)
-                rb[e] = (gk < K && n0 + b_col + e < N) ? bp[e] : 0.0;
-            else
-                rb[e] = bp[e];
+    const auto k_offsets = [&](int t) {          // the offsets of turn t's k, by the first sixteen lanes
+        if (!REG && tid < GM_BK) {
+            const uint32_t k = k_begin + (uint32_t)t * GM_BK + tid;
+            OFF a, b;
+            gett_offsets(g.k, k < k_end ? k : k_end - 1, &a, &b);
+            kA[t & 1][tid] = a * 8;
+            kB[t & 1][tid] = b * 8;
         }
     };
-    auto store_tiles = [&](int buf) {
+    for (int r = tid; r < BM; r += 256) {
+        int64_t a, c;
+        gett_offsets(g.m, m0 + r < g.M ? m0 + r : g.M - 1, &a, &c);
+        rowA[r] = (OFF)(a * 8);
+        rowC[r] = c;
+    }
+    for (int c = tid; c < BN; c += 256) {
+        int64_t b, d;
+        gett_offsets(g.n, n0 + c < g.N ? n0 + c : g.N - 1, &b, &d);
+        colB[c] = (OFF)(b * 8);
+        colC[c] = d;
+    }
+    k_offsets(0);
+    if (nt > 1)
+        k_offsets(1);
+    __syncthreads();
+
+    // thread -> elements of a turn's tiles: along the outer index (one row, E values of k) or along k (one k, E rows).
+    // REG: sixteen k of a turn are always equally spaced, so an element's offset from the turn's first k never
+    // changes: it stays in a register, the turn's part is added to the pointer by the scalar unit, and a turn costs
+    // no vector arithmetic at all - it would be taken from the matrix cores' time (4096^3: 2318 us with an add and a
+    // 64-bit shift per element, see the figures at GETT_SHAPES).
+    // RUN: a thread's elements follow each other along the contiguous index: one address, sixteen bytes a load.
+    const int a_k = RUN ? (A_M ? tid / 16 : tid * EA % 16) : A_M ? tid / BM : tid & 15;
+    const int a_r = RUN ? (A_M ? tid % 16 * EA : tid * EA / 16) : A_M ? tid % BM : tid >> 4;
+    const int b_k = RUN ? (B_N ? tid / 16 : tid * EB % 16) : B_N ? tid / BN : tid & 15;
+    const int b_c = RUN ? (B_N ? tid % 16 * EB : tid * EB / 16) : B_N ? tid % BN : tid >> 4;
+    const int last = g.k.nd - 1;
+    const int64_t sa = g.k.s0[last], sb = g.k.s1[last];          // strides of the innermost k
+    constexpr int NA = RUN || (A_M && !REG) ? 1 : EA, NB = RUN || (B_N && !REG) ? 1 : EB;
+    OFF ao[NA], bo[NB];
+    if constexpr (RUN) {           // a run beyond the last row (their number is a multiple of EA then) is the last one
+        const int ar = A_M && m0 + a_r >= g.M ? (int)(g.M - EA - m0) : a_r;
+        const int bc = B_N && n0 + b_c >= g.N ? (int)(g.N - EB - n0) : b_c;
+        ao[0] = (ar >= 0 ? rowA[ar] : rowA[0] - (OFF)(-ar * 8)) + (OFF)(a_k * sa * 8);
+        bo[0] = (bc >= 0 ? colB[bc] : colB[0] - (OFF)(-bc * 8)) + (OFF)(b_k * sb * 8);
+    } else {
 #pragma unroll
-        for (int e = 0; e < GM_EA; ++e)
-            As[buf][a_k + e][a_row] = ra[e];
+        for (int e = 0; e < NA; ++e)
+            ao[e] = A_M ? rowA[a_r] + (REG ? (OFF)((a_k + KSA * e) * sa * 8) : 0)
+                        : rowA[a_r + 16 * e] + (REG ? (OFF)(a_k * sa * 8) : 0);
 #pragma unroll
-        for (int e = 0; e < GM_EB; ++e)
-            Bs[buf][b_k][b_col + e] = rb[e];
+        for (int e = 0; e < NB; ++e)
+            bo[e] = B_N ? colB[b_c] + (REG ? (OFF)((b_k + KSB * e) * sb * 8) : 0)
+                        : colB[b_c + 16 * e] + (REG ? (OFF)(b_k * sb * 8) : 0);
+    }
+    double ra[EA], rb[EB];
+    // REG: where the turn to load next begins, and how many turns are left in the innermost dimension
+    const __amdgpu_buffer_rsrc_t Ab = gett_buffer(A), Bb = gett_buffer(B);
+    uint32_t At = 0, Bt = 0, k_next = k_begin, run = 0, outer = 0;
+
+    const auto load_tiles = [&](int t) {
+        const uint32_t left = k_end - k_begin - (uint32_t)t * GM_BK;
+        if constexpr (REG) {
+            if (run == 0) {
+                if (t > 0 && last == 1) {          // two dimensions: the next of the outer one, no divisions
+                    outer += 1;
+                    At = outer * (uint32_t)(g.k.s0[0] * 8);
+                    Bt = outer * (uint32_t)(g.k.s1[0] * 8);
+                    run = g.k.ext[1] / GM_BK;
+                } else {
+                    int64_t oa, ob;
+                    gett_offsets(g.k, k_next, &oa, &ob);
+                    At = (uint32_t)(oa * 8);
+                    Bt = (uint32_t)(ob * 8);
+                    outer = k_next / g.k.ext[last];
+                    run = last > 0 ? (g.k.ext[last] - k_next % g.k.ext[last]) / GM_BK : ~0u;
+                }
+            }
+            if constexpr (RUN) {          // whole turns only
+#pragma unroll
+                for (int e = 0; e < EA; e += 2) {
+                    const double2_t v = gett_fetch2(Ab, ao[0] + e * 8, At);
+                    ra[e] = v.x;
+                    ra[e + 1] = v.y;
+                }
+#pragma unroll
+                for (int e = 0; e < EB; e += 2) {
+                    const double2_t v = gett_fetch2(Bb, bo[0] + e * 8, Bt);
+                    rb[e] = v.x;
+                    rb[e + 1] = v.y;
+                }
+            } else if (left >= GM_BK) {
+#pragma unroll
+                for (int e = 0; e < EA; ++e)
+                    ra[e] = gett_fetch(Ab, ao[e], At);
+#pragma unroll
+                for (int e = 0; e < EB; ++e)
+                    rb[e] = gett_fetch(Bb, bo[e], Bt);
+            } else {          // the last turn: k beyond the end read the last k and count as zero
+#pragma unroll
+                for (int e = 0; e < EA; ++e) {
+                    const int k = A_M ? a_k + KSA * e : a_k, over = k < (int)left ? 0 : k - (int)left + 1;
+                    ra[e] = gett_fetch(Ab, (uint32_t)(ao[e] - (OFF)(over * sa * 8)), At);
+                    ra[e] = over ? 0.0 : ra[e];
+                }
+#pragma unroll
+                for (int e = 0; e < EB; ++e) {
+                    const int k = B_N ? b_k + KSB * e : b_k, over = k < (int)left ? 0 : k - (int)left + 1;
+                    rb[e] = gett_fetch(Bb, (uint32_t)(bo[e] - (OFF)(over * sb * 8)), Bt);
+                    rb[e] = over ? 0.0 : rb[e];
+                }
+            }
+            At += (uint32_t)(GM_BK * 8 * sa);
+            Bt += (uint32_t)(GM_BK * 8 * sb);
+            k_next += GM_BK;
+            --run;
+        } else {
+            const OFF *ka = kA[t & 1], *kb = kB[t & 1];
+#pragma unroll
+            for (int e = 0; e < EA; ++e)
+                ra[e] = gett_load(A, (OFF)(A_M ? ao[0] + ka[a_k + KSA * e] : ao[A_M ? 0 : e] + ka[a_k]));
+#pragma unroll
+            for (int e = 0; e < EB; ++e)
+                rb[e] = gett_load(B, (OFF)(B_N ? bo[0] + kb[b_k + KSB * e] : bo[B_N ? 0 : e] + kb[b_k]));
+            if (left < GM_BK) {
+#pragma unroll
+                for (int e = 0; e < EA; ++e)
+                    ra[e] = (uint32_t)(A_M ? a_k + KSA * e : a_k) < left ? ra[e] : 0.0;
+#pragma unroll
+                for (int e = 0; e < EB; ++e)
+                    rb[e] = (uint32_t)(B_N ? b_k + KSB * e : b_k) < left ? rb[e] : 0.0;
+            }
+        }
+    };
+    const auto store_tiles = [&](int buf) {
+        if constexpr (RUN) {
+#pragma unroll
+            for (int e = 0; e < EA; ++e)
+                As[buf][A_M ? a_k : a_k + e][A_M ? a_r + e : a_r] = ra[e];
+#pragma unroll
+            for (int e = 0; e < EB; ++e)
+                Bs[buf][B_N ? b_k : b_k + e][B_N ? b_c + e : b_c] = rb[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < EA; ++e)
+                As[buf][A_M ? a_k + KSA * e : a_k][A_M ? a_r : a_r + 16 * e] = ra[e];
+#pragma unroll
+            for (int e = 0; e < EB; ++e)
+                Bs[buf][B_N ? b_k + KSB * e : b_k][B_N ? b_c : b_c + 16 * e] = rb[e];
+        }
     };
 
-    double4_t acc[4][4];
+    double4_t acc[TM][TN];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < TN; ++j)
             acc[i][j] = (double4_t){0.0, 0.0, 0.0, 0.0};
 
-    const int64_t nk = (K + GM_BK - 1) / GM_BK;
     load_tiles(0);
     store_tiles(0);
     __syncthreads();
     const int fr = lane & 15, fk = lane >> 4;
-    for (int64_t kt = 0; kt < nk; ++kt) {
-        const int cur = (int)(kt & 1);
-        if (kt + 1 < nk)
-            load_tiles((kt + 1) * GM_BK);
+    for (int t = 0; t < nt; ++t) {
+        const int cur = t & 1;
+        double af[2][TM], bf[2][TN];
+        const auto fragments = [&](int ks) {          // the operands of the MFMAs of k ks .. ks + 3
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                af[ks / 4 & 1][i] = As[cur][ks + fk][wm * (TM * 16) + i * 16 + fr];
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                bf[ks / 4 & 1][j] = Bs[cur][ks + fk][wn * (TN * 16) + j * 16 + fr];
+        };
+        fragments(0);
+        if (t + 1 < nt)
+            load_tiles(t + 1);
+        if (!REG && t + 2 < nt)
+            k_offsets(t + 2);           // the slot turn t was loaded through
 #pragma unroll
         for (int ks = 0; ks < GM_BK; ks += 4) {
-            double af[4], bf[4];
+            if (ks + 4 < GM_BK)
+                fragments(ks + 4);
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                af[i] = As[cur][ks + fk][wm * 64 + i * 16 + fr];
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                bf[j] = Bs[cur][ks + fk][wn * 64 + j * 16 + fr];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bf[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < TN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[ks / 4 & 1][i], bf[ks / 4 & 1][j], acc[i][j], 0, 0, 0);
         }
-        if (kt + 1 < nk)
+        if (t + 1 < nt)
             store_tiles(cur ^ 1);
         __syncthreads();
     }
 
+    const bool whole = gridDim.y == 1, inside = m0 + BM <= g.M && n0 + BN <= g.N;
+    double *out = whole ? C : partial + (uint64_t)blockIdx.y * g.M * g.N;
+    int64_t cols[TN];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < TN; ++j) {
+        const int c = wn * (TN * 16) + j * 16 + fr;
+        cols[j] = whole ? colC[c] : (int64_t)(n0 + c);
+    }
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int64_t gm = m0 + wm * 64 + i * 16 + 4 * v + fk;
-                const int64_t gn = n0 + wn * 64 + j * 16 + fr;
-                if (!GUARD || (gm < M && gn < N)) {
-                    double r = acc[i][j][v];
-                    if (use_c)
-                        r = C[gm * N + gn] + r;
-                    C[gm * N + gn] = r;
-                }
+        for (int v = 0; v < 4; ++v) {
+            const int r = wm * (TM * 16) + i * 16 + 4 * v + fk;
+            double *row = out + (whole ? rowC[r] : (int64_t)(m0 + r) * g.N);
+            if (inside) {
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    row[cols[j]] = whole && use_c ? row[cols[j]] + acc[i][j][v] : acc[i][j][v];
+            } else if (m0 + r < g.M) {
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    if (n0 + wn * (TN * 16) + j * 16 + fr < g.N)
+                        row[cols[j]] = whole && use_c ? row[cols[j]] + acc[i][j][v] : acc[i][j][v];
             }
+        }
 }
 
+// C[m,n] (+)= the partial tiles in order of their k.  `group` threads of a workgroup share an output: each adds
+// every group-th partial, then the first adds what the others have.
+__global__ __launch_bounds__(256) void gett_reduce(GettArgs g, int splits, int group, const double *__restrict__ partial,
+                                                   double *__restrict__ C, int use_c)
+{
+    __shared__ double lds[256];
+    const int per = 256 / group, o = threadIdx.x % per, share = threadIdx.x / per;
+    const uint64_t total = (uint64_t)g.M * g.N, i = (uint64_t)blockIdx.x * per + o;
+    double s = 0.0;
+    if (i < total) {
+        int z = share;
+        for (; z + 3 * group < splits; z += 4 * group) {
+            const double p0 = partial[(uint64_t)z * total + i], p1 = partial[(uint64_t)(z + group) * total + i],
+                         p2 = partial[(uint64_t)(z + 2 * group) * total + i],
+                         p3 = partial[(uint64_t)(z + 3 * group) * total + i];
+            s = s + p0;
+            s = s + p1;
+            s = s + p2;
+            s = s + p3;
+        }
+        for (; z < splits; z += group)
+            s = s + partial[(uint64_t)z * total + i];
+    }
+    lds[threadIdx.x] = s;
+    __syncthreads();
+    if (share != 0 || i >= total)
+        return;
+    for (int q = 1; q < group; ++q)
+        s = s + lds[q * per + o];
+    int64_t ma, mc, nb, nc;
+    gett_offsets(g.m, (uint32_t)(i / g.N), &ma, &mc);
+    gett_offsets(g.n, (uint32_t)(i % g.N), &nb, &nc);
+    C[mc + nc] = use_c ? C[mc + nc] + s : s;
+}
+
+// The tile shapes: workgroups a CU holds, the time of a turn of 16 k divided by them on a full CU, and the time of a
+// turn of a workgroup that has its CU to itself (measured, us; 4096^3 takes 1908 / 2125 / 2440 / 3109 us with the four
+// shapes, the first at 92 % of the matrix cores' rate).  The launch takes the shape and the number of shares of k that
+// these figures make cheapest: small tiles and many shares where the outputs are few, the large tile where they are
+// not, and the narrow ones where one side of C is short.
+struct GettShape {
+    int bm, bn, resident;
+    double turn_us, alone_us;
+};
+constexpr GettShape GETT_SHAPES[] = {{128, 128, 2, 1.86, 2.65}, {64, 64, 4, 0.52, 1.2}, {64, 32, 6, 0.30, 0.71}, {128, 16, 4, 0.38, 0.83}};
+constexpr int GETT_NSHAPES = sizeof(GETT_SHAPES) / sizeof(GETT_SHAPES[0]);
+
+static Workspace g_gett_partial;
+
+template <int BM, int BN, int WM, int OCC, bool REG, bool RUN, typename OFF>
+static void gett_launch(bool a_m, bool b_n, dim3 grid, const GettArgs &g, const double *A, const double *B, double *C,
+                        double *partial, int use_c)
+{
+    const dim3 block(256);
+    if (a_m && b_n)
+        gett_mfma_kernel<BM, BN, WM, OCC, true, true, REG, RUN, OFF><<<grid, block, 0, stream()>>>(g, A, B, C, partial, use_c);
+    else if (a_m)
+        gett_mfma_kernel<BM, BN, WM, OCC, true, false, REG, RUN, OFF><<<grid, block, 0, stream()>>>(g, A, B, C, partial, use_c);
+    else if (b_n)
+        gett_mfma_kernel<BM, BN, WM, OCC, false, true, REG, RUN, OFF><<<grid, block, 0, stream()>>>(g, A, B, C, partial, use_c);
+    else
+        gett_mfma_kernel<BM, BN, WM, OCC, false, false, REG, RUN, OFF><<<grid, block, 0, stream()>>>(g, A, B, C, partial, use_c);
+}
+
+// The innermost dimension of an index comes last: `first` names the tensor (0 or 1) whose contiguous dimension it
+// should be, if that dimension is in the index.  Dimensions that follow each other in both tensors are merged.
+static bool gett_order(GettIndex *g, int first)
+{
+    GettIndex in = *g;
+    int last = -1;
+    for (int pass = 0; pass < 2 && last < 0; ++pass)
+        for (int d = 0; d < in.nd; ++d)
+            if (((pass == 0) == (first == 0) ? in.s0[d] : in.s1[d]) == 1)
+                last = d;
+    if (last < 0)
+        last = in.nd - 1;
+    const bool contiguous = in.nd > 0 && (first == 0 ? in.s0[last] : in.s1[last]) == 1;
+    // from the innermost outwards: first whatever continues the dimension before it in the tensor `first`
+    std::vector<int> order(1, last), rest;
+    for (int d = 0; d < in.nd; ++d)
+        if (d != last)
+            rest.push_back(d);
+    const int64_t *key = first == 0 ? in.s0 : in.s1;
+    std::sort(rest.begin(), rest.end(), [&](int x, int y) { return key[x] < key[y]; });
+    order.insert(order.end(), rest.begin(), rest.end());
+    g->nd = 0;
+    uint32_t ext[TR_MAXRANK];
+    int64_t s0[TR_MAXRANK], s1[TR_MAXRANK];
+    int n = 0;
+    for (int d : order) {
+        if (n > 0 && s0[n - 1] * ext[n - 1] == in.s0[d] && s1[n - 1] * ext[n - 1] == in.s1[d]) {
+            ext[n - 1] *= in.ext[d];
+        } else {
+            ext[n] = in.ext[d];
+            s0[n] = in.s0[d];
+            s1[n] = in.s1[d];
+            ++n;
+        }
+    }
+    g->nd = n;
+    for (int d = 0; d < n; ++d) {          // outermost first
+        g->ext[d] = ext[n - 1 - d];
+        g->s0[d] = s0[n - 1 - d];
+        g->s1[d] = s1[n - 1 - d];
+    }
+    return contiguous;
+}
+
+static void gett_add_dim(GettIndex *g, int64_t ext, int64_t s0, int64_t s1)
+{
+    if (ext == 1)
+        return;
+    g->ext[g->nd] = (uint32_t)ext;
+    g->s0[g->nd] = s0;
+    g->s1[g->nd] = s1;
+    ++g->nd;
+}
+
+// C (+)= A * B over the three indices; span: one more than the largest offset into any of the tensors.
+static int gett_device(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t N, int64_t K, int64_t span,
+                       const double *A, const double *B, double *C, double beta)
+{
+    if (M == 0 || N == 0)
+        return COMET_HIP_OK;
+    if (K == 0) {               // empty sums; C is whole and contiguous
+        if (beta == 0.0)
+            COMET_HIPCHK(hipMemsetAsync(C, 0, sizeof(double) * (size_t)(M * N), stream()));
+        return COMET_HIP_OK;
+    }
+    if (M >= (1ll << 31) || N >= (1ll << 31) || K >= (1ll << 31))
+        return set_error(COMET_HIP_ERR_SIZE, "contraction of %lld x %lld x %lld: an index exceeds 31 bits", (long long)M,
+                         (long long)N, (long long)K);
+    const auto unit_in_c = [](const GettIndex &g) {
+        for (int d = 0; d < g.nd; ++d)
+            if (g.s1[d] == 1)
+                return true;
+        return false;
+    };
+    // Which operand gives the columns: the shorter side when it is short enough for a narrow tile, else the one whose
+    // index is contiguous in C, so that sixteen lanes store sixteen neighbours.
+    const int64_t shorter = M < N ? M : N;
+    const bool swap = shorter <= 32 ? M < N : unit_in_c(m) && !unit_in_c(n);
+    if (swap) {
+        std::swap(m, n);
+        std::swap(M, N);
+        std::swap(A, B);
+        std::swap(k.s0, k.s1);
+    }
+    GettArgs g;
+    const bool a_m = gett_order(&m, 0);
+    const bool b_n = gett_order(&n, 0);
+    if (!a_m)
+        (void)gett_order(&m, 1);
+    if (!b_n)
+        (void)gett_order(&n, 1);
+    (void)gett_order(&k, a_m ? 1 : 0);
+    for (GettIndex *x : {&m, &n, &k})
+        if (x->nd == 0) {          // an index of one element
+            x->nd = 1;
+            x->ext[0] = 1;
+            x->s0[0] = x->s1[0] = 0;
+        }
+    g.m = m;
+    g.n = n;
+    g.k = k;
+    g.M = (uint32_t)M;
+    g.N = (uint32_t)N;
+    g.K = (uint32_t)K;
+    const int64_t nk = ceil_div(K, GM_BK);
+    const int64_t cus = num_cus() > 0 ? num_cus() : 256;
+    const bool wide = span >= (1ll << 29);          // byte offsets beyond 32 bits
+    int best = 0;
+    int64_t splits = 1;
+    double best_us = 0.0;
+    for (int c = 0; c < (wide ? 1 : GETT_NSHAPES); ++c) {
+        const GettShape &sh = GETT_SHAPES[c];
+        const int64_t tiles = ceil_div(M, sh.bm) * ceil_div(N, sh.bn);
+        for (int64_t s = 1; s <= nk && s <= 1024; s *= 2) {
+            const int64_t turns = ceil_div(nk, s), groups = tiles * ceil_div(nk, turns);
+            const int64_t rounds = ceil_div(groups, cus * sh.resident);
+            const double per_cu = (double)std::min<int64_t>(sh.resident, ceil_div(groups, cus));
+            const double turn = std::max(sh.alone_us, per_cu * sh.turn_us);
+            const double us = (double)rounds * ((double)turns * turn + 2.5) +
+                              (s > 1 ? 3.0 + (double)ceil_div(nk, turns) * (double)(M * N) * 16.0 / 3.0e6 : 0.0);
+            if (best_us == 0.0 || us < best_us) {
+                best_us = us;
+                best = c;
+                splits = ceil_div(nk, turns);
+                g.turns = (uint32_t)turns;
+            }
+        }
+    }
+    // COMET_HIP_GETT="shape,shares of k" overrides the choice (every shape is right for every product: the tests send
+    // the same one through all of them)
+    if (const char *e = getenv("COMET_HIP_GETT")) {
+        long long c = 0, s = 1;
+        if (sscanf(e, "%lld,%lld", &c, &s) == 2 && c >= 0 && c < (wide ? 1 : GETT_NSHAPES) && s >= 1 && s <= nk && s < 65536) {
+            best = (int)c;
+            g.turns = (uint32_t)ceil_div(nk, s);
+            splits = ceil_div(nk, (int64_t)g.turns);
+        }
+    }
+    const GettShape &sh = GETT_SHAPES[best];
+    const int64_t tiles = ceil_div(M, sh.bm) * ceil_div(N, sh.bn);
+    if (tiles > INT32_MAX)
+        return set_error(COMET_HIP_ERR_SIZE, "contraction of %lld x %lld outputs exceeds the launch grid", (long long)M,
+                         (long long)N);
+    double *partial = nullptr;
+    if (splits > 1) {
+        COMET_CHK(g_gett_partial.ensure(sizeof(double) * (size_t)splits * (size_t)M * (size_t)N, false));
+        partial = (double *)g_gett_partial.ptr;
+    }
+    const dim3 grid((unsigned)tiles, (unsigned)splits);
+    const int use_c = beta != 0.0;
+    {
+        KernelTimer t("gett_mfma_kernel");
+        const bool reg = k.nd == 1 || k.ext[k.nd - 1] % GM_BK == 0;
+        // sixteen bytes at a time: a thread's run along the contiguous index is unbroken and aligned
+        const auto runs = [](const GettIndex &x, const int64_t *s, bool along, int run) {
+            for (int d = 0; d < x.nd; ++d)
+                if (along && d == x.nd - 1 ? x.ext[d] % run != 0 || s[d] != 1 : s[d] % 2 != 0)
+                    return false;
+            return true;
+        };
+        const int ra = a_m ? sh.bm / 16 : 2, rb = b_n ? sh.bn / 16 : 2;
+        const bool pairs = reg && K % GM_BK == 0 && sh.bn >= 64 && (((uintptr_t)A | (uintptr_t)B) & 15) == 0 &&
+                           runs(m, m.s0, a_m, ra) && runs(k, k.s0, !a_m, 2) && runs(n, n.s0, b_n, rb) &&
+                           runs(k, k.s1, !b_n, 2);
+        const auto launch = [&](auto kernel_shape, auto wave_rows, auto occ) {
+            constexpr GettShape S = GETT_SHAPES[decltype(kernel_shape)::value];
+            constexpr int WM = decltype(wave_rows)::value, OCC = decltype(occ)::value;
+            if (pairs)
+                gett_launch<S.bm, S.bn >= 64 ? S.bn : 64, WM, OCC, true, true, uint32_t>(a_m, b_n, grid, g, A, B, C, partial, use_c);
+            else if (reg)
+                gett_launch<S.bm, S.bn, WM, OCC, true, false, uint32_t>(a_m, b_n, grid, g, A, B, C, partial, use_c);
+            else
+                gett_launch<S.bm, S.bn, WM, OCC, false, false, uint32_t>(a_m, b_n, grid, g, A, B, C, partial, use_c);
+        };
+        using std::integral_constant;
+        if (wide)
+            gett_launch<128, 128, 2, COMET_GM_OCC, false, false, int64_t>(a_m, b_n, grid, g, A, B, C, partial, use_c);
+        else if (best == 0)
+            launch(integral_constant<int, 0>(), integral_constant<int, 2>(), integral_constant<int, COMET_GM_OCC>());
+        else if (best == 1)
+            launch(integral_constant<int, 1>(), integral_constant<int, 2>(), integral_constant<int, 4>());
+        else if (best == 2)
+            launch(integral_constant<int, 2>(), integral_constant<int, 2>(), integral_constant<int, 4>());
+        else
+            launch(integral_constant<int, 3>(), integral_constant<int, 4>(), integral_constant<int, 4>());
+    }
+    if (splits > 1) {
+        int group = 1;
+        while (group < 16 && group * 8 <= splits)
+            group *= 2;
+        KernelTimer t("gett_reduce");
+        gett_reduce<<<dim3((unsigned)ceil_div(M * N, 256 / group)), dim3(256), 0, stream()>>>(g, (int)splits, group,
+                                                                                             partial, C, use_c);
+    }
+    COMET_HIPCHK(hipGetLastError());
+    return COMET_HIP_OK;
+}
+
+// Row-major C[M,N] = beta*C + A[M,K]*B[K,N].
 static int dgemm_device(int64_t M, int64_t N, int64_t K, const double *A, const double *B, double *C, double beta)
 {
     if (M < 0 || N < 0 || K < 0)
         return set_error(COMET_HIP_ERR_ARG, "negative GEMM size");
     if (beta != 0.0 && beta != 1.0)
         return set_error(COMET_HIP_ERR_ARG, "beta must be 0 or 1 (got %g)", beta);
-    if (M == 0 || N == 0)
-        return COMET_HIP_OK;
-    const int64_t gx = ceil_div(N, GM_BN), gy = ceil_div(M, GM_BM);
-    if (gy > 65535)
-        return set_error(COMET_HIP_ERR_SIZE, "M = %lld too large for the launch grid", (long long)M);
-    const bool aligned = (M % GM_BM == 0) && (N % GM_BN == 0) && (K % GM_BK == 0) && K > 0;
-    KernelTimer t("dgemm_mfma_kernel");
-    if (aligned)
-        dgemm_mfma_kernel<false><<<dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, stream()>>>(M, N, K, A, B, C,
-                                                                                             beta != 0.0);
-    else
-        dgemm_mfma_kernel<true><<<dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, stream()>>>(M, N, K, A, B, C,
-                                                                                            beta != 0.0);
-    COMET_HIPCHK(hipGetLastError());
-    return COMET_HIP_OK;
+    GettIndex m{}, n{}, k{};
+    gett_add_dim(&m, M, K, N);
+    gett_add_dim(&n, N, 1, 1);
+    gett_add_dim(&k, K, 1, N);
+    return gett_device(m, n, k, M, N, K, std::max(M * K, std::max(K * N, M * N)), A, B, C, beta);
 }
 
 // ============================================================================
@@ -473,6 +923,140 @@ static int make_plan(int32_t rankA, const int32_t *a_lab, int32_t rankB, const i
 }
 
 static Workspace g_tt_a, g_tt_b, g_tt_c;
+
+// The dimension of a tensor that the plan puts at position i of its matrix form.
+static int plan_dim(int32_t trans, const int32_t *perm, int i) { return trans ? perm[i] : i; }
+
+// Position of the first m, n and k dimension in the plan's forms of A, B and C (swapAB: A = [k m], B = [n k], C = [n m],
+// else A = [m k], B = [k n], C = [m n]), and whether the forms agree dimension by dimension.
+struct PlanDims {
+    int nm, nn, nk;
+    int am, ak, bn, bk, cm, cn;
+};
+static PlanDims plan_dims(const comet_ttgt_plan &p)
+{
+    PlanDims d;
+    d.nk = (p.rankA + p.rankB - p.rankC) / 2;
+    d.nm = p.rankA - d.nk;
+    d.nn = p.rankB - d.nk;
+    d.am = p.swapAB ? d.nk : 0;
+    d.ak = p.swapAB ? 0 : d.nm;
+    d.bn = p.swapAB ? 0 : d.nk;
+    d.bk = p.swapAB ? d.nn : 0;
+    d.cm = p.swapAB ? d.nn : 0;
+    d.cn = p.swapAB ? 0 : d.nm;
+    return d;
+}
+
+static bool gett_fits(const comet_ttgt_plan &p, const int64_t *a_shape, const int64_t *b_shape, const int64_t *c_shape)
+{
+    if ((p.rankA + p.rankB - p.rankC) % 2 != 0)
+        return false;
+    const PlanDims d = plan_dims(p);
+    if (d.nk < 0 || d.nm < 0 || d.nn < 0 || d.nm + d.nn != p.rankC)
+        return false;
+    const auto a = [&](int i) { return a_shape[plan_dim(p.transA, p.permA, i)]; };
+    const auto b = [&](int i) { return b_shape[plan_dim(p.transB, p.permB, i)]; };
+    const auto c = [&](int i) { return c_shape[plan_dim(p.transC, p.permC, i)]; };
+    int64_t M = 1, N = 1, K = 1;
+    for (int i = 0; i < d.nm; ++i) {
+        if (a(d.am + i) != c(d.cm + i))
+            return false;
+        M *= a(d.am + i);
+    }
+    for (int i = 0; i < d.nn; ++i) {
+        if (b(d.bn + i) != c(d.cn + i))
+            return false;
+        N *= b(d.bn + i);
+    }
+    for (int i = 0; i < d.nk; ++i) {
+        if (a(d.ak + i) != b(d.bk + i))
+            return false;
+        K *= a(d.ak + i);
+    }
+    return M == p.M && N == p.N && K == p.K && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31);
+}
+
+constexpr double GETT_TURN_MIN = 1.28e8;
+
+static int contract_strided(const comet_ttgt_plan &p, const int64_t *a_shape, const int64_t *b_shape,
+                            const int64_t *c_shape, const double *A, const double *B, double *C, double beta)
+{
+    const auto strides = [](const int64_t *shape, int rank, int64_t *out) {
+        int64_t s = 1;
+        for (int i = rank - 1; i >= 0; --i) {
+            out[i] = s;
+            s *= shape[i];
+        }
+        return s;
+    };
+    int64_t sa[8], sb[8], sc[8];
+    const int64_t span = std::max(strides(a_shape, p.rankA, sa),
+                                  std::max(strides(b_shape, p.rankB, sb), strides(c_shape, p.rankC, sc)));
+    const PlanDims d = plan_dims(p);
+    GettIndex m{}, n{}, k{};
+    const auto da = [&](int i) { return plan_dim(p.transA, p.permA, i); };
+    const auto db = [&](int i) { return plan_dim(p.transB, p.permB, i); };
+    const auto dc = [&](int i) { return plan_dim(p.transC, p.permC, i); };
+    for (int i = 0; i < d.nm; ++i)
+        gett_add_dim(&m, a_shape[da(d.am + i)], sa[da(d.am + i)], sc[dc(d.cm + i)]);
+    for (int i = 0; i < d.nn; ++i)
+        gett_add_dim(&n, b_shape[db(d.bn + i)], sb[db(d.bn + i)], sc[dc(d.cn + i)]);
+    for (int i = 0; i < d.nk; ++i)
+        gett_add_dim(&k, a_shape[da(d.ak + i)], sa[da(d.ak + i)], sb[db(d.bk + i)]);
+    // Both operands contiguous along k, but along different dimensions of it: whatever order k is taken in, one of
+    // them is read a cache line per element.  The smaller one is turned first: k outermost, in the other's order, and
+    // its outer index as C has it - the layout the kernel is fastest with.  Below GETT_TURN_MIN products the turn
+    // costs more than the scattered reads (323 x 396 x 483: 21 us without, 23 with; 1520 x 1716 x 1435: 830 and 216).
+    int ua = -1, ub = -1;
+    for (int i = 0; i < k.nd; ++i) {
+        ua = k.s0[i] == 1 ? i : ua;
+        ub = k.s1[i] == 1 ? i : ub;
+    }
+    if (ua >= 0 && ub >= 0 && ua != ub && (double)p.M * (double)p.N * (double)p.K >= GETT_TURN_MIN) {
+        const bool turn_a = p.M < p.N;
+        const int rank = turn_a ? p.rankA : p.rankB, nfree = turn_a ? d.nm : d.nn;
+        const int64_t *shape = turn_a ? a_shape : b_shape;
+        int32_t perm[8];
+        int64_t other[8];
+        std::vector<std::pair<int64_t, int32_t>> ks;          // (minus the stride in the other operand, dimension)
+        for (int i = 0; i < d.nk; ++i) {
+            const int32_t mine = turn_a ? da(d.ak + i) : db(d.bk + i);
+            ks.emplace_back(-(turn_a ? sb[db(d.bk + i)] : sa[da(d.ak + i)]), mine);
+        }
+        std::stable_sort(ks.begin(), ks.end());
+        std::vector<std::pair<int64_t, int32_t>> fs;
+        for (int i = 0; i < nfree; ++i) {
+            const int32_t mine = turn_a ? da(d.am + i) : db(d.bn + i);
+            fs.emplace_back(-(turn_a ? sc[dc(d.cm + i)] : sc[dc(d.cn + i)]), mine);
+        }
+        std::stable_sort(fs.begin(), fs.end());
+        int at = 0;
+        for (auto &e : ks)
+            perm[at++] = e.second;
+        for (auto &e : fs)
+            perm[at++] = e.second;
+        for (int i = 0; i < rank; ++i)
+            other[i] = shape[perm[i]];
+        Workspace &w = turn_a ? g_tt_a : g_tt_b;
+        COMET_CHK(w.ensure(sizeof(double) * (size_t)((turn_a ? p.M : p.N) * p.K), false));
+        COMET_CHK(transpose_device(rank, shape, perm, turn_a ? A : B, (double *)w.ptr));
+        int64_t st[8];
+        (void)strides(other, rank, st);
+        int64_t *s_mine = turn_a ? sa : sb;
+        for (int i = 0; i < rank; ++i)
+            s_mine[perm[i]] = st[i];
+        (turn_a ? A : B) = (const double *)w.ptr;
+        m = n = k = GettIndex{};
+        for (int i = 0; i < d.nm; ++i)
+            gett_add_dim(&m, a_shape[da(d.am + i)], sa[da(d.am + i)], sc[dc(d.cm + i)]);
+        for (int i = 0; i < d.nn; ++i)
+            gett_add_dim(&n, b_shape[db(d.bn + i)], sb[db(d.bn + i)], sc[dc(d.cn + i)]);
+        for (int i = 0; i < d.nk; ++i)
+            gett_add_dim(&k, a_shape[da(d.ak + i)], sa[da(d.ak + i)], sb[db(d.bk + i)]);
+    }
+    return gett_device(m, n, k, p.M, p.N, p.K, span, A, B, C, beta);
+}
 
 }  // namespace comet
 
@@ -596,6 +1180,9 @@ extern "C" int comet_hip_ttgt_contract(const comet_ttgt_plan *plan, const int64_
                          (long long)M, (long long)N, (long long)K);
     const double *A = (const double *)a_dptr, *B = (const double *)b_dptr;
     double *C = (double *)c_dptr;
+    if (gett_fits(*plan, a_shape, b_shape, c_shape))
+        return contract_strided(*plan, a_shape, b_shape, c_shape, A, B, C, beta);
+    // a plan whose transposed tensors do not share their dimensions one by one: as matrices, after transposes
     const double *Ause = A, *Buse = B;
     double *Cuse = C;
     if (plan->transA) {

@@ -29,3 +29,33 @@ def test_freed_blocks_come_back_only_when_nothing_uses_them(nbytes):
     b.free()
     assert rt.lib().comet_hip_free(old) != 0          # a second time
     assert np.array_equal(c.to_numpy(), twos)
+
+
+EXTENTS = [dict(a=5, b=7, c=3, d=11, e=16, f=2), dict(a=1, b=1, c=129, d=1, e=17, f=1), dict(a=8, b=16, c=8, d=17, e=16, f=3),
+           dict(a=16, b=9, c=32, d=4, e=32, f=16), dict(a=2, b=64, c=4, d=32, e=15, f=1), dict(a=3, b=43, c=1, d=1, e=7, f=31)]
+
+
+@pytest.mark.parametrize("forced", [None, "0,1", "1,1", "2,1", "3,1", "0,3", "1,2", "2,5", "3,4"])
+@pytest.mark.parametrize("a,b,c", [("ef", "fc", "ec"), ("aebf", "dfce", "abcd"), ("aebf", "efcd", "abcd"), ("eabf", "cdfe", "cdab"),
+                                   ("feab", "efcd", "dcba"), ("abef", "ef", "ab"), ("ab", "cd", "acbd")])
+def test_contraction_every_tile_shape_and_layout(a, b, c, forced, monkeypatch):
+    for i, extent in enumerate(EXTENTS):
+        rng = np.random.default_rng(i)
+        A, B = (rng.uniform(-1, 1, [extent[x] for x in lab]) for lab in (a, b))
+        C0 = rng.uniform(-1, 1, [extent[x] for x in c])
+        want, bound = (np.einsum(f"{a},{b}->{c}", f(A), f(B)) for f in (np.array, np.abs))
+        if forced:
+            monkeypatch.setenv("COMET_HIP_GETT", forced)
+        for beta in (0.0, 1.0):
+            dC = rt.DeviceArray.from_numpy(C0)
+            rt.ttgt_contract(a, b, c, rt.DeviceArray.from_numpy(A), rt.DeviceArray.from_numpy(B), dC, beta=beta)
+            assert np.all(np.abs(dC.to_numpy() - want - beta * C0) <= 1e-13 * (bound + 1.0)), (extent, beta)
+
+
+@pytest.mark.parametrize("extent", [dict(a=24, b=23, c=22, d=21, e=25, f=26), dict(a=32, b=16, c=32, d=17, e=32, f=16)])
+def test_contraction_with_a_turned_operand(extent):
+    rng = np.random.default_rng(7)
+    A, B = (rng.uniform(-1, 1, [extent[x] for x in lab]) for lab in ("aebf", "dfce"))
+    C, _ = rt.ttgt_contract("aebf", "dfce", "abcd", rt.DeviceArray.from_numpy(A), rt.DeviceArray.from_numpy(B))
+    want = np.tensordot(A, B, axes=([1, 3], [3, 1])).transpose(0, 1, 3, 2)
+    assert np.abs(C.to_numpy() - want).max() <= 1e-11
