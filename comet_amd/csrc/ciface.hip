@@ -8,6 +8,9 @@
 #include <stdio.h>
 #include <stdlib.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "common.h"
 
 using namespace comet;
@@ -52,13 +55,24 @@ void comet::forget_pending_product() { g_pending_c = 0; }
 namespace {
 
 template <typename I>
-int64_t upload(int64_t nrows, int64_t ncols, const I *pos, const I *crd, const double *val)
+int64_t upload(int64_t nrows, int64_t ncols, const I *pos, const I *crd, const double *val, std::vector<Piece> more = {})
 {
-    if constexpr (sizeof(I) == 8)
-        return comet_hip_csr_upload_i64(nrows, ncols, (const int64_t *)pos, (const int64_t *)crd, val);
-    else
-        return comet_hip_csr_upload_i32(nrows, ncols, (const int32_t *)pos, (const int32_t *)crd, val);
+    using W = typename std::conditional<sizeof(I) == 8, int64_t, int32_t>::type;
+    Csr *c = ensure_init() == COMET_HIP_OK
+                 ? csr_from_host(nrows, ncols, (const W *)pos, (const W *)crd, val, std::move(more))
+                 : nullptr;
+    return c ? csr_register(c) : 0;
 }
+
+// an operand of a call: room on the device, and its copies up and down
+struct DeviceOperand : DeviceBuf {
+    double *host;
+    size_t bytes;
+    DeviceOperand(double *h, int64_t elems) : DeviceBuf(elems * 8), host(h), bytes((size_t)elems * 8) {}
+    Piece up() const { return plain_up((void *)p, host, bytes); }
+    Piece down() const { return plain_down(host, (const void *)p, bytes); }
+    bool missing() const { return bytes > 0 && !p; }
+};
 
 template <typename I>
 void spmv_ciface(const char *who, comet_memref_1d *pos, comet_memref_1d *crd, comet_memref_1d *val,
@@ -69,16 +83,11 @@ void spmv_ciface(const char *who, comet_memref_1d *pos, comet_memref_1d *crd, co
         set_error(COMET_HIP_ERR_ARG, "y has %lld entries, A has %lld rows", (long long)y->sizes[0], (long long)nrows);
         die(who);
     }
-    int64_t a = upload<I>(nrows, ncols, data1<I>(pos, who), data1<I>(crd, who), data1<double>(val, who));
-    if (!a)
+    DeviceOperand dx((double *)data1<double>(x, who), ncols), dy((double *)data1<double>(y, who), nrows);
+    if (dx.missing() || dy.missing())
         die(who);
-    DeviceBuf dx(ncols * 8), dy(nrows * 8);
-    if ((ncols && !dx.p) || (nrows && !dy.p))
-        die(who);
-    double *hy = (double *)data1<double>(y, who);
-    if (comet_hip_memcpy(dx.p, (void *)data1<double>(x, who), ncols * 8, 0) ||
-        comet_hip_memcpy(dy.p, hy, nrows * 8, 0) || comet_hip_spmv_csr_f64(a, dx.p, dy.p, 1) ||
-        comet_hip_memcpy(dy.p, hy, nrows * 8, 1))
+    int64_t a = upload<I>(nrows, ncols, data1<I>(pos, who), data1<I>(crd, who), data1<double>(val, who), {dx.up(), dy.up()});
+    if (!a || comet_hip_spmv_csr_f64(a, dx.p, dy.p, 1) || transfer_down({dy.down()}))
         die(who);
     (void)comet_hip_csr_destroy(a);
 }
@@ -97,15 +106,11 @@ void spmm_ciface(const char *who, comet_memref_1d *pos, comet_memref_1d *crd, co
         set_error(COMET_HIP_ERR_ARG, "B/C must be contiguous row-major with matching shapes");
         die(who);
     }
-    int64_t a = upload<I>(nrows, ncols, data1<I>(pos, who), data1<I>(crd, who), data1<double>(val, who));
-    if (!a)
+    DeviceOperand db((double *)B->aligned + B->offset, ncols * K), dc((double *)C->aligned + C->offset, nrows * K);
+    if (db.missing() || dc.missing())
         die(who);
-    DeviceBuf db(ncols * K * 8), dc(nrows * K * 8);
-    if ((ncols * K && !db.p) || (nrows * K && !dc.p))
-        die(who);
-    double *hb = (double *)B->aligned + B->offset, *hc = (double *)C->aligned + C->offset;
-    if (comet_hip_memcpy(db.p, hb, ncols * K * 8, 0) || comet_hip_memcpy(dc.p, hc, nrows * K * 8, 0) ||
-        comet_hip_spmm_csr_f64(a, K, db.p, K, dc.p, K, 1) || comet_hip_memcpy(dc.p, hc, nrows * K * 8, 1))
+    int64_t a = upload<I>(nrows, ncols, data1<I>(pos, who), data1<I>(crd, who), data1<double>(val, who), {db.up(), dc.up()});
+    if (!a || comet_hip_spmm_csr_f64(a, K, db.p, K, dc.p, K, 1) || transfer_down({dc.down()}))
         die(who);
     (void)comet_hip_csr_destroy(a);
 }
@@ -374,14 +379,14 @@ extern "C" void _mlir_ciface_comet_hip_ttgt_contract_f64(int64_t rankA, void *A,
     comet_ttgt_plan plan;
     if (comet_hip_ttgt_plan((int32_t)a.rank, ids[0], (int32_t)b.rank, ids[1], (int32_t)c.rank, ids[2], extent, -1, &plan))
         die(who);
-    DeviceBuf da(a.elems * 8), db(b.elems * 8), dc(c.elems * 8);
-    if ((a.elems && !da.p) || (b.elems && !db.p) || (c.elems && !dc.p))
+    DeviceOperand da(a.data + a.offset, a.elems), db(b.data + b.offset, b.elems), dc(c.data + c.offset, c.elems);
+    if (da.missing() || db.missing() || dc.missing())
         die(who);
-    double *hc = c.data + c.offset;
-    if (comet_hip_memcpy(da.p, a.data + a.offset, a.elems * 8, 0) || comet_hip_memcpy(db.p, b.data + b.offset, b.elems * 8, 0) ||
-        (beta != 0.0 && comet_hip_memcpy(dc.p, hc, c.elems * 8, 0)) ||
-        comet_hip_ttgt_contract(&plan, a.shape, b.shape, c.shape, da.p, db.p, dc.p, beta) ||
-        comet_hip_memcpy(dc.p, hc, c.elems * 8, 1))
+    std::vector<Piece> up = {da.up(), db.up()};
+    if (beta != 0.0)
+        up.push_back(dc.up());
+    if (transfer_up(up) || comet_hip_ttgt_contract(&plan, a.shape, b.shape, c.shape, da.p, db.p, dc.p, beta) ||
+        transfer_down({dc.down()}))
         die(who);
 }
 

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -56,6 +57,23 @@ hipError_t dev_free(void *p);
 void dev_pool_release();
 // waits for stream(); the place where blocks freed before it become free to hand out again
 int stream_wait();
+
+// Copies between the caller's host arrays and the device (transfer.hip).  A piece is n elements of `elem` bytes on the
+// device; host(pinned, first, count) fills the pinned copy of elements [first, first + count) from the caller's array
+// (up) or takes them from it (down), on any of several threads at once.  Both calls are done with the host arrays when
+// they return; the device side of transfer_up is ordered on stream().
+struct Piece {
+    void *dev;
+    size_t n, elem;
+    std::function<void(void *pinned, size_t first, size_t count)> host;
+};
+int transfer_up(const std::vector<Piece> &pieces);
+int transfer_down(const std::vector<Piece> &pieces);
+Piece plain_up(void *dev, const void *host, size_t bytes);
+Piece plain_down(void *host, const void *dev, size_t bytes);
+
+// A word of host memory that kernels write and the host reads after stream_wait (a result without a copy back).
+int mailbox(void **host_word);
 
 // Grow-only device scratch buffer.  `zeroed` buffers are cleared when they are
 // (re)allocated and their users must leave them all-zero on return.
@@ -152,6 +170,11 @@ struct Csr {
     int spmm_uses = 0, spmv_uses = 0;
 };
 
+// host arrays -> a new matrix (checked, registered by the caller), `more` going up in the same transfer; nullptr on failure
+Csr *csr_from_host(int64_t nrows, int64_t ncols, const int64_t *pos, const int64_t *crd, const double *val,
+                   std::vector<Piece> more = {});
+Csr *csr_from_host(int64_t nrows, int64_t ncols, const int32_t *pos, const int32_t *crd, const double *val,
+                   std::vector<Piece> more = {});
 Csr *csr_from_handle(int64_t h, bool allow_poisoned = false);           // nullptr (and error set) if unknown
 int64_t csr_register(Csr *c);              // takes ownership of the struct
 int csr_alloc(Csr *c, int64_t nrows, int64_t ncols, int64_t nnz);   // allocates pos/crd/val, owns = true

@@ -449,22 +449,6 @@ KernelTimer::~KernelTimer()
 }
 
 // ------------------------------------------------------------------ kernels
-__global__ void narrow_i64_to_i32(const int64_t *__restrict__ in, int32_t *__restrict__ out, int64_t n)
-{
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t step = (int64_t)gridDim.x * blockDim.x;
-    for (; i < n; i += step)
-        out[i] = (int32_t)in[i];
-}
-
-__global__ void widen_i32_to_i64(const int32_t *__restrict__ in, int64_t *__restrict__ out, int64_t n)
-{
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t step = (int64_t)gridDim.x * blockDim.x;
-    for (; i < n; i += step)
-        out[i] = (int64_t)in[i];
-}
-
 __global__ void copy_f64_kernel(double *__restrict__ dst, const double *__restrict__ src, int64_t n)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -755,26 +739,157 @@ __global__ __launch_bounds__(256) void csr_check_device(int64_t nrows, int64_t n
     }
 }
 
-static Workspace g_check_flag;
+static int launch_device_check(const Csr *c, int32_t **flag)
+{
+    COMET_CHK(mailbox((void **)flag));
+    **flag = 0;
+    const unsigned blocks = (unsigned)std::min<int64_t>(std::max<int64_t>(ceil_div(c->nrows, 4), 1), 16384);
+    csr_check_device<<<dim3(blocks), dim3(256), 0, stream()>>>(c->nrows, c->ncols, c->nnz, c->pos, c->crd, *flag);
+    COMET_HIPCHK(hipGetLastError());
+    return COMET_HIP_OK;
+}
 
 static int validate_device_csr(const Csr *c)
 {
-    COMET_CHK(g_check_flag.ensure(sizeof(int32_t), false));
-    int32_t *flag = (int32_t *)g_check_flag.ptr;
-    COMET_HIPCHK(hipMemsetAsync(flag, 0, sizeof(int32_t), stream()));
-    const unsigned blocks = (unsigned)std::min<int64_t>(std::max<int64_t>(ceil_div(c->nrows, 4), 1), 16384);
-    csr_check_device<<<dim3(blocks), dim3(256), 0, stream()>>>(c->nrows, c->ncols, c->nnz, c->pos, c->crd, flag);
-    COMET_HIPCHK(hipGetLastError());
-    int32_t bad = 0;
-    COMET_HIPCHK(hipMemcpyAsync(&bad, flag, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
-    COMET_HIPCHK(hipStreamSynchronize(stream()));
-    if (bad)
+    int32_t *flag = nullptr;
+    COMET_CHK(launch_device_check(c, &flag));
+    COMET_CHK(stream_wait());
+    if (*(volatile int32_t *)flag)
         return set_error(COMET_HIP_ERR_ARG,
                          "device CSR arrays are not a valid matrix: pos must start at 0, never decrease and end at nnz; "
                          "columns must lie in [0, ncols) and must not decrease inside a row");
     return COMET_HIP_OK;
 }
 
+// The row pointers are looked at here (what is copied depends on them), the columns on their way up (range) and on the
+// device (order); only a matrix that fails is looked through again, for the message.
+template <typename I>
+static Csr *csr_from_host_impl(int64_t nrows, int64_t ncols, const I *pos, const I *crd, const double *val,
+                               std::vector<Piece> more)
+{
+    bool bad = nrows < 0 || ncols < 0 || !pos || nrows >= INT32_MAX || ncols >= INT32_MAX || pos[0] != 0;
+    if (!bad) {
+        int falls = 0;
+        for (int64_t i = 0; i < nrows; ++i)
+            falls |= pos[i + 1] < pos[i];
+        bad = falls != 0 || (pos[nrows] > 0 && (!crd || !val));
+    }
+    if (bad) {
+        (void)validate_host_csr(nrows, ncols, pos, crd, val);
+        return nullptr;
+    }
+    const int64_t nnz = (int64_t)pos[nrows];
+    Csr *c = new Csr();
+    const auto fail = [&]() -> Csr * {
+        csr_release(c);
+        return nullptr;
+    };
+    if (csr_alloc(c, nrows, ncols, nnz) != COMET_HIP_OK)
+        return fail();
+    std::atomic<int> outside{0};
+    std::vector<Piece> pieces;
+    pieces.push_back(Piece{c->pos, (size_t)nrows + 1, sizeof(int64_t), [pos](void *pin, size_t first, size_t count) {
+                               for (size_t i = 0; i < count; ++i)
+                                   ((int64_t *)pin)[i] = (int64_t)pos[first + i];
+                           }});
+    if (nnz > 0) {
+        pieces.push_back(Piece{c->crd, (size_t)nnz, sizeof(int32_t),
+                               [crd, ncols, &outside](void *pin, size_t first, size_t count) {
+                                   using U = typename std::make_unsigned<I>::type;
+                                   int out = 0;
+                                   for (size_t i = 0; i < count; ++i) {
+                                       const I v = crd[first + i];
+                                       out |= (U)v >= (U)ncols;
+                                       ((int32_t *)pin)[i] = (int32_t)v;
+                                   }
+                                   if (out)
+                                       outside = 1;
+                               }});
+        pieces.push_back(plain_up(c->val, val, sizeof(double) * (size_t)nnz));
+    }
+    for (Piece &p : more)
+        pieces.push_back(std::move(p));
+    int32_t *flag = nullptr;
+    if (transfer_up(pieces) != COMET_HIP_OK || launch_device_check(c, &flag) != COMET_HIP_OK ||
+        stream_wait() != COMET_HIP_OK)
+        return fail();
+    if (outside || *(volatile int32_t *)flag) {
+        if (validate_host_csr(nrows, ncols, pos, crd, val) == COMET_HIP_OK)
+            set_error(COMET_HIP_ERR_ARG, "the CSR arrays changed while they were copied");
+        return fail();
+    }
+    return c;
+}
+
+template <typename I>
+static int csr_to_host(const Csr *c, I *pos, I *crd, double *val)
+{
+    std::vector<Piece> pieces;
+    if (pos)
+        pieces.push_back(Piece{c->pos, (size_t)c->nrows + 1, sizeof(int64_t), [pos](void *pin, size_t first, size_t count) {
+                                   for (size_t i = 0; i < count; ++i)
+                                       pos[first + i] = (I)((const int64_t *)pin)[i];
+                               }});
+    if (crd && c->nnz)
+        pieces.push_back(Piece{c->crd, (size_t)c->nnz, sizeof(int32_t), [crd](void *pin, size_t first, size_t count) {
+                                   for (size_t i = 0; i < count; ++i)
+                                       crd[first + i] = (I)((const int32_t *)pin)[i];
+                               }});
+    if (val && c->nnz)
+        pieces.push_back(plain_down(val, c->val, sizeof(double) * (size_t)c->nnz));
+    return transfer_down(pieces);
+}
+
+namespace comet {
+
+Csr *csr_from_host(int64_t nrows, int64_t ncols, const int64_t *pos, const int64_t *crd, const double *val,
+                   std::vector<Piece> more)
+{
+    return csr_from_host_impl(nrows, ncols, pos, crd, val, std::move(more));
+}
+
+Csr *csr_from_host(int64_t nrows, int64_t ncols, const int32_t *pos, const int32_t *crd, const double *val,
+                   std::vector<Piece> more)
+{
+    return csr_from_host_impl(nrows, ncols, pos, crd, val, std::move(more));
+}
+
+// one word per thread (each waits for its own results), given back when the thread ends
+struct MailboxWords {
+    std::mutex mu;
+    std::vector<void *> words;
+};
+static MailboxWords *g_mailbox = new MailboxWords();          // outlives every thread
+struct MailboxOwner {
+    void *word = nullptr;
+    ~MailboxOwner()
+    {
+        if (word) {
+            std::lock_guard<std::mutex> lk(g_mailbox->mu);
+            g_mailbox->words.push_back(word);
+        }
+    }
+};
+
+int mailbox(void **host_word)
+{
+    static thread_local MailboxOwner mine;
+    if (!mine.word) {
+        std::lock_guard<std::mutex> lk(g_mailbox->mu);
+        if (g_mailbox->words.empty()) {
+            char *page = nullptr;
+            COMET_HIPCHK(hipHostMalloc((void **)&page, 4096, hipHostMallocDefault));
+            for (int i = 0; i < 64; ++i)
+                g_mailbox->words.push_back(page + 64 * i);
+        }
+        mine.word = g_mailbox->words.back();
+        g_mailbox->words.pop_back();
+    }
+    *host_word = mine.word;
+    return COMET_HIP_OK;
+}
+
+}  // namespace comet
 
 // ====================================================================== C ABI
 extern "C" {
@@ -861,10 +976,8 @@ int comet_hip_memcpy(int64_t dptr, void *host, int64_t bytes, int64_t direction)
         return set_error(COMET_HIP_ERR_ARG, "bad memcpy arguments");
     if (bytes == 0)
         return COMET_HIP_OK;
-    if (direction == 0)
-        COMET_HIPCHK(hipMemcpyAsync((void *)dptr, host, (size_t)bytes, hipMemcpyHostToDevice, stream()));
-    else
-        COMET_HIPCHK(hipMemcpyAsync(host, (void *)dptr, (size_t)bytes, hipMemcpyDeviceToHost, stream()));
+    COMET_CHK(direction == 0 ? transfer_up({plain_up((void *)dptr, host, (size_t)bytes)})
+                             : transfer_down({plain_down(host, (const void *)dptr, (size_t)bytes)}));
     return stream_wait();
 }
 
@@ -912,74 +1025,15 @@ void HipMemcpyIndex(int64_t dptr, void *p, void *aligned, int64_t offset, int64_
 int64_t comet_hip_csr_upload_i64(int64_t nrows, int64_t ncols, const int64_t *pos, const int64_t *crd,
                                  const double *val)
 {
-    if (ensure_init() != COMET_HIP_OK)
-        return 0;
-    if (validate_host_csr(nrows, ncols, pos, crd, val) != COMET_HIP_OK)
-        return 0;
-    int64_t nnz = pos[nrows];
-    Csr *c = new Csr();
-    int64_t *tmp = nullptr;
-    auto fail = [&]() -> int64_t {
-        if (tmp)
-            (void)dev_free(tmp);
-        csr_release(c);
-        return 0;
-    };
-    if (csr_alloc(c, nrows, ncols, nnz) != COMET_HIP_OK)
-        return fail();
-    hipStream_t s = stream();
-    if (hipMemcpyAsync(c->pos, pos, sizeof(int64_t) * (size_t)(nrows + 1), hipMemcpyHostToDevice, s) != hipSuccess)
-        return set_error(COMET_HIP_ERR_HIP, "pos upload failed"), fail();
-    if (nnz > 0) {
-        if (dev_malloc((void **)&tmp, sizeof(int64_t) * (size_t)nnz) != hipSuccess)
-            return set_error(COMET_HIP_ERR_HIP, "staging allocation failed"), fail();
-        if (hipMemcpyAsync(tmp, crd, sizeof(int64_t) * (size_t)nnz, hipMemcpyHostToDevice, s) != hipSuccess ||
-            hipMemcpyAsync(c->val, val, sizeof(double) * (size_t)nnz, hipMemcpyHostToDevice, s) != hipSuccess)
-            return set_error(COMET_HIP_ERR_HIP, "crd/val upload failed"), fail();
-        unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(nnz, 256), 65536);
-        narrow_i64_to_i32<<<dim3(blocks), dim3(256), 0, s>>>(tmp, c->crd, nnz);
-    }
-    if (hipStreamSynchronize(s) != hipSuccess)
-        return set_error(COMET_HIP_ERR_HIP, "upload synchronisation failed"), fail();
-    if (tmp)
-        (void)dev_free(tmp);
-    return csr_register(c);
+    Csr *c = ensure_init() == COMET_HIP_OK ? csr_from_host(nrows, ncols, pos, crd, val) : nullptr;
+    return c ? csr_register(c) : 0;
 }
 
 int64_t comet_hip_csr_upload_i32(int64_t nrows, int64_t ncols, const int32_t *pos, const int32_t *crd,
                                  const double *val)
 {
-    if (ensure_init() != COMET_HIP_OK)
-        return 0;
-    if (validate_host_csr(nrows, ncols, pos, crd, val) != COMET_HIP_OK)
-        return 0;
-    int64_t nnz = pos[nrows];
-    Csr *c = new Csr();
-    int32_t *tmp = nullptr;
-    auto fail = [&]() -> int64_t {
-        if (tmp)
-            (void)dev_free(tmp);
-        csr_release(c);
-        return 0;
-    };
-    if (csr_alloc(c, nrows, ncols, nnz) != COMET_HIP_OK)
-        return fail();
-    hipStream_t s = stream();
-    if (dev_malloc((void **)&tmp, sizeof(int32_t) * (size_t)(nrows + 1)) != hipSuccess)
-        return set_error(COMET_HIP_ERR_HIP, "staging allocation failed"), fail();
-    if (hipMemcpyAsync(tmp, pos, sizeof(int32_t) * (size_t)(nrows + 1), hipMemcpyHostToDevice, s) != hipSuccess)
-        return set_error(COMET_HIP_ERR_HIP, "pos upload failed"), fail();
-    unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(nrows + 1, 256), 65536);
-    widen_i32_to_i64<<<dim3(blocks), dim3(256), 0, s>>>(tmp, c->pos, nrows + 1);
-    if (nnz > 0) {
-        if (hipMemcpyAsync(c->crd, crd, sizeof(int32_t) * (size_t)nnz, hipMemcpyHostToDevice, s) != hipSuccess ||
-            hipMemcpyAsync(c->val, val, sizeof(double) * (size_t)nnz, hipMemcpyHostToDevice, s) != hipSuccess)
-            return set_error(COMET_HIP_ERR_HIP, "crd/val upload failed"), fail();
-    }
-    if (hipStreamSynchronize(s) != hipSuccess)
-        return set_error(COMET_HIP_ERR_HIP, "upload synchronisation failed"), fail();
-    (void)dev_free(tmp);
-    return csr_register(c);
+    Csr *c = ensure_init() == COMET_HIP_OK ? csr_from_host(nrows, ncols, pos, crd, val) : nullptr;
+    return c ? csr_register(c) : 0;
 }
 
 int64_t comet_hip_csr_wrap(int64_t nrows, int64_t ncols, int64_t nnz, int64_t pos_dptr, int64_t crd_dptr,
@@ -1035,24 +1089,7 @@ int comet_hip_csr_download_i64(int64_t csr, int64_t *pos, int64_t *crd, double *
     Csr *c = csr_from_handle(csr);
     if (!c)
         return COMET_HIP_ERR_HANDLE;
-    hipStream_t s = stream();
-    if (pos)
-        COMET_HIPCHK(hipMemcpyAsync(pos, c->pos, sizeof(int64_t) * (size_t)(c->nrows + 1), hipMemcpyDeviceToHost, s));
-    if (val && c->nnz)
-        COMET_HIPCHK(hipMemcpyAsync(val, c->val, sizeof(double) * (size_t)c->nnz, hipMemcpyDeviceToHost, s));
-    if (crd && c->nnz) {
-        int64_t *tmp = nullptr;
-        COMET_HIPCHK(dev_malloc((void **)&tmp, sizeof(int64_t) * (size_t)c->nnz));
-        unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(c->nnz, 256), 65536);
-        widen_i32_to_i64<<<dim3(blocks), dim3(256), 0, s>>>(c->crd, tmp, c->nnz);
-        hipError_t e = hipMemcpyAsync(crd, tmp, sizeof(int64_t) * (size_t)c->nnz, hipMemcpyDeviceToHost, s);
-        hipError_t e2 = hipStreamSynchronize(s);
-        (void)dev_free(tmp);
-        COMET_HIPCHK(e);
-        COMET_HIPCHK(e2);
-    }
-    COMET_HIPCHK(hipStreamSynchronize(s));
-    return COMET_HIP_OK;
+    return csr_to_host(c, pos, crd, val);
 }
 
 int comet_hip_csr_download_i32(int64_t csr, int32_t *pos, int32_t *crd, double *val)
@@ -1062,24 +1099,7 @@ int comet_hip_csr_download_i32(int64_t csr, int32_t *pos, int32_t *crd, double *
         return COMET_HIP_ERR_HANDLE;
     if (pos && c->nnz > INT32_MAX)
         return set_error(COMET_HIP_ERR_SIZE, "nnz %lld does not fit an int32 row pointer", (long long)c->nnz);
-    hipStream_t s = stream();
-    if (pos) {
-        int32_t *tmp = nullptr;
-        COMET_HIPCHK(dev_malloc((void **)&tmp, sizeof(int32_t) * (size_t)(c->nrows + 1)));
-        unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(c->nrows + 1, 256), 65536);
-        narrow_i64_to_i32<<<dim3(blocks), dim3(256), 0, s>>>(c->pos, tmp, c->nrows + 1);
-        hipError_t e = hipMemcpyAsync(pos, tmp, sizeof(int32_t) * (size_t)(c->nrows + 1), hipMemcpyDeviceToHost, s);
-        hipError_t e2 = hipStreamSynchronize(s);
-        (void)dev_free(tmp);
-        COMET_HIPCHK(e);
-        COMET_HIPCHK(e2);
-    }
-    if (crd && c->nnz)
-        COMET_HIPCHK(hipMemcpyAsync(crd, c->crd, sizeof(int32_t) * (size_t)c->nnz, hipMemcpyDeviceToHost, s));
-    if (val && c->nnz)
-        COMET_HIPCHK(hipMemcpyAsync(val, c->val, sizeof(double) * (size_t)c->nnz, hipMemcpyDeviceToHost, s));
-    COMET_HIPCHK(hipStreamSynchronize(s));
-    return COMET_HIP_OK;
+    return csr_to_host(c, pos, crd, val);
 }
 
 int comet_hip_csr_invalidate(int64_t csr)

@@ -758,15 +758,16 @@ static int gett_device(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t
             return true;
         };
         const int ra = a_m ? sh.bm / 16 : 2, rb = b_n ? sh.bn / 16 : 2;
-        const bool pairs = reg && K % GM_BK == 0 && sh.bn >= 64 && (((uintptr_t)A | (uintptr_t)B) & 15) == 0 &&
+        const bool unbroken = reg && K % GM_BK == 0 && sh.bn >= 64 && (((uintptr_t)A | (uintptr_t)B) & 15) == 0 &&
                            runs(m, m.s0, a_m, ra) && runs(k, k.s0, !a_m, 2) && runs(n, n.s0, b_n, rb) &&
                            runs(k, k.s1, !b_n, 2);
         const auto launch = [&](auto kernel_shape, auto wave_rows, auto occ) {
             constexpr GettShape S = GETT_SHAPES[decltype(kernel_shape)::value];
             constexpr int WM = decltype(wave_rows)::value, OCC = decltype(occ)::value;
-            if (pairs)
-                gett_launch<S.bm, S.bn >= 64 ? S.bn : 64, WM, OCC, true, true, uint32_t>(a_m, b_n, grid, g, A, B, C, partial, use_c);
-            else if (reg)
+            if constexpr (S.bn >= 64)
+                if (unbroken)
+                    return gett_launch<S.bm, S.bn, WM, OCC, true, true, uint32_t>(a_m, b_n, grid, g, A, B, C, partial, use_c);
+            if (reg)
                 gett_launch<S.bm, S.bn, WM, OCC, true, false, uint32_t>(a_m, b_n, grid, g, A, B, C, partial, use_c);
             else
                 gett_launch<S.bm, S.bn, WM, OCC, false, false, uint32_t>(a_m, b_n, grid, g, A, B, C, partial, use_c);

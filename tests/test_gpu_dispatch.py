@@ -59,3 +59,29 @@ def test_contraction_with_a_turned_operand(extent):
     C, _ = rt.ttgt_contract("aebf", "dfce", "abcd", rt.DeviceArray.from_numpy(A), rt.DeviceArray.from_numpy(B))
     want = np.tensordot(A, B, axes=([1, 3], [3, 1])).transpose(0, 1, 3, 2)
     assert np.abs(C.to_numpy() - want).max() <= 1e-11
+
+
+@pytest.mark.parametrize("nbytes", [1, 15, 16, (1 << 18) - 1, (1 << 18) + 1, (1 << 20) + 7, (1 << 20) * 7 + 16, (1 << 20) * 19 + 5])
+@pytest.mark.parametrize("offset", [0, 4, 16])
+def test_copies_between_host_and_device(nbytes, offset):
+    host = np.random.default_rng(nbytes).integers(0, 256, nbytes, dtype=np.uint8)
+    d = rt.DeviceArray(nbytes + 32, np.uint8, zero=True)
+    rt._check(rt.lib().comet_hip_memcpy(d.ptr + offset, rt._vptr(host), nbytes, 0))
+    back = np.zeros(nbytes, np.uint8)
+    rt._check(rt.lib().comet_hip_memcpy(d.ptr + offset, rt._vptr(back), nbytes, 1))
+    whole = d.to_numpy()
+    assert np.array_equal(back, host) and not whole[:offset].any() and not whole[offset + nbytes:].any()
+
+
+@pytest.mark.parametrize("idt", [np.int64, np.int32])
+@pytest.mark.parametrize("n,mean", [(1, 1.0), (700, 3.0), (90_001, 9.0), (400_000, 8.0)])
+def test_csr_goes_up_and_comes_back(n, mean, idt):
+    pos, crd, val = gen.poisson_csr(n=n, mean=mean, seed=3)
+    got = rt.CsrMatrix.from_arrays((n, n), pos.astype(idt), crd.astype(idt), val).to_arrays(idt)
+    assert all(np.array_equal(g, w) for g, w in zip(got, (pos, crd, val)))
+    if idt is np.int64 and len(crd):
+        for bad in (n, -1, (1 << 32) + int(crd[-1])):          # the last one would pass for a column in 32 bits
+            wrong = crd.copy()
+            wrong[-1] = bad
+            with pytest.raises(rt.CometHipError, match="outside"):
+                rt.CsrMatrix.from_arrays((n, n), pos, wrong, val)
