@@ -104,11 +104,29 @@ struct RowListEntry {
 };
 uint64_t next_csr_uid();
 
+// What masked products taken pair by pair keep (masked_pairs.h): the pairs of either side as lists of lists, and the
+// rows that have any as work items.
+struct PairSidePlan {
+    int64_t first = 0, pairs = 0, nheavy = 0, nlight = 0;
+    int64_t *kpos = nullptr, *place = nullptr, *counts = nullptr;
+    void *ent = nullptr, *heavy = nullptr;
+    double *weight = nullptr;
+    int32_t *light = nullptr, *padded = nullptr;
+};
+struct PairPlan {
+    uint64_t b_uid = 0, mask_uid = 0;
+    int kind = 0;                // 0: product, 1: sum, 2 and 3: sum with every row sent one way
+    int64_t first = 0, last = 0;
+    PairSidePlan side[2];
+};
+void pair_plan_free(PairPlan &p);
+
 struct Csr {
     // names this state of the matrix: new for every matrix and again whenever its arrays may have changed
     // (comet_hip_csr_invalidate), so that what other handles keep about it can tell that it is stale
     uint64_t uid = next_csr_uid();
     std::vector<RowListEntry> row_lists;
+    std::vector<PairPlan> pair_plans;
     int64_t nrows = 0, ncols = 0, nnz = 0;
     int64_t *pos = nullptr;
     int32_t *crd = nullptr;

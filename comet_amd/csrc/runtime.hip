@@ -318,8 +318,21 @@ uint64_t next_csr_uid()
     return next.fetch_add(1);
 }
 
+void pair_plan_free(PairPlan &p)
+{
+    for (PairSidePlan &s : p.side) {
+        for (void *q : {(void *)s.kpos, (void *)s.place, (void *)s.counts, s.ent, s.heavy, (void *)s.weight,
+                        (void *)s.light, (void *)s.padded})
+            (void)dev_free(q);
+        s = PairSidePlan();
+    }
+}
+
 static void csr_drop_plans(Csr *c)
 {
+    for (PairPlan &p : c->pair_plans)
+        pair_plan_free(p);
+    c->pair_plans.clear();
     c->uid = next_csr_uid();
     for (auto &e : c->row_lists) {
         (void)dev_free(e.rows);

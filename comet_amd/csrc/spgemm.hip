@@ -23,10 +23,11 @@
 // (spgemm_numeric_dense_kernel, the widest rows).
 // The order in which the products of one (i,j) are added is therefore not the
 // reference's ascending-k order: values agree to rounding, structure exactly.
+#include <algorithm>
+#include <cstring>
 #include <type_traits>
 
 #include "common.h"
-#include <cstring>
 
 namespace comet {
 
@@ -50,6 +51,12 @@ __device__ inline int64_t readlane_i64(int64_t v, int lane)
     lo = __builtin_amdgcn_readlane(lo, lane);
     hi = __builtin_amdgcn_readlane(hi, lane);
     return ((int64_t)hi << 32) | (uint32_t)lo;
+}
+
+__device__ inline int64_t uniform_i64_sg(int64_t v)
+{
+    return ((int64_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+           (uint32_t)__builtin_amdgcn_readfirstlane((int)(v & 0xffffffff));
 }
 
 __device__ inline double readlane_d(double v, int lane)
@@ -2279,341 +2286,6 @@ __global__ __launch_bounds__(SM_WAVES * 64) void spgemm_masked_sum_small_kernel(
     }
 }
 
-// ---------------------------------------------------------------------------
-// The same sums when every stored value of B is one number b (a pattern matrix): a product that meets the mask
-// adds a * b whatever its place in the row of B, so a row of B only has to be counted - how many of its columns
-// are in the mask row - and the count times a * b is what it contributes.  No value is fetched, nothing is
-// carried from the look-up to a later visit, and the walk shrinks to a load, an LDS read and a bit test per
-// product.  (Sums of whole numbers, as in a triangle count, are the same in either form; otherwise the two differ
-// by rounding, each within the bound the unmasked forms keep.)
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ int bitmap_bit(const uint32_t *bm, int j)
-{
-    return (int)((bm[(uint32_t)j >> 5] >> ((uint32_t)j & 31u)) & 1u);
-}
-__device__ __forceinline__ int bitmap_bits4(const uint32_t *bm, sg_i4u j)
-{
-    const uint32_t w0 = bm[(uint32_t)j.x >> 5], w1 = bm[(uint32_t)j.y >> 5], w2 = bm[(uint32_t)j.z >> 5],
-                   w3 = bm[(uint32_t)j.w >> 5];
-    return (int)(((w0 >> ((uint32_t)j.x & 31u)) & 1u) + ((w1 >> ((uint32_t)j.y & 31u)) & 1u) +
-                 ((w2 >> ((uint32_t)j.z & 31u)) & 1u) + ((w3 >> ((uint32_t)j.w & 31u)) & 1u));
-}
-// What a lane holds of a turn in flight: up to four 16-byte loads (four consecutive columns each) of the row of
-// B its group of lanes is on, one more column if the row's length is not a multiple of four, and the value
-// a * b every hit of this row is worth.
-struct IsoTurn {
-    sg_i4u q[4];
-    int tail;
-    uint32_t ok;        // bit x: q[x] holds columns; bit 4: tail does
-    double at;
-};
-// The loads of a turn.  `row` is the lane's row of B, `first` the first group of four columns the lane takes and
-// `stride` the distance to its next one, nq the number of full groups of four in the row; rest = the columns
-// beyond them if this is the row's last turn (else 0), taken by the first lanes of the group (sub = the lane's
-// number inside it).
-__device__ __forceinline__ void iso_issue(IsoTurn &t, const int32_t *__restrict__ row, int first, int stride, int nq,
-                                          int rest, int sub, double at)
-{
-    t.ok = 0;
-    t.at = at;
-    t.tail = 0;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-        const int qi = first + stride * x;
-        t.q[x] = sg_i4u{0, 0, 0, 0};
-        if (qi < nq) {
-            t.q[x] = *reinterpret_cast<const sg_i4u *>(row + 4 * qi);
-            t.ok |= 1u << x;
-        }
-    }
-    if (sub < rest) {
-        t.tail = row[4 * nq + sub];
-        t.ok |= 16u;
-    }
-}
-template <typename PROBE>
-__device__ __forceinline__ void iso_consume(const IsoTurn &t, const PROBE &probe, double &part)
-{
-    int hits = 0;
-#pragma unroll
-    for (int x = 0; x < 4; ++x)
-        if (t.ok & (1u << x))
-            hits += probe.four(t.q[x]);
-    if (t.ok & 16u)
-        hits += probe.one(t.tail);
-    if (hits)                   // a row without hits adds nothing, whatever its value (0 * inf would be NaN)
-        part += (double)hits * t.at;
-}
-// `todo` names lanes that hold a row of B each; the next G of them go to the G groups of 64 / G lanes of the
-// wavefront.  Returns the lane whose row this lane's group takes, or -1.
-template <int G>
-__device__ __forceinline__ int iso_pick(unsigned long long &todo, int lane)
-{
-    int pick = -1;
-    const int group = lane / (64 / G);
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const int t = todo ? __builtin_ctzll(todo) : -1;
-        todo = todo ? (todo & (todo - 1)) : 0;
-        pick = group == g ? t : pick;
-    }
-    return pick;
-}
-
-// The walk of one output row by a team of TEAM wavefronts (this is wavefront `wave` of it).  The entries of A's
-// row are dealt to the wavefronts one at a time, 64 per wavefront and pass.  What bounds a walk like this is
-// not the look-ups but the wait for a row of B to arrive, so rows are taken several at a time and a turn
-// ahead: rows of 512 entries and more by the whole wavefront, 1024 columns per turn; rows of 256 and more two at
-// a time, one per half; shorter ones four at a time, one per 16-lane quarter; and the loads of a turn are issued
-// before the look-ups of the turn before it, across rows.  probe.four(j4) / probe.one(j) say how many of the
-// columns are in the mask row.  Returns the lane's share of the sum.
-template <int TEAM, typename PROBE>
-__device__ __forceinline__ double iso_walk(int64_t as, int64_t ae, const int32_t *__restrict__ Acrd,
-                                           const double *__restrict__ Aval, const int64_t *__restrict__ Bpos,
-                                           const int32_t *__restrict__ Bcrd, double biso, const PROBE &probe, int wave,
-                                           int lane)
-{
-    double part = 0.0;
-    IsoTurn pend;
-    pend.ok = 0;
-    pend.at = 0.0;
-    pend.tail = 0;
-#pragma unroll
-    for (int x = 0; x < 4; ++x)
-        pend.q[x] = sg_i4u{0, 0, 0, 0};
-    for (int64_t base = as + wave; base < ae; base += (int64_t)TEAM * 64) {
-        const int64_t left = (ae - base + TEAM - 1) / TEAM;     // my entries from here on
-        const int cnt = (int)(left < 64 ? left : 64);
-        int64_t bs = 0;
-        int len = 0;
-        double a = 0.0;
-        if (lane < cnt) {
-            const int64_t p = base + (int64_t)lane * TEAM;
-            const int k = Acrd[p];
-            bs = Bpos[k];
-            len = (int)(Bpos[k + 1] - bs);      // a row holds fewer entries than the matrix has columns: < 2^31
-            a = Aval[p] * biso;
-        }
-        unsigned long long big = __ballot(len >= 512);
-        unsigned long long mid = __ballot(len >= 256 && len < 512);
-        unsigned long long small = __ballot(len > 0 && len < 256);
-        while (big) {
-            const int t = __builtin_ctzll(big);
-            big &= big - 1;
-            const int32_t *row = Bcrd + readlane_i64(bs, t);
-            const int n = __builtin_amdgcn_readlane(len, t);
-            const double at = readlane_d(a, t);
-            const int nq = n >> 2;
-            for (int tb = 0; tb == 0 || tb < nq; tb += 256) {
-                IsoTurn now;
-                iso_issue(now, row, tb + lane, 64, nq, tb + 256 >= nq ? (n & 3) : 0, lane, at);
-                iso_consume(pend, probe, part);
-                pend = now;
-            }
-        }
-        while (mid) {
-            const int pick = iso_pick<2>(mid, lane);
-            const int src = pick < 0 ? lane : pick;
-            // by every lane: a lane whose group sits this round out may be another's source
-            const int64_t s = ((int64_t)__shfl((int)(bs >> 32), src, 64) << 32) |
-                              (uint32_t)__shfl((int)(bs & 0xffffffff), src, 64);
-            const int n_src = __shfl(len, src, 64);
-            const double at = __hiloint2double(__shfl(__double2hiint(a), src, 64), __shfl(__double2loint(a), src, 64));
-            const int n = pick < 0 ? 0 : n_src;
-            IsoTurn now;
-            iso_issue(now, Bcrd + s, lane & 31, 32, n >> 2, n & 3, lane & 31, at);
-            iso_consume(pend, probe, part);
-            pend = now;
-        }
-        while (small) {
-            const int pick = iso_pick<4>(small, lane);
-            const int src = pick < 0 ? lane : pick;
-            const int64_t s = ((int64_t)__shfl((int)(bs >> 32), src, 64) << 32) |
-                              (uint32_t)__shfl((int)(bs & 0xffffffff), src, 64);
-            const int n_src = __shfl(len, src, 64);
-            const double at = __hiloint2double(__shfl(__double2hiint(a), src, 64), __shfl(__double2loint(a), src, 64));
-            const int n = pick < 0 ? 0 : n_src;
-            IsoTurn now;
-            iso_issue(now, Bcrd + s, lane & 15, 16, n >> 2, n & 3, lane & 15, at);
-            iso_consume(pend, probe, part);
-            pend = now;
-        }
-    }
-    iso_consume(pend, probe, part);
-    return part;
-}
-
-struct BitmapProbe {
-    const uint32_t *bm;
-    __device__ __forceinline__ int one(int j) const { return bitmap_bit(bm, j); }
-    __device__ __forceinline__ int four(sg_i4u j) const { return bitmap_bits4(bm, j); }
-};
-
-__global__ __launch_bounds__(SG_T) void spgemm_masked_sum_iso_kernel(
-    const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd, const double *__restrict__ Aval,
-    const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd, double biso,
-    const int64_t *__restrict__ Mpos, const int32_t *__restrict__ Mcrd, int nwords, unsigned long long *ticket,
-    RowList list, double *__restrict__ rowsum)
-{
-    // the workgroup kernel: rows from the heavy end of the list, the mask row as a bitmap of nwords words in LDS
-    __shared__ int64_t row_slot;
-    __shared__ double wave_part[SG_WAVES];
-    uint32_t *bm = sg_dyn_lds;
-    for (int w = threadIdx.x; w < nwords; w += SG_T)
-        bm[w] = 0;
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int64_t t_first, t_end;
-    list_range(list, 2, &t_first, &t_end);
-    int64_t tk = draw_front(ticket, t_end, &row_slot);
-    while (tk < t_end) {
-        const int64_t i = list.rows[tk];      // rows outside the list keep the zero the host put there
-        const int64_t as = Apos[i], ae = Apos[i + 1];
-        const int64_t ms = Mpos[i], me = Mpos[i + 1];
-        const bool work = as != ae && ms != me;
-        if (work) {
-            for (int64_t t = ms + threadIdx.x; t < me; t += SG_T) {
-                const uint32_t j = (uint32_t)Mcrd[t];
-                atomicOr(&bm[j >> 5], 1u << (j & 31u));
-            }
-            __syncthreads();
-            double part = iso_walk<SG_WAVES>(as, ae, Acrd, Aval, Bpos, Bcrd, biso, BitmapProbe{bm}, wave, lane);
-            part = wave_sum_f64(part);
-            if (lane == 0)
-                wave_part[wave] = part;
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                double total = 0.0;
-                for (int w = 0; w < SG_WAVES; ++w)
-                    total += wave_part[w];
-                rowsum[i] = total;
-            }
-            for (int64_t t = ms + threadIdx.x; t < me; t += SG_T)
-                bm[(uint32_t)Mcrd[t] >> 5] = 0;
-        }   // work
-        tk = draw_front(ticket, t_end, &row_slot);     // its barriers also close this row's bitmap clean-up
-    }
-}
-
-// The wavefront kernel for a pattern matrix B: the walk above with the mask row in a table of the wavefront's own.
-// The table is 64 buckets of four columns, the bucket a multiplicative hash of the column, so a look-up is one
-// 16-byte LDS read and four compares, without a loop.  A mask row goes in if no bucket overflows; three more
-// multipliers are tried before the row is searched by bisection in memory instead, as are mask rows of more than
-// SI_MASK_MAX entries (which sort to the other kernel's end of the list and only come here when this kernel gets
-// that far).
-constexpr int SI_MASK_MAX = 48;
-constexpr int SI_TRIES = 4;
-// a bucket read or cleared as one 16-byte access; may_alias, because the same words are also written one at a
-// time by atomicCAS through an int pointer, and without it the compiler is free to reorder the two kinds
-typedef int si_bucket __attribute__((ext_vector_type(4), may_alias));
-struct BucketProbe {
-    const int *tab;
-    uint32_t mult;
-    __device__ __forceinline__ static int bucket(int j, uint32_t mult)
-    {
-        return (int)((uint32_t)__umul24((uint32_t)j, mult) >> 26);      // __umul24 returns int: shift it as unsigned
-    }
-    __device__ __forceinline__ int one(int j) const
-    {
-        const si_bucket b = *reinterpret_cast<const si_bucket *>(tab + 4 * bucket(j, mult));
-        return (b.x == j) | (b.y == j) | (b.z == j) | (b.w == j);
-    }
-    __device__ __forceinline__ int four(sg_i4u j) const { return one(j.x) + one(j.y) + one(j.z) + one(j.w); }
-};
-struct BisectProbe {
-    const int32_t *m;       // the mask row, ascending
-    int n;
-    __device__ __forceinline__ int one(int j) const
-    {
-        int lo = 0, hi = n;
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (m[mid] < j)
-                lo = mid + 1;
-            else
-                hi = mid;
-        }
-        return lo < n && m[lo] == j;
-    }
-    __device__ __forceinline__ int four(sg_i4u j) const { return one(j.x) + one(j.y) + one(j.z) + one(j.w); }
-};
-
-__global__ __launch_bounds__(SM_WAVES * 64) void spgemm_masked_sum_small_iso_kernel(
-    const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd, const double *__restrict__ Aval,
-    const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd, double biso,
-    const int64_t *__restrict__ Mpos, const int32_t *__restrict__ Mcrd, unsigned long long *ticket, RowList list,
-    double *__restrict__ rowsum)
-{
-    __shared__ __align__(16) int table[SM_WAVES][SM_SLOTS];
-    const int lane = threadIdx.x & 63;
-    int *tab = table[threadIdx.x >> 6];
-    reinterpret_cast<si_bucket *>(tab)[lane] = si_bucket{-1, -1, -1, -1};
-    int64_t t_first, t_end;
-    list_range(list, 2, &t_first, &t_end);
-    int take = SM_BATCH;
-    for (;;) {
-        // rows from the light end of the list, as spgemm_masked_sum_small_kernel draws them
-        unsigned long long drawn = 0;
-        if (lane == 0)
-            drawn = atomicAdd(ticket, (unsigned long long)take << 32);
-        const int64_t f = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(drawn & 0xffffffffu));
-        const int64_t b = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(drawn >> 32));
-        if (f + b >= t_end)
-            break;
-        const int nb = (int)(b + take < t_end - f ? take : t_end - f - b);      // what the front had not reached
-        const int64_t taken = b + take;
-        take = taken < t_end / 2 ? SM_BATCH : taken < t_end - t_end / 4 ? SM_BATCH / 4 : 1;
-        // the rows of the batch and where they start and end in A and in the mask: one round trip for all of them
-        int bi = 0;
-        int64_t bas = 0, bae = 0, bms = 0, bme = 0;
-        if (lane < nb) {
-            bi = list.rows[t_end - 1 - (b + lane)];
-            bas = Apos[bi];
-            bae = Apos[bi + 1];
-            bms = Mpos[bi];
-            bme = Mpos[bi + 1];
-        }
-        for (int r = 0; r < nb; ++r) {
-            const int i = __builtin_amdgcn_readlane(bi, r);
-            const int64_t as = readlane_i64(bas, r), ae = readlane_i64(bae, r);
-            const int64_t ms = readlane_i64(bms, r), me = readlane_i64(bme, r);
-            if (as == ae || ms == me)
-                continue;               // rowsum[i] keeps the zero the host put there
-            const int mlen = (int)(me - ms < (int64_t)SI_MASK_MAX + 1 ? me - ms : SI_MASK_MAX + 1);
-            bool hashed = false;
-            uint32_t mult = 0;
-            if (mlen <= SI_MASK_MAX) {
-                const int j = lane < mlen ? Mcrd[ms + lane] : -1;
-                static_assert(SI_MASK_MAX <= 64, "a lane holds one column of the mask row");
-                for (int attempt = 0; attempt < SI_TRIES && !hashed; ++attempt) {
-                    mult = attempt == 0 ? 0x9E3779u : attempt == 1 ? 0x85EBCBu : attempt == 2 ? 0xC2B2AFu : 0x27D4EBu;
-                    bool placed = j < 0;
-                    if (j >= 0) {
-                        int *bk = tab + 4 * BucketProbe::bucket(j, mult);
-#pragma unroll
-                        for (int x = 0; x < 4; ++x)
-                            if (!placed)
-                                placed = atomicCAS(&bk[x], -1, j) == -1;
-                    }
-                    hashed = !__any(!placed);
-                    if (!hashed)
-                        reinterpret_cast<si_bucket *>(tab)[lane] = si_bucket{-1, -1, -1, -1};
-                }
-            }
-            double part;
-            if (hashed)
-                part = iso_walk<1>(as, ae, Acrd, Aval, Bpos, Bcrd, biso, BucketProbe{tab, mult}, 0, lane);
-            else
-                part = iso_walk<1>(as, ae, Acrd, Aval, Bpos, Bcrd, biso, BisectProbe{Mcrd + ms, (int)(me - ms)}, 0, lane);
-            part = wave_sum_f64(part);
-            if (lane == 0)
-                rowsum[i] = part;
-            if (hashed)
-                reinterpret_cast<si_bucket *>(tab)[lane] = si_bucket{-1, -1, -1, -1};
-        }
-    }
-}
-
 // whether all stored values of a matrix are one number (looked at once per matrix)
 __global__ void csr_values_differ(int64_t nnz, const double *__restrict__ val, int *__restrict__ flag)
 {
@@ -3492,6 +3164,29 @@ static int dot_no_duplicates(const Csr *x, bool *ok)
     return COMET_HIP_OK;
 }
 
+static int csr_is_iso(const Csr *x, bool *iso)
+{
+    Csr *m = const_cast<Csr *>(x);
+    if (m->iso_state == 0) {
+        int flag = 1;
+        if (m->nnz > 0) {
+            COMET_CHK(g_dot_flag.ensure(sizeof(int), false));
+            COMET_HIPCHK(hipMemsetAsync(g_dot_flag.ptr, 0, sizeof(int), stream()));
+            csr_values_differ<<<dim3((unsigned)ceil_div(m->nnz, 256)), dim3(256), 0, stream()>>>(m->nnz, m->val,
+                                                                                                (int *)g_dot_flag.ptr);
+            COMET_HIPCHK(hipGetLastError());
+            COMET_HIPCHK(hipMemcpyAsync(&flag, g_dot_flag.ptr, sizeof(int), hipMemcpyDeviceToHost, stream()));
+            COMET_HIPCHK(hipMemcpyAsync(&m->iso_value, m->val, sizeof(double), hipMemcpyDeviceToHost, stream()));
+            COMET_CHK(stream_wait());
+        }
+        m->iso_state = flag ? 2 : 1;
+    }
+    *iso = m->iso_state == 1;
+    return COMET_HIP_OK;
+}
+
+#include "masked_pairs.h"
+
 // A masked product runs as dot products when the table over k fits LDS and no list that goes into a table holds a
 // column twice.  COMET_HIP_SPGEMM_NO_DOT keeps the walk over the products of every row (the tests run both).
 static int dot_form_fits(const Csr *a, const Csr *b, const Csr *m, bool *fits)
@@ -3905,27 +3600,6 @@ extern "C" int64_t comet_hip_spgemm_csr_semiring(int64_t ah, int64_t bh, int64_t
     return csr_register(c);
 }
 
-static int csr_is_iso(const Csr *x, bool *iso)
-{
-    Csr *m = const_cast<Csr *>(x);
-    if (m->iso_state == 0) {
-        int flag = 1;
-        if (m->nnz > 0) {
-            COMET_CHK(g_dot_flag.ensure(sizeof(int), false));
-            COMET_HIPCHK(hipMemsetAsync(g_dot_flag.ptr, 0, sizeof(int), stream()));
-            csr_values_differ<<<dim3((unsigned)ceil_div(m->nnz, 256)), dim3(256), 0, stream()>>>(m->nnz, m->val,
-                                                                                                (int *)g_dot_flag.ptr);
-            COMET_HIPCHK(hipGetLastError());
-            COMET_HIPCHK(hipMemcpyAsync(&flag, g_dot_flag.ptr, sizeof(int), hipMemcpyDeviceToHost, stream()));
-            COMET_HIPCHK(hipMemcpyAsync(&m->iso_value, m->val, sizeof(double), hipMemcpyDeviceToHost, stream()));
-            COMET_CHK(stream_wait());
-        }
-        m->iso_state = flag ? 2 : 1;
-    }
-    *iso = m->iso_state == 1;
-    return COMET_HIP_OK;
-}
-
 extern "C" int comet_hip_spgemm_masked_sum(int64_t ah, int64_t bh, int64_t mh, double *out)
 {
     COMET_CHK(ensure_init());
@@ -3941,6 +3615,14 @@ extern "C" int comet_hip_spgemm_masked_sum(int64_t ah, int64_t bh, int64_t mh, d
     }
     SgGeom g;
     COMET_CHK(sg_geometry(b->ncols, &g));
+    bool iso = false;
+    if (g.lds)
+        COMET_CHK(csr_is_iso(b, &iso));
+    bool pairs = false;
+    if (iso)
+        COMET_CHK(pair_form_fits(a, b, m, &pairs));
+    if (pairs)
+        return pair_masked_sum(a, b, m, out);
     COMET_CHK(sg_reset_ticket());
     COMET_CHK(g_sg.rowcount.ensure(sizeof(double) * (size_t)a->nrows, false));
     uint32_t *gbm = nullptr;
@@ -3953,10 +3635,7 @@ extern "C" int comet_hip_spgemm_masked_sum(int64_t ah, int64_t bh, int64_t mh, d
     // rows whose mask row is too long for the wavefront kernel's table sort to the front, whatever their products:
     // the workgroup kernel, which starts there, looks a column up in one LDS read; the wavefront kernel would
     // bisect the mask row in memory for every product
-    bool iso = false;
-    if (g.lds)
-        COMET_CHK(csr_is_iso(b, &iso));
-    COMET_CHK(sg_row_list(a, b, 0, a->nrows, SG_NO_DENSE, SG_NO_DENSE, &list, m, iso ? SI_MASK_MAX : SM_MASK_MAX));
+    COMET_CHK(sg_row_list(a, b, 0, a->nrows, SG_NO_DENSE, SG_NO_DENSE, &list, m, SM_MASK_MAX));
     COMET_HIPCHK(hipMemsetAsync(rowsum, 0, sizeof(double) * (size_t)a->nrows, stream()));
     const dim3 grid((unsigned)g.groups), block(SG_T);
     // Two kernels side by side, the second on the auxiliary stream: a workgroup per row from the heavy end of
@@ -3973,21 +3652,6 @@ extern "C" int comet_hip_spgemm_masked_sum(int64_t ah, int64_t bh, int64_t mh, d
     const bool run_wg = !only || strcmp(only, "wavefront") != 0, run_wave = !only || strcmp(only, "workgroup") != 0;
     COMET_CHK(aux_fork());
     if (!run_wg) {
-    } else if (iso) {
-        const int nwords = (int)ceil_div(b->ncols, 32);
-        COMET_CHK(sg_allow_lds(spgemm_masked_sum_iso_kernel, sizeof(uint32_t) * (size_t)nwords));
-        KernelTimer t("spgemm_masked_sum");
-        // Not a workgroup for every CU: beside one, a CU's registers hold a single wavefront of the other kernel per
-        // SIMD, and the half million light rows that kernel takes each wait on memory four times in a row.  The
-        // CUs left free hold sixteen of its wavefronts (triangle count of the scale-20 graph: 5.2 ms with a
-        // workgroup on every CU, 4.76 ms on 208 to 224 of 256, 5.7 ms on 192).
-        // That single wavefront per SIMD is there only as long as this kernel keeps to 96 vector registers (four
-        // wavefronts of 96 and one of the other kernel's 112 make 496 of a SIMD's 512): with 97 it is allotted 104,
-        // the other kernel is left with the free CUs alone and the count takes 6.6 ms.
-        const dim3 igrid(g.groups == num_cus() ? (unsigned)(g.groups - 3 * (g.groups / 16)) : (unsigned)g.groups);
-        spgemm_masked_sum_iso_kernel<<<igrid, block, sizeof(uint32_t) * (size_t)nwords, stream()>>>(
-            a->pos, a->crd, a->val, b->pos, b->crd, b->iso_value, m->pos, m->crd, nwords,
-            (unsigned long long *)g_sg.ticket.ptr, list, rowsum);
     } else if (g.lds) {
         COMET_CHK(sg_allow_lds(spgemm_masked_sum_kernel<true>, g.lds_bytes));
         KernelTimer t("spgemm_masked_sum");
@@ -4000,12 +3664,7 @@ extern "C" int comet_hip_spgemm_masked_sum(int64_t ah, int64_t bh, int64_t mh, d
             a->nrows, a->pos, a->crd, a->val, b->pos, b->crd, b->val, m->pos, m->crd, g.logW, gbm,
             (unsigned long long *)g_sg.ticket.ptr, list, rowsum);
     }
-    if (run_wave && iso) {
-        KernelTimer t("spgemm_masked_sum_small", aux_stream());
-        spgemm_masked_sum_small_iso_kernel<<<dim3((unsigned)(num_cus() * 8)), dim3(SM_WAVES * 64), 0, aux_stream()>>>(
-            a->pos, a->crd, a->val, b->pos, b->crd, b->iso_value, m->pos, m->crd,
-            (unsigned long long *)g_sg.ticket.ptr, list, rowsum);
-    } else if (run_wave) {   // eight workgroups of four wavefronts per CU: four fit beside the kernel above, the rest follow it
+    if (run_wave) {   // eight workgroups of four wavefronts per CU: four fit beside the kernel above, the rest follow it
         KernelTimer t("spgemm_masked_sum_small", aux_stream());
         spgemm_masked_sum_small_kernel<<<dim3((unsigned)(num_cus() * 8)), dim3(SM_WAVES * 64), 0, aux_stream()>>>(
             a->pos, a->crd, a->val, b->pos, b->crd, b->val, m->pos, m->crd,
@@ -4168,9 +3827,9 @@ extern "C" int comet_hip_debug_masked_sum_registers(int *workgroup_kernel, int *
     if (!workgroup_kernel || !wavefront_kernel)
         return set_error(COMET_HIP_ERR_ARG, "null result pointer");
     hipFuncAttributes at;
-    COMET_HIPCHK(hipFuncGetAttributes(&at, reinterpret_cast<const void *>(spgemm_masked_sum_iso_kernel)));
+    COMET_HIPCHK(hipFuncGetAttributes(&at, reinterpret_cast<const void *>(pair_sum_heavy_kernel<true>)));
     *workgroup_kernel = at.numRegs;
-    COMET_HIPCHK(hipFuncGetAttributes(&at, reinterpret_cast<const void *>(spgemm_masked_sum_small_iso_kernel)));
+    COMET_HIPCHK(hipFuncGetAttributes(&at, reinterpret_cast<const void *>(pair_sum_light_kernel<true>)));
     *wavefront_kernel = at.numRegs;
     return COMET_HIP_OK;
 }

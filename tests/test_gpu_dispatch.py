@@ -85,3 +85,43 @@ def test_csr_goes_up_and_comes_back(n, mean, idt):
             wrong[-1] = bad
             with pytest.raises(rt.CometHipError, match="outside"):
                 rt.CsrMatrix.from_arrays((n, n), pos, wrong, val)
+
+
+def _rows(rng, n, lengths):
+    """A matrix whose first rows have the given lengths, columns drawn from all n."""
+    pos = np.concatenate([[0], np.cumsum(lengths), np.full(n - len(lengths), sum(lengths))]).astype(np.int64)
+    return pos, np.concatenate([np.sort(rng.choice(n, l, replace=False)) for l in lengths]).astype(np.int32)
+
+
+@pytest.mark.parametrize("only", [None, "workgroup", "wavefront"])
+@pytest.mark.parametrize("weights", [False, True])
+@pytest.mark.parametrize("double_b,double_m", [(False, False), (True, False), (False, True)])
+def test_masked_sum_of_every_list_and_table_length(only, weights, double_b, double_m, monkeypatch):
+    # lists around one quad, a row of 64 quads, a turn; tables around what a wavefront's holds; rows with pairs for one
+    # fetch and one more, and many; columns stored twice, where pairs may not change sides
+    if only:
+        monkeypatch.setenv("COMET_HIP_MASKED_SUM_ONLY", only)
+    n, rng = 6000, np.random.default_rng(5)
+    lengths = [1, 2, 3, 4, 5, 63, 64, 65, 191, 192, 193, 255, 256, 257, 511, 513, 1023, 1025, 2047, 2049, 4100] + [0, 7] * 60
+    bpos, bcrd = _rows(rng, n, lengths)
+    mpos, mcrd = _rows(rng, n, lengths[::-1])
+    apos, acrd = _rows(rng, n, [1, 64, 65, 129, 0, 900] * 24)
+    twice = lambda pos, crd: (2 * pos, np.repeat(crd, 2))
+    if double_b:
+        bpos, bcrd = twice(bpos, bcrd)
+    if double_m:
+        mpos, mcrd = twice(mpos, mcrd)
+    aval = rng.uniform(0.5, 1.5, len(acrd)) if weights else np.full(len(acrd), 0.25)
+    a, b, m = (apos, acrd, aval), (bpos, bcrd, np.full(len(bcrd), 1.5)), (mpos, mcrd, np.ones(len(mcrd)))
+    A, B, M = (rt.CsrMatrix.from_arrays((n, n), *x) for x in (a, b, m))
+    want = orc.reduce_sum(orc.spgemm(*a, *b, n, mask=(mpos, mcrd))[2])
+    got = [rt.spgemm_masked_sum(A, B, M) for _ in range(3)]
+    assert got[0] == got[1] == got[2] and abs(got[0] - want) <= 1e-12 * want
+
+
+@pytest.mark.parametrize("nnz", [0, 1, 3])
+def test_masked_sum_of_nearly_empty_matrices(nnz):
+    pos = np.array([0] + [nnz] * 5, np.int64)
+    x = (pos, np.arange(nnz, dtype=np.int32), np.ones(nnz))
+    A = rt.CsrMatrix.from_arrays((5, 5), *x)
+    assert rt.spgemm_masked_sum(A, A, A) == (nnz if nnz else 0)
