@@ -96,9 +96,8 @@ struct HeavyEnt {
 // their tickets over), kept in the left operand's handle: it depends only on the two structures, the row range and
 // the thresholds, so the seven lists a product of the benchmark takes are built once, not once per product.
 struct RowListEntry {
-    uint64_t b_uid = 0, mask_uid = 0, filter_uid = 0;
-    int64_t rb = 0, re = 0, dense_threshold = 0, wide_threshold = 0, mask_fill = 0, xlo = 0, xhi = 0;
-    int strict = 0;
+    uint64_t b_uid = 0, mask_uid = 0;
+    int64_t rb = 0, re = 0, dense_threshold = 0, wide_threshold = 0, mask_fill = 0;
     int32_t *rows = nullptr;     // device, re - rb entries
     int64_t *bounds = nullptr;   // device, 3 entries
 };
@@ -108,15 +107,17 @@ uint64_t next_csr_uid();
 // rows that have any as work items.
 struct PairSidePlan {
     int64_t first = 0, pairs = 0, nheavy = 0, nlight = 0;
-    int64_t *kpos = nullptr, *place = nullptr, *counts = nullptr;
+    int64_t *kpos = nullptr, *counts = nullptr;
+    uint32_t *place = nullptr;
     void *ent = nullptr, *heavy = nullptr;
-    double *weight = nullptr;
-    int32_t *light = nullptr, *padded = nullptr;
+    double *weight = nullptr, *padded = nullptr;
+    int32_t *light = nullptr;
 };
 struct PairPlan {
     uint64_t b_uid = 0, mask_uid = 0;
     int kind = 0;                // 0: product, 1: sum, 2 and 3: sum with every row sent one way
     int64_t first = 0, last = 0;
+    int64_t out0 = 0, outs = 0;  // product: the mask's entries of these rows
     PairSidePlan side[2];
 };
 void pair_plan_free(PairPlan &p);

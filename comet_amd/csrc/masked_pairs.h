@@ -26,7 +26,7 @@ struct PairSide {
     const int64_t *kpos;         // the pairs of row x: [kpos[x], kpos[x + 1])
     const PairEnt *ent;
     const double *weight;        // sum: A's value of the pair (null: one value for all, applied by the caller)
-    const int64_t *place;        // product: where the pair's result goes
+    const uint32_t *place;       // product: where the pair's result goes
     const int32_t *Lcrd;
     const double *Lval;
     uint32_t Lnnz;               // at least 4: a lane reads four columns at a time
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(256) void pair_pass(int64_t first, int64_t last, co
                                                  int64_t *__restrict__ kpos, int64_t *__restrict__ wpos,
                                                  PairEnt *__restrict__ ent, const double *__restrict__ Pval, double scale,
                                                  double *__restrict__ weight, const double *__restrict__ perm,
-                                                 int64_t out0, int64_t *__restrict__ place)
+                                                 int64_t out0, uint32_t *__restrict__ place)
 {
     constexpr int SEGS = PAIR_CHUNK / 64, PER = SEGS / 4;
     __shared__ int mark[PAIR_CHUNK];
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256) void pair_pass(int64_t first, int64_t last, co
                 if (weight)
                     weight[o] = Pval[p] * scale;
                 if (place)
-                    place[o] = (perm ? (int64_t)perm[p] : p) - out0;
+                    place[o] = (uint32_t)((perm ? (int64_t)perm[p] : p) - out0);
             }
         }
     }
@@ -312,6 +312,22 @@ __device__ __forceinline__ void wave_lds_order()
 
 constexpr int QUAD_MARKS = 32;           // bytes of LDS a wavefront's marks take at most, zero between walks
 
+// A row of 64 quads whose first lies at0 / 4 quads into the whole (at0: the lane's, four columns a quad): the list it
+// belongs to, where to read four columns that hold it - further in front than it begins where the array would end - and
+// which of the four are the list's; none where the quads have ended (there one place for all lanes is read).  m: the row's marks; before: lists that begin before
+// the row, less one.
+__device__ __forceinline__ void quad_place(uint2 m, uint32_t &before, int a0, int end, uint32_t at0, uint32_t most,
+                                           int &owner, uint32_t &from, uint32_t &mask)
+{
+    owner = (int)__builtin_amdgcn_mbcnt_hi(m.y, __builtin_amdgcn_mbcnt_lo(m.x, before));
+    before += __popc(m.x) + __popc(m.y);
+    const uint32_t at = (uint32_t)lane_value(a0, owner) + at0;
+    const int left = lane_value(end, owner) - (int)at;
+    from = left <= 0 ? 0u : at < most ? at : most;
+    const int n = left < 0 ? 0 : left < 4 ? left : 4;
+    mask = __builtin_amdgcn_ubfe(0xfu, 0, n) << ((at - from) & 31u);
+}
+
 // start, len, w: the lane's list and its weight; lanes without one (len 0) come after those with.  consume(turn) looks the
 // columns of a turn up; the last turn stays in `pend`, whose loads are under way when the next walk - of more lists,
 // against the same table - issues its own: the caller consumes it when there are no more.
@@ -348,19 +364,14 @@ __device__ __forceinline__ void quad_walk(QuadTurn<WEIGHTS, ROWS> &pend, uint32_
 #pragma unroll
         for (int r = 0; r < ROWS; ++r) {
             if (r < now.rows) {
-                const int owner = (int)__builtin_amdgcn_mbcnt_hi(m[r].y, __builtin_amdgcn_mbcnt_lo(m[r].x, before));
-                before += __popc(m[r].x) + __popc(m[r].y);
-                const uint32_t at = (uint32_t)lane_value(a0, owner) + at0 + 256u * r;
-                const int left = lane_value(end, owner) - (int)at;          // none where the quads have ended
+                int owner;
+                uint32_t from;
+                quad_place(m[r], before, a0, end, at0 + 256u * r, most, owner, from, now.mask[r]);
                 if constexpr (WEIGHTS) {
                     now.wlo[r] = lane_value(__double2loint(w), owner);
                     now.whi[r] = lane_value(__double2hiint(w), owner);
                 }
-                // four columns from `at` on, or from further in front where the array would end
-                const uint32_t b = at < most ? at : most;
-                const int n = left < 0 ? 0 : left < 4 ? left : 4;
-                now.q[r] = *reinterpret_cast<const sg_i4u *>(Lcrd + b);
-                now.mask[r] = __builtin_amdgcn_ubfe(0xfu, 0, n) << ((at - b) & 31u);
+                now.q[r] = *reinterpret_cast<const sg_i4u *>(Lcrd + from);
             }
         }
         wave_lds_order();
@@ -812,6 +823,10 @@ static int pair_ends(const Csr *x, int64_t first, int64_t last, int64_t *word, i
 }
 
 constexpr int64_t PAIR_ROOM_UNSEEN = 1 << 18;
+// From this number of pairs on the two kernels of a call run side by side: they leave each other room on the CUs, but the
+// second stream starts some 40 us late, which only longer walks make up for (sums: 134 us one after the other and 154 side
+// by side with 0.14 M pairs, 486 and 376 with 3.5 M, 1821 and 1648 with 15.6 M).
+constexpr int64_t PAIR_BESIDE = 1 << 20;
 
 // The plan of one side for rows [first, last) of T and P: built on the GPU.
 // val: P's values become weights (times scale), or null; places: the results' places are kept.
@@ -865,7 +880,7 @@ static int pair_side_plan(const Csr *T, const Csr *P, const Csr *L, int64_t firs
     if (weights)
         COMET_HIPCHK(dev_malloc((void **)&plan->weight, sizeof(double) * (size_t)(npairs > 0 ? npairs : 1)));
     if (places)
-        COMET_HIPCHK(dev_malloc((void **)&plan->place, sizeof(int64_t) * (size_t)(npairs > 0 ? npairs : 1)));
+        COMET_HIPCHK(dev_malloc((void **)&plan->place, sizeof(uint32_t) * (size_t)(npairs > 0 ? npairs : 1)));
     pair_pass<true><<<grid, block, 0, stream()>>>(first, last, T->pos, P->pos, P->crd, L->pos, strict, xlo, xhi, kept_before,
                                                   work_before, plan->kpos, wpos, (PairEnt *)plan->ent, P->val, scale,
                                                   plan->weight, perm, out0, plan->place);
@@ -880,9 +895,12 @@ static int pair_side_plan(const Csr *T, const Csr *P, const Csr *L, int64_t firs
     COMET_HIPCHK(dev_malloc((void **)&plan->light, sizeof(int32_t) * (size_t)(plan->nlight > 0 ? plan->nlight : 1)));
     pair_items<<<rows, block, 0, stream()>>>(first, n, parts, wpos, (uint2 *)plan->heavy, plan->light, plan->counts);
     if (L->nnz < 4) {          // a lane reads four columns at a time
-        COMET_HIPCHK(dev_malloc((void **)&plan->padded, 4 * sizeof(int32_t)));
-        COMET_HIPCHK(hipMemsetAsync(plan->padded, 0, 4 * sizeof(int32_t), stream()));
-        COMET_HIPCHK(hipMemcpyAsync(plan->padded, L->crd, sizeof(int32_t) * (size_t)L->nnz, hipMemcpyDeviceToDevice, stream()));
+        constexpr size_t room = 4 * (sizeof(double) + sizeof(int32_t));
+        COMET_HIPCHK(dev_malloc((void **)&plan->padded, room));
+        COMET_HIPCHK(hipMemsetAsync(plan->padded, 0, room, stream()));
+        COMET_HIPCHK(hipMemcpyAsync(plan->padded, L->val, sizeof(double) * (size_t)L->nnz, hipMemcpyDeviceToDevice, stream()));
+        COMET_HIPCHK(hipMemcpyAsync(plan->padded + 4, L->crd, sizeof(int32_t) * (size_t)L->nnz, hipMemcpyDeviceToDevice,
+                                    stream()));
     }
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
@@ -898,8 +916,8 @@ static PairSide pair_side(const PairSidePlan &p, const Csr *T, const Csr *L)
     s.ent = (const PairEnt *)p.ent;
     s.weight = p.weight;
     s.place = p.place;
-    s.Lcrd = p.padded ? p.padded : L->crd;
-    s.Lval = L->val;
+    s.Lcrd = p.padded ? reinterpret_cast<const int32_t *>(p.padded + 4) : L->crd;
+    s.Lval = p.padded ? p.padded : L->val;
     s.Lnnz = p.padded ? 4u : (uint32_t)L->nnz;
     s.heavy = (const uint2 *)p.heavy;
     s.light = p.light;
@@ -1032,10 +1050,7 @@ static int pair_masked_sum(Csr *a, Csr *b, Csr *m, double *result)
         out = (double *)g_pair_out.ptr;
         partial = (double *)g_pair_partial.ptr;
     }
-    // The two kernels leave each other room on the CUs; but the second stream starts some 40 us late, which only
-    // longer walks make up for (134 us one after the other and 154 side by side with 0.14 M pairs, 486 and 376 with
-    // 3.5 M, 1821 and 1648 with 15.6 M).
-    const bool beside = nheavy > 0 && nlight > 0 && plan->side[0].pairs + plan->side[1].pairs >= 1 << 20;
+    const bool beside = nheavy > 0 && nlight > 0 && plan->side[0].pairs + plan->side[1].pairs >= PAIR_BESIDE;
     if (beside)
         COMET_CHK(aux_fork());
     if (nheavy > 0) {

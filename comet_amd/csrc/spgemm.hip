@@ -1001,28 +1001,21 @@ constexpr size_t SG_DENSE_LDS = (size_t)SG_CB * 8 + (size_t)SG_CB / 8 + (size_t)
 static_assert(((size_t)SG_CB * 8) % 8 == 0 && ((size_t)SG_CB / 8) % 4 == 0 && ((size_t)SG_EMIT * sizeof(emit_t)) % 4 == 0,
               "the one-block kernel's LDS regions are aligned for their types");
 
-// products[i - row_begin] = sum over k in A_i of nnz(B_k); one wavefront per row.  With Tpos (the dot-product form of
-// a masked product, where row i's pairs k are shared out by which of the two lists is longer) only the k whose row
-// of B is shorter than row i of T (strict) or not longer (otherwise), and that lie in [xlo, xhi), count.
+// products[i - row_begin] = sum over k in A_i of nnz(B_k); one wavefront per row.
 __global__ __launch_bounds__(256) void spgemm_row_products(int64_t row_begin, int64_t row_end,
                                                            const int64_t *__restrict__ Apos,
                                                            const int32_t *__restrict__ Acrd,
                                                            const int64_t *__restrict__ Bpos,
-                                                           int64_t *__restrict__ products,
-                                                           const int64_t *__restrict__ Tpos = nullptr, int strict = 0,
-                                                           int64_t xlo = 0, int64_t xhi = 0)
+                                                           int64_t *__restrict__ products)
 {
     const int64_t i = row_begin + (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (i >= row_end)
         return;
     const int lane = threadIdx.x & 63;
-    const int64_t tlen = Tpos ? Tpos[i + 1] - Tpos[i] : 0;
     int64_t s = 0;
     for (int64_t p = Apos[i] + lane; p < Apos[i + 1]; p += 64) {
         const int k = Acrd[p];
-        const int64_t len = Bpos[k + 1] - Bpos[k];
-        if (!Tpos || ((strict ? len < tlen : len <= tlen) && k >= xlo && k < xhi))
-            s += len;
+        s += Bpos[k + 1] - Bpos[k];
     }
     for (int d = 32; d > 0; d >>= 1)
         s += __shfl_down(s, d, 64);
@@ -2364,384 +2357,11 @@ __global__ void eltwise_mult_dense_kernel(int64_t nrows, const int64_t *__restri
 // row i of A and column j of B; walking the products of row i (every entry of every B_k, k in A_i) costs |B_k|
 // look-ups per entry of A_i whatever the mask holds, the dot product of a stored pair (i, j) costs the shorter of
 // its two lists when that one is streamed against a table of the longer one.  So the pairs of the mask are split
-// by which list is longer.  One kernel serves both halves: a workgroup takes a row x of a matrix of pairs P,
-// puts the list T_x into its table, and for the pairs (x, y) of P_x that are its to do streams the list L_y
-// through the table.
+// by which list is longer, and for every row x of a matrix of pairs P the list T_x goes into a table that the lists
+// L_y of the pairs (x, y) of that half are streamed against (masked_dots.h).
 //   the row's half:     P = M,   T = A (rows),            L = B^T (columns of B);  pair (i, j) when |B^T_j| <= |A_i|
 //   the column's half:  P = M^T, T = B^T (columns of B),  L = A (rows);            pair (j, i) when |A_i| < |B^T_j|
-// The table is a bitmap over k in LDS with the number of set bits before every eighth word, so that a hit knows
-// its rank in T_x and with it where the value lies (a list in the table must not hold a column twice).  A pair's
-// products are added into a slot of LDS that belongs to the wavefront and the pair (64 pairs per wavefront at a
-// time) and leave, with the flag that says whether there was any, when the wavefront is through with its 64.
 // ---------------------------------------------------------------------------
-struct DotHit {
-    int hit;
-    double prod;
-};
-constexpr int DT_GROUP = 16;         // bitmap words per count
-constexpr int DT_WPT = 32;           // consecutive bitmap words a thread counts: SG_T * DT_WPT * 32 = 2^20 columns at most
-// The table of a list of at most SG_HASH_FILL entries is a hash table instead, key k + 1 and the value, in the same
-// LDS: nothing to count, and building and clearing it costs by the length of the list, not of the bitmap.
-// Words of LDS in front of the wavefronts' sums: the bitmap (one padding word after every 32, so that a thread's
-// 32 consecutive words lie in 32 banks) and the counts, or the hash table's keys and values, whichever is more
-constexpr int dot_bitmap_words(int words) { return words + words / 32 + words / DT_GROUP; }
-constexpr int dot_table_words(int words)
-{
-    return ((dot_bitmap_words(words) > 3 * SG_HASH_SLOTS ? dot_bitmap_words(words) : 3 * SG_HASH_SLOTS) + 1) & ~1;
-}
-constexpr size_t dot_lds_bytes(int words)
-{
-    return (size_t)dot_table_words(words) * 4 + (size_t)SG_WAVES * 64 * (8 + 4);
-}
-static_assert(dot_lds_bytes(SG_T * DT_WPT) <= 160 * 1024 - 256, "the table of 2^20 columns fits LDS");
-// the fp64 regions of the dot-product kernel: the hash table's values SG_HASH_SLOTS words in, the wavefronts' sums
-// dot_table_words(words) words in, for every table size the host can ask for (a multiple of DT_WPT words)
-constexpr bool dot_fp64_regions_aligned()
-{
-    if (SG_HASH_SLOTS % 2 != 0)
-        return false;
-    for (int w = DT_WPT; w <= SG_T * DT_WPT; w += DT_WPT)
-        if (dot_table_words(w) % 2 != 0)
-            return false;
-    return true;
-}
-static_assert(dot_fp64_regions_aligned(), "an fp64 region of the dot-product kernel's LDS is not 8-byte aligned");
-
-// The pairs [ms, me) of one row of P, dealt to the wavefronts like the entries of a row of A in
-// for_each_product_impl (the walk of a turn and its one-turn-late visits are the same); keep(y, len) says whether
-// a pair is this half's; f gets the pair's slot in the wavefront's batch; done(base, cnt, kept) ends a batch.
-// With VALUES the entries' values are loaded with their columns and handed to mid: in these products a fifth of the
-// look-ups hit, so nearly every cache line of the values is needed anyway, and fetched only for the hits they would
-// be a second trip to memory behind the first.
-// Without VALUES only whether a pair meets a product is asked, and decided(t) says that pair t of the wavefront's
-// batch already has: the rest of its list is then left out (a long list is through after a turn or two).
-template <bool VALUES, typename KEEP, typename PRE, typename MID, typename F, typename DONE, typename DECIDED>
-__device__ inline void for_each_pair(int64_t ms, int64_t me, const int32_t *__restrict__ Pcrd,
-                                     const int64_t *__restrict__ Lpos, const int32_t *__restrict__ Lcrd,
-                                     const double *__restrict__ Lval, KEEP keep, PRE pre, MID mid, F f, DONE done,
-                                     DECIDED decided)
-{
-    using T1 = decltype(pre(0));
-    using T2 = decltype(mid(0, 0.0, T1()));
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int quarter = lane >> 4, sub = lane & 15;
-    constexpr int NP = FEP_LONG_LOADS > FEP_SHORT_LOADS ? FEP_LONG_LOADS : FEP_SHORT_LOADS;
-    bool w_ok[NP];
-    int w_t[NP];
-    T2 w_md[NP];
-#pragma unroll
-    for (int x = 0; x < NP; ++x)
-        w_ok[x] = false;
-    const auto visit_pending = [&]() {
-#pragma unroll
-        for (int x = 0; x < NP; ++x)
-            if (w_ok[x])
-                f(w_t[x], w_md[x]);
-#pragma unroll
-        for (int x = 0; x < NP; ++x)
-            w_ok[x] = false;
-    };
-    const auto turn = [&](auto n_tag, const bool *ok, const int *k, const double *v, int t) {
-        constexpr int N = decltype(n_tag)::value;
-        T1 tk[N];
-#pragma unroll
-        for (int x = 0; x < N; ++x)
-            tk[x] = ok[x] ? pre(k[x]) : T1();
-        visit_pending();
-#pragma unroll
-        for (int x = 0; x < N; ++x) {
-            w_ok[x] = ok[x];
-            w_t[x] = t;
-            w_md[x] = ok[x] ? mid(k[x], v[x], tk[x]) : T2();
-        }
-    };
-    for (int64_t base = ms + wave; base < me; base += (int64_t)SG_WAVES * 64) {
-        const int64_t left = (me - base + SG_WAVES - 1) / SG_WAVES;     // my pairs from here on
-        const int cnt = (int)(left < 64 ? left : 64);
-        int64_t bs = 0, be = 0;
-        bool kept = false;
-        if (lane < cnt) {
-            const int y = Pcrd[base + (int64_t)lane * SG_WAVES];
-            bs = Lpos[y];
-            be = Lpos[y + 1];
-            kept = keep(y, be - bs);
-            if (!kept)
-                be = bs;
-        }
-        unsigned long long big = __ballot(be - bs >= FEP_SHORT);
-        unsigned long long todo = __ballot(bs < be && be - bs < FEP_SHORT);
-        while (big) {
-            const int t = __builtin_ctzll(big);
-            big &= big - 1;
-            const int64_t s = readlane_i64(bs, t), len = readlane_i64(be, t) - s;
-            int64_t o = lane;
-            if (len >= 64 * FEP_LONG_LOADS) {
-                bool all[FEP_LONG_LOADS];
-                int k[FEP_LONG_LOADS];
-                double v[FEP_LONG_LOADS];
-#pragma unroll
-                for (int x = 0; x < FEP_LONG_LOADS; ++x) {
-                    all[x] = true;
-                    k[x] = Lcrd[s + o + 64 * x];
-                    v[x] = VALUES ? Lval[s + o + 64 * x] : 0.0;
-                }
-                bool enough = false;
-                for (int64_t full = 64 * FEP_LONG_LOADS; full + 64 * FEP_LONG_LOADS <= len;
-                     full += 64 * FEP_LONG_LOADS) {
-                    if (!VALUES && decided(t)) {        // what earlier turns found (a turn's visits come one turn late)
-                        enough = true;
-                        break;
-                    }
-                    int kn[FEP_LONG_LOADS];
-                    double vn[FEP_LONG_LOADS];
-#pragma unroll
-                    for (int x = 0; x < FEP_LONG_LOADS; ++x) {
-                        kn[x] = Lcrd[s + o + 64 * (FEP_LONG_LOADS + x)];
-                        vn[x] = VALUES ? Lval[s + o + 64 * (FEP_LONG_LOADS + x)] : 0.0;
-                    }
-                    turn(std::integral_constant<int, FEP_LONG_LOADS>(), all, k, v, t);
-#pragma unroll
-                    for (int x = 0; x < FEP_LONG_LOADS; ++x) {
-                        k[x] = kn[x];
-                        v[x] = vn[x];
-                    }
-                    o += 64 * FEP_LONG_LOADS;
-                }
-                turn(std::integral_constant<int, FEP_LONG_LOADS>(), all, k, v, t);
-                o += 64 * FEP_LONG_LOADS;
-                if (enough)
-                    o = len;
-            }
-            if (o < len && (VALUES || !decided(t))) {
-                bool ok[FEP_LONG_LOADS];
-                int k[FEP_LONG_LOADS];
-                double v[FEP_LONG_LOADS];
-#pragma unroll
-                for (int x = 0; x < FEP_LONG_LOADS; ++x)
-                    ok[x] = o + 64 * x < len;
-#pragma unroll
-                for (int x = 0; x < FEP_LONG_LOADS; ++x)
-                    k[x] = ok[x] ? Lcrd[s + o + 64 * x] : 0;
-#pragma unroll
-                for (int x = 0; x < FEP_LONG_LOADS; ++x)
-                    v[x] = VALUES && ok[x] ? Lval[s + o + 64 * x] : 0.0;
-                turn(std::integral_constant<int, FEP_LONG_LOADS>(), ok, k, v, t);
-            }
-        }
-        while (todo) {
-            int pick = -1;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int t = todo ? __builtin_ctzll(todo) : -1;
-                todo = todo ? (todo & (todo - 1)) : 0;
-                pick = quarter == g ? t : pick;
-            }
-            const int src = pick < 0 ? lane : pick;
-            const int64_t s = ((int64_t)__shfl((int)(bs >> 32), src, 64) << 32) |
-                              (uint32_t)__shfl((int)(bs & 0xffffffff), src, 64);
-            const int64_t e = ((int64_t)__shfl((int)(be >> 32), src, 64) << 32) |
-                              (uint32_t)__shfl((int)(be & 0xffffffff), src, 64);
-            bool ok[FEP_SHORT_LOADS];
-            int k[FEP_SHORT_LOADS];
-            double v[FEP_SHORT_LOADS];
-#pragma unroll
-            for (int x = 0; x < FEP_SHORT_LOADS; ++x)
-                ok[x] = pick >= 0 && s + sub + 16 * x < e;
-#pragma unroll
-            for (int x = 0; x < FEP_SHORT_LOADS; ++x)
-                k[x] = ok[x] ? Lcrd[s + sub + 16 * x] : 0;
-#pragma unroll
-            for (int x = 0; x < FEP_SHORT_LOADS; ++x)
-                v[x] = VALUES && ok[x] ? Lval[s + sub + 16 * x] : 0.0;
-            turn(std::integral_constant<int, FEP_SHORT_LOADS>(), ok, k, v, src);
-        }
-        visit_pending();
-        done(base, cnt, kept);
-    }
-}
-
-// strict: a pair is kept when its streamed list is shorter than the table's (otherwise: not longer).  [xlo, xhi):
-// the pairs' other index must lie in it (the rows of M being computed, for the column's half).  perm: where pair p
-// of P lies in the row-major order of the mask (nullptr: at p); out0 is taken off either.
-// SEMI: another semiring than plus-times (reduce plus, min or max; `any` keeps the place of a product in B, which
-// this form does not have): a product is mult(a, b) with a the entry of A - the table's in the row's half, the
-// streamed one in the column's (swapped) - and a pair's slot holds a sum or the key of a minimum or maximum.
-template <bool VALUES, bool SEMI>
-__global__ __launch_bounds__(SG_T) void spgemm_dot_kernel(
-    int64_t row_begin, const int64_t *__restrict__ Tpos, const int32_t *__restrict__ Tcrd,
-    const double *__restrict__ Tval, const int64_t *__restrict__ Ppos, const int32_t *__restrict__ Pcrd,
-    const int64_t *__restrict__ Lpos, const int32_t *__restrict__ Lcrd, const double *__restrict__ Lval,
-    const double *__restrict__ perm, int64_t out0, int strict, int64_t xlo, int64_t xhi, int words,
-    unsigned long long *ticket, RowList list, double *__restrict__ pair_val, uint8_t *__restrict__ pair_hit,
-    int reduce_op, int mult_op, int swapped)
-{
-    __shared__ int64_t row_slot;
-    __shared__ int wave_tot[SG_WAVES];
-    uint32_t *bm = sg_dyn_lds;
-    uint32_t *cnt_before = bm + words + words / 32;    // [words / DT_GROUP]
-    uint32_t *hkey = sg_dyn_lds;                       // [SG_HASH_SLOTS], over the bitmap
-    double *hval = reinterpret_cast<double *>(sg_dyn_lds + SG_HASH_SLOTS);        // [SG_HASH_SLOTS]
-    const int table_words = dot_table_words(words);
-    double *wacc = reinterpret_cast<double *>(sg_dyn_lds + table_words);           // [SG_WAVES][64]
-    int *whit = reinterpret_cast<int *>(wacc + SG_WAVES * 64);                     // [SG_WAVES][64]
-    const BmAddr ad{5};
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    for (int w = threadIdx.x; w < table_words; w += SG_T)
-        sg_dyn_lds[w] = 0;
-    wacc[threadIdx.x] = 0.0;
-    whit[threadIdx.x] = 0;
-    lds_barrier();
-    bool values_left = false;       // a hash table's values lie where bitmap words are: cleared before the next bitmap
-    int64_t t_first, t_end;
-    list_range(list, 2, &t_first, &t_end);
-    int64_t tk = draw_row<true>(ticket, t_first, &row_slot);
-    while (tk < t_end) {
-        const int64_t x = row_begin + list.rows[tk];
-        const int64_t ts = Tpos[x], te = Tpos[x + 1];
-        const int64_t ps = Ppos[x], pe = Ppos[x + 1];
-        const int64_t tlen = te - ts;
-        const auto keep = [&](int y, int64_t len) {
-            return len > 0 && (strict ? len < tlen : len <= tlen) && y >= xlo && y < xhi;
-        };
-        const auto add = [&](int t, DotHit h) {
-            if (h.hit) {
-                whit[wave * 64 + t] = 1;
-                if constexpr (VALUES && SEMI) {
-                    if (reduce_op == SR_PLUS)
-                        __hip_atomic_fetch_add(&wacc[wave * 64 + t], h.prod, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    else
-                        __hip_atomic_fetch_max(reinterpret_cast<unsigned long long *>(&wacc[wave * 64 + t]),
-                                               reduce_op == SR_MIN ? ~f64_key(h.prod) : f64_key(h.prod), __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_WORKGROUP);
-                } else if constexpr (VALUES) {
-                    __hip_atomic_fetch_add(&wacc[wave * 64 + t], h.prod, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                }
-            }
-        };
-        // tv: the table's value, lv: the streamed entry's
-        const auto product = [&](double tv, double lv) {
-            if constexpr (SEMI)
-                return swapped ? semiring_mult(mult_op, lv, tv) : semiring_mult(mult_op, tv, lv);
-            else
-                return tv * lv;
-        };
-        // (uniform: t is; a wavefront's own LDS operations keep their order)
-        const auto decided = [&](int t) { return __builtin_amdgcn_readfirstlane(whit[wave * 64 + t]) != 0; };
-        const auto done = [&](int64_t base, int cnt, bool kept) {
-            // the slots belong to this wavefront, which has issued all its adds: LDS keeps a wavefront's order
-            if (lane < cnt && kept) {
-                const int64_t p = base + (int64_t)lane * SG_WAVES;
-                const int64_t at = (perm ? (int64_t)perm[p] : p) - out0;
-                pair_hit[at] = (uint8_t)whit[wave * 64 + lane];
-                if constexpr (VALUES && SEMI)
-                    pair_val[at] = semiring_lds_value(reinterpret_cast<unsigned long long *>(wacc)[wave * 64 + lane],
-                                                      reduce_op, mult_op, 0, nullptr, nullptr);
-                else if constexpr (VALUES)
-                    pair_val[at] = wacc[wave * 64 + lane];
-            }
-            wacc[wave * 64 + lane] = 0.0;
-            whit[wave * 64 + lane] = 0;
-        };
-        if (ts != te && ps != pe && tlen <= SG_HASH_FILL) {
-            for (int64_t t = ts + threadIdx.x; t < te; t += SG_T) {
-                const int k = Tcrd[t];
-                const uint32_t key = (uint32_t)k + 1u;
-                uint32_t sl = sg_hash_slot(k);
-                for (;;) {
-                    const uint32_t old = atomicCAS(&hkey[sl], 0u, key);
-                    if (old == 0u)
-                        break;
-                    sl = (sl + 1) & (SG_HASH_SLOTS - 1);
-                }
-                if constexpr (VALUES)
-                    hval[sl] = Tval[t];
-            }
-            values_left = VALUES;
-            lds_barrier();
-            for_each_pair<VALUES>(ps, pe, Pcrd, Lpos, Lcrd, Lval, keep,
-                [&](int k) { return hkey[sg_hash_slot(k)]; },
-                [&](int k, double lv, uint32_t k0) {
-                    DotHit h{0, 0.0};
-                    if (k0 != 0u) {
-                        uint32_t sl = sg_hash_slot(k);
-                        uint32_t key = k0;
-                        while (key != 0u && key != (uint32_t)k + 1u) {
-                            sl = (sl + 1) & (SG_HASH_SLOTS - 1);
-                            key = hkey[sl];
-                        }
-                        if (key != 0u) {
-                            h.hit = 1;
-                            if constexpr (VALUES)
-                                h.prod = product(hval[sl], lv);
-                        }
-                    }
-                    return h;
-                }, add, done, decided);
-            lds_barrier();
-            for (int sl = threadIdx.x; sl < SG_HASH_SLOTS; sl += SG_T)
-                hkey[sl] = 0u;
-        } else if (ts != te && ps != pe) {
-            if (values_left) {
-                for (int w = SG_HASH_SLOTS + threadIdx.x; w < 3 * SG_HASH_SLOTS; w += SG_T)
-                    sg_dyn_lds[w] = 0;
-                values_left = false;
-                lds_barrier();
-            }
-            for (int64_t t = ts + threadIdx.x; t < te; t += SG_T) {
-                const int k = Tcrd[t];
-                atomicOr(&bm[ad.word(k)], ad.bit(k));
-            }
-            lds_barrier();
-            {   // bits before every group of words: a thread counts DT_WPT consecutive words
-                const int w0 = (int)threadIdx.x * DT_WPT;
-                int mine = 0;
-                if (w0 < words) {
-#pragma unroll
-                    for (int c = 0; c < DT_WPT; ++c)
-                        mine += __popc(bm[w0 + c + (w0 >> 5)]);
-                }
-                const int inc = wave_inclusive_scan(mine);
-                if (lane == 63)
-                    wave_tot[wave] = inc;
-                lds_barrier();
-                const int tots = wave_inclusive_scan(lane < SG_WAVES ? wave_tot[lane] : 0);
-                int run = (wave ? __builtin_amdgcn_readlane(tots, wave - 1) : 0) + inc - mine;
-                if (w0 < words) {
-#pragma unroll
-                    for (int c = 0; c < DT_WPT; ++c) {
-                        if (c % DT_GROUP == 0)
-                            cnt_before[(w0 + c) / DT_GROUP] = (uint32_t)run;
-                        run += __popc(bm[w0 + c + (w0 >> 5)]);
-                    }
-                }
-                lds_barrier();
-            }
-            for_each_pair<VALUES>(ps, pe, Pcrd, Lpos, Lcrd, Lval, keep,
-                [&](int k) { return bm[ad.word(k)]; },
-                [&](int k, double lv, uint32_t word) {
-                    DotHit h{0, 0.0};
-                    if (word & ad.bit(k)) {
-                        h.hit = 1;
-                        if constexpr (VALUES) {
-                            const int w = k >> 5, wg = w & ~(DT_GROUP - 1);
-                            int rank = (int)cnt_before[w / DT_GROUP] + __popc(word & (ad.bit(k) - 1u));
-                            for (int v = wg; v < w; ++v)
-                                rank += __popc(bm[v + (v >> 5)]);
-                            h.prod = product(Tval[ts + rank], lv);
-                        }
-                    }
-                    return h;
-                }, add, done, decided);
-            lds_barrier();
-            for (int64_t t = ts + threadIdx.x; t < te; t += SG_T)
-                bm[ad.word(Tcrd[t])] = 0;
-        }
-        tk = draw_row<true>(ticket, t_first, &row_slot);      // its barriers also close this row's clean-up
-    }
-}
-
 // rowcount[i - rb] = stored pairs of mask row i that met a product
 __global__ __launch_bounds__(256) void spgemm_dot_count(int64_t rb, int64_t re, const int64_t *__restrict__ Mpos,
                                                         const uint8_t *__restrict__ pair_hit,
@@ -2758,33 +2378,6 @@ __global__ __launch_bounds__(256) void spgemm_dot_count(int64_t rb, int64_t re, 
     n = wave_sum_i32(n);
     if (lane == 0)
         rowcount[i - rb] = n;
-}
-
-// the pairs that met a product, in the order of the mask row, to the place Cpos gives the row
-__global__ __launch_bounds__(256) void spgemm_dot_compact(int64_t rb, int64_t re, const int64_t *__restrict__ Mpos,
-                                                          const int32_t *__restrict__ Mcrd,
-                                                          const double *__restrict__ pair_val,
-                                                          const uint8_t *__restrict__ pair_hit,
-                                                          const int64_t *__restrict__ Cpos, int32_t *__restrict__ Ccrd,
-                                                          double *__restrict__ Cval)
-{
-    const int64_t i = rb + (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i >= re)
-        return;
-    const int lane = threadIdx.x & 63;
-    const int64_t in0 = Mpos[rb];
-    int64_t at = Cpos[i] - Cpos[rb];
-    for (int64_t base = Mpos[i]; base < Mpos[i + 1]; base += 64) {
-        const int64_t p = base + lane;
-        const bool hit = p < Mpos[i + 1] && pair_hit[p - in0];
-        const unsigned long long m = __ballot(hit);
-        if (hit) {
-            const int64_t o = at + __popcll(m & ((1ull << lane) - 1ull));
-            Ccrd[o] = Mcrd[p];
-            Cval[o] = pair_val[p - in0];
-        }
-        at += __popcll(m);
-    }
 }
 
 // flag[0] |= 1 when a row holds a column twice (rows are sorted); a wavefront per row
@@ -2916,11 +2509,6 @@ struct SgRowLists {
 static SgRowLists g_rl;
 
 // Products per row of rows [rb, re) of A*B and the list of those rows by descending products.
-struct SgPairFilter {          // see spgemm_row_products
-    const Csr *towner = nullptr;        // tpos = towner->pos
-    int strict = 0;
-    int64_t xlo = 0, xhi = 0;
-};
 // The list depends on the two structures, the range and the thresholds only: it is kept in A's handle and found
 // again by the uids of the matrices it was made from (a matrix gets a new uid when it is invalidated), so a
 // product that is taken again, or taken in row blocks, sorts nothing.  COMET_HIP_SPGEMM_NO_LIST_CACHE turns the
@@ -2928,7 +2516,7 @@ struct SgPairFilter {          // see spgemm_row_products
 constexpr size_t SG_ROW_LISTS_KEPT = 24;
 static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64_t dense_threshold,
                        int64_t wide_threshold, RowList *out, const Csr *long_mask = nullptr,
-                       int64_t mask_fill = 0, SgPairFilter filter = SgPairFilter())
+                       int64_t mask_fill = 0)
 {
     const int64_t n = re - rb;
     static const bool keep = getenv("COMET_HIP_SPGEMM_NO_LIST_CACHE") == nullptr;
@@ -2936,20 +2524,15 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
     RowListEntry key;
     key.b_uid = b->uid;
     key.mask_uid = long_mask ? long_mask->uid : 0;
-    key.filter_uid = filter.towner ? filter.towner->uid : 0;
     key.rb = rb;
     key.re = re;
     key.dense_threshold = dense_threshold;
     key.wide_threshold = wide_threshold;
     key.mask_fill = mask_fill;
-    key.xlo = filter.xlo;
-    key.xhi = filter.xhi;
-    key.strict = filter.strict;
     if (keep)
         for (const RowListEntry &e : owner->row_lists)
-            if (e.b_uid == key.b_uid && e.mask_uid == key.mask_uid && e.filter_uid == key.filter_uid && e.rb == rb &&
-                e.re == re && e.dense_threshold == dense_threshold && e.wide_threshold == wide_threshold &&
-                e.mask_fill == mask_fill && e.xlo == key.xlo && e.xhi == key.xhi && e.strict == key.strict) {
+            if (e.b_uid == key.b_uid && e.mask_uid == key.mask_uid && e.rb == rb && e.re == re &&
+                e.dense_threshold == dense_threshold && e.wide_threshold == wide_threshold && e.mask_fill == mask_fill) {
                 out->rows = e.rows;
                 out->bounds = e.bounds;
                 return COMET_HIP_OK;
@@ -2964,8 +2547,7 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
     {
         KernelTimer t("spgemm_row_products");
         spgemm_row_products<<<dim3((unsigned)ceil_div(n, 4)), dim3(256), 0, stream()>>>(
-            rb, re, a->pos, a->crd, b->pos, rowprod, filter.towner ? filter.towner->pos : nullptr, filter.strict,
-            filter.xlo, filter.xhi);
+            rb, re, a->pos, a->crd, b->pos, rowprod);
         sg_row_keys<<<dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, stream()>>>(
             n, rowprod, long_mask ? long_mask->pos + rb : nullptr, mask_fill, (uint64_t *)g_rl.keys_in.ptr,
             (uint32_t *)g_rl.idx_in.ptr);
@@ -3004,8 +2586,8 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
 constexpr int64_t SG_NO_DENSE = 1ll << 61;     // a threshold no row reaches: every row stays on the slab path
 
 static int dot_form_fits(const Csr *a, const Csr *b, const Csr *m, bool *fits);
-static int dot_pairs(const Csr *a, const Csr *b, const Csr *m, int64_t rb, int64_t re, bool values, double **pair_val,
-                     uint8_t **pair_hit, int reduce_op = COMET_SR_PLUS, int mult_op = COMET_OP_TIMES);
+static int pair_dot_values(Csr *a, Csr *b, Csr *m, int64_t rb, int64_t re, double **pair_val, uint8_t **pair_hit,
+                           int64_t *pairs, int reduce_op, int mult_op);
 
 static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *rowcount)
 {
@@ -3014,7 +2596,9 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
     if (dots) {         // a masked product: which stored pairs of the mask meet a product
         double *pair_val = nullptr;
         uint8_t *pair_hit = nullptr;
-        COMET_CHK(dot_pairs(a, b, m, 0, a->nrows, false, &pair_val, &pair_hit));
+        int64_t pairs = 0;
+        COMET_CHK(pair_dot_values(const_cast<Csr *>(a), const_cast<Csr *>(b), const_cast<Csr *>(m), 0, a->nrows, &pair_val,
+                                  &pair_hit, &pairs, COMET_SR_PLUS, COMET_OP_TIMES));
         KernelTimer t("spgemm_symbolic_dot_count");
         spgemm_dot_count<<<dim3((unsigned)ceil_div(a->nrows, 4)), dim3(256), 0, stream()>>>(0, a->nrows, m->pos, pair_hit,
                                                                                             rowcount);
@@ -3186,13 +2770,15 @@ static int csr_is_iso(const Csr *x, bool *iso)
 }
 
 #include "masked_pairs.h"
+#include "masked_dots.h"
 
 // A masked product runs as dot products when the table over k fits LDS and no list that goes into a table holds a
 // column twice.  COMET_HIP_SPGEMM_NO_DOT keeps the walk over the products of every row (the tests run both).
 static int dot_form_fits(const Csr *a, const Csr *b, const Csr *m, bool *fits)
 {
     *fits = false;
-    if (!m || a->ncols > (1ll << 20) || a->nrows >= (1ll << 31) || b->ncols >= (1ll << 31) || m->nnz >= (1ll << 52) ||
+    if (!m || a->ncols > (1ll << 20) || a->nrows >= (1ll << 31) || b->ncols >= (1ll << 31) || m->nnz > PAIR_NNZ_MAX || a->nnz > PAIR_NNZ_MAX ||
+        b->nnz > PAIR_NNZ_MAX ||
         getenv("COMET_HIP_SPGEMM_NO_DOT") != nullptr)
         return COMET_HIP_OK;
     bool ok_a = false, ok_b = false, ok_m = false;
@@ -3200,70 +2786,6 @@ static int dot_form_fits(const Csr *a, const Csr *b, const Csr *m, bool *fits)
     COMET_CHK(dot_no_duplicates(b, &ok_b));
     COMET_CHK(dot_no_duplicates(m, &ok_m));
     *fits = ok_a && ok_b && ok_m;
-    return COMET_HIP_OK;
-}
-
-// pair_hit[p - Mpos[rb]] (and pair_val, with values) for every stored pair p of the mask rows [rb, re)
-static int dot_pairs(const Csr *a, const Csr *b, const Csr *m, int64_t rb, int64_t re, bool values, double **pair_val,
-                     uint8_t **pair_hit, int reduce_op, int mult_op)
-{
-    const bool semi = reduce_op != COMET_SR_PLUS || mult_op != COMET_OP_TIMES;
-    Csr *bt = nullptr, *mt = nullptr;
-    COMET_CHK(dot_transposed(b, &bt));
-    COMET_CHK(dot_transposed_index(m, &mt));
-    int64_t ends[2] = {0, 0};
-    COMET_HIPCHK(hipMemcpyAsync(&ends[0], m->pos + rb, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
-    COMET_HIPCHK(hipMemcpyAsync(&ends[1], m->pos + re, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
-    COMET_CHK(stream_wait());
-    const int64_t out0 = ends[0], npairs = ends[1] - ends[0];
-    COMET_CHK(g_dot_hit.ensure((size_t)(npairs > 0 ? npairs : 1), false));
-    COMET_CHK(g_dot_val.ensure(sizeof(double) * (size_t)(npairs > 0 ? npairs : 1), false));
-    *pair_hit = (uint8_t *)g_dot_hit.ptr;
-    *pair_val = (double *)g_dot_val.ptr;
-    if (npairs == 0)
-        return COMET_HIP_OK;
-    COMET_HIPCHK(hipMemsetAsync(*pair_hit, 0, (size_t)npairs, stream()));
-    if (values)
-        COMET_HIPCHK(hipMemsetAsync(*pair_val, 0, sizeof(double) * (size_t)npairs, stream()));
-    int words = (int)ceil_div(a->ncols > 0 ? a->ncols : 1, 32);
-    words = (int)ceil_div(words, DT_WPT) * DT_WPT;
-    const size_t lds = dot_lds_bytes(words);
-    if (dot_table_words(words) % 2 != 0 || words % DT_WPT != 0)        // the wavefronts' fp64 sums follow the table
-        return set_error(COMET_HIP_ERR_SIZE, "dot-product table of %d words leaves its sums misaligned", words);
-    const dim3 grid((unsigned)(num_cus() > 0 ? num_cus() : 256)), block(SG_T);
-    const int64_t everywhere = 1ll << 62;
-    for (int half = 0; half < 2; ++half) {
-        // the row's half: tables of the rows of A, the columns of B streamed; the column's half the other way round
-        const Csr *T = half == 0 ? a : bt, *P = half == 0 ? m : mt, *L = half == 0 ? bt : a;
-        const int64_t first = half == 0 ? rb : 0, last = half == 0 ? re : mt->nrows;
-        RowList list;        // the rows that have pairs of this half, by the entries these stream
-        SgPairFilter mine;
-        mine.towner = T;
-        mine.strict = half;
-        mine.xlo = half == 0 ? 0 : rb;
-        mine.xhi = half == 0 ? everywhere : re;
-        COMET_CHK(sg_row_list(P, L, first, last, SG_NO_DENSE, SG_NO_DENSE, &list, nullptr, 0, mine));
-        COMET_CHK(sg_reset_ticket());
-        KernelTimer t(values ? (half == 0 ? "spgemm_numeric_dot_rows" : "spgemm_numeric_dot_columns")
-                             : (half == 0 ? "spgemm_symbolic_dot_rows" : "spgemm_symbolic_dot_columns"));
-#define LAUNCH_DOT(V, S)                                                                                   \
-    do {                                                                                                   \
-        COMET_CHK(sg_allow_lds(spgemm_dot_kernel<V, S>, lds));                                             \
-        spgemm_dot_kernel<V, S><<<grid, block, lds, stream()>>>(                                           \
-            first, T->pos, T->crd, T->val, P->pos, P->crd, L->pos, L->crd, L->val,                         \
-            half == 0 ? nullptr : mt->val, out0, half, half == 0 ? 0 : rb, half == 0 ? everywhere : re,    \
-            words, (unsigned long long *)g_sg.ticket.ptr, list, *pair_val, *pair_hit, reduce_op, mult_op,  \
-            half);                                                                                         \
-    } while (0)
-        if (!values)
-            LAUNCH_DOT(false, false);
-        else if (semi)
-            LAUNCH_DOT(true, true);
-        else
-            LAUNCH_DOT(true, false);
-#undef LAUNCH_DOT
-        COMET_HIPCHK(hipGetLastError());
-    }
     return COMET_HIP_OK;
 }
 
@@ -3279,10 +2801,14 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         if (dots) {
             double *pair_val = nullptr;
             uint8_t *pair_hit = nullptr;
-            COMET_CHK(dot_pairs(a, b, m, rb, re, true, &pair_val, &pair_hit, reduce_op, mult_op));
+            int64_t pairs = 0, *before = nullptr, chunks = 0;
+            COMET_CHK(pair_dot_values(const_cast<Csr *>(a), b, const_cast<Csr *>(m), rb, re, &pair_val, &pair_hit, &pairs,
+                                      reduce_op, mult_op));
+            COMET_CHK(dot_chunks(pairs, pair_hit, &before, &chunks));
             KernelTimer t("spgemm_numeric_dot_compact");
-            spgemm_dot_compact<<<dim3((unsigned)ceil_div(re - rb, 4)), dim3(256), 0, stream()>>>(
-                rb, re, m->pos, m->crd, pair_val, pair_hit, Cpos, Ccrd, Cval);
+            if (chunks > 0)
+                dot_chunk_compact<<<dim3((unsigned)chunks), dim3(256), 0, stream()>>>(rb, re, m->pos, m->crd, pair_val, pair_hit,
+                                                                                      before, nullptr, Ccrd, Cval);
             COMET_HIPCHK(hipGetLastError());
             return COMET_HIP_OK;
         }
@@ -3513,8 +3039,12 @@ static int64_t masked_product_one_pass(const Csr *a, const Csr *b, const Csr *m,
     *done = true;
     double *pair_val = nullptr;
     uint8_t *pair_hit = nullptr;
-    if (dot_pairs(a, b, m, 0, a->nrows, true, &pair_val, &pair_hit, reduce_op, mult_op) != COMET_HIP_OK ||
-        g_sg.rowcount.ensure(sizeof(int64_t) * (size_t)a->nrows, false) != COMET_HIP_OK)
+    int64_t pairs = 0, *before = nullptr, chunks = 0;
+    void *word = nullptr;
+    if (mailbox(&word) != COMET_HIP_OK ||
+        pair_dot_values(const_cast<Csr *>(a), const_cast<Csr *>(b), const_cast<Csr *>(m), 0, a->nrows, &pair_val, &pair_hit,
+                        &pairs, reduce_op, mult_op) != COMET_HIP_OK ||
+        dot_chunks(pairs, pair_hit, &before, &chunks) != COMET_HIP_OK)
         return 0;
     Csr *c = new Csr();
     c->nrows = a->nrows;
@@ -3526,25 +3056,20 @@ static int64_t masked_product_one_pass(const Csr *a, const Csr *b, const Csr *m,
         csr_release(c);
         return 0;
     };
-    if (dev_malloc((void **)&c->pos, sizeof(int64_t) * (size_t)(a->nrows + 1)) != hipSuccess)
-        return fail("row pointer allocation failed");
-    {
-        KernelTimer t("spgemm_symbolic_dot_count");
-        spgemm_dot_count<<<dim3((unsigned)ceil_div(a->nrows, 4)), dim3(256), 0, stream()>>>(
-            0, a->nrows, m->pos, pair_hit, (int64_t *)g_sg.rowcount.ptr);
-    }
-    if (exclusive_scan_i64((const int64_t *)g_sg.rowcount.ptr, a->nrows, c->pos) != COMET_HIP_OK)
-        return fail(nullptr);
-    if (hipMemcpyAsync(&c->nnz, c->pos + a->nrows, sizeof(int64_t), hipMemcpyDeviceToHost, stream()) != hipSuccess ||
+    if (hipMemcpyAsync(word, before + chunks, sizeof(int64_t), hipMemcpyDeviceToHost, stream()) != hipSuccess ||
         stream_wait() != COMET_HIP_OK)
         return fail("reading the size of the product failed");
-    if (dev_malloc((void **)&c->crd, sizeof(int32_t) * (size_t)(c->nnz > 0 ? c->nnz : 1)) != hipSuccess ||
+    c->nnz = *(volatile int64_t *)word;
+    if (dev_malloc((void **)&c->pos, sizeof(int64_t) * (size_t)(a->nrows + 1)) != hipSuccess ||
+        dev_malloc((void **)&c->crd, sizeof(int32_t) * (size_t)(c->nnz > 0 ? c->nnz : 1)) != hipSuccess ||
         dev_malloc((void **)&c->val, sizeof(double) * (size_t)(c->nnz > 0 ? c->nnz : 1)) != hipSuccess)
         return fail("output allocation failed");
-    {
+    if (chunks == 0 && hipMemsetAsync(c->pos, 0, sizeof(int64_t) * (size_t)(a->nrows + 1), stream()) != hipSuccess)
+        return fail("clearing the row pointers failed");
+    if (chunks > 0) {
         KernelTimer t("spgemm_numeric_dot_compact");
-        spgemm_dot_compact<<<dim3((unsigned)ceil_div(a->nrows, 4)), dim3(256), 0, stream()>>>(
-            0, a->nrows, m->pos, m->crd, pair_val, pair_hit, c->pos, c->crd, c->val);
+        dot_chunk_compact<<<dim3((unsigned)chunks), dim3(256), 0, stream()>>>(0, a->nrows, m->pos, m->crd, pair_val, pair_hit,
+                                                                              before, c->pos, c->crd, c->val);
     }
     if (hipGetLastError() != hipSuccess)
         return fail("launching the compaction failed");
@@ -3835,11 +3360,8 @@ extern "C" int comet_hip_debug_masked_sum_registers(int *workgroup_kernel, int *
 }
 
 // Diagnostic: where the fp64 sums of the dot-product kernel begin in its LDS, in 32-bit words, for a bitmap of
-// `words` words (rounded up to what the host would ask for); lets a CPU-side test sweep the invariant "even".
+// `words` words (the counts beside it included); lets a CPU-side test sweep the invariant "even".
 extern "C" int comet_hip_debug_dot_table_words(int words)
 {
-    if (words < 1)
-        words = 1;
-    words = (int)ceil_div((int64_t)words, (int64_t)DT_WPT) * DT_WPT;
-    return dot_table_words(words);
+    return dot_table_words(32 * (int64_t)(words < 1 ? 1 : words));
 }

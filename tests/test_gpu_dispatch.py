@@ -125,3 +125,50 @@ def test_masked_sum_of_nearly_empty_matrices(nnz):
     x = (pos, np.arange(nnz, dtype=np.int32), np.ones(nnz))
     A = rt.CsrMatrix.from_arrays((5, 5), *x)
     assert rt.spgemm_masked_sum(A, A, A) == (nnz if nnz else 0)
+
+
+@pytest.mark.parametrize("semiring", [None, ("min", "plus")])
+@pytest.mark.parametrize("k", [1, 63, 6000, 300_001, 640_001, 1 << 20])
+def test_masked_product_of_every_list_and_table_length(k, semiring):
+    # tables in a wavefront's buckets, in a workgroup's with the values beside it and without, with a count for every word
+    # and for every eight; lists around a quad and a turn; mask rows for one fetch of pairs and more
+    rng = np.random.default_rng(9)
+    sizes = [x for x in (1, 2, 3, 4, 5, 63, 64, 65, 191, 192, 193, 255, 257, 900, 4000, 15_000) if x <= k]
+    la, lb = np.array(sizes * 3 + [0, 7 % (k + 1)] * 8), np.array(sizes[::-1] * 2 + [0, 1] * 40)
+    pick = np.sort(rng.choice(k, min(k, 20_000), replace=False))
+    rows = lambda lengths: (np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64),
+                            np.concatenate([np.sort(rng.choice(pick, l, replace=False)) for l in lengths]).astype(np.int32))
+    apos, acrd = rows(la)
+    bt_pos, bt_crd = rows(lb)          # B by columns
+    col = np.repeat(np.arange(len(lb)), lb)
+    order = np.lexsort((col, bt_crd))
+    bpos = np.concatenate([[0], np.cumsum(np.bincount(bt_crd, minlength=k))]).astype(np.int64)
+    a, b = (apos, acrd, rng.uniform(-1, 1, len(acrd))), (bpos, col[order].astype(np.int32), rng.uniform(-1, 1, len(col)))
+    n, m = len(la), len(lb)
+    for keep in (0.0, 0.01, 0.5, 1.0):
+        mask = rng.random((n, m)) < keep
+        mp, mc = np.concatenate([[0], np.cumsum(mask.sum(1))]).astype(np.int64), np.nonzero(mask)[1].astype(np.int32)
+        A, B, M = (rt.CsrMatrix.from_arrays(shape, *x) for shape, x in (((n, k), a), ((k, m), b), ((n, m), (mp, mc, np.ones(len(mc))))))
+        wp, wc, wv = orc.spgemm(*a, *b, m, mask=(mp, mc), semiring=semiring)
+        p, c, v = rt.spgemm(A, B, M, semiring=semiring).to_arrays()
+        assert np.array_equal(p, wp) and np.array_equal(c, wc)
+        if semiring:
+            assert np.array_equal(v, wv)
+        else:
+            bound = orc.spgemm(a[0], a[1], np.abs(a[2]), b[0], b[1], np.abs(b[2]), m, mask=(mp, mc))[2]
+            assert np.all(np.abs(v - wv) <= 1e-12 * bound)
+
+
+@pytest.mark.parametrize("nnz", [1, 2047, 2048, 2049, 6144])
+def test_masked_product_gathers_its_result_by_chunks(nnz):
+    # a diagonal A keeps every second row's mask entries; rows of one entry, empty rows, a row longer than a chunk
+    rng = np.random.default_rng(nnz)
+    lengths = np.bincount(rng.integers(0, 40, nnz), minlength=50) + np.where(np.arange(50) == 45, 2500, 0)
+    mp = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    mc = np.concatenate([np.sort(rng.choice(9000, l, replace=False)) for l in lengths]).astype(np.int32)
+    a = (np.repeat(np.arange(26), 2)[1:].astype(np.int64), np.zeros(25, np.int32), np.full(25, 3.0))
+    b = (np.array([0, 9000], np.int64), np.arange(9000, dtype=np.int32), rng.uniform(1, 2, 9000))
+    A, B, M = rt.CsrMatrix.from_arrays((50, 1), *a), rt.CsrMatrix.from_arrays((1, 9000), *b), rt.CsrMatrix.from_arrays(
+        (50, 9000), mp, mc, np.ones(len(mc)))
+    want = orc.spgemm(*a, *b, 9000, mask=(mp, mc))
+    assert all(np.array_equal(g, w) for g, w in zip(rt.spgemm(A, B, M).to_arrays(), want))
