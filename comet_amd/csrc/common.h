@@ -223,4 +223,17 @@ int sort_pairs_u64_u32(const uint64_t *keys_in, uint64_t *keys_out, const uint32
 // deterministic tree sum of a device array, result copied to the host
 int reduce_sum_device(const double *v, int64_t n, double *out_host);
 
+// the largest v of this lane and those before it; v >= 0
+__device__ __forceinline__ int wave_inclusive_max(int v)
+{
+    const auto step = [&](int o) { v = o > v ? o : v; };
+    step(__builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+    return v;
+}
+
 }  // namespace comet

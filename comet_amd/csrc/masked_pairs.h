@@ -48,18 +48,6 @@ __device__ __forceinline__ bool pair_kept(int strict, int64_t len, int64_t tlen)
     return strict == 2 || (strict ? len < tlen : len <= tlen);
 }
 
-__device__ __forceinline__ int wave_inclusive_max(int v)
-{
-    const auto step = [&](int o) { v = o > v ? o : v; };
-    step(__builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
-    step(__builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
-    step(__builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
-    step(__builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
-    step(__builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
-    step(__builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
-    return v;
-}
-
 // The entries of P, rows [first, last), are looked at PAIR_CHUNK at a time wherever the rows end - a column of a power-law
 // matrix has a hundred thousand times the entries of the next - and every kept one finds its place by counting those in
 // front of it.  (A wavefront per row: 2.2 ms a pass for 15.7 M entries, all but 0.2 of it the longest row's.)

@@ -9,6 +9,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <memory>
 #include <queue>
 #include <utility>
 #include <vector>
@@ -359,37 +360,42 @@ static int spmv_plan(Csr *a)
 }
 
 // ============================================================================
-// SpMM, nonzero-split: the nonzeros of A are cut into chunks of SPMM_CH and one
-// wavefront owns each chunk, whatever rows it covers, so Zipf-distributed row
-// lengths cost nothing in balance.  Lane l owns dense column (tile*64 + l): a
-// gather of one B row is a single coalesced 512-byte load, issued SPMM_U deep
-// before the dependent adds.  Rows that lie inside one chunk are finished by
-// that wavefront in nonzero order.  A row cut by a chunk boundary leaves its
-// pieces in `carry` (two 64-wide slots per chunk: [0] a piece whose row began
-// in an earlier chunk, [1] a piece whose row goes on into the next) and the
-// fix-up kernel adds the pieces in chunk order.
+// SpMM, nonzero-split: the nonzeros of A are cut into chunks of SPMM_CH (a half
+// or a quarter of that where there are not many) and one wavefront owns each
+// chunk, whatever rows it covers, so Zipf-distributed row lengths cost nothing
+// in balance.  A lane owns two dense columns, 16 bytes of a row of B, so that a
+// tile of kt columns takes kt / 2 lanes and a wavefront holds 64 / (kt / 2)
+// groups of them, each with a run of the chunk's nonzeros of its own, SPMM_U
+// gathers of B deep.  Which row a nonzero is of is worked out once per chunk in
+// LDS.  A row that lies inside one block of SPMM_CH nonzeros is summed by one
+// group, in nonzero order: where a boundary of a chunk or run would cut it, it
+// goes to the one it begins in.  The other rows are cut wherever that happens;
+// the pieces of a chunk are added in LDS, and what the chunk has of them goes to
+// `carry` (two 64-wide slots per chunk: [0] a piece whose row began in an
+// earlier chunk, [1] a piece whose row goes on into the next), from where the
+// wavefront that leaves the last piece of a row (`arrived` counts them, by the
+// chunk the row begins in; zero between calls) adds them in chunk order.
+// Bound by the gathers' way from the memory-side cache where B is larger than
+// an L2.  A lane per column and one nonzero at a time (K of 64 lanes busy, 8
+// bytes each) took 84 us for 60001 rows of 16 nonzeros and K = 33, this 69; 81 and 47 for
+// K = 14, 349 and 175 for 500000 rows and K = 3, 49 and 22 for 2000 rows.
 // ============================================================================
-#ifndef COMET_SPMM_CH
-#define COMET_SPMM_CH 256
-#endif
 #ifndef COMET_SPMM_U
-#define COMET_SPMM_U 16
+#define COMET_SPMM_U 8
 #endif
-#ifndef COMET_SPMM_WAVES
-#define COMET_SPMM_WAVES 4
-#endif
-constexpr int SPMM_CH = COMET_SPMM_CH;        // nonzeros per wavefront
-constexpr int SPMM_U = COMET_SPMM_U;          // B-row loads in flight per wavefront
-constexpr int SPMM_WAVES = COMET_SPMM_WAVES;  // wavefronts per workgroup
+constexpr int SPMM_CH = 256;                  // nonzeros per wavefront, at most
+constexpr int SPMM_GRAIN = 64;                // the row of every so many'th nonzero is kept
+constexpr int SPMM_U = COMET_SPMM_U;          // B-row loads in flight per lane
+constexpr int SPMM_WAVES = 4;                 // wavefronts per workgroup
 
-// chunk_row[c] = the row r with pos[r] <= c*SPMM_CH < pos[r+1]
-__global__ void spmm_chunk_rows(const int64_t *__restrict__ pos, int64_t nrows, int64_t nchunks,
+// chunk_row[c] = the row r with pos[r] <= c*grain < pos[r+1]
+__global__ void spmm_chunk_rows(const int64_t *__restrict__ pos, int64_t nrows, int64_t nchunks, int grain,
                                 int32_t *__restrict__ chunk_row)
 {
     int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nchunks)
         return;
-    const int64_t target = c * SPMM_CH;
+    const int64_t target = c * grain;
     int64_t lo = 0, hi = nrows;   // first index in pos[0..nrows] with pos > target lies in [1, nrows]
     while (lo < hi) {
         int64_t mid = (lo + hi) >> 1;
@@ -401,131 +407,251 @@ __global__ void spmm_chunk_rows(const int64_t *__restrict__ pos, int64_t nrows, 
     chunk_row[c] = (int32_t)lo;
 }
 
-template <bool ACC>
+typedef double spmm_pair __attribute__((ext_vector_type(2), aligned(8)));
+
+struct SpmmChunkLds {
+    union {
+        struct {
+            double val[SPMM_CH];
+            int32_t crd[SPMM_CH];
+        };
+        double piece[2][128];            // of every group: its head and its tail, over the entries
+    };
+    int32_t row[SPMM_CH + 4];            // the last one: whose row goes on past the chunk
+};
+
+// W: columns of a lane, 2 unless K is 1.  SMALL: B is within 4 GiB.
+template <bool ACC, int W, bool SMALL>
 __global__ __launch_bounds__(SPMM_WAVES * 64) void spmm_csr_nnzsplit(
     const int64_t *__restrict__ pos, const int32_t *__restrict__ crd, const double *__restrict__ val,
-    int64_t nnz, int64_t nrows, const int32_t *__restrict__ chunk_row, int64_t nchunks,
+    int64_t nnz, int64_t nrows, const int32_t *__restrict__ chunk_row, int grain, int chunk_len, int64_t nchunks,
     const double *__restrict__ B, int64_t ldb, double *__restrict__ C, int64_t ldc, int64_t K,
-    double *__restrict__ carry, const int32_t *__restrict__ rowmap)
+    double *__restrict__ carry, unsigned *__restrict__ arrived, const int32_t *__restrict__ rowmap)
 {
+    __shared__ __align__(16) SpmmChunkLds all[SPMM_WAVES];
     // rowmap: the matrix lists only some rows of C (row r of pos is row rowmap[r] of C); nullptr: all of them
     auto crow = [&](int64_t r) -> int64_t { return rowmap ? (int64_t)rowmap[r] : r; };
     const int lane = threadIdx.x & 63;
-    const int64_t chunk =
-        (int64_t)blockIdx.x * SPMM_WAVES + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t chunk = (int64_t)blockIdx.x * SPMM_WAVES + wave;
     if (chunk >= nchunks)
         return;
-    const int64_t col = (int64_t)blockIdx.y * 64 + lane;
-    const bool active = col < K;
-    const int64_t s = chunk * SPMM_CH;
-    const int64_t e = s + SPMM_CH < nnz ? s + SPMM_CH : nnz;
-    int64_t r = __builtin_amdgcn_readfirstlane(chunk_row[chunk]);
-    int64_t rend = pos[r + 1];
-    const bool head = pos[r] < s;      // the first row of this chunk began earlier
-    bool first_piece = true;
-    bool open = false;                 // the current row has consumed nonzeros of this chunk
-    double *carry0 = carry + (((int64_t)blockIdx.y * nchunks + chunk) * 2) * 64;
-
+    SpmmChunkLds &sh = all[wave];
+    const int64_t tile = (int64_t)blockIdx.y * 64;
+    const int kt = (int)(K - tile < 64 ? K - tile : 64);
+    const int L = (kt + W - 1) / W, G = 64 / L;               // lanes of a group, groups
+    const int g = lane / L, sub = lane - g * L;
+    // the last lane of an odd tile has one column, and reads the one before it as well
+    const bool half = W == 2 && sub == L - 1 && (kt & 1);
+    const int64_t col = tile + W * sub, from = col - (half ? 1 : 0);
+    // ---- the nonzeros [s, e) of the chunk, moved to the ends of rows that are not to be cut, and the rows they are of
+    const int64_t s_cut = chunk * chunk_len, e_cut = s_cut + chunk_len < nnz ? s_cut + chunk_len : nnz;
+    const int64_t block = s_cut / SPMM_CH * SPMM_CH;
+    const int64_t r0 = __builtin_amdgcn_readfirstlane(chunk_row[s_cut / grain]);
+    const int64_t rn = e_cut < nnz ? (int64_t)__builtin_amdgcn_readfirstlane(chunk_row[e_cut / grain]) : nrows;
+    int64_t s = s_cut, e = e_cut;
+    const int64_t p0 = pos[r0], q0 = pos[r0 + 1];
+    const bool head = p0 < s_cut && (p0 < block || q0 > block + SPMM_CH);          // the first row is a piece of one
+    if (p0 < s_cut && !head)                             // an earlier chunk's
+        s = q0;
+    bool tail = false;                                   // the last row goes on into the next block
+    if (rn < nrows) {
+        const int64_t pn = pos[rn], qn = pos[rn + 1];
+        if (pn < e_cut) {
+            tail = pn < block || qn > block + SPMM_CH;
+            e = tail ? e_cut : qn;
+        }
+    }
+    const int n = e > s ? (int)(e - s) : 0;
+    for (int t = lane; t < n; t += 64) {      // A is streamed once: keep it from displacing B in the caches
+        sh.crd[t] = __builtin_nontemporal_load(crd + s + t);
+        sh.val[t] = __builtin_nontemporal_load(val + s + t);
+    }
+    for (int t = lane; t < n; t += 64)
+        sh.row[t] = 0;
+    auto clear = [&](int64_t r) {
+        if (lane < kt)
+            C[crow(r) * ldc + tile + lane] = 0.0;
+    };
     // rows in front of the first stored nonzero are empty: chunk 0 clears them
-    if (!ACC && chunk == 0 && active)
-        for (int64_t z = 0; z < r; ++z)
-            C[crow(z) * ldc + col] = 0.0;
-
-    double acc = 0.0;
-    // a row that goes on past this chunk leaves its C value to the fix-up kernel
-    if (ACC && !head && rend <= e && active)
-        acc = C[crow(r) * ldc + col];
-
-    for (int64_t base = s; base < e; base += 64) {
-        const int cnt = (int)(e - base < 64 ? e - base : 64);
-        int my_crd = 0;
-        double my_val = 0.0;
-        if (lane < cnt) {      // A is streamed once: keep it from displacing B in the caches
-            my_crd = __builtin_nontemporal_load(crd + base + lane);
-            my_val = __builtin_nontemporal_load(val + base + lane);
+    if (!ACC && chunk == 0)
+        for (int64_t z = 0; z < r0; ++z)
+            clear(z);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    for (int64_t base = r0 + 1; base <= rn && base < nrows; base += 64) {
+        const int64_t r = base + lane;
+        int64_t p = 0, q = 0;
+        const bool in = r <= rn && r < nrows;
+        if (in) {
+            p = pos[r];
+            q = pos[r + 1];
         }
-        for (int t0 = 0; t0 < cnt; t0 += SPMM_U) {
-            double b[SPMM_U];
-#pragma unroll
-            for (int u = 0; u < SPMM_U; ++u) {
-                b[u] = 0.0;
-                if (t0 + u < cnt) {
-                    const int64_t j = __builtin_amdgcn_readlane(my_crd, t0 + u);
-                    if (active)
-                        b[u] = B[j * ldb + col];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < SPMM_U; ++u) {
-                if (t0 + u < cnt) {
-                    const double a = readlane_f64(my_val, t0 + u);
-                    const double prod = a * b[u];
-                    acc = acc + prod;
-                    open = true;
-                    const int64_t p = base + t0 + u + 1;
-                    bool holds = true;           // the first turn closes a row that holds nonzeros
-                    while (p == rend) {          // row r is complete; also walks over empty rows that follow
-                        if (active && (holds || !ACC)) {     // accumulating leaves empty rows untouched
-                            if (first_piece && head)
-                                carry0[lane] = acc;
-                            else     // C is written once and not read again by this kernel
-                                __builtin_nontemporal_store(acc, C + crow(r) * ldc + col);
-                        }
-                        first_piece = false;
-                        open = false;
-                        holds = false;
-                        ++r;
-                        if (r >= nrows)
-                            break;
-                        rend = pos[r + 1];
-                        acc = 0.0;
-                        // a row that starts here and ends later keeps its C value for the fix-up instead
-                        if (ACC && active && rend > p && rend <= e)
-                            acc = C[crow(r) * ldc + col];
-                    }
-                }
+        if (in && p < q && p < e)
+            sh.row[p - s] = (int32_t)(r - r0);
+        if constexpr (!ACC) {            // accumulating leaves empty rows untouched
+            unsigned long long empty = __ballot(in && p == q);
+            while (empty) {
+                clear(base + __builtin_ctzll(empty));
+                empty &= empty - 1;
             }
         }
     }
-    if (open && active) {                // the last row goes on into the next chunk
-        if (first_piece && head)
-            carry0[lane] = acc;
-        else
-            carry0[64 + lane] = acc;
+    if (n == 0)
+        return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    int last = 0;
+    for (int t = 0; t < n; t += 64) {
+        int m = wave_inclusive_max(t + lane < n ? sh.row[t + lane] : 0);
+        m = m > last ? m : last;
+        if (t + lane < n)
+            sh.row[t + lane] = m;
+        last = __builtin_amdgcn_readlane(m, 63);
     }
-}
+    if (lane == 0)
+        sh.row[n] = tail ? last : -1;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
 
-// One wavefront per chunk: if a row that began in an earlier chunk ends in this
-// one, add its pieces in chunk order and write the row.
-template <bool ACC>
-__global__ __launch_bounds__(SPMM_WAVES * 64) void spmm_csr_fixup(
-    const int64_t *__restrict__ pos, int64_t nnz, const int32_t *__restrict__ chunk_row, int64_t nchunks,
-    double *__restrict__ C, int64_t ldc, int64_t K, const double *__restrict__ carry,
-    const int32_t *__restrict__ rowmap)
-{
-    const int lane = threadIdx.x & 63;
-    const int64_t chunk =
-        (int64_t)blockIdx.x * SPMM_WAVES + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    if (chunk >= nchunks)
+    // ---- every group its run
+    const int run = (n + G - 1) / G;
+    auto cut = [&](int32_t r) { return (head && r == 0) || (tail && r == last); };
+    auto begin = [&](int x) -> int {
+        const int t = x * run < n ? x * run : n;
+        if (t == 0 || t == n)
+            return t;
+        const int32_t r = sh.row[t];
+        return sh.row[t - 1] != r || cut(r) ? t : (int)(pos[r0 + r + 1] - s);
+    };
+    const int a = begin(g), z = g < G ? begin(g + 1) : n;
+    const int longest = g < G ? z - a : 0;
+    double ax = 0.0, ay = 0.0, hx = 0.0, hy = 0.0;          // hx, hy: the piece of a row that began before
+    auto store = [&](int32_t r, double x, double y) {
+        double *to = C + crow(r0 + r) * ldc + col;
+        if (W == 2 && !half) {           // C is written once and not read again by this kernel
+            spmm_pair v;
+            v.x = x;
+            v.y = y;
+            __builtin_nontemporal_store(v, reinterpret_cast<spmm_pair *>(to));
+        } else {
+            __builtin_nontemporal_store(x, to);
+        }
+    };
+    for (int t0 = 0; __any(t0 < longest); t0 += SPMM_U) {
+        spmm_pair b[SPMM_U], c[ACC ? SPMM_U : 1];
+        double v[SPMM_U];
+        // bit u: the row of the batch's nonzero u ends with it (all of this read before the first is used: the adds of a
+        // long row are one chain, and a look into LDS in it costs more than the rest)
+        unsigned ends = 0;
+        int32_t r = sh.row[a + t0 < n ? a + t0 : n - 1];
+        const bool fresh = t0 == 0 || sh.row[a + t0 - 1 < n ? a + t0 - 1 : n - 1] != r;
+#pragma unroll
+        for (int u = 0; u < SPMM_U; ++u) {
+            const int t = a + t0 + u < n ? a + t0 + u : n - 1;
+            const uint32_t j = (uint32_t)sh.crd[t];
+            v[u] = sh.val[t];
+            const double *at = SMALL ? reinterpret_cast<const double *>(reinterpret_cast<const char *>(B) +
+                                                                        (j * (uint32_t)ldb + (uint32_t)from) * 8u)
+                                     : B + (int64_t)j * ldb + from;
+            if constexpr (W == 2)
+                b[u] = *reinterpret_cast<const spmm_pair *>(at);
+            else
+                b[u].x = *at;
+            const int32_t next = sh.row[t + 1];
+            if constexpr (ACC) {         // where a row begins; the value of a row in pieces is added with them
+                if (t0 + u < longest && (u == 0 ? fresh : (ends >> (u - 1) & 1u) != 0) && !cut(r)) {
+                    const double *to = C + crow(r0 + r) * ldc + from;
+                    if constexpr (W == 2)
+                        c[u] = *reinterpret_cast<const spmm_pair *>(to);
+                    else
+                        c[u].x = *to;
+                }
+            }
+            ends |= (unsigned)(next != r && t0 + u < longest) << u;
+            r = next;
+        }
+        bool begins = fresh;
+#pragma unroll
+        for (int u = 0; u < SPMM_U; ++u) {
+            if constexpr (ACC)
+                if (begins && t0 + u < longest && !cut(sh.row[a + t0 + u])) {
+                    ax = half ? c[u].y : c[u].x;
+                    ay = W == 2 ? c[u].y : 0.0;
+                }
+            const double x = ax + v[u] * (half ? b[u].y : b[u].x), y = W == 2 ? ay + v[u] * b[u].y : 0.0;
+            ax = t0 + u < longest ? x : ax;
+            ay = t0 + u < longest ? y : ay;
+            begins = (ends >> u & 1u) != 0;
+            if (begins) {
+                const int32_t mine = sh.row[a + t0 + u];
+                if (head && mine == 0) {
+                    hx = ax;
+                    hy = ay;
+                } else {
+                    store(mine, ax, ay);
+                }
+                ax = ay = 0.0;
+            }
+        }
+    }
+    if (!head && !tail)
         return;
-    const int64_t col = (int64_t)blockIdx.y * 64 + lane;
-    if (col >= K)
+    // ---- the pieces, a lane per column; what a group's run ends inside of is a piece of the first row or of the last
+    if (longest > 0 && head && sh.row[z - 1] == 0 && sh.row[z] == 0) {
+        hx = ax;
+        hy = ay;
+        ax = ay = 0.0;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    if (g < G) {
+        if (W == 2 && !half) {
+            sh.piece[0][g * kt + 2 * sub] = hx;
+            sh.piece[0][g * kt + 2 * sub + 1] = hy;
+            sh.piece[1][g * kt + 2 * sub] = ax;
+            sh.piece[1][g * kt + 2 * sub + 1] = ay;
+        } else {
+            sh.piece[0][g * kt + W * sub] = hx;
+            sh.piece[1][g * kt + W * sub] = ax;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    if (lane >= kt)
         return;
-    const int64_t s = chunk * SPMM_CH;
-    const int64_t e = s + SPMM_CH < nnz ? s + SPMM_CH : nnz;
-    const int64_t r = __builtin_amdgcn_readfirstlane(chunk_row[chunk]);
-    const int64_t rs = pos[r], re = pos[r + 1];
-    if (rs >= s || re > e)
-        return;
-    const int64_t c0 = rs / SPMM_CH;
-    const double *cb = carry + ((int64_t)blockIdx.y * nchunks * 2) * 64;
-    double acc = cb[(c0 * 2 + 1) * 64 + lane];
-    const int64_t cr = rowmap ? (int64_t)rowmap[r] : r;
-    if (ACC)
-        acc = C[cr * ldc + col] + acc;
-    for (int64_t c = c0 + 1; c <= chunk; ++c)
-        acc = acc + cb[(c * 2) * 64 + lane];
-    C[cr * ldc + col] = acc;
+    double *slots = carry + (int64_t)blockIdx.y * nchunks * 128 + lane;
+    double began = 0.0, goes_on = 0.0;
+    for (int x = 0; x < G; ++x) {
+        began += sh.piece[0][x * kt + lane];
+        goes_on += sh.piece[1][x * kt + lane];
+    }
+    const bool both = head && tail && last == 0;          // one row, through the chunk
+    if (head)
+        __hip_atomic_store(slots + chunk * 128, began, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tail && !both)
+        __hip_atomic_store(slots + chunk * 128 + 64, goes_on, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // Whoever leaves the last piece of a row adds all of them, in order.  The pieces are written and read past the L2s
+    // (agent scope), and this wavefront's have arrived before it counts itself in.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    auto finish = [&](int64_t r) {
+        const int64_t c0 = pos[r] / chunk_len, c1 = (pos[r + 1] - 1) / chunk_len;
+        unsigned *count = arrived + (int64_t)blockIdx.y * nchunks + c0;
+        unsigned before = 0;
+        if (lane == 0)
+            before = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((int64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)before) != c1 - c0)
+            return;
+        if (lane == 0)
+            __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);          // for the next call
+        double *to = C + crow(r) * ldc + tile + lane;
+        double sum = __hip_atomic_load(slots + c0 * 128 + 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (ACC)
+            sum = *to + sum;
+#pragma unroll 8
+        for (int64_t c = c0 + 1; c <= c1; ++c)
+            sum += __hip_atomic_load(slots + c * 128, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *to = sum;
+    };
+    if (head)
+        finish(r0);
+    if (tail && !both)
+        finish(rn);
 }
 
 // ============================================================================
@@ -872,11 +998,29 @@ __global__ void fill_rows_f64(double *__restrict__ C, int64_t nrows, int64_t K, 
         C[(i / K) * ldc + (i % K)] = v;
 }
 
-static Workspace g_spmm_carry;
+static Workspace g_spmm_carry, g_spmm_arrived;
+
+// Nonzeros of a chunk: a half or a quarter of SPMM_CH where that makes 8192 wavefronts at most, 32 for every CU.  (The
+// number is also what the scratch of the form without allocations holds, which cuts rows in the same places.)
+constexpr int64_t SPMM_SHORT_CHUNKS = 8192;
+static int spmm_chunk_len(int64_t nnz, int64_t tiles)
+{
+    for (int len = SPMM_CH / 4; len < SPMM_CH; len *= 2)
+        if (tiles * ceil_div(nnz, len) <= SPMM_SHORT_CHUNKS)
+            return len;
+    return SPMM_CH;
+}
+
+static int spmm_chunk_scratch(const Csr *a, int64_t K)
+{
+    const int64_t tiles = ceil_div(K, 64), slots = tiles * ceil_div(a->nnz, spmm_chunk_len(a->nnz, tiles));
+    COMET_CHK(g_spmm_carry.ensure(sizeof(double) * 128 * (size_t)slots, false));
+    return g_spmm_arrived.ensure(sizeof(unsigned) * (size_t)slots, true);
+}
 
 static int spmm_plan(Csr *a)
 {
-    const int64_t nchunks = ceil_div(a->nnz, SPMM_CH);
+    const int64_t nchunks = ceil_div(a->nnz, SPMM_GRAIN);
     if (a->spmm_chunk_row && a->spmm_nchunks == nchunks)
         return COMET_HIP_OK;
     if (a->spmm_chunk_row) {
@@ -888,7 +1032,7 @@ static int spmm_plan(Csr *a)
     if (nchunks > 0) {
         KernelTimer t("spmm_chunk_rows");
         spmm_chunk_rows<<<dim3((unsigned)ceil_div(nchunks, 256)), dim3(256), 0, stream()>>>(
-            a->pos, a->nrows, nchunks, a->spmm_chunk_row);
+            a->pos, a->nrows, nchunks, SPMM_GRAIN, a->spmm_chunk_row);
     }
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
@@ -1562,10 +1706,9 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
     const int G = a->heavy_groups;
     const bool overlap = a->light->nnz > 0 && G < SPMM_HG_ALONE;
     if (overlap) {
-        // what the chunk kernel needs from stream() - its chunk table, its carry slots - is in place before the fork
+        // what the chunk kernel needs from stream() - its chunk table, its scratch - is in place before the fork
         COMET_CHK(spmm_plan(a->light));
-        COMET_CHK(g_spmm_carry.ensure(
-            sizeof(double) * (size_t)(ceil_div(K, 64) * a->light->spmm_nchunks * 2 * 64), false));
+        COMET_CHK(spmm_chunk_scratch(a->light, K));
         COMET_CHK(aux_fork());
     } else if (a->light->nnz > 0)
         COMET_CHK(spmm_chunks(a->light, K, B, ldb, C, ldc, accumulate));
@@ -1620,12 +1763,32 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
     return COMET_HIP_OK;
 }
 
+// The chunk kernel: the row of every grain'th nonzero in chunk_row, chunks of len nonzeros (a multiple of grain), two
+// slots for each of them and column tile in carry and a zero in arrived.  timed: events may be recorded (not where the stream is being captured).
+static void spmm_chunk_launch(const Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate,
+                              const int32_t *chunk_row, int grain, int len, double *carry, unsigned *arrived, hipStream_t on, bool timed)
+{
+    const int64_t nchunks = ceil_div(a->nnz, len);
+    const dim3 grid((unsigned)ceil_div(nchunks, SPMM_WAVES), (unsigned)ceil_div(K, 64)), block(SPMM_WAVES * 64);
+    const auto split = [&](auto kernel) {
+        std::unique_ptr<KernelTimer> t(timed ? new KernelTimer("spmm_csr_nnzsplit", on) : nullptr);
+        kernel<<<grid, block, 0, on>>>(a->pos, a->crd, a->val, a->nnz, a->nrows, chunk_row, grain, len, nchunks, B, ldb, C, ldc,
+                                       K, carry, arrived, a->rowmap);
+    };
+    const bool small_b = K > 1 && a->ncols * ldb * 8 < (1ll << 32);
+    if (K == 1)
+        accumulate ? split(spmm_csr_nnzsplit<true, 1, false>) : split(spmm_csr_nnzsplit<false, 1, false>);
+    else if (small_b)
+        accumulate ? split(spmm_csr_nnzsplit<true, 2, true>) : split(spmm_csr_nnzsplit<false, 2, true>);
+    else
+        accumulate ? split(spmm_csr_nnzsplit<true, 2, false>) : split(spmm_csr_nnzsplit<false, 2, false>);
+}
+
 static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate,
                        hipStream_t on)
 {
     if (!on)
         on = stream();
-    const int64_t b_dptr = (int64_t)B;
     if (a->nnz == 0) {
         if (!accumulate) {
             KernelTimer t("fill_rows_f64", on);
@@ -1636,32 +1799,10 @@ static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *
         return COMET_HIP_OK;
     }
     COMET_CHK(spmm_plan(a));
-    const int64_t nchunks = a->spmm_nchunks;
     const int64_t tiles = ceil_div(K, 64);
-    COMET_CHK(g_spmm_carry.ensure(sizeof(double) * (size_t)(tiles * nchunks * 2 * 64), false));
-    double *carry = (double *)g_spmm_carry.ptr;
-    const dim3 grid((unsigned)ceil_div(nchunks, SPMM_WAVES), (unsigned)tiles);
-    const dim3 block(SPMM_WAVES * 64);
-    {
-        KernelTimer t("spmm_csr_nnzsplit", on);
-        if (accumulate)
-            spmm_csr_nnzsplit<true><<<grid, block, 0, on>>>(a->pos, a->crd, a->val, a->nnz, a->nrows,
-                                                                  a->spmm_chunk_row, nchunks, (const double *)b_dptr,
-                                                                  ldb, C, ldc, K, carry, a->rowmap);
-        else
-            spmm_csr_nnzsplit<false><<<grid, block, 0, on>>>(a->pos, a->crd, a->val, a->nnz, a->nrows,
-                                                                   a->spmm_chunk_row, nchunks, (const double *)b_dptr,
-                                                                   ldb, C, ldc, K, carry, a->rowmap);
-    }
-    {
-        KernelTimer t("spmm_csr_fixup", on);
-        if (accumulate)
-            spmm_csr_fixup<true><<<grid, block, 0, on>>>(a->pos, a->nnz, a->spmm_chunk_row, nchunks, C, ldc, K,
-                                                               carry, a->rowmap);
-        else
-            spmm_csr_fixup<false><<<grid, block, 0, on>>>(a->pos, a->nnz, a->spmm_chunk_row, nchunks, C, ldc, K,
-                                                                carry, a->rowmap);
-    }
+    COMET_CHK(spmm_chunk_scratch(a, K));
+    spmm_chunk_launch(a, K, B, ldb, C, ldc, accumulate, a->spmm_chunk_row, SPMM_GRAIN, spmm_chunk_len(a->nnz, tiles), (double *)g_spmm_carry.ptr,
+                      (unsigned *)g_spmm_arrived.ptr, on, true);
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
 }
@@ -1717,15 +1858,15 @@ extern "C" int comet_hip_gather_rows_bench(int64_t workgroups, int64_t per_wave,
 
 // ---------------------------------------------------------------------------
 // SpMM for callers that cannot allocate (code under graph capture, serving loops that forbid hipMalloc): the
-// chunk kernel and its fix-up with their scratch - the chunk -> row table and the carry slots of rows cut by a
-// chunk boundary - in one array that lives in the library's image instead of in allocated workspaces.  Every
+// chunk kernel with its scratch - the chunk -> row table, the carry slots of rows cut by a chunk boundary and the
+// counts of their pieces - in one array that lives in the library's image instead of in allocated workspaces.  Every
 // device holds its own copy at its own address; the address is looked up once per device, when the library is
 // initialised there, and host code uses that pointer, never the array's name.
 // ---------------------------------------------------------------------------
-constexpr int64_t SPMM_STATIC_SLOTS = 8192;      // (64-column tiles of K) x (chunks of 256 nonzeros) the array has room for
+constexpr int64_t SPMM_STATIC_SLOTS = SPMM_SHORT_CHUNKS;      // (64-column tiles of K) x (chunks of 256 nonzeros) the array has room for
 constexpr size_t SPMM_STATIC_TABLE_BYTES = sizeof(int32_t) * (size_t)SPMM_STATIC_SLOTS;
 constexpr size_t SPMM_STATIC_CARRY_BYTES = sizeof(double) * 2 * 64 * (size_t)SPMM_STATIC_SLOTS;
-static __device__ __align__(256) unsigned char spmm_static_scratch[SPMM_STATIC_TABLE_BYTES + SPMM_STATIC_CARRY_BYTES];
+static __device__ __align__(256) unsigned char spmm_static_scratch[2 * SPMM_STATIC_TABLE_BYTES + SPMM_STATIC_CARRY_BYTES];
 constexpr int SPMM_STATIC_MAX_DEVICES = 64;
 static unsigned char *g_spmm_static_ptr[SPMM_STATIC_MAX_DEVICES];     // device address of the array, per device
 
@@ -1781,24 +1922,15 @@ extern "C" int comet_hip_spmm_csr_f64_noalloc(int64_t csr, int64_t K, int64_t b_
         return COMET_HIP_OK;
     }
     // Every word the kernels read from the array is written earlier in the same call (the table in full, a carry
-    // slot by the chunk that leaves a piece of a row in it), so nothing has to be cleared between calls.
+    // slot by the chunk that leaves a piece of a row in it), or is a count that the one to reach it puts back to zero:
+    // nothing has to be cleared between calls.
     int32_t *chunk_row = reinterpret_cast<int32_t *>(scratch);
     double *carry = reinterpret_cast<double *>(scratch + SPMM_STATIC_TABLE_BYTES);
-    spmm_chunk_rows<<<dim3((unsigned)ceil_div(nchunks, 256)), dim3(256), 0, on>>>(a->pos, a->nrows, nchunks,
-                                                                                         chunk_row);
-    const dim3 grid((unsigned)ceil_div(nchunks, SPMM_WAVES), (unsigned)tiles), block(SPMM_WAVES * 64);
-    const double *B = (const double *)b_dptr;
-    if (accumulate) {
-        spmm_csr_nnzsplit<true><<<grid, block, 0, on>>>(a->pos, a->crd, a->val, a->nnz, a->nrows, chunk_row,
-                                                              nchunks, B, ldb, C, ldc, K, carry, nullptr);
-        spmm_csr_fixup<true><<<grid, block, 0, on>>>(a->pos, a->nnz, chunk_row, nchunks, C, ldc, K, carry,
-                                                           nullptr);
-    } else {
-        spmm_csr_nnzsplit<false><<<grid, block, 0, on>>>(a->pos, a->crd, a->val, a->nnz, a->nrows, chunk_row,
-                                                               nchunks, B, ldb, C, ldc, K, carry, nullptr);
-        spmm_csr_fixup<false><<<grid, block, 0, on>>>(a->pos, a->nnz, chunk_row, nchunks, C, ldc, K, carry,
-                                                            nullptr);
-    }
+    const int len = spmm_chunk_len(a->nnz, tiles);
+    const int64_t rows = ceil_div(a->nnz, len);
+    spmm_chunk_rows<<<dim3((unsigned)ceil_div(rows, 256)), dim3(256), 0, on>>>(a->pos, a->nrows, rows, len, chunk_row);
+    spmm_chunk_launch(a, K, (const double *)b_dptr, ldb, C, ldc, accumulate, chunk_row, len, len, carry,
+                      reinterpret_cast<unsigned *>(scratch + SPMM_STATIC_TABLE_BYTES + SPMM_STATIC_CARRY_BYTES), on, false);
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
 }

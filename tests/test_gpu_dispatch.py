@@ -172,3 +172,28 @@ def test_masked_product_gathers_its_result_by_chunks(nnz):
         (50, 9000), mp, mc, np.ones(len(mc)))
     want = orc.spgemm(*a, *b, 9000, mask=(mp, mc))
     assert all(np.array_equal(g, w) for g, w in zip(rt.spgemm(A, B, M).to_arrays(), want))
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("K", [1, 2, 3, 5, 21, 22, 33, 63, 64, 65, 130])
+@pytest.mark.parametrize("nrows", [1, 40, 4000, 14_000])
+def test_spmm_chunks_of_every_length_and_width(nrows, K, accumulate):
+    # chunks of 64, 128 and 256 nonzeros; rows that end with a chunk, that it would cut but that lie inside a block, that go
+    # through several blocks, empty ones in front, between and behind; groups of every number of lanes
+    rng = np.random.default_rng(nrows + K)
+    lens = np.resize([0, 0, 60, 4, 64, 0, 130, 62, 256, 1, 0, 511, 1, 700, 3, 1, 0], nrows)
+    pos = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    crd, val = rng.integers(0, 500, pos[-1]).astype(np.int32), rng.uniform(-1, 1, pos[-1])
+    crd = np.concatenate([np.sort(r) for r in np.split(crd, pos[1:-1])]).astype(np.int32)
+    B, C0 = rng.uniform(-1, 1, (500, K)), rng.uniform(-1, 1, (nrows, K))
+    A, dB = rt.CsrMatrix.from_arrays((nrows, 500), pos, crd, val), rt.DeviceArray.from_numpy(B)
+    want = orc.spmm(pos, crd, val, B, C0 if accumulate else None)
+    bound = orc.spmm(pos, crd, np.abs(val), np.abs(B), np.abs(C0))
+    whole = (lens == 0) | (pos[:-1] // 256 == (pos[1:] - 1) // 256)          # summed in the order of the nonzeros
+    for _ in range(3):
+        dC = rt.DeviceArray.from_numpy(C0)
+        rt.spmm(A, dB, dC, accumulate=accumulate)
+        got = dC.to_numpy()
+        assert np.all(np.abs(got - want) <= 1e-12 * bound)
+        if K < 16 or K % 2 or pos[-1] < 1 << 19:
+            assert np.array_equal(got[whole], want[whole])
