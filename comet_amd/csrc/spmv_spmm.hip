@@ -2032,20 +2032,23 @@ extern "C" int comet_hip_densemat_csr_f64(int64_t csr, int64_t M, int64_t a_dptr
 // (lib/Dialect/IndexTree/Transforms/KernelFusion.cpp:1049-1220; the test is
 // test/integration/kernels/sddmm.ta).  Either way a stored entry (i, j) gets
 // val * sum_k C[i,k] * D[k,j], the sum unfused and in ascending k.
-// A wavefront takes 32 consecutive stored entries.  Entry by entry it loads the
-// row of C and the (transposed) row of D with the lanes along k - two coalesced
-// loads - and leaves the 64 products in LDS; then lane e walks along the
-// products of entry e and adds them in ascending k.  D is transposed first, so
-// that its "row" for a column j is contiguous; the row of every entry comes
-// from a list kept in B's handle (searching pos per entry cost 80 % of the time).
+// A wavefront takes E stored entries at a time, 64 columns of C and D at a time:
+// a lane owns two of them, so that a group of kt / 2 lanes loads a row of C and a
+// (transposed) row of D, 16 bytes a lane, and there are as many groups as fit;
+// the products go to LDS, and lane e adds those of entry e in ascending k.  E is
+// what the products of 8 KiB allow.  D is transposed first, so that its "row"
+// for a column j is contiguous; the row of every entry comes from a list kept in
+// B's handle (searching pos per entry cost 80 % of the time).
+// Bound by the gathers of D where it is larger than an L2.  (A lane per column
+// and 16 entries took 313 us for 250000 rows of 16 entries and K = 9, this 114;
+// 628 and 158 for 500000 rows and K = 3, 94 and 88 for 60001 and K = 64.)
 // ============================================================================
-#ifndef COMET_SDDMM_E
-#define COMET_SDDMM_E 16
-#endif
-constexpr int SDDMM_E = COMET_SDDMM_E;          // entries per wavefront tile
-constexpr int SDDMM_W = 4;           // wavefronts per workgroup
-constexpr int SDDMM_LD = 65;         // tile row length in doubles: 64 products + 1, so a column walk hits all banks
+constexpr int SDDMM_W = 4;               // wavefronts per workgroup
+constexpr int SDDMM_ROUNDS = 4;          // loads of C and of D under way per lane
+constexpr int SDDMM_TILE = 1088;         // products of a wavefront in LDS: 16 entries of 64 columns and 4 doubles' padding
 
+// E: entries of a wavefront; KT: most columns of a row that are products at a time, E * (KT + 1) of them fit
+template <int E, int KT>
 __global__ __launch_bounds__(SDDMM_W * 64) void sddmm_kernel(int64_t nnz, const int32_t *__restrict__ entry_row,
                                                              const int32_t *__restrict__ crd,
                                                              const double *__restrict__ val,
@@ -2053,42 +2056,59 @@ __global__ __launch_bounds__(SDDMM_W * 64) void sddmm_kernel(int64_t nnz, const 
                                                              const double *__restrict__ Dt, int64_t K,
                                                              double *__restrict__ out)
 {
-    __shared__ double tiles[SDDMM_W][SDDMM_E * SDDMM_LD];
+    static_assert(E * (KT + 1) <= SDDMM_TILE, "the products fit");
+    __shared__ double tiles[SDDMM_W][SDDMM_TILE];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     double *tile = tiles[wave];
-    const int64_t base = ((int64_t)blockIdx.x * SDDMM_W + wave) * SDDMM_E;
+    const int64_t base = ((int64_t)blockIdx.x * SDDMM_W + wave) * E;
     if (base >= nnz)
         return;
-    const int cnt = (int)(nnz - base < SDDMM_E ? nnz - base : SDDMM_E);
+    const int cnt = (int)(nnz - base < E ? nnz - base : E);
     const int64_t p = base + (lane < cnt ? lane : cnt - 1);        // lane e < cnt owns entry base + e
     const int my_col = crd[p], my_row = entry_row[p];
     double t = 0.0;
-    for (int64_t kc = 0; kc < K; kc += 64) {
-        const int kn = (int)(K - kc < 64 ? K - kc : 64);
-        const int64_t k = kc + (lane < kn ? lane : 0);
-        double c[SDDMM_E], d[SDDMM_E];
+    for (int64_t kc = 0; kc < K; kc += KT) {
+        const int kn = (int)(K - kc < KT ? K - kc : KT);
+        const int L = (kn + 1) / 2, G = 64 / L, rounds = (cnt + G - 1) / G;
+        const int g = lane / L, sub = lane - g * L;
+        // the last lane of an odd kn has one column, and reads the one before it as well, if there is one
+        const bool half = sub == L - 1 && (kn & 1);
+        const int64_t from = kc + 2 * sub - (half && kc + 2 * sub > 0 ? 1 : 0);
+        const int ld = kn | 1;               // odd: lanes that walk a column of the tile hit all banks
+        for (int r0 = 0; r0 < rounds; r0 += SDDMM_ROUNDS) {
+            spmm_pair c[SDDMM_ROUNDS], d[SDDMM_ROUNDS];
 #pragma unroll
-        for (int e = 0; e < SDDMM_E; ++e) {          // past the end of a short tile: its last entry again
-            const int ec = e < cnt ? e : cnt - 1;
-            const int64_t j = __builtin_amdgcn_readlane(my_col, ec);
-            const int64_t r = __builtin_amdgcn_readlane(my_row, ec);
-            c[e] = C[r * ldc + k];
-            d[e] = Dt[j * K + k];
-        }
+            for (int u = 0; u < SDDMM_ROUNDS; ++u) {
+                const int e = (r0 + u) * G + g < cnt ? (r0 + u) * G + g : cnt - 1;
+                const int64_t r = __shfl(my_row, e, 64), j = __shfl(my_col, e, 64);
+                if (K > 1) {
+                    c[u] = *reinterpret_cast<const spmm_pair *>(C + r * ldc + from);
+                    d[u] = *reinterpret_cast<const spmm_pair *>(Dt + j * K + from);
+                } else {
+                    c[u].x = c[u].y = C[r * ldc];
+                    d[u].x = d[u].y = Dt[j];
+                }
+            }
 #pragma unroll
-        for (int e = 0; e < SDDMM_E; ++e)
-            tile[e * SDDMM_LD + lane] = c[e] * d[e];
-        if (lane < cnt) {
-            if (kn == 64) {
-#pragma unroll 16
-                for (int q = 0; q < 64; ++q)
-                    t = t + tile[lane * SDDMM_LD + q];
-            } else {
-                for (int q = 0; q < kn; ++q)
-                    t = t + tile[lane * SDDMM_LD + q];
+            for (int u = 0; u < SDDMM_ROUNDS; ++u) {
+                const int e = (r0 + u) * G + g;
+                if (g < G && e < cnt) {
+                    const spmm_pair q = c[u] * d[u];
+                    double *to = tile + e * ld + 2 * sub;
+                    to[0] = half ? q.y : q.x;
+                    if (!half)
+                        to[1] = q.y;
+                }
             }
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        if (lane < cnt) {
+#pragma unroll 8
+            for (int q = 0; q < kn; ++q)
+                t = t + tile[lane * ld + q];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
     }
     if (lane < cnt)
         out[p] = val[p] * t;
@@ -2111,8 +2131,16 @@ static int sddmm_values(Csr *b, int64_t K, int64_t c_dptr, int64_t ldc, int64_t 
     COMET_CHK(csr_entry_rows(b, &rows));
     {
         KernelTimer t("sddmm_kernel");
-        sddmm_kernel<<<dim3((unsigned)ceil_div(b->nnz, SDDMM_W * SDDMM_E)), dim3(SDDMM_W * 64), 0, stream()>>>(
-            b->nnz, rows, b->crd, b->val, (const double *)c_dptr, ldc, (const double *)g_sddmm_dt.ptr, K, out);
+        const auto launch = [&](auto kernel, int entries) {
+            kernel<<<dim3((unsigned)ceil_div(b->nnz, SDDMM_W * entries)), dim3(SDDMM_W * 64), 0, stream()>>>(
+                b->nnz, rows, b->crd, b->val, (const double *)c_dptr, ldc, (const double *)g_sddmm_dt.ptr, K, out);
+        };
+        if (K <= 16)
+            launch(sddmm_kernel<64, 16>, 64);
+        else if (K <= 32)
+            launch(sddmm_kernel<32, 32>, 32);
+        else
+            launch(sddmm_kernel<16, 64>, 16);
     }
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;

@@ -197,3 +197,18 @@ def test_spmm_chunks_of_every_length_and_width(nrows, K, accumulate):
         assert np.all(np.abs(got - want) <= 1e-12 * bound)
         if K < 16 or K % 2 or pos[-1] < 1 << 19:
             assert np.array_equal(got[whole], want[whole])
+
+
+@pytest.mark.parametrize("K", [1, 2, 3, 5, 16, 17, 31, 32, 33, 63, 64, 65, 66, 130])
+@pytest.mark.parametrize("nnz", [1, 15, 17, 63, 65, 4097])
+def test_sddmm_of_every_tile_and_width(nnz, K):
+    rng = np.random.default_rng(nnz + K)
+    n, m = 70, 130
+    cells = np.sort(rng.choice(n * m, nnz, replace=False))
+    pos = np.concatenate([[0], np.cumsum(np.bincount(cells // m, minlength=n))]).astype(np.int64)
+    crd, val = (cells % m).astype(np.int32), rng.uniform(-1, 1, nnz)
+    C, D = rng.uniform(-1, 1, (n, K)), rng.uniform(-1, 1, (K, m))
+    out = rt.DeviceArray.from_numpy(np.full(nnz + 1, 7.0))
+    rt.sddmm(rt.CsrMatrix.from_arrays((n, m), pos, crd, val), rt.DeviceArray.from_numpy(C), rt.DeviceArray.from_numpy(D), out_values=out)
+    got = out.to_numpy()
+    assert np.array_equal(got[:nnz], orc.sddmm(pos, crd, val, C, D)) and got[nnz] == 7.0
