@@ -186,7 +186,12 @@ struct Csr {
     double iso_value = 0.0;
     // products taken with this matrix on the left so far (0, 1, more): the SpMM and SpMV plans, which cost tens of
     // products, are built when a matrix is multiplied for the second time (plan_at_once() builds them at the first)
-    int spmm_uses = 0, spmv_uses = 0;
+    int spmm_uses = 0, spmv_uses = 0, sddmm_uses = 0;
+    // SDDMM: the stored entries in an order that keeps columns of D in an L2, XCD x's from sddmm_start[x] on
+    // (sddmm_state: 0 not looked at, 1 not worth it, 2 made)
+    int sddmm_state = 0;
+    int32_t *sddmm_order = nullptr;
+    int64_t sddmm_start[9] = {};
 };
 
 // host arrays -> a new matrix (checked, registered by the caller), `more` going up in the same transfer; nullptr on failure

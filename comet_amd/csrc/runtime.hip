@@ -365,7 +365,10 @@ static void csr_drop_plans(Csr *c)
     c->heavy_ent = nullptr;
     c->heavy_row = c->heavy_code = nullptr;
     c->heavy_state = 0;
-    c->spmm_uses = c->spmv_uses = 0;
+    c->spmm_uses = c->spmv_uses = c->sddmm_uses = 0;
+    (void)dev_free(c->sddmm_order);
+    c->sddmm_order = nullptr;
+    c->sddmm_state = 0;
     c->heavy_nnz = c->heavy_rows = 0;
     (void)dev_free(c->spmm_chunk_row);
     c->spmm_chunk_row = nullptr;

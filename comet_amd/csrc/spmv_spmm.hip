@@ -2039,34 +2039,44 @@ extern "C" int comet_hip_densemat_csr_f64(int64_t csr, int64_t M, int64_t a_dptr
 // what the products of 8 KiB allow.  D is transposed first, so that its "row"
 // for a column j is contiguous; the row of every entry comes from a list kept in
 // B's handle (searching pos per entry cost 80 % of the time).
-// Bound by the gathers of D where it is larger than an L2.  (A lane per column
-// and 16 entries took 313 us for 250000 rows of 16 entries and K = 9, this 114;
-// 628 and 158 for 500000 rows and K = 3, 94 and 88 for 60001 and K = 64.)
+// Bound by the gathers of D, where it is larger than an L2 by their way there.
+// (A lane per column and 16 entries took 313 us for 250000 rows of 16 entries
+// and K = 9, this 95; 628 and 150 for 500000 rows and K = 3, 94 and 77 for 60001
+// and K = 64.)
 // ============================================================================
 constexpr int SDDMM_W = 4;               // wavefronts per workgroup
-constexpr int SDDMM_ROUNDS = 4;          // loads of C and of D under way per lane
-constexpr int SDDMM_TILE = 1088;         // products of a wavefront in LDS: 16 entries of 64 columns and 4 doubles' padding
+constexpr int SDDMM_TILE = 1152;         // products of a wavefront in LDS: 64 entries of 16 columns and 2 doubles' padding
 
-// E: entries of a wavefront; KT: most columns of a row that are products at a time, E * (KT + 1) of them fit
-template <int E, int KT>
-__global__ __launch_bounds__(SDDMM_W * 64) void sddmm_kernel(int64_t nnz, const int32_t *__restrict__ entry_row,
+// E: entries of a wavefront; KT: most columns of a row that are products at a time; ROUNDS: loads of C and of D under way
+// per lane
+// order (or null: as stored): the entries' order, XCD x's from start.v[x] on
+struct SddmmStart { int64_t v[9]; };
+template <int E, int KT, int ROUNDS, bool SMALL>
+__global__ __launch_bounds__(SDDMM_W * 64) void sddmm_kernel(int64_t nnz, const int32_t *__restrict__ order,
+                                                             SddmmStart start, const int32_t *__restrict__ entry_row,
                                                              const int32_t *__restrict__ crd,
                                                              const double *__restrict__ val,
                                                              const double *__restrict__ C, int64_t ldc,
                                                              const double *__restrict__ Dt, int64_t K,
                                                              double *__restrict__ out)
 {
-    static_assert(E * (KT + 1) <= SDDMM_TILE, "the products fit");
-    __shared__ double tiles[SDDMM_W][SDDMM_TILE];
+    // a row of products: 16-byte accesses of consecutive lanes, one row apart, fall into different banks
+    constexpr int LD = KT + 2;
+    static_assert(E * LD <= SDDMM_TILE, "the products fit");
+    __shared__ __align__(16) double tiles[SDDMM_W][SDDMM_TILE];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     double *tile = tiles[wave];
-    const int64_t base = ((int64_t)blockIdx.x * SDDMM_W + wave) * E;
-    if (base >= nnz)
+    const int64_t first = order ? start.v[blockIdx.x & 7] : 0, end = order ? start.v[(blockIdx.x & 7) + 1] : nnz;
+    const int64_t base = first + ((int64_t)(order ? blockIdx.x >> 3 : blockIdx.x) * SDDMM_W + wave) * E;
+    if (base >= end)
         return;
-    const int cnt = (int)(nnz - base < E ? nnz - base : E);
-    const int64_t p = base + (lane < cnt ? lane : cnt - 1);        // lane e < cnt owns entry base + e
+    const int cnt = (int)(end - base < E ? end - base : E);
+    int64_t p = base + (lane < cnt ? lane : cnt - 1);        // lane e < cnt owns entry base + e
+    if (order)
+        p = order[p];
     const int my_col = crd[p], my_row = entry_row[p];
+    const double v = val[p];
     double t = 0.0;
     for (int64_t kc = 0; kc < K; kc += KT) {
         const int kn = (int)(K - kc < KT ? K - kc : KT);
@@ -2075,43 +2085,277 @@ __global__ __launch_bounds__(SDDMM_W * 64) void sddmm_kernel(int64_t nnz, const 
         // the last lane of an odd kn has one column, and reads the one before it as well, if there is one
         const bool half = sub == L - 1 && (kn & 1);
         const int64_t from = kc + 2 * sub - (half && kc + 2 * sub > 0 ? 1 : 0);
-        const int ld = kn | 1;               // odd: lanes that walk a column of the tile hit all banks
-        for (int r0 = 0; r0 < rounds; r0 += SDDMM_ROUNDS) {
-            spmm_pair c[SDDMM_ROUNDS], d[SDDMM_ROUNDS];
+        for (int r0 = 0; r0 < rounds; r0 += ROUNDS) {
+            spmm_pair c[ROUNDS], d[ROUNDS];
 #pragma unroll
-            for (int u = 0; u < SDDMM_ROUNDS; ++u) {
+            for (int u = 0; u < ROUNDS; ++u) {
                 const int e = (r0 + u) * G + g < cnt ? (r0 + u) * G + g : cnt - 1;
-                const int64_t r = __shfl(my_row, e, 64), j = __shfl(my_col, e, 64);
-                if (K > 1) {
-                    c[u] = *reinterpret_cast<const spmm_pair *>(C + r * ldc + from);
-                    d[u] = *reinterpret_cast<const spmm_pair *>(Dt + j * K + from);
+                const int r = __shfl(my_row, e, 64), j = __shfl(my_col, e, 64);
+                const double *cp, *dp;
+                if constexpr (SMALL) {
+                    cp = reinterpret_cast<const double *>(reinterpret_cast<const char *>(C) +
+                                                          (__umul24((unsigned)r, (unsigned)ldc * 8u) + (unsigned)from * 8u));
+                    dp = reinterpret_cast<const double *>(reinterpret_cast<const char *>(Dt) +
+                                                          (__umul24((unsigned)j, (unsigned)K * 8u) + (unsigned)from * 8u));
                 } else {
-                    c[u].x = c[u].y = C[r * ldc];
-                    d[u].x = d[u].y = Dt[j];
+                    cp = C + (int64_t)r * ldc + from;
+                    dp = Dt + (int64_t)j * K + from;
+                }
+                if (K > 1) {
+                    c[u] = *reinterpret_cast<const spmm_pair *>(cp);
+                    d[u] = *reinterpret_cast<const spmm_pair *>(dp);
+                } else {
+                    c[u].x = c[u].y = *cp;
+                    d[u].x = d[u].y = *dp;
                 }
             }
 #pragma unroll
-            for (int u = 0; u < SDDMM_ROUNDS; ++u) {
+            for (int u = 0; u < ROUNDS; ++u) {
                 const int e = (r0 + u) * G + g;
                 if (g < G && e < cnt) {
-                    const spmm_pair q = c[u] * d[u];
-                    double *to = tile + e * ld + 2 * sub;
-                    to[0] = half ? q.y : q.x;
-                    if (!half)
-                        to[1] = q.y;
+                    double2 q = make_double2(c[u].x * d[u].x, c[u].y * d[u].y);
+                    if (half)
+                        q.x = q.y;
+                    *reinterpret_cast<double2 *>(tile + e * LD + 2 * sub) = q;
                 }
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
         if (lane < cnt) {
+            const double2 *mine = reinterpret_cast<const double2 *>(tile + lane * LD);
+            int q = 0;
 #pragma unroll 8
-            for (int q = 0; q < kn; ++q)
-                t = t + tile[lane * ld + q];
+            for (; q < kn / 2; ++q) {
+                const double2 w = mine[q];
+                t = t + w.x;
+                t = t + w.y;
+            }
+            if (kn & 1)
+                t = t + mine[q].x;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
     }
     if (lane < cnt)
-        out[p] = val[p] * t;
+        out[p] = v * t;
+}
+
+// ---------------------------------------------------------------------------
+// The order of the entries that keeps D in the L2s.  Every gather of a row of D
+// is a trip to the memory-side cache when D is larger than an L2 and columns come
+// as they please.  But in a matrix with long rows most entries are theirs, and
+// the rows of C they need are few: those entries are taken by blocks of columns,
+// every block by one XCD (the blocks dealt so that the XCDs have equal shares),
+// and within a block as stored.  The other entries go behind them as stored.
+// (500000 rows of 16 entries, nine tenths of them in rows of 128 and more,
+// K = 15: 301 -> 215 us; K = 64 681 -> 616.  What is left is the vector memory
+// path's: its return side is busy nine tenths of the time.)
+// ---------------------------------------------------------------------------
+constexpr int64_t SDDMM_SLICE = 4608;               // columns of a block: 2.25 MiB of D at K = 64
+constexpr int SDDMM_BLOCKS_MOST = 4096;
+constexpr int64_t SDDMM_LONG_ROWS = 4096;           // long rows at most: 2 MiB of C at K = 64
+constexpr int64_t SDDMM_ORDER_NNZ = 1 << 19;        // fewer entries are not worth ordering
+constexpr int64_t SDDMM_ORDER_D = 8 << 20;          // bytes of D: less stays in the L2s by itself
+
+// rows[b], entries[b]: rows of [2^b, 2^(b + 1)) entries, and the entries in them
+__global__ __launch_bounds__(256) void sddmm_row_lengths(const int64_t *__restrict__ pos, int64_t nrows,
+                                                         unsigned long long *__restrict__ rows,
+                                                         unsigned long long *__restrict__ entries)
+{
+    __shared__ unsigned long long n[64], s[64];
+    if (threadIdx.x < 64)
+        n[threadIdx.x] = s[threadIdx.x] = 0;
+    __syncthreads();
+    for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < nrows; r += (int64_t)gridDim.x * 256) {
+        const unsigned long long len = (unsigned long long)(pos[r + 1] - pos[r]);
+        if (len) {
+            const int b = 63 - __clzll((long long)len);
+            atomicAdd(&n[b], 1ull);
+            atomicAdd(&s[b], len);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 64 && n[threadIdx.x]) {
+        atomicAdd(&rows[threadIdx.x], n[threadIdx.x]);
+        atomicAdd(&entries[threadIdx.x], s[threadIdx.x]);
+    }
+}
+
+// count[c / slice]: entries of long rows in the block
+__global__ __launch_bounds__(256) void sddmm_block_counts(int64_t nnz, const int32_t *__restrict__ entry_row,
+                                                          const int32_t *__restrict__ crd, const int64_t *__restrict__ pos,
+                                                          int64_t min_len, int64_t slice, int nblocks,
+                                                          unsigned *__restrict__ count)
+{
+    __shared__ unsigned n[SDDMM_BLOCKS_MOST];
+    for (int b = threadIdx.x; b < nblocks; b += 256)
+        n[b] = 0;
+    __syncthreads();
+    for (int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x; p < nnz; p += (int64_t)gridDim.x * 256) {
+        const int64_t r = entry_row[p];
+        if (pos[r + 1] - pos[r] >= min_len)
+            atomicAdd(&n[crd[p] / slice], 1u);
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < nblocks; b += 256)
+        if (n[b])
+            atomicAdd(&count[b], n[b]);
+}
+
+// where[first[b] + share]: the place of a share of block b in the order; short_ends[x]: the entries of short rows up to
+// this one are XCD x's, and come behind its blocks, at short_place[x]
+struct SddmmShort { int64_t ends[8]; int32_t place[8]; };
+__global__ __launch_bounds__(256) void sddmm_keys(int64_t nnz, const int32_t *__restrict__ entry_row,
+                                                  const int32_t *__restrict__ crd, const int64_t *__restrict__ pos,
+                                                  int64_t min_len, int64_t slice, const int32_t *__restrict__ first,
+                                                  const int32_t *__restrict__ where, SddmmShort shorts,
+                                                  uint64_t *__restrict__ keys, uint32_t *__restrict__ idx)
+{
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p >= nnz)
+        return;
+    const int64_t r = entry_row[p];
+    int key;
+    if (pos[r + 1] - pos[r] >= min_len) {
+        const int b = (int)(crd[p] / slice);
+        const int shares = first[b + 1] - first[b];
+        key = where[first[b] + (shares > 1 ? (int)(p * shares / nnz) : 0)];
+    } else {
+        int x = 0;
+        while (x < 7 && p >= shorts.ends[x])
+            ++x;
+        key = shorts.place[x];
+    }
+    keys[p] = (uint64_t)key;
+    idx[p] = (uint32_t)p;
+}
+
+// start[x] = first entry whose key is limit[x] or more
+__global__ void sddmm_starts(int64_t nnz, const uint64_t *__restrict__ keys, SddmmStart limit, int64_t *__restrict__ start)
+{
+    if (threadIdx.x >= 9)
+        return;
+    int64_t lo = 0, hi = nnz;
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if ((int64_t)keys[mid] < limit.v[threadIdx.x])
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    start[threadIdx.x] = lo;
+}
+
+static Workspace g_sddmm_plan;
+
+static int sddmm_order(Csr *b, const int32_t *rows)
+{
+    b->sddmm_state = 1;
+    if (b->nnz >= (1ll << 31))
+        return COMET_HIP_OK;
+    // ---- which rows are long
+    COMET_CHK(g_sddmm_plan.ensure(sizeof(uint64_t) * 128 + sizeof(int32_t) * 2 * (SDDMM_BLOCKS_MOST + 1) + 9 * sizeof(int64_t), false));
+    unsigned long long *hist = (unsigned long long *)g_sddmm_plan.ptr, lengths[128];
+    COMET_HIPCHK(hipMemsetAsync(hist, 0, sizeof lengths, stream()));
+    sddmm_row_lengths<<<dim3((unsigned)std::min<int64_t>(ceil_div(b->nrows, 256), 1024)), dim3(256), 0, stream()>>>(
+        b->pos, b->nrows, hist, hist + 64);
+    COMET_HIPCHK(hipMemcpyAsync(lengths, hist, sizeof lengths, hipMemcpyDeviceToHost, stream()));
+    COMET_CHK(stream_wait());
+    int bits = 63;
+    int64_t nlong = 0, in_long = 0;
+    while (bits >= 5 && nlong + (int64_t)lengths[bits] <= SDDMM_LONG_ROWS) {
+        nlong += (int64_t)lengths[bits];
+        in_long += (int64_t)lengths[64 + bits];
+        --bits;
+    }
+    const int64_t min_len = 1ll << (bits + 1);
+    if (in_long * 3 < b->nnz)          // less than a third of the entries: not worth a plan
+        return COMET_HIP_OK;
+    // ---- the blocks of columns, and which XCD takes which
+    const int64_t slice = std::max<int64_t>(SDDMM_SLICE, ceil_div(b->ncols, SDDMM_BLOCKS_MOST));
+    const int nblocks = (int)ceil_div(b->ncols, slice);
+    unsigned *count = (unsigned *)(hist + 128);
+    COMET_HIPCHK(hipMemsetAsync(count, 0, sizeof(unsigned) * (size_t)nblocks, stream()));
+    sddmm_block_counts<<<dim3((unsigned)std::min<int64_t>(ceil_div(b->nnz, 1024), 2048)), dim3(256), 0, stream()>>>(
+        b->nnz, rows, b->crd, b->pos, min_len, slice, nblocks, count);
+    std::vector<unsigned> counts((size_t)nblocks);
+    COMET_HIPCHK(hipMemcpyAsync(counts.data(), count, sizeof(unsigned) * (size_t)nblocks, hipMemcpyDeviceToHost, stream()));
+    COMET_CHK(stream_wait());
+    // a block with more than a 32nd of the entries is shared out
+    struct Share { int64_t size; int id; };
+    std::vector<int32_t> first((size_t)nblocks + 1, 0);
+    std::vector<Share> shares;
+    for (int c = 0; c < nblocks; ++c) {
+        const int n = (int)std::max<int64_t>(1, ceil_div((int64_t)counts[(size_t)c] * 32, in_long));
+        for (int k = 0; k < n; ++k)
+            shares.push_back({counts[(size_t)c] / n, first[(size_t)c] + k});
+        first[(size_t)c + 1] = first[(size_t)c] + n;
+    }
+    std::stable_sort(shares.begin(), shares.end(), [](const Share &a, const Share &c) { return a.size > c.size; });
+    int64_t load[8] = {};
+    std::vector<std::vector<int>> of(8);
+    for (const Share &s : shares) {
+        const int x = (int)(std::min_element(load, load + 8) - load);
+        load[x] += s.size;
+        of[(size_t)x].push_back(s.id);
+    }
+    // the short rows fill up to equal shares
+    SddmmShort shorts;
+    SddmmStart limit;
+    std::vector<int32_t> where((size_t)first[(size_t)nblocks]);
+    const double each = (double)b->nnz / 8, in_short = (double)(b->nnz - in_long);
+    double given = 0.0;
+    int32_t place = 0;
+    for (int x = 0; x < 8; ++x) {
+        limit.v[x] = place;
+        std::sort(of[(size_t)x].begin(), of[(size_t)x].end());
+        for (int id : of[(size_t)x])
+            where[(size_t)id] = place++;
+        given += std::max(0.0, each - (double)load[x]);
+        shorts.ends[x] = in_short > 0 ? (int64_t)((double)b->nnz * std::min(1.0, given / in_short)) : b->nnz;
+        shorts.place[x] = place++;
+    }
+    limit.v[8] = place;
+    int end_bit = 1;
+    while ((1ll << end_bit) <= place)
+        ++end_bit;
+    // ---- the order
+    int32_t *d_first = (int32_t *)count, *d_where = nullptr;
+    uint64_t *keys = nullptr;
+    uint32_t *idx = nullptr, *order = nullptr;
+    int64_t *d_start = (int64_t *)(hist + 128) + SDDMM_BLOCKS_MOST + 1;
+    const size_t n = (size_t)b->nnz;
+    int rc = COMET_HIP_OK;
+    if (dev_malloc((void **)&keys, 16 * n) != hipSuccess || dev_malloc((void **)&idx, 4 * n) != hipSuccess ||
+        dev_malloc((void **)&order, 4 * n) != hipSuccess ||
+        dev_malloc((void **)&d_where, sizeof(int32_t) * where.size()) != hipSuccess) {
+        (void)hipGetLastError();          // without the room the entries are taken as stored
+        (void)dev_free(order);
+        order = nullptr;
+    } else {
+        const auto run = [&]() -> int {
+            COMET_HIPCHK(hipMemcpyAsync(d_first, first.data(), sizeof(int32_t) * first.size(), hipMemcpyHostToDevice, stream()));
+            COMET_HIPCHK(hipMemcpyAsync(d_where, where.data(), sizeof(int32_t) * where.size(), hipMemcpyHostToDevice, stream()));
+            sddmm_keys<<<dim3((unsigned)ceil_div(b->nnz, 256)), dim3(256), 0, stream()>>>(
+                b->nnz, rows, b->crd, b->pos, min_len, slice, d_first, d_where, shorts, keys, idx);
+            COMET_CHK(sort_pairs_u64_u32(keys, keys + n, idx, order, b->nnz, end_bit));
+            sddmm_starts<<<dim3(1), dim3(64), 0, stream()>>>(b->nnz, keys + n, limit, d_start);
+            COMET_HIPCHK(hipMemcpyAsync(b->sddmm_start, d_start, sizeof b->sddmm_start, hipMemcpyDeviceToHost, stream()));
+            return stream_wait();
+        };
+        rc = run();
+    }
+    (void)dev_free(keys);
+    (void)dev_free(idx);
+    (void)dev_free(d_where);
+    if (rc != COMET_HIP_OK) {
+        (void)dev_free(order);
+        return rc;
+    }
+    if (order) {
+        b->sddmm_order = (int32_t *)order;
+        b->sddmm_state = 2;
+    }
+    return COMET_HIP_OK;
 }
 
 static Workspace g_sddmm_dt;
@@ -2129,18 +2373,35 @@ static int sddmm_values(Csr *b, int64_t K, int64_t c_dptr, int64_t ldc, int64_t 
     }
     const int32_t *rows = nullptr;
     COMET_CHK(csr_entry_rows(b, &rows));
+    // ordering the entries costs some five products: made when the matrix is sampled at again
+    const bool plan_now = b->sddmm_uses > 0 || plan_at_once();
+    b->sddmm_uses = 1;
+    const bool large = b->nnz >= SDDMM_ORDER_NNZ && b->ncols * K * 8 >= SDDMM_ORDER_D;
+    if (large && plan_now && b->sddmm_state == 0)
+        COMET_CHK(sddmm_order(b, rows));
+    const int32_t *order = large && b->sddmm_state == 2 ? b->sddmm_order : nullptr;
     {
         KernelTimer t("sddmm_kernel");
+        SddmmStart start{};
+        int64_t longest = 0;
+        for (int x = 0; x < 9 && order; ++x) {
+            start.v[x] = b->sddmm_start[x];
+            longest = x > 0 ? std::max(longest, start.v[x] - start.v[x - 1]) : 0;
+        }
         const auto launch = [&](auto kernel, int entries) {
-            kernel<<<dim3((unsigned)ceil_div(b->nnz, SDDMM_W * entries)), dim3(SDDMM_W * 64), 0, stream()>>>(
-                b->nnz, rows, b->crd, b->val, (const double *)c_dptr, ldc, (const double *)g_sddmm_dt.ptr, K, out);
+            const int64_t groups = order ? 8 * ceil_div(longest, SDDMM_W * entries) : ceil_div(b->nnz, SDDMM_W * entries);
+            kernel<<<dim3((unsigned)groups), dim3(SDDMM_W * 64), 0, stream()>>>(
+                b->nnz, order, start, rows, b->crd, b->val, (const double *)c_dptr, ldc, (const double *)g_sddmm_dt.ptr, K, out);
         };
+        // rows named in 24 bits, C and D within 4 GiB: an address is a 24-bit multiply and an add
+        const bool small = b->nrows <= 1 << 24 && b->ncols <= 1 << 24 && ldc * 8 < 1 << 24 && K * 8 < 1 << 24 &&
+                           b->nrows * ldc * 8 < (1ll << 32) && b->ncols * K * 8 < (1ll << 32);
         if (K <= 16)
-            launch(sddmm_kernel<64, 16>, 64);
+            small ? launch(sddmm_kernel<64, 16, 4, true>, 64) : launch(sddmm_kernel<64, 16, 4, false>, 64);
         else if (K <= 32)
-            launch(sddmm_kernel<32, 32>, 32);
+            small ? launch(sddmm_kernel<32, 32, 8, true>, 32) : launch(sddmm_kernel<32, 32, 8, false>, 32);
         else
-            launch(sddmm_kernel<16, 64>, 16);
+            small ? launch(sddmm_kernel<16, 64, 8, true>, 16) : launch(sddmm_kernel<16, 64, 8, false>, 16);
     }
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;

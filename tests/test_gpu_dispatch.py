@@ -212,3 +212,24 @@ def test_sddmm_of_every_tile_and_width(nnz, K):
     rt.sddmm(rt.CsrMatrix.from_arrays((n, m), pos, crd, val), rt.DeviceArray.from_numpy(C), rt.DeviceArray.from_numpy(D), out_values=out)
     got = out.to_numpy()
     assert np.array_equal(got[:nnz], orc.sddmm(pos, crd, val, C, D)) and got[nnz] == 7.0
+
+
+@pytest.mark.parametrize("K", [27, 64])
+@pytest.mark.parametrize("hub", [False, True])
+def test_sddmm_in_an_order_that_keeps_columns_close(K, hub):
+    # enough entries in long rows, and a D that is too large for an L2: the second call takes them by blocks of columns; with
+    # a hub half of them name columns of one block, which several XCDs then share
+    rng = np.random.default_rng(K)
+    n, m = 2500, 40_000
+    lens = np.where(np.arange(n) % 25 == 3, 6000, rng.integers(0, 9, n))
+    rows = [np.sort(rng.choice(m, l, replace=False)) if not hub or l < 100 else
+            np.sort(np.concatenate([rng.choice(4000, l // 2, replace=False), 4000 + rng.choice(m - 4000, l // 2, replace=False)]))
+            for l in lens]
+    pos, crd = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64), np.concatenate(rows).astype(np.int32)
+    val, C, D = rng.uniform(-1, 1, len(crd)), rng.uniform(-1, 1, (n, K)), rng.uniform(-1, 1, (K, m))
+    S, dC, dD = rt.CsrMatrix.from_arrays((n, m), pos, crd, val), rt.DeviceArray.from_numpy(C), rt.DeviceArray.from_numpy(D)
+    want = orc.sddmm(pos, crd, val, C, D)
+    for _ in range(3):
+        out = rt.DeviceArray(len(crd), zero=True)
+        rt.sddmm(S, dC, dD, out_values=out)
+        assert np.array_equal(out.to_numpy(), want)
