@@ -100,6 +100,7 @@ struct RowListEntry {
     int64_t rb = 0, re = 0, dense_threshold = 0, wide_threshold = 0, mask_fill = 0;
     int32_t *rows = nullptr;     // device, re - rb entries
     int64_t *bounds = nullptr;   // device, 3 entries
+    int64_t counts[3] = {-1, -1, -1};          // the same, where the host has asked for them
 };
 uint64_t next_csr_uid();
 
@@ -218,8 +219,8 @@ struct KernelTimer {
 
 static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// exclusive scan of int64 counts into pos[0..n] (pos[n] = total), on the stream
-int exclusive_scan_i64(const int64_t *counts, int64_t n, int64_t *pos);
+// exclusive scan of int64 counts into pos[0..n] (pos[n] = total), on the stream; total: a mailbox's word for the sum, or null
+int exclusive_scan_i64(const int64_t *counts, int64_t n, int64_t *pos, int64_t *total = nullptr);
 
 // stable radix sort of n (key, payload) pairs on the stream, comparing key bits [0, end_bit)
 int sort_pairs_u64_u32(const uint64_t *keys_in, uint64_t *keys_out, const uint32_t *vals_in, uint32_t *vals_out,

@@ -669,8 +669,9 @@ __global__ __launch_bounds__(256) void dot_chunk_compact(int64_t rb, int64_t re,
     }
 }
 
-// chunk_before[c]: pairs that met a product in front of chunk c of n; the number of all of them behind the last.
-static int dot_chunks(int64_t n, const uint8_t *pair_hit, int64_t **chunk_before, int64_t *chunks)
+// chunk_before[c]: pairs that met a product in front of chunk c of n; the number of all of them behind the last (and in
+// total, a mailbox's word).
+static int dot_chunks(int64_t n, const uint8_t *pair_hit, int64_t **chunk_before, int64_t *chunks, int64_t *total = nullptr)
 {
     *chunks = ceil_div(n, PAIR_CHUNK);
     COMET_CHK(g_pair_chunk.ensure(sizeof(int64_t) * 2 * (size_t)(*chunks + 1), false));
@@ -680,5 +681,5 @@ static int dot_chunks(int64_t n, const uint8_t *pair_hit, int64_t **chunk_before
         KernelTimer t("spgemm_symbolic_dot_count");
         dot_chunk_count<<<dim3((unsigned)*chunks), dim3(256), 0, stream()>>>(n, pair_hit, kept);
     }
-    return exclusive_scan_i64(kept, *chunks, *chunk_before);
+    return exclusive_scan_i64(kept, *chunks, *chunk_before, total);
 }

@@ -598,7 +598,7 @@ __global__ __launch_bounds__(SCAN_T) void scan_totals_inplace(int64_t *__restric
 
 __global__ __launch_bounds__(SCAN_T) void scan_apply(const int64_t *__restrict__ in, int64_t n,
                                                      const int64_t *__restrict__ block_off,
-                                                     int64_t nblocks, int64_t *__restrict__ pos)
+                                                     int64_t nblocks, int64_t *__restrict__ pos, int64_t *total)
 {
     __shared__ int64_t lds[SCAN_T / 64 + 1];
     int64_t base = (int64_t)blockIdx.x * SCAN_B + (int64_t)threadIdx.x * SCAN_E;
@@ -615,16 +615,21 @@ __global__ __launch_bounds__(SCAN_T) void scan_apply(const int64_t *__restrict__
             pos[base + e] = run;
         run += v[e];
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0)
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
         pos[n] = block_off[nblocks];
+        if (total)
+            *total = block_off[nblocks];
+    }
 }
 
 static Workspace g_scan_ws;
 
-int exclusive_scan_i64(const int64_t *counts, int64_t n, int64_t *pos)
+int exclusive_scan_i64(const int64_t *counts, int64_t n, int64_t *pos, int64_t *total)
 {
     if (n <= 0) {
         COMET_HIPCHK(hipMemsetAsync(pos, 0, sizeof(int64_t), stream()));
+        if (total)
+            *total = 0;
         return COMET_HIP_OK;
     }
     int64_t nblocks = ceil_div(n, SCAN_B);
@@ -640,7 +645,7 @@ int exclusive_scan_i64(const int64_t *counts, int64_t n, int64_t *pos)
     }
     {
         KernelTimer t("scan_apply");
-        scan_apply<<<dim3((unsigned)nblocks), dim3(SCAN_T), 0, stream()>>>(counts, n, tot, nblocks, pos);
+        scan_apply<<<dim3((unsigned)nblocks), dim3(SCAN_T), 0, stream()>>>(counts, n, tot, nblocks, pos, total);
     }
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;

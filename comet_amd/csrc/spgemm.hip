@@ -381,6 +381,7 @@ struct RowList {
     const int32_t *rows;       // row - row_begin, by descending number of products
     const int64_t *bounds;     // [0] rows with >= dense_threshold products, [1] rows with any product,
                                // [2] rows with >= wide_threshold products (a prefix of [0])
+    int64_t counts[3];         // the same on the host where it asked for them, else -1
 };
 __device__ inline void list_range(const RowList &l, int part, int64_t *first, int64_t *end)
 {
@@ -1590,7 +1591,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_kernel(
 // ticket, and a workgroup only ever waits for earlier tickets, which running workgroups hold: the one with the
 // earliest unfinished ticket waits for nobody.  The wait is bounded all the same (`patience` polls, after
 // which *gave_up is set and the row is wrong: the host then fails the call).
-// A ticket is DB_ROWS consecutive rows of the list, so that the loads which lead to a row's slices (its entries
+// A ticket is up to DB_ROWS consecutive rows of the list, so that the loads which lead to a row's slices (its entries
 // of A, their block pointers) are issued while the row before is walked.
 // ---------------------------------------------------------------------------
 struct DenseRow {
@@ -1625,7 +1626,7 @@ template <bool SEMI, typename COL>
 __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
     const DenseRow *__restrict__ rows, int64_t nd, const int32_t *__restrict__ Acrd, const double *__restrict__ Aval,
     const COL *__restrict__ Bcrd, const double *__restrict__ Bval, const int64_t *__restrict__ blkptr, int nblk,
-    unsigned long long *ticket, int32_t *before, int patience, int *gave_up, int32_t *__restrict__ Ccrd,
+    unsigned long long *ticket, int32_t *before, int rows_each, int patience, int *gave_up, int32_t *__restrict__ Ccrd,
     double *__restrict__ Cval, int reduce_op, int mult_op)
 {
     __shared__ int64_t row_slot;
@@ -1645,13 +1646,13 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
         block_touched[threadIdx.x] = 0;
     lds_barrier();
     int visit = 0;
-    const int64_t nchunks = (nd + DB_ROWS - 1) / DB_ROWS;
+    const int64_t nchunks = (nd + rows_each - 1) / rows_each;
     const int64_t u_end = nchunks * nblk;
     int64_t u = draw_row<true>(ticket, 0, &row_slot);
     while (u < u_end) {
         const int cb = (int)(u / nchunks);
-        const int64_t r0 = (u - cb * nchunks) * DB_ROWS;
-        const int nr = (int)(nd - r0 < DB_ROWS ? nd - r0 : DB_ROWS);
+        const int64_t r0 = (u - cb * nchunks) * rows_each;
+        const int nr = (int)(nd - r0 < rows_each ? nd - r0 : rows_each);
         const int col0 = cb << SG_CB_LOG;
         DenseRow mine;
         mine.as = mine.coff = 0;
@@ -1752,7 +1753,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
                     ahead = __hip_atomic_fetch_max(mark, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
                 if (ahead < 0) {
-                    __hip_atomic_store(gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);          // in host memory
                     ahead = 0;
                 }
                 return ahead;
@@ -2402,14 +2403,13 @@ __global__ void fill_iota_f64(int64_t n, double *__restrict__ out)
 }
 
 struct SgScratch {
-    Workspace ticket;     // one 64-bit row counter
+    Workspace ticket;     // SG_TICKETS 64-bit row counters
     Workspace rowcount;   // int64[nrows] / double[nrows]
     Workspace gbm;        // global bitmaps (only when the bitmap does not fit LDS)
     Workspace gmask;      // global mask bitmaps (masked numeric)
     Workspace slabs;      // dense accumulators, zero between calls
     Workspace dense_rows;     // DenseRow[] and before[] of spgemm_numeric_dense_blocks_kernel
     Workspace dense_before;
-    Workspace gave_up;        // its flag, zero between calls
 };
 static SgScratch g_sg;
 
@@ -2447,10 +2447,13 @@ static int sg_allow_lds(K kernel, size_t bytes)
     return COMET_HIP_OK;
 }
 
+// the row counters of a phase's kernels, one each
+constexpr int SG_TICKETS = 4;          // (32 bytes: one fill)
+static unsigned long long *sg_ticket(int k) { return (unsigned long long *)g_sg.ticket.ptr + k; }
 static int sg_reset_ticket()
 {
-    COMET_CHK(g_sg.ticket.ensure(sizeof(unsigned long long), false));
-    COMET_HIPCHK(hipMemsetAsync(g_sg.ticket.ptr, 0, sizeof(unsigned long long), stream()));
+    COMET_CHK(g_sg.ticket.ensure(SG_TICKETS * sizeof(unsigned long long), false));
+    COMET_HIPCHK(hipMemsetAsync(g_sg.ticket.ptr, 0, SG_TICKETS * sizeof(unsigned long long), stream()));
     return COMET_HIP_OK;
 }
 
@@ -2516,8 +2519,10 @@ static SgRowLists g_rl;
 constexpr size_t SG_ROW_LISTS_KEPT = 24;
 static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64_t dense_threshold,
                        int64_t wide_threshold, RowList *out, const Csr *long_mask = nullptr,
-                       int64_t mask_fill = 0)
+                       int64_t mask_fill = 0, bool want_counts = false)
 {
+    for (int64_t &c : out->counts)
+        c = -1;
     const int64_t n = re - rb;
     static const bool keep = getenv("COMET_HIP_SPGEMM_NO_LIST_CACHE") == nullptr;
     Csr *owner = const_cast<Csr *>(a);
@@ -2535,6 +2540,7 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
                 e.dense_threshold == dense_threshold && e.wide_threshold == wide_threshold && e.mask_fill == mask_fill) {
                 out->rows = e.rows;
                 out->bounds = e.bounds;
+                std::copy(e.counts, e.counts + 3, out->counts);
                 return COMET_HIP_OK;
             }
     COMET_CHK(g_rl.rowprod.ensure(sizeof(int64_t) * (size_t)n, false));
@@ -2576,6 +2582,14 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
         }
         COMET_HIPCHK(hipMemcpyAsync(key.rows, g_rl.idx_out.ptr, 4 * (size_t)n, hipMemcpyDeviceToDevice, stream()));
         COMET_HIPCHK(hipMemcpyAsync(key.bounds, g_rl.bounds.ptr, 24, hipMemcpyDeviceToDevice, stream()));
+        if (want_counts) {          // once per list instead of once per product
+            int64_t *word = nullptr;
+            COMET_CHK(mailbox((void **)&word));
+            COMET_HIPCHK(hipMemcpyAsync(word, key.bounds, 24, hipMemcpyDeviceToHost, stream()));
+            COMET_CHK(stream_wait());
+            std::copy(word, word + 3, key.counts);
+            std::copy(word, word + 3, out->counts);
+        }
         owner->row_lists.push_back(key);
         out->rows = key.rows;
         out->bounds = key.bounds;
@@ -2831,7 +2845,7 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     if (mdense)         // those rows sort in front (sg_row_keys): bounds[0] = bounds[2] = their number
         COMET_CHK(sg_row_list(a, b, rb, re, 1ll << 61, 1ll << 61, &list, m, SG_HASH_FILL));
     else
-        COMET_CHK(sg_row_list(a, b, rb, re, dense_threshold, dense ? wide : SG_NO_DENSE, &list));
+        COMET_CHK(sg_row_list(a, b, rb, re, dense_threshold, dense ? wide : SG_NO_DENSE, &list, nullptr, 0, dense));
     uint32_t *gbm = nullptr, *gmask = nullptr;
     if (!g.lds || m) {          // the output row's bitmap is in HBM when LDS holds the mask row instead
         COMET_CHK(g_sg.gbm.ensure(sizeof(uint32_t) * g.bm_words * (size_t)g.groups, true));
@@ -2858,7 +2872,9 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     do {                                                                                                   \
         if (semi) LAUNCH_NUM(L, M, true); else LAUNCH_NUM(L, M, false);                                    \
     } while (0)
-    if (g.lds) {
+    if (list.counts[1] >= 0 && list.counts[1] == list.counts[0])
+        ;          // every row with products is a heavy one
+    else if (g.lds) {
         if (m) LAUNCH_NUM_S(true, true); else LAUNCH_NUM_S(true, false);
     } else {
         if (m) LAUNCH_NUM_S(false, true); else LAUNCH_NUM_S(false, false);
@@ -2870,24 +2886,29 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     // tests run both)
     const bool by_blocks = dense && a->nnz < (1ll << 30) && getenv("COMET_HIP_SPGEMM_ROW_MAJOR") == nullptr;
     bool ran_blocks = false;
+    int64_t *word = nullptr;
+    COMET_CHK(mailbox((void **)&word));
+    int *gave_up = (int *)(word + 1);
     if (by_blocks) {
-        int64_t nd = 0;
-        COMET_HIPCHK(hipMemcpyAsync(&nd, list.bounds + 2, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
-        COMET_CHK(stream_wait());
+        int64_t nd = list.counts[2];
+        if (nd < 0) {
+            COMET_HIPCHK(hipMemcpyAsync(word, list.bounds + 2, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
+            COMET_CHK(stream_wait());
+            nd = *(volatile int64_t *)word;
+        }
         if (nd > 0) {
             ran_blocks = true;
             COMET_CHK(g_sg.dense_rows.ensure(sizeof(DenseRow) * (size_t)nd, false));
             COMET_CHK(g_sg.dense_before.ensure(sizeof(int32_t) * (size_t)nd * (size_t)nblk, false));
-            COMET_CHK(g_sg.gave_up.ensure(sizeof(int), true));
-            // cleared before every launch that can set it: a call that fails between the launch and the read
-            // below must not leave it set for the next product
-            COMET_HIPCHK(hipMemsetAsync(g_sg.gave_up.ptr, 0, sizeof(int), stream()));
-            COMET_CHK(sg_reset_ticket());
+            gave_up[0] = 0;
             int patience = DB_PATIENCE;
             if (const char *e = getenv("COMET_HIP_SPGEMM_PATIENCE"))
                 patience = atoi(e);
             KernelTimer t("spgemm_numeric_dense_blocks");
             const dim3 cus((unsigned)(num_cus() > 0 ? num_cus() : 256));
+            // as many rows to a ticket as leave every CU some four of them (8 to each of 50 CUs: 78 us for a graph of 1024
+            // vertices, the others idle)
+            const int rows_each = (int)std::max<int64_t>(1, std::min<int64_t>(DB_ROWS, nd * nblk / (4 * (int64_t)cus.x)));
             spgemm_dense_rows<<<dim3((unsigned)ceil_div(nd * nblk, 256)), dim3(256), 0, stream()>>>(
                 rb, list, nd, nblk, a->pos, Cpos, (DenseRow *)g_sg.dense_rows.ptr, (int32_t *)g_sg.dense_before.ptr);
 #define LAUNCH_BLOCKS_C(S, COL, CRD)                                                                       \
@@ -2895,8 +2916,8 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         COMET_CHK(sg_allow_lds(spgemm_numeric_dense_blocks_kernel<S, COL>, SG_DENSE_LDS));                 \
         spgemm_numeric_dense_blocks_kernel<S, COL><<<cus, block, SG_DENSE_LDS, stream()>>>(                \
             (const DenseRow *)g_sg.dense_rows.ptr, nd, a->crd, a->val, CRD, b->val, b->sg_blkptr, nblk,    \
-            (unsigned long long *)g_sg.ticket.ptr, (int32_t *)g_sg.dense_before.ptr, patience,             \
-            (int *)g_sg.gave_up.ptr, Ccrd, Cval, reduce_op, mult_op);                                      \
+            sg_ticket(1), (int32_t *)g_sg.dense_before.ptr, rows_each, patience, gave_up, Ccrd, Cval,      \
+            reduce_op, mult_op);                                                                           \
     } while (0)
 #define LAUNCH_BLOCKS(S)                                                                                   \
     do {                                                                                                   \
@@ -2912,7 +2933,6 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         }
     }
     if ((dense && !by_blocks) || mdense) {
-        COMET_CHK(sg_reset_ticket());
         KernelTimer t(mdense ? "spgemm_numeric_dense_masked" : "spgemm_numeric_dense");
         const dim3 cus((unsigned)(num_cus() > 0 ? num_cus() : 256));
 #define LAUNCH_DENSE_C(S, M, COL, CRD)                                                                     \
@@ -2920,8 +2940,7 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         COMET_CHK(sg_allow_lds(spgemm_numeric_dense_kernel<S, M, COL>, SG_DENSE_LDS));                     \
         spgemm_numeric_dense_kernel<S, M, COL><<<cus, block, SG_DENSE_LDS, stream()>>>(                    \
             rb, re, a->pos, a->crd, a->val, CRD, b->val, m ? m->pos : nullptr, m ? m->crd : nullptr,       \
-            b->sg_blkptr, nblk, (unsigned long long *)g_sg.ticket.ptr, list, Cpos, Ccrd, Cval, reduce_op,  \
-            mult_op);                                                                                      \
+            b->sg_blkptr, nblk, sg_ticket(1), list, Cpos, Ccrd, Cval, reduce_op, mult_op);                                                                                      \
     } while (0)
 #define LAUNCH_DENSE(S, M)                                                                                 \
     do {                                                                                                   \
@@ -2939,31 +2958,26 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
 #undef LAUNCH_DENSE
         COMET_HIPCHK(hipGetLastError());
     }
-    if (dense) {
-        COMET_CHK(sg_reset_ticket());
+    if (dense && (list.counts[0] < 0 || list.counts[0] > list.counts[2])) {
         KernelTimer t("spgemm_numeric_span");
         const dim3 cus((unsigned)(num_cus() > 0 ? num_cus() : 256));
         if (semi) {
             COMET_CHK(sg_allow_lds(spgemm_numeric_span_kernel<true>, SG_SPAN_LDS));
             spgemm_numeric_span_kernel<true><<<cus, block, SG_SPAN_LDS, stream()>>>(
                 rb, re, a->pos, a->crd, a->val, b->crd, b->val, b->sg_blkptr, nblk,
-                (unsigned long long *)g_sg.ticket.ptr, list, Cpos, Ccrd, Cval, reduce_op, mult_op);
+                sg_ticket(2), list, Cpos, Ccrd, Cval, reduce_op, mult_op);
         } else {
             COMET_CHK(sg_allow_lds(spgemm_numeric_span_kernel<false>, SG_SPAN_LDS));
             spgemm_numeric_span_kernel<false><<<cus, block, SG_SPAN_LDS, stream()>>>(
                 rb, re, a->pos, a->crd, a->val, b->crd, b->val, b->sg_blkptr, nblk,
-                (unsigned long long *)g_sg.ticket.ptr, list, Cpos, Ccrd, Cval, reduce_op, mult_op);
+                sg_ticket(2), list, Cpos, Ccrd, Cval, reduce_op, mult_op);
         }
         COMET_HIPCHK(hipGetLastError());
     }
     if (ran_blocks) {           // did a workgroup stop waiting for the block before its own
-        int gave_up = 0;
-        COMET_HIPCHK(hipMemcpyAsync(&gave_up, g_sg.gave_up.ptr, sizeof(int), hipMemcpyDeviceToHost, stream()));
         COMET_CHK(stream_wait());
-        if (gave_up) {
-            COMET_HIPCHK(hipMemsetAsync(g_sg.gave_up.ptr, 0, sizeof(int), stream()));
+        if (*(volatile int *)gave_up)
             return set_error(COMET_HIP_ERR_HIP, "spgemm numeric: a column block's place in its row never arrived");
-        }
     }
     return COMET_HIP_OK;
 }
@@ -2986,10 +3000,13 @@ extern "C" int comet_hip_spgemm_csr_symbolic(int64_t ah, int64_t bh, int64_t mh,
         COMET_CHK(g_sg.rowcount.ensure(sizeof(int64_t) * (size_t)a->nrows, false));
         COMET_CHK(symbolic_counts(a, b, m, (int64_t *)g_sg.rowcount.ptr));
     }
-    COMET_CHK(exclusive_scan_i64((const int64_t *)g_sg.rowcount.ptr, a->nrows, pos));
+    int64_t *word = nullptr;
+    if (nnz_out)
+        COMET_CHK(mailbox((void **)&word));
+    COMET_CHK(exclusive_scan_i64((const int64_t *)g_sg.rowcount.ptr, a->nrows, pos, word));
     if (nnz_out) {
-        COMET_HIPCHK(hipMemcpyAsync(nnz_out, pos + a->nrows, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
         COMET_CHK(stream_wait());
+        *nnz_out = *(volatile int64_t *)word;
     }
     return COMET_HIP_OK;
 }
@@ -3044,7 +3061,7 @@ static int64_t masked_product_one_pass(const Csr *a, const Csr *b, const Csr *m,
     if (mailbox(&word) != COMET_HIP_OK ||
         pair_dot_values(const_cast<Csr *>(a), const_cast<Csr *>(b), const_cast<Csr *>(m), 0, a->nrows, &pair_val, &pair_hit,
                         &pairs, reduce_op, mult_op) != COMET_HIP_OK ||
-        dot_chunks(pairs, pair_hit, &before, &chunks) != COMET_HIP_OK)
+        dot_chunks(pairs, pair_hit, &before, &chunks, (int64_t *)word) != COMET_HIP_OK)
         return 0;
     Csr *c = new Csr();
     c->nrows = a->nrows;
@@ -3056,8 +3073,7 @@ static int64_t masked_product_one_pass(const Csr *a, const Csr *b, const Csr *m,
         csr_release(c);
         return 0;
     };
-    if (hipMemcpyAsync(word, before + chunks, sizeof(int64_t), hipMemcpyDeviceToHost, stream()) != hipSuccess ||
-        stream_wait() != COMET_HIP_OK)
+    if (stream_wait() != COMET_HIP_OK)
         return fail("reading the size of the product failed");
     c->nnz = *(volatile int64_t *)word;
     if (dev_malloc((void **)&c->pos, sizeof(int64_t) * (size_t)(a->nrows + 1)) != hipSuccess ||
