@@ -543,7 +543,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_symbolic_kernel(
     int64_t nrows, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
     const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd, const int64_t *__restrict__ Mpos,
     const int32_t *__restrict__ Mcrd, int logW, uint32_t *__restrict__ gbm, unsigned long long *ticket,
-    RowList list, int64_t *__restrict__ rowcount)
+    RowList list, int part, int64_t *__restrict__ rowcount)
 {
     __shared__ int64_t row_slot;
     __shared__ int wave_cnt[SG_WAVES];
@@ -560,7 +560,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_symbolic_kernel(
     }
     __syncthreads();
     int64_t t_first, t_end;
-    list_range(list, 2, &t_first, &t_end);
+    list_range(list, part, &t_first, &t_end);
     int64_t t = draw_row(ticket, t_first, &row_slot);
     while (t < t_end) {
         const int64_t i = list.rows[t];       // rows outside the list keep the zero the host put there
@@ -2402,6 +2402,129 @@ __global__ void fill_iota_f64(int64_t n, double *__restrict__ out)
         out[i] = (double)i;
 }
 
+// ---------------------------------------------------------------------------
+// Rows with few products, SM_PRODUCTS at most, of matrices of few columns: a row is over in a handful of loads that wait
+// for each other, so what counts is how many rows are under way.  A workgroup of four wavefronts has the row's bitmap,
+// with the number of columns before every word of it, and a value for every product it can have: 21 to 29 KiB of LDS,
+// four to seven to a CU.  Sixteen lanes take an entry of A at a time.  (A workgroup of 1024 lanes to a row, one or two to a
+// CU, took 74 us more of the structure and 103 of the values of A*A for 16000 vertices, edge factor 8, which these take 30
+// and 88 for.)
+// ---------------------------------------------------------------------------
+constexpr int SM_T = 256, SM_PRODUCTS = 2048, SM_COLS = 1 << 16;
+struct SmallRowLds {                     // behind the bitmap
+    double val[SM_PRODUCTS];
+    uint16_t col[SM_PRODUCTS];
+    int wave_tot[SM_T / 64];
+};
+
+// f(column, a, b, place of a in the row + 1, place of b) for every product of the row [as, ae) of A
+template <bool VALUES, typename F>
+__device__ __forceinline__ void small_row_products(int64_t as, int64_t ae, const int32_t *__restrict__ Acrd,
+                                                   const double *__restrict__ Aval, const int64_t *__restrict__ Bpos,
+                                                   const int32_t *__restrict__ Bcrd, const double *__restrict__ Bval, F f)
+{
+    const int group = threadIdx.x >> 4, sub = threadIdx.x & 15;
+    for (int64_t p = as + group; p < ae; p += SM_T / 16) {
+        const int k = Acrd[p];
+        const double a = VALUES ? Aval[p] : 0.0;
+        const int64_t be = Bpos[k + 1];
+        for (int64_t q = Bpos[k] + sub; q < be; q += 16)
+            f(Bcrd[q], a, VALUES ? Bval[q] : 0.0, (int)(p - as) + 1, q);
+    }
+}
+// before[w] = set bits in front of word w, for a thread's share of the words; returns how many there are
+__device__ __forceinline__ int small_row_ranks(const uint32_t *bm, uint16_t *before, int words, int *wave_tot)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int per = (words + SM_T - 1) / SM_T, w0 = threadIdx.x * per;
+    int mine = 0;
+    for (int w = w0; w < w0 + per && w < words; ++w)
+        mine += __popc(bm[w]);
+    const int inc = wave_inclusive_scan(mine);
+    if (lane == 63)
+        wave_tot[wave] = inc;
+    lds_barrier();
+    int run = inc - mine, all = 0;
+    for (int x = 0; x < SM_T / 64; ++x) {
+        run += x < wave ? wave_tot[x] : 0;
+        all += wave_tot[x];
+    }
+    if (before)
+        for (int w = w0; w < w0 + per && w < words; ++w) {
+            before[w] = (uint16_t)run;
+            run += __popc(bm[w]);
+        }
+    return all;
+}
+
+__global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
+    int64_t row_begin, RowList list, int words, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
+    const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd, int64_t *__restrict__ rowcount)
+{
+    uint32_t *bm = sg_dyn_lds;
+    __shared__ int wave_tot[SM_T / 64];
+    for (int w = threadIdx.x; w < words; w += SM_T)
+        bm[w] = 0;
+    lds_barrier();
+    int64_t t_first, t_end;
+    list_range(list, 1, &t_first, &t_end);
+    for (int64_t t = t_first + blockIdx.x; t < t_end; t += gridDim.x) {
+        const int64_t r = list.rows[t], i = row_begin + r;
+        small_row_products<false>(Apos[i], Apos[i + 1], Acrd, nullptr, Bpos, Bcrd, nullptr,
+                                  [&](int j, double, double, int, int64_t) { atomicOr(&bm[j >> 5], 1u << (j & 31)); });
+        lds_barrier();
+        const int n = small_row_ranks(bm, nullptr, words, wave_tot);
+        if (threadIdx.x == 0)
+            rowcount[r] = n;
+        const int per = (words + SM_T - 1) / SM_T;
+        for (int w = threadIdx.x * per; w < (int)(threadIdx.x + 1) * per && w < words; ++w)          // its own words
+            bm[w] = 0;
+        lds_barrier();
+    }
+}
+
+template <bool SEMI>
+__global__ __launch_bounds__(SM_T) void spgemm_numeric_small_kernel(
+    int64_t row_begin, RowList list, int words, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
+    const double *__restrict__ Aval, const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd,
+    const double *__restrict__ Bval, const int64_t *__restrict__ Cpos, int32_t *__restrict__ Ccrd,
+    double *__restrict__ Cval, int reduce_op, int mult_op)
+{
+    uint32_t *bm = sg_dyn_lds;
+    uint16_t *before = reinterpret_cast<uint16_t *>(bm + words);
+    SmallRowLds &sh = *reinterpret_cast<SmallRowLds *>(bm + words + words / 2);
+    for (int w = threadIdx.x; w < words + words / 2 + (int)(sizeof sh / 4); w += SM_T)
+        bm[w] = 0;
+    lds_barrier();
+    int64_t t_first, t_end;
+    list_range(list, 1, &t_first, &t_end);
+    const int64_t c0 = Cpos[row_begin];
+    for (int64_t t = t_first + blockIdx.x; t < t_end; t += gridDim.x) {
+        const int64_t i = row_begin + list.rows[t], as = Apos[i], ae = Apos[i + 1], coff = Cpos[i] - c0;
+        small_row_products<false>(as, ae, Acrd, nullptr, Bpos, Bcrd, nullptr,
+                                  [&](int j, double, double, int, int64_t) { atomicOr(&bm[j >> 5], 1u << (j & 31)); });
+        lds_barrier();
+        const int total = small_row_ranks(bm, before, words, sh.wave_tot);
+        lds_barrier();
+        small_row_products<true>(as, ae, Acrd, Aval, Bpos, Bcrd, Bval, [&](int j, double a, double b, int pa, int64_t q) {
+            const int r = before[j >> 5] + __popc(bm[j >> 5] & ((1u << (j & 31)) - 1u));
+            sh.col[r] = (uint16_t)j;
+            if constexpr (SEMI)
+                semiring_lds_add(&sh.val[r], reduce_op, mult_op, a, b, pa, q);
+            else
+                __hip_atomic_fetch_add(&sh.val[r], a * b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        });
+        lds_barrier();
+        for (int q = threadIdx.x; q < total; q += SM_T) {
+            const int j = sh.col[q];
+            Ccrd[coff + q] = j;
+            Cval[coff + q] = dense_take<SEMI>(sh.val, q, reduce_op, mult_op, as, Aval, Bval);
+            bm[j >> 5] = 0;
+        }
+        lds_barrier();
+    }
+}
+
 struct SgScratch {
     Workspace ticket;     // SG_TICKETS 64-bit row counters
     Workspace rowcount;   // int64[nrows] / double[nrows]
@@ -2603,6 +2726,42 @@ static int dot_form_fits(const Csr *a, const Csr *b, const Csr *m, bool *fits);
 static int pair_dot_values(Csr *a, Csr *b, Csr *m, int64_t rb, int64_t re, double **pair_val, uint8_t **pair_hit,
                            int64_t *pairs, int reduce_op, int mult_op);
 
+constexpr int SG_DENSE_MAX_BLOCKS = 64;        // the dense path serves matrices of up to 2^20 columns
+// Rows with at least this many products per column block of the matrix keep their values in LDS (the span or
+// the block kernel); the others add into a slab in HBM through L2 atomics.  Measured as above, ms per product
+// with the span kernel in place: 128 per block 555, 64: 533, 32: 519, 16: 514, 8: 513.5, 4: 513, 1: 515.
+constexpr int64_t SG_DENSE_PER_BLOCK = 8;
+
+// Heavy rows with at least this many products per column block of the matrix stay with the block kernel, the
+// others go to the span kernel (measured on A*A of an R-MAT graph of scale 20, 64 blocks, ms per product:
+// 512 per block 583, 1024 572, 2048 559, 4096 557, 8192 570, every heavy row to the span kernel 604, none 613;
+// with the kernels as they are now 1024 per block 437, 2048 402, 4096 386, 6144 381, 8192 382, 12288 382, 16384 389).
+// COMET_HIP_SPGEMM_WIDE, a number of products per row, overrides the rule: either kernel is right for any row,
+// so the tests use it to send the same rows through both.
+constexpr int64_t SG_WIDE_PER_BLOCK = 6144;
+static int64_t sg_wide_threshold(int nblk)
+{
+    const char *e = getenv("COMET_HIP_SPGEMM_WIDE");
+    return e && *e ? atoll(e) : SG_WIDE_PER_BLOCK * nblk;
+}
+
+// From how many products on a row's values are kept in LDS by the large workgroups, and from how many on block by block.
+struct SgClasses { int64_t dense, wide; };
+static SgClasses sg_row_classes(int64_t ncols, bool small)
+{
+    const int nblk = (int)ceil_div(ncols > 0 ? ncols : 1, SG_CB);
+    SgClasses c;
+    c.dense = small ? SM_PRODUCTS + 1 : SG_DENSE_PER_BLOCK * nblk;
+    c.wide = std::max(sg_wide_threshold(nblk), c.dense);
+    return c;
+}
+static int sm_words(int64_t ncols) { return (int)ceil_div(ceil_div(ncols > 0 ? ncols : 1, 32), 4) * 4; }
+static dim3 sm_grid(const RowList &list)
+{
+    const int64_t most = (int64_t)num_cus() * 7;          // workgroups that fit the CUs
+    return dim3((unsigned)(list.counts[0] < 0 ? most : std::min(most, list.counts[1] - list.counts[0])));
+}
+
 static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *rowcount)
 {
     bool dots = false;
@@ -2623,8 +2782,23 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
     COMET_CHK(sg_geometry(b->ncols, &g));
     COMET_CHK(sg_reset_ticket());
     RowList list;
-    COMET_CHK(sg_row_list(a, b, 0, a->nrows, SG_NO_DENSE, SG_NO_DENSE, &list));
+    const bool small = !m && b->ncols <= SM_COLS;
+    const SgClasses classes = sg_row_classes(b->ncols, small);
+    if (small)          // the list the numeric phase takes
+        COMET_CHK(sg_row_list(a, b, 0, a->nrows, classes.dense, classes.wide, &list, nullptr, 0, true));
+    else
+        COMET_CHK(sg_row_list(a, b, 0, a->nrows, SG_NO_DENSE, SG_NO_DENSE, &list));
     COMET_HIPCHK(hipMemsetAsync(rowcount, 0, sizeof(int64_t) * (size_t)a->nrows, stream()));
+    if (small && list.counts[1] != list.counts[0]) {
+        const int words = sm_words(b->ncols);
+        KernelTimer t("spgemm_symbolic_small");
+        spgemm_symbolic_small_kernel<<<sm_grid(list), dim3(SM_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
+            0, list, words, a->pos, a->crd, b->pos, b->crd, rowcount);
+    }
+    if (small && list.counts[0] == 0) {
+        COMET_HIPCHK(hipGetLastError());
+        return COMET_HIP_OK;
+    }
     uint32_t *gbm = nullptr;
     if (!g.lds) {
         COMET_CHK(g_sg.gbm.ensure(sizeof(uint32_t) * g.bm_words * (size_t)g.groups, true));
@@ -2637,7 +2811,7 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
         KernelTimer t(M ? "spgemm_symbolic_masked" : "spgemm_symbolic");                                   \
         spgemm_symbolic_kernel<L, M><<<grid, block, g.lds_bytes, stream()>>>(                              \
             a->nrows, a->pos, a->crd, b->pos, b->crd, m ? m->pos : nullptr, m ? m->crd : nullptr, g.logW,  \
-            gbm, (unsigned long long *)g_sg.ticket.ptr, list, rowcount);                                   \
+            gbm, (unsigned long long *)g_sg.ticket.ptr, list, small ? 0 : 2, rowcount);                    \
     } while (0)
     if (g.lds) {
         if (m) LAUNCH_SYM(true, true); else LAUNCH_SYM(true, false);
@@ -2647,25 +2821,6 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
 #undef LAUNCH_SYM
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
-}
-
-constexpr int SG_DENSE_MAX_BLOCKS = 64;        // the dense path serves matrices of up to 2^20 columns
-// Rows with at least this many products per column block of the matrix keep their values in LDS (the span or
-// the block kernel); the others add into a slab in HBM through L2 atomics.  Measured as above, ms per product
-// with the span kernel in place: 128 per block 555, 64: 533, 32: 519, 16: 514, 8: 513.5, 4: 513, 1: 515.
-constexpr int64_t SG_DENSE_PER_BLOCK = 8;
-
-// Heavy rows with at least this many products per column block of the matrix stay with the block kernel, the
-// others go to the span kernel (measured on A*A of an R-MAT graph of scale 20, 64 blocks, ms per product:
-// 512 per block 583, 1024 572, 2048 559, 4096 557, 8192 570, every heavy row to the span kernel 604, none 613;
-// with the kernels as they are now 1024 per block 437, 2048 402, 4096 386, 6144 381, 8192 382, 12288 382, 16384 389).
-// COMET_HIP_SPGEMM_WIDE, a number of products per row, overrides the rule: either kernel is right for any row,
-// so the tests use it to send the same rows through both.
-constexpr int64_t SG_WIDE_PER_BLOCK = 6144;
-static int64_t sg_wide_threshold(int nblk)
-{
-    const char *e = getenv("COMET_HIP_SPGEMM_WIDE");
-    return e && *e ? atoll(e) : SG_WIDE_PER_BLOCK * nblk;
 }
 
 // Per-row block pointers of the right-hand operand, built once per matrix.
@@ -2837,25 +2992,28 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     const bool dense = !m && lds_rows;
     // masked: the rows whose mask row does not fit the slab kernel's hash table take the one-block kernel
     const bool mdense = m && lds_rows && g.lds && getenv("COMET_HIP_SPGEMM_NO_MASKED_DENSE") == nullptr;
-    const int64_t dense_threshold = dense ? SG_DENSE_PER_BLOCK * nblk : SG_NO_DENSE;
+    const bool small = dense && b->ncols <= SM_COLS;
+    const SgClasses classes = sg_row_classes(b->ncols, small);
     if (dense || mdense)
         COMET_CHK(sg_plan_blocks(b));
     RowList list;
-    const int64_t wide = sg_wide_threshold(nblk) > dense_threshold ? sg_wide_threshold(nblk) : dense_threshold;
     if (mdense)         // those rows sort in front (sg_row_keys): bounds[0] = bounds[2] = their number
         COMET_CHK(sg_row_list(a, b, rb, re, 1ll << 61, 1ll << 61, &list, m, SG_HASH_FILL));
     else
-        COMET_CHK(sg_row_list(a, b, rb, re, dense_threshold, dense ? wide : SG_NO_DENSE, &list, nullptr, 0, dense));
+        COMET_CHK(sg_row_list(a, b, rb, re, dense ? classes.dense : SG_NO_DENSE, dense ? classes.wide : SG_NO_DENSE, &list, nullptr,
+                              0, dense));
     uint32_t *gbm = nullptr, *gmask = nullptr;
-    if (!g.lds || m) {          // the output row's bitmap is in HBM when LDS holds the mask row instead
-        COMET_CHK(g_sg.gbm.ensure(sizeof(uint32_t) * g.bm_words * (size_t)g.groups, true));
-        gbm = (uint32_t *)g_sg.gbm.ptr;
+    if (!small) {
+        if (!g.lds || m) {          // the output row's bitmap is in HBM when LDS holds the mask row instead
+            COMET_CHK(g_sg.gbm.ensure(sizeof(uint32_t) * g.bm_words * (size_t)g.groups, true));
+            gbm = (uint32_t *)g_sg.gbm.ptr;
+        }
+        if (m && !g.lds) {
+            COMET_CHK(g_sg.gmask.ensure(sizeof(uint32_t) * g.bm_words * (size_t)g.groups, true));
+            gmask = (uint32_t *)g_sg.gmask.ptr;
+        }
+        COMET_CHK(g_sg.slabs.ensure(sizeof(double) * (size_t)(b->ncols > 0 ? b->ncols : 1) * (size_t)g.groups, true));
     }
-    if (m && !g.lds) {
-        COMET_CHK(g_sg.gmask.ensure(sizeof(uint32_t) * g.bm_words * (size_t)g.groups, true));
-        gmask = (uint32_t *)g_sg.gmask.ptr;
-    }
-    COMET_CHK(g_sg.slabs.ensure(sizeof(double) * (size_t)(b->ncols > 0 ? b->ncols : 1) * (size_t)g.groups, true));
     const dim3 grid((unsigned)g.groups), block(SG_T);
     // a masked product keeps either the mask row's bitmap or its hash table in LDS, whichever the row needs
     const size_t num_lds = m && g.lds && g.lds_bytes < SG_HASH_LDS ? SG_HASH_LDS : g.lds_bytes;
@@ -2872,9 +3030,16 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     do {                                                                                                   \
         if (semi) LAUNCH_NUM(L, M, true); else LAUNCH_NUM(L, M, false);                                    \
     } while (0)
-    if (list.counts[1] >= 0 && list.counts[1] == list.counts[0])
-        ;          // every row with products is a heavy one
-    else if (g.lds) {
+    if (list.counts[1] >= 0 && list.counts[1] == list.counts[0]) {
+        // every row with products is a heavy one
+    } else if (small) {
+        const int words = sm_words(b->ncols);
+        const size_t lds = sizeof(uint32_t) * (size_t)(words + words / 2) + sizeof(SmallRowLds);
+        KernelTimer t(semi ? "spgemm_numeric_semiring" : "spgemm_numeric");
+        const auto kernel = semi ? spgemm_numeric_small_kernel<true> : spgemm_numeric_small_kernel<false>;
+        kernel<<<sm_grid(list), dim3(SM_T), lds, stream()>>>(rb, list, words, a->pos, a->crd, a->val, b->pos, b->crd, b->val, Cpos,
+                                                             Ccrd, Cval, reduce_op, mult_op);
+    } else if (g.lds) {
         if (m) LAUNCH_NUM_S(true, true); else LAUNCH_NUM_S(true, false);
     } else {
         if (m) LAUNCH_NUM_S(false, true); else LAUNCH_NUM_S(false, false);

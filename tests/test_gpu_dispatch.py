@@ -233,3 +233,25 @@ def test_sddmm_in_an_order_that_keeps_columns_close(K, hub):
         out = rt.DeviceArray(len(crd), zero=True)
         rt.sddmm(S, dC, dD, out_values=out)
         assert np.array_equal(out.to_numpy(), want)
+
+
+@pytest.mark.parametrize("semiring", [None, ("min", "plus"), ("max", "times"), ("any", "second")])
+@pytest.mark.parametrize("ncols", [1, 31, 33, 1000, 65_535, 65_536, 65_537])
+def test_spgemm_rows_with_few_products(ncols, semiring):
+    # rows around the number of products, and matrices around the number of columns, that the small workgroups take
+    rng = np.random.default_rng(ncols)
+    csr = lambda rows: (np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int64),
+                        np.concatenate(rows).astype(np.int32), rng.uniform(0.5, 1.5, sum(map(len, rows))))
+    k, most = 1100, min(ncols, 1000)          # rows of B: two of 1000 entries (if there is room), a hundred of one, others
+    b = csr([np.sort(rng.choice(ncols, min(l, ncols), replace=False)) for l in [most] * 2 + [1] * 100 + [7, 15, 16, 17, 64, 513] * 166 + [3] * 2])
+    picks = [[], [0], [5], range(102, 110), range(102, 168)] + [[0, 1, *range(2, 2 + n)] for n in (0, 7, 47, 48, 49, 100)]
+    a = csr([np.array(p, np.int64) for p in picks * 5])
+    A, B = rt.CsrMatrix.from_arrays((5 * len(picks), k), *a), rt.CsrMatrix.from_arrays((k, ncols), *b)
+    want = orc.spgemm(*a, *b, ncols, semiring=semiring)
+    for _ in range(2):
+        p, c, v = rt.spgemm(A, B, semiring=semiring).to_arrays()
+        assert np.array_equal(p, want[0]) and np.array_equal(c, want[1])
+        if semiring is None:
+            assert np.all(np.abs(v - want[2]) <= 1e-12 * want[2])
+        else:
+            assert np.array_equal(v, want[2])
