@@ -381,7 +381,9 @@ struct RowList {
     const int32_t *rows;       // row - row_begin, by descending number of products
     const int64_t *bounds;     // [0] rows with >= dense_threshold products, [1] rows with any product,
                                // [2] rows with >= wide_threshold products (a prefix of [0])
-    int64_t counts[3];         // the same on the host where it asked for them, else -1
+    int64_t counts[3];         // the same on the host where it has them, else -1
+    // whether the host knows that every row with products is a heavy one (unknown counts are all -1, hence equal)
+    bool only_heavy() const { return counts[1] >= 0 && counts[1] == counts[0]; }
 };
 __device__ inline void list_range(const RowList &l, int part, int64_t *first, int64_t *end)
 {
@@ -2647,7 +2649,7 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
     for (int64_t &c : out->counts)
         c = -1;
     const int64_t n = re - rb;
-    static const bool keep = getenv("COMET_HIP_SPGEMM_NO_LIST_CACHE") == nullptr;
+    const bool keep = getenv("COMET_HIP_SPGEMM_NO_LIST_CACHE") == nullptr;
     Csr *owner = const_cast<Csr *>(a);
     RowListEntry key;
     key.b_uid = b->uid;
@@ -2789,7 +2791,7 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
     else
         COMET_CHK(sg_row_list(a, b, 0, a->nrows, SG_NO_DENSE, SG_NO_DENSE, &list));
     COMET_HIPCHK(hipMemsetAsync(rowcount, 0, sizeof(int64_t) * (size_t)a->nrows, stream()));
-    if (small && list.counts[1] != list.counts[0]) {
+    if (small && !list.only_heavy()) {
         const int words = sm_words(b->ncols);
         KernelTimer t("spgemm_symbolic_small");
         spgemm_symbolic_small_kernel<<<sm_grid(list), dim3(SM_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
@@ -3030,8 +3032,8 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     do {                                                                                                   \
         if (semi) LAUNCH_NUM(L, M, true); else LAUNCH_NUM(L, M, false);                                    \
     } while (0)
-    if (list.counts[1] >= 0 && list.counts[1] == list.counts[0]) {
-        // every row with products is a heavy one
+    if (list.only_heavy()) {
+        // nothing for these kernels
     } else if (small) {
         const int words = sm_words(b->ncols);
         const size_t lds = sizeof(uint32_t) * (size_t)(words + words / 2) + sizeof(SmallRowLds);

@@ -237,8 +237,12 @@ def test_sddmm_in_an_order_that_keeps_columns_close(K, hub):
 
 @pytest.mark.parametrize("semiring", [None, ("min", "plus"), ("max", "times"), ("any", "second")])
 @pytest.mark.parametrize("ncols", [1, 31, 33, 1000, 65_535, 65_536, 65_537])
-def test_spgemm_rows_with_few_products(ncols, semiring):
-    # rows around the number of products, and matrices around the number of columns, that the small workgroups take
+@pytest.mark.parametrize("kept", [True, False])
+def test_spgemm_rows_with_few_products(ncols, semiring, kept, monkeypatch):
+    # rows around the number of products, and matrices around the number of columns, that the small workgroups take; the
+    # host knows how many rows are small only where the list of rows is kept
+    if not kept:
+        monkeypatch.setenv("COMET_HIP_SPGEMM_NO_LIST_CACHE", "1")
     rng = np.random.default_rng(ncols)
     csr = lambda rows: (np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int64),
                         np.concatenate(rows).astype(np.int32), rng.uniform(0.5, 1.5, sum(map(len, rows))))
