@@ -37,7 +37,7 @@ EXTENTS = [dict(a=5, b=7, c=3, d=11, e=16, f=2), dict(a=1, b=1, c=129, d=1, e=17
 
 @pytest.mark.parametrize("forced", [None, "0,1", "1,1", "2,1", "3,1", "0,3", "1,2", "2,5", "3,4"])
 @pytest.mark.parametrize("a,b,c", [("ef", "fc", "ec"), ("aebf", "dfce", "abcd"), ("aebf", "efcd", "abcd"), ("eabf", "cdfe", "cdab"),
-                                   ("feab", "efcd", "dcba"), ("abef", "ef", "ab"), ("ab", "cd", "acbd")])
+                                   ("feab", "efcd", "dcba"), ("abef", "ef", "ab"), ("ab", "cd", "acbd"), ("ef", "f", "e"), ("f", "fa", "a")])
 def test_contraction_every_tile_shape_and_layout(a, b, c, forced, monkeypatch):
     for i, extent in enumerate(EXTENTS):
         rng = np.random.default_rng(i)
