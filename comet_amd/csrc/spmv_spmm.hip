@@ -374,7 +374,7 @@ static int spmv_plan(Csr *a)
 // `carry` (two 64-wide slots per chunk: [0] a piece whose row began in an
 // earlier chunk, [1] a piece whose row goes on into the next), from where the
 // wavefront that leaves the last piece of a row (`arrived` counts them, by the
-// chunk the row begins in; zero between calls) adds them in chunk order.
+// chunk the row begins in, from zero) adds them in chunk order.
 // Bound by the gathers' way from the memory-side cache where B is larger than
 // an L2.  A lane per column and one nonzero at a time (K of 64 lanes busy, 8
 // bytes each) took 84 us for 60001 rows of 16 nonzeros and K = 33, this 69; 81 and 47 for
@@ -388,13 +388,15 @@ constexpr int SPMM_GRAIN = 64;                // the row of every so many'th non
 constexpr int SPMM_U = COMET_SPMM_U;          // B-row loads in flight per lane
 constexpr int SPMM_WAVES = 4;                 // wavefronts per workgroup
 
-// chunk_row[c] = the row r with pos[r] <= c*grain < pos[r+1]
+// chunk_row[c] = the row r with pos[r] <= c*grain < pos[r+1]; arrived[0 .. counts) = 0 (counts 0: not asked for)
 __global__ void spmm_chunk_rows(const int64_t *__restrict__ pos, int64_t nrows, int64_t nchunks, int grain,
-                                int32_t *__restrict__ chunk_row)
+                                int32_t *__restrict__ chunk_row, unsigned *__restrict__ arrived, int64_t counts)
 {
     int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nchunks)
         return;
+    for (int64_t i = c; i < counts; i += nchunks)
+        arrived[i] = 0;
     const int64_t target = c * grain;
     int64_t lo = 0, hi = nrows;   // first index in pos[0..nrows] with pos > target lies in [1, nrows]
     while (lo < hi) {
@@ -638,7 +640,7 @@ __global__ __launch_bounds__(SPMM_WAVES * 64) void spmm_csr_nnzsplit(
         if ((int64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)before) != c1 - c0)
             return;
         if (lane == 0)
-            __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);          // for the next call
+            __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);          // for the next call on the workspace
         double *to = C + crow(r) * ldc + tile + lane;
         double sum = __hip_atomic_load(slots + c0 * 128 + 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (ACC)
@@ -1032,7 +1034,7 @@ static int spmm_plan(Csr *a)
     if (nchunks > 0) {
         KernelTimer t("spmm_chunk_rows");
         spmm_chunk_rows<<<dim3((unsigned)ceil_div(nchunks, 256)), dim3(256), 0, stream()>>>(
-            a->pos, a->nrows, nchunks, SPMM_GRAIN, a->spmm_chunk_row);
+            a->pos, a->nrows, nchunks, SPMM_GRAIN, a->spmm_chunk_row, nullptr, 0);
     }
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
@@ -1882,6 +1884,16 @@ int spmm_static_setup(int device)
 }
 }  // namespace comet
 
+extern "C" int64_t comet_hip_debug_noalloc_scratch(int64_t *bytes)
+{
+    int device = -1;
+    if (bytes)
+        *bytes = (int64_t)sizeof spmm_static_scratch;
+    if (!is_initialised() || hipGetDevice(&device) != hipSuccess || device < 0 || device >= SPMM_STATIC_MAX_DEVICES)
+        return 0;
+    return reinterpret_cast<int64_t>(g_spmm_static_ptr[device]);
+}
+
 extern "C" int comet_hip_spmm_csr_f64_noalloc(int64_t csr, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dptr,
                                               int64_t ldc, int accumulate, int64_t on_stream)
 {
@@ -1921,16 +1933,17 @@ extern "C" int comet_hip_spmm_csr_f64_noalloc(int64_t csr, int64_t K, int64_t b_
         }
         return COMET_HIP_OK;
     }
-    // Every word the kernels read from the array is written earlier in the same call (the table in full, a carry
-    // slot by the chunk that leaves a piece of a row in it), or is a count that the one to reach it puts back to zero:
-    // nothing has to be cleared between calls.
+    // Every word the kernels read from the array is written earlier in the same call: the table in full and a zero in
+    // every count by the first kernel, a carry slot by the chunk that leaves a piece of a row in it.  So what the array
+    // holds when a call begins - calls that overlapped may leave anything - does not matter.
     int32_t *chunk_row = reinterpret_cast<int32_t *>(scratch);
     double *carry = reinterpret_cast<double *>(scratch + SPMM_STATIC_TABLE_BYTES);
     const int len = spmm_chunk_len(a->nnz, tiles);
     const int64_t rows = ceil_div(a->nnz, len);
-    spmm_chunk_rows<<<dim3((unsigned)ceil_div(rows, 256)), dim3(256), 0, on>>>(a->pos, a->nrows, rows, len, chunk_row);
-    spmm_chunk_launch(a, K, (const double *)b_dptr, ldb, C, ldc, accumulate, chunk_row, len, len, carry,
-                      reinterpret_cast<unsigned *>(scratch + SPMM_STATIC_TABLE_BYTES + SPMM_STATIC_CARRY_BYTES), on, false);
+    unsigned *arrived = reinterpret_cast<unsigned *>(scratch + SPMM_STATIC_TABLE_BYTES + SPMM_STATIC_CARRY_BYTES);
+    spmm_chunk_rows<<<dim3((unsigned)ceil_div(rows, 256)), dim3(256), 0, on>>>(a->pos, a->nrows, rows, len, chunk_row, arrived,
+                                                                               tiles * rows);
+    spmm_chunk_launch(a, K, (const double *)b_dptr, ldb, C, ldc, accumulate, chunk_row, len, len, carry, arrived, on, false);
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
 }

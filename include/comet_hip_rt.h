@@ -131,8 +131,9 @@ int comet_hip_spmm_csr_f64(int64_t csr, int64_t K, int64_t b_dptr, int64_t ldb,
 /* The same product for callers that cannot allocate device memory (code under
  * HIP graph capture, serving loops and harnesses that forbid hipMalloc).  It has
  * no counterpart in the reference.  Nothing is allocated or freed: the scratch
- * of its kernels (chunk table and carry slots) is an 8 MiB array in the
- * library's image, one copy per device.  Limits: comet_hip_init must have run;
+ * of its kernels (chunk table, carry slots and counts) is an array of 8 MiB + 64 KiB in the
+ * library's image, one copy per device, and a call does not depend on what it
+ * holds when the call begins.  Limits: comet_hip_init must have run;
  * ceil(K/64) * ceil(nnz/256) <= 8192 (nnz <= 2,097,152 at K <= 64), larger
  * products return COMET_HIP_ERR_SIZE.  Rows are summed exactly as
  * comet_hip_spmm_csr_f64 sums them for a matrix below its long-row threshold.
@@ -445,6 +446,10 @@ int comet_hip_mfma_f64_peak(int64_t iters, double *tflops);
  * kernel begin in its LDS for a bitmap of `words` 32-bit words; always even (an
  * odd offset would misalign its 64-bit LDS atomics).  Runs on the host. */
 int comet_hip_debug_dot_table_words(int words);
+/* Diagnostic: the device address of the array that comet_hip_spmm_csr_f64_noalloc
+ * keeps its scratch in on the current device, and its size (0 before
+ * comet_hip_init): a call must not depend on what the array holds when it begins. */
+int64_t comet_hip_debug_noalloc_scratch(int64_t *bytes);
 /* Diagnostic: vector registers per lane of the two kernels of the pattern-matrix
  * masked sum (comet_hip_spgemm_masked_sum) in the loaded code object.  They share
  * the CUs, and do so only while four wavefronts of the first and one of the second

@@ -71,6 +71,23 @@ def test_noalloc_spmm_matches_ordinary_entry_point_twice_in_a_row():
     assert np.array_equal(ref3, got3) and np.array_equal(got3, got1)
 
 
+@pytest.mark.parametrize("K", [40, 130])
+@pytest.mark.parametrize("byte", [0x01, 0xff])
+def test_noalloc_spmm_does_not_depend_on_what_the_scratch_holds(byte, K):
+    # as calls that overlapped may leave it
+    import ctypes
+    n = ctypes.c_int64(0)
+    scratch = rt.lib().comet_hip_debug_noalloc_scratch(ctypes.byref(n))
+    assert scratch and n.value > 8 << 20
+    junk = np.full(n.value, byte, np.uint8)
+    for _ in range(2):
+        rt._check(rt.lib().comet_hip_memcpy(scratch, rt._vptr(junk), n.value, 0))
+        (ref, got), _ = _product(7_000, 12.0, K, seed=31, accumulate=True)
+        assert np.array_equal(ref, got)
+    (ref, got), _ = _product(7_000, 12.0, K, seed=31, accumulate=False)          # nor on what that call left
+    assert np.array_equal(ref, got)
+
+
 def test_noalloc_spmm_runs_on_the_callers_stream():
     # a stream of the caller's own: the kernels go there (and the result is there once that stream is through)
     s = rt.lib().comet_hip_stream_create()
