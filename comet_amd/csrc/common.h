@@ -69,6 +69,7 @@ struct Piece {
 };
 int transfer_up(const std::vector<Piece> &pieces);
 int transfer_down(const std::vector<Piece> &pieces);
+void transfer_release();          // comet_hip_finalize: what is kept for transfers belongs to the device
 Piece plain_up(void *dev, const void *host, size_t bytes);
 Piece plain_down(void *host, const void *dev, size_t bytes);
 

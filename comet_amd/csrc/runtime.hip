@@ -940,6 +940,7 @@ int comet_hip_finalize(void)
     for (Workspace *w : g_workspaces)
         w->release();
     dev_pool_release();
+    transfer_release();
     (void)hipStreamSynchronize(g_aux);
     (void)hipEventDestroy(g_fork);
     (void)hipEventDestroy(g_join);

@@ -53,13 +53,14 @@ __global__ __launch_bounds__(256) void move_segments(Segments p, char *pinned)
     }
 }
 
-// The threads, parked between transfers, and the pinned slots.  Made at the first transfer and kept for the life of
-// the process.
+// The threads, parked between transfers, and the pinned slots.  Made at the first transfer; the threads are kept for
+// the life of the process and take the device of each transfer, the slots and their events go with the device when
+// the library is closed.
 struct Crew {
     std::mutex mu;
     std::condition_variable start, done;
     uint64_t generation = 0;
-    int running = 0;
+    int running = 0, device = 0;
     const std::function<void()> *job = nullptr;
     char *pinned = nullptr;
     hipEvent_t moved[SLOTS];          // the last group in the slot is across
@@ -69,22 +70,39 @@ struct Crew {
     {
         if (pinned)
             return COMET_HIP_OK;
+        char *room = nullptr;
+        COMET_HIPCHK(hipHostMalloc((void **)&room, SLOTS * SLOT, hipHostMallocDefault));
         for (hipEvent_t &e : moved)
             COMET_HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        COMET_HIPCHK(hipHostMalloc((void **)&pinned, SLOTS * SLOT, hipHostMallocDefault));
+        pinned = room;
         return COMET_HIP_OK;
     }
-    void loop(int device)
+    void release()
     {
-        (void)hipSetDevice(device);
+        if (!pinned)
+            return;
+        for (hipEvent_t e : moved)
+            (void)hipEventDestroy(e);
+        (void)hipHostFree(pinned);
+        pinned = nullptr;
+    }
+    void loop()
+    {
         uint64_t seen = 0;
+        int current = -1;
         for (;;) {
             const std::function<void()> *mine;
+            int wanted;
             {
                 std::unique_lock<std::mutex> lk(mu);
                 start.wait(lk, [&] { return generation != seen; });
                 seen = generation;
                 mine = job;
+                wanted = device;
+            }
+            if (wanted != current) {
+                (void)hipSetDevice(wanted);
+                current = wanted;
             }
             (*mine)();
             std::lock_guard<std::mutex> lk(mu);
@@ -96,12 +114,11 @@ struct Crew {
     void run(bool alone, const std::function<void()> &work)
     {
         if (!alone) {
-            int device = 0;
-            (void)hipGetDevice(&device);
             std::lock_guard<std::mutex> lk(mu);
+            (void)hipGetDevice(&device);
             if (!threads) {
                 for (int h = 1; h < WORKERS; ++h)
-                    std::thread([this, device] { loop(device); }).detach();
+                    std::thread([this] { loop(); }).detach();
                 threads = true;
             }
             job = &work;
@@ -241,6 +258,12 @@ int transfer(const std::vector<Piece> &pieces, bool up)
 
 int transfer_up(const std::vector<Piece> &pieces) { return transfer(pieces, true); }
 int transfer_down(const std::vector<Piece> &pieces) { return transfer(pieces, false); }
+
+void transfer_release()
+{
+    std::lock_guard<std::mutex> lk(g_crew_mu);
+    g_crew->release();
+}
 
 Piece plain_up(void *dev, const void *host, size_t bytes)
 {

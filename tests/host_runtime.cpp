@@ -1,0 +1,231 @@
+// A stand-in for the HIP runtime, for checks of what the library does on the host: two devices that exist in name only,
+// memory that is counted, streams and events that know their device, and one kernel, the one that moves a group of a
+// transfer.  Its functions take the place of the real ones because the program that is asked for a symbol first is the
+// executable.  Each scenario of main() prints what went wrong and returns non-zero.
+#include <hip/hip_runtime_api.h>
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+#include <sys/mman.h>
+#include <sys/resource.h>
+
+#include <chrono>
+#include <map>
+#include <mutex>
+#include <string>
+#include <thread>
+#include <vector>
+
+#include "comet_hip_rt.h"
+
+namespace {
+
+using Clock = std::chrono::steady_clock;
+std::mutex mu;
+constexpr int DEVICES = 2;
+size_t total[DEVICES] = {288ull << 30, 288ull << 30}, used[DEVICES];
+struct Block { size_t bytes; int device; };
+std::map<char *, Block> blocks;
+struct Stream { int device; bool live; Clock::time_point idle; };
+struct Event { int device; bool live; Clock::time_point done; };
+std::map<const void *, std::string> &kernels()          // asked for before this file's own statics are made
+{
+    static auto *k = new std::map<const void *, std::string>;
+    return *k;
+}
+thread_local int current = 0;
+thread_local hipError_t last = hipSuccess;
+thread_local struct { dim3 grid, block; size_t lds; hipStream_t stream; } config;
+
+hipError_t fail(hipError_t e, const char *what)
+{
+    fprintf(stderr, "fake hip: %s\n", what);
+    return last = e;
+}
+Stream *stream_of(hipStream_t s) { return reinterpret_cast<Stream *>(s); }
+Event *event_of(hipEvent_t e) { return reinterpret_cast<Event *>(e); }
+bool on_device(const char *p, size_t bytes, int device)
+{
+    std::lock_guard<std::mutex> lk(mu);
+    auto it = blocks.upper_bound(const_cast<char *>(p));
+    if (it == blocks.begin())
+        return false;
+    --it;
+    return it->second.device == device && p + bytes <= it->first + it->second.bytes;
+}
+
+}  // namespace
+
+extern "C" {
+
+void **__hipRegisterFatBinary(const void *) { static void *h; return &h; }
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *, void *, void *, void *, int *)
+{
+    kernels()[host] = name;
+}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s)
+{
+    config = {g, b, lds, s};
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t *s)
+{
+    *g = config.grid;
+    *b = config.block;
+    *lds = config.lds;
+    *s = config.stream;
+    return hipSuccess;
+}
+hipError_t hipGetDeviceCount(int *n) { *n = DEVICES; return hipSuccess; }
+hipError_t hipSetDevice(int d) { current = d; return hipSuccess; }
+hipError_t hipGetDevice(int *d) { *d = current; return hipSuccess; }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *p, int)
+{
+    memset(p, 0, sizeof *p);
+    strcpy(p->gcnArchName, "gfx950");
+    p->multiProcessorCount = 256;
+    return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void **p, const void *) { static char room[16 << 20]; *p = room; return hipSuccess; }
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "fake error"; }
+hipError_t hipGetLastError(void) { const hipError_t e = last; last = hipSuccess; return e; }
+
+hipError_t hipMalloc(void **p, size_t bytes)
+{
+    std::lock_guard<std::mutex> lk(mu);
+    if (used[current] + bytes > total[current])
+        return last = hipErrorOutOfMemory;
+    *p = mmap(nullptr, bytes, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+    if (*p == MAP_FAILED)
+        return fail(hipErrorOutOfMemory, "mmap");
+    used[current] += bytes;
+    blocks[(char *)*p] = Block{bytes, current};
+    return hipSuccess;
+}
+hipError_t hipFree(void *p)
+{
+    std::lock_guard<std::mutex> lk(mu);
+    auto it = blocks.find((char *)p);
+    if (it == blocks.end())
+        return fail(hipErrorInvalidValue, "free of something else");
+    used[it->second.device] -= it->second.bytes;
+    munmap(p, it->second.bytes);
+    blocks.erase(it);
+    return hipSuccess;
+}
+hipError_t hipMemGetInfo(size_t *f, size_t *t)
+{
+    *t = total[current];
+    *f = total[current] - used[current];
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { *p = aligned_alloc(4096, (bytes + 4095) & ~4095ull); return hipSuccess; }
+hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
+
+hipError_t hipStreamCreate(hipStream_t *s) { *s = reinterpret_cast<hipStream_t>(new Stream{current, true, Clock::now()}); return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return hipStreamCreate(s); }
+hipError_t hipStreamDestroy(hipStream_t s) { stream_of(s)->live = false; return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) { std::this_thread::sleep_until(stream_of(s)->idle); return hipSuccess; }
+hipError_t hipStreamQuery(hipStream_t s) { return Clock::now() < stream_of(s)->idle ? hipErrorNotReady : hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
+
+hipError_t hipEventCreate(hipEvent_t *e) { *e = reinterpret_cast<hipEvent_t>(new Event{current, true, Clock::now()}); return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t e) { event_of(e)->live = false; return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
+{
+    if (!event_of(e)->live || !stream_of(s)->live)
+        return fail(hipErrorInvalidHandle, "record of or on what was destroyed");
+    if (event_of(e)->device != stream_of(s)->device)
+        return fail(hipErrorInvalidHandle, "event recorded on a stream of another device");
+    std::lock_guard<std::mutex> lk(mu);
+    event_of(e)->done = stream_of(s)->idle;
+    return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t e)
+{
+    if (!event_of(e)->live)
+        return fail(hipErrorInvalidHandle, "query of an event that was destroyed");
+    std::lock_guard<std::mutex> lk(mu);
+    return Clock::now() < event_of(e)->done ? hipErrorNotReady : hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e) { std::this_thread::sleep_until(event_of(e)->done); return hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t a, hipEvent_t b)
+{
+    if (!event_of(a)->live || !event_of(b)->live)
+        return fail(hipErrorInvalidHandle, "time between events that were destroyed");
+    *ms = 1.0f;
+    return hipSuccess;
+}
+hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t) { memset(p, v, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void *to, const void *from, size_t n, hipMemcpyKind, hipStream_t) { memcpy(to, from, n); return hipSuccess; }
+
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t s)
+{
+    const std::string &name = kernels()[f];
+    if (!stream_of(s)->live || stream_of(s)->device != current)
+        return fail(hipErrorInvalidHandle, "launch on a stream of another device, or one that was destroyed");
+    if (name.find("move_segments") == std::string::npos)
+        return fail(hipErrorInvalidValue, ("no such kernel here: " + name).c_str());
+    struct Segments { char *dev[12]; uint32_t at[12], bytes[12]; int n; };
+    const Segments &p = *static_cast<const Segments *>(args[0]);
+    char *pinned = *static_cast<char **>(args[1]);
+    for (int i = 0; i < p.n; ++i) {
+        if (!on_device(p.dev[i], p.bytes[i], current))
+            return fail(hipErrorInvalidValue, "a copy touches memory that is not the device's");
+        if (name.find("ILb1E") != std::string::npos)
+            memcpy(p.dev[i], pinned + p.at[i], p.bytes[i]);
+        else
+            memcpy(pinned + p.at[i], p.dev[i], p.bytes[i]);
+    }
+    return hipSuccess;
+}
+
+}  // extern "C"
+
+#define REQUIRE(what)                                                                               \
+    do {                                                                                            \
+        if (!(what)) {                                                                              \
+            fprintf(stderr, "line %d: %s (%s)\n", __LINE__, #what, comet_hip_last_error());         \
+            return 1;                                                                               \
+        }                                                                                           \
+    } while (0)
+
+static int there_and_back(size_t bytes, size_t offset)
+{
+    std::vector<unsigned char> out(bytes), in(bytes, 0);
+    for (size_t i = 0; i < bytes; ++i)
+        out[i] = (unsigned char)(i * 2654435761u >> 11);
+    const int64_t d = comet_hip_malloc((int64_t)(bytes + offset));
+    REQUIRE(d != 0);
+    REQUIRE(comet_hip_memcpy(d + (int64_t)offset, out.data(), (int64_t)bytes, 0) == 0);
+    REQUIRE(comet_hip_memcpy(d + (int64_t)offset, in.data(), (int64_t)bytes, 1) == 0);
+    REQUIRE(in == out);
+    REQUIRE(comet_hip_free(d) == 0);
+    return 0;
+}
+
+// the library closed on one device and opened on another
+static int another_device()
+{
+    for (int device : {0, 1, 0}) {
+        REQUIRE(comet_hip_init(device) == 0);
+        for (size_t bytes : {100ul, 700ul << 10, 30ul << 20})
+            REQUIRE(there_and_back(bytes, 0) == 0);
+        REQUIRE(comet_hip_finalize() == 0);
+    }
+    return 0;
+}
+
+int main(int, char **argv)
+{
+    const std::string what = argv[1];
+    if (what == "another_device")
+        return another_device();
+    fprintf(stderr, "no scenario %s\n", argv[1]);
+    return 2;
+}
