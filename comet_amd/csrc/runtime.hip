@@ -113,11 +113,13 @@ static std::vector<std::pair<size_t, void *>> g_pool_pending;        // free, po
 static std::list<void *> g_pool_age;                                 // the free blocks, longest free first
 static size_t g_pool_free_bytes = 0, g_pool_cap = 0;
 
-// Sizes in eighths of a power of two: requests of about the same size find each other's blocks.
+// Sizes in eighths of a power of two: requests of about the same size find each other's blocks.  From half a gigabyte
+// on in steps of POOL_STEP, so that what rounding takes from the device stays small (an eighth of 130 GiB is not).
+constexpr size_t POOL_STEP = 32 << 20;
 static size_t pool_size(size_t bytes)
 {
     size_t step = 512;
-    while (step * 16 <= bytes)
+    while (step * 16 <= bytes && step < POOL_STEP)
         step *= 2;
     return bytes > 0 ? (bytes + step - 1) / step * step : step;
 }
@@ -170,7 +172,7 @@ static void *pool_take(size_t bytes)
 hipError_t dev_malloc(void **out, size_t need)
 {
     std::lock_guard<std::mutex> lk(g_pool_mu);
-    const size_t bytes = pool_size(need);
+    size_t bytes = pool_size(need);
     void *p = pool_take(bytes);
     if (!p) {
         for (const auto &q : g_pool_pending) {
@@ -189,6 +191,11 @@ hipError_t dev_malloc(void **out, size_t need)
         if (e != hipSuccess && g_pool_free_bytes > 0) {
             (void)hipGetLastError();
             pool_trim(0, 0);
+            e = hipMalloc(&p, bytes);
+        }
+        if (e != hipSuccess && need > 0 && need < bytes) {          // what was asked for, without the rounding
+            (void)hipGetLastError();
+            bytes = need;
             e = hipMalloc(&p, bytes);
         }
         if (e != hipSuccess)

@@ -221,11 +221,36 @@ static int another_device()
     return 0;
 }
 
+// what fits the device can be had, whatever is kept or rounded
+static int whole_device()
+{
+    const int64_t GiB = 1ll << 30;
+    REQUIRE(comet_hip_init(0) == 0);
+    for (int round = 0; round < 2; ++round) {
+        const int64_t a = comet_hip_malloc(130 * GiB), b = comet_hip_malloc(130 * GiB), c = comet_hip_malloc(20 * GiB),
+                      d = comet_hip_malloc(7 * GiB);
+        REQUIRE(a && b && c && d);
+        for (int64_t p : {a, b, c, d})
+            REQUIRE(comet_hip_free(p) == 0);
+        const int64_t e = comet_hip_malloc(260 * GiB), f = comet_hip_malloc(27 * GiB + 12345);
+        REQUIRE(e && f);
+        REQUIRE(comet_hip_malloc(GiB) == 0);
+        const int64_t rest = (int64_t)(total[0] - used[0]);          // to the last page
+        const int64_t g = comet_hip_malloc(rest - rest % 4096);
+        REQUIRE(g);
+        for (int64_t p : {e, f, g})
+            REQUIRE(comet_hip_free(p) == 0);
+    }
+    return 0;
+}
+
 int main(int, char **argv)
 {
     const std::string what = argv[1];
     if (what == "another_device")
         return another_device();
+    if (what == "whole_device")
+        return whole_device();
     fprintf(stderr, "no scenario %s\n", argv[1]);
     return 2;
 }
