@@ -998,6 +998,13 @@ int comet_hip_free(int64_t dptr)
     return COMET_HIP_OK;
 }
 
+int comet_hip_release_memory(void)
+{
+    COMET_CHK(ensure_init());
+    dev_pool_release();
+    return COMET_HIP_OK;
+}
+
 int comet_hip_memcpy(int64_t dptr, void *host, int64_t bytes, int64_t direction)
 {
     COMET_CHK(ensure_init());

@@ -131,6 +131,7 @@ SIGNATURES = {
     "comet_hip_stream_sync": (_int, [_i64]),
     "comet_hip_stream_destroy": (_int, [_i64]),
     "comet_hip_stream_bench": (_int, [_int, _i64, _i64, _i64, _int]),
+    "comet_hip_release_memory": (_int, []),
     "comet_hip_mem_info": (_int, [C.POINTER(_i64), C.POINTER(_i64)]),
     "comet_hip_mfma_f64_peak": (_int, [_i64, C.POINTER(C.c_double)]),
     "comet_hip_gather_rows_bench": (_int, [_i64, _i64, _i64, _i64, _i64, _i64]),
@@ -197,6 +198,11 @@ def device_name():
 
 def sync():
     _check(lib().comet_hip_sync(), "comet_hip_sync")
+
+
+def release_memory():
+    """Gives freed device memory that the library keeps back to the device, for other allocators of the process."""
+    _check(lib().comet_hip_release_memory())
 
 
 def _vptr(a):

@@ -51,6 +51,11 @@ int comet_hip_device_name(char *buf, int64_t cap);
  * and HipMemcpy* (:80-124; direction 0 = host to device, 1 = device to host). */
 int64_t comet_hip_malloc(int64_t bytes);            /* 0 on failure */
 int comet_hip_free(int64_t dptr);
+/* Device memory that is freed, by the caller or inside the library, is kept for
+ * the next request of about its size: at most a sixteenth of the device.  It is
+ * given back when an allocation of this library fails, at comet_hip_finalize, and
+ * by this call, for other allocators of the process (waits for the device). */
+int comet_hip_release_memory(void);
 int comet_hip_memcpy(int64_t dptr, void *host, int64_t bytes, int64_t direction);
 int comet_hip_memset(int64_t dptr, int byte_value, int64_t bytes);
 int comet_hip_sync(void);

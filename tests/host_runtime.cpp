@@ -244,6 +244,23 @@ static int whole_device()
     return 0;
 }
 
+// freed memory that is kept can be had back for others, and so can memory of a device that the library has left
+static int given_back()
+{
+    REQUIRE(comet_hip_init(0) == 0);
+    const size_t before = used[0];
+    const int64_t a = comet_hip_malloc(5ll << 30), b = comet_hip_malloc(1000);
+    REQUIRE(a && b);
+    REQUIRE(comet_hip_free(a) == 0);
+    REQUIRE(used[0] >= before + (5ull << 30));
+    REQUIRE(comet_hip_release_memory() == 0);
+    REQUIRE(used[0] >= before + 1000 && used[0] < before + (1ull << 20));
+    REQUIRE(comet_hip_free(b) == 0);
+    REQUIRE(comet_hip_release_memory() == 0);
+    REQUIRE(used[0] == before);
+    return 0;
+}
+
 int main(int, char **argv)
 {
     const std::string what = argv[1];
@@ -251,6 +268,8 @@ int main(int, char **argv)
         return another_device();
     if (what == "whole_device")
         return whole_device();
+    if (what == "given_back")
+        return given_back();
     fprintf(stderr, "no scenario %s\n", argv[1]);
     return 2;
 }
