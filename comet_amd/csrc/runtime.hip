@@ -102,6 +102,7 @@ int ensure_init()
 // ------------------------------------------------------------------ device memory
 struct PoolBlock {
     size_t bytes;
+    int device;
     bool live;
     std::list<void *>::iterator age;         // of a free block: its place in g_pool_age
 };
@@ -200,7 +201,7 @@ hipError_t dev_malloc(void **out, size_t need)
         }
         if (e != hipSuccess)
             return e;
-        g_pool_blocks[p] = PoolBlock{bytes, true, g_pool_age.end()};
+        g_pool_blocks[p] = PoolBlock{bytes, g_device, true, g_pool_age.end()};
     }
     *out = p;
     return hipSuccess;
@@ -216,6 +217,10 @@ hipError_t dev_free(void *p)
         return hipFree(p);
     if (!it->second.live)
         return hipErrorInvalidValue;         // freed twice
+    if (it->second.device != g_device) {     // had before the library was closed and opened on another device
+        g_pool_blocks.erase(it);
+        return hipFree(p);
+    }
     if (g_pool_cap == 0) {
         size_t f = 0, t = 0;
         g_pool_cap = hipMemGetInfo(&f, &t) == hipSuccess && t >= POOL_SHARE ? t / POOL_SHARE : 1;
@@ -232,6 +237,7 @@ void dev_pool_release()
 {
     std::lock_guard<std::mutex> lk(g_pool_mu);
     pool_trim(0, 0);
+    g_pool_cap = 0;          // a share of the device at hand
 }
 
 int stream_wait()
@@ -446,6 +452,19 @@ static void drain_pending()
         g_event_pool.push_back(p.b);
     }
     g_pending.clear();
+}
+
+static void release_events()
+{
+    drain_pending();
+    for (hipEvent_t e : g_event_pool)
+        (void)hipEventDestroy(e);
+    g_event_pool.clear();
+    for (hipEvent_t *e : {&g_t0, &g_t1}) {
+        if (*e)
+            (void)hipEventDestroy(*e);
+        *e = nullptr;
+    }
 }
 
 KernelTimer::KernelTimer(const char *name) : KernelTimer(name, g_stream) {}
@@ -948,6 +967,7 @@ int comet_hip_finalize(void)
         w->release();
     dev_pool_release();
     transfer_release();
+    release_events();
     (void)hipStreamSynchronize(g_aux);
     (void)hipEventDestroy(g_fork);
     (void)hipEventDestroy(g_join);

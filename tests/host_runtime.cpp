@@ -214,6 +214,8 @@ static int another_device()
 {
     for (int device : {0, 1, 0}) {
         REQUIRE(comet_hip_init(device) == 0);
+        double ms = 0.0;
+        REQUIRE(comet_hip_timer_start() == 0 && comet_hip_timer_stop(&ms) == 0 && ms > 0.0);
         for (size_t bytes : {100ul, 700ul << 10, 30ul << 20})
             REQUIRE(there_and_back(bytes, 0) == 0);
         REQUIRE(comet_hip_finalize() == 0);
@@ -261,6 +263,21 @@ static int given_back()
     return 0;
 }
 
+// memory that was had on a device the library has left is given back to that device, not handed out on another
+static int block_of_another_device()
+{
+    REQUIRE(comet_hip_init(0) == 0);
+    const int64_t kept = comet_hip_malloc(3 << 20);
+    REQUIRE(kept);
+    REQUIRE(comet_hip_finalize() == 0);
+    REQUIRE(comet_hip_init(1) == 0);
+    REQUIRE(comet_hip_free(kept) == 0);
+    REQUIRE(there_and_back(3 << 20, 0) == 0);
+    REQUIRE(comet_hip_finalize() == 0);
+    REQUIRE(used[0] == 0 && used[1] == 0);
+    return 0;
+}
+
 int main(int, char **argv)
 {
     const std::string what = argv[1];
@@ -270,6 +287,8 @@ int main(int, char **argv)
         return whole_device();
     if (what == "given_back")
         return given_back();
+    if (what == "block_of_another_device")
+        return block_of_another_device();
     fprintf(stderr, "no scenario %s\n", argv[1]);
     return 2;
 }
