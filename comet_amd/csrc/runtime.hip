@@ -107,12 +107,19 @@ struct PoolBlock {
     std::list<void *>::iterator age;         // of a free block: its place in g_pool_age
 };
 constexpr size_t POOL_BLOCKS = 512;                                  // free blocks kept at most: the lists stay short
+struct PoolPending {
+    size_t bytes;
+    void *p;
+    uint64_t freed;                          // how many blocks had been freed before it
+};
+// Guards what follows, for the time it takes to look: nobody waits for the device with it held.
 static std::mutex g_pool_mu;
 static std::unordered_map<void *, PoolBlock> g_pool_blocks;          // every block that came from hipMalloc here
 static std::multimap<size_t, void *> g_pool_clean;                   // free, and the device was drained since
-static std::vector<std::pair<size_t, void *>> g_pool_pending;        // free, possibly still in use by launched work
+static std::vector<PoolPending> g_pool_pending;                      // free, possibly still in use by launched work
 static std::list<void *> g_pool_age;                                 // the free blocks, longest free first
 static size_t g_pool_free_bytes = 0, g_pool_cap = 0;
+static uint64_t g_pool_freed = 0;
 
 // Sizes in eighths of a power of two: requests of about the same size find each other's blocks.  From half a gigabyte
 // on in steps of POOL_STEP, so that what rounding takes from the device stays small (an eighth of 130 GiB is not).
@@ -125,10 +132,14 @@ static size_t pool_size(size_t bytes)
     return bytes > 0 ? (bytes + step - 1) / step * step : step;
 }
 
-static void pool_promote()
+// the device was drained after `freed` blocks had been freed: these are in use no longer
+static void pool_promote(uint64_t freed)
 {
-    g_pool_clean.insert(g_pool_pending.begin(), g_pool_pending.end());
-    g_pool_pending.clear();
+    const auto first = std::stable_partition(g_pool_pending.begin(), g_pool_pending.end(),
+                                             [&](const PoolPending &q) { return q.freed >= freed; });
+    for (auto it = first; it != g_pool_pending.end(); ++it)
+        g_pool_clean.emplace(it->bytes, it->p);
+    g_pool_pending.erase(first, g_pool_pending.end());
 }
 
 static void pool_leave(PoolBlock &b)         // a block leaves the free ones
@@ -137,23 +148,37 @@ static void pool_leave(PoolBlock &b)         // a block leaves the free ones
     g_pool_free_bytes -= b.bytes;
 }
 
-static void pool_trim(size_t keep_bytes, size_t keep_blocks)         // hipFree itself waits for the device
+// takes the blocks out that are too many; the caller gives them to hipFree, which waits for the device
+static std::vector<void *> pool_trim(size_t keep_bytes, size_t keep_blocks)
 {
+    std::vector<void *> out;
     while (!g_pool_age.empty() && (g_pool_free_bytes > keep_bytes || g_pool_age.size() > keep_blocks)) {
         void *p = g_pool_age.front();
         PoolBlock &b = g_pool_blocks[p];
-        const std::pair<size_t, void *> entry(b.bytes, p);
         auto range = g_pool_clean.equal_range(b.bytes);
         for (auto it = range.first; it != range.second; ++it)
             if (it->second == p) {
                 g_pool_clean.erase(it);
                 break;
             }
-        g_pool_pending.erase(std::remove(g_pool_pending.begin(), g_pool_pending.end(), entry), g_pool_pending.end());
+        g_pool_pending.erase(std::remove_if(g_pool_pending.begin(), g_pool_pending.end(),
+                                            [&](const PoolPending &q) { return q.p == p; }), g_pool_pending.end());
         pool_leave(b);
         g_pool_blocks.erase(p);
-        (void)hipFree(p);
+        out.push_back(p);
     }
+    return out;
+}
+
+static void pool_give_back(std::unique_lock<std::mutex> &lk, size_t keep_bytes, size_t keep_blocks)
+{
+    const std::vector<void *> blocks = pool_trim(keep_bytes, keep_blocks);
+    if (blocks.empty())
+        return;
+    lk.unlock();
+    for (void *p : blocks)
+        (void)hipFree(p);
+    lk.lock();
 }
 
 // a clean block of at least `bytes` that wastes at most a quarter of the request
@@ -172,26 +197,25 @@ static void *pool_take(size_t bytes)
 
 hipError_t dev_malloc(void **out, size_t need)
 {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
+    std::unique_lock<std::mutex> lk(g_pool_mu);
     size_t bytes = pool_size(need);
     void *p = pool_take(bytes);
-    if (!p) {
-        for (const auto &q : g_pool_pending) {
-            if (q.first < bytes || q.first > bytes + bytes / 4)
-                continue;
-            const hipError_t e = hipDeviceSynchronize();
-            if (e != hipSuccess)
-                return e;
-            pool_promote();
-            p = pool_take(bytes);
-            break;
-        }
+    if (!p && std::any_of(g_pool_pending.begin(), g_pool_pending.end(),
+                          [&](const PoolPending &q) { return q.bytes >= bytes && q.bytes <= bytes + bytes / 4; })) {
+        const uint64_t freed = g_pool_freed;
+        lk.unlock();
+        const hipError_t e = hipDeviceSynchronize();
+        lk.lock();
+        if (e != hipSuccess)
+            return e;
+        pool_promote(freed);
+        p = pool_take(bytes);
     }
     if (!p) {
         hipError_t e = hipMalloc(&p, bytes);
         if (e != hipSuccess && g_pool_free_bytes > 0) {
             (void)hipGetLastError();
-            pool_trim(0, 0);
+            pool_give_back(lk, 0, 0);
             e = hipMalloc(&p, bytes);
         }
         if (e != hipSuccess && need > 0 && need < bytes) {          // what was asked for, without the rounding
@@ -211,14 +235,17 @@ hipError_t dev_free(void *p)
 {
     if (!p)
         return hipSuccess;
-    std::lock_guard<std::mutex> lk(g_pool_mu);
+    std::unique_lock<std::mutex> lk(g_pool_mu);
     auto it = g_pool_blocks.find(p);
-    if (it == g_pool_blocks.end())           // not one of ours
+    if (it == g_pool_blocks.end()) {         // not one of ours
+        lk.unlock();
         return hipFree(p);
+    }
     if (!it->second.live)
         return hipErrorInvalidValue;         // freed twice
     if (it->second.device != g_device) {     // had before the library was closed and opened on another device
         g_pool_blocks.erase(it);
+        lk.unlock();
         return hipFree(p);
     }
     if (g_pool_cap == 0) {
@@ -227,28 +254,32 @@ hipError_t dev_free(void *p)
     }
     it->second.live = false;
     it->second.age = g_pool_age.insert(g_pool_age.end(), p);
-    g_pool_pending.emplace_back(it->second.bytes, p);
+    g_pool_pending.push_back(PoolPending{it->second.bytes, p, g_pool_freed++});
     g_pool_free_bytes += it->second.bytes;
-    pool_trim(g_pool_cap, POOL_BLOCKS);
+    pool_give_back(lk, g_pool_cap, POOL_BLOCKS);
     return hipSuccess;
 }
 
 void dev_pool_release()
 {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
-    pool_trim(0, 0);
+    std::unique_lock<std::mutex> lk(g_pool_mu);
+    pool_give_back(lk, 0, 0);
     g_pool_cap = 0;          // a share of the device at hand
 }
 
 int stream_wait()
 {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
-    if (g_pool_pending.empty()) {
+    std::unique_lock<std::mutex> lk(g_pool_mu);
+    const bool pending = !g_pool_pending.empty();
+    const uint64_t freed = g_pool_freed;
+    lk.unlock();
+    if (!pending) {
         COMET_HIPCHK(hipStreamSynchronize(stream()));
         return COMET_HIP_OK;
     }
     COMET_HIPCHK(hipDeviceSynchronize());
-    pool_promote();
+    lk.lock();
+    pool_promote(freed);
     return COMET_HIP_OK;
 }
 

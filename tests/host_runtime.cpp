@@ -9,6 +9,7 @@
 #include <sys/mman.h>
 #include <sys/resource.h>
 
+#include <algorithm>
 #include <chrono>
 #include <map>
 #include <mutex>
@@ -27,6 +28,7 @@ size_t total[DEVICES] = {288ull << 30, 288ull << 30}, used[DEVICES];
 struct Block { size_t bytes; int device; };
 std::map<char *, Block> blocks;
 struct Stream { int device; bool live; Clock::time_point idle; };
+std::vector<Stream *> streams;
 struct Event { int device; bool live; Clock::time_point done; };
 std::map<const void *, std::string> &kernels()          // asked for before this file's own statics are made
 {
@@ -125,13 +127,26 @@ hipError_t hipMemGetInfo(size_t *f, size_t *t)
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { *p = aligned_alloc(4096, (bytes + 4095) & ~4095ull); return hipSuccess; }
 hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 
-hipError_t hipStreamCreate(hipStream_t *s) { *s = reinterpret_cast<hipStream_t>(new Stream{current, true, Clock::now()}); return hipSuccess; }
+hipError_t hipStreamCreate(hipStream_t *s)
+{
+    streams.push_back(new Stream{current, true, Clock::now()});
+    *s = reinterpret_cast<hipStream_t>(streams.back());
+    return hipSuccess;
+}
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return hipStreamCreate(s); }
 hipError_t hipStreamDestroy(hipStream_t s) { stream_of(s)->live = false; return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) { std::this_thread::sleep_until(stream_of(s)->idle); return hipSuccess; }
 hipError_t hipStreamQuery(hipStream_t s) { return Clock::now() < stream_of(s)->idle ? hipErrorNotReady : hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
-hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
+hipError_t hipDeviceSynchronize(void)
+{
+    Clock::time_point until = Clock::now();          // what has been launched by now
+    for (Stream *s : streams)
+        if (s->live && s->device == current)
+            until = std::max(until, s->idle);
+    std::this_thread::sleep_until(until);
+    return hipSuccess;
+}
 
 hipError_t hipEventCreate(hipEvent_t *e) { *e = reinterpret_cast<hipEvent_t>(new Event{current, true, Clock::now()}); return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
@@ -186,6 +201,14 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
 }
 
 }  // extern "C"
+
+// from now on the device has something to do
+static void busy(int ms)
+{
+    for (Stream *s : streams)
+        s->idle = Clock::now() + std::chrono::milliseconds(ms);
+}
+static double ms_since(Clock::time_point t) { return std::chrono::duration<double, std::milli>(Clock::now() - t).count(); }
 
 #define REQUIRE(what)                                                                               \
     do {                                                                                            \
@@ -278,6 +301,44 @@ static int block_of_another_device()
     return 0;
 }
 
+// one thread waits for the device, another one wants memory
+static int memory_while_another_waits()
+{
+    REQUIRE(comet_hip_init(0) == 0);
+    std::vector<char> host(100);
+    const int64_t a = comet_hip_malloc(100), b = comet_hip_malloc(5000);
+    REQUIRE(a && b);
+    for (bool pending : {false, true}) {
+        if (pending)
+            REQUIRE(comet_hip_free(b) == 0);
+        int rc = -1;
+        busy(600);
+        const auto t0 = Clock::now();
+        std::thread waits([&] { rc = comet_hip_memcpy(a, host.data(), 100, 0); });
+        std::this_thread::sleep_for(std::chrono::milliseconds(100));
+        const int64_t c = comet_hip_malloc(pending ? 3 << 20 : 1 << 20);
+        REQUIRE(c && comet_hip_free(c) == 0);
+        const double ms = ms_since(t0);
+        waits.join();
+        REQUIRE(rc == 0 && ms_since(t0) >= 590);
+        REQUIRE(ms < 400);
+    }
+    // what was freed while that thread waited is not free to hand out: the work launched before may use it
+    busy(0);
+    const int64_t d = comet_hip_malloc(70000);
+    REQUIRE(d);
+    busy(300);
+    std::thread waits([&] { (void)comet_hip_memcpy(a, host.data(), 100, 0); });
+    std::this_thread::sleep_for(std::chrono::milliseconds(100));
+    busy(600);                                      // launched after that wait began
+    REQUIRE(comet_hip_free(d) == 0);
+    waits.join();
+    const auto t0 = Clock::now();
+    const int64_t e = comet_hip_malloc(70000);
+    REQUIRE(e && (e != d || ms_since(t0) > 100));
+    return 0;
+}
+
 int main(int, char **argv)
 {
     const std::string what = argv[1];
@@ -289,6 +350,8 @@ int main(int, char **argv)
         return given_back();
     if (what == "block_of_another_device")
         return block_of_another_device();
+    if (what == "memory_while_another_waits")
+        return memory_while_another_waits();
     fprintf(stderr, "no scenario %s\n", argv[1]);
     return 2;
 }

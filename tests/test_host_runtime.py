@@ -23,7 +23,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["another_device", "whole_device", "given_back", "block_of_another_device"])
+@pytest.mark.parametrize("scenario", ["another_device", "whole_device", "given_back", "block_of_another_device",
+                                      "memory_while_another_waits"])
 def test_host_side(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
