@@ -73,4 +73,56 @@ static void gett_add_dim(GettIndex *g, int64_t ext, int64_t s0, int64_t s1)
     ++g->nd;
 }
 
+// One more than the largest offset of an element whose two indices have the strides sx and sy in its tensor.
+static int64_t gett_span(const GettIndex &x, const int64_t *sx, const GettIndex &y, const int64_t *sy)
+{
+    int64_t last = 0;
+    for (int d = 0; d < x.nd; ++d)
+        last += ((int64_t)x.ext[d] - 1) * sx[d];
+    for (int d = 0; d < y.nd; ++d)
+        last += ((int64_t)y.ext[d] - 1) * sy[d];
+    return last + 1;
+}
+
+// Where a contraction is cut in two: dimension d of the index `which` (0: m, 1: n, 2: k), `first` values of it go to
+// the first half.  which < 0: it need not be cut.
+struct GettCut {
+    int which, d;
+    uint32_t first;
+};
+
+// The kernel adds 32-bit byte offsets to the operands, which is what lets it read them without vector arithmetic, so
+// an operand of more elements than `limit` is cut along the dimension that spans most of it.  Halves of this size
+// keep every CU busy for milliseconds; where the sum is cut, C is read and written once more.
+static GettCut gett_cut(const GettIndex &m, const GettIndex &n, const GettIndex &k, int64_t limit)
+{
+    GettCut cut{-1, 0, 0};
+    int64_t most = 0;
+    const auto look = [&](const GettIndex &x, const int64_t *s, int which) {
+        for (int d = 0; d < x.nd; ++d)
+            if (((int64_t)x.ext[d] - 1) * s[d] > most) {
+                most = ((int64_t)x.ext[d] - 1) * s[d];
+                const uint32_t half = x.ext[d] / 2 + x.ext[d] % 2, whole = (half + 127) / 128 * 128;
+                cut = GettCut{which, d, whole < x.ext[d] ? whole : half};          // whole tiles, if there are any
+            }
+    };
+    if (gett_span(m, m.s0, k, k.s0) > limit) {
+        look(m, m.s0, 0);
+        look(k, k.s0, 2);
+    } else if (gett_span(n, n.s0, k, k.s1) > limit) {
+        look(n, n.s0, 1);
+        look(k, k.s1, 2);
+    }
+    return cut;
+}
+
+// The index with `ext` values of dimension d.
+static GettIndex gett_part(const GettIndex &g, int d, uint32_t ext)
+{
+    GettIndex out{};
+    for (int i = 0; i < g.nd; ++i)
+        gett_add_dim(&out, i == d ? ext : g.ext[i], g.s0[i], g.s1[i]);
+    return out;
+}
+
 }  // namespace comet

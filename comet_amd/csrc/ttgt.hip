@@ -249,8 +249,7 @@ struct GettArgs {
 };
 
 // an element by its byte offset from a pointer that is the same for the whole wavefront
-template <typename OFF>
-__device__ __forceinline__ double gett_load(const double *base, OFF bytes)
+__device__ __forceinline__ double gett_load(const double *base, uint32_t bytes)
 {
     return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(base) + bytes);
 }
@@ -285,7 +284,7 @@ __device__ __forceinline__ void gett_offsets(const GettIndex &g, uint32_t i, OFF
     *o1 = b + (OFF)i * (OFF)g.s1[0];
 }
 
-template <int BM, int BN, int WM, int OCC, bool A_M, bool B_N, bool REG, bool RUN, typename OFF>
+template <int BM, int BN, int WM, int OCC, bool A_M, bool B_N, bool REG, bool RUN>
 __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const double *__restrict__ A,
                                                              const double *__restrict__ B, double *__restrict__ C,
                                                              double *__restrict__ partial, int use_c)
@@ -297,7 +296,7 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
     __shared__ double As[2][GM_BK][LDA];
     __shared__ double Bs[2][GM_BK][LDB];
     // offsets in bytes of the rows (A), the columns (B) and, unless they are regular, of the k of two turns
-    __shared__ OFF rowA[BM], colB[BN], kA[2][GM_BK], kB[2][GM_BK];
+    __shared__ uint32_t rowA[BM], colB[BN], kA[2][GM_BK], kB[2][GM_BK];
     __shared__ int64_t rowC[BM], colC[BN];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WN, wn = wave % WN;
@@ -310,7 +309,7 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
     const auto k_offsets = [&](int t) {          // the offsets of turn t's k, by the first sixteen lanes
         if (!REG && tid < GM_BK) {
             const uint32_t k = k_begin + (uint32_t)t * GM_BK + tid;
-            OFF a, b;
+            uint32_t a, b;
             gett_offsets(g.k, k < k_end ? k : k_end - 1, &a, &b);
             kA[t & 1][tid] = a * 8;
             kB[t & 1][tid] = b * 8;
@@ -319,13 +318,13 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
     for (int r = tid; r < BM; r += 256) {
         int64_t a, c;
         gett_offsets(g.m, m0 + r < g.M ? m0 + r : g.M - 1, &a, &c);
-        rowA[r] = (OFF)(a * 8);
+        rowA[r] = (uint32_t)(a * 8);
         rowC[r] = c;
     }
     for (int c = tid; c < BN; c += 256) {
         int64_t b, d;
         gett_offsets(g.n, n0 + c < g.N ? n0 + c : g.N - 1, &b, &d);
-        colB[c] = (OFF)(b * 8);
+        colB[c] = (uint32_t)(b * 8);
         colC[c] = d;
     }
     k_offsets(0);
@@ -346,21 +345,21 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
     const int last = g.k.nd - 1;
     const int64_t sa = g.k.s0[last], sb = g.k.s1[last];          // strides of the innermost k
     constexpr int NA = RUN || (A_M && !REG) ? 1 : EA, NB = RUN || (B_N && !REG) ? 1 : EB;
-    OFF ao[NA], bo[NB];
+    uint32_t ao[NA], bo[NB];
     if constexpr (RUN) {           // a run beyond the last row (their number is a multiple of EA then) is the last one
         const int ar = A_M && m0 + a_r >= g.M ? (int)(g.M - EA - m0) : a_r;
         const int bc = B_N && n0 + b_c >= g.N ? (int)(g.N - EB - n0) : b_c;
-        ao[0] = (ar >= 0 ? rowA[ar] : rowA[0] - (OFF)(-ar * 8)) + (OFF)(a_k * sa * 8);
-        bo[0] = (bc >= 0 ? colB[bc] : colB[0] - (OFF)(-bc * 8)) + (OFF)(b_k * sb * 8);
+        ao[0] = (ar >= 0 ? rowA[ar] : rowA[0] - (uint32_t)(-ar * 8)) + (uint32_t)(a_k * sa * 8);
+        bo[0] = (bc >= 0 ? colB[bc] : colB[0] - (uint32_t)(-bc * 8)) + (uint32_t)(b_k * sb * 8);
     } else {
 #pragma unroll
         for (int e = 0; e < NA; ++e)
-            ao[e] = A_M ? rowA[a_r] + (REG ? (OFF)((a_k + KSA * e) * sa * 8) : 0)
-                        : rowA[a_r + 16 * e] + (REG ? (OFF)(a_k * sa * 8) : 0);
+            ao[e] = A_M ? rowA[a_r] + (REG ? (uint32_t)((a_k + KSA * e) * sa * 8) : 0)
+                        : rowA[a_r + 16 * e] + (REG ? (uint32_t)(a_k * sa * 8) : 0);
 #pragma unroll
         for (int e = 0; e < NB; ++e)
-            bo[e] = B_N ? colB[b_c] + (REG ? (OFF)((b_k + KSB * e) * sb * 8) : 0)
-                        : colB[b_c + 16 * e] + (REG ? (OFF)(b_k * sb * 8) : 0);
+            bo[e] = B_N ? colB[b_c] + (REG ? (uint32_t)((b_k + KSB * e) * sb * 8) : 0)
+                        : colB[b_c + 16 * e] + (REG ? (uint32_t)(b_k * sb * 8) : 0);
     }
     double ra[EA], rb[EB];
     // REG: where the turn to load next begins, and how many turns are left in the innermost dimension
@@ -409,13 +408,13 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
 #pragma unroll
                 for (int e = 0; e < EA; ++e) {
                     const int k = A_M ? a_k + KSA * e : a_k, over = k < (int)left ? 0 : k - (int)left + 1;
-                    ra[e] = gett_fetch(Ab, (uint32_t)(ao[e] - (OFF)(over * sa * 8)), At);
+                    ra[e] = gett_fetch(Ab, ao[e] - (uint32_t)(over * sa * 8), At);
                     ra[e] = over ? 0.0 : ra[e];
                 }
 #pragma unroll
                 for (int e = 0; e < EB; ++e) {
                     const int k = B_N ? b_k + KSB * e : b_k, over = k < (int)left ? 0 : k - (int)left + 1;
-                    rb[e] = gett_fetch(Bb, (uint32_t)(bo[e] - (OFF)(over * sb * 8)), Bt);
+                    rb[e] = gett_fetch(Bb, bo[e] - (uint32_t)(over * sb * 8), Bt);
                     rb[e] = over ? 0.0 : rb[e];
                 }
             }
@@ -424,13 +423,13 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
             k_next += GM_BK;
             --run;
         } else {
-            const OFF *ka = kA[t & 1], *kb = kB[t & 1];
+            const uint32_t *ka = kA[t & 1], *kb = kB[t & 1];
 #pragma unroll
             for (int e = 0; e < EA; ++e)
-                ra[e] = gett_load(A, (OFF)(A_M ? ao[0] + ka[a_k + KSA * e] : ao[A_M ? 0 : e] + ka[a_k]));
+                ra[e] = gett_load(A, A_M ? ao[0] + ka[a_k + KSA * e] : ao[A_M ? 0 : e] + ka[a_k]);
 #pragma unroll
             for (int e = 0; e < EB; ++e)
-                rb[e] = gett_load(B, (OFF)(B_N ? bo[0] + kb[b_k + KSB * e] : bo[B_N ? 0 : e] + kb[b_k]));
+                rb[e] = gett_load(B, B_N ? bo[0] + kb[b_k + KSB * e] : bo[B_N ? 0 : e] + kb[b_k]);
             if (left < GM_BK) {
 #pragma unroll
                 for (int e = 0; e < EA; ++e)
@@ -577,32 +576,25 @@ constexpr int GETT_NSHAPES = sizeof(GETT_SHAPES) / sizeof(GETT_SHAPES[0]);
 
 static Workspace g_gett_partial;
 
-template <int BM, int BN, int WM, int OCC, bool REG, bool RUN, typename OFF>
+template <int BM, int BN, int WM, int OCC, bool REG, bool RUN>
 static void gett_launch(bool a_m, bool b_n, dim3 grid, const GettArgs &g, const double *A, const double *B, double *C,
                         double *partial, int use_c)
 {
     const dim3 block(256);
     if (a_m && b_n)
-        gett_mfma_kernel<BM, BN, WM, OCC, true, true, REG, RUN, OFF><<<grid, block, 0, stream()>>>(g, A, B, C, partial, use_c);
+        gett_mfma_kernel<BM, BN, WM, OCC, true, true, REG, RUN><<<grid, block, 0, stream()>>>(g, A, B, C, partial, use_c);
     else if (a_m)
-        gett_mfma_kernel<BM, BN, WM, OCC, true, false, REG, RUN, OFF><<<grid, block, 0, stream()>>>(g, A, B, C, partial, use_c);
+        gett_mfma_kernel<BM, BN, WM, OCC, true, false, REG, RUN><<<grid, block, 0, stream()>>>(g, A, B, C, partial, use_c);
     else if (b_n)
-        gett_mfma_kernel<BM, BN, WM, OCC, false, true, REG, RUN, OFF><<<grid, block, 0, stream()>>>(g, A, B, C, partial, use_c);
+        gett_mfma_kernel<BM, BN, WM, OCC, false, true, REG, RUN><<<grid, block, 0, stream()>>>(g, A, B, C, partial, use_c);
     else
-        gett_mfma_kernel<BM, BN, WM, OCC, false, false, REG, RUN, OFF><<<grid, block, 0, stream()>>>(g, A, B, C, partial, use_c);
+        gett_mfma_kernel<BM, BN, WM, OCC, false, false, REG, RUN><<<grid, block, 0, stream()>>>(g, A, B, C, partial, use_c);
 }
 
-// C (+)= A * B over the three indices; span: one more than the largest offset into any of the tensors.
-static int gett_device(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t N, int64_t K, int64_t span,
-                       const double *A, const double *B, double *C, double beta)
+// C (+)= A * B over the three indices, none of them empty, A and B within the reach of 32-bit byte offsets.
+static int gett_run(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t N, int64_t K, const double *A,
+                    const double *B, double *C, double beta)
 {
-    if (M == 0 || N == 0)
-        return COMET_HIP_OK;
-    if (K == 0) {               // empty sums; C is whole and contiguous
-        if (beta == 0.0)
-            COMET_HIPCHK(hipMemsetAsync(C, 0, sizeof(double) * (size_t)(M * N), stream()));
-        return COMET_HIP_OK;
-    }
     if (M >= (1ll << 31) || N >= (1ll << 31) || K >= (1ll << 31))
         return set_error(COMET_HIP_ERR_SIZE, "contraction of %lld x %lld x %lld: an index exceeds 31 bits", (long long)M,
                          (long long)N, (long long)K);
@@ -644,11 +636,10 @@ static int gett_device(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t
     g.K = (uint32_t)K;
     const int64_t nk = ceil_div(K, GM_BK);
     const int64_t cus = num_cus() > 0 ? num_cus() : 256;
-    const bool wide = span >= (1ll << 29);          // byte offsets beyond 32 bits
     int best = 0;
     int64_t splits = 1;
     double best_us = 0.0;
-    for (int c = 0; c < (wide ? 1 : GETT_NSHAPES); ++c) {
+    for (int c = 0; c < GETT_NSHAPES; ++c) {
         const GettShape &sh = GETT_SHAPES[c];
         const int64_t tiles = ceil_div(M, sh.bm) * ceil_div(N, sh.bn);
         for (int64_t s = 1; s <= nk && s <= 1024; s *= 2) {
@@ -670,7 +661,7 @@ static int gett_device(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t
     // the same one through all of them)
     if (const char *e = getenv("COMET_HIP_GETT")) {
         long long c = 0, s = 1;
-        if (sscanf(e, "%lld,%lld", &c, &s) == 2 && c >= 0 && c < (wide ? 1 : GETT_NSHAPES) && s >= 1 && s <= nk && s < 65536) {
+        if (sscanf(e, "%lld,%lld", &c, &s) == 2 && c >= 0 && c < GETT_NSHAPES && s >= 1 && s <= nk && s < 65536) {
             best = (int)c;
             g.turns = (uint32_t)ceil_div(nk, s);
             splits = ceil_div(nk, (int64_t)g.turns);
@@ -707,16 +698,14 @@ static int gett_device(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t
             constexpr int WM = decltype(wave_rows)::value, OCC = decltype(occ)::value;
             if constexpr (S.bn >= 64)
                 if (unbroken)
-                    return gett_launch<S.bm, S.bn, WM, OCC, true, true, uint32_t>(a_m, b_n, grid, g, A, B, C, partial, use_c);
+                    return gett_launch<S.bm, S.bn, WM, OCC, true, true>(a_m, b_n, grid, g, A, B, C, partial, use_c);
             if (reg)
-                gett_launch<S.bm, S.bn, WM, OCC, true, false, uint32_t>(a_m, b_n, grid, g, A, B, C, partial, use_c);
+                gett_launch<S.bm, S.bn, WM, OCC, true, false>(a_m, b_n, grid, g, A, B, C, partial, use_c);
             else
-                gett_launch<S.bm, S.bn, WM, OCC, false, false, uint32_t>(a_m, b_n, grid, g, A, B, C, partial, use_c);
+                gett_launch<S.bm, S.bn, WM, OCC, false, false>(a_m, b_n, grid, g, A, B, C, partial, use_c);
         };
         using std::integral_constant;
-        if (wide)
-            gett_launch<128, 128, 2, COMET_GM_OCC, false, false, int64_t>(a_m, b_n, grid, g, A, B, C, partial, use_c);
-        else if (best == 0)
+        if (best == 0)
             launch(integral_constant<int, 0>(), integral_constant<int, 2>(), integral_constant<int, COMET_GM_OCC>());
         else if (best == 1)
             launch(integral_constant<int, 1>(), integral_constant<int, 2>(), integral_constant<int, 4>());
@@ -737,6 +726,50 @@ static int gett_device(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t
     return COMET_HIP_OK;
 }
 
+// Elements an operand may have to be read through 32-bit byte offsets (its last byte is one that a buffer may hold).
+constexpr int64_t GETT_SPAN = (1ll << 29) - 1;
+
+static int gett_pieces(const GettIndex &m, const GettIndex &n, const GettIndex &k, int64_t limit, int64_t M, int64_t N,
+                       int64_t K, const double *A, const double *B, double *C, double beta)
+{
+    const GettCut cut = gett_cut(m, n, k, limit);
+    if (cut.which < 0)
+        return gett_run(m, n, k, M, N, K, A, B, C, beta);
+    const GettIndex &x = cut.which == 0 ? m : cut.which == 1 ? n : k;
+    const uint32_t ext = x.ext[cut.d];
+    const int64_t o0 = x.s0[cut.d] * cut.first, o1 = x.s1[cut.d] * cut.first;
+    for (int half = 0; half < 2; ++half) {
+        const uint32_t part = half == 0 ? cut.first : ext - cut.first;
+        const GettIndex p = gett_part(x, cut.d, part);
+        if (cut.which == 0)
+            COMET_CHK(gett_pieces(p, n, k, limit, M / ext * part, N, K, A + (half ? o0 : 0), B, C + (half ? o1 : 0), beta));
+        else if (cut.which == 1)
+            COMET_CHK(gett_pieces(m, p, k, limit, M, N / ext * part, K, A, B + (half ? o0 : 0), C + (half ? o1 : 0), beta));
+        else          // the second half of the sum adds to the first
+            COMET_CHK(gett_pieces(m, n, p, limit, M, N, K / ext * part, A + (half ? o0 : 0), B + (half ? o1 : 0), C,
+                                  half ? 1.0 : beta));
+    }
+    return COMET_HIP_OK;
+}
+
+// C (+)= A * B over the three indices.
+static int gett_device(const GettIndex &m, const GettIndex &n, const GettIndex &k, int64_t M, int64_t N, int64_t K,
+                       const double *A, const double *B, double *C, double beta)
+{
+    if (M == 0 || N == 0)
+        return COMET_HIP_OK;
+    if (K == 0) {               // empty sums; C is whole and contiguous
+        if (beta == 0.0)
+            COMET_HIPCHK(hipMemsetAsync(C, 0, sizeof(double) * (size_t)(M * N), stream()));
+        return COMET_HIP_OK;
+    }
+    // COMET_HIP_GETT_SPAN=elements cuts smaller operands (the pieces make the same result: the tests cut small ones)
+    int64_t limit = GETT_SPAN;
+    if (const char *e = getenv("COMET_HIP_GETT_SPAN"))
+        limit = std::max<int64_t>(1, std::min<int64_t>(limit, atoll(e)));
+    return gett_pieces(m, n, k, limit, M, N, K, A, B, C, beta);
+}
+
 // Row-major C[M,N] = beta*C + A[M,K]*B[K,N].
 static int dgemm_device(int64_t M, int64_t N, int64_t K, const double *A, const double *B, double *C, double beta)
 {
@@ -748,7 +781,7 @@ static int dgemm_device(int64_t M, int64_t N, int64_t K, const double *A, const 
     gett_add_dim(&m, M, K, N);
     gett_add_dim(&n, N, 1, 1);
     gett_add_dim(&k, K, 1, N);
-    return gett_device(m, n, k, M, N, K, std::max(M * K, std::max(K * N, M * N)), A, B, C, beta);
+    return gett_device(m, n, k, M, N, K, A, B, C, beta);
 }
 
 // ============================================================================
@@ -930,11 +963,11 @@ static int contract_strided(const comet_ttgt_plan &p, const int64_t *a_shape, co
             out[i] = s;
             s *= shape[i];
         }
-        return s;
     };
     int64_t sa[8], sb[8], sc[8];
-    const int64_t span = std::max(strides(a_shape, p.rankA, sa),
-                                  std::max(strides(b_shape, p.rankB, sb), strides(c_shape, p.rankC, sc)));
+    strides(a_shape, p.rankA, sa);
+    strides(b_shape, p.rankB, sb);
+    strides(c_shape, p.rankC, sc);
     const PlanDims d = plan_dims(p);
     GettIndex m{}, n{}, k{};
     const auto da = [&](int i) { return plan_dim(p.transA, p.permA, i); };
@@ -984,7 +1017,7 @@ static int contract_strided(const comet_ttgt_plan &p, const int64_t *a_shape, co
         COMET_CHK(w.ensure(sizeof(double) * (size_t)((turn_a ? p.M : p.N) * p.K), false));
         COMET_CHK(transpose_device(rank, shape, perm, turn_a ? A : B, (double *)w.ptr));
         int64_t st[8];
-        (void)strides(other, rank, st);
+        strides(other, rank, st);
         int64_t *s_mine = turn_a ? sa : sb;
         for (int i = 0; i < rank; ++i)
             s_mine[perm[i]] = st[i];
@@ -997,7 +1030,7 @@ static int contract_strided(const comet_ttgt_plan &p, const int64_t *a_shape, co
         for (int i = 0; i < d.nk; ++i)
             gett_add_dim(&k, a_shape[da(d.ak + i)], sa[da(d.ak + i)], sb[db(d.bk + i)]);
     }
-    return gett_device(m, n, k, p.M, p.N, p.K, span, A, B, C, beta);
+    return gett_device(m, n, k, p.M, p.N, p.K, A, B, C, beta);
 }
 
 }  // namespace comet

@@ -52,6 +52,36 @@ def test_contraction_every_tile_shape_and_layout(a, b, c, forced, monkeypatch):
             assert np.all(np.abs(dC.to_numpy() - want - beta * C0) <= 1e-13 * (bound + 1.0)), (extent, beta)
 
 
+@pytest.mark.parametrize("pieces", [2, 3, 7])
+@pytest.mark.parametrize("a,b,c", [("ef", "fc", "ec"), ("aebf", "dfce", "abcd"), ("aebf", "efcd", "abcd"), ("feab", "efcd", "dcba"),
+                                   ("abef", "ef", "ab"), ("ab", "cd", "acbd"), ("f", "fa", "a")])
+def test_contraction_in_pieces(a, b, c, pieces, monkeypatch):
+    # operands beyond 4 GiB are cut; here small ones are, along every index
+    for i, extent in enumerate(EXTENTS + [dict(a=300, b=1, c=2, d=2, e=1, f=260), dict(a=3, b=1, c=280, d=1, e=2, f=530)]):
+        rng = np.random.default_rng(i)
+        A, B = (rng.uniform(-1, 1, [extent[x] for x in lab]) for lab in (a, b))
+        C0 = rng.uniform(-1, 1, [extent[x] for x in c])
+        want, bound = (np.einsum(f"{a},{b}->{c}", f(A), f(B)) for f in (np.array, np.abs))
+        monkeypatch.setenv("COMET_HIP_GETT_SPAN", str(max(A.size, B.size) // pieces + 1))
+        for beta in (0.0, 1.0):
+            dC = rt.DeviceArray.from_numpy(C0)
+            rt.ttgt_contract(a, b, c, rt.DeviceArray.from_numpy(A), rt.DeviceArray.from_numpy(B), dC, beta=beta)
+            assert np.all(np.abs(dC.to_numpy() - want - beta * C0) <= 1e-13 * (bound + 1.0)), (extent, beta)
+
+
+def test_contraction_of_an_operand_beyond_4_gib():
+    # 1,500,672 x 361 doubles, the same 1536 rows over and over
+    block, times, k = 1536, 977, 361
+    A, B = (np.random.default_rng(i).uniform(-1, 1, s) for i, s in enumerate([(block, k), (k, 3)]))
+    dA, dB = rt.DeviceArray((block * times, k)), rt.DeviceArray.from_numpy(B)
+    assert 8 * block * times * k > 1 << 32
+    for i in range(times):
+        rt._check(rt.lib().comet_hip_memcpy(dA.ptr + 8 * i * block * k, rt._vptr(A), A.nbytes, 0))
+    C, _ = rt.ttgt_contract("ab", "bc", "ac", dA, dB)
+    got = C.to_numpy().reshape(times, block, 3)
+    assert np.all(np.abs(got - A @ B) <= 1e-13 * (np.abs(A) @ np.abs(B)))
+
+
 @pytest.mark.parametrize("extent", [dict(a=24, b=23, c=22, d=21, e=25, f=26), dict(a=32, b=16, c=32, d=17, e=32, f=16)])
 def test_contraction_with_a_turned_operand(extent):
     rng = np.random.default_rng(7)
