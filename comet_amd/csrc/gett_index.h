@@ -13,7 +13,7 @@ constexpr int GETT_MAXRANK = 8;
 // A multi-index: extents (outermost first) and the strides of its dimensions in the two tensors it appears in.
 struct GettIndex {
     int nd;
-    uint32_t ext[GETT_MAXRANK];
+    int64_t ext[GETT_MAXRANK];
     int64_t s0[GETT_MAXRANK], s1[GETT_MAXRANK];
 };
 
@@ -41,8 +41,7 @@ static bool gett_order(GettIndex *g, int first)
     std::sort(rest.begin(), rest.end(), [&](int x, int y) { return key[x] < key[y]; });
     order.insert(order.end(), rest.begin(), rest.end());
     g->nd = 0;
-    uint32_t ext[GETT_MAXRANK];
-    int64_t s0[GETT_MAXRANK], s1[GETT_MAXRANK];
+    int64_t ext[GETT_MAXRANK], s0[GETT_MAXRANK], s1[GETT_MAXRANK];
     int n = 0;
     for (int d : order) {
         if (n > 0 && s0[n - 1] * ext[n - 1] == in.s0[d] && s1[n - 1] * ext[n - 1] == in.s1[d]) {
@@ -67,7 +66,7 @@ static void gett_add_dim(GettIndex *g, int64_t ext, int64_t s0, int64_t s1)
 {
     if (ext == 1)
         return;
-    g->ext[g->nd] = (uint32_t)ext;
+    g->ext[g->nd] = ext;
     g->s0[g->nd] = s0;
     g->s1[g->nd] = s1;
     ++g->nd;
@@ -78,9 +77,9 @@ static int64_t gett_span(const GettIndex &x, const int64_t *sx, const GettIndex 
 {
     int64_t last = 0;
     for (int d = 0; d < x.nd; ++d)
-        last += ((int64_t)x.ext[d] - 1) * sx[d];
+        last += (x.ext[d] - 1) * sx[d];
     for (int d = 0; d < y.nd; ++d)
-        last += ((int64_t)y.ext[d] - 1) * sy[d];
+        last += (y.ext[d] - 1) * sy[d];
     return last + 1;
 }
 
@@ -88,11 +87,12 @@ static int64_t gett_span(const GettIndex &x, const int64_t *sx, const GettIndex 
 // the first half.  which < 0: it need not be cut.
 struct GettCut {
     int which, d;
-    uint32_t first;
+    int64_t first;
 };
 
 // The kernel adds 32-bit byte offsets to the operands, which is what lets it read them without vector arithmetic, so
-// an operand of more elements than `limit` is cut along the dimension that spans most of it.  Halves of this size
+// an operand of more elements than `limit` is cut along the dimension that spans most of it.  (So are the indices kept
+// within 32 bits: none of a piece has more elements than the operands it is in.)  Halves of this size
 // keep every CU busy for milliseconds; where the sum is cut, C is read and written once more.
 static GettCut gett_cut(const GettIndex &m, const GettIndex &n, const GettIndex &k, int64_t limit)
 {
@@ -100,9 +100,9 @@ static GettCut gett_cut(const GettIndex &m, const GettIndex &n, const GettIndex 
     int64_t most = 0;
     const auto look = [&](const GettIndex &x, const int64_t *s, int which) {
         for (int d = 0; d < x.nd; ++d)
-            if (((int64_t)x.ext[d] - 1) * s[d] > most) {
-                most = ((int64_t)x.ext[d] - 1) * s[d];
-                const uint32_t half = x.ext[d] / 2 + x.ext[d] % 2, whole = (half + 127) / 128 * 128;
+            if ((x.ext[d] - 1) * s[d] > most) {
+                most = (x.ext[d] - 1) * s[d];
+                const int64_t half = x.ext[d] / 2 + x.ext[d] % 2, whole = (half + 127) / 128 * 128;
                 cut = GettCut{which, d, whole < x.ext[d] ? whole : half};          // whole tiles, if there are any
             }
     };
@@ -117,7 +117,7 @@ static GettCut gett_cut(const GettIndex &m, const GettIndex &n, const GettIndex 
 }
 
 // The index with `ext` values of dimension d.
-static GettIndex gett_part(const GettIndex &g, int d, uint32_t ext)
+static GettIndex gett_part(const GettIndex &g, int d, int64_t ext)
 {
     GettIndex out{};
     for (int i = 0; i < g.nd; ++i)

@@ -242,8 +242,14 @@ constexpr int GM_BK = 16, GM_PAD = 4;
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
+// The same as the kernel takes it.
+struct GettDims {
+    int nd;
+    uint32_t ext[GETT_MAXRANK];
+    int64_t s0[GETT_MAXRANK], s1[GETT_MAXRANK];
+};
 struct GettArgs {
-    GettIndex m, n, k;           // m: A, C   n: B, C   k: A, B
+    GettDims m, n, k;            // m: A, C   n: B, C   k: A, B
     uint32_t M, N, K;
     uint32_t turns;              // turns of 16 k per split
 };
@@ -271,7 +277,7 @@ __device__ __forceinline__ double2_t gett_fetch2(__amdgpu_buffer_rsrc_t p, uint3
 }
 
 template <typename OFF>
-__device__ __forceinline__ void gett_offsets(const GettIndex &g, uint32_t i, OFF *o0, OFF *o1)
+__device__ __forceinline__ void gett_offsets(const GettDims &g, uint32_t i, OFF *o0, OFF *o1)
 {
     OFF a = 0, b = 0;
     for (int d = g.nd - 1; d > 0; --d) {
@@ -595,9 +601,6 @@ static void gett_launch(bool a_m, bool b_n, dim3 grid, const GettArgs &g, const 
 static int gett_run(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t N, int64_t K, const double *A,
                     const double *B, double *C, double beta)
 {
-    if (M >= (1ll << 31) || N >= (1ll << 31) || K >= (1ll << 31))
-        return set_error(COMET_HIP_ERR_SIZE, "contraction of %lld x %lld x %lld: an index exceeds 31 bits", (long long)M,
-                         (long long)N, (long long)K);
     const auto unit_in_c = [](const GettIndex &g) {
         for (int d = 0; d < g.nd; ++d)
             if (g.s1[d] == 1)
@@ -628,9 +631,17 @@ static int gett_run(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t N,
             x->ext[0] = 1;
             x->s0[0] = x->s1[0] = 0;
         }
-    g.m = m;
-    g.n = n;
-    g.k = k;
+    const auto dims = [](const GettIndex &x, GettDims *out) {
+        out->nd = x.nd;
+        for (int d = 0; d < x.nd; ++d) {
+            out->ext[d] = (uint32_t)x.ext[d];
+            out->s0[d] = x.s0[d];
+            out->s1[d] = x.s1[d];
+        }
+    };
+    dims(m, &g.m);
+    dims(n, &g.n);
+    dims(k, &g.k);
     g.M = (uint32_t)M;
     g.N = (uint32_t)N;
     g.K = (uint32_t)K;
@@ -736,10 +747,10 @@ static int gett_pieces(const GettIndex &m, const GettIndex &n, const GettIndex &
     if (cut.which < 0)
         return gett_run(m, n, k, M, N, K, A, B, C, beta);
     const GettIndex &x = cut.which == 0 ? m : cut.which == 1 ? n : k;
-    const uint32_t ext = x.ext[cut.d];
+    const int64_t ext = x.ext[cut.d];
     const int64_t o0 = x.s0[cut.d] * cut.first, o1 = x.s1[cut.d] * cut.first;
     for (int half = 0; half < 2; ++half) {
-        const uint32_t part = half == 0 ? cut.first : ext - cut.first;
+        const int64_t part = half == 0 ? cut.first : ext - cut.first;
         const GettIndex p = gett_part(x, cut.d, part);
         if (cut.which == 0)
             COMET_CHK(gett_pieces(p, n, k, limit, M / ext * part, N, K, A + (half ? o0 : 0), B, C + (half ? o1 : 0), beta));
@@ -949,7 +960,7 @@ static bool gett_fits(const comet_ttgt_plan &p, const int64_t *a_shape, const in
             return false;
         K *= a(d.ak + i);
     }
-    return M == p.M && N == p.N && K == p.K && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31);
+    return M == p.M && N == p.N && K == p.K;
 }
 
 constexpr double GETT_TURN_MIN = 1.28e8;

@@ -98,7 +98,8 @@ LIMIT = (1 << 29) - 1
     ([(32768, 32768, 32768)], [(32768, 1, 1)], [(32768, 1, 32768)]),                                  # both operands, m and k
     ([(1 << 29, 1, 1)], [(1, 1, 1)], [(3, 1 << 29, 1)]),                                              # k is outermost
     ([(160, 160**3, 160**3), (160, 160, 160**2)], [(160, 160**3, 1), (160, 160, 160)], [(160, 160**2, 1), (160, 1, 160**2)]),
-    ([], [], [((1 << 31) - 1, 1, 1)]), ([((1 << 31) - 1, 1, 1)], [], []), ([(2, 1 << 30, 1)], [(5, 1, 2)], [(1 << 30, 1, 5)])])
+    ([], [], [((1 << 31) - 1, 1, 1)]), ([((1 << 31) - 1, 1, 1)], [], []),
+    ([], [], [((1 << 33) + 3, 1, 1)]), ([((1 << 32) + 1, 1, 1)], [], []), ([], [((1 << 31) + 7, 1, 1)], [(2, 1, (1 << 31) + 7)]), ([(2, 1 << 30, 1)], [(5, 1, 2)], [(1 << 30, 1, 5)])])
 def test_pieces_cover_a_large_contraction_once(order, m, n, k):
     drop = lambda x: [d for d in x if d[0] > 1]
     todo, done, total = [(drop(m), drop(n), drop(k))], 0, 1

@@ -82,6 +82,17 @@ def test_contraction_of_an_operand_beyond_4_gib():
     assert np.all(np.abs(got - A @ B) <= 1e-13 * (np.abs(A) @ np.abs(B)))
 
 
+def test_contraction_over_an_index_beyond_31_bits():
+    block, times = 1 << 21, 1025
+    a, b = (np.random.default_rng(i).uniform(-1, 1, block) for i in (3, 4))
+    dA, dB = rt.DeviceArray((1, block * times)), rt.DeviceArray((block * times, 1))
+    for d, h in ((dA, a), (dB, b)):
+        for i in range(times):
+            rt._check(rt.lib().comet_hip_memcpy(d.ptr + 8 * block * i, rt._vptr(h), h.nbytes, 0))
+    C, _ = rt.ttgt_contract("ak", "kb", "ab", dA, dB)
+    assert abs(C.to_numpy()[0, 0] - times * (a @ b)) <= 1e-13 * times * (np.abs(a) @ np.abs(b))
+
+
 @pytest.mark.parametrize("extent", [dict(a=24, b=23, c=22, d=21, e=25, f=26), dict(a=32, b=16, c=32, d=17, e=32, f=16)])
 def test_contraction_with_a_turned_operand(extent):
     rng = np.random.default_rng(7)
