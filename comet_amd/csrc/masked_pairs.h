@@ -16,7 +16,9 @@
 struct PairEnt {
     uint32_t start, len;         // first entry of the list, number of entries
 };
-constexpr int64_t PAIR_NNZ_MAX = (1ll << 31) - 1;          // entries of a matrix that a PairEnt can name
+// Entries of a matrix that a PairEnt can name.  (The transposes that the plans are made from number them in 32 bits too,
+// and a launch with a lane for each has to stay below 2^32 lanes.)
+constexpr int64_t PAIR_NNZ_MAX = (1ll << 32) - (1 << 12);
 
 // One side of a pair problem on the device.
 struct PairSide {
@@ -310,7 +312,7 @@ __device__ __forceinline__ void quad_place(uint2 m, uint32_t &before, int a0, in
     owner = (int)__builtin_amdgcn_mbcnt_hi(m.y, __builtin_amdgcn_mbcnt_lo(m.x, before));
     before += __popc(m.x) + __popc(m.y);
     const uint32_t at = (uint32_t)lane_value(a0, owner) + at0;
-    const int left = lane_value(end, owner) - (int)at;
+    const int left = (int)((uint32_t)lane_value(end, owner) - at);          // right across 2^31 too
     from = left <= 0 ? 0u : at < most ? at : most;
     const int n = left < 0 ? 0 : left < 4 ? left : 4;
     mask = __builtin_amdgcn_ubfe(0xfu, 0, n) << ((at - from) & 31u);

@@ -1,5 +1,7 @@
 """The sizes at which a kernel or a rule of a dispatch can go wrong: edges of tiles, remainders, both sides of a
 threshold - against the oracle or numpy."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -166,6 +168,43 @@ def test_masked_sum_of_nearly_empty_matrices(nnz):
     x = (pos, np.arange(nnz, dtype=np.int32), np.ones(nnz))
     A = rt.CsrMatrix.from_arrays((5, 5), *x)
     assert rt.spgemm_masked_sum(A, A, A) == (nnz if nnz else 0)
+
+
+def test_masked_sum_of_a_matrix_beyond_31_bits_of_entries():
+    # 1,048,577 rows of 2051 columns, the same 4096 rows over and over; the lists asked for lie at both ends of the arrays
+    # and where entry 2^31 is
+    rng = np.random.default_rng(9)
+    ncols, per, block = 5000, 2051, 4096
+    n = (1 << 20) + 1
+    nnz = n * per
+    assert nnz > 1 << 31
+    cols = np.sort(np.argsort(rng.random((block, ncols)), axis=1)[:, :per].astype(np.int32), axis=1)
+    crd, val = rt.DeviceArray(nnz, np.int32), rt.DeviceArray(nnz)
+    threes = np.full(block * per, 3.0)
+    L = rt.lib()
+    for r in range(0, n, block):
+        rows = min(block, n - r)
+        rt._check(L.comet_hip_memcpy(crd.ptr + 4 * r * per, rt._vptr(cols), 4 * rows * per, 0))
+        rt._check(L.comet_hip_memcpy(val.ptr + 8 * r * per, rt._vptr(threes), 8 * rows * per, 0))
+    pos = rt.DeviceArray.from_numpy(np.arange(n + 1, dtype=np.int64) * per)
+    b = L.comet_hip_csr_wrap(n, ncols, nnz, pos.ptr, crd.ptr, val.ptr)
+    assert b, L.comet_hip_last_error()
+    middle = (1 << 31) // per
+    ks = np.unique(np.concatenate([[0, 1, n - 2, n - 1], middle + np.arange(-3, 4), rng.integers(0, n, 400)])).astype(np.int32)
+    mrows = [np.sort(rng.choice(ncols, l, replace=False)).astype(np.int32) for l in (4000, 100, 1)]
+    csr = lambda rows, m, v: rt.CsrMatrix.from_arrays((len(rows), m), np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int64),
+                                                      np.concatenate(rows), np.full(sum(map(len, rows)), v))
+    A, M = csr([ks] * 3, n, 2.0), csr(mrows, ncols, 1.0)
+    got = C.c_double(0.0)
+    rt.profile_reset()
+    rt.profile_enable(True)
+    rt._check(L.comet_hip_spgemm_masked_sum(A.handle, b, M.handle, C.byref(got)))
+    taken = rt.profile_report()
+    rt.profile_enable(False)
+    rt._check(L.comet_hip_csr_destroy(b))
+    hits = sum(np.isin(cols[ks % block], r).sum() for r in mrows)
+    assert got.value == 6.0 * hits
+    assert "spgemm_pair_plan" in taken
 
 
 @pytest.mark.parametrize("semiring", [None, ("min", "plus")])
