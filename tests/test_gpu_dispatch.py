@@ -1,6 +1,7 @@
 """The sizes at which a kernel or a rule of a dispatch can go wrong: edges of tiles, remainders, both sides of a
 threshold - against the oracle or numpy."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -105,15 +106,32 @@ def test_contraction_with_a_turned_operand(extent):
 
 
 @pytest.mark.parametrize("nbytes", [1, 15, 16, (1 << 18) - 1, (1 << 18) + 1, (1 << 20) + 7, (1 << 20) * 7 + 16, (1 << 20) * 19 + 5])
-@pytest.mark.parametrize("offset", [0, 4, 16])
+@pytest.mark.parametrize("offset", [0, 1, 4, 8, 15, 16, 27])
 def test_copies_between_host_and_device(nbytes, offset):
     host = np.random.default_rng(nbytes).integers(0, 256, nbytes, dtype=np.uint8)
-    d = rt.DeviceArray(nbytes + 32, np.uint8, zero=True)
+    d = rt.DeviceArray(nbytes + 64, np.uint8, zero=True)
     rt._check(rt.lib().comet_hip_memcpy(d.ptr + offset, rt._vptr(host), nbytes, 0))
     back = np.zeros(nbytes, np.uint8)
     rt._check(rt.lib().comet_hip_memcpy(d.ptr + offset, rt._vptr(back), nbytes, 1))
     whole = d.to_numpy()
     assert np.array_equal(back, host) and not whole[:offset].any() and not whole[offset + nbytes:].any()
+    assert np.array_equal(whole[offset:offset + nbytes], host)
+
+
+def test_copies_are_as_fast_wherever_they_begin():
+    # byte by byte it would take twice as long
+    nbytes = 60 << 10
+    host = np.zeros(nbytes, np.uint8)
+    d = rt.DeviceArray(nbytes + 64, np.uint8)
+    def best(offset):
+        times = []
+        for _ in range(50):
+            t = time.perf_counter()
+            rt._check(rt.lib().comet_hip_memcpy(d.ptr + offset, rt._vptr(host), nbytes, 0))
+            times.append(time.perf_counter() - t)
+        return min(times)
+    best(0)
+    assert best(8) <= 1.5 * best(0)
 
 
 @pytest.mark.parametrize("idt", [np.int64, np.int32])
