@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <functional>
 #include <mutex>
@@ -140,14 +141,30 @@ struct Crew {
     }
 };
 
-std::mutex g_crew_mu;          // one transfer at a time
+std::mutex g_crew_mu;          // one transfer at a time: the next one's copies come after this one's on the stream anyway
 Crew *g_crew = new Crew();     // never destroyed: its threads outlive main
 
-int spin_until(hipEvent_t e)
-{
-    hipError_t s;
-    while ((s = hipEventQuery(e)) == hipErrorNotReady) {
+// Asking again and again sees the end of a wait at once, and for as long as the copies of a call take - or the short
+// product before a download: threads that have to be woken first cost it 60 us - that is worth four CPUs.  After ASKING
+// the device is at something long, and naps of a thirtieth of the wait, a millisecond at most, do.
+constexpr std::chrono::microseconds ASKING(1000), LONGEST_NAP(1000);
+struct Waiting {
+    std::chrono::steady_clock::time_point begin = std::chrono::steady_clock::now();
+    void pause() const
+    {
+        const auto waited = std::chrono::steady_clock::now() - begin;
+        if (waited > ASKING)
+            std::this_thread::sleep_for(std::min<std::chrono::nanoseconds>(waited / 32, LONGEST_NAP));
     }
+};
+
+template <typename QUERY>
+int wait_for(QUERY query)
+{
+    const Waiting waiting;
+    hipError_t s;
+    while ((s = query()) == hipErrorNotReady)
+        waiting.pause();
     COMET_HIPCHK(s);
     return COMET_HIP_OK;
 }
@@ -218,7 +235,8 @@ int transfer(const std::vector<Piece> &pieces, bool up)
         state[(size_t)g] = 1;
     };
     const auto wait_across = [&](int g) {          // one thread at a time asks the runtime
-        while (state[(size_t)g] != 2 && !failed)
+        const Waiting waiting;
+        for (; state[(size_t)g] != 2 && !failed; waiting.pause())
             if (state[(size_t)g] == 1 && asking.try_lock()) {
                 if (state[(size_t)g] == 1) {
                     const hipError_t e = hipEventQuery(crew.moved[g % SLOTS]);
@@ -250,7 +268,7 @@ int transfer(const std::vector<Piece> &pieces, bool up)
         }
     };
     for (hipEvent_t e : crew.moved)          // the transfer before may still be reading the slots
-        COMET_CHK(spin_until(e));
+        COMET_CHK(wait_for([&] { return hipEventQuery(e); }));
     if (!up)
         for (int g = 0; g < SLOTS && g < ngroups; ++g)
             launch(g);

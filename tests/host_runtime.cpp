@@ -339,6 +339,34 @@ static int memory_while_another_waits()
     return 0;
 }
 
+// a copy that has to wait for the device does not keep the CPUs busy meanwhile
+static int waiting_is_cheap()
+{
+    REQUIRE(comet_hip_init(0) == 0);
+    const int64_t bytes = 40 << 20;
+    std::vector<char> host((size_t)bytes, 1);
+    const int64_t d = comet_hip_malloc(bytes);
+    REQUIRE(d);
+    const auto cpu_ms = [] {
+        rusage u;
+        getrusage(RUSAGE_SELF, &u);
+        return (double)(u.ru_utime.tv_sec + u.ru_stime.tv_sec) * 1e3 + (double)(u.ru_utime.tv_usec + u.ru_stime.tv_usec) / 1e3;
+    };
+    for (int64_t n : {bytes, (int64_t)1000})
+        for (int direction : {0, 1, 0, 1}) {
+            REQUIRE(comet_hip_memcpy(d, host.data(), n, direction) == 0);          // what it costs with an idle device
+            const double c0 = cpu_ms();
+            REQUIRE(comet_hip_memcpy(d, host.data(), n, direction) == 0);
+            const double c1 = cpu_ms();
+            busy(600);
+            const auto t0 = Clock::now();
+            REQUIRE(comet_hip_memcpy(d, host.data(), n, direction) == 0);
+            REQUIRE(ms_since(t0) >= 590);
+            REQUIRE(cpu_ms() - c1 <= 3 * (c1 - c0) + 150);
+        }
+    return 0;
+}
+
 int main(int, char **argv)
 {
     const std::string what = argv[1];
@@ -352,6 +380,8 @@ int main(int, char **argv)
         return block_of_another_device();
     if (what == "memory_while_another_waits")
         return memory_while_another_waits();
+    if (what == "waiting_is_cheap")
+        return waiting_is_cheap();
     fprintf(stderr, "no scenario %s\n", argv[1]);
     return 2;
 }
