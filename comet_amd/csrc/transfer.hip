@@ -15,6 +15,7 @@
 #include <condition_variable>
 #include <functional>
 #include <mutex>
+#include <system_error>
 #include <thread>
 
 #include "common.h"
@@ -71,7 +72,7 @@ struct Crew {
     const std::function<void()> *job = nullptr;
     char *pinned = nullptr;
     hipEvent_t moved[SLOTS];          // the last group in the slot is across
-    bool threads = false;
+    int threads = 0;                  // how many have been made
 
     int prepare()
     {
@@ -93,9 +94,8 @@ struct Crew {
         (void)hipHostFree(pinned);
         pinned = nullptr;
     }
-    void loop()
+    void loop(uint64_t seen)
     {
-        uint64_t seen = 0;
         int current = -1;
         for (;;) {
             const std::function<void()> *mine;
@@ -123,13 +123,13 @@ struct Crew {
         if (!alone) {
             std::lock_guard<std::mutex> lk(mu);
             (void)hipGetDevice(&device);
-            if (!threads) {
-                for (int h = 1; h < WORKERS; ++h)
-                    std::thread([this] { loop(); }).detach();
-                threads = true;
+            try {
+                for (const uint64_t now = generation; threads < WORKERS - 1; ++threads)
+                    std::thread([this, now] { loop(now); }).detach();
+            } catch (const std::system_error &) {          // there are no more to be had: with those there are
             }
             job = &work;
-            running = WORKERS - 1;
+            running = threads;
             ++generation;
             start.notify_all();
         }

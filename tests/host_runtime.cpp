@@ -2,7 +2,10 @@
 // memory that is counted, streams and events that know their device, and one kernel, the one that moves a group of a
 // transfer.  Its functions take the place of the real ones because the program that is asked for a symbol first is the
 // executable.  Each scenario of main() prints what went wrong and returns non-zero.
+#include <dlfcn.h>
+#include <errno.h>
 #include <hip/hip_runtime_api.h>
+#include <pthread.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -58,8 +61,17 @@ bool on_device(const char *p, size_t bytes, int device)
 
 }  // namespace
 
+static int threads_left = 1 << 20;          // how many more the system has
+
 extern "C" {
 
+int pthread_create(pthread_t *t, const pthread_attr_t *a, void *(*f)(void *), void *arg)
+{
+    static const auto real = (int (*)(pthread_t *, const pthread_attr_t *, void *(*)(void *), void *))dlsym(RTLD_NEXT, "pthread_create");
+    if (threads_left-- <= 0)
+        return EAGAIN;
+    return real(t, a, f, arg);
+}
 void **__hipRegisterFatBinary(const void *) { static void *h; return &h; }
 void __hipUnregisterFatBinary(void **) {}
 void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *, void *, void *, void *, int *)
@@ -367,6 +379,18 @@ static int waiting_is_cheap()
     return 0;
 }
 
+// a process that may have no more threads still copies
+static int few_threads(int n)
+{
+    REQUIRE(comet_hip_init(0) == 0);
+    threads_left = n;
+    for (int i = 0; i < 3; ++i)
+        REQUIRE(there_and_back(30 << 20, 8) == 0);
+    threads_left = 1 << 20;
+    REQUIRE(there_and_back(30 << 20, 8) == 0);
+    return 0;
+}
+
 int main(int, char **argv)
 {
     const std::string what = argv[1];
@@ -382,6 +406,10 @@ int main(int, char **argv)
         return memory_while_another_waits();
     if (what == "waiting_is_cheap")
         return waiting_is_cheap();
+    if (what == "no_threads")
+        return few_threads(0);
+    if (what == "two_threads")
+        return few_threads(2);
     fprintf(stderr, "no scenario %s\n", argv[1]);
     return 2;
 }
