@@ -352,11 +352,9 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
     const int64_t sa = g.k.s0[last], sb = g.k.s1[last];          // strides of the innermost k
     constexpr int NA = RUN || (A_M && !REG) ? 1 : EA, NB = RUN || (B_N && !REG) ? 1 : EB;
     uint32_t ao[NA], bo[NB];
-    if constexpr (RUN) {           // a run beyond the last row (their number is a multiple of EA then) is the last one
-        const int ar = A_M && m0 + a_r >= g.M ? (int)(g.M - EA - m0) : a_r;
-        const int bc = B_N && n0 + b_c >= g.N ? (int)(g.N - EB - n0) : b_c;
-        ao[0] = (ar >= 0 ? rowA[ar] : rowA[0] - (uint32_t)(-ar * 8)) + (uint32_t)(a_k * sa * 8);
-        bo[0] = (bc >= 0 ? colB[bc] : colB[0] - (uint32_t)(-bc * 8)) + (uint32_t)(b_k * sb * 8);
+    if constexpr (RUN) {           // a run beyond the last row is the last one (their number is a multiple of EA then)
+        ao[0] = rowA[A_M && m0 + a_r >= g.M ? g.M - EA - m0 : a_r] + (uint32_t)(a_k * sa * 8);
+        bo[0] = colB[B_N && n0 + b_c >= g.N ? g.N - EB - n0 : b_c] + (uint32_t)(b_k * sb * 8);
     } else {
 #pragma unroll
         for (int e = 0; e < NA; ++e)
