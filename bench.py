@@ -338,10 +338,11 @@ def bench_ttgt(rt, orc, gen, args):
         rt._check(rt.lib().comet_hip_mfma_f64_peak(20000, C.byref(peak)), "comet_hip_mfma_f64_peak")
     perm_bytes = 2 * 8 * e ** 4        # both operands are contiguous along k in different dimensions: one is turned
     return {
-        "metric": "TTGT contraction TFLOP/s (fp64 MFMA GEMM + LDS-tiled transposes) on 1 MI355X",
+        "metric": "TTGT contraction TFLOP/s (fp64 MFMA on the tensors' own strides, one operand turned) on 1 MI355X",
         "value": flops / (dev_ms * 1e-3) / 1e12, "unit": "TFLOP/s", "ms_per_step": dev_ms, "dtype": "f64",
         "config": {"workload": "ttgt_aebf_dfce_abcd", "extent": e, "gemm": [M, N, K], "candidate": plan.candidate,
-                   "transposes": {"A": plan.transA, "B": plan.transB, "C": plan.transC}, "beta": 0.0},
+                   "plan_transposes": {"A": plan.transA, "B": plan.transB, "C": plan.transC},
+                   "turned_operands": int(any(k.startswith("transpose") for k in kt)), "beta": 0.0},
         "roofline": {"bound": "mfma", "achieved": flops / (dom_ms * 1e-3) / 1e12, "peak": FP64_MFMA_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": flops / (dom_ms * 1e-3) / 1e12 / FP64_MFMA_PEAK_TFLOPS, "traffic": None,
                      "kernel": dom, "kernel_avg_ms": dom_ms, "transpose_bytes": int(perm_bytes),

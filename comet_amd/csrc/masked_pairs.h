@@ -478,7 +478,7 @@ __device__ __forceinline__ PairItem pair_item_read(const PairItem &l)
 // The rows of long tables: a workgroup per part of a row, the table's row as a bitmap of nwords words in LDS.  The
 // pairs of the part are dealt to the wavefronts in batches - as they come when hits are counted, in a fixed order
 // when weights are added, so that the sum does not depend on scheduling.
-// Bound by the lists' way from the memory-side cache (10.1 GB a call on the scale-20 graph, 6.8 TB/s) and, at two thirds
+// Bound by the lists' way from the memory-side cache (8.7 GB a call on the scale-20 graph, 5.6 TB/s) and, at two thirds
 // of the LDS cycles, by the look-ups' bank conflicts; registers for two wavefronts' workgroups a CU keep both busy.
 // Whole call, triangle counts: n = 2^20 4.8 -> 1.7 ms, 200003 1.1 -> 0.38, 20351 2.0 -> 0.13, 1000 0.22 -> 0.04.
 struct PairHeavyShared {                 // in LDS behind the bitmap

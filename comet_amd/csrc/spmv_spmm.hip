@@ -2162,8 +2162,12 @@ __global__ __launch_bounds__(SDDMM_W * 64) void sddmm_kernel(int64_t nnz, const 
 // (500000 rows of 16 entries, nine tenths of them in rows of 128 and more,
 // K = 15: 301 -> 215 us; K = 64 681 -> 616.  What is left is the vector memory
 // path's: its return side is busy nine tenths of the time.)
+// The sizes are what fits an L2 at K = 64.  They are kept for every K: wider rows are taken 64 columns at a time, and a
+// slice that only half fits still saves most of its trips.  Kernel as stored / in order, us: 200000 rows, 3.7 M entries,
+// K = 24 129 / 108, 48 209 / 222, 64 266 / 245, 128 525 / 442, 256 1058 / 900; 1000000 rows, 15 M entries, K = 24
+// 557 / 517, 48 982 / 967, 64 1233 / 1037, 128 2508 / 1824, 256 5177 / 3602; 60000 rows of 52, K = 48 168 / 170, 256 835 / 704.
 // ---------------------------------------------------------------------------
-constexpr int64_t SDDMM_SLICE = 4608;               // columns of a block: 2.25 MiB of D at K = 64
+constexpr int64_t SDDMM_SLICE = 4608;               // columns of a block, at least: 2.25 MiB of D at K = 64
 constexpr int SDDMM_BLOCKS_MOST = 4096;
 constexpr int64_t SDDMM_LONG_ROWS = 4096;           // long rows at most: 2 MiB of C at K = 64
 constexpr int64_t SDDMM_ORDER_NNZ = 1 << 19;        // fewer entries are not worth ordering

@@ -357,7 +357,9 @@ int64_t comet_hip_csr_transpose(int64_t csr);
  * count * (a's entry * that number): sums of whole numbers, such as a triangle
  * count, are exact; other values agree with the product-by-product sum to
  * rounding.  Which entry is taken from which side is planned on the first call and
- * kept in a's handle for four (b, mask) at most (8 bytes per entry of a).
+ * kept in a's handle for four (b, mask) at most (8 bytes per entry of a, and a
+ * copy of a's values in the plan's order where they are not all one number, so a
+ * caller that writes into a's arrays calls comet_hip_csr_invalidate here too).
  * COMET_HIP_MASKED_SUM_ONLY=workgroup|wavefront in the environment
  * sends every row through one of the two kernels (a diagnostic: the tests use it). */
 int comet_hip_spgemm_masked_sum(int64_t a, int64_t b, int64_t mask, double *out);
