@@ -263,7 +263,7 @@ static int whole_device()
 {
     const int64_t GiB = 1ll << 30;
     REQUIRE(comet_hip_init(0) == 0);
-    for (int round = 0; round < 2; ++round) {
+    for (int turn = 0; turn < 2; ++turn) {
         const int64_t a = comet_hip_malloc(130 * GiB), b = comet_hip_malloc(130 * GiB), c = comet_hip_malloc(20 * GiB),
                       d = comet_hip_malloc(7 * GiB);
         REQUIRE(a && b && c && d);
