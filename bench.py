@@ -68,13 +68,16 @@ def mem_free(rt):
 def first_call(rt, fn):
     """Wall time of the first call of `fn` (device drained before and after) and the device memory it keeps:
     what a program that multiplies once pays on top of a steady-state step (plans cached in the handle,
-    workspaces)."""
+    workspaces; not freed memory that the library has ready for the next request)."""
     rt.sync()
+    rt.release_memory()
     free0 = mem_free(rt)
     t0 = time.perf_counter()
     fn()
     rt.sync()
-    return (time.perf_counter() - t0) * 1e3, free0 - mem_free(rt)
+    ms = (time.perf_counter() - t0) * 1e3
+    rt.release_memory()
+    return ms, free0 - mem_free(rt)
 
 
 _T0 = time.perf_counter()
