@@ -775,7 +775,8 @@ static int gett_device(const GettIndex &m, const GettIndex &n, const GettIndex &
     // COMET_HIP_GETT_SPAN=elements cuts smaller operands (the pieces make the same result: the tests cut small ones)
     int64_t limit = GETT_SPAN;
     if (const char *e = getenv("COMET_HIP_GETT_SPAN"))
-        limit = std::max<int64_t>(1, std::min<int64_t>(limit, atoll(e)));
+        if (const long long asked = atoll(e); asked > 0 && asked < limit)
+            limit = asked;
     return gett_pieces(m, n, k, limit, M, N, K, A, B, C, beta);
 }
 

@@ -324,30 +324,30 @@ static int memory_while_another_waits()
         if (pending)
             REQUIRE(comet_hip_free(b) == 0);
         int rc = -1;
-        busy(600);
+        busy(1500);
         const auto t0 = Clock::now();
         std::thread waits([&] { rc = comet_hip_memcpy(a, host.data(), 100, 0); });
-        std::this_thread::sleep_for(std::chrono::milliseconds(100));
+        std::this_thread::sleep_for(std::chrono::milliseconds(300));
         const int64_t c = comet_hip_malloc(pending ? 3 << 20 : 1 << 20);
         REQUIRE(c && comet_hip_free(c) == 0);
         const double ms = ms_since(t0);
         waits.join();
-        REQUIRE(rc == 0 && ms_since(t0) >= 590);
-        REQUIRE(ms < 400);
+        REQUIRE(rc == 0 && ms_since(t0) >= 1490);
+        REQUIRE(ms < 1200);
     }
     // what was freed while that thread waited is not free to hand out: the work launched before may use it
     busy(0);
     const int64_t d = comet_hip_malloc(70000);
     REQUIRE(d);
-    busy(300);
+    busy(900);
     std::thread waits([&] { (void)comet_hip_memcpy(a, host.data(), 100, 0); });
-    std::this_thread::sleep_for(std::chrono::milliseconds(100));
-    busy(600);                                      // launched after that wait began
+    std::this_thread::sleep_for(std::chrono::milliseconds(300));
+    busy(2000);                                     // launched after that wait began
     REQUIRE(comet_hip_free(d) == 0);
     waits.join();
     const auto t0 = Clock::now();
     const int64_t e = comet_hip_malloc(70000);
-    REQUIRE(e && (e != d || ms_since(t0) > 100));
+    REQUIRE(e && (e != d || ms_since(t0) > 300));
     return 0;
 }
 
