@@ -189,7 +189,8 @@ struct Csr {
     // products taken with this matrix on the left so far (0, 1, more): the SpMM and SpMV plans, which cost tens of
     // products, are built when a matrix is multiplied for the second time (plan_at_once() builds them at the first)
     int spmm_uses = 0, spmv_uses = 0, sddmm_uses = 0;
-    // SDDMM: the stored entries in an order that keeps columns of D in an L2, XCD x's from sddmm_start[x] on
+    // SDDMM: the stored entries in an order that keeps columns of D in an L2, XCD x's from sddmm_start[x] on: their
+    // places, then their rows, then their columns
     // (sddmm_state: 0 not looked at, 1 not worth it, 2 made)
     int sddmm_state = 0;
     int32_t *sddmm_order = nullptr;

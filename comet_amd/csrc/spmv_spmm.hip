@@ -2045,38 +2045,52 @@ extern "C" int comet_hip_densemat_csr_f64(int64_t csr, int64_t M, int64_t a_dptr
 // (lib/Dialect/IndexTree/Transforms/KernelFusion.cpp:1049-1220; the test is
 // test/integration/kernels/sddmm.ta).  Either way a stored entry (i, j) gets
 // val * sum_k C[i,k] * D[k,j], the sum unfused and in ascending k.
-// A wavefront takes E stored entries at a time, 64 columns of C and D at a time:
-// a lane owns two of them, so that a group of kt / 2 lanes loads a row of C and a
-// (transposed) row of D, 16 bytes a lane, and there are as many groups as fit;
-// the products go to LDS, and lane e adds those of entry e in ascending k.  E is
-// what the products of 8 KiB allow.  D is transposed first, so that its "row"
-// for a column j is contiguous; the row of every entry comes from a list kept in
-// B's handle (searching pos per entry cost 80 % of the time).
-// Bound by the gathers of D, where it is larger than an L2 by their way there.
-// (A lane per column and 16 entries took 313 us for 250000 rows of 16 entries
-// and K = 9, this 95; 628 and 150 for 500000 rows and K = 3, 94 and 77 for 60001
-// and K = 64.)
+// A wavefront takes 64 stored entries, KT = 16 columns of C and of the transposed D at a time: a group of eight lanes has
+// eight entries next to each other, and loads 128 bytes of each one's row of D, 16 a lane - the row of C only where it
+// is not that of the entry before, and entries of one row lie together.  The products go to LDS, and lane e adds those
+// of entry e in ascending k while the next 16 columns are on their way.  (Sixteen entries and 64 columns at a time read C
+// for every entry and left three quarters of the lanes idle in the sums: whole call, 250000 rows of 16 entries, K = 64
+// 301 -> 227 us, K = 48 217 -> 140, K = 33 213 -> 170; 500000 rows, K = 15 217 -> 199, K = 3 150 -> 137.)  Bound by the
+// way of D's rows from the L2s: 16 of the 18.6 M lines that the CUs ask for at K = 64, 80 of them under way a CU, a third
+// of them beyond the L2.  D is transposed first, so that its "row" for a
+// column j is contiguous; the row of every entry comes from a list kept in B's handle (searching pos per entry cost
+// 80 % of the time).
 // ============================================================================
 constexpr int SDDMM_W = 4;               // wavefronts per workgroup
-constexpr int SDDMM_TILE = 1152;         // products of a wavefront in LDS: 64 entries of 16 columns and 2 doubles' padding
 
-// E: entries of a wavefront; KT: most columns of a row that are products at a time; ROUNDS: loads of C and of D under way
-// per lane
-// order (or null: as stored): the entries' order, XCD x's from start.v[x] on
+// order (or null: as stored): the places of the entries in B, XCD x's from start.v[x] on; rows, cols: theirs, in that order
+// SMALL: an address is a 24-bit multiply and an add
 struct SddmmStart { int64_t v[9]; };
-template <int E, int KT, int ROUNDS, bool SMALL>
-__global__ __launch_bounds__(SDDMM_W * 64) void sddmm_kernel(int64_t nnz, const int32_t *__restrict__ order,
-                                                             SddmmStart start, const int32_t *__restrict__ entry_row,
-                                                             const int32_t *__restrict__ crd,
+template <bool SMALL>
+struct SddmmAt {
+    using Off = std::conditional_t<SMALL, uint32_t, int64_t>;
+    __device__ static Off row(int r, int64_t ld, int64_t col)
+    {
+        if constexpr (SMALL)
+            return __umul24((unsigned)r, (unsigned)ld * 8u) + (unsigned)col * 8u;
+        else
+            return ((int64_t)r * ld + col) * 8;
+    }
+    __device__ static const double *at(const double *base, Off o)
+    {
+        return reinterpret_cast<const double *>(reinterpret_cast<const char *>(base) + o);
+    }
+};
+// KT: columns of a row that are products at a time; R: entries of KT / 2 lanes
+template <bool SMALL, int KT, int R>
+__global__ __launch_bounds__(SDDMM_W * 64, 4) void sddmm_kernel(int64_t nnz, const int32_t *__restrict__ order,
+                                                             SddmmStart start, const int32_t *__restrict__ rows,
+                                                             const int32_t *__restrict__ cols,
                                                              const double *__restrict__ val,
                                                              const double *__restrict__ C, int64_t ldc,
-                                                             const double *__restrict__ Dt, int64_t K,
+                                                             const double *__restrict__ Dt, int64_t ldt, int64_t K,
                                                              double *__restrict__ out)
 {
-    // a row of products: 16-byte accesses of consecutive lanes, one row apart, fall into different banks
+    using At = SddmmAt<SMALL>;
+    constexpr int LANES = KT / 2, E = 64 / LANES * R;
+    // a row of products in LDS: 16-byte accesses of consecutive lanes, one row apart, fall into different banks
     constexpr int LD = KT + 2;
-    static_assert(E * LD <= SDDMM_TILE, "the products fit");
-    __shared__ __align__(16) double tiles[SDDMM_W][SDDMM_TILE];
+    __shared__ __align__(16) double tiles[SDDMM_W][E * LD];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     double *tile = tiles[wave];
@@ -2085,68 +2099,103 @@ __global__ __launch_bounds__(SDDMM_W * 64) void sddmm_kernel(int64_t nnz, const 
     if (base >= end)
         return;
     const int cnt = (int)(end - base < E ? end - base : E);
-    int64_t p = base + (lane < cnt ? lane : cnt - 1);        // lane e < cnt owns entry base + e
-    if (order)
-        p = order[p];
-    const int my_col = crd[p], my_row = entry_row[p];
+    // lane e owns entry base + e; behind the last one, that one again
+    const int64_t at = base + (lane < cnt ? lane : cnt - 1);
+    const int my_col = cols[at], my_row = rows[at];
+    const int64_t p = order ? order[at] : at;
     const double v = val[p];
+    const int prev = __shfl_up(my_row, 1, 64);
+    const unsigned long long again = __ballot(lane > 0 && my_row == prev);      // entries in the row of the one before
     double t = 0.0;
-    for (int64_t kc = 0; kc < K; kc += KT) {
-        const int kn = (int)(K - kc < KT ? K - kc : KT);
-        const int L = (kn + 1) / 2, G = 64 / L, rounds = (cnt + G - 1) / G;
+    const auto sum = [&](int n) {
+        const double2 *mine = reinterpret_cast<const double2 *>(tile + (lane & (E - 1)) * LD);
+        int q = 0;
+#pragma unroll 8
+        for (; q < n / 2; ++q) {
+            const double2 w = mine[q];
+            t = t + w.x;
+            t = t + w.y;
+        }
+        if (n & 1)
+            t = t + mine[q].x;
+    };
+    int64_t kc = 0;
+    if (K >= KT) {
+        const int g = lane / LANES, sub = lane % LANES;
+        const unsigned kept = (unsigned)(again >> (R * g)) & ~1u;      // bit u: the row of C is there already
+        typename At::Off co[R], dO[R];
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            co[u] = At::row(__shfl(my_row, R * g + u, 64), ldc, 2 * sub);
+            dO[u] = At::row(__shfl(my_col, R * g + u, 64), ldt, 2 * sub);
+        }
+        spmm_pair c[R], d[R];
+        const auto load = [&](int64_t k) {
+            const double *Ck = C + k, *Dk = Dt + k;
+#pragma unroll
+            for (int u = 0; u < R; ++u) {
+                if (!(kept >> u & 1u))
+                    c[u] = *reinterpret_cast<const spmm_pair *>(At::at(Ck, co[u]));
+                d[u] = *reinterpret_cast<const spmm_pair *>(At::at(Dk, dO[u]));
+            }
+        };
+        load(0);
+        for (; kc + KT <= K; kc += KT) {
+            spmm_pair cur = c[0];
+#pragma unroll
+            for (int u = 0; u < R; ++u) {
+                cur.x = kept >> u & 1u ? cur.x : c[u].x;
+                cur.y = kept >> u & 1u ? cur.y : c[u].y;
+                *reinterpret_cast<double2 *>(tile + (R * g + u) * LD + 2 * sub) =
+                    make_double2(cur.x * d[u].x, cur.y * d[u].y);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+            if (kc + 2 * KT <= K)
+                load(kc + KT);
+            sum(KT);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        }
+    }
+    if (kc < K) {                        // fewer than 16 columns: as many lanes to an entry as they take, two columns a lane
+        const int kn = (int)(K - kc), L = (kn + 1) / 2, G = 64 / L, rounds = (E + G - 1) / G;
         const int g = lane / L, sub = lane - g * L;
         // the last lane of an odd kn has one column, and reads the one before it as well, if there is one
         const bool half = sub == L - 1 && (kn & 1);
         const int64_t from = kc + 2 * sub - (half && kc + 2 * sub > 0 ? 1 : 0);
-        for (int r0 = 0; r0 < rounds; r0 += ROUNDS) {
-            spmm_pair c[ROUNDS], d[ROUNDS];
+        const int e0 = g * rounds;
+        const unsigned kept = (unsigned)(again >> (e0 & 63)) & ~1u;
+        spmm_pair c[R], d[R];
 #pragma unroll
-            for (int u = 0; u < ROUNDS; ++u) {
-                const int e = (r0 + u) * G + g < cnt ? (r0 + u) * G + g : cnt - 1;
+        for (int u = 0; u < R; ++u) {
+            if (u < rounds) {
+                const int e = e0 + u < E ? e0 + u : E - 1;
                 const int r = __shfl(my_row, e, 64), j = __shfl(my_col, e, 64);
-                const double *cp, *dp;
-                if constexpr (SMALL) {
-                    cp = reinterpret_cast<const double *>(reinterpret_cast<const char *>(C) +
-                                                          (__umul24((unsigned)r, (unsigned)ldc * 8u) + (unsigned)from * 8u));
-                    dp = reinterpret_cast<const double *>(reinterpret_cast<const char *>(Dt) +
-                                                          (__umul24((unsigned)j, (unsigned)K * 8u) + (unsigned)from * 8u));
-                } else {
-                    cp = C + (int64_t)r * ldc + from;
-                    dp = Dt + (int64_t)j * K + from;
-                }
+                const double *cp = At::at(C, At::row(r, ldc, from)), *dp = At::at(Dt, At::row(j, ldt, from));
                 if (K > 1) {
-                    c[u] = *reinterpret_cast<const spmm_pair *>(cp);
+                    if (!(kept >> u & 1u))
+                        c[u] = *reinterpret_cast<const spmm_pair *>(cp);
                     d[u] = *reinterpret_cast<const spmm_pair *>(dp);
                 } else {
                     c[u].x = c[u].y = *cp;
                     d[u].x = d[u].y = *dp;
                 }
             }
+        }
+        spmm_pair cur = c[0];
 #pragma unroll
-            for (int u = 0; u < ROUNDS; ++u) {
-                const int e = (r0 + u) * G + g;
-                if (g < G && e < cnt) {
-                    double2 q = make_double2(c[u].x * d[u].x, c[u].y * d[u].y);
-                    if (half)
-                        q.x = q.y;
-                    *reinterpret_cast<double2 *>(tile + e * LD + 2 * sub) = q;
-                }
+        for (int u = 0; u < R; ++u) {
+            const int e = e0 + u;
+            if (u < rounds && g < G && e < E) {
+                cur.x = K > 1 && (kept >> u & 1u) ? cur.x : c[u].x;
+                cur.y = K > 1 && (kept >> u & 1u) ? cur.y : c[u].y;
+                double2 q = make_double2(cur.x * d[u].x, cur.y * d[u].y);
+                if (half)
+                    q.x = q.y;
+                *reinterpret_cast<double2 *>(tile + e * LD + 2 * sub) = q;
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-        if (lane < cnt) {
-            const double2 *mine = reinterpret_cast<const double2 *>(tile + lane * LD);
-            int q = 0;
-#pragma unroll 8
-            for (; q < kn / 2; ++q) {
-                const double2 w = mine[q];
-                t = t + w.x;
-                t = t + w.y;
-            }
-            if (kn & 1)
-                t = t + mine[q].x;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        sum(kn);
     }
     if (lane < cnt)
         out[p] = v * t;
@@ -2159,13 +2208,10 @@ __global__ __launch_bounds__(SDDMM_W * 64) void sddmm_kernel(int64_t nnz, const 
 // the rows of C they need are few: those entries are taken by blocks of columns,
 // every block by one XCD (the blocks dealt so that the XCDs have equal shares),
 // and within a block as stored.  The other entries go behind them as stored.
-// (500000 rows of 16 entries, nine tenths of them in rows of 128 and more,
-// K = 15: 301 -> 215 us; K = 64 681 -> 616.  What is left is the vector memory
-// path's: its return side is busy nine tenths of the time.)
 // The sizes are what fits an L2 at K = 64.  They are kept for every K: wider rows are taken 64 columns at a time, and a
-// slice that only half fits still saves most of its trips.  Kernel as stored / in order, us: 200000 rows, 3.7 M entries,
-// K = 24 129 / 108, 48 209 / 222, 64 266 / 245, 128 525 / 442, 256 1058 / 900; 1000000 rows, 15 M entries, K = 24
-// 557 / 517, 48 982 / 967, 64 1233 / 1037, 128 2508 / 1824, 256 5177 / 3602; 60000 rows of 52, K = 48 168 / 170, 256 835 / 704.
+// slice that only half fits still saves most of its trips.  Whole call as stored / in order, us: 200000 rows, 3.7 M
+// entries, K = 3 51 / 51, 9 91 / 65, 24 135 / 89, 48 204 / 140, 64 271 / 178, 128 533 / 361, 256 1077 / 831; 1000000 rows,
+// 15 M entries, K = 3 340 / 287, 24 719 / 572, 48 1039 / 817, 64 1383 / 1068, 128 2929 / 2137.
 // ---------------------------------------------------------------------------
 constexpr int64_t SDDMM_SLICE = 4608;               // columns of a block, at least: 2.25 MiB of D at K = 64
 constexpr int SDDMM_BLOCKS_MOST = 4096;
@@ -2244,6 +2290,19 @@ __global__ __launch_bounds__(256) void sddmm_keys(int64_t nnz, const int32_t *__
     }
     keys[p] = (uint64_t)key;
     idx[p] = (uint32_t)p;
+}
+
+// the entries' rows and columns in the order of their places
+__global__ __launch_bounds__(256) void sddmm_gather(int64_t nnz, const int32_t *__restrict__ order,
+                                                    const int32_t *__restrict__ entry_row, const int32_t *__restrict__ crd,
+                                                    int32_t *__restrict__ rows, int32_t *__restrict__ cols)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nnz)
+        return;
+    const int p = order[i];
+    rows[i] = entry_row[p];
+    cols[i] = crd[p];
 }
 
 // start[x] = first entry whose key is limit[x] or more
@@ -2343,7 +2402,7 @@ static int sddmm_order(Csr *b, const int32_t *rows)
     const size_t n = (size_t)b->nnz;
     int rc = COMET_HIP_OK;
     if (dev_malloc((void **)&keys, 16 * n) != hipSuccess || dev_malloc((void **)&idx, 4 * n) != hipSuccess ||
-        dev_malloc((void **)&order, 4 * n) != hipSuccess ||
+        dev_malloc((void **)&order, 12 * n) != hipSuccess ||
         dev_malloc((void **)&d_where, sizeof(int32_t) * where.size()) != hipSuccess) {
         (void)hipGetLastError();          // without the room the entries are taken as stored
         (void)dev_free(order);
@@ -2355,6 +2414,8 @@ static int sddmm_order(Csr *b, const int32_t *rows)
             sddmm_keys<<<dim3((unsigned)ceil_div(b->nnz, 256)), dim3(256), 0, stream()>>>(
                 b->nnz, rows, b->crd, b->pos, min_len, slice, d_first, d_where, shorts, keys, idx);
             COMET_CHK(sort_pairs_u64_u32(keys, keys + n, idx, order, b->nnz, end_bit));
+            sddmm_gather<<<dim3((unsigned)ceil_div(b->nnz, 256)), dim3(256), 0, stream()>>>(
+                b->nnz, (const int32_t *)order, rows, b->crd, (int32_t *)order + n, (int32_t *)order + 2 * n);
             sddmm_starts<<<dim3(1), dim3(64), 0, stream()>>>(b->nnz, keys + n, limit, d_start);
             COMET_HIPCHK(hipMemcpyAsync(b->sddmm_start, d_start, sizeof b->sddmm_start, hipMemcpyDeviceToHost, stream()));
             return stream_wait();
@@ -2384,9 +2445,14 @@ static int sddmm_values(Csr *b, int64_t K, int64_t c_dptr, int64_t ldc, int64_t 
                          (long long)K, (long long)ldc, (long long)ldd);
     if (b->nnz == 0)
         return COMET_HIP_OK;
+    // Rows of D begin at a line of 128 bytes, 16 columns are one line then, unless that makes them nearly twice as long
+    // (200000 rows, 3.7 M entries, us, packed / so: K = 3 50 / 71, 9 69 / 65, 15 80 / 73, 17 86 / 91, 18 85 / 79, 28 117 /
+    // 105, 50 219 / 179, 61 253 / 197, 100 390 / 317) or D very large.
+    const int64_t whole = ceil_div(K, 16) * 16;
+    const int64_t ldt = K > 0 && whole * 5 <= K * 9 && b->ncols <= (1ll << 32) / 8 / whole ? whole : K;
     if (K > 0) {
-        COMET_CHK(g_sddmm_dt.ensure(sizeof(double) * (size_t)b->ncols * (size_t)K, false));
-        COMET_CHK(transpose2d((const double *)d_dptr, ldd, K, b->ncols, (double *)g_sddmm_dt.ptr, K));
+        COMET_CHK(g_sddmm_dt.ensure(sizeof(double) * (size_t)b->ncols * (size_t)ldt, false));
+        COMET_CHK(transpose2d((const double *)d_dptr, ldd, K, b->ncols, (double *)g_sddmm_dt.ptr, ldt));
     }
     const int32_t *rows = nullptr;
     COMET_CHK(csr_entry_rows(b, &rows));
@@ -2405,20 +2471,29 @@ static int sddmm_values(Csr *b, int64_t K, int64_t c_dptr, int64_t ldc, int64_t 
             start.v[x] = b->sddmm_start[x];
             longest = x > 0 ? std::max(longest, start.v[x] - start.v[x - 1]) : 0;
         }
-        const auto launch = [&](auto kernel, int entries) {
-            const int64_t groups = order ? 8 * ceil_div(longest, SDDMM_W * entries) : ceil_div(b->nnz, SDDMM_W * entries);
-            kernel<<<dim3((unsigned)groups), dim3(SDDMM_W * 64), 0, stream()>>>(
-                b->nnz, order, start, rows, b->crd, b->val, (const double *)c_dptr, ldc, (const double *)g_sddmm_dt.ptr, K, out);
-        };
+        // 64 entries to a wavefront, 32 where there are too few to keep every CU in wavefronts that way (us, 64 / 32: 3.9 M
+        // entries K = 64 228 / 231, 8 M K = 15 198 / 207; 0.64 M K = 33 32.9 / 32.7; 0.32 M K = 50 30.6 / 28.5, K = 10 13.3 / 11.9).
+        // 32 with 32 columns at a time where a row of D comes from beyond the L2s, which give two lines next to each other
+        // quicker than one now and one later (3.7 M entries as stored, 16 / 32 columns: K = 24 135 / 143, 32 142 / 137, 48
+        // 214 / 204, 64 285 / 271, 128 570 / 533, 256 1161 / 1077; in order K = 48 140 / 170, 64 178 / 184).
+        const bool wide = !order && large && K >= 32;
+        const int per_group = SDDMM_W * (wide || b->nnz < SDDMM_ORDER_NNZ ? 32 : 64);
+        const dim3 grid((unsigned)(order ? 8 * ceil_div(longest, per_group) : ceil_div(b->nnz, per_group)));
+        const dim3 block(SDDMM_W * 64);
+        const int32_t *by_row = order ? order + b->nnz : rows, *by_col = order ? order + 2 * b->nnz : b->crd;
+        const double *C = (const double *)c_dptr, *Dt = (const double *)g_sddmm_dt.ptr;
         // rows named in 24 bits, C and D within 4 GiB: an address is a 24-bit multiply and an add
-        const bool small = b->nrows <= 1 << 24 && b->ncols <= 1 << 24 && ldc * 8 < 1 << 24 && K * 8 < 1 << 24 &&
-                           b->nrows * ldc * 8 < (1ll << 32) && b->ncols * K * 8 < (1ll << 32);
-        if (K <= 16)
-            small ? launch(sddmm_kernel<64, 16, 4, true>, 64) : launch(sddmm_kernel<64, 16, 4, false>, 64);
-        else if (K <= 32)
-            small ? launch(sddmm_kernel<32, 32, 8, true>, 32) : launch(sddmm_kernel<32, 32, 8, false>, 32);
+        const bool small = b->nrows <= 1 << 24 && b->ncols <= 1 << 24 && ldc * 8 < 1 << 24 && ldt * 8 < 1 << 24 &&
+                           b->nrows * ldc * 8 < (1ll << 32) && b->ncols * ldt * 8 < (1ll << 32);
+        const auto launch = [&](auto kernel) {
+            kernel<<<grid, block, 0, stream()>>>(b->nnz, order, start, by_row, by_col, b->val, C, ldc, Dt, ldt, K, out);
+        };
+        if (wide)
+            small ? launch(sddmm_kernel<true, 32, 8>) : launch(sddmm_kernel<false, 32, 8>);
+        else if (b->nnz >= SDDMM_ORDER_NNZ)
+            small ? launch(sddmm_kernel<true, 16, 8>) : launch(sddmm_kernel<false, 16, 8>);
         else
-            small ? launch(sddmm_kernel<16, 64, 8, true>, 16) : launch(sddmm_kernel<16, 64, 8, false>, 16);
+            small ? launch(sddmm_kernel<true, 16, 4>) : launch(sddmm_kernel<false, 16, 4>);
     }
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;

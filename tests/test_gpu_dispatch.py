@@ -312,7 +312,25 @@ def test_sddmm_of_every_tile_and_width(nnz, K):
     assert np.array_equal(got[:nnz], orc.sddmm(pos, crd, val, C, D)) and got[nnz] == 7.0
 
 
-@pytest.mark.parametrize("K", [27, 64])
+@pytest.mark.parametrize("K", [1, 2, 15, 16, 17, 33, 47, 64])
+@pytest.mark.parametrize("nnz", [(1 << 19) - 1, 1 << 19, (1 << 19) + 37])
+def test_sddmm_of_many_entries(nnz, K):
+    # the numbers of entries from which on a wavefront takes 64 of them; rows of one entry and rows of thousands
+    rng = np.random.default_rng(nnz + K)
+    n, m = 1500, 2000
+    share = rng.pareto(1.0, n) + 1e-3
+    lens = np.minimum(m, np.floor(share / share.sum() * nnz)).astype(np.int64)
+    lens = lens + np.bincount(np.repeat(np.arange(n), m - lens)[: nnz - lens.sum()], minlength=n)
+    pos = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    crd = np.concatenate([np.sort(rng.permutation(m)[:l]) for l in lens]).astype(np.int32)
+    val, C, D = rng.uniform(-1, 1, nnz), rng.uniform(-1, 1, (n, K)), rng.uniform(-1, 1, (K, m))
+    out = rt.DeviceArray.from_numpy(np.full(nnz + 1, 7.0))
+    rt.sddmm(rt.CsrMatrix.from_arrays((n, m), pos, crd, val), rt.DeviceArray.from_numpy(C), rt.DeviceArray.from_numpy(D), out_values=out)
+    got = out.to_numpy()
+    assert np.array_equal(got[:nnz], orc.sddmm(pos, crd, val, C, D)) and got[nnz] == 7.0
+
+
+@pytest.mark.parametrize("K", [27, 31, 32, 33, 64, 65])
 @pytest.mark.parametrize("hub", [False, True])
 def test_sddmm_in_an_order_that_keeps_columns_close(K, hub):
     # enough entries in long rows, and a D that is too large for an L2: the second call takes them by blocks of columns; with
