@@ -293,13 +293,6 @@ struct QuadTurn {
     uint32_t mask[ROWS];            // which of the four columns are the list's
 };
 
-__device__ __forceinline__ int lane_value(int v, int from) { return __builtin_amdgcn_ds_bpermute(from << 2, v); }
-// orders a wavefront's own LDS accesses for the compiler; the hardware keeps their order
-__device__ __forceinline__ void wave_lds_order()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-}
-
 constexpr int QUAD_MARKS = 32;           // bytes of LDS a wavefront's marks take at most, zero between walks
 
 // A row of 64 quads whose first lies at0 / 4 quads into the whole (at0: the lane's, four columns a quad): the list it

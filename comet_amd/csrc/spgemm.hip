@@ -414,6 +414,13 @@ __device__ __forceinline__ int wave_inclusive_scan(int v)
     v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);    // row_bcast:31 into rows 2 and 3
     return v;
 }
+__device__ __forceinline__ int lane_value(int v, int from) { return __builtin_amdgcn_ds_bpermute(from << 2, v); }
+// orders a wavefront's own LDS accesses for the compiler; the hardware keeps their order
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+}
+
 template <bool LDS_ONLY = false>
 __device__ inline int64_t draw_row(unsigned long long *ticket, int64_t first, int64_t *slot)
 {
@@ -1624,30 +1631,228 @@ __global__ void spgemm_dense_rows(int64_t row_begin, RowList list, int64_t nd, i
     }
 }
 
+// The slices of a row of the product inside a block lie in LDS for all wavefronts: 64 to a batch, the batch's own slices
+// that are not empty in front, and they are streamed end to end.  A batch is cut into quads of four entries wherever its
+// slices end, 64 quads are a turn, and the turns of all batches go to the wavefronts one by one: every wavefront has its
+// share of the row whatever the lengths are, and the loads of two turns (5 KiB a wavefront) are under way while a third
+// goes into LDS.  (A slice at a time to the wavefront that holds its entry of A waited for memory at every slice and for
+// the wavefront with the longest ones at the end.)
+// Bound by the LDS, two thirds of the time busy: 36 clocks for 64 additions of doubles, 14 of them bank conflicts.  A*A of
+// R-MAT graphs, whole product: 65536 vertices, edge factor 16 5.31 -> 4.76 ms (with the walk alone, accumulators beside a
+// bitmap as before, 5.23), 30000 and 10 1.74 -> 1.47; 2^20 and 16 349 -> 329 ms.
+constexpr int DB_LEN_MOST = SG_CB;               // entries of a slice that are staged; more only with repeated columns
+constexpr int DB_END_BITS = 21;
+constexpr int64_t DB_NNZ_MOST = 1ll << 35;       // a place in B and 64 slices fit a word
+struct alignas(16) SliceRec {
+    int64_t where;                   // first entry less 4 x quads before it << 27 | lane that brought it << 21 | end
+    double a;                        // A's value
+};
+struct SliceStage {
+    SliceRec rec[SG_T];
+    int first[SG_T];                 // quads of its batch before a slice
+    uint32_t marks[SG_WAVES][2];     // zero between turns
+    int turns[SG_WAVES];             // of each batch
+};
+constexpr size_t DB_LDS = (size_t)SG_CB * 8 + sizeof(SliceStage);
+static_assert(64 * DB_LEN_MOST < 1 << DB_END_BITS, "the end of a batch's last slice fits");
+static_assert(DB_LDS + 256 <= 160 * 1024, "accumulators and slices fit LDS");
+
+template <typename COL>
+struct SliceTurn {
+    typename SgCol4<COL>::type j;
+    sg_d2u v0, v1;
+    double a;
+    int64_t q;                       // the place in B of the four entries
+    uint32_t mask;                   // which of them are the slice's
+    int pa;                          // the place of a among the row's staged entries
+};
+
+// a lane's slice [lo, hi) of this pass and its entry of A
+__device__ __forceinline__ void slice_put(SliceStage &st, int64_t lo, int64_t hi, double a, int lane, int wave)
+{
+    const int len = hi - lo > DB_LEN_MOST ? DB_LEN_MOST : (int)(hi - lo);
+    const unsigned long long has = __ballot(len > 0);
+    const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(has >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)has, 0));
+    const int slot = wave * 64 + (len > 0 ? below : __popcll(has) + lane - below);
+    const int quads = (len + 3) >> 2, inc = wave_inclusive_scan(quads), pre = inc - quads;
+    SliceRec r;
+    r.where = (lo - 4 * pre) << (DB_END_BITS + 6) | (int64_t)lane << DB_END_BITS | (int64_t)(len + 4 * pre);
+    r.a = a;
+    st.rec[slot] = r;
+    st.first[slot] = len > 0 ? pre : 1 << 30;
+    if (lane == 63)
+        st.turns[wave] = (inc + 63) >> 6;
+}
+
+// four(turn) for this wavefront's turns of the staged slices; returns the number of turns of all wavefronts
+template <typename COL, typename FOUR>
+__device__ __forceinline__ int slice_walk(SliceStage &st, const COL *__restrict__ Bcrd, const double *__restrict__ Bval,
+                                          int64_t nnz, int lane, int wave, FOUR four)
+{
+    typedef typename SgCol4<COL>::type col4;
+    const int own = lane < SG_WAVES ? st.turns[lane] : 0;
+    const int upto = wave_inclusive_scan(own);
+    const int total = __builtin_amdgcn_readlane(upto, 63);
+    uint32_t *marks = st.marks[wave];
+    int batch = -1, pre = 0;
+    const auto issue = [&](SliceTurn<COL> &t, int g) {
+        t.mask = 0;
+        if (g >= total)
+            return;
+        const int b = __builtin_ctzll(__ballot(upto > g));
+        const int base = (g - (__builtin_amdgcn_readlane(upto, b) - __builtin_amdgcn_readlane(own, b))) * 64;
+        if (b != batch) {
+            batch = b;
+            pre = st.first[b * 64 + lane];
+        }
+        // a slice that begins at quad s > base sets bit s - 1 - base: the bits below a quad are the slices up to its own
+        const uint32_t bit = (uint32_t)(pre - 1 - base);
+        if (bit < 64u)
+            atomicOr(&marks[bit >> 5], 1u << (bit & 31u));
+        const int before = __popcll(__ballot(pre <= base)) - 1;
+        wave_lds_order();
+        const uint2 m = *reinterpret_cast<const uint2 *>(marks);
+        wave_lds_order();
+        if (lane < 2)
+            marks[lane] = 0;
+        const int owner = (int)__builtin_amdgcn_mbcnt_hi(m.y, __builtin_amdgcn_mbcnt_lo(m.x, (uint32_t)before));
+        const SliceRec r = st.rec[b * 64 + owner];
+        const int q4 = 4 * (base + lane);
+        const int left = (int)(r.where & ((1 << DB_END_BITS) - 1)) - q4;
+        int64_t q = (r.where >> (DB_END_BITS + 6)) + q4;
+        t.a = r.a;
+        t.pa = b * 64 + ((int)(r.where >> DB_END_BITS) & 63);
+        const int n = left < 0 ? 0 : left < 4 ? left : 4;
+        t.mask = (1u << n) - 1u;
+        if (n == 0)
+            q = 0;
+        if (q > nnz - 4) {               // the last entries of B
+            t.mask <<= (int)(q - (nnz - 4));
+            q = nnz - 4;
+        }
+        t.q = q;
+        t.j = *reinterpret_cast<const col4 *>(Bcrd + q);
+        t.v0 = *reinterpret_cast<const sg_d2u *>(Bval + q);
+        t.v1 = *reinterpret_cast<const sg_d2u *>(Bval + q + 2);
+        wave_lds_order();
+    };
+    SliceTurn<COL> x, y;
+    issue(x, wave);
+    issue(y, wave + SG_WAVES);
+    for (int g = wave; g < total; g += 2 * SG_WAVES) {
+        four(x);
+        issue(x, g + 2 * SG_WAVES);
+        if (g + SG_WAVES < total)
+            four(y);
+        issue(y, g + 3 * SG_WAVES);
+    }
+    return total;
+}
+
+// An accumulator of the block that has received nothing holds a value that no sum and no key can be, and so the block
+// needs no bitmap: -0.0 where products are added (every product is made +0.0 if it is -0.0 first, as an accumulator
+// that starts at +0.0 would have it; a sum of others is never -0.0), 0 where keys are kept (the one NaN whose key is 0
+// takes the next one's).
+__device__ __forceinline__ unsigned long long block_empty(int reduce_op)
+{
+    return reduce_op == SR_PLUS ? 0x8000000000000000ull : 0ull;
+}
+template <bool SEMI>
+__device__ __forceinline__ void block_add(double *slot, double a, double b, int pa, int64_t q, int reduce_op, int mult_op)
+{
+    if constexpr (SEMI) {
+        unsigned long long *key = reinterpret_cast<unsigned long long *>(slot);
+        if (reduce_op == SR_ANY) {
+            semiring_lds_add(slot, reduce_op, mult_op, a, b, pa, q);
+        } else {
+            const double e = semiring_mult(mult_op, a, b);
+            if (reduce_op == SR_PLUS) {
+                __hip_atomic_fetch_add(slot, e + 0.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            } else {
+                const unsigned long long k = reduce_op == SR_MIN ? ~f64_key(e) : f64_key(e);
+                __hip_atomic_fetch_max(key, k ? k : 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+        }
+    } else {
+        __hip_atomic_fetch_add(slot, a * b + 0.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+}
+
+// Writes out what the accumulators of a block hold, in order of the columns, and leaves them empty; place(total) as in
+// dense_emit_block.  A wavefront has 1024 columns to itself: it takes them into registers, and its part of acc becomes
+// the list, half of the columns at a time, from which every lane writes the entry at its own place.
+template <bool SEMI, typename VALUE, typename PLACE>
+__device__ __forceinline__ void block_emit(double *acc, int *wave_tot, int lane, int wave, int col0, int reduce_op,
+                                           int32_t *__restrict__ Ccrd, double *__restrict__ Cval, VALUE value, PLACE place)
+{
+    constexpr int MINE = SG_CB / SG_WAVES, ROWS = MINE / 64, HALF = ROWS / 2;
+    static_assert(MINE / 2 * (8 + 2) <= MINE * 8, "the list of half the columns fits their accumulators");
+    const unsigned long long empty = block_empty(SEMI ? reduce_op : SR_PLUS);
+    unsigned long long *own = reinterpret_cast<unsigned long long *>(acc) + wave * MINE;
+    uint16_t *own_col = reinterpret_cast<uint16_t *>(own + MINE / 2);
+    unsigned long long v[ROWS], held[ROWS];
+    int cnt = 0;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+        v[r] = own[r * 64 + lane];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        held[r] = __ballot(v[r] != empty);
+        cnt += __popcll(held[r]);
+    }
+    if (lane == 0)
+        wave_tot[wave] = cnt;
+    lds_barrier();
+    const int tots = wave_inclusive_scan(lane < SG_WAVES ? wave_tot[lane] : 0);
+    const int total = __builtin_amdgcn_readlane(tots, SG_WAVES - 1);
+    int64_t off = place(total) + (wave ? __builtin_amdgcn_readlane(tots, wave - 1) : 0);
+    const int first = col0 + wave * MINE;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        int n = 0;
+#pragma unroll
+        for (int r = h * HALF; r < (h + 1) * HALF; ++r) {
+            const unsigned long long m = held[r];
+            const int at = n + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+            if (m >> lane & 1ull) {
+                own[at] = v[r];
+                own_col[at] = (uint16_t)(r * 64 + lane);
+            }
+            n += __popcll(m);
+        }
+        wave_lds_order();
+        for (int q = lane; q < n; q += 64) {
+            store_streaming(&Ccrd[off + q], first + (int)own_col[q]);
+            store_streaming(&Cval[off + q], value(own[q]));
+        }
+        wave_lds_order();
+        off += n;
+    }
+    const ulonglong2 none = make_ulonglong2(empty, empty);
+#pragma unroll
+    for (int r = 0; r < ROWS / 2; ++r)
+        reinterpret_cast<ulonglong2 *>(own)[r * 64 + lane] = none;
+}
+
 template <bool SEMI, typename COL>
 __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
     const DenseRow *__restrict__ rows, int64_t nd, const int32_t *__restrict__ Acrd, const double *__restrict__ Aval,
-    const COL *__restrict__ Bcrd, const double *__restrict__ Bval, const int64_t *__restrict__ blkptr, int nblk,
+    const COL *__restrict__ Bcrd, const double *__restrict__ Bval, int64_t Bnnz, const int64_t *__restrict__ blkptr, int nblk,
     unsigned long long *ticket, int32_t *before, int rows_each, int patience, int *gave_up, int32_t *__restrict__ Ccrd,
     double *__restrict__ Cval, int reduce_op, int mult_op)
 {
     __shared__ int64_t row_slot;
     __shared__ int wave_tot[SG_WAVES];
-    __shared__ int block_touched[3];            // see visit_flag
     __shared__ int ahead_slot;                  // the row's entries ahead of the block
     double *acc = reinterpret_cast<double *>(sg_dyn_lds);
-    uint32_t *bm = sg_dyn_lds + SG_CB * 2;
-    emit_t *emit_col = reinterpret_cast<emit_t *>(bm + SG_CB / 32);
+    SliceStage &st = *reinterpret_cast<SliceStage *>(acc + SG_CB);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     for (int j = threadIdx.x; j < SG_CB; j += SG_T)
-        acc[j] = 0.0;
-    if (threadIdx.x < SG_CB / 32)
-        bm[threadIdx.x] = 0;
-    if (threadIdx.x < 3)
-        block_touched[threadIdx.x] = 0;
+        reinterpret_cast<unsigned long long *>(acc)[j] = block_empty(SEMI ? reduce_op : SR_PLUS);
+    if (lane < 2)
+        st.marks[wave][lane] = 0;
     lds_barrier();
-    int visit = 0;
     const int64_t nchunks = (nd + rows_each - 1) / rows_each;
     const int64_t u_end = nchunks * nblk;
     int64_t u = draw_row<true>(ticket, 0, &row_slot);
@@ -1668,7 +1873,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
             a = 0.0;
             if (x < nr) {
                 const int cnt = __builtin_amdgcn_readlane(mine.cnt, x);
-                const int p = wave + lane * SG_WAVES;
+                const int p = (int)threadIdx.x;
                 if (p < cnt) {
                     const int64_t as = ((int64_t)__builtin_amdgcn_readlane((int)(mine.as >> 32), x) << 32) |
                                        (uint32_t)__builtin_amdgcn_readlane((int)mine.as, x);
@@ -1691,6 +1896,8 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
         load_entry(0, k0, a0);
         load_entry(1, k1, a1);
         load_slice(k0, lo0, hi0);
+        slice_put(st, lo0, hi0, a0, lane, wave);
+        lds_barrier();
         for (int x = 0; x < nr; ++x) {
             load_slice(k1, lo1, hi1);
             load_entry(x + 2, k2, a2);
@@ -1699,13 +1906,21 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
                                (uint32_t)__builtin_amdgcn_readlane((int)mine.as, x);
             const int64_t coff = ((int64_t)__builtin_amdgcn_readlane((int)(mine.coff >> 32), x) << 32) |
                                  (uint32_t)__builtin_amdgcn_readlane((int)mine.coff, x);
-            const auto add = [&](int j, double a, double b, int pa, int64_t q) {
-                dense_add<SEMI, COL>(acc, bm, col0, j, a, b, pa, q, reduce_op, mult_op);
+            const int from0 = sizeof(COL) == 4 ? col0 : 0;
+            // the staged slices; what of a slice with repeated columns is not staged is its lane's
+            const auto walk = [&](int pa0, int64_t lo, int64_t hi, double a) {
+                const int turns = slice_walk<COL>(st, Bcrd, Bval, Bnnz, lane, wave, [&](const SliceTurn<COL> &t) {
+                    const int j[4] = {(int)t.j.x, (int)t.j.y, (int)t.j.z, (int)t.j.w};
+                    const double b[4] = {t.v0.x, t.v0.y, t.v1.x, t.v1.y};
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+                        if (t.mask >> x & 1u)
+                            block_add<SEMI>(&acc[j[x] - from0], t.a, b[x], pa0 + t.pa + 1, t.q + x, reduce_op, mult_op);
+                });
+                for (int64_t q = lo + DB_LEN_MOST; q < hi; ++q)
+                    block_add<SEMI>(&acc[(int)Bcrd[q] - from0], a, Bval[q], pa0 + (int)threadIdx.x + 1, q, reduce_op, mult_op);
+                return turns;
             };
-            const auto add4 = [&](auto j, double a, auto v0, auto v1, int pa, int64_t q) {
-                dense_add4<SEMI, COL>(acc, bm, col0, j, a, v0, v1, pa, q, reduce_op, mult_op);
-            };
-            const auto take = [&](int j) { return dense_take<SEMI>(acc, j, reduce_op, mult_op, as, Aval, Bval); };
             // What lies ahead of this block comes from whoever counted the block before it.  That was many tickets
             // ago as a rule, so the answer is asked for before the walk and the trip to memory it takes is over by
             // the time the walk is; only if it was not there yet is it waited for, behind the walk.
@@ -1713,41 +1928,48 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
             int early = 0;
             if (threadIdx.x == 0 && cb > 0)
                 early = __hip_atomic_fetch_max(mark, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const int mine_p = wave + lane * SG_WAVES;          // the entry this lane holds of a batch of SG_T
-            int touched = for_each_in_slices<true>(lo0, hi0, a0, mine_p + 1, lane, Bcrd, Bval, add, add4);
-            if (cnt > SG_T) {
-                // the entries of A beyond the first SG_T, SG_T at a time: a batch's entries are loaded two batches
+            int turns;
+            if (cnt <= SG_T) {
+                turns = walk(0, lo0, hi0, a0);
+                lds_barrier();
+            } else {
+                // the entries of A beyond the first SG_T, SG_T at a time: a pass's entries are loaded two passes
                 // ahead and its slices one, so that a walk does not begin with two trips to memory
                 const auto load_more = [&](int base, int &k, double &a) {
                     k = -1;
                     a = 0.0;
-                    if (base + mine_p < cnt) {
-                        k = Acrd[as + base + mine_p];
-                        a = Aval[as + base + mine_p];
+                    if (base + (int)threadIdx.x < cnt) {
+                        k = Acrd[as + base + threadIdx.x];
+                        a = Aval[as + base + threadIdx.x];
                     }
                 };
-                int kb, kn;
-                double ab, an;
-                int64_t lob, hib;
-                load_more(SG_T, kb, ab);
-                load_more(2 * SG_T, kn, an);
-                load_slice(kb, lob, hib);
-                for (int base = SG_T; base < cnt; base += SG_T) {
+                int kn;
+                double ab = a0, an;
+                int64_t lob = lo0, hib = hi0;
+                load_more(SG_T, kn, an);
+                turns = 0;
+                for (int base = 0; base < cnt; base += SG_T) {
                     int64_t lon, hin;
                     load_slice(kn, lon, hin);
                     int kf;
                     double af;
                     load_more(base + 2 * SG_T, kf, af);
-                    touched |= for_each_in_slices<true>(lob, hib, ab, base + mine_p + 1, lane, Bcrd, Bval, add, add4);
+                    turns += walk(base, lob, hib, ab);
+                    lds_barrier();
                     lob = lon;
                     hib = hin;
                     ab = an;
                     kn = kf;
                     an = af;
+                    if (base + SG_T < cnt) {
+                        slice_put(st, lob, hib, ab, lane, wave);
+                        lds_barrier();
+                    }
                 }
             }
-            const int any = visit_flag(block_touched, visit, touched, lane);
-            visit = visit == 2 ? 0 : visit + 1;
+            // the next row's slices, read behind the barriers of the write-out
+            slice_put(st, lo1, hi1, a1, lane, wave);
+            const int any = turns;          // every wavefront counts the same
             const auto await = [&]() {
                 int ahead = early;
                 for (int polls = 1; ahead < 0 && polls < patience; ++polls) {
@@ -1767,16 +1989,21 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
             if (any) {
                 if (threadIdx.x == 0)
                     ahead_slot = await();          // (read behind the first barrier of the write-out)
-                dense_emit_block<false>(bm, nullptr, acc, emit_col, wave_tot, lane, wave, col0, Ccrd, Cval, take,
-                                        [&](int total) {
-                                            const int ahead = ahead_slot;
-                                            if (threadIdx.x == 0)
-                                                hand_on(ahead + total);
-                                            return coff + ahead;
-                                        });
+                block_emit<SEMI>(acc, wave_tot, lane, wave, col0, reduce_op, Ccrd, Cval,
+                                 [&](unsigned long long v) {
+                                     return SEMI ? semiring_lds_value(v, reduce_op, mult_op, as, Aval, Bval)
+                                                 : __longlong_as_double((long long)v);
+                                 },
+                                 [&](int total) {
+                                     const int ahead = ahead_slot;
+                                     if (threadIdx.x == 0)
+                                         hand_on(ahead + total);
+                                     return coff + ahead;
+                                 });
             } else if (threadIdx.x == 0) {
                 hand_on(await());
             }
+            lds_barrier();
             k0 = k1;
             a0 = a1;
             lo0 = lo1;
@@ -3051,7 +3278,8 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     COMET_HIPCHK(hipGetLastError());
     // the rows of the one-block kernel block by block (COMET_HIP_SPGEMM_ROW_MAJOR keeps them row by row; the
     // tests run both)
-    const bool by_blocks = dense && a->nnz < (1ll << 30) && getenv("COMET_HIP_SPGEMM_ROW_MAJOR") == nullptr;
+    const bool by_blocks = dense && a->nnz < (1ll << 30) && b->nnz >= 4 && b->nnz < DB_NNZ_MOST &&
+                           getenv("COMET_HIP_SPGEMM_ROW_MAJOR") == nullptr;
     bool ran_blocks = false;
     int64_t *word = nullptr;
     COMET_CHK(mailbox((void **)&word));
@@ -3080,9 +3308,9 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
                 rb, list, nd, nblk, a->pos, Cpos, (DenseRow *)g_sg.dense_rows.ptr, (int32_t *)g_sg.dense_before.ptr);
 #define LAUNCH_BLOCKS_C(S, COL, CRD)                                                                       \
     do {                                                                                                   \
-        COMET_CHK(sg_allow_lds(spgemm_numeric_dense_blocks_kernel<S, COL>, SG_DENSE_LDS));                 \
-        spgemm_numeric_dense_blocks_kernel<S, COL><<<cus, block, SG_DENSE_LDS, stream()>>>(                \
-            (const DenseRow *)g_sg.dense_rows.ptr, nd, a->crd, a->val, CRD, b->val, b->sg_blkptr, nblk,    \
+        COMET_CHK(sg_allow_lds(spgemm_numeric_dense_blocks_kernel<S, COL>, DB_LDS));                       \
+        spgemm_numeric_dense_blocks_kernel<S, COL><<<cus, block, DB_LDS, stream()>>>(                      \
+            (const DenseRow *)g_sg.dense_rows.ptr, nd, a->crd, a->val, CRD, b->val, b->nnz, b->sg_blkptr, nblk, \
             sg_ticket(1), (int32_t *)g_sg.dense_before.ptr, rows_each, patience, gave_up, Ccrd, Cval,      \
             reduce_op, mult_op);                                                                           \
     } while (0)

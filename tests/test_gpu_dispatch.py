@@ -375,3 +375,32 @@ def test_spgemm_rows_with_few_products(ncols, semiring, kept, monkeypatch):
             assert np.all(np.abs(v - want[2]) <= 1e-12 * want[2])
         else:
             assert np.array_equal(v, want[2])
+
+
+@pytest.mark.parametrize("semiring", [None, ("min", "plus"), ("max", "times"), ("any", "second"), ("plus", "first")])
+@pytest.mark.parametrize("repeats", [1, 40])
+def test_spgemm_block_by_block_slices(semiring, repeats, monkeypatch):
+    # slices of every length around a quad and a turn, the last entries of B, rows of A around the entries that are staged
+    # at a time; columns stored more than once make slices longer than the block is wide.  Values are whole numbers and
+    # zeros of either sign: sums are exact, and those of nothing but zeros and cancelled ones stay stored.
+    monkeypatch.setenv("COMET_HIP_SPGEMM_WIDE", "0")
+    rng = np.random.default_rng(repeats)
+    m, lens = 16_384 + 700, [0, 1, 2, 3, 4, 5, 7, 8, 63, 64, 65, 255, 256, 257, 259, 1030] * 75
+    if repeats > 1:
+        lens = lens[:48]
+    k = len(lens)
+    bpos = np.concatenate([[0], np.cumsum(np.array(lens) * repeats)]).astype(np.int64)
+    bcrd = np.concatenate([np.repeat(np.sort(rng.choice(m, l, replace=False)), repeats) for l in lens]).astype(np.int64)
+    pick = np.array([-3.0, -1.0, -0.0, 0.0, 1.0, 2.0])
+    bval = rng.choice(pick, len(bcrd))
+    counts = [c for c in (1, 2, 40, 47, 63, 64, 65, 130, 1023, 1024, 1025, 1200) if c <= k] * 3
+    apos = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
+    acrd = np.concatenate([np.sort(rng.choice(k, c, replace=False)) for c in counts])
+    aval = rng.choice(pick, len(acrd))
+    A, B = rt.CsrMatrix.from_arrays((len(counts), k), apos, acrd, aval), rt.CsrMatrix.from_arrays((k, m), bpos, bcrd, bval)
+    want = orc.spgemm(apos, acrd, aval, bpos, bcrd, bval, m, semiring=semiring)
+    for _ in range(2):
+        p, c, v = rt.spgemm(A, B, semiring=semiring).to_arrays()
+        assert np.array_equal(p, want[0]) and np.array_equal(c, want[1]) and np.array_equal(v, want[2])
+        if semiring is None or semiring[0] == "plus":
+            assert not np.any(np.signbit(v[v == 0]))          # an accumulator that starts at zero
