@@ -689,6 +689,7 @@ constexpr int spmm_hrows(int g) { return g * (SPMM_HW - 1) * SPMM_HR; }    // lo
 constexpr int SPMM_MED_MIN_LEN = COMET_SPMM_MED_MIN;   // such a row has at least this many nonzeros
 constexpr int SPMM_MSLOTS = 288;                        // sums a workgroup keeps in LDS: 144 KiB
 constexpr int SPMM_HEAVY_MIN_LEN = COMET_SPMM_HEAVY_MIN;              // a long row has at least this many nonzeros
+constexpr int64_t SPMM_UNEVEN_SWEEP = 24 << 20;         // bytes of B from which on rows of any alignment are swept
 constexpr int SPMM_HCB = 32;                         // column blocks a wavefront's list is cut into
 
 // One workgroup per (XCD x, row group g); workgroup w runs on XCD w % 8.  XCD x
@@ -716,58 +717,72 @@ constexpr int SPMM_HCB = 32;                         // column blocks a wavefron
 // run - runs are padded to even length by the plan, the pad carries no value -
 // and their sums are added once, at the end.
 //
-// A wavefront holds 64 entries of its list at a time, one per lane, and hands
-// them out with readlane; the next 64 are fetched while these are used.  The
+// A wavefront holds 64 entries of its list at a time in LDS, where a half reads
+// its entry with one 16-byte access; the next 64 are fetched while these are
+// used.  (Entries one per lane, handed out by shuffles, and a branch for the pad
+// of every pair took 23 instructions a pair, these 14.)  The
 // gathers go out in batches of 8 pairs (16 rows of B) and the batch is added
-// before the next one is issued: a second batch in flight while the first is
-// added made the sweep slower (0.205 against 0.193 ms for the long rows alone,
-// 0.227 ms when the waits were made exact so that both batches really stayed in
-// flight; batches of 4 or 16 pairs: 0.25 ms) - with sixteen wavefronts per CU
-// the memory path is kept busy by the other wavefronts, and more requests
-// queued per wavefront only lengthen the queues.
+// before the next one is issued: with sixteen wavefronts per CU the memory path
+// is kept busy by the other wavefronts, and more requests queued per wavefront
+// only lengthen the queues (batches of 4 or 16 pairs: 0.25 ms for the long rows
+// alone instead of 0.19).  What bounds it is that path: 29 M lines a product of
+// 500000 rows and K = 64, 60 of them under way a CU, back in 257 clocks on
+// average - 1.5 times as long as where every line comes from the L2.
 // Entry = column - first column of the XCD's range (the low 24 bits, so that the byte offset of the row of B is one
-// 24-bit multiply-add on the entry as it is) | real, first-of-run, kept-in-LDS | owned row << SPMM_E_ROW.  The slot of
+// 24-bit multiply-add on the entry as it is) | real, first-of-run, kept-in-LDS | owned row << SPMM_E_ROW | partner-is-a-pad.  The slot of
 // a row kept in LDS is the entry's second word.
 constexpr int SPMM_HP = 8;       // pairs of entries per batch of gathers
 constexpr int SPMM_E_REAL = 1 << 24;           // not a pad
 constexpr int SPMM_E_FIRST = 1 << 25;          // the entry opens a run of one owned row
 constexpr int SPMM_E_MED = 1 << 26;            // the entry adds into a sum kept in LDS, in the slot its second word names
 constexpr int SPMM_E_ROW = 27;                 // where the owned row sits
+constexpr int SPMM_E_LONE = 1 << (SPMM_E_ROW + SPMM_HRB);          // the odd entry of the pair is a pad
 constexpr unsigned SPMM_E_COLMASK = 0xffffffu;
-static_assert(SPMM_HCOLB <= 24 && SPMM_E_ROW + SPMM_HRB <= 32, "an entry is 32 bits");
+static_assert(SPMM_HCOLB <= 24 && SPMM_E_ROW + SPMM_HRB < 31, "an entry is 32 bits");
 constexpr int SPMM_HWL = SPMM_HW - 1;          // wavefronts of a workgroup that own long rows
 
 // SMALL: B spans less than 4 GiB and has fewer than 2^24 rows of fewer than 2^24 bytes, so the byte offset of a
 // gather is one 24-bit multiply and one add in 32 bits on top of a scalar base, instead of a 64-bit multiply.
+typedef int spmm_v4i __attribute__((ext_vector_type(4)));
+typedef double spmm_v2d __attribute__((ext_vector_type(2)));
+
+// A batch: the entries of SPMM_HP pairs, each half its own, and the rows of B they name.
+struct HeavyBatch {
+    spmm_v4i q[SPMM_HP];
+    spmm_pair b[SPMM_HP];
+};
+
+// ring_half: the wavefront's 64 entries in LDS, from the half's first one on
 template <bool SMALL>
-__device__ inline void heavy_issue(double2 (&b)[SPMM_HP], int ents, int t0, int npairs, int half,
+__device__ inline void heavy_issue(HeavyBatch &x, const spmm_v4i *ring_half, int t0, int npairs,
                                    const double *__restrict__ B, int64_t ldb, int64_t col)
 {
 #pragma unroll
     for (int u = 0; u < SPMM_HP; ++u) {
         const int t = t0 + u < npairs ? t0 + u : npairs - 1;     // past the end: reload the last one, never used
-        const unsigned mine = (unsigned)__shfl(ents, 2 * t + half, 64);       // each half its own entry
+        x.q[u] = ring_half[2 * t];
+    }
+#pragma unroll
+    for (int u = 0; u < SPMM_HP; ++u) {
+        const unsigned mine = (unsigned)x.q[u].x;
         if constexpr (SMALL) {
             const unsigned off = __umul24(mine, (unsigned)ldb * 8u) + (unsigned)col * 8u;
-            b[u] = *reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(B) + off);
+            x.b[u] = *reinterpret_cast<const spmm_pair *>(reinterpret_cast<const char *>(B) + off);
         } else {
             const int64_t j = (int64_t)(mine & SPMM_E_COLMASK);
-            b[u] = *reinterpret_cast<const double2 *>(B + j * ldb + col);
+            x.b[u] = *reinterpret_cast<const spmm_pair *>(B + j * ldb + col);
         }
     }
 }
 
 extern __shared__ double spmm_medium_sums[];
 __device__ inline void heavy_add(double (&accx)[SPMM_HR], double (&accy)[SPMM_HR], double2 &run, int &run_slot,
-                                 const double2 (&b)[SPMM_HP], int ents, int slots,
-                                 double vals, int t0, int npairs, int half, int sub, bool active)
+                                 const HeavyBatch &x, int t0, int npairs, int at, bool active)
 {
 #pragma unroll
     for (int u = 0; u < SPMM_HP; ++u) {
         if (t0 + u < npairs) {
-            const int t = t0 + u;
-            const int e0 = __builtin_amdgcn_readlane(ents, 2 * t);
-            const bool med = (e0 & SPMM_E_MED) != 0;       // both entries of a pair are of the same kind
+            const int e0 = __builtin_amdgcn_readfirstlane(x.q[u].x);
             if (e0 & SPMM_E_FIRST) {             // a run starts on an even entry
                 accx[run_slot] = run.x;
                 accy[run_slot] = run.y;
@@ -775,34 +790,28 @@ __device__ inline void heavy_add(double (&accx)[SPMM_HR], double (&accy)[SPMM_HR
                 run.x = accx[run_slot];
                 run.y = accy[run_slot];
             }
-            const int mine = __shfl(ents, 2 * t + half, 64);
-            const double v = __hiloint2double(__shfl(__double2hiint(vals), 2 * t + half, 64),
-                                              __shfl(__double2loint(vals), 2 * t + half, 64));
-            if (med) {
-                const double px = v * b[u].x, py = v * b[u].y;
-                const int slot = __shfl(slots, 2 * t + half, 64);
+            const double v = __hiloint2double(x.q[u].w, x.q[u].z);
+            if (!(e0 & (SPMM_E_MED | SPMM_E_LONE))) {
+                run.x = __builtin_fma(v, x.b[u].x, run.x);
+                run.y = __builtin_fma(v, x.b[u].y, run.y);
+            } else if (e0 & SPMM_E_MED) {        // both entries of a pair are of the same kind
+                const double px = v * x.b[u].x, py = v * x.b[u].y;
                 // a row of middling length: its sum lives in LDS.  An add that returns nothing is issued and
                 // forgotten; all entries of such a row are in this wavefront's list, in column order, and the adds
                 // of one wavefront to one address are carried out in the order it issued them.
-                if ((mine & SPMM_E_REAL) && active) {
-                    double *sum = spmm_medium_sums + slot * 64 + 2 * sub;
-                    __hip_atomic_fetch_add(sum, px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                if ((x.q[u].x & SPMM_E_REAL) && active) {
+                    double *sum = spmm_medium_sums + x.q[u].y * 64 + at;
+                    if (!(at & 1))                   // (an odd one is the neighbour's second column)
+                        __hip_atomic_fetch_add(sum, px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     __hip_atomic_fetch_add(sum + 1, py, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
-            } else if (mine & SPMM_E_REAL) {     // a pad carries no value
-                // A branch over the lanes of a pad, not a select: two fused multiply-adds instead of two
-                // multiplications, two additions and four selects (a long row's sum is to rounding in any case:
-                // it is added from sixteen partial sums).
-                asm volatile("" ::: "memory");
-                run.x = __builtin_fma(v, b[u].x, run.x);
-                run.y = __builtin_fma(v, b[u].y, run.y);
+            } else if (x.q[u].x & SPMM_E_REAL) {         // a pad carries no value, not even zero times a row of B
+                run.x = __builtin_fma(v, x.b[u].x, run.x);
+                run.y = __builtin_fma(v, x.b[u].y, run.y);
             }
         }
     }
 }
-
-typedef int spmm_v4i __attribute__((ext_vector_type(4)));
-typedef double spmm_v2d __attribute__((ext_vector_type(2)));
 
 // The list of rows with one nonzero: a stream of pairs of entries, one entry per half-wavefront; each is one
 // gather of B and one store to C.  Loads and stores share one in-order counter, so the loop is built to have
@@ -812,7 +821,7 @@ typedef double spmm_v2d __attribute__((ext_vector_type(2)));
 // branched around.  A wait for a batch of gathers then never includes the stores issued behind it.
 // NB = pairs per batch; KB = where the turn's 32 entries start in the ring.
 template <bool SMALL, bool ACC, int NB, int KB>
-__device__ inline void single_issue(double2 (&b)[NB], double2 (&c)[NB], const spmm_v4i *ring_half, int t,
+__device__ inline void single_issue(spmm_pair (&b)[NB], spmm_pair (&c)[NB], const spmm_v4i *ring_half, int t,
                                     const double *__restrict__ B, int64_t ldb, const double *__restrict__ C,
                                     int64_t ldc, int64_t col)
 {
@@ -822,19 +831,19 @@ __device__ inline void single_issue(double2 (&b)[NB], double2 (&c)[NB], const sp
         const unsigned mine = (unsigned)q.x;
         if constexpr (SMALL) {
             const unsigned off = __umul24(mine, (unsigned)ldb * 8u) + (unsigned)col * 8u;
-            b[u] = *reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(B) + off);
+            b[u] = *reinterpret_cast<const spmm_pair *>(reinterpret_cast<const char *>(B) + off);
         } else {
             const int64_t j = (int64_t)(mine & SPMM_E_COLMASK);
-            b[u] = *reinterpret_cast<const double2 *>(B + j * ldb + col);
+            b[u] = *reinterpret_cast<const spmm_pair *>(B + j * ldb + col);
         }
         if constexpr (ACC)
-            c[u] = *reinterpret_cast<const double2 *>(C + (int64_t)q.y * ldc + col);
+            c[u] = *reinterpret_cast<const spmm_pair *>(C + (int64_t)q.y * ldc + col);
     }
     __builtin_amdgcn_sched_barrier(0);       // the gathers stay in front of the stores of the other batch
 }
 
 template <bool ACC, int NB, int KB>
-__device__ inline void single_store(const double2 (&b)[NB], const double2 (&c)[NB], const spmm_v4i *ring_half, int t,
+__device__ inline void single_store(const spmm_pair (&b)[NB], const spmm_pair (&c)[NB], const spmm_v4i *ring_half, int t,
                                     int64_t pair0, int64_t npairs, double *__restrict__ C, int64_t ldc, int64_t col,
                                     bool active, double *__restrict__ dump)
 {
@@ -842,24 +851,54 @@ __device__ inline void single_store(const double2 (&b)[NB], const double2 (&c)[N
     for (int u = 0; u < NB; ++u) {
         const spmm_v4i q = ring_half[(KB + 2 * (t + u)) & 63];
         const double v = __hiloint2double(q.w, q.z);
-        spmm_v2d o;
+        spmm_pair o;
         o.x = (ACC ? c[u].x : 0.0) + v * b[u].x;
         o.y = (ACC ? c[u].y : 0.0) + v * b[u].y;
         const bool ok = pair0 + t + u < npairs && active && (q.x & SPMM_E_REAL);
         double *dst = ok ? C + (int64_t)q.y * ldc + col : dump;
-        __builtin_nontemporal_store(o, reinterpret_cast<spmm_v2d *>(dst));       // C is written once, not read again
+        __builtin_nontemporal_store(o, reinterpret_cast<spmm_pair *>(dst));       // C is written once, not read again
         if (u & 1)
             __builtin_amdgcn_sched_barrier(0);       // two pairs at a time: keeps the entries read ahead few
     }
 }
 
+// Where the wavefronts of a workgroup are in their lists, in steps of 1024 columns: one that is more than `slack` steps
+// ahead of the last one waits for it.  The last one waits for nobody.  Left alone the four wavefronts of a SIMD drift
+// apart - the older one wins every arbitration - and rows of B leave the L2 before the slow ones come to them (500000
+// rows, K = 64: 11 M lines from beyond the L2s instead of 5, 374 us instead of 311).  us by columns that a wavefront may
+// be ahead, 2048 / 3072 / 4096 / 8192: K = 64 311 / 313 / 318 / 341, 48 269 / 269 / 273 / 284, 32 231 / 223 / 225 / 232,
+// 16 215 / 205 / 206 / 211.
+constexpr int SPMM_PACE_LOG = 10;
+struct SweepPace {
+    int *at;                 // of every wavefront, in LDS
+    int slack, wave, mine;
+    __device__ inline void reach(int ent)
+    {
+        const int here = (int)((unsigned)__builtin_amdgcn_readfirstlane(ent) & SPMM_E_COLMASK) >> SPMM_PACE_LOG;
+        if (here == mine)
+            return;
+        mine = here;
+        const int lane = threadIdx.x & 63;
+        if (lane == 0)
+            __hip_atomic_store(&at[wave], here, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const int l = lane & (SPMM_HW - 1);
+        while (__any(__hip_atomic_load(&at[l], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < here - slack))
+            __builtin_amdgcn_s_sleep(1);
+    }
+    __device__ inline void done()
+    {
+        if ((threadIdx.x & 63) == 0)
+            __hip_atomic_store(&at[wave], 1 << 30, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+};
+
 template <bool SMALL, bool ACC>
 __device__ inline void single_rows(const spmm_v4i *__restrict__ list, int64_t n, int lane, int half,
                                    const double *__restrict__ B, int64_t ldb, double *__restrict__ C, int64_t ldc,
-                                   int64_t col, bool active, spmm_v4i *ring, double *__restrict__ dump)
+                                   int64_t col, bool active, spmm_v4i *ring, double *__restrict__ dump, SweepPace &pace)
 {
     constexpr int NB = ACC ? 4 : 8;
-    double2 b0[NB], b1[NB], c0[NB], c1[NB];
+    spmm_pair b0[NB], b1[NB], c0[NB], c1[NB];
     const int64_t npairs = n >> 1;           // the list has an even number of entries
     const int l32 = lane & 31;
     auto fetch = [&](int64_t turn) {         // the 32 entries of a turn, one per lane of each half
@@ -873,6 +912,7 @@ __device__ inline void single_rows(const spmm_v4i *__restrict__ list, int64_t n,
     // a turn = 16 pairs: its entries, and those of the next turn for the gathers issued ahead, are in the ring
     auto turn = [&](auto kb, int64_t k) {
         constexpr int KB = decltype(kb)::value;
+        pace.reach(next.x);
         ring[((KB + 32) & 63) + l32] = next;            // turn k + 1, over the entries of turn k - 1
         next = fetch(k + 2);
         for (int t = 0; t < 16; t += 2 * NB) {
@@ -892,24 +932,33 @@ template <bool SMALL, bool ACC>
 __global__ __launch_bounds__(SPMM_HW * 64) void spmm_heavy_sweep(
     const int64_t *__restrict__ seg, const HeavyEnt *__restrict__ hent, const double *__restrict__ B, int64_t ldb,
     int64_t K, double *__restrict__ partial, double *__restrict__ C, int64_t ldc, int G, int64_t xcols, int nslots,
-    double *__restrict__ partial_medium)
+    double *__restrict__ partial_medium, int slack)
 {
     const int lane = threadIdx.x & 63, half = lane >> 5, sub = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int x = blockIdx.x & 7, g = blockIdx.x >> 3;
     B += (int64_t)x * xcols * ldb;          // the entries count columns from the first one of this XCD's range
-    int64_t col = (int64_t)blockIdx.y * 64 + 2 * sub;          // K is even: a lane's two columns exist or neither
+    // A lane's two columns.  Where K is odd, the last lane has the last two: the first of them is its neighbour's second,
+    // and both lanes add it and store it alike.  Idle lanes gather a valid address and store nothing.
+    int64_t col = (int64_t)blockIdx.y * 64 + 2 * sub;
     const bool active = col < K;
-    if (!active)
-        col = K - 2;            // idle lanes gather a valid address and store nothing
+    if (col > K - 2)
+        col = K - 2;
+    const int at = (int)(col - (int64_t)blockIdx.y * 64);          // in the tile (of an active lane)
     const int64_t bin = ((int64_t)x * G + g) * SPMM_HW + wave;
     const int64_t s = seg[bin], e = seg[bin + 1];          // both even
     const spmm_v4i *list = reinterpret_cast<const spmm_v4i *>(hent);
+    __shared__ spmm_v4i rings[SPMM_HW][64];          // entries of every wavefront's list
+    __shared__ int reached[SPMM_HW];
+    if (lane == 0)
+        reached[wave] = s < e ? 0 : 1 << 30;
+    __syncthreads();
+    SweepPace pace{reached, slack, wave, 0};
     if (wave == SPMM_HWL) {                   // the wavefront of the rows with one nonzero
-        __shared__ spmm_v4i single_ring[64];
         if (s < e)             // this wavefront's slots of `partial` hold no row: the dump
-            single_rows<SMALL, ACC>(list + s, e - s, lane, half, B, ldb, C, ldc, col, active, single_ring,
-                                    partial + bin * SPMM_HR * K + col);
+            single_rows<SMALL, ACC>(list + s, e - s, lane, half, B, ldb, C, ldc, col, active, rings[wave],
+                                    partial + bin * SPMM_HR * K + col, pace);
+        pace.done();
         return;
     }
     double accx[SPMM_HR], accy[SPMM_HR];      // two plain arrays: each is indexed through M0, a double2 array is not
@@ -920,47 +969,49 @@ __global__ __launch_bounds__(SPMM_HW * 64) void spmm_heavy_sweep(
     for (int sl = wave; sl < nslots; sl += SPMM_HWL)
         spmm_medium_sums[sl * 64 + lane] = 0.0;
     if (s < e) {
-        double2 b[SPMM_HP];
+        HeavyBatch x;
         double2 run = make_double2(0.0, 0.0);
         int run_slot = 0;
-        int cnt = (int)(e - s < 64 ? e - s : 64);
-        int c_ent = 0, c_slot = 0;
-        double c_val = 0.0;
-        if (lane < cnt) {
-            const spmm_v4i q = __builtin_nontemporal_load(list + s + lane);
-            c_ent = q.x;
-            c_slot = q.y;
-            c_val = __hiloint2double(q.w, q.z);
-        }
-        heavy_issue<SMALL>(b, c_ent, 0, cnt >> 1, half, B, ldb, col);
-        for (int64_t base = s; base < e; base += 64) {
-            const int64_t left = e - base - 64;
-            const int ncnt = (int)(left < 0 ? 0 : (left < 64 ? left : 64));
-            int n_ent = 0, n_slot = 0;
-            double n_val = 0.0;
-            if (lane < ncnt) {
-                const spmm_v4i q = __builtin_nontemporal_load(list + base + 64 + lane);
-                n_ent = q.x;
-                n_slot = q.y;
-                n_val = __hiloint2double(q.w, q.z);
-            }
-            const int np = cnt >> 1;
-            heavy_add(accx, accy, run, run_slot, b, c_ent, c_slot, c_val, 0, np, half, sub, active);
+        spmm_v4i *ring = rings[wave];
+        const spmm_v4i *ring_half = ring + half;
+        const auto fetch = [&](int64_t at) {         // behind the list's last entry: that one
+            const int64_t i = at + lane;
+            return __builtin_nontemporal_load(list + (i < e ? i : e - 1));
+        };
+        const auto put = [&](spmm_v4i q) {           // the wavefront's own reads of the ring are issued before
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+            ring[lane] = q;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        };
+        put(fetch(s));
+        spmm_v4i next = fetch(s + 64);
+        int64_t base = s;
+        // 32 pairs at a time, the first batch of the next 32 in flight over the loop's back edge
+        heavy_issue<SMALL>(x, ring_half, 0, (int)((e - s < 64 ? e - s : 64) >> 1), B, ldb, col);
+        while (e - base >= 64) {
 #pragma unroll
-            for (int t0 = SPMM_HP; t0 < 32; t0 += SPMM_HP)
-                if (np > t0) {
-                    heavy_issue<SMALL>(b, c_ent, t0, np, half, B, ldb, col);
-                    heavy_add(accx, accy, run, run_slot, b, c_ent, c_slot, c_val, t0, np, half, sub, active);
-                }
-            if (ncnt > 0)         // the first batch of the next 64 entries: in flight over the loop's back edge
-                heavy_issue<SMALL>(b, n_ent, 0, ncnt >> 1, half, B, ldb, col);
-            c_ent = n_ent;
-            c_slot = n_slot;
-            c_val = n_val;
-            cnt = ncnt;
+            for (int t0 = 0; t0 < 32; t0 += SPMM_HP) {
+                heavy_add(accx, accy, run, run_slot, x, 0, SPMM_HP, at, active);
+                if (t0 + SPMM_HP < 32)
+                    heavy_issue<SMALL>(x, ring_half, t0 + SPMM_HP, 32, B, ldb, col);
+            }
+            base += 64;
+            if (base < e) {
+                pace.reach(next.x);
+                put(next);
+                next = fetch(base + 64);
+                heavy_issue<SMALL>(x, ring_half, 0, (int)((e - base < 64 ? e - base : 64) >> 1), B, ldb, col);
+            }
+        }
+        const int np = (int)((e - base) >> 1);
+        for (int t0 = 0; t0 < np; t0 += SPMM_HP) {
+            heavy_add(accx, accy, run, run_slot, x, t0, np, at, active);
+            if (t0 + SPMM_HP < np)
+                heavy_issue<SMALL>(x, ring_half, t0 + SPMM_HP, np, B, ldb, col);
         }
         accx[run_slot] = run.x;
         accy[run_slot] = run.y;
+        pace.done();
     }
     {   // this wavefront's sums in LDS: one partial sum per row and XCD, like the long rows'
         const int64_t c1 = (int64_t)blockIdx.y * 64 + lane;
@@ -1196,8 +1247,11 @@ __global__ void heavy_fill(int64_t n, const uint64_t *__restrict__ keys, const u
         out.row = 0;
         out.val = val[idx[e]];
     }
+    const bool lone = e + 1 == start[r + 1] && ((start[r + 1] - start[r]) & 1);          // last entry of a run of odd length
+    if (lone)
+        out.ent |= SPMM_E_LONE;
     hent[p] = out;
-    if (e + 1 == start[r + 1] && ((start[r + 1] - start[r]) & 1)) {     // last entry of a run of odd length
+    if (lone) {
         out.ent &= ~(SPMM_E_REAL | SPMM_E_FIRST);      // same column (a valid address), no value
         out.val = 0.0;
         hent[p + 1] = out;
@@ -1692,9 +1746,13 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
     if (ceil_div(K, 64) > 65535)
         return set_error(COMET_HIP_ERR_SIZE, "K = %lld needs more than 65535 column tiles", (long long)K);
     // long rows: column sweep with the sums on chip; everything else: one wavefront per 256 nonzeros
-    // (the sweep loads B and stores C sixteen bytes at a time: two columns per lane, rows aligned to that)
-    const bool sweep_fits = K >= 16 && K <= 2048 && (K & 1) == 0 && (ldb & 1) == 0 && (b_dptr & 15) == 0 &&
-                            (ldc & 1) == 0 && (c_dptr & 15) == 0 && getenv("COMET_SPMM_NO_SWEEP") == nullptr;
+    // Rows of B and C that are no multiple of 16 bytes are swept where B is so large that its gathers come from far away
+    // (chunks / sweep, us: K = 33 40000 rows 51 / 65, 60001 69 / 68, 120000 121 / 87, 250000 242 / 153, 500000 477 / 277;
+    // K = 63 40000 71 / 74, 60001 102 / 77, 500000 758 / 358; K = 17 60001 52 / 60, 500000 348 / 230), and where no tile of
+    // columns holds a single one.
+    const bool even = (K & 1) == 0 && (ldb & 1) == 0 && (b_dptr & 15) == 0 && (ldc & 1) == 0 && (c_dptr & 15) == 0;
+    const bool uneven_pays = K % 64 != 1 && a->ncols * ldb * 8 >= SPMM_UNEVEN_SWEEP;
+    const bool sweep_fits = K >= 16 && K <= 2048 && (even || uneven_pays) && getenv("COMET_SPMM_NO_SWEEP") == nullptr;
     // The plan (the long rows as per-XCD lists, the rest re-packed) costs some forty products: a matrix multiplied
     // once goes through the chunk kernel whole, the plan is made when it is multiplied again.
     const bool plan_now = a->spmm_uses > 0 || plan_at_once();
@@ -1732,18 +1790,19 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
         KernelTimer t("spmm_heavy_sweep");
         const bool small_b = a->ncols < (1 << 24) && ldb * 8 < (1 << 24) && a->ncols * ldb * 8 < (1ll << 32);
         const dim3 grid(8 * G, tiles), block(SPMM_HW * 64);
+        const int slack = K >= 48 ? 2 : 3;
         if (small_b && accumulate)
             sweep_launch(spmm_heavy_sweep<true, true>, grid, block, medium_lds, a->heavy_seg, a->heavy_ent, B, ldb, K, partial, C, ldc,
-                         G, ceil_div(a->ncols, 8), nslots, partial_medium);
+                         G, ceil_div(a->ncols, 8), nslots, partial_medium, slack);
         else if (small_b)
             sweep_launch(spmm_heavy_sweep<true, false>, grid, block, medium_lds, a->heavy_seg, a->heavy_ent, B, ldb, K, partial, C, ldc,
-                         G, ceil_div(a->ncols, 8), nslots, partial_medium);
+                         G, ceil_div(a->ncols, 8), nslots, partial_medium, slack);
         else if (accumulate)
             sweep_launch(spmm_heavy_sweep<false, true>, grid, block, medium_lds, a->heavy_seg, a->heavy_ent, B, ldb, K, partial, C, ldc,
-                         G, ceil_div(a->ncols, 8), nslots, partial_medium);
+                         G, ceil_div(a->ncols, 8), nslots, partial_medium, slack);
         else
             sweep_launch(spmm_heavy_sweep<false, false>, grid, block, medium_lds, a->heavy_seg, a->heavy_ent, B, ldb, K, partial, C, ldc,
-                         G, ceil_div(a->ncols, 8), nslots, partial_medium);
+                         G, ceil_div(a->ncols, 8), nslots, partial_medium, slack);
     }
     if (overlap) {      // the rows in between, on the CUs the sweep leaves free
         COMET_CHK(spmm_chunks(a->light, K, B, ldb, C, ldc, accumulate, aux_stream()));

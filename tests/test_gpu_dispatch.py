@@ -404,3 +404,40 @@ def test_spgemm_block_by_block_slices(semiring, repeats, monkeypatch):
         assert np.array_equal(p, want[0]) and np.array_equal(c, want[1]) and np.array_equal(v, want[2])
         if semiring is None or semiring[0] == "plus":
             assert not np.any(np.signbit(v[v == 0]))          # an accumulator that starts at zero
+
+
+@pytest.mark.parametrize("medium", [False, True])
+@pytest.mark.parametrize("K,ldb,ldc,shift,accumulate", [(63, 63, 63, 0, False), (63, 63, 63, 0, True), (17, 53, 40, 0, True),
+                                                        (64, 64, 64, 1, False), (64, 65, 67, 0, True), (99, 99, 100, 1, False)])
+def test_spmm_sweep_of_rows_that_are_no_multiple_of_16_bytes(K, ldb, ldc, shift, accumulate, medium, monkeypatch):
+    # odd widths, odd leading dimensions and addresses 8 bytes off, where B is large enough for the sweep; the last column
+    # is a lane's own and its neighbour's; nothing outside C's columns is written, B's last row is the end of its array
+    if medium:
+        monkeypatch.setenv("COMET_HIP_SPMM_MEDIUM", "1")
+    n = 60_000
+    pos, crd, val = gen.zipf_csr(n=n, mean=16.0, cap=4096, seed=7)
+    crd[-1] = n - 1 if pos[-1] > pos[-2] else crd[-1]
+    assert len(crd) >= 1 << 19 and n * ldb * 8 >= 24 << 20
+    rng = np.random.default_rng(K)
+    B, C0 = rng.uniform(-1, 1, (n, K)), rng.uniform(-1, 1, (n, K))
+    flatB, flatC = np.full(shift + (n - 1) * ldb + K, 5.0), np.full(shift + n * ldc, 7.0)
+    view = lambda flat, ld: np.lib.stride_tricks.as_strided(flat[shift:], (n, K), (8 * ld, 8))
+    view(flatB, ldb)[:] = B
+    view(flatC, ldc)[:] = C0
+    dB, dC = rt.DeviceArray.from_numpy(flatB), rt.DeviceArray.from_numpy(flatC)
+    A = rt.CsrMatrix.from_arrays((n, n), pos, crd, val)
+    rt.profile_reset()
+    rt.profile_enable(True)
+    for _ in range(1 if accumulate else 2):
+        rt._check(rt.lib().comet_hip_spmm_csr_f64(A.handle, K, dB.ptr + 8 * shift, ldb, dC.ptr + 8 * shift, ldc, int(accumulate)), "spmm")
+    rt.sync()
+    assert "spmm_heavy_sweep" in rt.profile_report()
+    rt.profile_enable(False)
+    want = orc.spmm(pos, crd, val, B, C0 if accumulate else None)
+    bound = orc.spmm(pos, crd, np.abs(val), np.abs(B), np.abs(C0) if accumulate else None)
+    out = dC.to_numpy()
+    got = view(out, ldc).copy()
+    assert np.all(np.abs(got - want) <= 1e-12 * bound)
+    assert np.array_equal(got[np.diff(pos) <= 1], want[np.diff(pos) <= 1])
+    view(out, ldc)[:] = 7.0
+    assert np.all(out == 7.0)
