@@ -467,7 +467,26 @@ __device__ __forceinline__ PairItem pair_item_read(const PairItem &l)
     return it;
 }
 
-// tickets[0]: next heavy part, [1]: hits (ONE)
+// The number of hits of a workgroup goes to a place of its own.  (Added by every wavefront to one word, 14 ns each for all
+// XCDs, they took 70 us for the 5120 wavefronts of the short rows alone.)
+__device__ __forceinline__ void pair_block_hits(unsigned long long *wave_hits, unsigned long long hits, int waves,
+                                                unsigned long long *__restrict__ block_hits)
+{
+    for (int d = 32; d > 0; d >>= 1)
+        hits += ((unsigned long long)(unsigned)__shfl_down((int)(hits >> 32), d, 64) << 32) +
+                (unsigned long long)(unsigned)__shfl_down((int)(hits & 0xffffffffu), d, 64);
+    if ((threadIdx.x & 63) == 0)
+        wave_hits[threadIdx.x >> 6] = hits;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long all = 0;
+        for (int w = 0; w < waves; ++w)
+            all += wave_hits[w];
+        block_hits[blockIdx.x] = all;
+    }
+}
+
+// tickets[0]: next heavy part; block_hits: every workgroup's hits (ONE)
 // The rows of long tables: a workgroup per part of a row, the table's row as a bitmap of nwords words in LDS.  The
 // pairs of the part are dealt to the wavefronts in batches - as they come when hits are counted, in a fixed order
 // when weights are added, so that the sum does not depend on scheduling.
@@ -477,12 +496,14 @@ __device__ __forceinline__ PairItem pair_item_read(const PairItem &l)
 struct PairHeavyShared {                 // in LDS behind the bitmap
     PairItem slot[2];
     double wave_part[SG_WAVES];
+    unsigned long long wave_hits[SG_WAVES];
     alignas(16) uint32_t marks[SG_WAVES][QUAD_MARKS / 4];
     int batch_next;
 };
 template <bool ONE>
 __global__ __launch_bounds__(SG_T) void pair_sum_heavy_kernel(PairSide s0, PairSide s1, int nwords,
                                                               unsigned long long *__restrict__ tickets,
+                                                              unsigned long long *__restrict__ block_hits,
                                                               double *__restrict__ out)
 {
     uint32_t *bm = sg_dyn_lds;
@@ -574,11 +595,8 @@ __global__ __launch_bounds__(SG_T) void pair_sum_heavy_kernel(PairSide s0, PairS
         it = pair_item_read(sh.slot[cur]);
         lds_barrier();
     }
-    if constexpr (ONE) {
-        const int lo = wave_sum_i32((int)(all_hits & 0xffffff)), hi = wave_sum_i32((int)(all_hits >> 24));
-        if (lane == 0 && (lo | hi))
-            atomicAdd(&tickets[1], (unsigned long long)(uint32_t)lo + ((unsigned long long)(uint32_t)hi << 24));
-    }
+    if constexpr (ONE)
+        pair_block_hits(sh.wave_hits, all_hits, SG_WAVES, block_hits);
 }
 
 // The rows of short tables: a wavefront per row, the table's row in buckets of four columns in LDS - a look-up is one
@@ -591,13 +609,13 @@ constexpr int PAIR_LIGHT_OCC = 5;             // workgroups of four wavefronts o
 constexpr int PAIR_LIGHT_WAVES = 4;
 
 template <bool ONE>
-__global__ __launch_bounds__(PAIR_LIGHT_WAVES * 64, PAIR_LIGHT_OCC) void pair_sum_light_kernel(PairSide s0, PairSide s1,
-                                                                               unsigned long long *__restrict__ tickets,
-                                                                               double *__restrict__ out)
+__global__ __launch_bounds__(PAIR_LIGHT_WAVES * 64, PAIR_LIGHT_OCC) void pair_sum_light_kernel(
+    PairSide s0, PairSide s1, unsigned long long *__restrict__ block_hits, double *__restrict__ out)
 {
     constexpr int NB = 1 << PAIR_LIGHT_LOG;
     __shared__ __align__(16) int table[PAIR_LIGHT_WAVES][NB * 4];
     __shared__ __align__(16) uint32_t all_marks[PAIR_LIGHT_WAVES][QUAD_MARKS / 4];
+    __shared__ unsigned long long wave_hits[PAIR_LIGHT_WAVES];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     int *tab = table[wv];
     uint32_t *marks = all_marks[wv];
@@ -733,11 +751,8 @@ __global__ __launch_bounds__(PAIR_LIGHT_WAVES * 64, PAIR_LIGHT_OCC) void pair_su
             wave_lds_order();
         }
     }
-    if constexpr (ONE) {
-        const int lo = wave_sum_i32((int)(all_hits & 0xffffff)), hi = wave_sum_i32((int)(all_hits >> 24));
-        if (lane == 0 && (lo | hi))
-            atomicAdd(&tickets[1], (unsigned long long)(uint32_t)lo + ((unsigned long long)(uint32_t)hi << 24));
-    }
+    if constexpr (ONE)
+        pair_block_hits(wave_hits, all_hits, PAIR_LIGHT_WAVES, block_hits);
 }
 
 // partial[block] = sum of a fixed share of the rows' sums
@@ -761,32 +776,38 @@ __global__ __launch_bounds__(256) void pair_sum_partial(PairSide s0, PairSide s1
         partial[blockIdx.x] = lds[0];
 }
 
-// The result to the host's word, the tickets back to zero for the next call.
+// The result to the host's word, the ticket back to zero for the next call.  partial: n sums, or null: block_hits, n counts.
 __global__ __launch_bounds__(256) void pair_sum_finish(unsigned long long *__restrict__ tickets,
-                                                       const double *__restrict__ partial, int n, double each,
+                                                       const double *__restrict__ partial,
+                                                       const unsigned long long *__restrict__ block_hits, int n, double each,
                                                        double *__restrict__ result)
 {
     __shared__ double lds[256];
-    if (partial) {
-        lds[threadIdx.x] = (int)threadIdx.x < n ? partial[threadIdx.x] : 0.0;
-        __syncthreads();
-        for (int d = 128; d > 0; d >>= 1) {
-            if ((int)threadIdx.x < d)
-                lds[threadIdx.x] += lds[threadIdx.x + d];
-            __syncthreads();
+    __shared__ unsigned long long counts[256];
+    unsigned long long mine = 0;
+    if (!partial)
+        for (int i = threadIdx.x; i < n; i += 256)
+            mine += block_hits[i];
+    counts[threadIdx.x] = mine;
+    lds[threadIdx.x] = partial && (int)threadIdx.x < n ? partial[threadIdx.x] : 0.0;
+    __syncthreads();
+    for (int d = 128; d > 0; d >>= 1) {
+        if ((int)threadIdx.x < d) {
+            lds[threadIdx.x] += lds[threadIdx.x + d];
+            counts[threadIdx.x] += counts[threadIdx.x + d];
         }
+        __syncthreads();
     }
     if (threadIdx.x == 0) {
-        const unsigned long long count = tickets[1];
-        *result = partial ? lds[0] * each : count ? (double)count * each : 0.0;
-        tickets[0] = tickets[1] = 0;
+        *result = partial ? lds[0] * each : counts[0] ? (double)counts[0] * each : 0.0;
+        tickets[0] = 0;
     }
 }
 
 // ---------------------------------------------------------------------------
 // Plans
 // ---------------------------------------------------------------------------
-static Workspace g_pair_chunk, g_pair_row, g_pair_turn, g_pair_tickets, g_pair_out, g_pair_partial;
+static Workspace g_pair_chunk, g_pair_row, g_pair_turn, g_pair_tickets, g_pair_out, g_pair_partial, g_pair_hits;
 
 // pos[first] and pos[last] of x
 static int pair_ends(const Csr *x, int64_t first, int64_t last, int64_t *word, int64_t *ends)
@@ -970,11 +991,34 @@ static int pair_turned(const Csr *a, Csr *turned)
     return COMET_HIP_OK;
 }
 
+// Whether every row is sent one way: 1 to workgroups, 2 to wavefronts (the tests send each class of rows through both).
+static int pair_only()
+{
+    const char *env = getenv("COMET_HIP_MASKED_SUM_ONLY");
+    return !env ? 0 : strcmp(env, "workgroup") == 0 ? 1 : strcmp(env, "wavefront") == 0 ? 2 : 0;
+}
+
+// Workgroups of the two kernels of a sum, and the LDS of those of the long rows.
+struct PairGrids {
+    unsigned heavy, light;
+    int nwords;
+    size_t lds;
+};
+static PairGrids pair_grids(int64_t nheavy, int64_t nlight, int64_t ncols)
+{
+    PairGrids g;
+    g.nwords = (int)ceil_div(ceil_div(ncols, 32), 4) * 4;
+    g.lds = sizeof(uint32_t) * (size_t)g.nwords + sizeof(PairHeavyShared);
+    const int per_cu = (int)std::max<size_t>(1, std::min<size_t>(2, (size_t)(150 * 1024) / g.lds));
+    g.heavy = (unsigned)std::min<int64_t>(nheavy, (int64_t)num_cus() * per_cu);
+    g.light = (unsigned)std::min<int64_t>(ceil_div(nlight, PAIR_LIGHT_WAVES), (int64_t)num_cus() * PAIR_LIGHT_OCC);
+    return g;
+}
+
 // SUM of C<M> = A*B for a pattern matrix B (every value is b->iso_value).
 static int pair_masked_sum(Csr *a, Csr *b, Csr *m, double *result)
 {
-    const char *env = getenv("COMET_HIP_MASKED_SUM_ONLY");
-    const int only = !env ? 0 : strcmp(env, "workgroup") == 0 ? 1 : strcmp(env, "wavefront") == 0 ? 2 : 0;
+    const int only = pair_only();
     bool one = false;
     COMET_CHK(csr_is_iso(a, &one));
     PairPlan key;
@@ -1034,31 +1078,32 @@ static int pair_masked_sum(Csr *a, Csr *b, Csr *m, double *result)
         partial = (double *)g_pair_partial.ptr;
     }
     const bool beside = nheavy > 0 && nlight > 0 && plan->side[0].pairs + plan->side[1].pairs >= PAIR_BESIDE;
+    const PairGrids grids = pair_grids(nheavy, nlight, b->ncols);
+    COMET_CHK(g_pair_hits.ensure(sizeof(unsigned long long) * (size_t)(grids.heavy + grids.light + 1), false));
+    unsigned long long *hits = (unsigned long long *)g_pair_hits.ptr;
     if (beside)
         COMET_CHK(aux_fork());
     if (nheavy > 0) {
-        const int nwords = (int)ceil_div(ceil_div(b->ncols, 32), 4) * 4;
-        const size_t lds = sizeof(uint32_t) * (size_t)nwords + sizeof(PairHeavyShared);
-        const int per_cu = (int)std::max<size_t>(1, std::min<size_t>(2, (size_t)(150 * 1024) / lds));
-        const dim3 grid((unsigned)std::min<int64_t>(nheavy, (int64_t)num_cus() * per_cu)), block(SG_T);
+        const int nwords = grids.nwords;
+        const size_t lds = grids.lds;
+        const dim3 grid(grids.heavy), block(SG_T);
         KernelTimer t("spgemm_masked_sum");
         if (one) {
             COMET_CHK(sg_allow_lds(pair_sum_heavy_kernel<true>, lds));
-            pair_sum_heavy_kernel<true><<<grid, block, lds, stream()>>>(s0, s1, nwords, tickets, out);
+            pair_sum_heavy_kernel<true><<<grid, block, lds, stream()>>>(s0, s1, nwords, tickets, hits, out);
         } else {
             COMET_CHK(sg_allow_lds(pair_sum_heavy_kernel<false>, lds));
-            pair_sum_heavy_kernel<false><<<grid, block, lds, stream()>>>(s0, s1, nwords, tickets, out);
+            pair_sum_heavy_kernel<false><<<grid, block, lds, stream()>>>(s0, s1, nwords, tickets, hits, out);
         }
     }
     if (nlight > 0) {
-        const dim3 grid((unsigned)std::min<int64_t>(ceil_div(nlight, PAIR_LIGHT_WAVES), (int64_t)num_cus() * PAIR_LIGHT_OCC)),
-            block(PAIR_LIGHT_WAVES * 64);
+        const dim3 grid(grids.light), block(PAIR_LIGHT_WAVES * 64);
         const hipStream_t on = beside ? aux_stream() : stream();
         KernelTimer t("spgemm_masked_sum_small", on);
         if (one)
-            pair_sum_light_kernel<true><<<grid, block, 0, on>>>(s0, s1, tickets, out);
+            pair_sum_light_kernel<true><<<grid, block, 0, on>>>(s0, s1, hits + grids.heavy, out);
         else
-            pair_sum_light_kernel<false><<<grid, block, 0, on>>>(s0, s1, tickets, out);
+            pair_sum_light_kernel<false><<<grid, block, 0, on>>>(s0, s1, hits + grids.heavy, out);
     }
     if (beside)
         COMET_CHK(aux_join());
@@ -1066,7 +1111,8 @@ static int pair_masked_sum(Csr *a, Csr *b, Csr *m, double *result)
         KernelTimer t("spgemm_masked_sum_reduce");
         pair_sum_partial<<<dim3(256), dim3(256), 0, stream()>>>(s0, s1, out, partial);
     }
-    pair_sum_finish<<<dim3(1), dim3(256), 0, stream()>>>(tickets, partial, 256, one ? a->iso_value * b->iso_value : 1.0, word);
+    pair_sum_finish<<<dim3(1), dim3(256), 0, stream()>>>(tickets, partial, hits, one ? (int)(grids.heavy + grids.light) : 256,
+                                                         one ? a->iso_value * b->iso_value : 1.0, word);
     COMET_HIPCHK(hipGetLastError());
     COMET_CHK(stream_wait());
     *result = *(volatile double *)word;
