@@ -123,6 +123,13 @@ struct PairPlan {
     PairSidePlan side[2];
 };
 void pair_plan_free(PairPlan &p);
+// A triangle count's (triangles.h): the rows of words, where they begin, and the pairs.
+struct TriPlan {
+    uint32_t *words = nullptr;
+    int64_t *tpos = nullptr;
+    PairSidePlan side;
+};
+void tri_plan_free(TriPlan &p);
 
 struct Csr {
     // names this state of the matrix: new for every matrix and again whenever its arrays may have changed
@@ -188,7 +195,10 @@ struct Csr {
     double iso_value = 0.0;
     // products taken with this matrix on the left so far (0, 1, more): the SpMM and SpMV plans, which cost tens of
     // products, are built when a matrix is multiplied for the second time (plan_at_once() builds them at the first)
-    int spmm_uses = 0, spmv_uses = 0, sddmm_uses = 0;
+    int spmm_uses = 0, spmv_uses = 0, sddmm_uses = 0, tri_uses = 0;
+    // triangle counts (tri_state: 0 not looked at, 1 not of the kind, 2 made)
+    int tri_state = 0;
+    TriPlan tri;
     // SDDMM: the stored entries in an order that keeps columns of D in an L2, XCD x's from sddmm_start[x] on: their
     // places, then their rows, then their columns
     // (sddmm_state: 0 not looked at, 1 not worth it, 2 made)

@@ -362,14 +362,25 @@ uint64_t next_csr_uid()
     return next.fetch_add(1);
 }
 
+static void pair_side_free(PairSidePlan &s)
+{
+    for (void *q : {(void *)s.kpos, (void *)s.place, (void *)s.counts, s.ent, s.heavy, (void *)s.weight,
+                    (void *)s.light, (void *)s.padded})
+        (void)dev_free(q);
+    s = PairSidePlan();
+}
 void pair_plan_free(PairPlan &p)
 {
-    for (PairSidePlan &s : p.side) {
-        for (void *q : {(void *)s.kpos, (void *)s.place, (void *)s.counts, s.ent, s.heavy, (void *)s.weight,
-                        (void *)s.light, (void *)s.padded})
-            (void)dev_free(q);
-        s = PairSidePlan();
-    }
+    for (PairSidePlan &s : p.side)
+        pair_side_free(s);
+}
+void tri_plan_free(TriPlan &p)
+{
+    (void)dev_free(p.words);
+    (void)dev_free(p.tpos);
+    p.words = nullptr;
+    p.tpos = nullptr;
+    pair_side_free(p.side);
 }
 
 static void csr_drop_plans(Csr *c)
@@ -377,6 +388,8 @@ static void csr_drop_plans(Csr *c)
     for (PairPlan &p : c->pair_plans)
         pair_plan_free(p);
     c->pair_plans.clear();
+    tri_plan_free(c->tri);
+    c->tri_state = c->tri_uses = 0;
     c->uid = next_csr_uid();
     for (auto &e : c->row_lists) {
         (void)dev_free(e.rows);

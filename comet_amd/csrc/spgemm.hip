@@ -3169,6 +3169,7 @@ static int csr_is_iso(const Csr *x, bool *iso)
 
 #include "masked_pairs.h"
 #include "masked_dots.h"
+#include "triangles.h"
 
 // A masked product runs as dot products when the table over k fits LDS and no list that goes into a table holds a
 // column twice.  COMET_HIP_SPGEMM_NO_DOT keeps the walk over the products of every row (the tests run both).
@@ -3557,6 +3558,14 @@ extern "C" int comet_hip_spgemm_masked_sum(int64_t ah, int64_t bh, int64_t mh, d
     bool pairs = false;
     if (iso)
         COMET_CHK(pair_form_fits(a, b, m, &pairs));
+    if (pairs && a == b && a == m) {
+        const bool plan_now = a->tri_uses > 0 || plan_at_once();
+        a->tri_uses = 1;
+        if (plan_now && a->tri_state == 0)
+            COMET_CHK(tri_plan(a, pair_only()));
+        if (a->tri_state == 2)
+            return tri_count(a, out);
+    }
     if (pairs)
         return pair_masked_sum(a, b, m, out);
     COMET_CHK(sg_reset_ticket());

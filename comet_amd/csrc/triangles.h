@@ -1,0 +1,628 @@
+// Triangle counts: SUM of C<L> = L*L for one strictly triangular matrix L of equal values (included by spgemm.hip after
+// masked_pairs.h).  What is counted are the triangles of the graph with an edge for every entry, and their number does not
+// depend on how the vertices are called.  So they get new numbers, most edges first, and every vertex a row: its neighbours
+// with smaller numbers.  Nobody has many of those - 672 at most for the R-MAT graph of 2^20 vertices, where rows of L have
+// up to 20698 entries -, and they are close together, because a few thousand vertices are most of all neighbours.
+// Rows are therefore kept as words: the number of a group of sixteen vertices and a bit for each of them.  A triangle is
+// an edge and a vertex that both ends' rows hold; an edge costs the words of the shorter row, looked up in a table of the
+// longer one, and a word is a look-up for all its vertices: 1.1 G look-ups of 4 bytes instead of 2.3 G.
+// The plan costs three to ten counts (3 ms for 2^20 vertices, 0.6 for 20351), so it is made when a matrix is counted for
+// the second time.  us a count, edge factor 16: n = 2^20 1571 -> 890, 200003 349 -> 260, 60000 148 -> 108, 20351 80 -> 70,
+// 1000 41 -> 22.  Bound by the rows' way from the memory-side cache for large graphs (5 TB/s), by the chain of a wavefront
+// - bounds of a row, its table, its lists - for small ones.
+
+constexpr int TRI_GROUP_LOG = 4;                         // vertices of a word: bits 0-15; bits 16-31: which sixteen
+constexpr int64_t TRI_MOST = 1ll << (16 + TRI_GROUP_LOG);       // vertices that can be named
+
+// flags[0]: some row has an entry on or above the diagonal, flags[1]: on or below it
+__global__ __launch_bounds__(256) void tri_sides(int64_t n, const int64_t *__restrict__ pos, const int32_t *__restrict__ crd,
+                                                 int *__restrict__ flags)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n || pos[i] == pos[i + 1])
+        return;
+    if (crd[pos[i + 1] - 1] >= i)            // columns ascend
+        flags[0] = 1;
+    if (crd[pos[i]] <= i)
+        flags[1] = 1;
+}
+
+// degree[v]: entries in row and column v, tpos the transpose's row pointers; without them (a small matrix) the columns are
+// counted one by one, a wavefront per row.  (15.7 M entries so: 2.5 ms, a long column's atomics wait for each other.)
+__global__ __launch_bounds__(256) void tri_degrees(int64_t n, const int64_t *__restrict__ pos,
+                                                   const int32_t *__restrict__ crd, const int64_t *__restrict__ tpos,
+                                                   unsigned *__restrict__ degree)
+{
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (tpos) {
+        if (t < n)
+            degree[t] = (unsigned)(pos[t + 1] - pos[t] + tpos[t + 1] - tpos[t]);
+        return;
+    }
+    const int lane = threadIdx.x & 63;
+    const int64_t i = t >> 6;
+    if (i >= n)
+        return;
+    const int64_t s = pos[i], e = pos[i + 1];
+    for (int64_t p = s + lane; p < e; p += 64)
+        atomicAdd(&degree[crd[p]], 1u);
+    if (lane == 0 && e > s)
+        atomicAdd(&degree[i], (unsigned)(e - s));
+}
+
+__global__ __launch_bounds__(256) void tri_rank_keys(int64_t n, const unsigned *__restrict__ degree,
+                                                     uint64_t *__restrict__ keys, uint32_t *__restrict__ idx)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) {
+        keys[i] = 0xffffffffu - degree[i];
+        idx[i] = (uint32_t)i;
+    }
+}
+
+__global__ __launch_bounds__(256) void tri_ranks(int64_t n, const uint32_t *__restrict__ by_degree, uint32_t *__restrict__ rank)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n)
+        rank[by_degree[i]] = (uint32_t)i;
+}
+
+// keys[p] = larger new number << bits | smaller one, whatever rows the entries are of (a wavefront per row: 0.49 ms for
+// 15.7 M entries, most of it the longest row's)
+__global__ __launch_bounds__(256) void tri_edge_keys(int64_t n, int64_t nnz, const int64_t *__restrict__ pos,
+                                                     const int32_t *__restrict__ crd, const uint32_t *__restrict__ rank,
+                                                     int bits, uint64_t *__restrict__ keys)
+{
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t first = uniform_i64_sg(p - (threadIdx.x & 63));
+    if (first >= nnz)
+        return;
+    // the last row that begins at or before an entry: the wavefront's first one, then each lane's from there on
+    const auto row_of = [&](int64_t q, int64_t lo, int64_t hi) {
+        while (lo < hi) {
+            const int64_t mid = (lo + hi + 1) >> 1;
+            if (pos[mid] <= q)
+                lo = mid;
+            else
+                hi = mid - 1;
+        }
+        return lo;
+    };
+    const int64_t last = first + 63 < nnz ? first + 63 : nnz - 1;
+    const int64_t lo = row_of(first, 0, n - 1), hi = row_of(last, lo, n - 1);
+    if (p < nnz) {
+        const uint64_t a = rank[row_of(p, lo, hi)], b = rank[crd[p]];
+        keys[p] = a > b ? a << bits | b : b << bits | a;
+    }
+}
+
+// opens[p] = 1 where sorted key p begins a word
+__global__ __launch_bounds__(256) void tri_opens(int64_t nnz, const uint64_t *__restrict__ keys, int64_t *__restrict__ opens)
+{
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p < nnz)
+        opens[p] = p == 0 || keys[p - 1] >> TRI_GROUP_LOG != keys[p] >> TRI_GROUP_LOG;
+}
+
+// at[r] = first p with keys[p] >> bits >= r, for r in [0, n]
+__global__ __launch_bounds__(256) void tri_row_starts(int64_t n, int64_t nnz, const uint64_t *__restrict__ keys, int bits,
+                                                      int64_t *__restrict__ at)
+{
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (r > n)
+        return;
+    int64_t lo = 0, hi = nnz;
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if ((int64_t)(keys[mid] >> bits) < r)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    at[r] = lo;
+}
+
+// quads[r]: four words each, of row r; word_at[p]: words that begin before key p
+__global__ __launch_bounds__(256) void tri_row_quads(int64_t n, const int64_t *__restrict__ row_at,
+                                                     const int64_t *__restrict__ word_at, int64_t *__restrict__ quads)
+{
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (r < n)
+        quads[r] = (word_at[row_at[r + 1]] - word_at[row_at[r]] + 3) >> 2;
+}
+
+// tpos[r] = first word of row r; the quad in front of all rows is empty
+__global__ __launch_bounds__(256) void tri_word_starts(int64_t n, const int64_t *__restrict__ quads_before,
+                                                       int64_t *__restrict__ tpos)
+{
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (r <= n)
+        tpos[r] = 4 * (quads_before[r] + 1);
+}
+
+__global__ __launch_bounds__(256) void tri_words(int64_t nnz, const uint64_t *__restrict__ keys, int bits,
+                                                 const int64_t *__restrict__ row_at, const int64_t *__restrict__ word_at,
+                                                 const int64_t *__restrict__ tpos, uint32_t *__restrict__ words)
+{
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p >= nnz || word_at[p] == word_at[p + 1])
+        return;
+    const uint64_t group = keys[p] >> TRI_GROUP_LOG;
+    const int64_t r = (int64_t)(keys[p] >> bits);
+    uint32_t in = 0;
+    for (int64_t q = p; q < nnz && keys[q] >> TRI_GROUP_LOG == group; ++q)
+        in |= 1u << ((uint32_t)keys[q] & ((1u << TRI_GROUP_LOG) - 1u));
+    const uint32_t which = (uint32_t)(group & ((1ull << (bits - TRI_GROUP_LOG)) - 1ull));
+    words[tpos[r] + word_at[p] - word_at[row_at[r]]] = which << 16 | in;
+}
+
+// An edge is looked at from the end with the longer row: keys = that end (n: the other has no row, nothing to do),
+// lists = the other end.
+__global__ __launch_bounds__(256) void tri_pairs(int64_t n, int64_t nnz, const uint64_t *__restrict__ edges, int bits,
+                                                 const int64_t *__restrict__ tpos, uint64_t *__restrict__ keys,
+                                                 uint32_t *__restrict__ lists)
+{
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p >= nnz)
+        return;
+    const int64_t a = (int64_t)(edges[p] >> bits), b = (int64_t)(edges[p] & ((1ull << bits) - 1ull));
+    const int64_t la = tpos[a + 1] - tpos[a], lb = tpos[b + 1] - tpos[b];
+    keys[p] = (uint64_t)(lb == 0 ? n : la > lb ? a : b);
+    lists[p] = (uint32_t)(la > lb ? b : a);
+}
+
+__global__ __launch_bounds__(256) void tri_entries(int64_t n, int64_t nnz, const uint64_t *__restrict__ keys,
+                                                   const uint32_t *__restrict__ lists, const int64_t *__restrict__ tpos,
+                                                   PairEnt *__restrict__ ent, int64_t *__restrict__ work)
+{
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p >= nnz)
+        return;
+    const int64_t l = lists[p], s = tpos[l], len = tpos[l + 1] - s;
+    const bool in = (int64_t)keys[p] < n;
+    ent[p] = PairEnt{(uint32_t)(s >> 2), in ? (uint32_t)(len >> 2) : 0u};
+    work[p] = in ? len + PAIR_LIST_COST : 0;
+}
+
+__global__ __launch_bounds__(256) void tri_row_work(int64_t n, const int64_t *__restrict__ kpos,
+                                                    const int64_t *__restrict__ work_before, int64_t *__restrict__ wpos)
+{
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (r <= n)
+        wpos[r] = work_before[kpos[r]];
+}
+
+// ---------------------------------------------------------------------------
+// The walk of masked_pairs.h on rows that are whole quads: no lane needs a mask, one that has no quad takes the empty one.
+// ---------------------------------------------------------------------------
+template <int ROWS>
+struct TriTurn {
+    uint4 q[ROWS];
+    int rows;
+};
+
+template <int ROWS, typename CONSUME>
+__device__ __forceinline__ void tri_walk(TriTurn<ROWS> &pend, uint32_t start, int quads, const uint4 *__restrict__ rows,
+                                         uint32_t *marks, int lane, CONSUME consume)
+{
+    const int inc = wave_inclusive_scan(quads), pre = inc - quads;
+    const int Q = __builtin_amdgcn_readlane(inc, 63);
+    const int a0 = (int)(start - (uint32_t)pre), end = (int)(start + (uint32_t)quads);
+    uint32_t before = 0;                 // lists that begin before this row of quads, less one
+    for (int base = 0; base < Q; base += 64 * ROWS) {
+        const uint32_t bit = (uint32_t)(pre - 1 - base);
+        if (quads > 0 && bit < 64u * ROWS)
+            atomicOr(&marks[bit >> 5], 1u << (bit & 31u));
+        wave_lds_order();
+        uint2 m[ROWS];
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r)
+            m[r] = reinterpret_cast<const uint2 *>(marks)[r];
+        wave_lds_order();
+        if (lane < 2 * ROWS)
+            marks[lane] = 0;
+        TriTurn<ROWS> now;
+        now.rows = (Q - base + 63) >> 6 < ROWS ? (Q - base + 63) >> 6 : ROWS;
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            if (r < now.rows) {
+                const int owner = (int)__builtin_amdgcn_mbcnt_hi(m[r].y, __builtin_amdgcn_mbcnt_lo(m[r].x, before));
+                before += __popc(m[r].x) + __popc(m[r].y);
+                const uint32_t at = (uint32_t)lane_value(a0, owner) + (uint32_t)(base + 64 * r + lane);
+                now.q[r] = rows[at < (uint32_t)lane_value(end, owner) ? at : 0u];
+            }
+        }
+        wave_lds_order();
+        consume(pend);
+        pend = now;
+    }
+}
+
+// the table of a long row: its sixteen bits of every group, at address 0 of the LDS
+struct TriBitsProbe {
+    __device__ __forceinline__ uint32_t common(uint32_t w) const
+    {
+        return *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>(w >> 15 & 0x1fffeu) & w;
+    }
+};
+// of a short one: its words in buckets of four
+struct TriBucketProbe {
+    const int *tab;
+    uint32_t mult;
+    int shift;               // 32 - log2 of the buckets
+    __device__ __forceinline__ uint32_t common(uint32_t w) const
+    {
+        const si_bucket b = *reinterpret_cast<const si_bucket *>(tab + 4 * BucketProbe::bucket((int)(w >> 16), mult, shift));
+        const uint32_t x[4] = {(uint32_t)b.x ^ w, (uint32_t)b.y ^ w, (uint32_t)b.z ^ w, (uint32_t)b.w ^ w};
+        uint32_t same = 0;           // where the group is the same: the bits that differ, turned over
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            same |= x[c] < 0x10000u ? ~x[c] : 0u;
+        return same & w & 0xffffu;
+    }
+};
+struct TriBisectProbe {
+    const uint32_t *row;    // the table's words, ascending, behind them empty ones
+    int n;
+    __device__ __forceinline__ uint32_t common(uint32_t w) const
+    {
+        int lo = 0, hi = n;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            const uint32_t v = row[mid];
+            if (v != 0 && v >> 16 < w >> 16)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        return lo < n && row[lo] >> 16 == w >> 16 ? row[lo] & w & 0xffffu : 0u;
+    }
+};
+
+template <int ROWS, typename PROBE>
+__device__ __forceinline__ void tri_sum(const TriTurn<ROWS> &t, const PROBE &probe, uint32_t &hits)
+{
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        if (r < t.rows) {
+            const uint32_t a = probe.common(t.q[r].x), b = probe.common(t.q[r].y), c = probe.common(t.q[r].z),
+                           d = probe.common(t.q[r].w);
+            hits += __popc(a | b << 16) + __popc(c | d << 16);
+        }
+    }
+}
+
+// As pair_sum_heavy_kernel.  nwords: 32-bit words of the table.
+__global__ __launch_bounds__(SG_T) void tri_heavy_kernel(PairSide s, int nwords, unsigned long long *__restrict__ tickets,
+                                                         unsigned long long *__restrict__ block_hits)
+{
+    uint16_t *bits = reinterpret_cast<uint16_t *>(sg_dyn_lds);
+    PairHeavyShared &sh = *reinterpret_cast<PairHeavyShared *>(sg_dyn_lds + nwords);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    uint32_t *marks = sh.marks[wave];
+    const uint32_t *words = reinterpret_cast<const uint32_t *>(s.Tcrd);
+    const uint4 *rows = reinterpret_cast<const uint4 *>(s.Lcrd);
+    for (int w = threadIdx.x; w < nwords + (int)(sizeof sh / 4); w += SG_T)
+        sg_dyn_lds[w] = 0;
+    __syncthreads();
+    const uint32_t n = (uint32_t)(s.counts[0] & 0xffffffff);
+    if (threadIdx.x == 0)
+        sh.slot[0] = pair_item(s, s, n, 0, atomicAdd(&tickets[0], 1ull));
+    __syncthreads();
+    PairItem it = pair_item_read(sh.slot[0]);
+    int cur = 0;
+    unsigned long long all_hits = 0;
+    const TriBitsProbe probe;
+    while (it.index >= 0) {
+        for (int t = threadIdx.x; t < it.tlen; t += SG_T) {
+            const uint32_t w = words[it.ts + t];
+            if (w)
+                bits[w >> 16] = (uint16_t)w;
+        }
+        if (threadIdx.x == 0)
+            sh.batch_next = SG_WAVES;
+        lds_barrier();
+        if (threadIdx.x == 0)
+            sh.slot[cur ^ 1] = pair_item(s, s, n, 0, atomicAdd(&tickets[0], 1ull));
+        const int mine = (it.kn + it.parts - 1) / it.parts;          // pairs of a part, about
+        int B = mine / (4 * SG_WAVES);
+        B = B > 64 ? 64 : B < 2 ? 2 : B;
+        const int nb = (it.kn + B - 1) / B;
+        PairEnt e{0, 0};
+        const auto fetch = [&](int j) {
+            const int64_t p = (int64_t)(it.part + it.parts * j) * B + lane;
+            e.len = 0;
+            if (lane < B && p < it.kn)
+                e = s.ent[it.ks + p];
+        };
+        TriTurn<4> pend;
+        pend.rows = 0;
+        uint32_t hits = 0;
+        int j = wave;
+        fetch(j);
+        while (it.part + it.parts * j < nb) {
+            const PairEnt now = e;
+            int d = 0;
+            if (lane == 0)
+                d = atomicAdd(&sh.batch_next, 1);
+            j = __builtin_amdgcn_readfirstlane(d);
+            fetch(j);          // the next batch's pairs arrive while this one is walked
+            tri_walk(pend, now.start, (int)now.len, rows, marks, lane,
+                     [&](const TriTurn<4> &t) { tri_sum(t, probe, hits); });
+        }
+        tri_sum(pend, probe, hits);
+        all_hits += hits;
+        lds_barrier();
+        for (int t = threadIdx.x; t < it.tlen; t += SG_T)
+            bits[words[it.ts + t] >> 16] = 0;
+        cur ^= 1;
+        it = pair_item_read(sh.slot[cur]);
+        lds_barrier();
+    }
+    pair_block_hits(sh.wave_hits, all_hits, SG_WAVES, block_hits);
+}
+
+// As pair_sum_light_kernel.
+__global__ __launch_bounds__(PAIR_LIGHT_WAVES * 64, PAIR_LIGHT_OCC) void tri_light_kernel(
+    PairSide s, unsigned long long *__restrict__ block_hits)
+{
+    constexpr int NB = 1 << PAIR_LIGHT_LOG;
+    __shared__ __align__(16) int table[PAIR_LIGHT_WAVES][NB * 4];
+    __shared__ __align__(16) uint32_t all_marks[PAIR_LIGHT_WAVES][QUAD_MARKS / 4];
+    __shared__ unsigned long long wave_hits[PAIR_LIGHT_WAVES];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    int *tab = table[wv];
+    uint32_t *marks = all_marks[wv];
+    const uint32_t *words = reinterpret_cast<const uint32_t *>(s.Tcrd);
+    const uint4 *rows = reinterpret_cast<const uint4 *>(s.Lcrd);
+    const auto clear = [&](int buckets) {
+        for (int b = lane; b < buckets; b += 64)
+            reinterpret_cast<si_bucket *>(tab)[b] = si_bucket{0, 0, 0, 0};
+    };
+    clear(NB);
+    if (lane < QUAD_MARKS / 4)
+        marks[lane] = 0;
+    wave_lds_order();
+    const unsigned long long n = (unsigned long long)s.counts[0] >> 32;
+    unsigned long long all_hits = 0;
+    const unsigned long long waves = (unsigned long long)gridDim.x * PAIR_LIGHT_WAVES;
+    const unsigned long long wave_id = blockIdx.x + (unsigned long long)gridDim.x * wv;
+    for (unsigned long long tk = wave_id; tk < n; tk += 64 * waves) {
+        const unsigned long long left = (n - 1 - tk) / waves + 1;
+        const int nr = (int)(left < 64 ? left : 64);
+        int64_t l_ts = 0, l_ks = 0;
+        int l_tlen = 0, l_kn = 0;
+        if (lane < nr) {
+            const int x = s.light[tk + lane * waves];
+            l_ts = s.Tpos[x];
+            l_tlen = (int)(s.Tpos[x + 1] - l_ts);
+            l_ks = s.kpos[x];
+            l_kn = (int)(s.kpos[x + 1] - l_ks);
+        }
+        // the words and the first 64 pairs of the next row arrive while this one is walked
+        constexpr int PER = (PAIR_LIGHT_MAX + 63) / 64;
+        uint32_t wn[PER];
+        PairEnt en{0, 0};
+        const auto ahead = [&](int r) {
+            const int64_t ts = readlane_i64(l_ts, r), ks = readlane_i64(l_ks, r);
+            const int tlen = __builtin_amdgcn_readlane(l_tlen, r), kn = __builtin_amdgcn_readlane(l_kn, r);
+#pragma unroll
+            for (int u = 0; u < PER; ++u)
+                wn[u] = 64 * u + lane < tlen ? words[ts + 64 * u + lane] : 0u;
+            en.len = 0;
+            if (lane < kn)
+                en = s.ent[ks + lane];
+        };
+        ahead(0);
+        for (int r = 0; r < nr; ++r) {
+            const int64_t ts = readlane_i64(l_ts, r), ks = readlane_i64(l_ks, r);
+            const int tlen = __builtin_amdgcn_readlane(l_tlen, r), kn = __builtin_amdgcn_readlane(l_kn, r);
+            PairEnt e = en;
+            uint32_t w[PER];
+#pragma unroll
+            for (int u = 0; u < PER; ++u)
+                w[u] = wn[u];
+            if (r + 1 < nr)
+                ahead(r + 1);
+            const auto fetch = [&](int b) {
+                e.len = 0;
+                if (b + lane < kn)
+                    e = s.ent[ks + b + lane];
+            };
+            bool hashed = false;
+            uint32_t mult = 0;
+            // as many buckets as keep them three quarters of a word full, 64 at least
+            int log_nb = 6;
+            while (log_nb < PAIR_LIGHT_LOG && tlen > (1 << log_nb) * 3 / 4)
+                ++log_nb;
+            const int shift = 32 - log_nb;
+            if (tlen <= PAIR_LIGHT_MAX) {
+                for (int attempt = 0; attempt < 4 && !hashed; ++attempt) {
+                    mult = attempt == 0 ? 0x9E3779u : attempt == 1 ? 0x85EBCBu : attempt == 2 ? 0xC2B2AFu : 0x27D4EBu;
+                    bool placed = true;
+#pragma unroll
+                    for (int u = 0; u < PER; ++u) {
+                        bool in = w[u] == 0;
+                        if (!in) {
+                            int *bk = tab + 4 * BucketProbe::bucket((int)(w[u] >> 16), mult, shift);
+#pragma unroll
+                            for (int x = 0; x < 4; ++x)
+                                if (!in)
+                                    in = atomicCAS(&bk[x], 0, (int)w[u]) == 0;
+                        }
+                        placed = placed && in;
+                    }
+                    hashed = !__any(!placed);
+                    if (!hashed)
+                        clear(1 << log_nb);
+                }
+            }
+            wave_lds_order();
+            uint32_t hits = 0;
+            TriTurn<PAIR_LIGHT_ROWS> pend;
+            pend.rows = 0;
+            const auto walk = [&](const auto &probe) {
+                for (int b = 0; b < kn; b += 64) {
+                    const PairEnt now = e;
+                    fetch(b + 64);
+                    tri_walk(pend, now.start, (int)now.len, rows, marks, lane,
+                             [&](const TriTurn<PAIR_LIGHT_ROWS> &t) { tri_sum(t, probe, hits); });
+                }
+                tri_sum(pend, probe, hits);
+            };
+            if (hashed)
+                walk(TriBucketProbe{tab, mult, shift});
+            else
+                walk(TriBisectProbe{words + ts, tlen});
+            all_hits += hits;
+            wave_lds_order();
+            if (hashed)
+                clear(1 << log_nb);
+            wave_lds_order();
+        }
+    }
+    pair_block_hits(wave_hits, all_hits, PAIR_LIGHT_WAVES, block_hits);
+}
+
+// ---------------------------------------------------------------------------
+// The plan, kept in the handle as tri (its side holds the pairs) with tri_state 2; 1: the matrix is not of the kind.
+// ---------------------------------------------------------------------------
+static int tri_plan(Csr *a, int only)
+{
+    a->tri_state = 1;
+    const int64_t n = a->nrows, nnz = a->nnz;
+    if (n != a->ncols || n > TRI_MOST || nnz == 0 || nnz >= (1ll << 31))
+        return COMET_HIP_OK;
+    bool alone = false;
+    COMET_CHK(dot_no_duplicates(a, &alone));
+    if (!alone)
+        return COMET_HIP_OK;
+    int64_t *word = nullptr;
+    COMET_CHK(mailbox((void **)&word));
+    const dim3 block(256), per_row((unsigned)ceil_div(n + 1, 256)), per_entry((unsigned)ceil_div(nnz, 256));
+    int bits = TRI_GROUP_LOG;
+    while ((1ll << bits) < n + 1)
+        ++bits;
+    TriPlan &plan = a->tri;
+    PairSidePlan &side = plan.side;
+    // scratch: two arrays of a 64-bit and one of a 32-bit word for every entry, and some for every row
+    uint64_t *k0 = nullptr, *k1 = nullptr;
+    uint32_t *i0 = nullptr, *i1 = nullptr;
+    int64_t *w0 = nullptr, *r0 = nullptr, *r1 = nullptr;
+    const size_t entries = (size_t)std::max(nnz, n) + 1, rows = (size_t)n + 2;
+    const int64_t quads_most = nnz / 4 + n + 2;
+    const bool room =
+        dev_malloc((void **)&k0, 8 * entries) == hipSuccess && dev_malloc((void **)&k1, 8 * entries) == hipSuccess &&
+        dev_malloc((void **)&i0, 4 * entries) == hipSuccess && dev_malloc((void **)&i1, 4 * entries) == hipSuccess &&
+        dev_malloc((void **)&w0, 8 * entries) == hipSuccess && dev_malloc((void **)&r0, 8 * rows) == hipSuccess &&
+        dev_malloc((void **)&r1, 8 * rows) == hipSuccess && dev_malloc((void **)&plan.words, 16 * (size_t)quads_most) == hipSuccess &&
+        dev_malloc((void **)&plan.tpos, 8 * rows) == hipSuccess && dev_malloc((void **)&side.kpos, 8 * rows) == hipSuccess &&
+        dev_malloc((void **)&side.counts, 8) == hipSuccess && dev_malloc(&side.ent, sizeof(PairEnt) * (size_t)nnz) == hipSuccess;
+    const auto run = [&]() -> int {
+        KernelTimer t("triangle_plan");
+        unsigned *degree = (unsigned *)i1;
+        uint32_t *rank = i0;
+        COMET_HIPCHK(hipMemsetAsync(r0, 0, 8, stream()));
+        tri_sides<<<per_row, block, 0, stream()>>>(n, a->pos, a->crd, (int *)r0);
+        COMET_HIPCHK(hipMemcpyAsync(word, r0, 8, hipMemcpyDeviceToHost, stream()));
+        COMET_CHK(stream_wait());
+        const volatile int *flags = (const volatile int *)word;
+        if (flags[0] && flags[1])
+            return COMET_HIP_OK;                 // neither strictly lower nor strictly upper
+        // ---- the vertices by their number of edges
+        if (nnz <= PAIR_ROOM_UNSEEN) {
+            COMET_HIPCHK(hipMemsetAsync(degree, 0, 4 * (size_t)n, stream()));
+            tri_degrees<<<dim3((unsigned)ceil_div(n, 4)), block, 0, stream()>>>(n, a->pos, a->crd, nullptr, degree);
+        } else {
+            Csr *turned = nullptr;
+            COMET_CHK(dot_transposed(a, &turned));          // (the first count's plan has left it)
+            tri_degrees<<<per_row, block, 0, stream()>>>(n, a->pos, a->crd, turned->pos, degree);
+        }
+        tri_rank_keys<<<per_row, block, 0, stream()>>>(n, degree, k0, i0);
+        COMET_CHK(sort_pairs_u64_u32(k0, k1, i0, i1, n, 32));
+        tri_ranks<<<per_row, block, 0, stream()>>>(n, i1, rank);
+        // ---- their rows
+        tri_edge_keys<<<per_entry, block, 0, stream()>>>(n, nnz, a->pos, a->crd, rank, bits, k0);
+        COMET_CHK(sort_pairs_u64_u32(k0, k1, i1, (uint32_t *)w0, nnz, 2 * bits));          // (what goes along is not used)
+        int64_t *opens = (int64_t *)k0;
+        tri_opens<<<per_entry, block, 0, stream()>>>(nnz, k1, opens);
+        COMET_CHK(exclusive_scan_i64(opens, nnz, w0));
+        tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, k1, bits, r0);
+        tri_row_quads<<<per_row, block, 0, stream()>>>(n, r0, w0, r1);
+        COMET_CHK(exclusive_scan_i64(r1, n, side.kpos));
+        tri_word_starts<<<per_row, block, 0, stream()>>>(n, side.kpos, plan.tpos);
+        COMET_HIPCHK(hipMemsetAsync(plan.words, 0, 16 * (size_t)quads_most, stream()));
+        tri_words<<<per_entry, block, 0, stream()>>>(nnz, k1, bits, r0, w0, plan.tpos, plan.words);
+        // ---- the edges by the end they are looked at from
+        tri_pairs<<<per_entry, block, 0, stream()>>>(n, nnz, k1, bits, plan.tpos, k0, i0);
+        COMET_CHK(sort_pairs_u64_u32(k0, k1, i0, i1, nnz, bits));
+        tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, k1, 0, side.kpos);
+        int64_t *work = (int64_t *)k0;
+        tri_entries<<<per_entry, block, 0, stream()>>>(n, nnz, k1, i1, plan.tpos, (PairEnt *)side.ent, work);
+        COMET_CHK(exclusive_scan_i64(work, nnz, w0));
+        tri_row_work<<<per_row, block, 0, stream()>>>(n, side.kpos, w0, r0);
+        pair_parts<<<per_row, block, 0, stream()>>>(0, n, plan.tpos, side.kpos, r0, only, PAIR_LIGHT_MAX, r1);
+        COMET_CHK(exclusive_scan_i64(r1, n, r0));
+        COMET_HIPCHK(hipMemcpyAsync(word, r0 + n, 8, hipMemcpyDeviceToHost, stream()));
+        COMET_CHK(stream_wait());
+        const int64_t packed = *(volatile int64_t *)word;
+        side.nheavy = packed & 0xffffffff;
+        side.nlight = packed >> 32;
+        side.pairs = nnz;
+        COMET_HIPCHK(dev_malloc(&side.heavy, sizeof(uint2) * (size_t)(side.nheavy > 0 ? side.nheavy : 1)));
+        COMET_HIPCHK(dev_malloc((void **)&side.light, sizeof(int32_t) * (size_t)(side.nlight > 0 ? side.nlight : 1)));
+        pair_items<<<per_row, block, 0, stream()>>>(0, n, r1, r0, (uint2 *)side.heavy, side.light, side.counts);
+        COMET_HIPCHK(hipGetLastError());
+        a->tri_state = 2;
+        // the pairs of L as it is are of no use any more
+        for (size_t x = a->pair_plans.size(); x-- > 0;)
+            if (a->pair_plans[x].kind == 1 && a->pair_plans[x].b_uid == a->uid && a->pair_plans[x].mask_uid == a->uid) {
+                pair_plan_free(a->pair_plans[x]);
+                a->pair_plans.erase(a->pair_plans.begin() + (std::ptrdiff_t)x);
+            }
+        return COMET_HIP_OK;
+    };
+    int rc = COMET_HIP_OK;
+    if (room)
+        rc = run();
+    else
+        (void)hipGetLastError();                 // without the room the pairs of L stay as they are
+    for (void *p : {(void *)k0, (void *)k1, (void *)i0, (void *)i1, (void *)w0, (void *)r0, (void *)r1})
+        (void)dev_free(p);
+    if (a->tri_state != 2)
+        tri_plan_free(plan);
+    if (rc != COMET_HIP_OK)
+        a->tri_state = 0;
+    return rc;
+}
+
+// (The two kernels side by side: 889 us instead of 875 for n = 2^20, 260 / 255 for 200003, 92 / 70 for 20351.)
+static int tri_count(Csr *a, double *result)
+{
+    PairSide s = pair_side(a->tri.side, a, a);
+    s.Tpos = a->tri.tpos;
+    s.Tcrd = s.Lcrd = reinterpret_cast<const int32_t *>(a->tri.words);
+    const int64_t nheavy = a->tri.side.nheavy, nlight = a->tri.side.nlight;
+    unsigned long long *tickets = nullptr;
+    double *word = nullptr;
+    COMET_CHK(pair_tickets(&tickets));
+    COMET_CHK(mailbox((void **)&word));
+    const PairGrids grids = pair_grids(nheavy, nlight, a->ncols);
+    COMET_CHK(g_pair_hits.ensure(sizeof(unsigned long long) * (size_t)(grids.heavy + grids.light + 1), false));
+    unsigned long long *hits = (unsigned long long *)g_pair_hits.ptr;
+    if (nheavy > 0) {
+        COMET_CHK(sg_allow_lds(tri_heavy_kernel, grids.lds));
+        KernelTimer t("spgemm_masked_sum");
+        tri_heavy_kernel<<<dim3(grids.heavy), dim3(SG_T), grids.lds, stream()>>>(s, grids.nwords, tickets, hits);
+    }
+    if (nlight > 0) {
+        KernelTimer t("spgemm_masked_sum_small");
+        tri_light_kernel<<<dim3(grids.light), dim3(PAIR_LIGHT_WAVES * 64), 0, stream()>>>(s, hits + grids.heavy);
+    }
+    pair_sum_finish<<<dim3(1), dim3(256), 0, stream()>>>(tickets, nullptr, hits, (int)(grids.heavy + grids.light), a->iso_value * a->iso_value, word);
+    COMET_HIPCHK(hipGetLastError());
+    COMET_CHK(stream_wait());
+    *result = *(volatile double *)word;
+    return COMET_HIP_OK;
+}

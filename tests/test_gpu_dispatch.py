@@ -441,3 +441,88 @@ def test_spmm_sweep_of_rows_that_are_no_multiple_of_16_bytes(K, ldb, ldc, shift,
     assert np.array_equal(got[np.diff(pos) <= 1], want[np.diff(pos) <= 1])
     view(out, ldc)[:] = 7.0
     assert np.all(out == 7.0)
+
+
+def _edges(kind, rng):
+    """Pairs of vertices (u > v) and the number of vertices."""
+    if kind == "complete":
+        n = 70
+        u, v = np.tril_indices(n, -1)
+    elif kind == "dense":               # rows of more words than a wavefront's table takes
+        n = 3400
+        u, v = np.tril_indices(n, -1)
+        keep = rng.random(len(u)) < 0.9
+        u, v = u[keep], v[keep]
+    elif kind == "star":                # no triangles, one vertex with all edges
+        n = 5000
+        u, v = np.arange(1, n), np.zeros(n - 1, np.int64)
+    elif kind == "wheel":               # its rim closes one triangle for every vertex
+        n = 40_000
+        u = np.concatenate([np.arange(1, n), np.arange(2, n), [n - 1]])
+        v = np.concatenate([np.zeros(n - 1, np.int64), np.arange(1, n - 1), [1]])
+    else:
+        n, m = kind
+        u, v = rng.integers(0, n, (2, m)) if m else np.zeros((2, 0), np.int64)
+        u, v = np.maximum(u, v)[u != v], np.minimum(u, v)[u != v]
+    key = np.unique(np.asarray(u, np.int64) * n + v)
+    return n, key // n, key % n
+
+
+@pytest.mark.parametrize("only", [None, "workgroup", "wavefront"])
+@pytest.mark.parametrize("upper", [False, True])
+@pytest.mark.parametrize("kind", ["complete", "dense", "star", "wheel", (1, 0), (2, 1), (15, 60), (16, 90), (17, 100), (33, 300),
+                                  (4097, 60_000), (100_003, 900_000), (1 << 20, 2_000_000), ((1 << 20) + 1, 500_000)])
+def test_triangle_counts_of_every_kind_of_graph(kind, upper, only, monkeypatch):
+    # both triangles of the matrix, rows through either kernel, numbers of vertices around a word's and the most that are
+    # named in 16 + 4 bits; the first count walks L as it is, the others the vertices by their number of edges
+    monkeypatch.delenv("COMET_HIP_PLAN_AT_ONCE")
+    if only:
+        monkeypatch.setenv("COMET_HIP_MASKED_SUM_ONLY", only)
+    rng = np.random.default_rng(7)
+    n, u, v = _edges(kind, rng)
+    shuffle = rng.permutation(n)
+    u, v = np.maximum(shuffle[u], shuffle[v]), np.minimum(shuffle[u], shuffle[v])
+    if upper:
+        u, v = v, u
+    order = np.lexsort((v, u))
+    u, v = u[order], v[order]
+    pos = np.concatenate([[0], np.cumsum(np.bincount(u, minlength=n))]).astype(np.int64)
+    L = rt.CsrMatrix.from_arrays((n, n), pos, v.astype(np.int64), np.full(len(u), 0.5))
+    if kind == "dense":
+        D = np.zeros((n, n))
+        D[u, v] = 1.0
+        want = float(((D @ D) * D).sum())
+    else:
+        want = orc.tricount_masked(pos, v.astype(np.int64), np.ones(len(u)))
+    assert [rt.triangle_count(L) for _ in range(4)] == [0.25 * want] * 4
+
+
+def test_sums_that_are_no_triangle_count_stay_as_they_are():
+    # one handle three times, but with a diagonal, with entries on both sides, with a column twice, with more columns than
+    # rows of other vertices; and values that change under the handle
+    rng = np.random.default_rng(3)
+    n, u, v = _edges((300, 6000), rng)
+    csr = lambda a, b, val: (np.concatenate([[0], np.cumsum(np.bincount(a, minlength=n))]).astype(np.int64), b.astype(np.int64), val)
+    diagonal = np.arange(n)
+    for a, b in ((np.concatenate([u, diagonal]), np.concatenate([v, diagonal])), (np.concatenate([u, v]), np.concatenate([v, u])),
+                 (np.concatenate([u, u[:50]]), np.concatenate([v, v[:50]]))):
+        order = np.lexsort((b, a))
+        pos, crd, val = csr(a[order], b[order], np.ones(len(a)))
+        L = rt.CsrMatrix.from_arrays((n, n), pos, crd, val)
+        rows = np.repeat(np.arange(n), np.diff(pos))
+        D = np.zeros((n, n))
+        np.add.at(D, (rows, crd), 1.0)
+        want = float(((D @ D) * (D > 0)).sum())
+        assert rt.triangle_count(L) == rt.triangle_count(L) == want
+    pos, crd, val = csr(u, v, np.ones(len(u)))
+    D = np.zeros((n, n))
+    D[u, v] = 1.0
+    L = rt.CsrMatrix.from_arrays((n, n), pos, crd, val)
+    count = float(((D @ D) * D).sum())
+    assert rt.triangle_count(L) == rt.triangle_count(L) == count
+    val = rng.integers(1, 4, len(u)).astype(np.float64)
+    rt._check(rt.lib().comet_hip_memcpy(L.device_arrays()[2], rt._vptr(val), val.nbytes, 0))
+    rt._check(rt.lib().comet_hip_csr_invalidate(L.handle), "invalidate")
+    W = np.zeros((n, n))
+    W[u, v] = val
+    assert rt.triangle_count(L) == rt.triangle_count(L) == float(((W @ W) * D).sum())
