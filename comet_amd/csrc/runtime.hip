@@ -692,6 +692,62 @@ __global__ __launch_bounds__(SCAN_T) void scan_apply(const int64_t *__restrict__
     }
 }
 
+// Few counts in one launch by one workgroup, SCAN_ONE_E to a lane: three launches take 13 us whatever they do, this 5 for
+// 16384 counts and 4 for 1000.
+constexpr int SCAN_ONE_T = 1024, SCAN_ONE_E = 16;
+constexpr int64_t SCAN_ONE_MOST = (int64_t)SCAN_ONE_T * SCAN_ONE_E;
+__device__ __forceinline__ int64_t wave_inclusive_scan_i64(int64_t v)
+{
+#define COMET_SCAN_STEP(ctrl, rows)                                                                              \
+    v += (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_update_dpp(0, (int)(v >> 32), ctrl, rows, 0xf, false) << 32 | \
+                   (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false));
+    COMET_SCAN_STEP(0x111, 0xf)          // row_shr:1, 2, 4, 8: within sixteen lanes
+    COMET_SCAN_STEP(0x112, 0xf)
+    COMET_SCAN_STEP(0x114, 0xf)
+    COMET_SCAN_STEP(0x118, 0xf)
+    COMET_SCAN_STEP(0x142, 0xa)          // row_bcast:15 into rows 1 and 3, row_bcast:31 into rows 2 and 3
+    COMET_SCAN_STEP(0x143, 0xc)
+#undef COMET_SCAN_STEP
+    return v;
+}
+__global__ __launch_bounds__(SCAN_ONE_T) void scan_one(const int64_t *__restrict__ in, int n, int64_t *__restrict__ pos,
+                                                       int64_t *total)
+{
+    __shared__ int64_t wave_tot[SCAN_ONE_T / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int rows = (n + SCAN_ONE_T - 1) / SCAN_ONE_T;          // of 64 counts, a wavefront's one behind the other
+    const int base = wave * rows * 64 + lane;
+    int64_t v[SCAN_ONE_E], before[SCAN_ONE_E];
+#pragma unroll
+    for (int r = 0; r < SCAN_ONE_E; ++r)
+        v[r] = r < rows && base + 64 * r < n ? in[base + 64 * r] : 0;
+    int64_t run = 0;
+#pragma unroll
+    for (int r = 0; r < SCAN_ONE_E; ++r) {
+        if (r < rows) {
+            const int64_t inc = wave_inclusive_scan_i64(v[r]);
+            before[r] = run + inc - v[r];
+            run += (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(inc >> 32), 63) << 32 |
+                             (uint32_t)__builtin_amdgcn_readlane((int)inc, 63));
+        }
+    }
+    if (lane == 0)
+        wave_tot[wave] = run;
+    __syncthreads();
+    const int64_t mine = lane < SCAN_ONE_T / 64 ? wave_tot[lane] : 0;
+    const int64_t off = wave_inclusive_scan_i64(mine) - mine;          // of the wavefront with the lane's number
+    const int64_t own = (int64_t)((uint64_t)(uint32_t)__shfl((int)(off >> 32), wave, 64) << 32 | (uint32_t)__shfl((int)off, wave, 64));
+#pragma unroll
+    for (int r = 0; r < SCAN_ONE_E; ++r)
+        if (r < rows && base + 64 * r < n)
+            pos[base + 64 * r] = own + before[r];
+    if (wave == SCAN_ONE_T / 64 - 1 && lane == 0) {
+        pos[n] = own + run;
+        if (total)
+            *total = own + run;
+    }
+}
+
 static Workspace g_scan_ws;
 
 int exclusive_scan_i64(const int64_t *counts, int64_t n, int64_t *pos, int64_t *total)
@@ -700,6 +756,12 @@ int exclusive_scan_i64(const int64_t *counts, int64_t n, int64_t *pos, int64_t *
         COMET_HIPCHK(hipMemsetAsync(pos, 0, sizeof(int64_t), stream()));
         if (total)
             *total = 0;
+        return COMET_HIP_OK;
+    }
+    if (n <= SCAN_ONE_MOST) {
+        KernelTimer t("scan_one");
+        scan_one<<<dim3(1), dim3(SCAN_ONE_T), 0, stream()>>>(counts, (int)n, pos, total);
+        COMET_HIPCHK(hipGetLastError());
         return COMET_HIP_OK;
     }
     int64_t nblocks = ceil_div(n, SCAN_B);

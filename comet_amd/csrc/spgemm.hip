@@ -2800,7 +2800,16 @@ static int sg_allow_lds(K kernel, size_t bytes)
 }
 
 // the row counters of a phase's kernels, one each
-constexpr int SG_TICKETS = 4;          // (32 bytes: one fill)
+// 0-3: a phase's own, which clears them; 4-7: the numeric phase's where the symbolic one of the same call has cleared them
+constexpr int SG_TICKETS = 8;
+__global__ __launch_bounds__(256) void sg_clear(unsigned long long *__restrict__ tickets, int64_t *__restrict__ rowcount, int64_t n)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < SG_TICKETS)
+        tickets[i] = 0;
+    if (i < n)
+        rowcount[i] = 0;
+}
 static unsigned long long *sg_ticket(int k) { return (unsigned long long *)g_sg.ticket.ptr + k; }
 static int sg_reset_ticket()
 {
@@ -2967,11 +2976,16 @@ constexpr int64_t SG_DENSE_PER_BLOCK = 8;
 // with the kernels as they are now 1024 per block 437, 2048 402, 4096 386, 6144 381, 8192 382, 12288 382, 16384 389).
 // COMET_HIP_SPGEMM_WIDE, a number of products per row, overrides the rule: either kernel is right for any row,
 // so the tests use it to send the same rows through both.
-constexpr int64_t SG_WIDE_PER_BLOCK = 6144;
-static int64_t sg_wide_threshold(int nblk)
+// With one or two blocks the line lies higher, us by products per block, 6144 / 10240: 10000 vertices, edge factor 16 572 /
+// 536, 16000 and 16 849 / 809, 30000 and 10 1379 / 1239 (three blocks: 45000 and 12 2990 / 3064).  A matrix that fills no
+// more than half a block sends all its heavy rows there, a launch less: 1024 and 8 117 / 97, 4096 and 8 178 / 153, 8000 and
+// 4 162 / 139, 8192 and 16 346 / 331.
+constexpr int64_t SG_WIDE_PER_BLOCK = 6144, SG_WIDE_PER_BLOCK_FEW = 10240;
+constexpr int64_t SG_NARROW = SG_CB / 2;
+static int64_t sg_wide_threshold(int64_t ncols, int nblk)
 {
     const char *e = getenv("COMET_HIP_SPGEMM_WIDE");
-    return e && *e ? atoll(e) : SG_WIDE_PER_BLOCK * nblk;
+    return e && *e ? atoll(e) : ncols <= SG_NARROW ? 0 : (nblk <= 2 ? SG_WIDE_PER_BLOCK_FEW : SG_WIDE_PER_BLOCK) * nblk;
 }
 
 // From how many products on a row's values are kept in LDS by the large workgroups, and from how many on block by block.
@@ -2981,7 +2995,7 @@ static SgClasses sg_row_classes(int64_t ncols, bool small)
     const int nblk = (int)ceil_div(ncols > 0 ? ncols : 1, SG_CB);
     SgClasses c;
     c.dense = small ? SM_PRODUCTS + 1 : SG_DENSE_PER_BLOCK * nblk;
-    c.wide = std::max(sg_wide_threshold(nblk), c.dense);
+    c.wide = std::max(sg_wide_threshold(ncols, nblk), c.dense);
     return c;
 }
 static int sm_words(int64_t ncols) { return (int)ceil_div(ceil_div(ncols > 0 ? ncols : 1, 32), 4) * 4; }
@@ -3009,7 +3023,6 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
     }
     SgGeom g;
     COMET_CHK(sg_geometry(b->ncols, &g));
-    COMET_CHK(sg_reset_ticket());
     RowList list;
     const bool small = !m && b->ncols <= SM_COLS;
     const SgClasses classes = sg_row_classes(b->ncols, small);
@@ -3017,7 +3030,9 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
         COMET_CHK(sg_row_list(a, b, 0, a->nrows, classes.dense, classes.wide, &list, nullptr, 0, true));
     else
         COMET_CHK(sg_row_list(a, b, 0, a->nrows, SG_NO_DENSE, SG_NO_DENSE, &list));
-    COMET_HIPCHK(hipMemsetAsync(rowcount, 0, sizeof(int64_t) * (size_t)a->nrows, stream()));
+    COMET_CHK(g_sg.ticket.ensure(SG_TICKETS * sizeof(unsigned long long), false));
+    sg_clear<<<dim3((unsigned)ceil_div(std::max<int64_t>(a->nrows, SG_TICKETS), 256)), dim3(256), 0, stream()>>>(sg_ticket(0), rowcount,
+                                                                                                    a->nrows);
     if (small && !list.only_heavy()) {
         const int words = sm_words(b->ncols);
         KernelTimer t("spgemm_symbolic_small");
@@ -3189,7 +3204,7 @@ static int dot_form_fits(const Csr *a, const Csr *b, const Csr *m, bool *fits)
 }
 
 static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos, int64_t rb, int64_t re,
-                        int32_t *Ccrd, double *Cval, int reduce_op, int mult_op)
+                        int32_t *Ccrd, double *Cval, int reduce_op, int mult_op, bool tickets_clear = false)
 {
     if (reduce_op < 0 || reduce_op > COMET_SR_ANY || mult_op < 0 || mult_op > COMET_OP_DIV)
         return set_error(COMET_HIP_ERR_ARG, "unknown semiring (reduce %d, mult %d)", reduce_op, mult_op);
@@ -3214,7 +3229,9 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     }
     SgGeom g;
     COMET_CHK(sg_geometry(b->ncols, &g));
-    COMET_CHK(sg_reset_ticket());
+    if (!tickets_clear)
+        COMET_CHK(sg_reset_ticket());
+    unsigned long long *tickets = sg_ticket(tickets_clear ? SG_TICKETS / 2 : 0);
     // rows with many products go to the LDS-accumulator kernel (unmasked products only)
     const int nblk = (int)ceil_div(b->ncols > 0 ? b->ncols : 1, SG_CB);
     // (the `any` semiring keeps a product's place in B in 32 bits of its accumulator)
@@ -3254,7 +3271,7 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         spgemm_numeric_kernel<L, M, S><<<grid, block, num_lds, stream()>>>(                                \
             rb, re, b->ncols, a->pos, a->crd, a->val, b->pos, b->crd, b->val, m ? m->pos : nullptr,        \
             m ? m->crd : nullptr, g.logW, gbm, gmask, (double *)g_sg.slabs.ptr,                            \
-            (unsigned long long *)g_sg.ticket.ptr, list, 1, reduce_op, mult_op, Cpos, Ccrd, Cval);         \
+            tickets, list, 1, reduce_op, mult_op, Cpos, Ccrd, Cval);         \
     } while (0)
 #define LAUNCH_NUM_S(L, M)                                                                                 \
     do {                                                                                                   \
@@ -3312,7 +3329,7 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         COMET_CHK(sg_allow_lds(spgemm_numeric_dense_blocks_kernel<S, COL>, DB_LDS));                       \
         spgemm_numeric_dense_blocks_kernel<S, COL><<<cus, block, DB_LDS, stream()>>>(                      \
             (const DenseRow *)g_sg.dense_rows.ptr, nd, a->crd, a->val, CRD, b->val, b->nnz, b->sg_blkptr, nblk, \
-            sg_ticket(1), (int32_t *)g_sg.dense_before.ptr, rows_each, patience, gave_up, Ccrd, Cval,      \
+            tickets + 1, (int32_t *)g_sg.dense_before.ptr, rows_each, patience, gave_up, Ccrd, Cval,      \
             reduce_op, mult_op);                                                                           \
     } while (0)
 #define LAUNCH_BLOCKS(S)                                                                                   \
@@ -3336,7 +3353,7 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         COMET_CHK(sg_allow_lds(spgemm_numeric_dense_kernel<S, M, COL>, SG_DENSE_LDS));                     \
         spgemm_numeric_dense_kernel<S, M, COL><<<cus, block, SG_DENSE_LDS, stream()>>>(                    \
             rb, re, a->pos, a->crd, a->val, CRD, b->val, m ? m->pos : nullptr, m ? m->crd : nullptr,       \
-            b->sg_blkptr, nblk, sg_ticket(1), list, Cpos, Ccrd, Cval, reduce_op, mult_op);                                                                                      \
+            b->sg_blkptr, nblk, tickets + 1, list, Cpos, Ccrd, Cval, reduce_op, mult_op);                                                                                      \
     } while (0)
 #define LAUNCH_DENSE(S, M)                                                                                 \
     do {                                                                                                   \
@@ -3361,12 +3378,12 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
             COMET_CHK(sg_allow_lds(spgemm_numeric_span_kernel<true>, SG_SPAN_LDS));
             spgemm_numeric_span_kernel<true><<<cus, block, SG_SPAN_LDS, stream()>>>(
                 rb, re, a->pos, a->crd, a->val, b->crd, b->val, b->sg_blkptr, nblk,
-                sg_ticket(2), list, Cpos, Ccrd, Cval, reduce_op, mult_op);
+                tickets + 2, list, Cpos, Ccrd, Cval, reduce_op, mult_op);
         } else {
             COMET_CHK(sg_allow_lds(spgemm_numeric_span_kernel<false>, SG_SPAN_LDS));
             spgemm_numeric_span_kernel<false><<<cus, block, SG_SPAN_LDS, stream()>>>(
                 rb, re, a->pos, a->crd, a->val, b->crd, b->val, b->sg_blkptr, nblk,
-                sg_ticket(2), list, Cpos, Ccrd, Cval, reduce_op, mult_op);
+                tickets + 2, list, Cpos, Ccrd, Cval, reduce_op, mult_op);
         }
         COMET_HIPCHK(hipGetLastError());
     }
@@ -3527,7 +3544,7 @@ extern "C" int64_t comet_hip_spgemm_csr_semiring(int64_t ah, int64_t bh, int64_t
         delete c;
         return 0;
     }
-    if (nnz > 0 && numeric_rows(a, b, m, pos, 0, a->nrows, c->crd, c->val, reduce_op, mult_op) != COMET_HIP_OK) {
+    if (nnz > 0 && numeric_rows(a, b, m, pos, 0, a->nrows, c->crd, c->val, reduce_op, mult_op, !m) != COMET_HIP_OK) {
         (void)dev_free(c->crd);
         (void)dev_free(c->val);
         (void)dev_free(pos);
