@@ -1612,23 +1612,32 @@ struct DenseRow {
 constexpr int DB_ROWS = 8;
 constexpr int DB_PATIENCE = 1 << 24;
 
+// Where the rows come from: the first of the list, as rows of A and C.
+struct RowSource {
+    const int32_t *list;
+    int64_t row_begin;
+    const int64_t *Apos, *Cpos;
+};
+__device__ __forceinline__ DenseRow dense_row(const RowSource &s, int64_t x)
+{
+    const int64_t i = s.row_begin + s.list[x];
+    DenseRow r;
+    r.as = s.Apos[i];
+    r.cnt = (int32_t)(s.Apos[i + 1] - r.as);         // (the host sends matrices of under 2^30 entries here)
+    r.coff = s.Cpos[i] - s.Cpos[s.row_begin];
+    r.pad = 0;
+    return r;
+}
+
 // rows[r] for the nd first rows of the list and before[] in its initial state: nothing ahead of block 0, the rest open
-__global__ void spgemm_dense_rows(int64_t row_begin, RowList list, int64_t nd, int nblk, const int64_t *__restrict__ Apos,
-                                  const int64_t *__restrict__ Cpos, DenseRow *__restrict__ rows,
+__global__ void spgemm_dense_rows(RowSource source, int64_t nd, int nblk, DenseRow *__restrict__ rows,
                                   int32_t *__restrict__ before)
 {
     const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (x < nd * nblk)
         before[x] = x % nblk == 0 ? 0 : -1;
-    if (x < nd) {
-        const int64_t i = row_begin + list.rows[x];
-        DenseRow r;
-        r.as = Apos[i];
-        r.cnt = (int32_t)(Apos[i + 1] - r.as);         // (the host sends matrices of under 2^30 entries here)
-        r.coff = Cpos[i] - Cpos[row_begin];
-        r.pad = 0;
-        rows[x] = r;
-    }
+    if (x < nd)
+        rows[x] = dense_row(source, x);
 }
 
 // The slices of a row of the product inside a block lie in LDS for all wavefronts: 64 to a batch, the batch's own slices
@@ -1834,9 +1843,10 @@ __device__ __forceinline__ void block_emit(double *acc, int *wave_tot, int lane,
         reinterpret_cast<ulonglong2 *>(own)[r * 64 + lane] = none;
 }
 
-template <bool SEMI, typename COL>
+// ALONE: the matrix is one block wide, a row's entries leave at once; nobody has listed the rows (rows is null then).
+template <bool SEMI, typename COL, bool ALONE>
 __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
-    const DenseRow *__restrict__ rows, int64_t nd, const int32_t *__restrict__ Acrd, const double *__restrict__ Aval,
+    const DenseRow *__restrict__ rows, RowSource source, int64_t nd, const int32_t *__restrict__ Acrd, const double *__restrict__ Aval,
     const COL *__restrict__ Bcrd, const double *__restrict__ Bval, int64_t Bnnz, const int64_t *__restrict__ blkptr, int nblk,
     unsigned long long *ticket, int32_t *before, int rows_each, int patience, int *gave_up, int32_t *__restrict__ Ccrd,
     double *__restrict__ Cval, int reduce_op, int mult_op)
@@ -1854,18 +1864,22 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
         st.marks[wave][lane] = 0;
     lds_barrier();
     const int64_t nchunks = (nd + rows_each - 1) / rows_each;
-    const int64_t u_end = nchunks * nblk;
+    const int64_t u_end = ALONE ? nchunks : nchunks * nblk;
     int64_t u = draw_row<true>(ticket, 0, &row_slot);
     while (u < u_end) {
-        const int cb = (int)(u / nchunks);
+        const int cb = ALONE ? 0 : (int)(u / nchunks);
         const int64_t r0 = (u - cb * nchunks) * rows_each;
         const int nr = (int)(nd - r0 < rows_each ? nd - r0 : rows_each);
         const int col0 = cb << SG_CB_LOG;
         DenseRow mine;
         mine.as = mine.coff = 0;
         mine.cnt = 0;
-        if (lane < nr)
-            mine = rows[r0 + lane];
+        if (lane < nr) {
+            if constexpr (ALONE)
+                mine = dense_row(source, r0 + lane);
+            else
+                mine = rows[r0 + lane];
+        }
         // the entry of A a lane holds of row x of the ticket (of its first SG_T entries: a longer row loads the others
         // as it goes), and the slice of its row of B inside the block
         const auto load_entry = [&](int x, int &k, double &a) {
@@ -1885,7 +1899,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
         const auto load_slice = [&](int k, int64_t &lo, int64_t &hi) {
             lo = hi = 0;
             if (k >= 0) {
-                const int64_t *bp = blkptr + (int64_t)k * (nblk + 1) + cb;
+                const int64_t *bp = blkptr + (ALONE ? 2 * (int64_t)k : (int64_t)k * (nblk + 1) + cb);
                 lo = bp[0];
                 hi = bp[1];
             }
@@ -1924,9 +1938,9 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
             // What lies ahead of this block comes from whoever counted the block before it.  That was many tickets
             // ago as a rule, so the answer is asked for before the walk and the trip to memory it takes is over by
             // the time the walk is; only if it was not there yet is it waited for, behind the walk.
-            int32_t *mark = before + (r0 + x) * nblk + cb;
+            int32_t *mark = ALONE ? nullptr : before + (r0 + x) * nblk + cb;
             int early = 0;
-            if (threadIdx.x == 0 && cb > 0)
+            if (!ALONE && threadIdx.x == 0 && cb > 0)
                 early = __hip_atomic_fetch_max(mark, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             int turns;
             if (cnt <= SG_T) {
@@ -1972,6 +1986,8 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
             const int any = turns;          // every wavefront counts the same
             const auto await = [&]() {
                 int ahead = early;
+                if constexpr (ALONE)
+                    return 0;
                 for (int polls = 1; ahead < 0 && polls < patience; ++polls) {
                     __builtin_amdgcn_s_sleep(4);
                     ahead = __hip_atomic_fetch_max(mark, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1983,7 +1999,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
                 return ahead;
             };
             const auto hand_on = [&](int ahead) {
-                if (cb + 1 < nblk)
+                if (!ALONE && cb + 1 < nblk)
                     __hip_atomic_exchange(mark + 1, ahead, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             };
             if (any) {
@@ -3311,8 +3327,12 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         }
         if (nd > 0) {
             ran_blocks = true;
-            COMET_CHK(g_sg.dense_rows.ensure(sizeof(DenseRow) * (size_t)nd, false));
-            COMET_CHK(g_sg.dense_before.ensure(sizeof(int32_t) * (size_t)nd * (size_t)nblk, false));
+            const bool alone = nblk == 1;
+            if (!alone) {
+                COMET_CHK(g_sg.dense_rows.ensure(sizeof(DenseRow) * (size_t)nd, false));
+                COMET_CHK(g_sg.dense_before.ensure(sizeof(int32_t) * (size_t)nd * (size_t)nblk, false));
+            }
+            const RowSource source{list.rows, rb, a->pos, Cpos};
             gave_up[0] = 0;
             int patience = DB_PATIENCE;
             if (const char *e = getenv("COMET_HIP_SPGEMM_PATIENCE"))
@@ -3322,22 +3342,28 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
             // as many rows to a ticket as leave every CU some four of them (8 to each of 50 CUs: 78 us for a graph of 1024
             // vertices, the others idle)
             const int rows_each = (int)std::max<int64_t>(1, std::min<int64_t>(DB_ROWS, nd * nblk / (4 * (int64_t)cus.x)));
-            spgemm_dense_rows<<<dim3((unsigned)ceil_div(nd * nblk, 256)), dim3(256), 0, stream()>>>(
-                rb, list, nd, nblk, a->pos, Cpos, (DenseRow *)g_sg.dense_rows.ptr, (int32_t *)g_sg.dense_before.ptr);
-#define LAUNCH_BLOCKS_C(S, COL, CRD)                                                                       \
+            if (!alone)
+                spgemm_dense_rows<<<dim3((unsigned)ceil_div(nd * nblk, 256)), dim3(256), 0, stream()>>>(
+                    source, nd, nblk, (DenseRow *)g_sg.dense_rows.ptr, (int32_t *)g_sg.dense_before.ptr);
+#define LAUNCH_BLOCKS_C(S, COL, CRD, ALONE)                                                                \
     do {                                                                                                   \
-        COMET_CHK(sg_allow_lds(spgemm_numeric_dense_blocks_kernel<S, COL>, DB_LDS));                       \
-        spgemm_numeric_dense_blocks_kernel<S, COL><<<cus, block, DB_LDS, stream()>>>(                      \
-            (const DenseRow *)g_sg.dense_rows.ptr, nd, a->crd, a->val, CRD, b->val, b->nnz, b->sg_blkptr, nblk, \
-            tickets + 1, (int32_t *)g_sg.dense_before.ptr, rows_each, patience, gave_up, Ccrd, Cval,      \
-            reduce_op, mult_op);                                                                           \
+        COMET_CHK(sg_allow_lds(spgemm_numeric_dense_blocks_kernel<S, COL, ALONE>, DB_LDS));                \
+        spgemm_numeric_dense_blocks_kernel<S, COL, ALONE><<<cus, block, DB_LDS, stream()>>>(               \
+            (const DenseRow *)g_sg.dense_rows.ptr, source, nd, a->crd, a->val, CRD, b->val, b->nnz,        \
+            b->sg_blkptr, nblk, tickets + 1, (int32_t *)g_sg.dense_before.ptr, rows_each, patience,        \
+            gave_up, Ccrd, Cval, reduce_op, mult_op);                                                      \
     } while (0)
 #define LAUNCH_BLOCKS(S)                                                                                   \
     do {                                                                                                   \
-        if (b->sg_crd16 && getenv("COMET_HIP_SPGEMM_WIDE_COLUMNS") == nullptr)                             \
-            LAUNCH_BLOCKS_C(S, uint16_t, b->sg_crd16);                                                     \
+        const bool narrow = b->sg_crd16 && getenv("COMET_HIP_SPGEMM_WIDE_COLUMNS") == nullptr;             \
+        if (narrow && alone)                                                                               \
+            LAUNCH_BLOCKS_C(S, uint16_t, b->sg_crd16, true);                                               \
+        else if (narrow)                                                                                   \
+            LAUNCH_BLOCKS_C(S, uint16_t, b->sg_crd16, false);                                              \
+        else if (alone)                                                                                    \
+            LAUNCH_BLOCKS_C(S, int32_t, b->crd, true);                                                     \
         else                                                                                               \
-            LAUNCH_BLOCKS_C(S, int32_t, b->crd);                                                           \
+            LAUNCH_BLOCKS_C(S, int32_t, b->crd, false);                                                    \
     } while (0)
             if (semi) LAUNCH_BLOCKS(true); else LAUNCH_BLOCKS(false);
 #undef LAUNCH_BLOCKS_C
