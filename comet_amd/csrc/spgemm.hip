@@ -2649,33 +2649,106 @@ __global__ void fill_iota_f64(int64_t n, double *__restrict__ out)
 
 // ---------------------------------------------------------------------------
 // Rows with few products, SM_PRODUCTS at most, of matrices of few columns: a row is over in a handful of loads that wait
-// for each other, so what counts is how many rows are under way.  A workgroup of four wavefronts has the row's bitmap,
-// with the number of columns before every word of it, and a value for every product it can have: 21 to 29 KiB of LDS,
-// four to seven to a CU.  Sixteen lanes take an entry of A at a time.  (A workgroup of 1024 lanes to a row, one or two to a
-// CU, took 74 us more of the structure and 103 of the values of A*A for 16000 vertices, edge factor 8, which these take 30
-// and 88 for.)
+// for each other, so what counts is how few they are and how many rows are under way.  A workgroup of four wavefronts has
+// the row's bitmap, with the number of columns before every word of it, and a value for every product it can have: 26 to
+// 38 KiB of LDS, four to six to a CU.  A lane looks up one entry of A, the products are laid end to end over the lanes,
+// eight to a lane, which finds the entry of each by counting the beginnings before it: five loads one after the other
+// whatever the row looks like, and the products stay in registers for the second time they are needed.  (With sixteen
+// lanes to an entry a row of two hundred entries was thirteen times three loads one after the other, twice.)  us, structure
+// and values: A*A of R-MAT graphs of 65536 vertices, edge factor 16 96 + 379 -> 56 + 95, 30000 and 10 47 + 156 -> 26 + 48,
+// 16000 and 8 24 + 84 -> 17 + 34, 5000 and 12 17 + 36 -> 10 + 21.
 // ---------------------------------------------------------------------------
 constexpr int SM_T = 256, SM_PRODUCTS = 2048, SM_COLS = 1 << 16;
+constexpr int SM_PER = SM_PRODUCTS / SM_T;          // products of a lane
+struct SmallStage {
+    int64_t start[SM_T];                 // of the entries of A that have any: where their products begin in B, less their
+    double a[SM_T];                      // place among the products; A's value; the entry's place in the row
+    int place[SM_T];
+    uint32_t marks[SM_PRODUCTS / 32];    // a bit where an entry's products begin; zero between passes
+    int tot[2][SM_T / 64];
+};
 struct SmallRowLds {                     // behind the bitmap
     double val[SM_PRODUCTS];
+    SmallStage stage;
     uint16_t col[SM_PRODUCTS];
     int wave_tot[SM_T / 64];
 };
+template <bool VALUES>
+struct SmallProducts {
+    int col[SM_PER];                     // -1: none
+    double a[VALUES ? SM_PER : 1], b[VALUES ? SM_PER : 1];
+    int place[VALUES ? SM_PER : 1];
+    int64_t q[VALUES ? SM_PER : 1];      // the place in B
+};
 
-// f(column, a, b, place of a in the row + 1, place of b) for every product of the row [as, ae) of A
-template <bool VALUES, typename F>
-__device__ __forceinline__ void small_row_products(int64_t as, int64_t ae, const int32_t *__restrict__ Acrd,
-                                                   const double *__restrict__ Aval, const int64_t *__restrict__ Bpos,
-                                                   const int32_t *__restrict__ Bcrd, const double *__restrict__ Bval, F f)
+// The lane's products of the entries [p0, ae) of a row of A, SM_T of them at most.  The marks are left set: small_clear
+// behind the next barrier.
+template <bool VALUES>
+__device__ __forceinline__ void small_products(SmallStage &st, int64_t as, int64_t p0, int64_t ae,
+                                               const int32_t *__restrict__ Acrd, const double *__restrict__ Aval,
+                                               const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd,
+                                               const double *__restrict__ Bval, SmallProducts<VALUES> &out)
 {
-    const int group = threadIdx.x >> 4, sub = threadIdx.x & 15;
-    for (int64_t p = as + group; p < ae; p += SM_T / 16) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t p = p0 + tid;
+    int64_t bs = 0;
+    int len = 0;
+    double a = 0.0;
+    if (p < ae) {
         const int k = Acrd[p];
-        const double a = VALUES ? Aval[p] : 0.0;
-        const int64_t be = Bpos[k + 1];
-        for (int64_t q = Bpos[k] + sub; q < be; q += 16)
-            f(Bcrd[q], a, VALUES ? Bval[q] : 0.0, (int)(p - as) + 1, q);
+        bs = Bpos[k];
+        len = (int)(Bpos[k + 1] - bs);
+        if constexpr (VALUES)
+            a = Aval[p];
     }
+    const int inc = wave_inclusive_scan(len);
+    const unsigned long long has = __ballot(len > 0);
+    if (lane == 63) {
+        st.tot[0][wave] = inc;
+        st.tot[1][wave] = __popcll(has);
+    }
+    lds_barrier();
+    int off = inc - len, slot = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(has >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)has, 0));
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < SM_T / 64; ++w) {
+        off += w < wave ? st.tot[0][w] : 0;
+        slot += w < wave ? st.tot[1][w] : 0;
+        total += st.tot[0][w];
+    }
+    if (len > 0) {
+        st.start[slot] = bs - off;
+        if constexpr (VALUES) {
+            st.a[slot] = a;
+            st.place[slot] = (int)(p - as) + 1;
+        }
+        atomicOr(&st.marks[off >> 5], 1u << (off & 31));
+    }
+    lds_barrier();
+    static_assert(SM_PRODUCTS / 32 == 64, "a word of marks to a lane");
+    const int word = (int)st.marks[lane], before = wave_inclusive_scan(__popc((uint32_t)word)) - __popc((uint32_t)word);
+#pragma unroll
+    for (int x = 0; x < SM_PER; ++x) {
+        const int t = tid + SM_T * x, w = t >> 5;
+        const int m = lane_value(word, w), c = lane_value(before, w);
+        out.col[x] = -1;
+        if (t < total) {
+            const int owner = c + __popc((uint32_t)m & (uint32_t)((2ull << (t & 31)) - 1ull)) - 1;
+            const int64_t q = st.start[owner] + t;
+            out.col[x] = Bcrd[q];
+            if constexpr (VALUES) {
+                out.q[x] = q;
+                out.b[x] = Bval[q];
+                out.a[x] = st.a[owner];
+                out.place[x] = st.place[owner];
+            }
+        }
+    }
+}
+__device__ __forceinline__ void small_clear(SmallStage &st)
+{
+    if (threadIdx.x < SM_PRODUCTS / 32)
+        st.marks[threadIdx.x] = 0;
 }
 // before[w] = set bits in front of word w, for a thread's share of the words; returns how many there are
 __device__ __forceinline__ int small_row_ranks(const uint32_t *bm, uint16_t *before, int words, int *wave_tot)
@@ -2701,23 +2774,55 @@ __device__ __forceinline__ int small_row_ranks(const uint32_t *bm, uint16_t *bef
         }
     return all;
 }
+// the rows a workgroup takes, their bounds fetched while the row before is worked on
+struct SmallRows {
+    const RowList &list;
+    const int64_t *Apos;
+    int64_t row_begin, t, t_end;
+    int64_t r, rn, as, ae;               // this row (counted from row_begin), the next one, this one's entries of A
+    __device__ __forceinline__ SmallRows(const RowList &l, const int64_t *pos, int64_t begin)
+        : list(l), Apos(pos), row_begin(begin)
+    {
+        int64_t t_first;
+        list_range(list, 1, &t_first, &t_end);
+        t = t_first + blockIdx.x;
+        r = t < t_end ? list.rows[t] : 0;
+        rn = t + gridDim.x < t_end ? list.rows[t + gridDim.x] : r;
+        as = Apos[row_begin + r];
+        ae = Apos[row_begin + r + 1];
+    }
+    __device__ __forceinline__ bool more() const { return t < t_end; }
+};
 
 __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
     int64_t row_begin, RowList list, int words, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
     const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd, int64_t *__restrict__ rowcount)
 {
     uint32_t *bm = sg_dyn_lds;
+    __shared__ SmallStage stage;
     __shared__ int wave_tot[SM_T / 64];
     for (int w = threadIdx.x; w < words; w += SM_T)
         bm[w] = 0;
+    small_clear(stage);
     lds_barrier();
-    int64_t t_first, t_end;
-    list_range(list, 1, &t_first, &t_end);
-    for (int64_t t = t_first + blockIdx.x; t < t_end; t += gridDim.x) {
-        const int64_t r = list.rows[t], i = row_begin + r;
-        small_row_products<false>(Apos[i], Apos[i + 1], Acrd, nullptr, Bpos, Bcrd, nullptr,
-                                  [&](int j, double, double, int, int64_t) { atomicOr(&bm[j >> 5], 1u << (j & 31)); });
-        lds_barrier();
+    SmallRows rows(list, Apos, row_begin);
+    while (rows.more()) {
+        const int64_t r = rows.r, as = rows.as, ae = rows.ae;
+        rows.t += gridDim.x;
+        rows.r = rows.rn;
+        rows.as = Apos[row_begin + rows.rn];
+        rows.ae = Apos[row_begin + rows.rn + 1];
+        rows.rn = rows.t + gridDim.x < rows.t_end ? list.rows[rows.t + gridDim.x] : rows.rn;
+        for (int64_t p0 = as; p0 < ae; p0 += SM_T) {
+            SmallProducts<false> it;
+            small_products<false>(stage, as, p0, ae, Acrd, nullptr, Bpos, Bcrd, nullptr, it);
+#pragma unroll
+            for (int x = 0; x < SM_PER; ++x)
+                if (it.col[x] >= 0)
+                    atomicOr(&bm[it.col[x] >> 5], 1u << (it.col[x] & 31));
+            lds_barrier();
+            small_clear(stage);
+        }
         const int n = small_row_ranks(bm, nullptr, words, wave_tot);
         if (threadIdx.x == 0)
             rowcount[r] = n;
@@ -2741,24 +2846,44 @@ __global__ __launch_bounds__(SM_T) void spgemm_numeric_small_kernel(
     for (int w = threadIdx.x; w < words + words / 2 + (int)(sizeof sh / 4); w += SM_T)
         bm[w] = 0;
     lds_barrier();
-    int64_t t_first, t_end;
-    list_range(list, 1, &t_first, &t_end);
     const int64_t c0 = Cpos[row_begin];
-    for (int64_t t = t_first + blockIdx.x; t < t_end; t += gridDim.x) {
-        const int64_t i = row_begin + list.rows[t], as = Apos[i], ae = Apos[i + 1], coff = Cpos[i] - c0;
-        small_row_products<false>(as, ae, Acrd, nullptr, Bpos, Bcrd, nullptr,
-                                  [&](int j, double, double, int, int64_t) { atomicOr(&bm[j >> 5], 1u << (j & 31)); });
-        lds_barrier();
+    SmallRows rows(list, Apos, row_begin);
+    while (rows.more()) {
+        const int64_t as = rows.as, ae = rows.ae, coff = Cpos[row_begin + rows.r] - c0;
+        rows.t += gridDim.x;
+        rows.r = rows.rn;
+        rows.as = Apos[row_begin + rows.rn];
+        rows.ae = Apos[row_begin + rows.rn + 1];
+        rows.rn = rows.t + gridDim.x < rows.t_end ? list.rows[rows.t + gridDim.x] : rows.rn;
+        SmallProducts<true> it;
+        for (int64_t p0 = as; p0 < ae; p0 += SM_T) {
+            small_products<true>(sh.stage, as, p0, ae, Acrd, Aval, Bpos, Bcrd, Bval, it);
+#pragma unroll
+            for (int x = 0; x < SM_PER; ++x)
+                if (it.col[x] >= 0)
+                    atomicOr(&bm[it.col[x] >> 5], 1u << (it.col[x] & 31));
+            lds_barrier();
+            small_clear(sh.stage);
+        }
         const int total = small_row_ranks(bm, before, words, sh.wave_tot);
         lds_barrier();
-        small_row_products<true>(as, ae, Acrd, Aval, Bpos, Bcrd, Bval, [&](int j, double a, double b, int pa, int64_t q) {
-            const int r = before[j >> 5] + __popc(bm[j >> 5] & ((1u << (j & 31)) - 1u));
-            sh.col[r] = (uint16_t)j;
-            if constexpr (SEMI)
-                semiring_lds_add(&sh.val[r], reduce_op, mult_op, a, b, pa, q);
-            else
-                __hip_atomic_fetch_add(&sh.val[r], a * b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        });
+        for (int64_t p0 = as; p0 < ae; p0 += SM_T) {
+            if (ae - as > SM_T) {          // more entries than lanes: their products once more
+                small_products<true>(sh.stage, as, p0, ae, Acrd, Aval, Bpos, Bcrd, Bval, it);
+                lds_barrier();
+                small_clear(sh.stage);
+            }
+#pragma unroll
+            for (int x = 0; x < SM_PER; ++x)
+                if (it.col[x] >= 0) {
+                    const int j = it.col[x], r = before[j >> 5] + __popc(bm[j >> 5] & ((1u << (j & 31)) - 1u));
+                    sh.col[r] = (uint16_t)j;
+                    if constexpr (SEMI)
+                        semiring_lds_add(&sh.val[r], reduce_op, mult_op, it.a[x], it.b[x], it.place[x], it.q[x]);
+                    else
+                        __hip_atomic_fetch_add(&sh.val[r], it.a[x] * it.b[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
+        }
         lds_barrier();
         for (int q = threadIdx.x; q < total; q += SM_T) {
             const int j = sh.col[q];
