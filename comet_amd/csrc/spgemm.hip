@@ -1138,23 +1138,6 @@ __device__ __forceinline__ void turn_of_slice(int64_t s, int64_t o, int64_t len,
             f(j[x], at, v[x], pt, q[x]);
 }
 
-// A turn in which every lane has all its entries, the lane taking SG_LONG_LOADS consecutive ones (see the full turns of
-// for_each_in_slices): f4(j, a, v0, v1, pa, q) for the entries q .. q + 3.
-template <bool VALUES, typename COL, typename F4>
-__device__ __forceinline__ void full_turn_of_slice(int64_t s, int lane, double at, int pt, const COL *__restrict__ Bcrd,
-                                                   const double *__restrict__ Bval, F4 f4)
-{
-    typedef typename SgCol4<COL>::type col4;
-    const int64_t c = s + 4 * (int64_t)lane;
-    const col4 j = *reinterpret_cast<const col4 *>(Bcrd + c);
-    sg_d2u v0 = {0.0, 0.0}, v1 = {0.0, 0.0};
-    if constexpr (VALUES) {
-        v0 = *reinterpret_cast<const sg_d2u *>(Bval + c);
-        v1 = *reinterpret_cast<const sg_d2u *>(Bval + c + 2);
-    }
-    f4(j, at, v0, v1, pt, c);
-}
-
 struct SgOneByOne {};          // in place of f4: the four entries of a lane in a full turn go through f one by one
 template <bool VALUES, typename COL, typename F, typename F4 = SgOneByOne>
 __device__ __forceinline__ int for_each_in_slices(int64_t lo, int64_t hi, double a, int pa, int lane,
@@ -1649,21 +1632,23 @@ __global__ void spgemm_dense_rows(RowSource source, int64_t nd, int nblk, DenseR
 // Bound by the LDS, two thirds of the time busy: 36 clocks for 64 additions of doubles, 14 of them bank conflicts.  A*A of
 // R-MAT graphs, whole product: 65536 vertices, edge factor 16 5.31 -> 4.76 ms (with the walk alone, accumulators beside a
 // bitmap as before, 5.23), 30000 and 10 1.74 -> 1.47; 2^20 and 16 349 -> 329 ms.
-constexpr int DB_LEN_MOST = SG_CB;               // entries of a slice that are staged; more only with repeated columns
-constexpr int DB_END_BITS = 21;
-constexpr int64_t DB_NNZ_MOST = 1ll << 35;       // a place in B and 64 slices fit a word
+constexpr int64_t SLICE_NNZ_MOST = 1ll << 32;    // a place in B and the end of 64 slices fit a word
 struct alignas(16) SliceRec {
-    int64_t where;                   // first entry less 4 x quads before it << 27 | lane that brought it << 21 | end
+    int64_t where;                   // first entry less 4 x quads before it << END_BITS + 6 | lane that brought it << END_BITS | end
     double a;                        // A's value
 };
+// ENTRIES of A at a time; slices of MOST entries at most are staged: longer ones only with repeated columns
+template <int ENTRIES, int MOST_, int END_BITS_>
 struct SliceStage {
-    SliceRec rec[SG_T];
-    int first[SG_T];                 // quads of its batch before a slice
+    static constexpr int SLICES = ENTRIES, MOST = MOST_, END_BITS = END_BITS_;
+    static_assert(64ll * MOST < 1ll << END_BITS && END_BITS + 6 + 34 <= 64, "the end of a batch's last slice fits, and a place");
+    SliceRec rec[ENTRIES];
+    int first[ENTRIES];              // quads of its batch before a slice
     uint32_t marks[SG_WAVES][2];     // zero between turns
-    int turns[SG_WAVES];             // of each batch
+    int turns[ENTRIES / 64];         // of each batch
 };
-constexpr size_t DB_LDS = (size_t)SG_CB * 8 + sizeof(SliceStage);
-static_assert(64 * DB_LEN_MOST < 1 << DB_END_BITS, "the end of a batch's last slice fits");
+typedef SliceStage<SG_T, SG_CB, 21> BlockStage;
+constexpr size_t DB_LDS = (size_t)SG_CB * 8 + sizeof(BlockStage);
 static_assert(DB_LDS + 256 <= 160 * 1024, "accumulators and slices fit LDS");
 
 template <typename COL>
@@ -1676,10 +1661,12 @@ struct SliceTurn {
     int pa;                          // the place of a among the row's staged entries
 };
 
-// a lane's slice [lo, hi) of this pass and its entry of A
-__device__ __forceinline__ void slice_put(SliceStage &st, int64_t lo, int64_t hi, double a, int lane, int wave)
+// a lane's slice [lo, hi) of this pass and its entry of A; the wavefronts of the entries that are staged call it
+template <typename STAGE>
+__device__ __forceinline__ void slice_put(STAGE &st, int64_t lo, int64_t hi, double a, int lane, int wave)
 {
-    const int len = hi - lo > DB_LEN_MOST ? DB_LEN_MOST : (int)(hi - lo);
+    constexpr int DB_END_BITS = STAGE::END_BITS;
+    const int len = hi - lo > STAGE::MOST ? STAGE::MOST : (int)(hi - lo);
     const unsigned long long has = __ballot(len > 0);
     const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(has >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)has, 0));
     const int slot = wave * 64 + (len > 0 ? below : __popcll(has) + lane - below);
@@ -1693,13 +1680,15 @@ __device__ __forceinline__ void slice_put(SliceStage &st, int64_t lo, int64_t hi
         st.turns[wave] = (inc + 63) >> 6;
 }
 
-// four(turn) for this wavefront's turns of the staged slices; returns the number of turns of all wavefronts
-template <typename COL, typename FOUR>
-__device__ __forceinline__ int slice_walk(SliceStage &st, const COL *__restrict__ Bcrd, const double *__restrict__ Bval,
+// four(turn) for this wavefront's turns of the staged slices (without VALUES B's are not read); returns the number of turns
+// of all wavefronts
+template <bool VALUES, typename COL, typename STAGE, typename FOUR>
+__device__ __forceinline__ int slice_walk(STAGE &st, const COL *__restrict__ Bcrd, const double *__restrict__ Bval,
                                           int64_t nnz, int lane, int wave, FOUR four)
 {
     typedef typename SgCol4<COL>::type col4;
-    const int own = lane < SG_WAVES ? st.turns[lane] : 0;
+    constexpr int DB_END_BITS = STAGE::END_BITS;
+    const int own = lane < STAGE::SLICES / 64 ? st.turns[lane] : 0;
     const int upto = wave_inclusive_scan(own);
     const int total = __builtin_amdgcn_readlane(upto, 63);
     uint32_t *marks = st.marks[wave];
@@ -1741,8 +1730,10 @@ __device__ __forceinline__ int slice_walk(SliceStage &st, const COL *__restrict_
         }
         t.q = q;
         t.j = *reinterpret_cast<const col4 *>(Bcrd + q);
-        t.v0 = *reinterpret_cast<const sg_d2u *>(Bval + q);
-        t.v1 = *reinterpret_cast<const sg_d2u *>(Bval + q + 2);
+        if constexpr (VALUES) {
+            t.v0 = *reinterpret_cast<const sg_d2u *>(Bval + q);
+            t.v1 = *reinterpret_cast<const sg_d2u *>(Bval + q + 2);
+        }
         wave_lds_order();
     };
     SliceTurn<COL> x, y;
@@ -1855,7 +1846,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
     __shared__ int wave_tot[SG_WAVES];
     __shared__ int ahead_slot;                  // the row's entries ahead of the block
     double *acc = reinterpret_cast<double *>(sg_dyn_lds);
-    SliceStage &st = *reinterpret_cast<SliceStage *>(acc + SG_CB);
+    BlockStage &st = *reinterpret_cast<BlockStage *>(acc + SG_CB);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     for (int j = threadIdx.x; j < SG_CB; j += SG_T)
@@ -1923,7 +1914,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
             const int from0 = sizeof(COL) == 4 ? col0 : 0;
             // the staged slices; what of a slice with repeated columns is not staged is its lane's
             const auto walk = [&](int pa0, int64_t lo, int64_t hi, double a) {
-                const int turns = slice_walk<COL>(st, Bcrd, Bval, Bnnz, lane, wave, [&](const SliceTurn<COL> &t) {
+                const int turns = slice_walk<true, COL>(st, Bcrd, Bval, Bnnz, lane, wave, [&](const SliceTurn<COL> &t) {
                     const int j[4] = {(int)t.j.x, (int)t.j.y, (int)t.j.z, (int)t.j.w};
                     const double b[4] = {t.v0.x, t.v0.y, t.v1.x, t.v1.y};
 #pragma unroll
@@ -1931,7 +1922,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
                         if (t.mask >> x & 1u)
                             block_add<SEMI>(&acc[j[x] - from0], t.a, b[x], pa0 + t.pa + 1, t.q + x, reduce_op, mult_op);
                 });
-                for (int64_t q = lo + DB_LEN_MOST; q < hi; ++q)
+                for (int64_t q = lo + BlockStage::MOST; q < hi; ++q)
                     block_add<SEMI>(&acc[(int)Bcrd[q] - from0], a, Bval[q], pa0 + (int)threadIdx.x + 1, q, reduce_op, mult_op);
                 return turns;
             };
@@ -2047,52 +2038,100 @@ constexpr int SP_BLOCK_WORDS = SG_CB / 32;                // bitmap words of one
 constexpr int SP_WORDS = SP_BLOCKS * SP_BLOCK_WORDS;      // bitmap words of a span
 constexpr int SP_WPT = SP_WORDS / SG_T;                   // consecutive bitmap words per thread
 constexpr int SP_CAP = SG_CB;                             // entries of C per visit at most
-constexpr int SP_CHUNK = 64 * SG_LONG_LOADS;              // entries of a slice that a wavefront takes in one turn
-constexpr size_t SG_SPAN_LDS = (size_t)SP_CAP * 8 + (size_t)SP_WORDS * 4 + (size_t)SP_WORDS * 2;   // values, bitmap, ranks
-static_assert(((size_t)SP_CAP * 8) % 8 == 0 && ((size_t)SP_WORDS * 4) % 4 == 0,
-              "the span kernel's values (fp64) come first in its LDS, bitmap and ranks follow on word boundaries");
+constexpr int SP_ENTRIES = 256;                           // entries of A that are staged at a time
+typedef SliceStage<SP_ENTRIES, SP_BLOCKS * SG_CB, 24> SpanStage;
+constexpr size_t SG_SPAN_LDS = (size_t)SP_CAP * 8 + (size_t)SP_WORDS * 4 + (size_t)SP_WORDS * 2 +       // values, bitmap, ranks
+                               sizeof(SpanStage);
+static_assert(((size_t)SP_WORDS * 6) % 16 == 0, "the values (fp64) come first, the staged slices begin on 16 bytes");
+static_assert(SG_SPAN_LDS + 512 <= 160 * 1024, "all of it fits LDS");
 static_assert(SP_WORDS % SG_T == 0 && SP_BLOCK_WORDS % SP_WPT == 0 && SP_CAP >= SG_CB && SP_CAP <= 65535,
               "a thread's words lie in one block, one block fits the value array, ranks fit 16 bits");
 
 template <bool SEMI>
 __global__ __launch_bounds__(SG_T) void spgemm_numeric_span_kernel(
-    int64_t row_begin, int64_t row_end, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
-    const double *__restrict__ Aval, const int32_t *__restrict__ Bcrd, const double *__restrict__ Bval,
-    const int64_t *__restrict__ blkptr, int nblk,
-    unsigned long long *ticket, RowList list,
+    int64_t row_begin, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
+    const double *__restrict__ Aval, const int32_t *__restrict__ Bcrd, const double *__restrict__ Bval, int64_t Bnnz,
+    const int64_t *__restrict__ blkptr, int nblk, RowList list,
     const int64_t *__restrict__ Cpos, int32_t *__restrict__ Ccrd, double *__restrict__ Cval, int reduce_op,
     int mult_op)
 {
-    __shared__ int64_t row_slot;
     __shared__ int wave_tot[SG_WAVES];
     __shared__ int blk_pre[SP_BLOCKS + 1];      // entries of the span before each of its blocks, and in all
-    __shared__ int span_touched[3];             // see visit_flag below
     double *val = reinterpret_cast<double *>(sg_dyn_lds);
     uint32_t *bm = sg_dyn_lds + SP_CAP * 2;
     uint16_t *pre = reinterpret_cast<uint16_t *>(bm + SP_WORDS);
+    SpanStage &st = *reinterpret_cast<SpanStage *>(pre + SP_WORDS);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     for (int j = threadIdx.x; j < SP_CAP; j += SG_T)
         val[j] = 0.0;
     for (int w = threadIdx.x; w < SP_WORDS; w += SG_T)
         bm[w] = 0;
-    if (threadIdx.x < 3)
-        span_touched[threadIdx.x] = 0;
+    if (lane < 2)
+        st.marks[wave][lane] = 0;
     lds_barrier();
-    int visit = 0;
     const int64_t out0 = Cpos[row_begin];
     int64_t t_first, t_end;
     list_range(list, 4, &t_first, &t_end);
-    int64_t t = draw_row<true>(ticket, t_first, &row_slot);
-    while (t < t_end) {
+    // Rows dealt out in advance: the list goes down by products, so every workgroup gets about the same, and what leads to
+    // a row's slices can be fetched ahead - the bounds of 64 rows at a time, a row's first entries of A two rows ahead and
+    // their slices one.
+    int64_t l_as = 0, l_coff = 0;
+    int l_cnt = 0;
+    const auto load_entry = [&](int r, int base, int &k, double &a) {
+        k = -1;
+        a = 0.0;
+        const int cnt = __builtin_amdgcn_readlane(l_cnt, r & 63);
+        if (r < 64 && (int)threadIdx.x < SP_ENTRIES && base + (int)threadIdx.x < cnt) {
+            const int64_t p = readlane_i64(l_as, r & 63) + base + threadIdx.x;
+            k = Acrd[p];
+            a = Aval[p];
+        }
+    };
+    const auto load_slice = [&](int k, int cbf, int cbt, int64_t &lo, int64_t &hi) {
+        lo = hi = 0;
+        if (k >= 0) {
+            const int64_t *bp = blkptr + (int64_t)k * (nblk + 1);
+            lo = bp[cbf];
+            hi = bp[cbt];
+        }
+    };
+    const auto put = [&](int64_t lo, int64_t hi, double a) {
+        if (wave < SP_ENTRIES / 64)
+            slice_put(st, lo, hi, a, lane, wave);
+    };
+    const int span0 = nblk < SP_BLOCKS ? nblk : SP_BLOCKS;
+    for (int64_t t0 = t_first + blockIdx.x; t0 < t_end; t0 += 64 * (int64_t)gridDim.x) {
+    const int64_t t = t0 + lane * (int64_t)gridDim.x;
+    l_cnt = 0;
+    if (t < t_end) {
         const int64_t i = row_begin + list.rows[t];
-        const int64_t as = Apos[i], ae = Apos[i + 1];
-        if (ae - as == 1) {
+        l_as = Apos[i];
+        l_cnt = (int)(Apos[i + 1] - l_as);               // (the host sends matrices of under 2^30 entries here)
+        l_coff = Cpos[i] - out0;
+    }
+    const int64_t left = (t_end - 1 - t0) / gridDim.x + 1;
+    const int nr = __builtin_amdgcn_readfirstlane((int)(left < 64 ? left : 64));
+    int k0, k1;
+    double a0, a1;
+    int64_t lo0, hi0;
+    load_entry(0, 0, k0, a0);
+    load_entry(1, 0, k1, a1);
+    load_slice(k0, 0, span0, lo0, hi0);
+    for (int r = 0; r < nr; ++r) {
+        int k2;
+        double a2;
+        int64_t lo1, hi1;
+        load_slice(k1, 0, span0, lo1, hi1);
+        load_entry(r + 2, 0, k2, a2);
+        const int64_t as = readlane_i64(l_as, r), coff = readlane_i64(l_coff, r);
+        const int cnt = __builtin_amdgcn_readlane(l_cnt, r);
+        if (cnt == 1) {
             // one entry of A: the row of C is that row of B times the entry (0 + a * b, as an accumulator that
             // starts at zero gives it).  70,000 rows of the R-MAT product at scale 20 are like that, each the
             // copy of a hub's row.
             const int64_t *bp = blkptr + (int64_t)Acrd[as] * (nblk + 1);
-            const int64_t bs = bp[0], len = bp[nblk] - bs, off = Cpos[i] - out0;
+            const int64_t bs = bp[0], len = bp[nblk] - bs, off = coff;
             const double a = Aval[as];
             for (int64_t q = threadIdx.x; q < len; q += SG_T) {
                 store_streaming(&Ccrd[off + q], Bcrd[bs + q]);
@@ -2105,100 +2144,60 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_span_kernel(
                     store_streaming(&Cval[off + q], 0.0 + a * Bval[bs + q]);
                 }
             }
-        } else if (as != ae) {
-            int64_t off = Cpos[i] - out0;
-            // A row of at most one entry of A per lane (nearly all rows) keeps the entry, the place of its block
-            // pointers and the slice of the span in registers; the end of the next span is loaded a visit ahead.
-            // A row of at most 64 entries of A (the usual heavy row that is not wide has 5..140) is held whole by
-            // every wavefront, entry l in lane l, and its slices are dealt to the wavefronts in chunks of
-            // SP_CHUNK entries: with an entry per wavefront, 5 entries would leave 11 wavefronts idle.
-            const int held = __builtin_amdgcn_readfirstlane((int)(ae - as <= SG_T));
-            const int small = __builtin_amdgcn_readfirstlane((int)(ae - as <= 64));
-            double h_a = 0.0;
-            int h_pa = 0;
-            const int64_t *h_bp = nullptr;
-            int64_t h_lo = 0, h_hi = 0;
-            if (held) {
-                const int64_t p = small ? as + lane : as + wave + (int64_t)lane * SG_WAVES;
-                if (p < ae) {
-                    h_bp = blkptr + (int64_t)Acrd[p] * (nblk + 1);
-                    h_a = Aval[p];
-                    h_pa = (int)(p - as + 1);
-                    h_lo = h_bp[0];
-                    h_hi = h_bp[nblk < SP_BLOCKS ? nblk : SP_BLOCKS];
-                }
-            }
-            // f over the products of the row whose columns lie in the blocks [cbf, cbt); a held row's slice of these
-            // blocks is [held_lo, held_hi)
-            const auto walk = [&](int cbf, int cbt, int64_t held_lo, int64_t held_hi, auto values, auto f, auto f4) -> int {
-                constexpr bool VALUES = decltype(values)::value;
-                int touched = 0;
-                if (small) {
-                    const int mine = (int)((held_hi - held_lo + SP_CHUNK - 1) / SP_CHUNK);
-                    const int upto = wave_inclusive_scan(mine);             // chunks of the entries 0..lane
-                    const int chunks = __builtin_amdgcn_readlane(upto, 63);
-                    touched = chunks > 0;
-                    for (int g = wave; g < chunks; g += SG_WAVES) {
-                        const int e = __builtin_ctzll(__ballot(upto > g));   // the entry that chunk g belongs to
-                        const int c = g - (__builtin_amdgcn_readlane(upto, e) - __builtin_amdgcn_readlane(mine, e));
-                        const int64_t s = readlane_i64(held_lo, e) + (int64_t)c * SP_CHUNK;
-                        const int64_t left = readlane_i64(held_hi, e) - s;
-                        if (left >= SP_CHUNK)
-                            full_turn_of_slice<VALUES>(s, lane, readlane_d(h_a, e), __builtin_amdgcn_readlane(h_pa, e), Bcrd,
-                                                       Bval, f4);
-                        else
-                            turn_of_slice<VALUES>(s, lane, left, readlane_d(h_a, e), __builtin_amdgcn_readlane(h_pa, e),
-                                                  Bcrd, Bval, f);
-                    }
-                } else if (held)
-                    touched = for_each_in_slices<VALUES>(held_lo, held_hi, h_a, h_pa, lane, Bcrd, Bval, f, f4);
-                for (int64_t base = as + wave; !held && base < ae; base += (int64_t)SG_WAVES * 64) {
-                    const int64_t left = (ae - base + SG_WAVES - 1) / SG_WAVES;
-                    const int cnt = (int)(left < 64 ? left : 64);
-                    int64_t lo = 0, hi = 0;
-                    double a = 0.0;
-                    int pa = 0;
-                    if (lane < cnt) {
-                        const int64_t p = base + (int64_t)lane * SG_WAVES;
-                        const int64_t *bp = blkptr + (int64_t)Acrd[p] * (nblk + 1);
-                        lo = bp[cbf];
-                        hi = bp[cbt];
-                        a = Aval[p];
-                        pa = (int)(p - as + 1);
-                    }
-                    touched |= for_each_in_slices<VALUES>(lo, hi, a, pa, lane, Bcrd, Bval, f, f4);
-                }
-                return touched;
-            };
+        } else if (cnt > 1) {
+            int64_t off = coff;
             int cb = 0;
             while (cb < nblk) {
                 const int nbv = nblk - cb < SP_BLOCKS ? nblk - cb : SP_BLOCKS;
                 const int col0 = cb << SG_CB_LOG;
-                int64_t h_next = h_hi;      // where the span after this one ends
-                if (h_bp && cb + nbv < nblk)
-                    h_next = h_bp[cb + nbv + SP_BLOCKS < nblk ? cb + nbv + SP_BLOCKS : nblk];
-                const int touched = walk(cb, cb + nbv, h_lo, h_hi, std::false_type{},
-                                         [&](int j, double, double, int, int64_t) {
-                    j -= col0;
-                    atomicOr(&bm[j >> 5], 1u << (j & 31));
-                }, [&](sg_i4u j4, double, sg_d2u, sg_d2u, int, int64_t) {
-                    // four consecutive entries of a sorted row: the bits that fall into one word go there together
-                    const int j[4] = {j4.x - col0, j4.y - col0, j4.z - col0, j4.w - col0};
-                    int w = j[0] >> 5;
-                    uint32_t bits = 1u << (j[0] & 31);
-#pragma unroll
-                    for (int x = 1; x < 4; ++x) {
-                        if ((j[x] >> 5) != w) {
-                            atomicOr(&bm[w], bits);
-                            w = j[x] >> 5;
-                            bits = 0u;
+                // f4(columns, mask, ...) over the products whose columns lie in the blocks [cb, cbt), SP_ENTRIES entries
+                // of A at a time; staged: the slices of the one pass there is are in LDS already.  Returns the turns.
+                const auto walk = [&](int cbt, bool staged, auto values, auto f) -> int {
+                    constexpr bool VALUES = decltype(values)::value;
+                    int turns = 0;
+                    for (int base = 0; base < cnt; base += SP_ENTRIES) {
+                        int k = k0;
+                        double a = a0;
+                        int64_t lo = lo0, hi = hi0;
+                        if (base > 0)
+                            load_entry(r, base, k, a);
+                        if (base > 0 || cb > 0 || cbt != span0)
+                            load_slice(k, cb, cbt, lo, hi);
+                        if (!staged || base > 0) {
+                            put(lo, hi, a);
+                            lds_barrier();
                         }
-                        bits |= 1u << (j[x] & 31);
+                        turns += slice_walk<VALUES, int32_t>(st, Bcrd, Bval, Bnnz, lane, wave, [&](const SliceTurn<int32_t> &u) {
+                            const int j[4] = {u.j.x - col0, u.j.y - col0, u.j.z - col0, u.j.w - col0};
+                            f(j, u.mask, u.a, u.v0, u.v1, base + u.pa + 1, u.q);
+                        });
+                        // what of a slice with repeated columns is not staged is its lane's, one entry at a time
+                        for (int64_t q = lo + SpanStage::MOST; q < hi; ++q) {
+                            const int j[4] = {Bcrd[q] - col0, 0, 0, 0};
+                            f(j, 1u, a, sg_d2u{Bval[q], 0.0}, sg_d2u{0.0, 0.0}, base + (int)threadIdx.x + 1, q);
+                        }
+                        lds_barrier();
                     }
-                    atomicOr(&bm[w], bits);
+                    return turns;
+                };
+                const int any = walk(cb + nbv, false, std::false_type{},
+                                     [&](const int (&j)[4], uint32_t mask, double, sg_d2u, sg_d2u, int, int64_t) {
+                    // entries of a sorted row: the bits that fall into one word go there together
+                    int w = 0;
+                    uint32_t bits = 0u;
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+                        if (mask >> x & 1u) {
+                            if (bits && (j[x] >> 5) != w) {
+                                atomicOr(&bm[w], bits);
+                                bits = 0u;
+                            }
+                            w = j[x] >> 5;
+                            bits |= 1u << (j[x] & 31);
+                        }
+                    if (bits)
+                        atomicOr(&bm[w], bits);
                 });
-                const int any = visit_flag(span_touched, visit, touched, lane);
-                visit = visit == 2 ? 0 : visit + 1;
                 int nb = nbv;
                 if (any) {
                     // ranks: thread t owns the words [SP_WPT * t, SP_WPT * (t + 1))
@@ -2232,14 +2231,8 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_span_kernel(
                     for (int b = 2; b <= nbv; ++b)
                         nb = __builtin_amdgcn_readfirstlane(blk_pre[b]) <= SP_CAP ? b : nb;
                     const int total = __builtin_amdgcn_readfirstlane(blk_pre[nb]);
-                    if (nb < nbv) {              // cut: this visit ends, and the next span starts, at block cb + nb
-                        if (h_bp) {
-                            h_hi = h_bp[cb + nb];
-                            h_next = h_bp[cb + nb + SP_BLOCKS < nblk ? cb + nb + SP_BLOCKS : nblk];
-                        }
-                    }
+                    // (a cut visit ends, and the next span starts, at block cb + nb)
                     const auto add_at_rank = [&](int j, double a, double b, int pa, int64_t q) {
-                        j -= col0;
                         const uint32_t below = bm[j >> 5] & ((1u << (j & 31)) - 1u);
                         const int r = pre[j >> 5] + __popc(below);
                         if constexpr (SEMI)
@@ -2247,14 +2240,14 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_span_kernel(
                         else
                             __hip_atomic_fetch_add(&val[r], a * b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     };
-                    walk(cb, cb + nb, h_lo, h_hi, std::true_type{}, add_at_rank,
-                         [&](sg_i4u j4, double a, sg_d2u v0, sg_d2u v1, int pa, int64_t q) {
-                        add_at_rank(j4.x, a, v0.x, pa, q);
-                        add_at_rank(j4.y, a, v0.y, pa, q + 1);
-                        add_at_rank(j4.z, a, v1.x, pa, q + 2);
-                        add_at_rank(j4.w, a, v1.y, pa, q + 3);
+                    walk(cb + nb, cnt <= SP_ENTRIES && nb == nbv, std::true_type{},
+                         [&](const int (&j)[4], uint32_t mask, double a, sg_d2u v0, sg_d2u v1, int pa, int64_t q) {
+                        const double b[4] = {v0.x, v0.y, v1.x, v1.y};
+#pragma unroll
+                        for (int x = 0; x < 4; ++x)
+                            if (mask >> x & 1u)
+                                add_at_rank(j[x], a, b[x], pa, q + x);
                     });
-                    lds_barrier();
                     for (int q = threadIdx.x; q < total; q += SG_T) {
                         if constexpr (SEMI)
                             store_streaming(&Cval[off + q],
@@ -2285,11 +2278,15 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_span_kernel(
                     off += total;
                 }
                 cb += nb;
-                h_lo = h_hi;
-                h_hi = h_next;
             }
         }
-        t = draw_row<true>(ticket, t_first, &row_slot);
+        k0 = k1;
+        a0 = a1;
+        lo0 = lo1;
+        hi0 = hi1;
+        k1 = k2;
+        a1 = a2;
+    }
     }
 }
 
@@ -3381,7 +3378,11 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     // masked: the rows whose mask row does not fit the slab kernel's hash table take the one-block kernel
     const bool mdense = m && lds_rows && g.lds && getenv("COMET_HIP_SPGEMM_NO_MASKED_DENSE") == nullptr;
     const bool small = dense && b->ncols <= SM_COLS;
-    const SgClasses classes = sg_row_classes(b->ncols, small);
+    SgClasses classes = sg_row_classes(b->ncols, small);
+    // the kernels that stream staged slices take four entries of B at a time and keep a place in B and an end in a word
+    const bool slices = dense && a->nnz < (1ll << 30) && b->nnz >= 4 && b->nnz < SLICE_NNZ_MOST;
+    if (!slices)                 // every heavy row to the kernel that takes the others block by block
+        classes.wide = classes.dense;
     if (dense || mdense)
         COMET_CHK(sg_plan_blocks(b));
     RowList list;
@@ -3437,8 +3438,7 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     COMET_HIPCHK(hipGetLastError());
     // the rows of the one-block kernel block by block (COMET_HIP_SPGEMM_ROW_MAJOR keeps them row by row; the
     // tests run both)
-    const bool by_blocks = dense && a->nnz < (1ll << 30) && b->nnz >= 4 && b->nnz < DB_NNZ_MOST &&
-                           getenv("COMET_HIP_SPGEMM_ROW_MAJOR") == nullptr;
+    const bool by_blocks = slices && getenv("COMET_HIP_SPGEMM_ROW_MAJOR") == nullptr;
     bool ran_blocks = false;
     int64_t *word = nullptr;
     COMET_CHK(mailbox((void **)&word));
@@ -3528,13 +3528,11 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         if (semi) {
             COMET_CHK(sg_allow_lds(spgemm_numeric_span_kernel<true>, SG_SPAN_LDS));
             spgemm_numeric_span_kernel<true><<<cus, block, SG_SPAN_LDS, stream()>>>(
-                rb, re, a->pos, a->crd, a->val, b->crd, b->val, b->sg_blkptr, nblk,
-                tickets + 2, list, Cpos, Ccrd, Cval, reduce_op, mult_op);
+                rb, a->pos, a->crd, a->val, b->crd, b->val, b->nnz, b->sg_blkptr, nblk, list, Cpos, Ccrd, Cval, reduce_op, mult_op);
         } else {
             COMET_CHK(sg_allow_lds(spgemm_numeric_span_kernel<false>, SG_SPAN_LDS));
             spgemm_numeric_span_kernel<false><<<cus, block, SG_SPAN_LDS, stream()>>>(
-                rb, re, a->pos, a->crd, a->val, b->crd, b->val, b->sg_blkptr, nblk,
-                tickets + 2, list, Cpos, Ccrd, Cval, reduce_op, mult_op);
+                rb, a->pos, a->crd, a->val, b->crd, b->val, b->nnz, b->sg_blkptr, nblk, list, Cpos, Ccrd, Cval, reduce_op, mult_op);
         }
         COMET_HIPCHK(hipGetLastError());
     }
