@@ -1638,13 +1638,13 @@ struct alignas(16) SliceRec {
     double a;                        // A's value
 };
 // ENTRIES of A at a time; slices of MOST entries at most are staged: longer ones only with repeated columns
-template <int ENTRIES, int MOST_, int END_BITS_>
+template <int ENTRIES, int MOST_, int END_BITS_, int WAVES_ = SG_WAVES>
 struct SliceStage {
-    static constexpr int SLICES = ENTRIES, MOST = MOST_, END_BITS = END_BITS_;
+    static constexpr int SLICES = ENTRIES, MOST = MOST_, END_BITS = END_BITS_, WAVES = WAVES_;
     static_assert(64ll * MOST < 1ll << END_BITS && END_BITS + 6 + 34 <= 64, "the end of a batch's last slice fits, and a place");
     SliceRec rec[ENTRIES];
     int first[ENTRIES];              // quads of its batch before a slice
-    uint32_t marks[SG_WAVES][2];     // zero between turns
+    uint32_t marks[WAVES][2];        // zero between turns
     int turns[ENTRIES / 64];         // of each batch
 };
 typedef SliceStage<SG_T, SG_CB, 21> BlockStage;
@@ -1736,15 +1736,16 @@ __device__ __forceinline__ int slice_walk(STAGE &st, const COL *__restrict__ Bcr
         }
         wave_lds_order();
     };
+    constexpr int WAVES = STAGE::WAVES;
     SliceTurn<COL> x, y;
     issue(x, wave);
-    issue(y, wave + SG_WAVES);
-    for (int g = wave; g < total; g += 2 * SG_WAVES) {
+    issue(y, wave + WAVES);
+    for (int g = wave; g < total; g += 2 * WAVES) {
         four(x);
-        issue(x, g + 2 * SG_WAVES);
-        if (g + SG_WAVES < total)
+        issue(x, g + 2 * WAVES);
+        if (g + WAVES < total)
             four(y);
-        issue(y, g + 3 * SG_WAVES);
+        issue(y, g + 3 * WAVES);
     }
     return total;
 }
@@ -2830,6 +2831,108 @@ __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
     }
 }
 
+// The structure of the other rows of such a matrix: eight wavefronts to a row, its rows of B streamed as staged slices, and
+// as many workgroups as make 32 wavefronts a CU.  (Sixteen wavefronts, all that a
+// CU then held, a row of B at a time took, us, A*A of 65536 vertices, edge factor 16 971, 30000 and 10 240, 16000 and 8 86,
+// 5000 and 12 48, so 739, 168, 66, 38.)
+constexpr int SMID_T = 512, SMID_WAVES = SMID_T / 64;
+typedef SliceStage<SMID_T, SM_COLS, 23, SMID_WAVES> RowStage;
+__global__ __launch_bounds__(SMID_T, 8) void spgemm_symbolic_rows_kernel(
+    int64_t row_begin, RowList list, int words, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
+    const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd, int64_t Bnnz, int64_t *__restrict__ rowcount)
+{
+    uint32_t *bm = sg_dyn_lds;
+    __shared__ RowStage st;
+    __shared__ int wave_cnt[SMID_WAVES];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    for (int w = threadIdx.x; w < words; w += SMID_T)
+        bm[w] = 0;
+    if (lane < 2)
+        st.marks[wave][lane] = 0;
+    int64_t t_first, t_end;
+    list_range(list, 0, &t_first, &t_end);
+    // rows dealt out in advance, heaviest first; the bounds of 64 at a time, entries of A and their rows of B ahead
+    for (int64_t t0 = t_first + blockIdx.x; t0 < t_end; t0 += 64 * (int64_t)gridDim.x) {
+        const int64_t t = t0 + lane * (int64_t)gridDim.x;
+        int64_t l_as = 0;
+        int l_cnt = 0, l_row = 0;
+        if (t < t_end) {
+            l_row = list.rows[t];
+            l_as = Apos[row_begin + l_row];
+            l_cnt = (int)(Apos[row_begin + l_row + 1] - l_as);
+        }
+        const int64_t left = (t_end - 1 - t0) / gridDim.x + 1;
+        const int nr = __builtin_amdgcn_readfirstlane((int)(left < 64 ? left : 64));
+        const auto load_entry = [&](int r, int base) {
+            const int cnt = __builtin_amdgcn_readlane(l_cnt, r & 63);
+            return r < 64 && base + (int)threadIdx.x < cnt ? Acrd[readlane_i64(l_as, r & 63) + base + threadIdx.x] : -1;
+        };
+        const auto load_row = [&](int k, int64_t &lo, int64_t &hi) {
+            lo = hi = 0;
+            if (k >= 0) {
+                lo = Bpos[k];
+                hi = Bpos[k + 1];
+            }
+        };
+        int k0 = load_entry(0, 0), k1 = load_entry(1, 0);
+        int64_t lo0, hi0;
+        load_row(k0, lo0, hi0);
+        for (int r = 0; r < nr; ++r) {
+            int64_t lo1, hi1;
+            load_row(k1, lo1, hi1);
+            const int k2 = load_entry(r + 2, 0);
+            const int cnt = __builtin_amdgcn_readlane(l_cnt, r);
+            for (int base = 0; base < cnt; base += SMID_T) {
+                int64_t lo = lo0, hi = hi0;
+                if (base > 0)
+                    load_row(load_entry(r, base), lo, hi);
+                slice_put(st, lo, hi, 0.0, lane, wave);
+                lds_barrier();
+                slice_walk<false, int32_t>(st, Bcrd, nullptr, Bnnz, lane, wave, [&](const SliceTurn<int32_t> &u) {
+                    const int j[4] = {u.j.x, u.j.y, u.j.z, u.j.w};
+                    int w = 0;
+                    uint32_t bits = 0u;
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+                        if (u.mask >> x & 1u) {
+                            if (bits && (j[x] >> 5) != w) {
+                                atomicOr(&bm[w], bits);
+                                bits = 0u;
+                            }
+                            w = j[x] >> 5;
+                            bits |= 1u << (j[x] & 31);
+                        }
+                    if (bits)
+                        atomicOr(&bm[w], bits);
+                });
+                for (int64_t q = lo + RowStage::MOST; q < hi; ++q)          // a row of B with repeated columns
+                    atomicOr(&bm[Bcrd[q] >> 5], 1u << (Bcrd[q] & 31));
+                lds_barrier();
+            }
+            int n = 0;
+            for (int w = threadIdx.x; w < words; w += SMID_T) {
+                n += __popc(bm[w]);
+                bm[w] = 0;
+            }
+            n = wave_sum_i32(n);
+            if (lane == 0)
+                wave_cnt[wave] = n;
+            lds_barrier();
+            if (threadIdx.x == 0) {
+                int all = 0;
+                for (int w = 0; w < SMID_WAVES; ++w)
+                    all += wave_cnt[w];
+                rowcount[__builtin_amdgcn_readlane(l_row, r)] = all;
+            }
+            k0 = k1;
+            lo0 = lo1;
+            hi0 = hi1;
+            k1 = k2;
+        }
+    }
+}
+
 template <bool SEMI>
 __global__ __launch_bounds__(SM_T) void spgemm_numeric_small_kernel(
     int64_t row_begin, RowList list, int words, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
@@ -3176,6 +3279,18 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
         KernelTimer t("spgemm_symbolic_small");
         spgemm_symbolic_small_kernel<<<sm_grid(list), dim3(SM_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
             0, list, words, a->pos, a->crd, b->pos, b->crd, rowcount);
+    }
+    if (small && b->nnz >= 4 && b->nnz < SLICE_NNZ_MOST && a->nnz < (1ll << 30)) {
+        if (list.counts[0] != 0) {
+            const int words = sm_words(b->ncols);
+            const int64_t most = (int64_t)num_cus() * 4;
+            const dim3 grid((unsigned)(list.counts[0] < 0 ? most : std::min(most, list.counts[0])));
+            KernelTimer t("spgemm_symbolic");
+            spgemm_symbolic_rows_kernel<<<grid, dim3(SMID_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
+                0, list, words, a->pos, a->crd, b->pos, b->crd, b->nnz, rowcount);
+        }
+        COMET_HIPCHK(hipGetLastError());
+        return COMET_HIP_OK;
     }
     if (small && list.counts[0] == 0) {
         COMET_HIPCHK(hipGetLastError());
