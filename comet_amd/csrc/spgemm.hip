@@ -380,17 +380,21 @@ __device__ inline double wave_sum_f64(double v)
 struct RowList {
     const int32_t *rows;       // row - row_begin, by descending number of products
     const int64_t *bounds;     // [0] rows with >= dense_threshold products, [1] rows with any product,
-                               // [2] rows with >= wide_threshold products (a prefix of [0])
-    int64_t counts[3];         // the same on the host where it has them, else -1
-    // whether the host knows that every row with products is a heavy one (unknown counts are all -1, hence equal)
+                               // [2] rows with >= wide_threshold products (a prefix of [0]),
+                               // [3] rows with >= mid_threshold products ([0] is a prefix of it)
+    int64_t counts[4];         // the same on the host where it has them, else -1
+    // whether the host knows that there are none such (unknown counts are all -1, hence equal)
     bool only_heavy() const { return counts[1] >= 0 && counts[1] == counts[0]; }
+    bool none_small() const { return counts[1] >= 0 && counts[1] == counts[3]; }
+    bool none_mid() const { return counts[0] >= 0 && counts[0] == counts[3]; }
 };
 __device__ inline void list_range(const RowList &l, int part, int64_t *first, int64_t *end)
 {
     // part 0: the heavy rows, 1: the others that have products, 2: both, 3: the widest of the heavy rows,
-    // 4: the heavy rows that are not among the widest
-    *first = part == 1 ? l.bounds[0] : part == 4 ? l.bounds[2] : 0;
-    *end = part == 0 || part == 4 ? l.bounds[0] : part == 3 ? l.bounds[2] : l.bounds[1];
+    // 4: the heavy rows that are not among the widest, 5: the small rows, 6: those between the small and the heavy ones,
+    // 7: all but the small ones
+    *first = part == 1 || part == 6 ? l.bounds[0] : part == 4 ? l.bounds[2] : part == 5 ? l.bounds[3] : 0;
+    *end = part == 0 || part == 4 ? l.bounds[0] : part == 3 ? l.bounds[2] : part == 6 || part == 7 ? l.bounds[3] : l.bounds[1];
 }
 // A workgroup barrier that orders LDS traffic only.  __syncthreads() also makes every wavefront wait until its
 // global stores have been acknowledged, a microsecond that a kernel whose stores nobody reads back (the rows
@@ -2656,20 +2660,24 @@ __global__ void fill_iota_f64(int64_t n, double *__restrict__ out)
 // and values: A*A of R-MAT graphs of 65536 vertices, edge factor 16 96 + 379 -> 56 + 95, 30000 and 10 47 + 156 -> 26 + 48,
 // 16000 and 8 24 + 84 -> 17 + 34, 5000 and 12 17 + 36 -> 10 + 21.
 // ---------------------------------------------------------------------------
-constexpr int SM_T = 256, SM_PRODUCTS = 2048, SM_COLS = 1 << 16;
-constexpr int SM_PER = SM_PRODUCTS / SM_T;          // products of a lane
+constexpr int SM_PER = 8;                           // products of a lane
+constexpr int SM_T = 256, SM_COLS = 1 << 16;
+constexpr int SM_MID_T = 512;                       // the lanes of a workgroup for twice as many
+constexpr int SM_PRODUCTS = SM_PER * SM_T, SM_MID_PRODUCTS = SM_PER * SM_MID_T;
+template <int T>
 struct SmallStage {
-    int64_t start[SM_T];                 // of the entries of A that have any: where their products begin in B, less their
-    double a[SM_T];                      // place among the products; A's value; the entry's place in the row
-    int place[SM_T];
-    uint32_t marks[SM_PRODUCTS / 32];    // a bit where an entry's products begin; zero between passes
-    int tot[2][SM_T / 64];
+    int64_t start[T];                    // of the entries of A that have any: where their products begin in B, less their
+    double a[T];                         // place among the products; A's value; the entry's place in the row
+    int place[T];
+    unsigned long long marks[SM_PER * T / 64];       // a bit where an entry's products begin; zero between passes
+    int tot[2][T / 64];
 };
+template <int T>
 struct SmallRowLds {                     // behind the bitmap
-    double val[SM_PRODUCTS];
-    SmallStage stage;
-    uint16_t col[SM_PRODUCTS];
-    int wave_tot[SM_T / 64];
+    double val[SM_PER * T];
+    SmallStage<T> stage;
+    uint16_t col[SM_PER * T];
+    int wave_tot[T / 64];
 };
 template <bool VALUES>
 struct SmallProducts {
@@ -2679,10 +2687,10 @@ struct SmallProducts {
     int64_t q[VALUES ? SM_PER : 1];      // the place in B
 };
 
-// The lane's products of the entries [p0, ae) of a row of A, SM_T of them at most.  The marks are left set: small_clear
+// The lane's products of the entries [p0, ae) of a row of A, T of them at most.  The marks are left set: small_clear
 // behind the next barrier.
-template <bool VALUES>
-__device__ __forceinline__ void small_products(SmallStage &st, int64_t as, int64_t p0, int64_t ae,
+template <bool VALUES, int T>
+__device__ __forceinline__ void small_products(SmallStage<T> &st, int64_t as, int64_t p0, int64_t ae,
                                                const int32_t *__restrict__ Acrd, const double *__restrict__ Aval,
                                                const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd,
                                                const double *__restrict__ Bval, SmallProducts<VALUES> &out)
@@ -2709,7 +2717,7 @@ __device__ __forceinline__ void small_products(SmallStage &st, int64_t as, int64
     int off = inc - len, slot = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(has >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)has, 0));
     int total = 0;
 #pragma unroll
-    for (int w = 0; w < SM_T / 64; ++w) {
+    for (int w = 0; w < T / 64; ++w) {
         off += w < wave ? st.tot[0][w] : 0;
         slot += w < wave ? st.tot[1][w] : 0;
         total += st.tot[0][w];
@@ -2720,18 +2728,20 @@ __device__ __forceinline__ void small_products(SmallStage &st, int64_t as, int64
             st.a[slot] = a;
             st.place[slot] = (int)(p - as) + 1;
         }
-        atomicOr(&st.marks[off >> 5], 1u << (off & 31));
+        atomicOr(&st.marks[off >> 6], 1ull << (off & 63));
     }
     lds_barrier();
-    static_assert(SM_PRODUCTS / 32 == 64, "a word of marks to a lane");
-    const int word = (int)st.marks[lane], before = wave_inclusive_scan(__popc((uint32_t)word)) - __popc((uint32_t)word);
+    static_assert(SM_PER * T / 64 <= 64, "a word of marks to a lane");
+    const unsigned long long word = lane < SM_PER * T / 64 ? st.marks[lane] : 0;
+    const int before = wave_inclusive_scan(__popcll(word)) - __popcll(word);
 #pragma unroll
     for (int x = 0; x < SM_PER; ++x) {
-        const int t = tid + SM_T * x, w = t >> 5;
-        const int m = lane_value(word, w), c = lane_value(before, w);
+        const int t = tid + T * x, w = t >> 6;
+        const unsigned lo = (unsigned)lane_value((int)word, w), hi = (unsigned)lane_value((int)(word >> 32), w);
+        const int c = lane_value(before, w);
         out.col[x] = -1;
         if (t < total) {
-            const int owner = c + __popc((uint32_t)m & (uint32_t)((2ull << (t & 31)) - 1ull)) - 1;
+            const int owner = c + __popcll(((unsigned long long)hi << 32 | lo) & ((2ull << (t & 63)) - 1ull)) - 1;
             const int64_t q = st.start[owner] + t;
             out.col[x] = Bcrd[q];
             if constexpr (VALUES) {
@@ -2743,16 +2753,18 @@ __device__ __forceinline__ void small_products(SmallStage &st, int64_t as, int64
         }
     }
 }
-__device__ __forceinline__ void small_clear(SmallStage &st)
+template <int T>
+__device__ __forceinline__ void small_clear(SmallStage<T> &st)
 {
-    if (threadIdx.x < SM_PRODUCTS / 32)
+    if (threadIdx.x < SM_PER * T / 64)
         st.marks[threadIdx.x] = 0;
 }
 // before[w] = set bits in front of word w, for a thread's share of the words; returns how many there are
+template <int T>
 __device__ __forceinline__ int small_row_ranks(const uint32_t *bm, uint16_t *before, int words, int *wave_tot)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int per = (words + SM_T - 1) / SM_T, w0 = threadIdx.x * per;
+    const int per = (words + T - 1) / T, w0 = threadIdx.x * per;
     int mine = 0;
     for (int w = w0; w < w0 + per && w < words; ++w)
         mine += __popc(bm[w]);
@@ -2761,7 +2773,7 @@ __device__ __forceinline__ int small_row_ranks(const uint32_t *bm, uint16_t *bef
         wave_tot[wave] = inc;
     lds_barrier();
     int run = inc - mine, all = 0;
-    for (int x = 0; x < SM_T / 64; ++x) {
+    for (int x = 0; x < T / 64; ++x) {
         run += x < wave ? wave_tot[x] : 0;
         all += wave_tot[x];
     }
@@ -2778,11 +2790,11 @@ struct SmallRows {
     const int64_t *Apos;
     int64_t row_begin, t, t_end;
     int64_t r, rn, as, ae;               // this row (counted from row_begin), the next one, this one's entries of A
-    __device__ __forceinline__ SmallRows(const RowList &l, const int64_t *pos, int64_t begin)
+    __device__ __forceinline__ SmallRows(const RowList &l, int part, const int64_t *pos, int64_t begin)
         : list(l), Apos(pos), row_begin(begin)
     {
         int64_t t_first;
-        list_range(list, 1, &t_first, &t_end);
+        list_range(list, part, &t_first, &t_end);
         t = t_first + blockIdx.x;
         r = t < t_end ? list.rows[t] : 0;
         rn = t + gridDim.x < t_end ? list.rows[t + gridDim.x] : r;
@@ -2797,13 +2809,13 @@ __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
     const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd, int64_t *__restrict__ rowcount)
 {
     uint32_t *bm = sg_dyn_lds;
-    __shared__ SmallStage stage;
+    __shared__ SmallStage<SM_T> stage;
     __shared__ int wave_tot[SM_T / 64];
     for (int w = threadIdx.x; w < words; w += SM_T)
         bm[w] = 0;
     small_clear(stage);
     lds_barrier();
-    SmallRows rows(list, Apos, row_begin);
+    SmallRows rows(list, 5, Apos, row_begin);
     while (rows.more()) {
         const int64_t r = rows.r, as = rows.as, ae = rows.ae;
         rows.t += gridDim.x;
@@ -2813,7 +2825,7 @@ __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
         rows.rn = rows.t + gridDim.x < rows.t_end ? list.rows[rows.t + gridDim.x] : rows.rn;
         for (int64_t p0 = as; p0 < ae; p0 += SM_T) {
             SmallProducts<false> it;
-            small_products<false>(stage, as, p0, ae, Acrd, nullptr, Bpos, Bcrd, nullptr, it);
+            small_products<false, SM_T>(stage, as, p0, ae, Acrd, nullptr, Bpos, Bcrd, nullptr, it);
 #pragma unroll
             for (int x = 0; x < SM_PER; ++x)
                 if (it.col[x] >= 0)
@@ -2821,7 +2833,7 @@ __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
             lds_barrier();
             small_clear(stage);
         }
-        const int n = small_row_ranks(bm, nullptr, words, wave_tot);
+        const int n = small_row_ranks<SM_T>(bm, nullptr, words, wave_tot);
         if (threadIdx.x == 0)
             rowcount[r] = n;
         const int per = (words + SM_T - 1) / SM_T;
@@ -2851,7 +2863,7 @@ __global__ __launch_bounds__(SMID_T, 8) void spgemm_symbolic_rows_kernel(
     if (lane < 2)
         st.marks[wave][lane] = 0;
     int64_t t_first, t_end;
-    list_range(list, 0, &t_first, &t_end);
+    list_range(list, 7, &t_first, &t_end);
     // rows dealt out in advance, heaviest first; the bounds of 64 at a time, entries of A and their rows of B ahead
     for (int64_t t0 = t_first + blockIdx.x; t0 < t_end; t0 += 64 * (int64_t)gridDim.x) {
         const int64_t t = t0 + lane * (int64_t)gridDim.x;
@@ -2933,8 +2945,8 @@ __global__ __launch_bounds__(SMID_T, 8) void spgemm_symbolic_rows_kernel(
     }
 }
 
-template <bool SEMI>
-__global__ __launch_bounds__(SM_T) void spgemm_numeric_small_kernel(
+template <bool SEMI, int T>
+__global__ __launch_bounds__(T) void spgemm_numeric_small_kernel(
     int64_t row_begin, RowList list, int words, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
     const double *__restrict__ Aval, const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd,
     const double *__restrict__ Bval, const int64_t *__restrict__ Cpos, int32_t *__restrict__ Ccrd,
@@ -2942,12 +2954,12 @@ __global__ __launch_bounds__(SM_T) void spgemm_numeric_small_kernel(
 {
     uint32_t *bm = sg_dyn_lds;
     uint16_t *before = reinterpret_cast<uint16_t *>(bm + words);
-    SmallRowLds &sh = *reinterpret_cast<SmallRowLds *>(bm + words + words / 2);
-    for (int w = threadIdx.x; w < words + words / 2 + (int)(sizeof sh / 4); w += SM_T)
+    SmallRowLds<T> &sh = *reinterpret_cast<SmallRowLds<T> *>(bm + words + words / 2);
+    for (int w = threadIdx.x; w < words + words / 2 + (int)(sizeof sh / 4); w += T)
         bm[w] = 0;
     lds_barrier();
     const int64_t c0 = Cpos[row_begin];
-    SmallRows rows(list, Apos, row_begin);
+    SmallRows rows(list, T == SM_T ? 5 : 6, Apos, row_begin);
     while (rows.more()) {
         const int64_t as = rows.as, ae = rows.ae, coff = Cpos[row_begin + rows.r] - c0;
         rows.t += gridDim.x;
@@ -2956,8 +2968,8 @@ __global__ __launch_bounds__(SM_T) void spgemm_numeric_small_kernel(
         rows.ae = Apos[row_begin + rows.rn + 1];
         rows.rn = rows.t + gridDim.x < rows.t_end ? list.rows[rows.t + gridDim.x] : rows.rn;
         SmallProducts<true> it;
-        for (int64_t p0 = as; p0 < ae; p0 += SM_T) {
-            small_products<true>(sh.stage, as, p0, ae, Acrd, Aval, Bpos, Bcrd, Bval, it);
+        for (int64_t p0 = as; p0 < ae; p0 += T) {
+            small_products<true, T>(sh.stage, as, p0, ae, Acrd, Aval, Bpos, Bcrd, Bval, it);
 #pragma unroll
             for (int x = 0; x < SM_PER; ++x)
                 if (it.col[x] >= 0)
@@ -2965,11 +2977,11 @@ __global__ __launch_bounds__(SM_T) void spgemm_numeric_small_kernel(
             lds_barrier();
             small_clear(sh.stage);
         }
-        const int total = small_row_ranks(bm, before, words, sh.wave_tot);
+        const int total = small_row_ranks<T>(bm, before, words, sh.wave_tot);
         lds_barrier();
-        for (int64_t p0 = as; p0 < ae; p0 += SM_T) {
-            if (ae - as > SM_T) {          // more entries than lanes: their products once more
-                small_products<true>(sh.stage, as, p0, ae, Acrd, Aval, Bpos, Bcrd, Bval, it);
+        for (int64_t p0 = as; p0 < ae; p0 += T) {
+            if (ae - as > T) {          // more entries than lanes: their products once more
+                small_products<true, T>(sh.stage, as, p0, ae, Acrd, Aval, Bpos, Bcrd, Bval, it);
                 lds_barrier();
                 small_clear(sh.stage);
             }
@@ -2985,7 +2997,7 @@ __global__ __launch_bounds__(SM_T) void spgemm_numeric_small_kernel(
                 }
         }
         lds_barrier();
-        for (int q = threadIdx.x; q < total; q += SM_T) {
+        for (int q = threadIdx.x; q < total; q += T) {
             const int j = sh.col[q];
             Ccrd[coff + q] = j;
             Cval[coff + q] = dense_take<SEMI>(sh.val, q, reduce_op, mult_op, as, Aval, Bval);
@@ -3089,14 +3101,16 @@ __global__ void sg_row_keys(int64_t n, const int64_t *__restrict__ rowprod, cons
 
 // bounds[0] = rows with >= threshold products, bounds[1] = rows with any, bounds[2] = rows with >= wide products,
 // in the sorted key array
-__global__ void sg_row_bounds(int64_t n, const uint64_t *__restrict__ keys, int64_t threshold, int64_t wide,
+__global__ void sg_row_bounds(int64_t n, const uint64_t *__restrict__ keys, int64_t threshold, int64_t wide, int64_t middle,
                               int64_t *__restrict__ bounds)
 {
-    if (threadIdx.x > 2 || blockIdx.x > 0)
+    if (threadIdx.x > 3 || blockIdx.x > 0)
         return;
     // first key that is larger than the limit: keys ascend as products descend
     const uint64_t limit = threadIdx.x == 1 ? (uint64_t)((1ll << 62) - 1)
-                                            : (uint64_t)((1ll << 62) - (threadIdx.x == 0 ? threshold : wide));
+                                            : (uint64_t)((1ll << 62) - (threadIdx.x == 0   ? threshold
+                                                                        : threadIdx.x == 2 ? wide
+                                                                                           : middle));
     int64_t lo = 0, hi = n;
     while (lo < hi) {
         const int64_t mid = (lo + hi) >> 1;
@@ -3121,10 +3135,12 @@ static SgRowLists g_rl;
 constexpr size_t SG_ROW_LISTS_KEPT = 24;
 static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64_t dense_threshold,
                        int64_t wide_threshold, RowList *out, const Csr *long_mask = nullptr,
-                       int64_t mask_fill = 0, bool want_counts = false)
+                       int64_t mask_fill = 0, bool want_counts = false, int64_t mid_threshold = -1)
 {
     for (int64_t &c : out->counts)
         c = -1;
+    if (mid_threshold < 0)
+        mid_threshold = dense_threshold;
     const int64_t n = re - rb;
     const bool keep = getenv("COMET_HIP_SPGEMM_NO_LIST_CACHE") == nullptr;
     Csr *owner = const_cast<Csr *>(a);
@@ -3135,14 +3151,16 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
     key.re = re;
     key.dense_threshold = dense_threshold;
     key.wide_threshold = wide_threshold;
+    key.mid_threshold = mid_threshold;
     key.mask_fill = mask_fill;
     if (keep)
         for (const RowListEntry &e : owner->row_lists)
             if (e.b_uid == key.b_uid && e.mask_uid == key.mask_uid && e.rb == rb && e.re == re &&
-                e.dense_threshold == dense_threshold && e.wide_threshold == wide_threshold && e.mask_fill == mask_fill) {
+                e.dense_threshold == dense_threshold && e.wide_threshold == wide_threshold &&
+                e.mid_threshold == mid_threshold && e.mask_fill == mask_fill) {
                 out->rows = e.rows;
                 out->bounds = e.bounds;
-                std::copy(e.counts, e.counts + 3, out->counts);
+                std::copy(e.counts, e.counts + 4, out->counts);
                 return COMET_HIP_OK;
             }
     COMET_CHK(g_rl.rowprod.ensure(sizeof(int64_t) * (size_t)n, false));
@@ -3150,7 +3168,7 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
     COMET_CHK(g_rl.keys_out.ensure(8 * (size_t)n, false));
     COMET_CHK(g_rl.idx_in.ensure(4 * (size_t)n, false));
     COMET_CHK(g_rl.idx_out.ensure(4 * (size_t)n, false));
-    COMET_CHK(g_rl.bounds.ensure(24, false));
+    COMET_CHK(g_rl.bounds.ensure(32, false));
     int64_t *rowprod = (int64_t *)g_rl.rowprod.ptr;
     {
         KernelTimer t("spgemm_row_products");
@@ -3164,7 +3182,7 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
     COMET_CHK(sort_pairs_u64_u32((const uint64_t *)g_rl.keys_in.ptr, (uint64_t *)g_rl.keys_out.ptr,
                                  (const uint32_t *)g_rl.idx_in.ptr, (uint32_t *)g_rl.idx_out.ptr, n, 63));
     sg_row_bounds<<<dim3(1), dim3(64), 0, stream()>>>(n, (const uint64_t *)g_rl.keys_out.ptr, dense_threshold,
-                                                      wide_threshold, (int64_t *)g_rl.bounds.ptr);
+                                                      wide_threshold, mid_threshold, (int64_t *)g_rl.bounds.ptr);
     COMET_HIPCHK(hipGetLastError());
     out->rows = (const int32_t *)g_rl.idx_out.ptr;
     out->bounds = (const int64_t *)g_rl.bounds.ptr;
@@ -3177,20 +3195,20 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
             owner->row_lists.erase(owner->row_lists.begin());
         }
         if (dev_malloc((void **)&key.rows, 4 * (size_t)n) != hipSuccess ||
-            dev_malloc((void **)&key.bounds, 24) != hipSuccess) {
+            dev_malloc((void **)&key.bounds, 32) != hipSuccess) {
             (void)hipGetLastError();
             (void)dev_free(key.rows);
             return COMET_HIP_OK;
         }
         COMET_HIPCHK(hipMemcpyAsync(key.rows, g_rl.idx_out.ptr, 4 * (size_t)n, hipMemcpyDeviceToDevice, stream()));
-        COMET_HIPCHK(hipMemcpyAsync(key.bounds, g_rl.bounds.ptr, 24, hipMemcpyDeviceToDevice, stream()));
+        COMET_HIPCHK(hipMemcpyAsync(key.bounds, g_rl.bounds.ptr, 32, hipMemcpyDeviceToDevice, stream()));
         if (want_counts) {          // once per list instead of once per product
             int64_t *word = nullptr;
             COMET_CHK(mailbox((void **)&word));
-            COMET_HIPCHK(hipMemcpyAsync(word, key.bounds, 24, hipMemcpyDeviceToHost, stream()));
+            COMET_HIPCHK(hipMemcpyAsync(word, key.bounds, 32, hipMemcpyDeviceToHost, stream()));
             COMET_CHK(stream_wait());
-            std::copy(word, word + 3, key.counts);
-            std::copy(word, word + 3, out->counts);
+            std::copy(word, word + 4, key.counts);
+            std::copy(word, word + 4, out->counts);
         }
         owner->row_lists.push_back(key);
         out->rows = key.rows;
@@ -3230,20 +3248,25 @@ static int64_t sg_wide_threshold(int64_t ncols, int nblk)
 }
 
 // From how many products on a row's values are kept in LDS by the large workgroups, and from how many on block by block.
-struct SgClasses { int64_t dense, wide; };
+// small: the matrix has few enough columns for the kernels of rows with few products; mid and more products are too many
+// for a workgroup of 256 lanes.  Rows of mid up to dense products go to one of 512 lanes: 7000 of the rows of a product of
+// 65536 rows (R-MAT, 16 edges a row), 74 us there and 127 less in the kernel that visits the blocks, 12 and 40 of 980 us
+// in all with 30000 rows.  A matrix of half a block has no such rows: the kernel of whole blocks visits it once.
+struct SgClasses { int64_t mid, dense, wide; };
 static SgClasses sg_row_classes(int64_t ncols, bool small)
 {
     const int nblk = (int)ceil_div(ncols > 0 ? ncols : 1, SG_CB);
     SgClasses c;
-    c.dense = small ? SM_PRODUCTS + 1 : SG_DENSE_PER_BLOCK * nblk;
+    c.dense = !small ? SG_DENSE_PER_BLOCK * nblk : ncols <= SG_NARROW ? SM_PRODUCTS + 1 : SM_MID_PRODUCTS + 1;
+    c.mid = small ? SM_PRODUCTS + 1 : c.dense;
     c.wide = std::max(sg_wide_threshold(ncols, nblk), c.dense);
     return c;
 }
 static int sm_words(int64_t ncols) { return (int)ceil_div(ceil_div(ncols > 0 ? ncols : 1, 32), 4) * 4; }
-static dim3 sm_grid(const RowList &list)
+static dim3 sm_grid(int64_t rows, int per_cu)          // rows < 0: how many is not known
 {
-    const int64_t most = (int64_t)num_cus() * 7;          // workgroups that fit the CUs
-    return dim3((unsigned)(list.counts[0] < 0 ? most : std::min(most, list.counts[1] - list.counts[0])));
+    const int64_t most = (int64_t)num_cus() * per_cu;          // workgroups that fit the CUs
+    return dim3((unsigned)(rows < 0 ? most : std::min(most, rows)));
 }
 
 static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *rowcount)
@@ -3268,31 +3291,31 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
     const bool small = !m && b->ncols <= SM_COLS;
     const SgClasses classes = sg_row_classes(b->ncols, small);
     if (small)          // the list the numeric phase takes
-        COMET_CHK(sg_row_list(a, b, 0, a->nrows, classes.dense, classes.wide, &list, nullptr, 0, true));
+        COMET_CHK(sg_row_list(a, b, 0, a->nrows, classes.dense, classes.wide, &list, nullptr, 0, true, classes.mid));
     else
         COMET_CHK(sg_row_list(a, b, 0, a->nrows, SG_NO_DENSE, SG_NO_DENSE, &list));
     COMET_CHK(g_sg.ticket.ensure(SG_TICKETS * sizeof(unsigned long long), false));
-    sg_clear<<<dim3((unsigned)ceil_div(std::max<int64_t>(a->nrows, SG_TICKETS), 256)), dim3(256), 0, stream()>>>(sg_ticket(0), rowcount,
-                                                                                                    a->nrows);
-    if (small && !list.only_heavy()) {
+    const int64_t words = std::max<int64_t>(a->nrows, SG_TICKETS);
+    sg_clear<<<dim3((unsigned)ceil_div(words, 256)), dim3(256), 0, stream()>>>(sg_ticket(0), rowcount, a->nrows);
+    const bool known = list.counts[0] >= 0;
+    if (small && !list.none_small()) {
         const int words = sm_words(b->ncols);
         KernelTimer t("spgemm_symbolic_small");
-        spgemm_symbolic_small_kernel<<<sm_grid(list), dim3(SM_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
+        const dim3 grid = sm_grid(known ? list.counts[1] - list.counts[3] : -1, 7);
+        spgemm_symbolic_small_kernel<<<grid, dim3(SM_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
             0, list, words, a->pos, a->crd, b->pos, b->crd, rowcount);
     }
     if (small && b->nnz >= 4 && b->nnz < SLICE_NNZ_MOST && a->nnz < (1ll << 30)) {
-        if (list.counts[0] != 0) {
+        if (list.counts[3] != 0) {
             const int words = sm_words(b->ncols);
-            const int64_t most = (int64_t)num_cus() * 4;
-            const dim3 grid((unsigned)(list.counts[0] < 0 ? most : std::min(most, list.counts[0])));
             KernelTimer t("spgemm_symbolic");
-            spgemm_symbolic_rows_kernel<<<grid, dim3(SMID_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
+            spgemm_symbolic_rows_kernel<<<sm_grid(list.counts[3], 4), dim3(SMID_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
                 0, list, words, a->pos, a->crd, b->pos, b->crd, b->nnz, rowcount);
         }
         COMET_HIPCHK(hipGetLastError());
         return COMET_HIP_OK;
     }
-    if (small && list.counts[0] == 0) {
+    if (small && list.counts[3] == 0) {
         COMET_HIPCHK(hipGetLastError());
         return COMET_HIP_OK;
     }
@@ -3308,7 +3331,7 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
         KernelTimer t(M ? "spgemm_symbolic_masked" : "spgemm_symbolic");                                   \
         spgemm_symbolic_kernel<L, M><<<grid, block, g.lds_bytes, stream()>>>(                              \
             a->nrows, a->pos, a->crd, b->pos, b->crd, m ? m->pos : nullptr, m ? m->crd : nullptr, g.logW,  \
-            gbm, (unsigned long long *)g_sg.ticket.ptr, list, small ? 0 : 2, rowcount);                    \
+            gbm, (unsigned long long *)g_sg.ticket.ptr, list, small ? 7 : 2, rowcount);                    \
     } while (0)
     if (g.lds) {
         if (m) LAUNCH_SYM(true, true); else LAUNCH_SYM(true, false);
@@ -3496,7 +3519,7 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     SgClasses classes = sg_row_classes(b->ncols, small);
     // the kernels that stream staged slices take four entries of B at a time and keep a place in B and an end in a word
     const bool slices = dense && a->nnz < (1ll << 30) && b->nnz >= 4 && b->nnz < SLICE_NNZ_MOST;
-    if (!slices)                 // every heavy row to the kernel that takes the others block by block
+    if (!slices)                 // every heavy row to the kernel that takes the widest block by block
         classes.wide = classes.dense;
     if (dense || mdense)
         COMET_CHK(sg_plan_blocks(b));
@@ -3505,7 +3528,7 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         COMET_CHK(sg_row_list(a, b, rb, re, 1ll << 61, 1ll << 61, &list, m, SG_HASH_FILL));
     else
         COMET_CHK(sg_row_list(a, b, rb, re, dense ? classes.dense : SG_NO_DENSE, dense ? classes.wide : SG_NO_DENSE, &list, nullptr,
-                              0, dense));
+                              0, dense, dense ? classes.mid : -1));
     uint32_t *gbm = nullptr, *gmask = nullptr;
     if (!small) {
         if (!g.lds || m) {          // the output row's bitmap is in HBM when LDS holds the mask row instead
@@ -3534,15 +3557,25 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     do {                                                                                                   \
         if (semi) LAUNCH_NUM(L, M, true); else LAUNCH_NUM(L, M, false);                                    \
     } while (0)
-    if (list.only_heavy()) {
-        // nothing for these kernels
-    } else if (small) {
+    if (small) {
         const int words = sm_words(b->ncols);
-        const size_t lds = sizeof(uint32_t) * (size_t)(words + words / 2) + sizeof(SmallRowLds);
-        KernelTimer t(semi ? "spgemm_numeric_semiring" : "spgemm_numeric");
-        const auto kernel = semi ? spgemm_numeric_small_kernel<true> : spgemm_numeric_small_kernel<false>;
-        kernel<<<sm_grid(list), dim3(SM_T), lds, stream()>>>(rb, list, words, a->pos, a->crd, a->val, b->pos, b->crd, b->val, Cpos,
-                                                             Ccrd, Cval, reduce_op, mult_op);
+        const bool known = list.counts[0] >= 0;
+        const auto launch = [&](auto kernel, int lanes, size_t behind, int64_t rows, int per_cu) -> int {
+            const size_t lds = sizeof(uint32_t) * (size_t)(words + words / 2) + behind;
+            KernelTimer t(semi ? "spgemm_numeric_semiring" : "spgemm_numeric");
+            COMET_CHK(sg_allow_lds(kernel, lds));
+            kernel<<<sm_grid(known ? rows : -1, per_cu), dim3(lanes), lds, stream()>>>(
+                rb, list, words, a->pos, a->crd, a->val, b->pos, b->crd, b->val, Cpos, Ccrd, Cval, reduce_op, mult_op);
+            return COMET_HIP_OK;
+        };
+        if (!list.none_small())
+            COMET_CHK(launch(semi ? spgemm_numeric_small_kernel<true, SM_T> : spgemm_numeric_small_kernel<false, SM_T>, SM_T,
+                             sizeof(SmallRowLds<SM_T>), list.counts[1] - list.counts[3], 7));
+        if (classes.mid < classes.dense && !list.none_mid())
+            COMET_CHK(launch(semi ? spgemm_numeric_small_kernel<true, SM_MID_T> : spgemm_numeric_small_kernel<false, SM_MID_T>,
+                             SM_MID_T, sizeof(SmallRowLds<SM_MID_T>), list.counts[3] - list.counts[0], 2));
+    } else if (list.only_heavy()) {
+        // nothing for these kernels
     } else if (g.lds) {
         if (m) LAUNCH_NUM_S(true, true); else LAUNCH_NUM_S(true, false);
     } else {

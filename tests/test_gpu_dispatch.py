@@ -365,6 +365,7 @@ def test_spgemm_rows_with_few_products(ncols, semiring, kept, monkeypatch):
     k, most = 1100, min(ncols, 1000)          # rows of B: two of 1000 entries (if there is room), a hundred of one, others
     b = csr([np.sort(rng.choice(ncols, min(l, ncols), replace=False)) for l in [most] * 2 + [1] * 100 + [7, 15, 16, 17, 64, 513] * 166 + [3] * 2])
     picks = [[], [0], [5], range(102, 110), range(102, 168)] + [[0, 1, *range(2, 2 + n)] for n in (0, 7, 47, 48, 49, 100)]
+    picks += [[0, 1, *range(2, 2 + n), *sorted([*range(107, 125, 6), *range(106, 154, 6)])] for n in (44, 45, 46)]
     a = csr([np.array(p, np.int64) for p in picks * 5])
     A, B = rt.CsrMatrix.from_arrays((5 * len(picks), k), *a), rt.CsrMatrix.from_arrays((k, ncols), *b)
     want = orc.spgemm(*a, *b, ncols, semiring=semiring)
