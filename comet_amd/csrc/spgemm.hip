@@ -1088,13 +1088,11 @@ __device__ __forceinline__ int visit_flag(int *flags, int visit, int touched, in
 
 // Visits the products of one slice per lane: f(j, a, b, pa, q) for the entries [lo, hi) of a row of B (the part of
 // it inside the column block or blocks being swept), j the column, a the entry of A (and pa the tag the caller
-// gave it: its place in the row of A, which only the `any` semiring needs), b the entry of B (0 without VALUES,
-// when the value array is not read) and q its place in B.  Returns whether this wavefront had anything to visit.
+// gave it: its place in the row of A, which only the `any` semiring needs), b the entry of B and q its place there;
+// f4(j, a, v0, v1, pa, q) for four consecutive entries q .. q + 3 of one row of B, columns j, values v0.x, v0.y, v1.x,
+// v1.y.  Returns whether this wavefront had anything to visit.
 
-#ifndef COMET_SG_SHORT
-#define COMET_SG_SHORT 32
-#endif
-constexpr int SG_SHORT = COMET_SG_SHORT;          // slices shorter than this are laid end to end, the others take turns of their own
+constexpr int SG_SHORT = 32;          // slices shorter than this are laid end to end, the others take turns of their own
 constexpr int SG_SHORT_LOADS = 2;                 // entries of the short slices per lane and batch
 constexpr int SG_LONG_LOADS = 4;                  // entries of a long slice per lane and turn
 
@@ -1117,7 +1115,7 @@ struct SgCol4<uint16_t> {
     typedef sg_h4u type;
 };
 
-template <bool VALUES, typename COL, typename F>
+template <typename COL, typename F>
 __device__ __forceinline__ void turn_of_slice(int64_t s, int64_t o, int64_t len, double at, int pt,
                                               const COL *__restrict__ Bcrd, const double *__restrict__ Bval, F f)
 {
@@ -1135,32 +1133,19 @@ __device__ __forceinline__ void turn_of_slice(int64_t s, int64_t o, int64_t len,
         j[x] = ok[x] ? (int)Bcrd[q[x]] : 0;
 #pragma unroll
     for (int x = 0; x < SG_LONG_LOADS; ++x)
-        v[x] = VALUES && ok[x] ? Bval[q[x]] : 0.0;
+        v[x] = ok[x] ? Bval[q[x]] : 0.0;
 #pragma unroll
     for (int x = 0; x < SG_LONG_LOADS; ++x)
         if (ok[x])
             f(j[x], at, v[x], pt, q[x]);
 }
 
-struct SgOneByOne {};          // in place of f4: the four entries of a lane in a full turn go through f one by one
-template <bool VALUES, typename COL, typename F, typename F4 = SgOneByOne>
+template <typename COL, typename F, typename F4>
 __device__ __forceinline__ int for_each_in_slices(int64_t lo, int64_t hi, double a, int pa, int lane,
                                                   const COL *__restrict__ Bcrd,
-                                                  const double *__restrict__ Bval, F f, F4 f4 = F4())
+                                                  const double *__restrict__ Bval, F f, F4 f4)
 {
     typedef typename SgCol4<COL>::type col4;
-    // f4(j, a, v0, v1, pa, q): the four consecutive entries q .. q + 3 of one row of B, columns j, values v0.x, v0.y,
-    // v1.x, v1.y
-    const auto four = [&](col4 j, double at, auto v0, auto v1, int pt, int64_t c) {
-        if constexpr (std::is_same<F4, SgOneByOne>::value) {
-            f((int)j.x, at, v0.x, pt, c);
-            f((int)j.y, at, v0.y, pt, c + 1);
-            f((int)j.z, at, v1.x, pt, c + 2);
-            f((int)j.w, at, v1.y, pt, c + 3);
-        } else {
-            f4(j, at, v0, v1, pt, c);
-        }
-    };
     // Long slices take the whole wavefront, one at a time; short ones (a slice of one block often holds a
     // dozen entries) are laid end to end and dealt to the lanes entry by entry (below).  A wavefront runs its
     // turns one after the other (there is room for one workgroup per CU, so nobody else hides the latency), and
@@ -1190,33 +1175,26 @@ __device__ __forceinline__ int for_each_in_slices(int64_t lo, int64_t hi, double
             static_assert(SG_LONG_LOADS == 4, "a lane's entries of a full turn are one 16-byte load of columns");
             int64_t c = s + 4 * (int64_t)lane;          // this lane's first entry of the turn
             col4 j = *reinterpret_cast<const col4 *>(Bcrd + c);
-            sg_d2u v0 = {0.0, 0.0}, v1 = {0.0, 0.0};
-            if constexpr (VALUES) {
-                v0 = *reinterpret_cast<const sg_d2u *>(Bval + c);
-                v1 = *reinterpret_cast<const sg_d2u *>(Bval + c + 2);
-            }
+            sg_d2u v0 = *reinterpret_cast<const sg_d2u *>(Bval + c), v1 = *reinterpret_cast<const sg_d2u *>(Bval + c + 2);
             int64_t done = 0;
             for (int64_t full = 64 * SG_LONG_LOADS; full + 64 * SG_LONG_LOADS <= len; full += 64 * SG_LONG_LOADS) {
                 const int64_t cn = c + 64 * SG_LONG_LOADS;
                 const col4 jn = *reinterpret_cast<const col4 *>(Bcrd + cn);
-                sg_d2u v0n = {0.0, 0.0}, v1n = {0.0, 0.0};
-                if constexpr (VALUES) {
-                    v0n = *reinterpret_cast<const sg_d2u *>(Bval + cn);
-                    v1n = *reinterpret_cast<const sg_d2u *>(Bval + cn + 2);
-                }
-                four(j, at, v0, v1, pt, c);
+                const sg_d2u v0n = *reinterpret_cast<const sg_d2u *>(Bval + cn);
+                const sg_d2u v1n = *reinterpret_cast<const sg_d2u *>(Bval + cn + 2);
+                f4(j, at, v0, v1, pt, c);
                 j = jn;
                 v0 = v0n;
                 v1 = v1n;
                 c = cn;
                 done += 64 * SG_LONG_LOADS;
             }
-            four(j, at, v0, v1, pt, c);
+            f4(j, at, v0, v1, pt, c);
             done += 64 * SG_LONG_LOADS;
             o += done;
         }
         if (o < len)
-            turn_of_slice<VALUES, COL>(s, o, len, at, pt, Bcrd, Bval, f);
+            turn_of_slice<COL>(s, o, len, at, pt, Bcrd, Bval, f);
     }
     // The short slices are laid end to end and dealt to the lanes entry by entry, 64 at a time, so that every load
     // and every LDS operation has all its lanes (a quarter-wavefront per slice left two thirds of them idle: a
@@ -1250,10 +1228,10 @@ __device__ __forceinline__ int for_each_in_slices(int64_t lo, int64_t hi, double
             }
 #pragma unroll
             for (int x = 0; x < SG_SHORT_LOADS; ++x)
-                j[x] = (ok[x] ? (int)Bcrd[q[x]] : 0);
+                j[x] = ok[x] ? (int)Bcrd[q[x]] : 0;
 #pragma unroll
             for (int x = 0; x < SG_SHORT_LOADS; ++x)
-                v[x] = (VALUES && ok[x] ? Bval[q[x]] : 0.0);
+                v[x] = ok[x] ? Bval[q[x]] : 0.0;
         };
         bool ok[SG_SHORT_LOADS];
         int64_t q[SG_SHORT_LOADS];
@@ -1540,7 +1518,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_kernel(
                     int64_t next = h_hi;
                     if (h_bp && cb + 1 < nblk)
                         next = h_bp[cb + 2];
-                    touched = for_each_in_slices<true>(h_lo, h_hi, h_a, h_pa, lane, Bcrd, Bval, add, add4);
+                    touched = for_each_in_slices(h_lo, h_hi, h_a, h_pa, lane, Bcrd, Bval, add, add4);
                     h_lo = h_hi;
                     h_hi = next;
                 }
@@ -1558,7 +1536,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_kernel(
                         a = Aval[p];
                         pa = (int)(p - as + 1);
                     }
-                    touched |= for_each_in_slices<true>(lo, hi, a, pa, lane, Bcrd, Bval, add, add4);
+                    touched |= for_each_in_slices(lo, hi, a, pa, lane, Bcrd, Bval, add, add4);
                 }
                 const int any = visit_flag(block_touched, visit, touched, lane);
                 visit = visit == 2 ? 0 : visit + 1;

@@ -18,14 +18,6 @@
 
 namespace comet {
 
-__device__ inline double readlane_f64(double v, int lane)
-{
-    int lo = __double2loint(v), hi = __double2hiint(v);
-    lo = __builtin_amdgcn_readlane(lo, lane);
-    hi = __builtin_amdgcn_readlane(hi, lane);
-    return __hiloint2double(hi, lo);
-}
-
 // ============================================================================
 // SpMV: 256 rows per workgroup, one lane per row.  The workgroup streams the
 // contiguous nonzero range of its rows through LDS in passes of SPMV_PASS
