@@ -10,8 +10,9 @@ typedef double pair_d2 __attribute__((ext_vector_type(2), aligned(8)));
 struct DotTurn {
     sg_i4u q;
     pair_d2 lo, hi;
-    uint32_t mask;                       // bits 0-3: which of the four columns are the list's; 4: the list's last quad
+    uint32_t mask;                       // bits 0-3: which of the four columns are the list's
     int owner;                           // the list's lane
+    unsigned long long ends;             // bit l: lane l has its list's last quad in this turn (the same in all lanes)
 };
 
 // 64 lists, one per lane, streamed end to end as in quad_walk
@@ -35,15 +36,16 @@ struct DotLists {
         if (bit < 64u)
             atomicOr(&marks[bit >> 5], 1u << (bit & 31u));
         wave_lds_order();
-        const uint2 m = *reinterpret_cast<const uint2 *>(marks);
+        uint2 m = *reinterpret_cast<const uint2 *>(marks);
         wave_lds_order();
         if (lane < 2)
             marks[lane] = 0;
+        m.x = (uint32_t)__builtin_amdgcn_readfirstlane((int)m.x);
+        m.y = (uint32_t)__builtin_amdgcn_readfirstlane((int)m.y);
         uint32_t from;
         quad_place(m, before, a0, end, 4u * (uint32_t)(base + lane), s.Lnnz - 4u, t.owner, from, t.mask);
         // a mark at a quad is the beginning of the next list behind it
-        const bool last = lane == 63 || ((lane < 32 ? m.x : m.y) >> (lane & 31) & 1u);
-        t.mask |= last ? 16u : 0u;
+        t.ends = (unsigned long long)m.y << 32 | m.x | 1ull << 63;
         t.q = *reinterpret_cast<const sg_i4u *>(s.Lcrd + from);
         t.lo = *reinterpret_cast<const pair_d2 *>(s.Lval + from);
         t.hi = *reinterpret_cast<const pair_d2 *>(s.Lval + from + 2);
@@ -51,22 +53,31 @@ struct DotLists {
     }
 };
 
-// v summed over the lanes of one list (o: the list, ascending over the lanes), complete in the last of them
-__device__ __forceinline__ double list_sum_f64(double v, int o)
+// v summed over the lanes of one list (ends: their last lanes), complete in the last of them.  Which lanes take part in a
+// step is the same for the whole wavefront and costs its vector unit, the busiest part of these kernels, nothing: a bit of
+// a scalar register selects what is added.
+__device__ __forceinline__ double list_sum_f64(double v, unsigned long long ends)
 {
-#define COMET_LIST_STEP(ctrl, rows)                                                                            \
+    const unsigned long long starts = ends << 1;
+    const auto below = [](uint32_t x) { return (x - 1u) & ~x; };          // the bits below the lowest one that is set
+    // bit l: the 1, 2, 4, 8 lanes up to l go on with the list of the lane before each, in the same row of 16 lanes
+    const unsigned long long m1 = ~starts & 0xfffefffefffefffeull, m2 = m1 & m1 << 1, m4 = m2 & m2 << 2, m8 = m4 & m4 << 4;
+    // so do all lanes up to l of an odd row; of the upper half
+    const unsigned long long m16 = (unsigned long long)(below((uint32_t)(starts >> 48)) & 0xffffu) << 48 |
+                                   (unsigned long long)(below((uint32_t)starts >> 16) & 0xffffu) << 16;
+    const unsigned long long m32 = (unsigned long long)below((uint32_t)(starts >> 32)) << 32;
+#define COMET_LIST_STEP(ctrl, lanes)                                                                           \
     {                                                                                                          \
-        const int p = __builtin_amdgcn_update_dpp(-1, o, ctrl, rows, 0xf, false);                              \
-        const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, rows, 0xf, false);              \
-        const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, rows, 0xf, false);              \
-        v += p == o ? __hiloint2double(hi, lo) : 0.0;                                                          \
+        const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, 0xf, 0xf, true);                \
+        const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, 0xf, 0xf, true);                \
+        v += __builtin_amdgcn_inverse_ballot_w64(lanes) ? __hiloint2double(hi, lo) : 0.0;                      \
     }
-    COMET_LIST_STEP(0x111, 0xf)
-    COMET_LIST_STEP(0x112, 0xf)
-    COMET_LIST_STEP(0x114, 0xf)
-    COMET_LIST_STEP(0x118, 0xf)
-    COMET_LIST_STEP(0x142, 0xa)
-    COMET_LIST_STEP(0x143, 0xc)
+    COMET_LIST_STEP(0x111, m1)
+    COMET_LIST_STEP(0x112, m2)
+    COMET_LIST_STEP(0x114, m4)
+    COMET_LIST_STEP(0x118, m8)
+    COMET_LIST_STEP(0x142, m16)
+    COMET_LIST_STEP(0x143, m32)
 #undef COMET_LIST_STEP
     return v;
 }
@@ -109,8 +120,8 @@ __device__ __forceinline__ void dot_turn(const DotTurn &t, const PROBE &probe, d
                 const double e = tv[c] * lv[c];
                 p += met[c] ? e : 0.0;
             }
-            p = list_sum_f64(p, t.owner);
-            if (t.mask & 16u)
+            p = list_sum_f64(p, t.ends);
+            if (__builtin_amdgcn_inverse_ballot_w64(t.ends))
                 acc[t.owner] += p;
         }
         if (any)
@@ -141,20 +152,28 @@ __device__ __forceinline__ void dot_walk(DotLists &lists, const PairSide &s, uin
 }
 
 // ---------------------------------------------------------------------------
-// Rows of long tables: a workgroup per part of a row.  Bound by the lists' way from the memory-side cache (33 GB a call of
-// 200003 vertices, edge factor 16, at 7.7 TB/s; a part of the lists for every XCD found more of them in its L2 but built
-// eight times the tables: 4.0 ms instead of 3.3).  Whole product: n = 200003 21.7 -> 3.6 ms, 20351 0.70 -> 0.24.
+// Rows of long tables: a workgroup per part of a row.  Large graphs are bound by the lists' way from the memory-side cache
+// (33 GB a call of 200003 vertices, edge factor 16, at 7.7 TB/s; a part of the lists for every XCD found more of them in
+// its L2 but built eight times the tables: 4.0 ms instead of 3.3), smaller ones, whose lists the L2 holds, by the vector
+// unit, busy two thirds of the time.  The first item of a workgroup is its own, not drawn: with one word to draw from, the
+// last of 256 began 3 us after the first.  Whole product: n = 200003 21.7 -> 3.6 ms, 20351 0.70 -> 0.24.  With values
+// read from LDS rather than by flat loads, sums over the lanes of a list by scalar masks, and two workgroups to a CU, us:
+// 200003 and 16 3624 -> 3513, 60000 and 12 623 -> 473, 30000 and 8 228 -> 166, 16000 and 16 236 -> 169.
 // The table is a bitmap in LDS with, beside every word (BIG: for
 // every 8 words), the number of entries before it, so that a column's place in the row is that and the bits below; the
 // row's values lie in LDS as well where they fit, behind the table.
 // ---------------------------------------------------------------------------
 typedef const __attribute__((address_space(3))) uint32_t dot_lds_word;
+typedef const __attribute__((address_space(3))) uint64_t dot_lds_pair;
+typedef const __attribute__((address_space(3))) double dot_lds_f64;
 
-template <bool BIG>
+// IN_LDS: the row's values lie at byte vals_at of the LDS, else in memory.  (One pointer to either made every look at a
+// value a flat load, which waits for all loads under way, the next turn's among them.)
+template <bool BIG, bool IN_LDS>
 struct RankProbe {                       // the table at address 0 of the LDS
     const uint32_t *before;              // BIG: of every 8 words
-    bool in_lds;
-    const double *vals, *Tval;           // the row's values in LDS, or in memory
+    uint32_t vals_at;
+    const double *Tval;
     __device__ __forceinline__ void find(const int (&j)[4], uint32_t valid, bool (&met)[4], int (&at)[4]) const
     {
         uint32_t w[4], b[4];
@@ -164,9 +183,9 @@ struct RankProbe {                       // the table at address 0 of the LDS
                 w[c] = *reinterpret_cast<dot_lds_word *>((uint32_t)j[c] >> 5 << 2);
                 b[c] = 0;
             } else {
-                const auto e = reinterpret_cast<dot_lds_word *>((uint32_t)j[c] >> 5 << 3);
-                w[c] = e[0];
-                b[c] = e[1];
+                const uint64_t e = *reinterpret_cast<dot_lds_pair *>((uint32_t)j[c] >> 5 << 3);
+                w[c] = (uint32_t)e;
+                b[c] = (uint32_t)(e >> 32);
             }
         }
 #pragma unroll
@@ -187,22 +206,21 @@ struct RankProbe {                       // the table at address 0 of the LDS
     }
     __device__ __forceinline__ void values(const int (&at)[4], double (&tv)[4]) const
     {
-        if (in_lds) {
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-                tv[c] = vals[at[c]];
-        } else {
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
+        for (int c = 0; c < 4; ++c) {
+            if constexpr (IN_LDS)
+                tv[c] = *reinterpret_cast<dot_lds_f64 *>(vals_at + 8u * (uint32_t)at[c]);
+            else
                 tv[c] = Tval[at[c]];
         }
     }
 };
 
+template <int T>
 struct DotHeavyShared {                  // in LDS behind the table
-    double acc[SG_WAVES][64];
-    uint32_t marks[SG_WAVES][2];
-    int hit[SG_WAVES][64];
+    double acc[T / 64][64];
+    uint32_t marks[T / 64][2];
+    int hit[T / 64][64];
     PairItem slot[2];
     int batch_next;
 };
@@ -217,34 +235,44 @@ constexpr int dot_table_words(int64_t ncols, bool big)
 }
 constexpr bool dot_table_big(int64_t ncols)
 {
-    return sizeof(uint32_t) * (size_t)dot_table_words(ncols, false) + sizeof(DotHeavyShared) > DOT_LDS_MOST;
+    return sizeof(uint32_t) * (size_t)dot_table_words(ncols, false) + sizeof(DotHeavyShared<SG_T>) > DOT_LDS_MOST;
 }
 constexpr int dot_table_words(int64_t ncols) { return dot_table_words(ncols, dot_table_big(ncols)); }
-static_assert(dot_table_words(1 << 20) * sizeof(uint32_t) + sizeof(DotHeavyShared) <= DOT_LDS_MOST,
+static_assert(dot_table_words(1 << 20) * sizeof(uint32_t) + sizeof(DotHeavyShared<SG_T>) <= DOT_LDS_MOST,
               "the table of 2^20 columns fits LDS");
+
+// Two workgroups of half the wavefronts to a CU, one building or clearing its table while the other looks up, where tables
+// are small enough to leave the rows' values room in half the LDS and there are items enough for both.  us of the long
+// rows, two / one: 100000 vertices, edge factor 8 394 / 433, 60000 and 16 524 / 555, 30000 and 8 110 / 128, 16000 and 16
+// 128 / 150; 140000 and 10 1233 / 1088, 200003 and 16 3922 / 3192; few items: 8000 and 6 34 / 29, 5000 and 12 45 / 43.
+constexpr int DOT_TWO_T = 512;
+constexpr int64_t DOT_TWO_COLS = 1 << 17;
+constexpr size_t DOT_TWO_LDS_MOST = 80 * 1024 - 256;
+static_assert(dot_table_words(DOT_TWO_COLS) * sizeof(uint32_t) + sizeof(DotHeavyShared<DOT_TWO_T>) <= DOT_TWO_LDS_MOST / 2,
+              "half of a workgroup's LDS is left for values");
 
 // pair_val, pair_hit: the result of a pair and whether a product met it, at the pair's place.
 // nvals: values of a row that fit LDS behind the shared part
-template <bool BIG, bool SEMI>
-__global__ __launch_bounds__(SG_T) void pair_dot_heavy_kernel(PairSide s0, PairSide s1, int table_words, int before_at, int nvals,
+template <int T, bool BIG, bool SEMI>
+__global__ __launch_bounds__(T, 4) void pair_dot_heavy_kernel(PairSide s0, PairSide s1, int table_words, int before_at, int nvals,
                                                               unsigned long long *__restrict__ tickets,
                                                               double *__restrict__ pair_val,
                                                               uint8_t *__restrict__ pair_hit, DotSemiring op)
 {
     uint32_t *tab = sg_dyn_lds;
-    DotHeavyShared &sh = *reinterpret_cast<DotHeavyShared *>(sg_dyn_lds + table_words);
+    DotHeavyShared<T> &sh = *reinterpret_cast<DotHeavyShared<T> *>(sg_dyn_lds + table_words);
     double *vals = reinterpret_cast<double *>(&sh + 1);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     uint32_t *marks = sh.marks[wave];
     double *acc = sh.acc[wave];
     int *hit = sh.hit[wave];
-    for (int w = threadIdx.x; w < table_words + (int)(sizeof sh / 4); w += SG_T)
+    for (int w = threadIdx.x; w < table_words + (int)(sizeof sh / 4); w += T)
         sg_dyn_lds[w] = 0;
     __syncthreads();
     const uint32_t n0 = (uint32_t)(s0.counts[0] & 0xffffffff), n1 = (uint32_t)(s1.counts[0] & 0xffffffff);
     if (threadIdx.x == 0)
-        sh.slot[0] = pair_item(s0, s1, n0, n1, atomicAdd(&tickets[0], 1ull));
+        sh.slot[0] = pair_item(s0, s1, n0, n1, blockIdx.x);
     __syncthreads();
     PairItem it = pair_item_read(sh.slot[0]);
     int cur = 0;
@@ -252,7 +280,7 @@ __global__ __launch_bounds__(SG_T) void pair_dot_heavy_kernel(PairSide s0, PairS
     while (it.index >= 0) {
         const PairSide s = it.side ? s1 : s0;
         const bool in_lds = it.tlen <= nvals;
-        for (int t = threadIdx.x; t < it.tlen; t += SG_T) {
+        for (int t = threadIdx.x; t < it.tlen; t += T) {
             const int k = s.Tcrd[it.ts + t], prev = t > 0 ? s.Tcrd[it.ts + t - 1] : -1;
             if constexpr (BIG) {
                 atomicOr(&tab[k >> 5], 1u << (k & 31));
@@ -267,14 +295,13 @@ __global__ __launch_bounds__(SG_T) void pair_dot_heavy_kernel(PairSide s0, PairS
                 vals[t] = s.Tval[it.ts + t];
         }
         if (threadIdx.x == 0)
-            sh.batch_next = SG_WAVES;
+            sh.batch_next = T / 64;
         lds_barrier();
         if (threadIdx.x == 0)
-            sh.slot[cur ^ 1] = pair_item(s0, s1, n0, n1, atomicAdd(&tickets[0], 1ull));
-        const RankProbe<BIG> probe{before, in_lds, vals, s.Tval + it.ts};
+            sh.slot[cur ^ 1] = pair_item(s0, s1, n0, n1, gridDim.x + atomicAdd(&tickets[0], 1ull));
         const int mine = (it.kn + it.parts - 1) / it.parts;          // pairs of a part, about
-        int B = mine / (4 * SG_WAVES);
-        B = B > 64 ? 64 : B < 2 ? 2 : B;
+        int B = mine / (4 * (T / 64));
+        B = B > 64 ? 64 : B < 4 ? 4 : B;          // four lists fill a turn or two
         const int nb = (it.kn + B - 1) / B;
         PairEnt e;
         uint32_t place;
@@ -284,31 +311,38 @@ __global__ __launch_bounds__(SG_T) void pair_dot_heavy_kernel(PairSide s0, PairS
             e = s.ent[q];
             place = s.place[q];
         };
-        int j = wave;
-        fetch(j);
-        while (it.part + it.parts * j < nb) {
-            const bool own = lane < B && (int64_t)(it.part + it.parts * j) * B + lane < it.kn;
-            const uint32_t at = place;
-            DotLists lists;
-            lists.take(e.start, own ? (int)e.len : 0);
-            int d = 0;
-            if (lane == 0)
-                d = atomicAdd(&sh.batch_next, 1);
-            j = __builtin_amdgcn_readfirstlane(d);
-            fetch(j);          // the next batch's pairs arrive while this one is walked
-            dot_walk<SEMI>(lists, s, marks, lane, probe, acc, hit, op, it.side != 0);
-            if (own) {
-                pair_hit[at] = (uint8_t)hit[lane];
-                pair_val[at] = SEMI ? semiring_lds_value(reinterpret_cast<unsigned long long *>(acc)[lane], op.reduce_op,
-                                                         op.mult_op, 0, nullptr, nullptr)
-                                    : acc[lane];
+        const auto walk = [&](const auto &probe) {
+            int j = wave;
+            fetch(j);
+            while (it.part + it.parts * j < nb) {
+                const bool own = lane < B && (int64_t)(it.part + it.parts * j) * B + lane < it.kn;
+                const uint32_t at = place;
+                DotLists lists;
+                lists.take(e.start, own ? (int)e.len : 0);
+                int d = 0;
+                if (lane == 0)
+                    d = atomicAdd(&sh.batch_next, 1);
+                j = __builtin_amdgcn_readfirstlane(d);
+                fetch(j);          // the next batch's pairs arrive while this one is walked
+                dot_walk<SEMI>(lists, s, marks, lane, probe, acc, hit, op, it.side != 0);
+                if (own) {
+                    pair_hit[at] = (uint8_t)hit[lane];
+                    pair_val[at] = SEMI ? semiring_lds_value(reinterpret_cast<unsigned long long *>(acc)[lane], op.reduce_op,
+                                                             op.mult_op, 0, nullptr, nullptr)
+                                        : acc[lane];
+                }
+                acc[lane] = 0.0;
+                hit[lane] = 0;
+                wave_lds_order();
             }
-            acc[lane] = 0.0;
-            hit[lane] = 0;
-            wave_lds_order();
-        }
+        };
+        const uint32_t vals_at = (uint32_t)sizeof(uint32_t) * (uint32_t)table_words + (uint32_t)sizeof sh;
+        if (in_lds)
+            walk(RankProbe<BIG, true>{before, vals_at, nullptr});
+        else
+            walk(RankProbe<BIG, false>{before, 0, s.Tval + it.ts});
         lds_barrier();
-        for (int t = threadIdx.x; t < it.tlen; t += SG_T) {
+        for (int t = threadIdx.x; t < it.tlen; t += T) {
             const int k = s.Tcrd[it.ts + t];
             tab[BIG ? k >> 5 : k >> 5 << 1] = 0;
         }
@@ -549,25 +583,30 @@ static int pair_dot_values(Csr *a, Csr *b, Csr *m, int64_t rb, int64_t re, doubl
         const bool big = dot_table_big(a->ncols);
         const int words = dot_table_words(a->ncols);
         const int before_at = (int)ceil_div(a->ncols, 256) * 8;
-        const size_t fixed = sizeof(uint32_t) * (size_t)words + sizeof(DotHeavyShared);
-        const int nvals = (int)((DOT_LDS_MOST - fixed) / sizeof(double)) & ~1;
+        const bool two = a->ncols <= DOT_TWO_COLS && nheavy >= 4 * (int64_t)num_cus();
+        const size_t fixed = sizeof(uint32_t) * (size_t)words + (two ? sizeof(DotHeavyShared<DOT_TWO_T>) : sizeof(DotHeavyShared<SG_T>));
+        const int nvals = (int)(((two ? DOT_TWO_LDS_MOST : DOT_LDS_MOST) - fixed) / sizeof(double)) & ~1;
         const size_t lds = fixed + sizeof(double) * (size_t)nvals;
-        const dim3 grid((unsigned)std::min<int64_t>(nheavy, (int64_t)num_cus())), block(SG_T);
+        const dim3 grid((unsigned)std::min<int64_t>(nheavy, (int64_t)num_cus() * (two ? 2 : 1))), block(two ? DOT_TWO_T : SG_T);
         KernelTimer t("spgemm_numeric_dot");
-#define LAUNCH_DOT(BIG, SEMI)                                                                                          \
+#define LAUNCH_DOT(T, BIG, SEMI)                                                                                       \
     do {                                                                                                               \
-        COMET_CHK(sg_allow_lds(pair_dot_heavy_kernel<BIG, SEMI>, lds));                                                \
-        pair_dot_heavy_kernel<BIG, SEMI><<<grid, block, lds, stream()>>>(s0, s1, words, before_at, nvals, tickets,     \
-                                                                         *pair_val, *pair_hit, op);                               \
+        COMET_CHK(sg_allow_lds(pair_dot_heavy_kernel<T, BIG, SEMI>, lds));                                             \
+        pair_dot_heavy_kernel<T, BIG, SEMI><<<grid, block, lds, stream()>>>(s0, s1, words, before_at, nvals, tickets,  \
+                                                                            *pair_val, *pair_hit, op);                 \
     } while (0)
-        if (big && semi)
-            LAUNCH_DOT(true, true);
+        if (two && semi)
+            LAUNCH_DOT(DOT_TWO_T, false, true);
+        else if (two)
+            LAUNCH_DOT(DOT_TWO_T, false, false);
+        else if (big && semi)
+            LAUNCH_DOT(SG_T, true, true);
         else if (big)
-            LAUNCH_DOT(true, false);
+            LAUNCH_DOT(SG_T, true, false);
         else if (semi)
-            LAUNCH_DOT(false, true);
+            LAUNCH_DOT(SG_T, false, true);
         else
-            LAUNCH_DOT(false, false);
+            LAUNCH_DOT(SG_T, false, false);
 #undef LAUNCH_DOT
         COMET_HIPCHK(hipMemsetAsync(tickets, 0, sizeof *tickets, stream()));
     }

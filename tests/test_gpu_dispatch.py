@@ -378,6 +378,43 @@ def test_spgemm_rows_with_few_products(ncols, semiring, kept, monkeypatch):
             assert np.array_equal(v, want[2])
 
 
+@pytest.mark.parametrize("semiring", [None, ("min", "plus")])
+@pytest.mark.parametrize("rows", [1020, 1030])          # around four to a CU of 256
+@pytest.mark.parametrize("ncols", [1 << 17, (1 << 17) + 1])
+def test_masked_dots_two_workgroups_a_cu(ncols, rows, semiring):
+    # rows of more entries than a wavefront's table holds, as many of them and as many columns as decide whether two
+    # workgroups share a CU; one row whose values fit a whole CU's LDS and not half of it, one that fits neither
+    rng = np.random.default_rng(rows)
+    pool = np.sort(rng.choice(ncols, 16_000, replace=False))
+    pool[-1] = ncols - 1
+    lens = np.full(rows, 200)
+    lens[5], lens[9], lens[11] = 6000, 16_000, 0
+    apos = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    acrd = np.concatenate([np.sort(rng.choice(pool, l, replace=False)) for l in lens]).astype(np.int64)
+    m = 70
+    near = np.unique(np.concatenate([acrd[apos[r]:apos[r + 1]][:40] for r in range(0, rows, 20)]))
+    bcols = [np.sort(rng.choice(near, l, replace=False)) for l in rng.integers(0, 199, m)]
+    k = np.concatenate(bcols)
+    order = np.lexsort((np.repeat(np.arange(m), [len(c) for c in bcols]), k))
+    bcrd = np.repeat(np.arange(m), [len(c) for c in bcols])[order].astype(np.int64)
+    bpos = np.concatenate([[0], np.cumsum(np.bincount(k, minlength=ncols))]).astype(np.int64)
+    keep = rng.random((rows, m)) < 0.8
+    mpos = np.concatenate([[0], np.cumsum(keep.sum(1))]).astype(np.int64)
+    mcrd = np.nonzero(keep)[1].astype(np.int64)
+    a, b = (apos, acrd, rng.uniform(0.5, 1.5, len(acrd))), (bpos, bcrd, rng.uniform(0.5, 1.5, len(bcrd)))
+    A, B = rt.CsrMatrix.from_arrays((rows, ncols), *a), rt.CsrMatrix.from_arrays((ncols, m), *b)
+    M = rt.CsrMatrix.from_arrays((rows, m), mpos, mcrd, np.ones(len(mcrd)))
+    want = orc.spgemm(*a, *b, m, mask=(mpos, mcrd), semiring=semiring)
+    assert want[0][-1] > 1000
+    for _ in range(2):
+        p, c, v = rt.spgemm(A, B, M, semiring=semiring).to_arrays()
+        assert np.array_equal(p, want[0]) and np.array_equal(c, want[1])
+        if semiring is None:          # positive terms, 198 at most
+            assert np.all(np.abs(v - want[2]) <= 200 * 2.0 ** -53 * want[2])
+        else:
+            assert np.array_equal(v, want[2])
+
+
 @pytest.mark.parametrize("semiring", [None, ("min", "plus"), ("max", "times"), ("any", "second"), ("plus", "first")])
 @pytest.mark.parametrize("repeats", [1, 40])
 def test_spgemm_block_by_block_slices(semiring, repeats, monkeypatch):
