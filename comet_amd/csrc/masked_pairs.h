@@ -516,7 +516,7 @@ __global__ __launch_bounds__(SG_T) void pair_sum_heavy_kernel(PairSide s0, PairS
     __syncthreads();
     const uint32_t n0 = (uint32_t)(s0.counts[0] & 0xffffffff), n1 = (uint32_t)(s1.counts[0] & 0xffffffff);
     if (threadIdx.x == 0)
-        sh.slot[0] = pair_item(s0, s1, n0, n1, atomicAdd(&tickets[0], 1ull));
+        sh.slot[0] = pair_item(s0, s1, n0, n1, blockIdx.x);
     __syncthreads();
     PairItem it = pair_item_read(sh.slot[0]);
     int cur = 0;
@@ -533,7 +533,7 @@ __global__ __launch_bounds__(SG_T) void pair_sum_heavy_kernel(PairSide s0, PairS
             sh.batch_next = SG_WAVES;
         lds_barrier();
         if (threadIdx.x == 0)
-            sh.slot[cur ^ 1] = pair_item(s0, s1, n0, n1, atomicAdd(&tickets[0], 1ull));
+            sh.slot[cur ^ 1] = pair_item(s0, s1, n0, n1, gridDim.x + atomicAdd(&tickets[0], 1ull));
         // batches of 64 pairs, or fewer where that leaves the wavefronts less than four each
         const int mine = (it.kn + it.parts - 1) / it.parts;          // pairs of a part, about
         int B = mine / (4 * SG_WAVES);

@@ -308,7 +308,7 @@ __global__ __launch_bounds__(SG_T) void tri_heavy_kernel(PairSide s, int nwords,
     __syncthreads();
     const uint32_t n = (uint32_t)(s.counts[0] & 0xffffffff);
     if (threadIdx.x == 0)
-        sh.slot[0] = pair_item(s, s, n, 0, atomicAdd(&tickets[0], 1ull));
+        sh.slot[0] = pair_item(s, s, n, 0, blockIdx.x);
     __syncthreads();
     PairItem it = pair_item_read(sh.slot[0]);
     int cur = 0;
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(SG_T) void tri_heavy_kernel(PairSide s, int nwords,
             sh.batch_next = SG_WAVES;
         lds_barrier();
         if (threadIdx.x == 0)
-            sh.slot[cur ^ 1] = pair_item(s, s, n, 0, atomicAdd(&tickets[0], 1ull));
+            sh.slot[cur ^ 1] = pair_item(s, s, n, 0, gridDim.x + atomicAdd(&tickets[0], 1ull));
         const int mine = (it.kn + it.parts - 1) / it.parts;          // pairs of a part, about
         int B = mine / (4 * SG_WAVES);
         B = B > 64 ? 64 : B < 2 ? 2 : B;
