@@ -1865,7 +1865,9 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
     lds_barrier();
     const int64_t nchunks = (nd + rows_each - 1) / rows_each;
     const int64_t u_end = ALONE ? nchunks : nchunks * nblk;
-    int64_t u = draw_row<true>(ticket, 0, &row_slot);
+    // (ALONE: the first by number - 256 draws from one word take 3 us; the others' order is what lets a block wait for the
+    // one before it)
+    int64_t u = ALONE ? (int64_t)blockIdx.x : draw_row<true>(ticket, 0, &row_slot);
     while (u < u_end) {
         const int cb = ALONE ? 0 : (int)(u / nchunks);
         const int64_t r0 = (u - cb * nchunks) * rows_each;
@@ -2027,7 +2029,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
             k1 = k2;
             a1 = a2;
         }
-        u = draw_row<true>(ticket, 0, &row_slot);
+        u = draw_row<true>(ticket, ALONE ? gridDim.x : 0, &row_slot);
     }
 }
 
