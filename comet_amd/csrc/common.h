@@ -159,6 +159,10 @@ struct Csr {
     // of row k whose column is >= cb * 2^14, so that the slice of a row inside one block of 16384 columns is
     // found without searching.
     int64_t *sg_blkptr = nullptr;
+    // and for its structure, one allocation: bitmaps of its longest rows, 16 bytes at a time, which rows they are of, and
+    // for every row the number of its bitmap or -1
+    uint32_t *sg_hub_bits = nullptr;
+    int32_t *sg_hub_slot = nullptr;
     int sg_nblk = 0;
     uint16_t *sg_crd16 = nullptr;            // the columns inside their block of 2^14 (null: not kept)
     // SpMM plan for long rows (heavy_state: 0 undecided, 1 not worth it, 2 in use): the long rows re-stored as

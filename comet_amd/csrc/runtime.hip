@@ -433,6 +433,9 @@ static void csr_drop_plans(Csr *c)
     (void)dev_free(c->sg_blkptr);
     (void)dev_free(c->sg_crd16);
     c->sg_blkptr = nullptr;
+    (void)dev_free(c->sg_hub_bits);
+    c->sg_hub_bits = nullptr;
+    c->sg_hub_slot = nullptr;
     c->sg_crd16 = nullptr;
     c->sg_nblk = 0;
     (void)dev_free(c->spmv_bpos);

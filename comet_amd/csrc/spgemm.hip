@@ -2855,19 +2855,66 @@ __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
 // 5000 and 12 48, so 739, 168, 66, 38.)
 constexpr int SMID_T = 512, SMID_WAVES = SMID_T / 64;
 typedef SliceStage<SMID_T, SM_COLS, 23, SMID_WAVES> RowStage;
+// The longest rows of B, a sixty-fourth of the columns and more, are taken as bitmaps, 16 bytes to a lane, which keeps its
+// words of the row in registers: of A*A of 65536 vertices, edge factor 16, 137 of them hold 834 of 1236 M products.  us, this
+// phase without them, with rows from a 32nd, a 64th and a 128th of the columns on: 65536 and 16 736, 565, 472, 514; 30000
+// and 10 158, 150, 134, 157; 20000 and 12 152, 129, 131, 141; 16000 and 8 62, 60, 61, 76.
+constexpr int SMID_HUB_PART = 64, SMID_HUBS = 4;          // so many at a time
+static_assert(SM_COLS / 32 <= SMID_T * 4, "a lane has four words of a bitmap");
+__global__ void spgemm_hub_rows(int64_t nrows, const int64_t *__restrict__ Bpos, int64_t least, int32_t *__restrict__ slot,
+                                int32_t *__restrict__ hub, int32_t *__restrict__ hubs)
+{
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= nrows)
+        return;
+    int s = -1;
+    if (Bpos[k + 1] - Bpos[k] >= least) {
+        s = atomicAdd(hubs, 1);
+        hub[s] = (int32_t)k;
+    }
+    slot[k] = s;
+}
+__global__ __launch_bounds__(256) void spgemm_hub_bits(const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd,
+                                                       const int32_t *__restrict__ hub, const int32_t *__restrict__ hubs,
+                                                       int words, uint32_t *__restrict__ bits)
+{
+    __shared__ uint32_t bm[SM_COLS / 32];
+    const int n = *hubs;
+    for (int s = blockIdx.x; s < n; s += gridDim.x) {
+        for (int w = threadIdx.x; w < words; w += 256)
+            bm[w] = 0;
+        __syncthreads();
+        const int64_t end = Bpos[hub[s] + 1];
+        for (int64_t q = Bpos[hub[s]] + threadIdx.x; q < end; q += 256)
+            atomicOr(&bm[Bcrd[q] >> 5], 1u << (Bcrd[q] & 31));
+        __syncthreads();
+        for (int w = threadIdx.x; w < words; w += 256)
+            bits[(int64_t)s * words + w] = bm[w];
+        __syncthreads();
+    }
+}
+
+// HUBS: with such bitmaps (hub_slot, hub_bits; else null)
+template <bool HUBS>
 __global__ __launch_bounds__(SMID_T, 8) void spgemm_symbolic_rows_kernel(
     int64_t row_begin, RowList list, int words, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
-    const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd, int64_t Bnnz, int64_t *__restrict__ rowcount)
+    const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd, int64_t Bnnz, const int32_t *__restrict__ hub_slot,
+    const uint4 *__restrict__ hub_bits, int64_t *__restrict__ rowcount)
 {
     uint32_t *bm = sg_dyn_lds;
     __shared__ RowStage st;
-    __shared__ int wave_cnt[SMID_WAVES];
+    __shared__ int wave_cnt[SMID_WAVES], hub[HUBS ? SMID_T : 1], hubs[2];
+    const bool mine = (int)threadIdx.x < words / 4;          // four words of a bitmap
+    int pass = 0;
+    if (threadIdx.x < 2)
+        hubs[threadIdx.x] = 0;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     for (int w = threadIdx.x; w < words; w += SMID_T)
         bm[w] = 0;
     if (lane < 2)
         st.marks[wave][lane] = 0;
+    lds_barrier();          // the first pass counts its hubs before its own
     int64_t t_first, t_end;
     list_range(list, 7, &t_first, &t_end);
     // rows dealt out in advance, heaviest first; the bounds of 64 at a time, entries of A and their rows of B ahead
@@ -2886,27 +2933,66 @@ __global__ __launch_bounds__(SMID_T, 8) void spgemm_symbolic_rows_kernel(
             const int cnt = __builtin_amdgcn_readlane(l_cnt, r & 63);
             return r < 64 && base + (int)threadIdx.x < cnt ? Acrd[readlane_i64(l_as, r & 63) + base + threadIdx.x] : -1;
         };
-        const auto load_row = [&](int k, int64_t &lo, int64_t &hi) {
+        const auto load_row = [&](int k, int64_t &lo, int64_t &hi, int &slot) {
             lo = hi = 0;
+            slot = -1;
             if (k >= 0) {
                 lo = Bpos[k];
                 hi = Bpos[k + 1];
+                if constexpr (HUBS)
+                    slot = hub_slot[k];
             }
         };
-        int k0 = load_entry(0, 0), k1 = load_entry(1, 0);
+        int k0 = load_entry(0, 0), k1 = load_entry(1, 0), slot0;
         int64_t lo0, hi0;
-        load_row(k0, lo0, hi0);
+        load_row(k0, lo0, hi0, slot0);
         for (int r = 0; r < nr; ++r) {
             int64_t lo1, hi1;
-            load_row(k1, lo1, hi1);
+            int slot1;
+            load_row(k1, lo1, hi1, slot1);
             const int k2 = load_entry(r + 2, 0);
             const int cnt = __builtin_amdgcn_readlane(l_cnt, r);
+            uint4 own = make_uint4(0, 0, 0, 0);
             for (int base = 0; base < cnt; base += SMID_T) {
                 int64_t lo = lo0, hi = hi0;
+                int slot = slot0;
                 if (base > 0)
-                    load_row(load_entry(r, base), lo, hi);
+                    load_row(load_entry(r, base), lo, hi, slot);
+                if (slot >= 0)
+                    hi = lo;
                 slice_put(st, lo, hi, 0.0, lane, wave);
+                if constexpr (HUBS) {
+                    const unsigned long long has = __ballot(slot >= 0);
+                    if (has) {
+                        int first = 0;
+                        if (lane == 0)
+                            first = atomicAdd(&hubs[pass], __popcll(has));
+                        first = __builtin_amdgcn_readfirstlane(first);
+                        if (slot >= 0)
+                            hub[__builtin_amdgcn_mbcnt_hi((uint32_t)(has >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)has, first))] = slot;
+                    }
+                }
                 lds_barrier();
+                if constexpr (HUBS) {
+                    const int nh = __builtin_amdgcn_readfirstlane(hubs[pass]);
+                    pass ^= 1;
+                    if (threadIdx.x == 0)
+                        hubs[pass] = 0;
+                    for (int h = 0; h < nh; h += SMID_HUBS) {
+                        const int which = hub[h + (lane < SMID_HUBS && h + lane < nh ? lane : 0)];          // past the last one, h again
+                        uint4 v[SMID_HUBS];
+    #pragma unroll
+                        for (int x = 0; x < SMID_HUBS; ++x)
+                            v[x] = hub_bits[(int64_t)__builtin_amdgcn_readlane(which, x) * (words / 4) + (mine ? threadIdx.x : 0)];
+    #pragma unroll
+                        for (int x = 0; x < SMID_HUBS; ++x) {
+                            own.x |= v[x].x;
+                            own.y |= v[x].y;
+                            own.z |= v[x].z;
+                            own.w |= v[x].w;
+                        }
+                    }
+                }
                 slice_walk<false, false, int32_t>(st, Bcrd, nullptr, Bnnz, lane, wave, [&](const SliceTurn<int32_t> &u) {
                     const int j[4] = {u.j.x, u.j.y, u.j.z, u.j.w};
                     int w = 0;
@@ -2929,9 +3015,11 @@ __global__ __launch_bounds__(SMID_T, 8) void spgemm_symbolic_rows_kernel(
                 lds_barrier();
             }
             int n = 0;
-            for (int w = threadIdx.x; w < words; w += SMID_T) {
-                n += __popc(bm[w]);
-                bm[w] = 0;
+            if (mine) {
+                uint4 &at = reinterpret_cast<uint4 *>(bm)[threadIdx.x];
+                const uint4 b = at;
+                at = make_uint4(0, 0, 0, 0);
+                n = __popc(b.x | own.x) + __popc(b.y | own.y) + __popc(b.z | own.z) + __popc(b.w | own.w);
             }
             n = wave_sum_i32(n);
             if (lane == 0)
@@ -2946,6 +3034,7 @@ __global__ __launch_bounds__(SMID_T, 8) void spgemm_symbolic_rows_kernel(
             k0 = k1;
             lo0 = lo1;
             hi0 = hi1;
+            slot0 = slot1;
             k1 = k2;
         }
     }
@@ -3275,6 +3364,32 @@ static dim3 sm_grid(int64_t rows, int per_cu)          // rows < 0: how many is 
     return dim3((unsigned)(rows < 0 ? most : std::min(most, rows)));
 }
 
+// The bitmaps of b's long rows, words to each; a matrix of few columns or none such rows goes without, and so does one for
+// which there is no memory.
+static int sg_plan_hubs(Csr *b, int words)
+{
+    const int64_t least = ceil_div(b->ncols, SMID_HUB_PART);
+    if (b->sg_hub_bits || b->ncols <= SG_NARROW || b->nrows >= 1ll << 31 || b->nnz < least)
+        return COMET_HIP_OK;
+    const int64_t most = std::min(b->nnz / least, b->nrows);
+    const size_t bits = sizeof(uint32_t) * (size_t)words * (size_t)most;
+    if (dev_malloc((void **)&b->sg_hub_bits, bits + sizeof(int32_t) * (size_t)(b->nrows + most + 1)) != hipSuccess) {
+        (void)hipGetLastError();        // an allocation that may fail: its error must not reach the next check
+        b->sg_hub_bits = nullptr;
+        return COMET_HIP_OK;
+    }
+    b->sg_hub_slot = (int32_t *)((char *)b->sg_hub_bits + bits);
+    int32_t *hub = b->sg_hub_slot + b->nrows, *hubs = hub + most;
+    KernelTimer t("spgemm_hub_bits");
+    COMET_HIPCHK(hipMemsetAsync(hubs, 0, sizeof(int32_t), stream()));
+    spgemm_hub_rows<<<dim3((unsigned)ceil_div(b->nrows, 256)), dim3(256), 0, stream()>>>(b->nrows, b->pos, least, b->sg_hub_slot,
+                                                                                       hub, hubs);
+    spgemm_hub_bits<<<dim3((unsigned)std::min<int64_t>(most, 2 * (int64_t)num_cus())), dim3(256), 0, stream()>>>(
+        b->pos, b->crd, hub, hubs, words, b->sg_hub_bits);
+    COMET_HIPCHK(hipGetLastError());
+    return COMET_HIP_OK;
+}
+
 static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *rowcount)
 {
     bool dots = false;
@@ -3314,9 +3429,12 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
     if (small && b->nnz >= 4 && b->nnz < SLICE_NNZ_MOST && a->nnz < (1ll << 30)) {
         if (list.counts[3] != 0) {
             const int words = sm_words(b->ncols);
+            Csr *right = const_cast<Csr *>(b);           // what is kept in a handle is not part of the matrix
+            COMET_CHK(sg_plan_hubs(right, words));
             KernelTimer t("spgemm_symbolic");
-            spgemm_symbolic_rows_kernel<<<sm_grid(list.counts[3], 4), dim3(SMID_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
-                0, list, words, a->pos, a->crd, b->pos, b->crd, b->nnz, rowcount);
+            const auto kernel = b->sg_hub_bits ? spgemm_symbolic_rows_kernel<true> : spgemm_symbolic_rows_kernel<false>;
+            kernel<<<sm_grid(list.counts[3], 4), dim3(SMID_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
+                0, list, words, a->pos, a->crd, b->pos, b->crd, b->nnz, b->sg_hub_slot, (const uint4 *)b->sg_hub_bits, rowcount);
         }
         COMET_HIPCHK(hipGetLastError());
         return COMET_HIP_OK;

@@ -378,6 +378,31 @@ def test_spgemm_rows_with_few_products(ncols, semiring, kept, monkeypatch):
             assert np.array_equal(v, want[2])
 
 
+@pytest.mark.parametrize("ncols", [8192, 8193, 20_011, 65_535, 65_536])
+def test_spgemm_structure_of_rows_with_long_rows_of_b(ncols):
+    # rows of B around a sixty-fourth of the columns, the first and the last column among them, some with every column
+    # twice; rows of A with none to nine of those, beyond the 512 entries that are looked at together, and with nothing else
+    rng = np.random.default_rng(ncols)
+    least = -(-ncols // 64)
+    lens = np.array([least - 1, least, least + 1, 4 * least, ncols // 2, 0] * 2 + [7] * 900)
+    cols = [np.sort(rng.choice(ncols, l, replace=False)) for l in lens]
+    cols[1][0], cols[2][-1] = 0, ncols - 1
+    cols[7] = np.repeat(np.sort(rng.choice(ncols, least, replace=False)), 2)
+    bpos = np.concatenate([[0], np.cumsum([len(c) for c in cols])]).astype(np.int64)
+    b = (bpos, np.concatenate(cols).astype(np.int64), rng.uniform(0.5, 1.5, bpos[-1]))
+    picks = [range(h, 12) for h in range(13)] + [[*range(h), *range(12, 12 + n)] for h in (0, 3, 9, 12) for n in (300, 511, 512, 513, 800)]
+    picks += [[0, 6, *range(12, 700)], [1, 3, 4, 5, *range(300, 912)]]
+    apos = np.concatenate([[0], np.cumsum([len(p) for p in picks])]).astype(np.int64)
+    acrd = np.concatenate([np.array(p, np.int64) for p in picks])
+    a = (apos, acrd, rng.uniform(0.5, 1.5, len(acrd)))
+    A, B = rt.CsrMatrix.from_arrays((len(picks), len(lens)), *a), rt.CsrMatrix.from_arrays((len(lens), ncols), *b)
+    want = orc.spgemm(*a, *b, ncols)
+    for _ in range(2):
+        p, c, v = rt.spgemm(A, B).to_arrays()
+        assert np.array_equal(p, want[0]) and np.array_equal(c, want[1])
+        assert np.all(np.abs(v - want[2]) <= 1e-12 * want[2])
+
+
 @pytest.mark.parametrize("semiring", [None, ("min", "plus")])
 @pytest.mark.parametrize("rows", [1020, 1030])          # around four to a CU of 256
 @pytest.mark.parametrize("ncols", [1 << 17, (1 << 17) + 1])
