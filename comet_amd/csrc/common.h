@@ -25,6 +25,23 @@ int ensure_init();
 int spmm_static_setup(int device);
 bool is_initialised();     // has any call brought the device up yet
 int set_error(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
+// While one is alive, this thread's errors are answered by the caller in another way: COMET_HIP_ABORT_ON_ERROR does not
+// end the process for them.
+struct ErrorsAnswered {
+    ErrorsAnswered();
+    ~ErrorsAnswered();
+};
+// A plan that a call can do without: false where it could not be made, for want of memory as a rule, and nothing is left
+// of the error.
+template <typename PLAN>
+static inline bool plan_made(PLAN make)
+{
+    ErrorsAnswered here;
+    if (make() == COMET_HIP_OK)
+        return true;
+    (void)hipGetLastError();
+    return false;
+}
 int num_cus();
 // comet_hip_finalize destroys every handle: the two places that keep one between calls drop theirs
 void forget_pending_reads();       // formats.hip: reader "sizes" call -> "read" call

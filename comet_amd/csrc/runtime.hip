@@ -47,6 +47,10 @@ int aux_join()
 }
 int num_cus() { return g_num_cus; }
 
+static thread_local int g_answered = 0;
+ErrorsAnswered::ErrorsAnswered() { ++g_answered; }
+ErrorsAnswered::~ErrorsAnswered() { --g_answered; }
+
 int set_error(int code, const char *fmt, ...)
 {
     char buf[1024];
@@ -56,7 +60,7 @@ int set_error(int code, const char *fmt, ...)
     va_end(ap);
     g_last_error = buf;
     const char *abort_env = getenv("COMET_HIP_ABORT_ON_ERROR");
-    if (abort_env && abort_env[0] == '1') {
+    if (abort_env && abort_env[0] == '1' && g_answered == 0) {
         fprintf(stderr, "comet_hip error %d: %s\n", code, buf);
         exit(1);
     }
@@ -120,6 +124,7 @@ static std::vector<PoolPending> g_pool_pending;                      // free, po
 static std::list<void *> g_pool_age;                                 // the free blocks, longest free first
 static size_t g_pool_free_bytes = 0, g_pool_cap = 0;
 static uint64_t g_pool_freed = 0;
+static int64_t g_fail_after = 0, g_fail_count = 0;          // comet_hip_debug_fail_allocations
 
 // Sizes in eighths of a power of two: requests of about the same size find each other's blocks.  From half a gigabyte
 // on in steps of POOL_STEP, so that what rounding takes from the device stays small (an eighth of 130 GiB is not).
@@ -198,6 +203,10 @@ static void *pool_take(size_t bytes)
 hipError_t dev_malloc(void **out, size_t need)
 {
     std::unique_lock<std::mutex> lk(g_pool_mu);
+    if (g_fail_count > 0 && g_fail_after-- <= 0) {
+        --g_fail_count;
+        return hipMalloc(out, (size_t)1 << 60);          // as a full device refuses it, its error left behind
+    }
     size_t bytes = pool_size(need);
     void *p = pool_take(bytes);
     if (!p && std::any_of(g_pool_pending.begin(), g_pool_pending.end(),
@@ -1125,6 +1134,13 @@ int comet_hip_free(int64_t dptr)
         return COMET_HIP_OK;
     COMET_HIPCHK(dev_free((void *)dptr));
     return COMET_HIP_OK;
+}
+
+void comet_hip_debug_fail_allocations(int64_t after, int64_t count)
+{
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    g_fail_after = after;
+    g_fail_count = count;
 }
 
 int comet_hip_release_memory(void)

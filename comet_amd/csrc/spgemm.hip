@@ -4000,7 +4000,7 @@ extern "C" int comet_hip_spgemm_masked_sum(int64_t ah, int64_t bh, int64_t mh, d
         const bool plan_now = a->tri_uses > 0 || plan_at_once();
         a->tri_uses = 1;
         if (plan_now && a->tri_state == 0)
-            COMET_CHK(tri_plan(a, pair_only()));
+            (void)plan_made([&] { return tri_plan(a, pair_only()); });
         if (a->tri_state == 2)
             return tri_count(a, out);
     }

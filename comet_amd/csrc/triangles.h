@@ -486,7 +486,8 @@ __global__ __launch_bounds__(PAIR_LIGHT_WAVES * 64, PAIR_LIGHT_OCC) void tri_lig
 }
 
 // ---------------------------------------------------------------------------
-// The plan, kept in the handle as tri (its side holds the pairs) with tri_state 2; 1: the matrix is not of the kind.
+// The plan, kept in the handle as tri (its side holds the pairs) with tri_state 2; 1: the matrix is not of the kind, or the
+// plan could not be made, and the pairs of L as it is serve all its counts.
 // ---------------------------------------------------------------------------
 static int tri_plan(Csr *a, int only)
 {
@@ -583,17 +584,11 @@ static int tri_plan(Csr *a, int only)
             }
         return COMET_HIP_OK;
     };
-    int rc = COMET_HIP_OK;
-    if (room)
-        rc = run();
-    else
-        (void)hipGetLastError();                 // without the room the pairs of L stay as they are
+    const int rc = room ? run() : COMET_HIP_ERR_HIP;
     for (void *p : {(void *)k0, (void *)k1, (void *)i0, (void *)i1, (void *)w0, (void *)r0, (void *)r1})
         (void)dev_free(p);
     if (a->tri_state != 2)
         tri_plan_free(plan);
-    if (rc != COMET_HIP_OK)
-        a->tri_state = 0;
     return rc;
 }
 

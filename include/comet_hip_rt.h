@@ -462,6 +462,9 @@ int64_t comet_hip_debug_noalloc_scratch(int64_t *bytes);
  * the CUs, and do so only while four wavefronts of the first and one of the second
  * fit a SIMD's 512 registers. */
 int comet_hip_debug_masked_sum_registers(int *workgroup_kernel, int *wavefront_kernel);
+/* Diagnostic: of the library's requests for device memory, `after` more are met
+ * as ever and the `count` behind them refused, as on a device that is full. */
+void comet_hip_debug_fail_allocations(int64_t after, int64_t count);
 int comet_hip_gather_rows_bench(int64_t workgroups, int64_t per_wave, int64_t idx_dptr,
                                 int64_t table_dptr, int64_t table_rows, int64_t out_dptr);
 
