@@ -207,16 +207,17 @@ struct Csr {
     // the transpose, built the first time a dense-times-sparse product needs it
     Csr *transposed = nullptr;
     // the transpose of the structure with, as values, the place of every entry in this matrix (a mask's, for masked
-    // products taken pair by pair); dup_state: 0 not looked at, 1 no row holds a column twice, 2 some row does
+    // products taken pair by pair); dup_state: 0 not looked at, 1 no row holds a column twice, 2 some row does; looked at
+    // with it, whether some entry lies on or above the diagonal (sides & 1) and on or below it (sides & 2)
     Csr *transposed_index = nullptr;
-    int dup_state = 0;
+    int dup_state = 0, sides = 0;
     // whether all stored values are the same number (a pattern matrix, as graph kernels use them): 0 not looked
     // at, 1 they are (iso_value), 2 they are not
     int iso_state = 0;
     double iso_value = 0.0;
     // products taken with this matrix on the left so far (0, 1, more): the SpMM and SpMV plans, which cost tens of
     // products, are built when a matrix is multiplied for the second time (plan_at_once() builds them at the first)
-    int spmm_uses = 0, spmv_uses = 0, sddmm_uses = 0, tri_uses = 0;
+    int spmm_uses = 0, spmv_uses = 0, sddmm_uses = 0;
     // triangle counts (tri_state: 0 not looked at, 1 not of the kind, 2 made)
     int tri_state = 0;
     TriPlan tri;
@@ -258,6 +259,9 @@ int exclusive_scan_i64(const int64_t *counts, int64_t n, int64_t *pos, int64_t *
 // stable radix sort of n (key, payload) pairs on the stream, comparing key bits [0, end_bit)
 int sort_pairs_u64_u32(const uint64_t *keys_in, uint64_t *keys_out, const uint32_t *vals_in, uint32_t *vals_out,
                        int64_t n, int end_bit);
+// radix sort of n keys on the stream, comparing bits [begin_bit, end_bit)
+template <typename KEY>
+int sort_keys(const KEY *in, KEY *out, int64_t n, int begin_bit, int end_bit);
 
 // deterministic tree sum of a device array, result copied to the host
 int reduce_sum_device(const double *v, int64_t n, double *out_host);

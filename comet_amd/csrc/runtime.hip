@@ -398,7 +398,7 @@ static void csr_drop_plans(Csr *c)
         pair_plan_free(p);
     c->pair_plans.clear();
     tri_plan_free(c->tri);
-    c->tri_state = c->tri_uses = 0;
+    c->tri_state = 0;
     c->uid = next_csr_uid();
     for (auto &e : c->row_lists) {
         (void)dev_free(e.rows);

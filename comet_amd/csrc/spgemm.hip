@@ -2533,14 +2533,6 @@ __global__ __launch_bounds__(SM_WAVES * 64) void spgemm_masked_sum_small_kernel(
     }
 }
 
-// whether all stored values of a matrix are one number (looked at once per matrix)
-__global__ void csr_values_differ(int64_t nnz, const double *__restrict__ val, int *__restrict__ flag)
-{
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < nnz && val[p] != val[0])
-        *flag = 1;
-}
-
 // ---------------------------------------------------------------------------
 // CSR .* CSR -> CSR, one lane per row, two-pointer merge of the sorted rows
 // (lib/Conversion/IndexTreeToSCF/IndexTreeToSCF.cpp:864-1053).
@@ -2634,18 +2626,53 @@ __global__ __launch_bounds__(256) void spgemm_dot_count(int64_t rb, int64_t re, 
         rowcount[i - rb] = n;
 }
 
-// flag[0] |= 1 when a row holds a column twice (rows are sorted); a wavefront per row
-__global__ __launch_bounds__(256) void csr_find_duplicates(int64_t nrows, const int64_t *__restrict__ pos,
-                                                           const int32_t *__restrict__ crd, int *__restrict__ flag)
+// What a matrix is like, looked at once.  Of its structure (rows are sorted): some row holds a column twice, some entry lies
+// on or above the diagonal, some lies on or below it; of its values: they are not all the same, and the first one.
+struct CsrTraits {
+    int twice, above, below, differ;
+    double first;
+};
+// crd or val null: that part is not looked at.  A lane to every entry and to every row: of the few entries whose right
+// neighbour has the same column it is looked up whether a row ends between them.  (A wavefront to a row took 293 us for the
+// 15.7 M entries of the scale-20 R-MAT graph's lower triangle, the longest rows' way from turn to turn; 40 us now.)
+__global__ __launch_bounds__(256) void csr_traits(int64_t nrows, int64_t nnz, const int64_t *__restrict__ pos,
+                                                  const int32_t *__restrict__ crd, const double *__restrict__ val,
+                                                  CsrTraits *__restrict__ out)
 {
-    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (r >= nrows)
-        return;
-    bool twice = false;
-    for (int64_t p = pos[r] + (threadIdx.x & 63); p + 1 < pos[r + 1]; p += 64)
-        twice = twice || crd[p] == crd[p + 1];
-    if (twice)
-        atomicOr(flag, 1);
+    const int64_t most = nnz > nrows ? nnz : nrows;
+    const double first = val ? val[0] : 0.0;
+    bool twice = false, above = false, below = false, differ = false;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < most; t += (int64_t)gridDim.x * 256) {
+        if (val && t < nnz)
+            differ = differ || val[t] != first;
+        if (!crd)
+            continue;
+        if (t < nrows) {
+            const int64_t s = pos[t], e = pos[t + 1];
+            above = above || (s < e && crd[e - 1] >= t);
+            below = below || (s < e && crd[s] <= t);
+        }
+        if (t + 1 < nnz && crd[t] == crd[t + 1]) {
+            int64_t lo = 0, hi = nrows;          // the first row that begins behind entry t
+            while (lo < hi) {
+                const int64_t mid = (lo + hi) >> 1;
+                if (pos[mid] <= t)
+                    lo = mid + 1;
+                else
+                    hi = mid;
+            }
+            twice = twice || pos[lo] != t + 1;
+        }
+    }
+    const bool any[4] = {__any(twice) != 0, __any(above) != 0, __any(below) != 0, __any(differ) != 0};
+    if ((threadIdx.x & 63) == 0) {
+        int *flags = &out->twice;
+        for (int k = 0; k < 4; ++k)
+            if (any[k])
+                flags[k] = 1;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        out->first = first;
 }
 
 __global__ void fill_iota_f64(int64_t n, double *__restrict__ out)
@@ -3542,43 +3569,51 @@ static int dot_transposed_index(const Csr *x, Csr **out)
     return COMET_HIP_OK;
 }
 
-// whether no row of x holds a column twice (looked at once per matrix)
-static int dot_no_duplicates(const Csr *x, bool *ok)
+// fills in what is not known yet of the two states; both together take one look and one wait
+static int csr_look(const Csr *x, bool structure, bool values)
 {
     Csr *m = const_cast<Csr *>(x);
-    if (m->dup_state == 0) {
-        COMET_CHK(g_dot_flag.ensure(sizeof(int), false));
-        COMET_HIPCHK(hipMemsetAsync(g_dot_flag.ptr, 0, sizeof(int), stream()));
-        if (m->nrows > 0)
-            csr_find_duplicates<<<dim3((unsigned)ceil_div(m->nrows, 4)), dim3(256), 0, stream()>>>(m->nrows, m->pos, m->crd,
-                                                                                                   (int *)g_dot_flag.ptr);
-        int flag = 0;
-        COMET_HIPCHK(hipMemcpyAsync(&flag, g_dot_flag.ptr, sizeof(int), hipMemcpyDeviceToHost, stream()));
+    structure = structure && m->dup_state == 0;
+    values = values && m->iso_state == 0;
+    if (!structure && !values)
+        return COMET_HIP_OK;
+    CsrTraits *seen = nullptr;
+    COMET_CHK(mailbox((void **)&seen));
+    *seen = CsrTraits{0, 0, 0, 1, 0.0};
+    if (m->nnz > 0) {
+        COMET_CHK(g_dot_flag.ensure(sizeof *seen, false));
+        COMET_HIPCHK(hipMemsetAsync(g_dot_flag.ptr, 0, sizeof *seen, stream()));
+        const int64_t blocks = ceil_div(std::max(m->nnz, m->nrows), 256);
+        csr_traits<<<dim3((unsigned)std::min<int64_t>(blocks, 1 << 16)), dim3(256), 0, stream()>>>(
+            m->nrows, m->nnz, m->pos, structure ? m->crd : nullptr, values ? m->val : nullptr, (CsrTraits *)g_dot_flag.ptr);
+        COMET_HIPCHK(hipGetLastError());
+        COMET_HIPCHK(hipMemcpyAsync(seen, g_dot_flag.ptr, sizeof *seen, hipMemcpyDeviceToHost, stream()));
         COMET_CHK(stream_wait());
-        m->dup_state = flag ? 2 : 1;
     }
-    *ok = m->dup_state == 1;
+    const volatile CsrTraits *t = seen;
+    if (structure) {
+        m->sides = (t->above ? 1 : 0) | (t->below ? 2 : 0);
+        m->dup_state = t->twice ? 2 : 1;
+    }
+    if (values) {
+        m->iso_value = t->first;
+        m->iso_state = t->differ ? 2 : 1;
+    }
+    return COMET_HIP_OK;
+}
+
+// whether no row of x holds a column twice
+static int dot_no_duplicates(const Csr *x, bool *ok)
+{
+    COMET_CHK(csr_look(x, true, false));
+    *ok = x->dup_state == 1;
     return COMET_HIP_OK;
 }
 
 static int csr_is_iso(const Csr *x, bool *iso)
 {
-    Csr *m = const_cast<Csr *>(x);
-    if (m->iso_state == 0) {
-        int flag = 1;
-        if (m->nnz > 0) {
-            COMET_CHK(g_dot_flag.ensure(sizeof(int), false));
-            COMET_HIPCHK(hipMemsetAsync(g_dot_flag.ptr, 0, sizeof(int), stream()));
-            csr_values_differ<<<dim3((unsigned)ceil_div(m->nnz, 256)), dim3(256), 0, stream()>>>(m->nnz, m->val,
-                                                                                                (int *)g_dot_flag.ptr);
-            COMET_HIPCHK(hipGetLastError());
-            COMET_HIPCHK(hipMemcpyAsync(&flag, g_dot_flag.ptr, sizeof(int), hipMemcpyDeviceToHost, stream()));
-            COMET_HIPCHK(hipMemcpyAsync(&m->iso_value, m->val, sizeof(double), hipMemcpyDeviceToHost, stream()));
-            COMET_CHK(stream_wait());
-        }
-        m->iso_state = flag ? 2 : 1;
-    }
-    *iso = m->iso_state == 1;
+    COMET_CHK(csr_look(x, false, true));
+    *iso = x->iso_state == 1;
     return COMET_HIP_OK;
 }
 
@@ -3991,15 +4026,15 @@ extern "C" int comet_hip_spgemm_masked_sum(int64_t ah, int64_t bh, int64_t mh, d
     SgGeom g;
     COMET_CHK(sg_geometry(b->ncols, &g));
     bool iso = false;
+    if (g.lds && a == b && a == m)
+        COMET_CHK(csr_look(a, true, true));
     if (g.lds)
         COMET_CHK(csr_is_iso(b, &iso));
     bool pairs = false;
     if (iso)
         COMET_CHK(pair_form_fits(a, b, m, &pairs));
     if (pairs && a == b && a == m) {
-        const bool plan_now = a->tri_uses > 0 || plan_at_once();
-        a->tri_uses = 1;
-        if (plan_now && a->tri_state == 0)
+        if (a->tri_state == 0)
             (void)plan_made([&] { return tri_plan(a, pair_only()); });
         if (a->tri_state == 2)
             return tri_count(a, out);

@@ -6,58 +6,70 @@
 // Rows are therefore kept as words: the number of a group of sixteen vertices and a bit for each of them.  A triangle is
 // an edge and a vertex that both ends' rows hold; an edge costs the words of the shorter row, looked up in a table of the
 // longer one, and a word is a look-up for all its vertices: 1.1 G look-ups of 4 bytes instead of 2.3 G.
-// The plan costs three to ten counts (3 ms for 2^20 vertices, 0.6 for 20351), so it is made when a matrix is counted for
-// the second time.  us a count, edge factor 16: n = 2^20 1571 -> 890, 200003 349 -> 260, 60000 148 -> 108, 20351 80 -> 70,
-// 1000 41 -> 22.  Bound by the rows' way from the memory-side cache for large graphs (5 TB/s), by the chain of a wavefront
-// - bounds of a row, its table, its lists - for small ones.
+// The plan is made at the first count, in the place of the plan of L's pairs, which costs as much: us of a first count /
+// and of each one after it, this form | the pairs of L as it is, R-MAT with 16 edges a vertex: n = 2^20 3790 / 903 | 4640 /
+// 1560, 200003 1146 / 279 | 1220 / 339, 60000 610 / 101 | 730 / 158, 20351 432 / 65 | 545 / 79, 1000 174 / 22 | 240 / 40.
+// Graphs without hubs gain less: uniform edges, n = 300000 and 3 a vertex 691 / 108 | 762 / 122, 16 a vertex 1360 / 164 |
+// 1296 / 211; a triangulated mesh of 10^6 1431 / 431 | 1288 / 423; and those of n = 5000 with 40 edges a vertex lose (301 / 59 |
+// 280 / 45: rows just above what a wavefront takes).  A band of 32 diagonals, n = 300000: 2009 / 153 | 2728 / 1183.
+// Bound by the rows' way from the memory-side cache for large graphs (5 TB/s), by the chain of a wavefront - bounds of a
+// row, its table, its lists - for small ones.
 
 constexpr int TRI_GROUP_LOG = 4;                         // vertices of a word: bits 0-15; bits 16-31: which sixteen
 constexpr int64_t TRI_MOST = 1ll << (16 + TRI_GROUP_LOG);       // vertices that can be named
 
-// flags[0]: some row has an entry on or above the diagonal, flags[1]: on or below it
-__global__ __launch_bounds__(256) void tri_sides(int64_t n, const int64_t *__restrict__ pos, const int32_t *__restrict__ crd,
-                                                 int *__restrict__ flags)
+// The lanes of a wavefront that have the same k: how many, which of them is the first, and how many are before this one.
+struct TriAlike {
+    int all, first, before;
+};
+__device__ __forceinline__ TriAlike tri_alike(int k, int lane)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n || pos[i] == pos[i + 1])
-        return;
-    if (crd[pos[i + 1] - 1] >= i)            // columns ascend
-        flags[0] = 1;
-    if (crd[pos[i]] <= i)
-        flags[1] = 1;
-}
-
-// degree[v]: entries in row and column v, tpos the transpose's row pointers; without them (a small matrix) the columns are
-// counted one by one, a wavefront per row.  (15.7 M entries so: 2.5 ms, a long column's atomics wait for each other.)
-__global__ __launch_bounds__(256) void tri_degrees(int64_t n, const int64_t *__restrict__ pos,
-                                                   const int32_t *__restrict__ crd, const int64_t *__restrict__ tpos,
-                                                   unsigned *__restrict__ degree)
-{
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (tpos) {
-        if (t < n)
-            degree[t] = (unsigned)(pos[t + 1] - pos[t] + tpos[t + 1] - tpos[t]);
-        return;
+    TriAlike t{0, 0, 0};
+    uint64_t left = ~0ull;
+    while (left) {
+        const int first = __builtin_ctzll(left);
+        const uint64_t same = __ballot(k == __builtin_amdgcn_readlane(k, first));
+        if (same >> lane & 1)
+            t = TriAlike{(int)__popcll(same), first, (int)__popcll(same & ((1ull << lane) - 1ull))};
+        left &= ~same;
     }
-    const int lane = threadIdx.x & 63;
-    const int64_t i = t >> 6;
-    if (i >= n)
-        return;
-    const int64_t s = pos[i], e = pos[i + 1];
-    for (int64_t p = s + lane; p < e; p += 64)
-        atomicAdd(&degree[crd[p]], 1u);
-    if (lane == 0 && e > s)
-        atomicAdd(&degree[i], (unsigned)(e - s));
+    return t;
 }
 
-__global__ __launch_bounds__(256) void tri_rank_keys(int64_t n, const unsigned *__restrict__ degree,
+// Up to this many edges the plan counts - the entries of every column, the pairs of every end - where it sorts longer
+// arrays: a sort of so few entries takes twenty launches.  A first count, us, counting / sorting: 5000 vertices and 79
+// thousand edges 309 / 382, 20351 and 0.35 M 498 / 652, 60000 and 0.9 M 678 / 856; 200003 and 1.8 M 958 / 846, 3.5 M 1357 /
+// 1277, 2^20 and 15.7 M 5260 / 4180.
+constexpr int64_t TRI_COUNTED = 1 << 20;
+
+// counts[c][v]: entries of column v that the workgroups c, c + copies, ... come to; copies is a power of two.  (Atomics on
+// one word wait for each other, 14 ns each.)
+__global__ __launch_bounds__(256) void tri_columns(int64_t n, int64_t nnz, const int32_t *__restrict__ crd, unsigned copies,
+                                                   unsigned *__restrict__ counts)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int v = p < nnz ? crd[p] : -1;
+    const TriAlike t = tri_alike(v, lane);
+    if (v >= 0 && t.first == lane)
+        atomicAdd(&counts[(blockIdx.x & (copies - 1)) * n + v], (unsigned)t.all);
+}
+
+// a vertex has the entries of its row and of its column; starts, if given: entries of the columns before each
+__global__ __launch_bounds__(256) void tri_rank_keys(int64_t n, const int64_t *__restrict__ pos, unsigned copies,
+                                                     const unsigned *__restrict__ counts, const int64_t *__restrict__ starts,
                                                      uint64_t *__restrict__ keys, uint32_t *__restrict__ idx)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) {
-        keys[i] = 0xffffffffu - degree[i];
-        idx[i] = (uint32_t)i;
-    }
+    if (i >= n)
+        return;
+    unsigned degree = (unsigned)(pos[i + 1] - pos[i]);
+    if (starts)
+        degree += (unsigned)(starts[i + 1] - starts[i]);
+    for (unsigned c = 0; c < copies; ++c)
+        degree += counts[c * n + i];
+    keys[i] = 0xffffffffu - degree;
+    idx[i] = (uint32_t)i;
 }
 
 __global__ __launch_bounds__(256) void tri_ranks(int64_t n, const uint32_t *__restrict__ by_degree, uint32_t *__restrict__ rank)
@@ -105,7 +117,8 @@ __global__ __launch_bounds__(256) void tri_opens(int64_t nnz, const uint64_t *__
 }
 
 // at[r] = first p with keys[p] >> bits >= r, for r in [0, n]
-__global__ __launch_bounds__(256) void tri_row_starts(int64_t n, int64_t nnz, const uint64_t *__restrict__ keys, int bits,
+template <typename KEY>
+__global__ __launch_bounds__(256) void tri_row_starts(int64_t n, int64_t nnz, const KEY *__restrict__ keys, int bits,
                                                       int64_t *__restrict__ at)
 {
     const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -157,18 +170,48 @@ __global__ __launch_bounds__(256) void tri_words(int64_t nnz, const uint64_t *__
 }
 
 // An edge is looked at from the end with the longer row: keys = that end (n: the other has no row, nothing to do),
-// lists = the other end.
+// lists = the other end.  count, where there is one: pairs of every end.
 __global__ __launch_bounds__(256) void tri_pairs(int64_t n, int64_t nnz, const uint64_t *__restrict__ edges, int bits,
                                                  const int64_t *__restrict__ tpos, uint64_t *__restrict__ keys,
-                                                 uint32_t *__restrict__ lists)
+                                                 uint32_t *__restrict__ lists, unsigned long long *__restrict__ count)
 {
     const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (p >= nnz)
-        return;
-    const int64_t a = (int64_t)(edges[p] >> bits), b = (int64_t)(edges[p] & ((1ull << bits) - 1ull));
-    const int64_t la = tpos[a + 1] - tpos[a], lb = tpos[b + 1] - tpos[b];
-    keys[p] = (uint64_t)(lb == 0 ? n : la > lb ? a : b);
-    lists[p] = (uint32_t)(la > lb ? b : a);
+    int64_t end = n;
+    if (p < nnz) {
+        const int64_t a = (int64_t)(edges[p] >> bits), b = (int64_t)(edges[p] & ((1ull << bits) - 1ull));
+        const int64_t la = tpos[a + 1] - tpos[a], lb = tpos[b + 1] - tpos[b];
+        end = lb == 0 ? n : la > lb ? a : b;
+        keys[p] = (uint64_t)end;
+        lists[p] = (uint32_t)(la > lb ? b : a);
+    }
+    if (count) {
+        const int lane = threadIdx.x & 63;
+        const TriAlike t = tri_alike((int)end, lane);
+        if (end < n && t.first == lane)
+            atomicAdd(&count[end], (unsigned long long)t.all);
+    }
+}
+
+// The pairs of an end next to each other, in any order: left[x] of those of x have no place yet.  (A place behind the last
+// one's is never read: the pairs of all ends may be fewer than the edges.)
+__global__ __launch_bounds__(256) void tri_place(int64_t n, int64_t nnz, const uint64_t *__restrict__ keys,
+                                                 const uint32_t *__restrict__ lists, const int64_t *__restrict__ tpos,
+                                                 const int64_t *__restrict__ kpos, unsigned long long *__restrict__ left,
+                                                 PairEnt *__restrict__ ent, int64_t *__restrict__ work)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int end = p < nnz ? (int)keys[p] : (int)n;
+    const TriAlike t = tri_alike(end, lane);
+    int before = 0;
+    if (end < n && t.first == lane)
+        before = (int)atomicAdd(&left[end], 0ull - (unsigned long long)t.all) - t.all;
+    before = __shfl(before, t.first, 64);
+    if (end < n) {
+        const int64_t l = lists[p], s = tpos[l], len = tpos[l + 1] - s, at = kpos[end] + before + t.before;
+        ent[at] = PairEnt{(uint32_t)(s >> 2), (uint32_t)(len >> 2)};
+        work[at] = len + PAIR_LIST_COST;
+    }
 }
 
 __global__ __launch_bounds__(256) void tri_entries(int64_t n, int64_t nnz, const uint64_t *__restrict__ keys,
@@ -497,75 +540,80 @@ static int tri_plan(Csr *a, int only)
         return COMET_HIP_OK;
     bool alone = false;
     COMET_CHK(dot_no_duplicates(a, &alone));
-    if (!alone)
+    if (!alone || a->sides == 3)                 // 3: neither strictly lower nor strictly upper
         return COMET_HIP_OK;
     int64_t *word = nullptr;
     COMET_CHK(mailbox((void **)&word));
     const dim3 block(256), per_row((unsigned)ceil_div(n + 1, 256)), per_entry((unsigned)ceil_div(nnz, 256));
-    int bits = TRI_GROUP_LOG;
-    while ((1ll << bits) < n + 1)
+    int bits = TRI_GROUP_LOG;                    // of a vertex
+    while ((1ll << bits) < n)
         ++bits;
     TriPlan &plan = a->tri;
     PairSidePlan &side = plan.side;
-    // scratch: two arrays of a 64-bit and one of a 32-bit word for every entry, and some for every row
-    uint64_t *k0 = nullptr, *k1 = nullptr;
-    uint32_t *i0 = nullptr, *i1 = nullptr;
-    int64_t *w0 = nullptr, *r0 = nullptr, *r1 = nullptr;
-    const size_t entries = (size_t)std::max(nnz, n) + 1, rows = (size_t)n + 2;
+    // Scratch: three arrays of a 64-bit and two of a 32-bit word for every entry, two of a 64-bit word for every row, in one
+    // allocation (each costs about as much as a small count).
+    char *scratch = nullptr;
+    const size_t entries = ((size_t)std::max(nnz, n) + 64) & ~(size_t)63, rows = ((size_t)n + 65) & ~(size_t)63;
     const int64_t quads_most = nnz / 4 + n + 2;
     const bool room =
-        dev_malloc((void **)&k0, 8 * entries) == hipSuccess && dev_malloc((void **)&k1, 8 * entries) == hipSuccess &&
-        dev_malloc((void **)&i0, 4 * entries) == hipSuccess && dev_malloc((void **)&i1, 4 * entries) == hipSuccess &&
-        dev_malloc((void **)&w0, 8 * entries) == hipSuccess && dev_malloc((void **)&r0, 8 * rows) == hipSuccess &&
-        dev_malloc((void **)&r1, 8 * rows) == hipSuccess && dev_malloc((void **)&plan.words, 16 * (size_t)quads_most) == hipSuccess &&
+        dev_malloc((void **)&scratch, 32 * entries + 16 * rows) == hipSuccess &&
+        dev_malloc((void **)&plan.words, 16 * (size_t)quads_most) == hipSuccess &&
         dev_malloc((void **)&plan.tpos, 8 * rows) == hipSuccess && dev_malloc((void **)&side.kpos, 8 * rows) == hipSuccess &&
         dev_malloc((void **)&side.counts, 8) == hipSuccess && dev_malloc(&side.ent, sizeof(PairEnt) * (size_t)nnz) == hipSuccess;
+    uint64_t *k0 = (uint64_t *)scratch, *k1 = k0 + entries;
+    int64_t *w0 = (int64_t *)(k1 + entries), *r0 = w0 + entries, *r1 = r0 + rows;
+    uint32_t *i0 = (uint32_t *)(r1 + rows), *i1 = i0 + entries;
     const auto run = [&]() -> int {
         KernelTimer t("triangle_plan");
-        unsigned *degree = (unsigned *)i1;
         uint32_t *rank = i0;
-        COMET_HIPCHK(hipMemsetAsync(r0, 0, 8, stream()));
-        tri_sides<<<per_row, block, 0, stream()>>>(n, a->pos, a->crd, (int *)r0);
-        COMET_HIPCHK(hipMemcpyAsync(word, r0, 8, hipMemcpyDeviceToHost, stream()));
-        COMET_CHK(stream_wait());
-        const volatile int *flags = (const volatile int *)word;
-        if (flags[0] && flags[1])
-            return COMET_HIP_OK;                 // neither strictly lower nor strictly upper
         // ---- the vertices by their number of edges
-        if (nnz <= PAIR_ROOM_UNSEEN) {
-            COMET_HIPCHK(hipMemsetAsync(degree, 0, 4 * (size_t)n, stream()));
-            tri_degrees<<<dim3((unsigned)ceil_div(n, 4)), block, 0, stream()>>>(n, a->pos, a->crd, nullptr, degree);
+        if (nnz <= TRI_COUNTED) {
+            unsigned copies = 16, *counts = (unsigned *)k1;
+            while (sizeof(unsigned) * copies * (size_t)n > 8 * entries)
+                copies /= 2;
+            COMET_HIPCHK(hipMemsetAsync(counts, 0, sizeof(unsigned) * copies * (size_t)n, stream()));
+            tri_columns<<<per_entry, block, 0, stream()>>>(n, nnz, a->crd, copies, counts);
+            tri_rank_keys<<<per_row, block, 0, stream()>>>(n, a->pos, copies, counts, nullptr, k0, i0);
         } else {
-            Csr *turned = nullptr;
-            COMET_CHK(dot_transposed(a, &turned));          // (the first count's plan has left it)
-            tri_degrees<<<per_row, block, 0, stream()>>>(n, a->pos, a->crd, turned->pos, degree);
+            uint32_t *columns = (uint32_t *)k0;
+            COMET_CHK(sort_keys((const uint32_t *)a->crd, columns, nnz, 0, bits));
+            tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, (const uint32_t *)columns, 0, r0);
+            tri_rank_keys<<<per_row, block, 0, stream()>>>(n, a->pos, 0, nullptr, r0, k0, i0);
         }
-        tri_rank_keys<<<per_row, block, 0, stream()>>>(n, degree, k0, i0);
         COMET_CHK(sort_pairs_u64_u32(k0, k1, i0, i1, n, 32));
         tri_ranks<<<per_row, block, 0, stream()>>>(n, i1, rank);
         // ---- their rows
         tri_edge_keys<<<per_entry, block, 0, stream()>>>(n, nnz, a->pos, a->crd, rank, bits, k0);
-        COMET_CHK(sort_pairs_u64_u32(k0, k1, i1, (uint32_t *)w0, nnz, 2 * bits));          // (what goes along is not used)
+        // (as far as the group of the smaller number: the order of the entries of a word does not matter)
+        COMET_CHK(sort_keys((const uint64_t *)k0, k1, nnz, TRI_GROUP_LOG, 2 * bits));
         int64_t *opens = (int64_t *)k0;
         tri_opens<<<per_entry, block, 0, stream()>>>(nnz, k1, opens);
         COMET_CHK(exclusive_scan_i64(opens, nnz, w0));
-        tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, k1, bits, r0);
+        tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, (const uint64_t *)k1, bits, r0);
         tri_row_quads<<<per_row, block, 0, stream()>>>(n, r0, w0, r1);
         COMET_CHK(exclusive_scan_i64(r1, n, side.kpos));
         tri_word_starts<<<per_row, block, 0, stream()>>>(n, side.kpos, plan.tpos);
         COMET_HIPCHK(hipMemsetAsync(plan.words, 0, 16 * (size_t)quads_most, stream()));
         tri_words<<<per_entry, block, 0, stream()>>>(nnz, k1, bits, r0, w0, plan.tpos, plan.words);
         // ---- the edges by the end they are looked at from
-        tri_pairs<<<per_entry, block, 0, stream()>>>(n, nnz, k1, bits, plan.tpos, k0, i0);
-        COMET_CHK(sort_pairs_u64_u32(k0, k1, i0, i1, nnz, bits));
-        tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, k1, 0, side.kpos);
         int64_t *work = (int64_t *)k0;
-        tri_entries<<<per_entry, block, 0, stream()>>>(n, nnz, k1, i1, plan.tpos, (PairEnt *)side.ent, work);
+        if (nnz <= TRI_COUNTED) {
+            unsigned long long *count = (unsigned long long *)r1;
+            COMET_HIPCHK(hipMemsetAsync(count, 0, 8 * (size_t)n, stream()));
+            tri_pairs<<<per_entry, block, 0, stream()>>>(n, nnz, k1, bits, plan.tpos, k0, i0, count);
+            COMET_CHK(exclusive_scan_i64(r1, n, side.kpos));
+            work = (int64_t *)k1;
+            tri_place<<<per_entry, block, 0, stream()>>>(n, nnz, k0, i0, plan.tpos, side.kpos, count, (PairEnt *)side.ent, work);
+        } else {
+            tri_pairs<<<per_entry, block, 0, stream()>>>(n, nnz, k1, bits, plan.tpos, k0, i0, nullptr);
+            COMET_CHK(sort_pairs_u64_u32(k0, k1, i0, i1, nnz, bits + 1));          // n is among the keys
+            tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, (const uint64_t *)k1, 0, side.kpos);
+            tri_entries<<<per_entry, block, 0, stream()>>>(n, nnz, k1, i1, plan.tpos, (PairEnt *)side.ent, work);
+        }
         COMET_CHK(exclusive_scan_i64(work, nnz, w0));
         tri_row_work<<<per_row, block, 0, stream()>>>(n, side.kpos, w0, r0);
         pair_parts<<<per_row, block, 0, stream()>>>(0, n, plan.tpos, side.kpos, r0, only, PAIR_LIGHT_MAX, r1);
-        COMET_CHK(exclusive_scan_i64(r1, n, r0));
-        COMET_HIPCHK(hipMemcpyAsync(word, r0 + n, 8, hipMemcpyDeviceToHost, stream()));
+        COMET_CHK(exclusive_scan_i64(r1, n, r0, word));
         COMET_CHK(stream_wait());
         const int64_t packed = *(volatile int64_t *)word;
         side.nheavy = packed & 0xffffffff;
@@ -576,17 +624,10 @@ static int tri_plan(Csr *a, int only)
         pair_items<<<per_row, block, 0, stream()>>>(0, n, r1, r0, (uint2 *)side.heavy, side.light, side.counts);
         COMET_HIPCHK(hipGetLastError());
         a->tri_state = 2;
-        // the pairs of L as it is are of no use any more
-        for (size_t x = a->pair_plans.size(); x-- > 0;)
-            if (a->pair_plans[x].kind == 1 && a->pair_plans[x].b_uid == a->uid && a->pair_plans[x].mask_uid == a->uid) {
-                pair_plan_free(a->pair_plans[x]);
-                a->pair_plans.erase(a->pair_plans.begin() + (std::ptrdiff_t)x);
-            }
         return COMET_HIP_OK;
     };
     const int rc = room ? run() : COMET_HIP_ERR_HIP;
-    for (void *p : {(void *)k0, (void *)k1, (void *)i0, (void *)i1, (void *)w0, (void *)r0, (void *)r1})
-        (void)dev_free(p);
+    (void)dev_free(scratch);
     if (a->tri_state != 2)
         tri_plan_free(plan);
     return rc;

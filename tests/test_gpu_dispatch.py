@@ -537,7 +537,7 @@ def _edges(kind, rng):
                                   (4097, 60_000), (100_003, 900_000), (1 << 20, 2_000_000), ((1 << 20) + 1, 500_000)])
 def test_triangle_counts_of_every_kind_of_graph(kind, upper, only, monkeypatch):
     # both triangles of the matrix, rows through either kernel, numbers of vertices around a word's and the most that are
-    # named in 16 + 4 bits; the first count walks L as it is, the others the vertices by their number of edges
+    # named in 16 + 4 bits; counts of one handle walk the vertices by their number of edges, a mask of its own walks L as it is
     monkeypatch.delenv("COMET_HIP_PLAN_AT_ONCE")
     if only:
         monkeypatch.setenv("COMET_HIP_MASKED_SUM_ONLY", only)
@@ -557,7 +557,40 @@ def test_triangle_counts_of_every_kind_of_graph(kind, upper, only, monkeypatch):
         want = float(((D @ D) * D).sum())
     else:
         want = orc.tricount_masked(pos, v.astype(np.int64), np.ones(len(u)))
-    assert [rt.triangle_count(L) for _ in range(4)] == [0.25 * want] * 4
+    assert [rt.triangle_count(L) for _ in range(3)] == [0.25 * want] * 3
+    mask = rt.CsrMatrix.from_arrays((n, n), pos, v.astype(np.int64), np.full(len(u), 2.0))
+    assert [rt.spgemm_masked_sum(L, L, mask) for _ in range(2)] == [0.25 * want] * 2
+
+
+def test_the_plan_of_triangle_counts_is_made_once_and_where_it_serves(monkeypatch):
+    # at the first count and never again, for matrices that are strictly on one side and hold no column twice - the last
+    # column of a row and the first of the next may be the same -; the others' sums take the pairs as they are
+    monkeypatch.delenv("COMET_HIP_PLAN_AT_ONCE")
+    rng = np.random.default_rng(11)
+    for what in ("lower", "upper", "star", "diagonal", "both sides", "twice", "last row twice"):
+        n, u, v = (700, np.arange(1, 700), np.zeros(699, np.int64)) if what == "star" else _edges((700, 9000), rng)
+        if what == "upper":
+            u, v = v, u
+        extra = {"diagonal": ([5], [5]), "both sides": (v[:1], u[:1]), "twice": (u[100:101], v[100:101]),
+                 "last row twice": (u[-1:], v[-1:])}.get(what, ([], []))
+        u, v = np.concatenate([u, extra[0]]).astype(np.int64), np.concatenate([v, extra[1]]).astype(np.int64)
+        order = np.lexsort((v, u))
+        u, v = u[order], v[order]
+        pos = np.concatenate([[0], np.cumsum(np.bincount(u, minlength=n))]).astype(np.int64)
+        L = rt.CsrMatrix.from_arrays((n, n), pos, v, np.ones(len(u)))
+        D = np.zeros((n, n))
+        np.add.at(D, (u, v), 1.0)
+        want = float(((D @ D) * (D > 0)).sum())
+        plans = []
+        for _ in range(2):
+            rt.profile_reset()
+            rt.profile_enable(True)
+            assert rt.triangle_count(L) == want
+            report = rt.profile_report()
+            rt.profile_enable(False)
+            plans.append([k for k in ("triangle_plan", "spgemm_pair_plan") if k in report])
+        renumbered = what in ("lower", "upper", "star")
+        assert plans == [["triangle_plan" if renumbered else "spgemm_pair_plan"], []], what
 
 
 def test_sums_that_are_no_triangle_count_stay_as_they_are():
