@@ -859,7 +859,7 @@ __device__ inline void single_store(const spmm_pair (&b)[NB], const spmm_pair (&
 // apart - the older one wins every arbitration - and rows of B leave the L2 before the slow ones come to them (500000
 // rows, K = 64: 11 M lines from beyond the L2s instead of 5, 374 us instead of 311).  us by columns that a wavefront may
 // be ahead, 2048 / 3072 / 4096 / 8192: K = 64 311 / 313 / 318 / 341, 48 269 / 269 / 273 / 284, 32 231 / 223 / 225 / 232,
-// 16 215 / 205 / 206 / 211.
+// 16 215 / 205 / 206 / 211.  sweep_slack says how far that may be.
 constexpr int SPMM_PACE_LOG = 10;
 struct SweepPace {
     int *at;                 // of every wavefront, in LDS
@@ -1022,6 +1022,17 @@ __global__ __launch_bounds__(SPMM_HW * 64) void spmm_heavy_sweep(
             out[(int64_t)r * K + col + 1] = accy[r] + oy;
         }
     }
+}
+
+// Steps that a wavefront of the sweep may be ahead of the last one.  Within a block of columns a list goes from row to row,
+// each time from the block's first column to its last: both ends of a block have to be close enough, or wavefronts wait for
+// others that are in the same block.  2 or 3 steps hold a block of up to 2048 or 3072 columns, 524288 or 786432 in all; us
+// with 2, 3 steps | with what the block takes | without waiting, K = 64: 10^6 columns 765 | 4: 744 | 1004, 500000 rows of
+// 4 M columns 825 | 16: 587 | 713, 250000 of 8 M 803 | 31: 408 | 415; K = 16: 10^6 373 | 4: 368 | 383.
+static int sweep_slack(int64_t xcols, int64_t K)
+{
+    const int64_t block = ceil_div(xcols, SPMM_HCB);
+    return (int)std::max<int64_t>(K >= 48 ? 2 : 3, ((block - 1) >> SPMM_PACE_LOG) + 1);
 }
 
 // C[rows[i]][0..K) = 0
@@ -1714,6 +1725,11 @@ static int spmv_run(Csr *a, int64_t x_dptr, int64_t y_dptr, int accumulate)
     return COMET_HIP_OK;
 }
 
+extern "C" int comet_hip_debug_sweep_slack(int64_t ncols, int64_t K)
+{
+    return sweep_slack(ceil_div(ncols, 8), K);
+}
+
 extern "C" int comet_hip_spmm_csr_f64(int64_t csr, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dptr,
                                       int64_t ldc, int accumulate)
 {
@@ -1782,7 +1798,7 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
         KernelTimer t("spmm_heavy_sweep");
         const bool small_b = a->ncols < (1 << 24) && ldb * 8 < (1 << 24) && a->ncols * ldb * 8 < (1ll << 32);
         const dim3 grid(8 * G, tiles), block(SPMM_HW * 64);
-        const int slack = K >= 48 ? 2 : 3;
+        const int slack = sweep_slack(ceil_div(a->ncols, 8), K);
         if (small_b && accumulate)
             sweep_launch(spmm_heavy_sweep<true, true>, grid, block, medium_lds, a->heavy_seg, a->heavy_ent, B, ldb, K, partial, C, ldc,
                          G, ceil_div(a->ncols, 8), nslots, partial_medium, slack);

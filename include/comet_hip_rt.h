@@ -465,6 +465,9 @@ int comet_hip_debug_masked_sum_registers(int *workgroup_kernel, int *wavefront_k
 /* Diagnostic: of the library's requests for device memory, `after` more are met
  * as ever and the `count` behind them refused, as on a device that is full. */
 void comet_hip_debug_fail_allocations(int64_t after, int64_t count);
+/* Diagnostic: how far apart, in steps of 1024 columns, the wavefronts of the SpMM
+ * column sweep may be in a matrix of ncols columns.  Runs on the host. */
+int comet_hip_debug_sweep_slack(int64_t ncols, int64_t K);
 int comet_hip_gather_rows_bench(int64_t workgroups, int64_t per_wave, int64_t idx_dptr,
                                 int64_t table_dptr, int64_t table_rows, int64_t out_dptr);
 

@@ -167,3 +167,17 @@ def test_lds_fp64_regions_start_on_eight_bytes():
         off = L.comet_hip_debug_dot_table_words(words)
         assert off > 0 and off % 2 == 0, (words, off)
 
+
+
+@pytest.mark.parametrize("ncols", [1, 9, 250_000, 500_000, 524_288, 524_289, 786_433, 1_000_000, 4_000_000, 8_388_608])
+def test_wavefronts_of_one_column_block_do_not_wait_for_each_other(ncols):
+    """The SpMM sweep's lists run through a block of columns once for every row, an XCD's eighth of the columns in 32
+    blocks: the slack between wavefronts, in steps of 1024 columns, has to hold a whole block, and little more."""
+    xcols = -(-ncols // 8)
+    cols = np.arange(xcols, dtype=np.int64)
+    block, step = cols * 32 // xcols, cols >> 10
+    first = np.searchsorted(block, np.unique(block))
+    span = int((np.maximum.reduceat(step, first) - np.minimum.reduceat(step, first)).max())
+    for K in (16, 33, 48, 64, 130):
+        slack = rt.lib().comet_hip_debug_sweep_slack(ncols, K)
+        assert max(span, 2) <= slack <= max(span + 1, 3), K
