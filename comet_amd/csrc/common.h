@@ -176,8 +176,9 @@ struct Csr {
     // of row k whose column is >= cb * 2^14, so that the slice of a row inside one block of 16384 columns is
     // found without searching.
     int64_t *sg_blkptr = nullptr;
-    // and for its structure, one allocation: bitmaps of its longest rows, 16 bytes at a time, which rows they are of, and
-    // for every row the number of its bitmap or -1
+    // and for its structure: bitmaps of its longest rows, 16 bytes at a time, and for every row the number of its bitmap or
+    // -1, with which rows they are of behind (sg_hub_state: 0 not looked at, 1 none, 2 made)
+    int sg_hub_state = 0;
     uint32_t *sg_hub_bits = nullptr;
     int32_t *sg_hub_slot = nullptr;
     int sg_nblk = 0;

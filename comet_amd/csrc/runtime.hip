@@ -443,8 +443,10 @@ static void csr_drop_plans(Csr *c)
     (void)dev_free(c->sg_crd16);
     c->sg_blkptr = nullptr;
     (void)dev_free(c->sg_hub_bits);
+    (void)dev_free(c->sg_hub_slot);
     c->sg_hub_bits = nullptr;
     c->sg_hub_slot = nullptr;
+    c->sg_hub_state = 0;
     c->sg_crd16 = nullptr;
     c->sg_nblk = 0;
     (void)dev_free(c->spmv_bpos);

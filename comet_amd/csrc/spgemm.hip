@@ -3392,29 +3392,45 @@ static dim3 sm_grid(int64_t rows, int per_cu)          // rows < 0: how many is 
 }
 
 // The bitmaps of b's long rows, words to each; a matrix of few columns or none such rows goes without, and so does one for
-// which there is no memory.
+// which there is no memory.  (The host waits once for how many there are: a bound on them from the entries alone is 8 bytes
+// of bitmaps for every one, also where no row is long.)
 static int sg_plan_hubs(Csr *b, int words)
 {
     const int64_t least = ceil_div(b->ncols, SMID_HUB_PART);
-    if (b->sg_hub_bits || b->ncols <= SG_NARROW || b->nrows >= 1ll << 31 || b->nnz < least)
+    if (b->sg_hub_state != 0 || b->ncols <= SG_NARROW || b->nrows >= 1ll << 31 || b->nnz < least)
         return COMET_HIP_OK;
+    b->sg_hub_state = 1;
     const int64_t most = std::min(b->nnz / least, b->nrows);
-    const size_t bits = sizeof(uint32_t) * (size_t)words * (size_t)most;
-    if (dev_malloc((void **)&b->sg_hub_bits, bits + sizeof(int32_t) * (size_t)(b->nrows + most + 1)) != hipSuccess) {
-        (void)hipGetLastError();        // an allocation that may fail: its error must not reach the next check
-        b->sg_hub_bits = nullptr;
-        return COMET_HIP_OK;
-    }
-    b->sg_hub_slot = (int32_t *)((char *)b->sg_hub_bits + bits);
-    int32_t *hub = b->sg_hub_slot + b->nrows, *hubs = hub + most;
+    int32_t *slot = nullptr, *n = nullptr;
+    uint32_t *bits = nullptr;
+    COMET_CHK(mailbox((void **)&n));
     KernelTimer t("spgemm_hub_bits");
-    COMET_HIPCHK(hipMemsetAsync(hubs, 0, sizeof(int32_t), stream()));
-    spgemm_hub_rows<<<dim3((unsigned)ceil_div(b->nrows, 256)), dim3(256), 0, stream()>>>(b->nrows, b->pos, least, b->sg_hub_slot,
-                                                                                       hub, hubs);
-    spgemm_hub_bits<<<dim3((unsigned)std::min<int64_t>(most, 2 * (int64_t)num_cus())), dim3(256), 0, stream()>>>(
-        b->pos, b->crd, hub, hubs, words, b->sg_hub_bits);
-    COMET_HIPCHK(hipGetLastError());
-    return COMET_HIP_OK;
+    const auto run = [&]() -> int {
+        COMET_HIPCHK(dev_malloc((void **)&slot, sizeof(int32_t) * (size_t)(b->nrows + most + 1)));
+        int32_t *hub = slot + b->nrows, *hubs = hub + most;
+        COMET_HIPCHK(hipMemsetAsync(hubs, 0, sizeof(int32_t), stream()));
+        spgemm_hub_rows<<<dim3((unsigned)ceil_div(b->nrows, 256)), dim3(256), 0, stream()>>>(b->nrows, b->pos, least, slot, hub,
+                                                                                           hubs);
+        COMET_HIPCHK(hipMemcpyAsync(n, hubs, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
+        COMET_CHK(stream_wait());
+        const int64_t found = *(volatile int32_t *)n;
+        if (found == 0)
+            return COMET_HIP_OK;
+        COMET_HIPCHK(dev_malloc((void **)&bits, sizeof(uint32_t) * (size_t)words * (size_t)found));
+        spgemm_hub_bits<<<dim3((unsigned)std::min<int64_t>(found, 2 * (int64_t)num_cus())), dim3(256), 0, stream()>>>(
+            b->pos, b->crd, hub, hubs, words, bits);
+        COMET_HIPCHK(hipGetLastError());
+        b->sg_hub_slot = slot;
+        b->sg_hub_bits = bits;
+        b->sg_hub_state = 2;
+        return COMET_HIP_OK;
+    };
+    const int rc = run();
+    if (b->sg_hub_state != 2) {
+        (void)dev_free(slot);
+        (void)dev_free(bits);
+    }
+    return rc;
 }
 
 static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *rowcount)
@@ -3457,7 +3473,7 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
         if (list.counts[3] != 0) {
             const int words = sm_words(b->ncols);
             Csr *right = const_cast<Csr *>(b);           // what is kept in a handle is not part of the matrix
-            COMET_CHK(sg_plan_hubs(right, words));
+            (void)plan_made([&] { return sg_plan_hubs(right, words); });
             KernelTimer t("spgemm_symbolic");
             const auto kernel = b->sg_hub_bits ? spgemm_symbolic_rows_kernel<true> : spgemm_symbolic_rows_kernel<false>;
             kernel<<<sm_grid(list.counts[3], 4), dim3(SMID_T), sizeof(uint32_t) * (size_t)words, stream()>>>(

@@ -639,3 +639,36 @@ def test_a_plan_without_memory_is_done_without_triangle_count():
         finally:
             fail(0, 0)
         assert got == [want] * 3, k
+
+
+@pytest.mark.parametrize("long_rows", [0, 3])
+def test_what_a_structure_keeps_is_for_rows_that_are_long(long_rows):
+    # bitmaps of rows with a 64th of the columns: for as many as there are, and nothing for a matrix without
+    n = 20_000
+    rng = np.random.default_rng(1)
+    lengths = rng.integers(60, 100, n)
+    lengths[:long_rows] = n // 64 + 1
+    crd = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for k in lengths]).astype(np.int64)
+    pos = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    val = np.ones(len(crd))
+
+    def free():
+        rt.sync()
+        rt.release_memory()
+        got = [C.c_int64(), C.c_int64()]
+        rt._check(rt.lib().comet_hip_mem_info(*map(C.byref, got)))
+        return got[0].value
+
+    kept = []
+    for _ in range(2):              # the first of them brings up what the library keeps for all matrices
+        A = rt.CsrMatrix.from_arrays((n, n), pos, crd, val)
+        before = free()
+        dpos, nnz = rt.spgemm_symbolic(A, A)
+        counts = np.diff(dpos.to_numpy())
+        dpos.free()
+        kept.append(before - free())
+    assert kept[1] < len(crd), kept
+    import scipy.sparse as sp
+    S = sp.csr_matrix((val, crd, pos), shape=(n, n))
+    want = (S[:200] @ S).astype(bool)
+    assert np.array_equal(counts[:200], np.diff(want.indptr))
