@@ -59,6 +59,8 @@ int set_error(int code, const char *fmt, ...)
     vsnprintf(buf, sizeof buf, fmt, ap);
     va_end(ap);
     g_last_error = buf;
+    if (code == COMET_HIP_ERR_HIP)
+        (void)hipGetLastError();          // it has been reported: the next launch's check must not find it
     const char *abort_env = getenv("COMET_HIP_ABORT_ON_ERROR");
     if (abort_env && abort_env[0] == '1' && g_answered == 0) {
         fprintf(stderr, "comet_hip error %d: %s\n", code, buf);

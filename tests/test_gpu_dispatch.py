@@ -624,21 +624,39 @@ def test_sums_that_are_no_triangle_count_stay_as_they_are():
     assert rt.triangle_count(L) == rt.triangle_count(L) == float(((W @ W) * D).sum())
 
 
+def _refusing(k, call):
+    """call() with its k-th request for device memory refused."""
+    rt.lib().comet_hip_debug_fail_allocations(k, 1)
+    try:
+        return call()
+    finally:
+        rt.lib().comet_hip_debug_fail_allocations(0, 0)
+
+
+def test_a_refused_request_fails_its_own_call_only():
+    pos, crd, val = gen.poisson_csr(n=3000, mean=4.0, seed=5)
+    A = rt.CsrMatrix.from_arrays((3000, 3000), pos, crd, val)
+    for k in range(4):
+        with pytest.raises(rt.CometHipError):
+            rt.lib().comet_hip_debug_fail_allocations(k, 100)
+            try:
+                rt.spgemm(A, A)
+            finally:
+                rt.lib().comet_hip_debug_fail_allocations(0, 0)
+        B = rt.CsrMatrix.from_arrays((3000, 3000), pos, crd, val)          # copies and launches look at what failed before
+        assert np.array_equal(B.to_arrays()[2], val)
+    assert rt.spgemm(A, A).nnz == rt.spgemm(B, A).nnz > 0
+
+
 def test_a_plan_without_memory_is_done_without_triangle_count():
     n, u, v = _edges((60_001, 900_000), np.random.default_rng(5))
     pos = np.concatenate([[0], np.cumsum(np.bincount(u, minlength=n))]).astype(np.int64)
     new = lambda: rt.CsrMatrix.from_arrays((n, n), pos, v, np.ones(len(u)))
     want = orc.tricount_masked(pos, v, np.ones(len(u)))
     assert rt.triangle_count(new()) == want          # what the library keeps for all matrices is there
-    fail = rt.lib().comet_hip_debug_fail_allocations
-    for k in range(40):
+    for k in range(20):
         L = new()
-        fail(k, 1)
-        try:
-            got = [rt.triangle_count(L) for _ in range(3)]
-        finally:
-            fail(0, 0)
-        assert got == [want] * 3, k
+        assert _refusing(k, lambda: [rt.triangle_count(L) for _ in range(3)]) == [want] * 3, k
 
 
 @pytest.mark.parametrize("long_rows", [0, 3])
