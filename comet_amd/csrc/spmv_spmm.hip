@@ -1608,6 +1608,10 @@ static int spmm_heavy_plan(Csr *a)
     } else {
         HEAVY_TRY(hipMemsetAsync(light->pos, 0, 8, stream()));
     }
+    if (light->nnz > 0 && spmm_plan(light) != COMET_HIP_OK) {          // its chunk table
+        cleanup(true);
+        return COMET_HIP_ERR_HIP;
+    }
     HEAVY_TRY(hipGetLastError());
     HEAVY_TRY(hipStreamSynchronize(stream()));
 #undef HEAVY_TRY
@@ -1680,8 +1684,8 @@ static int spmv_run(Csr *a, int64_t x_dptr, int64_t y_dptr, int accumulate)
     // is made when it is multiplied again.
     const bool plan_now = a->spmv_uses > 0 || plan_at_once();
     a->spmv_uses = a->spmv_uses < 2 ? a->spmv_uses + 1 : 2;
-    if (plan_now)
-        COMET_CHK(spmv_plan(a));
+    if (plan_now && !plan_made([&] { return spmv_plan(a); }))
+        a->spmv_nb = 1;
     const int nb = a->spmv_nb > 0 ? a->spmv_nb : 1;
     const unsigned blocks = (unsigned)ceil_div(a->nrows, SPMV_T);
     const double *x = (const double *)x_dptr;
@@ -1766,17 +1770,27 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
     const bool plan_now = a->spmm_uses > 0 || plan_at_once();
     a->spmm_uses = a->spmm_uses < 2 ? a->spmm_uses + 1 : 2;
     if (sweep_fits && plan_now)
-        COMET_CHK(spmm_heavy_plan(a));
+        (void)plan_made([&] { return spmm_heavy_plan(a); });          // or the chunk kernel goes on taking all rows
     if (a->heavy_state != 2 || !sweep_fits)
         return spmm_chunks(a, K, B, ldb, C, ldc, accumulate);
+    const int G = a->heavy_groups;
+    // rows of middling length: ceil(rows / G) sums of 64 doubles in the LDS of every workgroup
+    const int nslots = (int)ceil_div(a->medium_rows, G);
+    const size_t medium_lds = sizeof(double) * 64 * (size_t)nslots;
+    // what the kernels leave sums in; without room for it the chunk kernel takes all rows
+    const auto scratch = [&]() -> int {
+        COMET_CHK(g_heavy_partial.ensure(sizeof(double) * 8 * (size_t)spmm_hslots(G) * (size_t)K, false));
+        COMET_CHK(g_medium_partial.ensure(sizeof(double) * 8 * (size_t)G * (size_t)(nslots > 0 ? nslots : 1) * (size_t)K, false));
+        return a->light->nnz > 0 ? spmm_chunk_scratch(a->light, K) : COMET_HIP_OK;
+    };
+    if (!plan_made(scratch))
+        return spmm_chunks(a, K, B, ldb, C, ldc, accumulate);
+    double *partial = (double *)g_heavy_partial.ptr, *partial_medium = (double *)g_medium_partial.ptr;
     // rows of two and more nonzeros that are not long: one wavefront per 256 nonzeros
     // with CUs left free by the sweep, the chunk kernel of the rows in between runs beside it on a second stream
-    const int G = a->heavy_groups;
     const bool overlap = a->light->nnz > 0 && G < SPMM_HG_ALONE;
     if (overlap) {
-        // what the chunk kernel needs from stream() - its chunk table, its scratch - is in place before the fork
-        COMET_CHK(spmm_plan(a->light));
-        COMET_CHK(spmm_chunk_scratch(a->light, K));
+        // (what it needs from stream() - its chunk table, its scratch - is in place before the fork)
         COMET_CHK(aux_fork());
     } else if (a->light->nnz > 0)
         COMET_CHK(spmm_chunks(a->light, K, B, ldb, C, ldc, accumulate));
@@ -1787,13 +1801,6 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
         zero_listed_rows_f64<<<dim3(blocks), dim3(256), 0, stream()>>>(C, a->empty_rows, a->nempty, K, ldc);
     }
     // long rows (sums on chip, left in `partial`) and rows of one nonzero (stored to C)
-    COMET_CHK(g_heavy_partial.ensure(sizeof(double) * 8 * (size_t)spmm_hslots(G) * (size_t)K, false));
-    double *partial = (double *)g_heavy_partial.ptr;
-    // rows of middling length: ceil(rows / G) sums of 64 doubles in the LDS of every workgroup
-    const int nslots = (int)ceil_div(a->medium_rows, G);
-    const size_t medium_lds = sizeof(double) * 64 * (size_t)nslots;
-    COMET_CHK(g_medium_partial.ensure(sizeof(double) * 8 * (size_t)G * (size_t)(nslots > 0 ? nslots : 1) * (size_t)K, false));
-    double *partial_medium = (double *)g_medium_partial.ptr;
     {
         KernelTimer t("spmm_heavy_sweep");
         const bool small_b = a->ncols < (1 << 24) && ldb * 8 < (1 << 24) && a->ncols * ldb * 8 < (1ll << 32);
@@ -2528,7 +2535,7 @@ static int sddmm_values(Csr *b, int64_t K, int64_t c_dptr, int64_t ldc, int64_t 
     b->sddmm_uses = 1;
     const bool large = b->nnz >= SDDMM_ORDER_NNZ && b->ncols * K * 8 >= SDDMM_ORDER_D;
     if (large && plan_now && b->sddmm_state == 0)
-        COMET_CHK(sddmm_order(b, rows));
+        (void)plan_made([&] { return sddmm_order(b, rows); });
     const int32_t *order = large && b->sddmm_state == 2 ? b->sddmm_order : nullptr;
     {
         KernelTimer t("sddmm_kernel");

@@ -648,6 +648,64 @@ def test_a_refused_request_fails_its_own_call_only():
     assert rt.spgemm(A, A).nnz == rt.spgemm(B, A).nnz > 0
 
 
+@pytest.mark.parametrize("op,K", [("spmm", 64), ("spmm", 81), ("spmv", 1), ("sddmm", 40)])
+def test_a_plan_without_memory_is_done_without(op, K, monkeypatch):
+    # the second call on a handle makes its plan; where that finds no memory the call goes the way of the first
+    monkeypatch.delenv("COMET_HIP_PLAN_AT_ONCE")
+    n = 700_001 if op == "spmv" else 40_001
+    pos, crd, val = (gen.poisson_csr(n=n, mean=3.0, seed=5) if op == "spmv" else gen.zipf_csr(n=n, mean=16.0, cap=4096, seed=7))
+    rng = np.random.default_rng(2)
+    x = rng.uniform(-1, 1, n) if op == "spmv" else rng.uniform(-1, 1, (n, K))
+    dx = rt.DeviceArray.from_numpy(x)
+    dt = rt.DeviceArray.from_numpy(np.ascontiguousarray(x.T)) if op == "sddmm" else None
+    out = rt.DeviceArray(len(crd) if op == "sddmm" else x.shape)
+
+    def call(A):
+        if op == "spmv":
+            rt.spmv(A, dx, out, accumulate=False)
+        elif op == "spmm":
+            rt.spmm(A, dx, out, accumulate=False)
+        else:
+            rt.sddmm(A, dx, dt, out_values=out)
+        return out.to_numpy()
+
+    def plans():
+        A = rt.CsrMatrix.from_arrays((n, n), pos, crd, val)
+        return A, call(A)
+
+    A, want = plans()
+    planned = call(A)                       # what the library keeps for all matrices is there
+    bound = {"spmv": lambda: orc.spmv(pos, crd, np.abs(val), np.abs(x)), "spmm": lambda: orc.spmm(pos, crd, np.abs(val), np.abs(x)),
+             "sddmm": lambda: np.abs(want)}[op]()
+    assert np.all(np.abs(planned - want) <= 1e-12 * bound)
+    for k in range(24):
+        A, first = plans()
+        assert np.array_equal(first, want)
+        got = _refusing(k, lambda: call(A))
+        assert np.all(np.abs(got - want) <= 1e-12 * bound), k
+        assert np.all(np.abs(call(A) - want) <= 1e-12 * bound), k
+
+
+def test_a_sweep_without_room_for_its_sums_is_done_without():
+    # a planned matrix meets a wider B than any before: scratch for the sums, and for the chunk kernel, is refused in turn
+    n = 40_001
+    pos, crd, val = gen.zipf_csr(n=n, mean=16.0, cap=4096, seed=7)
+    A = rt.CsrMatrix.from_arrays((n, n), pos, crd, val)
+    rng = np.random.default_rng(2)
+    rt.spmm(A, rt.DeviceArray.from_numpy(rng.uniform(-1, 1, (n, 16))))
+    for k, K in ((0, 2040), (1, 2046), (0, 2048)):
+        few = rng.integers(0, K, 8)
+        x = np.zeros((n, K))
+        x[:, few] = rng.uniform(-1, 1, (n, len(few)))
+        dx, out = rt.DeviceArray.from_numpy(x), rt.DeviceArray((n, K))
+        _refusing(k, lambda: rt.spmm(A, dx, out, accumulate=False))
+        got = out.to_numpy()
+        bound = orc.spmm(pos, crd, np.abs(val), np.abs(x[:, few]))
+        assert np.all(np.abs(got[:, few] - orc.spmm(pos, crd, val, x[:, few])) <= 1e-12 * bound)
+        got[:, few] = 0.0
+        assert not got.any()
+
+
 def test_a_plan_without_memory_is_done_without_triangle_count():
     n, u, v = _edges((60_001, 900_000), np.random.default_rng(5))
     pos = np.concatenate([[0], np.cumsum(np.bincount(u, minlength=n))]).astype(np.int64)
