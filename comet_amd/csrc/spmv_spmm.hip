@@ -2521,11 +2521,14 @@ static int sddmm_values(Csr *b, int64_t K, int64_t c_dptr, int64_t ldc, int64_t 
         return COMET_HIP_OK;
     // Rows of D begin at a line of 128 bytes, 16 columns are one line then, unless that makes them nearly twice as long
     // (200000 rows, 3.7 M entries, us, packed / so: K = 3 50 / 71, 9 69 / 65, 15 80 / 73, 17 86 / 91, 18 85 / 79, 28 117 /
-    // 105, 50 219 / 179, 61 253 / 197, 100 390 / 317) or D very large.
+    // 105, 50 219 / 179, 61 253 / 197, 100 390 / 317), D very large, or no room for it.
     const int64_t whole = ceil_div(K, 16) * 16;
-    const int64_t ldt = K > 0 && whole * 5 <= K * 9 && b->ncols <= (1ll << 32) / 8 / whole ? whole : K;
+    int64_t ldt = K > 0 && whole * 5 <= K * 9 && b->ncols <= (1ll << 32) / 8 / whole ? whole : K;
     if (K > 0) {
-        COMET_CHK(g_sddmm_dt.ensure(sizeof(double) * (size_t)b->ncols * (size_t)ldt, false));
+        const auto room = [&] { return g_sddmm_dt.ensure(sizeof(double) * (size_t)b->ncols * (size_t)ldt, false); };
+        if (ldt > K && !plan_made(room))
+            ldt = K;
+        COMET_CHK(room());
         COMET_CHK(transpose2d((const double *)d_dptr, ldd, K, b->ncols, (double *)g_sddmm_dt.ptr, ldt));
     }
     const int32_t *rows = nullptr;

@@ -706,6 +706,24 @@ def test_a_sweep_without_room_for_its_sums_is_done_without():
         assert not got.any()
 
 
+def test_an_sddmm_without_room_for_whole_lines_takes_its_rows_packed():
+    m, n, K = 50, 5_000_000, 9          # D turned over in lines of 128 bytes: 640 MB, packed 360
+    rng = np.random.default_rng(4)
+    crd = np.sort(rng.choice(n, (m, 40), replace=False), axis=1).ravel().astype(np.int64)
+    pos = np.arange(0, 40 * m + 1, 40).astype(np.int64)
+    val = rng.uniform(-1, 1, len(crd))
+    C0, D = rng.uniform(-1, 1, (m, K)), rng.uniform(-1, 1, (K, n))
+    S = rt.CsrMatrix.from_arrays((m, n), pos, crd, val)
+    dC, dD, out = rt.DeviceArray.from_numpy(C0), rt.DeviceArray.from_numpy(D), rt.DeviceArray(len(crd))
+    _refusing(0, lambda: rt.sddmm(S, dC, dD, out_values=out))
+    rows = np.repeat(np.arange(m), 40)
+    want = np.zeros(len(crd))
+    for k in range(K):
+        want += C0[rows, k] * D[k, crd]
+    got = out.to_numpy()
+    assert np.all(np.abs(got - val * want) <= 1e-14 * K)
+
+
 def test_a_plan_without_memory_is_done_without_triangle_count():
     n, u, v = _edges((60_001, 900_000), np.random.default_rng(5))
     pos = np.concatenate([[0], np.cumsum(np.bincount(u, minlength=n))]).astype(np.int64)
