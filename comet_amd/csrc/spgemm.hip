@@ -1761,7 +1761,8 @@ __device__ __forceinline__ int slice_walk(STAGE &st, const COL *__restrict__ Bcr
 // An accumulator of the block that has received nothing holds a value that no sum and no key can be, and so the block
 // needs no bitmap: -0.0 where products are added (every product is made +0.0 if it is -0.0 first, as an accumulator
 // that starts at +0.0 would have it; a sum of others is never -0.0), 0 where keys are kept (the one NaN whose key is 0
-// takes the next one's).
+// takes the next one's).  The product and the +0.0 must stay two operations: fused, a negative product that underflows gives
+// -0.0, and its entry, counted in the structure, would be missing from the row.
 __device__ __forceinline__ unsigned long long block_empty(int reduce_op)
 {
     return reduce_op == SR_PLUS ? 0x8000000000000000ull : 0ull;
@@ -1769,6 +1770,7 @@ __device__ __forceinline__ unsigned long long block_empty(int reduce_op)
 template <bool SEMI>
 __device__ __forceinline__ void block_add(double *slot, double a, double b, int pa, int64_t q, int reduce_op, int mult_op)
 {
+#pragma clang fp contract(off)
     if constexpr (SEMI) {
         unsigned long long *key = reinterpret_cast<unsigned long long *>(slot);
         if (reduce_op == SR_ANY) {

@@ -469,6 +469,24 @@ def test_spgemm_block_by_block_slices(semiring, repeats, monkeypatch):
             assert not np.any(np.signbit(v[v == 0]))          # an accumulator that starts at zero
 
 
+@pytest.mark.parametrize("wide", [0, 1 << 40])
+def test_spgemm_keeps_entries_whose_products_underflow(wide, monkeypatch):
+    # the block kernel tells an empty accumulator by its sign: a product of no size and of either sign is an entry, +0.0
+    monkeypatch.setenv("COMET_HIP_SPGEMM_WIDE", str(wide))
+    rng = np.random.default_rng(3)
+    n, m = 200, 20_000
+    S = np.sort(np.stack([rng.choice(m, 300, replace=False) for _ in range(n)]), axis=1)
+    bpos, bcrd = np.arange(0, 300 * n + 1, 300).astype(np.int64), S.ravel().astype(np.int64)
+    apos = np.array([0, 1, 1 + n, 61 + n]).astype(np.int64)
+    acrd = np.concatenate([[7], np.arange(n), np.arange(60)]).astype(np.int64)
+    aval, bval = (rng.choice([-1e-200, 1e-200], k) for k in (len(acrd), len(bcrd)))
+    A, B = rt.CsrMatrix.from_arrays((3, n), apos, acrd, aval), rt.CsrMatrix.from_arrays((n, m), bpos, bcrd, bval)
+    want = orc.spgemm(apos, acrd, aval, bpos, bcrd, bval, m)
+    p, c, v = rt.spgemm(A, B).to_arrays()
+    assert np.array_equal(p, want[0]) and np.array_equal(c, want[1])
+    assert not v.any() and not np.any(np.signbit(v))
+
+
 @pytest.mark.parametrize("medium", [False, True])
 @pytest.mark.parametrize("K,ldb,ldc,shift,accumulate", [(63, 63, 63, 0, False), (63, 63, 63, 0, True), (17, 53, 40, 0, True),
                                                         (64, 64, 64, 1, False), (64, 65, 67, 0, True), (99, 99, 100, 1, False)])
