@@ -209,9 +209,11 @@ struct Csr {
     Csr *transposed = nullptr;
     // the transpose of the structure with, as values, the place of every entry in this matrix (a mask's, for masked
     // products taken pair by pair); dup_state: 0 not looked at, 1 no row holds a column twice, 2 some row does; looked at
-    // with it, whether some entry lies on or above the diagonal (sides & 1) and on or below it (sides & 2)
+    // with it, whether some entry lies on or above the diagonal (sides & 1) and on or below it (sides & 2), and whether some
+    // row is much longer than the mean
     Csr *transposed_index = nullptr;
     int dup_state = 0, sides = 0;
+    bool uneven = false;
     // whether all stored values are the same number (a pattern matrix, as graph kernels use them): 0 not looked
     // at, 1 they are (iso_value), 2 they are not
     int iso_state = 0;
@@ -257,12 +259,9 @@ static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // exclusive scan of int64 counts into pos[0..n] (pos[n] = total), on the stream; total: a mailbox's word for the sum, or null
 int exclusive_scan_i64(const int64_t *counts, int64_t n, int64_t *pos, int64_t *total = nullptr);
 
-// stable radix sort of n (key, payload) pairs on the stream, comparing key bits [0, end_bit)
+// stable radix sort of n (key, payload) pairs on the stream, comparing key bits [begin_bit, end_bit)
 int sort_pairs_u64_u32(const uint64_t *keys_in, uint64_t *keys_out, const uint32_t *vals_in, uint32_t *vals_out,
-                       int64_t n, int end_bit);
-// radix sort of n keys on the stream, comparing bits [begin_bit, end_bit)
-template <typename KEY>
-int sort_keys(const KEY *in, KEY *out, int64_t n, int begin_bit, int end_bit);
+                       int64_t n, int end_bit, int begin_bit = 0);
 
 // deterministic tree sum of a device array, result copied to the host
 int reduce_sum_device(const double *v, int64_t n, double *out_host);

@@ -310,42 +310,22 @@ struct CachedBuf {
 };
 
 int sort_pairs_u64_u32(const uint64_t *keys_in, uint64_t *keys_out, const uint32_t *vals_in, uint32_t *vals_out,
-                       int64_t n, int end_bit)
+                       int64_t n, int end_bit, int begin_bit)
 {
     static Workspace tmp;
     if (n <= 0)
         return COMET_HIP_OK;
     size_t tmp_bytes = 0;
-    if (rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys_in, keys_out, vals_in, vals_out, (size_t)n, 0u,
+    if (rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys_in, keys_out, vals_in, vals_out, (size_t)n, (unsigned)begin_bit,
                                   (unsigned)end_bit, stream()) != hipSuccess)
         return set_error(COMET_HIP_ERR_HIP, "sort workspace query failed");
     COMET_CHK(tmp.ensure(tmp_bytes ? tmp_bytes : 1, false));
     KernelTimer t("radix_sort_pairs");
-    if (rocprim::radix_sort_pairs(tmp.ptr, tmp_bytes, keys_in, keys_out, vals_in, vals_out, (size_t)n, 0u,
+    if (rocprim::radix_sort_pairs(tmp.ptr, tmp_bytes, keys_in, keys_out, vals_in, vals_out, (size_t)n, (unsigned)begin_bit,
                                   (unsigned)end_bit, stream()) != hipSuccess)
         return set_error(COMET_HIP_ERR_HIP, "sorting %lld pairs failed", (long long)n);
     return COMET_HIP_OK;
 }
-
-template <typename KEY>
-int sort_keys(const KEY *in, KEY *out, int64_t n, int begin_bit, int end_bit)
-{
-    static Workspace tmp;
-    if (n <= 0)
-        return COMET_HIP_OK;
-    size_t tmp_bytes = 0;
-    if (rocprim::radix_sort_keys(nullptr, tmp_bytes, in, out, (size_t)n, (unsigned)begin_bit, (unsigned)end_bit, stream()) !=
-        hipSuccess)
-        return set_error(COMET_HIP_ERR_HIP, "sort workspace query failed");
-    COMET_CHK(tmp.ensure(tmp_bytes ? tmp_bytes : 1, false));
-    KernelTimer t("radix_sort_keys");
-    if (rocprim::radix_sort_keys(tmp.ptr, tmp_bytes, in, out, (size_t)n, (unsigned)begin_bit, (unsigned)end_bit, stream()) !=
-        hipSuccess)
-        return set_error(COMET_HIP_ERR_HIP, "sorting %lld keys failed", (long long)n);
-    return COMET_HIP_OK;
-}
-template int sort_keys<uint32_t>(const uint32_t *, uint32_t *, int64_t, int, int);
-template int sort_keys<uint64_t>(const uint64_t *, uint64_t *, int64_t, int, int);
 
 static inline dim3 grid_for(int64_t n) { return dim3((unsigned)(n > 0 ? ceil_div(n, 256) : 1)); }
 

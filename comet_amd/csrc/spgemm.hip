@@ -2629,9 +2629,10 @@ __global__ __launch_bounds__(256) void spgemm_dot_count(int64_t rb, int64_t re, 
 }
 
 // What a matrix is like, looked at once.  Of its structure (rows are sorted): some row holds a column twice, some entry lies
-// on or above the diagonal, some lies on or below it; of its values: they are not all the same, and the first one.
+// on or above the diagonal, some lies on or below it, some row is much longer than the mean; of its values: they are not all
+// the same, and the first one.
 struct CsrTraits {
-    int twice, above, below, differ;
+    int twice, above, below, uneven, differ, unused;
     double first;
 };
 // crd or val null: that part is not looked at.  A lane to every entry and to every row: of the few entries whose right
@@ -2639,11 +2640,11 @@ struct CsrTraits {
 // 15.7 M entries of the scale-20 R-MAT graph's lower triangle, the longest rows' way from turn to turn; 40 us now.)
 __global__ __launch_bounds__(256) void csr_traits(int64_t nrows, int64_t nnz, const int64_t *__restrict__ pos,
                                                   const int32_t *__restrict__ crd, const double *__restrict__ val,
-                                                  CsrTraits *__restrict__ out)
+                                                  int64_t even, CsrTraits *__restrict__ out)
 {
     const int64_t most = nnz > nrows ? nnz : nrows;
     const double first = val ? val[0] : 0.0;
-    bool twice = false, above = false, below = false, differ = false;
+    bool twice = false, above = false, below = false, uneven = false, differ = false;
     for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < most; t += (int64_t)gridDim.x * 256) {
         if (val && t < nnz)
             differ = differ || val[t] != first;
@@ -2653,6 +2654,7 @@ __global__ __launch_bounds__(256) void csr_traits(int64_t nrows, int64_t nnz, co
             const int64_t s = pos[t], e = pos[t + 1];
             above = above || (s < e && crd[e - 1] >= t);
             below = below || (s < e && crd[s] <= t);
+            uneven = uneven || e - s > even;
         }
         if (t + 1 < nnz && crd[t] == crd[t + 1]) {
             int64_t lo = 0, hi = nrows;          // the first row that begins behind entry t
@@ -2666,10 +2668,10 @@ __global__ __launch_bounds__(256) void csr_traits(int64_t nrows, int64_t nnz, co
             twice = twice || pos[lo] != t + 1;
         }
     }
-    const bool any[4] = {__any(twice) != 0, __any(above) != 0, __any(below) != 0, __any(differ) != 0};
+    const bool any[5] = {__any(twice) != 0, __any(above) != 0, __any(below) != 0, __any(uneven) != 0, __any(differ) != 0};
     if ((threadIdx.x & 63) == 0) {
         int *flags = &out->twice;
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < 5; ++k)
             if (any[k])
                 flags[k] = 1;
     }
@@ -3587,6 +3589,9 @@ static int dot_transposed_index(const Csr *x, Csr **out)
     return COMET_HIP_OK;
 }
 
+// rows are even where none is longer than this and this many times the mean
+constexpr int64_t CSR_EVEN_ROW = 24, CSR_EVEN_FACTOR = 8;
+
 // fills in what is not known yet of the two states; both together take one look and one wait
 static int csr_look(const Csr *x, bool structure, bool values)
 {
@@ -3597,13 +3602,14 @@ static int csr_look(const Csr *x, bool structure, bool values)
         return COMET_HIP_OK;
     CsrTraits *seen = nullptr;
     COMET_CHK(mailbox((void **)&seen));
-    *seen = CsrTraits{0, 0, 0, 1, 0.0};
+    *seen = CsrTraits{0, 0, 0, 0, 1, 0, 0.0};
     if (m->nnz > 0) {
         COMET_CHK(g_dot_flag.ensure(sizeof *seen, false));
         COMET_HIPCHK(hipMemsetAsync(g_dot_flag.ptr, 0, sizeof *seen, stream()));
         const int64_t blocks = ceil_div(std::max(m->nnz, m->nrows), 256);
         csr_traits<<<dim3((unsigned)std::min<int64_t>(blocks, 1 << 16)), dim3(256), 0, stream()>>>(
-            m->nrows, m->nnz, m->pos, structure ? m->crd : nullptr, values ? m->val : nullptr, (CsrTraits *)g_dot_flag.ptr);
+            m->nrows, m->nnz, m->pos, structure ? m->crd : nullptr, values ? m->val : nullptr,
+            CSR_EVEN_ROW + CSR_EVEN_FACTOR * (m->nnz / m->nrows), (CsrTraits *)g_dot_flag.ptr);
         COMET_HIPCHK(hipGetLastError());
         COMET_HIPCHK(hipMemcpyAsync(seen, g_dot_flag.ptr, sizeof *seen, hipMemcpyDeviceToHost, stream()));
         COMET_CHK(stream_wait());
@@ -3611,6 +3617,7 @@ static int csr_look(const Csr *x, bool structure, bool values)
     const volatile CsrTraits *t = seen;
     if (structure) {
         m->sides = (t->above ? 1 : 0) | (t->below ? 2 : 0);
+        m->uneven = t->uneven != 0;
         m->dup_state = t->twice ? 2 : 1;
     }
     if (values) {

@@ -6,12 +6,15 @@
 // Rows are therefore kept as words: the number of a group of sixteen vertices and a bit for each of them.  A triangle is
 // an edge and a vertex that both ends' rows hold; an edge costs the words of the shorter row, looked up in a table of the
 // longer one, and a word is a look-up for all its vertices: 1.1 G look-ups of 4 bytes instead of 2.3 G.
-// The plan is made at the first count, in the place of the plan of L's pairs, which costs as much: us of a first count /
-// and of each one after it, this form | the pairs of L as it is, R-MAT with 16 edges a vertex: n = 2^20 3790 / 903 | 4640 /
-// 1560, 200003 1146 / 279 | 1220 / 339, 60000 610 / 101 | 730 / 158, 20351 432 / 65 | 545 / 79, 1000 174 / 22 | 240 / 40.
-// Graphs without hubs gain less: uniform edges, n = 300000 and 3 a vertex 691 / 108 | 762 / 122, 16 a vertex 1360 / 164 |
-// 1296 / 211; a triangulated mesh of 10^6 1431 / 431 | 1288 / 423; and those of n = 5000 with 40 edges a vertex lose (301 / 59 |
-// 280 / 45: rows just above what a wavefront takes).  A band of 32 diagonals, n = 300000: 2009 / 153 | 2728 / 1183.
+// A graph whose rows of L are about equally long keeps its numbers: there are no hubs to bring together, its rows are as
+// short as they would be, and neighbours that lie next to each other stay there.
+// The plan is made at the first count, in the place of the plan of L's pairs, which costs as much or more: us of a first
+// count / of each one after it, this form | the pairs of L as it is, R-MAT with 16 edges a vertex: n = 2^20 4190 / 900 | 4650 /
+// 1560, 200003 1170 / 248 | 1220 / 339, 60000 640 / 101 | 725 / 158, 20351 455 / 66 | 535 / 79, 1000 200 / 23 | 235 / 40; rows
+// about equally long, uniform edges, 300000 vertices and 16 a vertex 820 / 166 | 1296 / 212, 30000 and 3 159 / 27 | 280 / 28, a
+// triangulated mesh of 10^6 947 / 430 | 1290 / 423, a band of 32 diagonals, 300000 1280 / 153 | 2730 / 1180.  Uniform graphs of
+// 30 to 100 edges a vertex and up to 20000 vertices have rows just above what a wavefront takes: 5000 and 40 184 / 58 |
+// 280 / 45.
 // Bound by the rows' way from the memory-side cache for large graphs (5 TB/s), by the chain of a wavefront - bounds of a
 // row, its table, its lists - for small ones.
 
@@ -39,7 +42,7 @@ __device__ __forceinline__ TriAlike tri_alike(int k, int lane)
 // Up to this many edges the plan counts - the entries of every column, the pairs of every end - where it sorts longer
 // arrays: a sort of so few entries takes twenty launches.  A first count, us, counting / sorting: 5000 vertices and 79
 // thousand edges 309 / 382, 20351 and 0.35 M 498 / 652, 60000 and 0.9 M 678 / 856; 200003 and 1.8 M 958 / 846, 3.5 M 1357 /
-// 1277, 2^20 and 15.7 M 5260 / 4180.
+// 1277, 2^20 and 15.7 M 5260 / 4180 (all with the vertices sorted by their edges, 50 to 200 us more than now).
 constexpr int64_t TRI_COUNTED = 1 << 20;
 
 // counts[c][v]: entries of column v that the workgroups c, c + copies, ... come to; copies is a power of two.  (Atomics on
@@ -55,35 +58,91 @@ __global__ __launch_bounds__(256) void tri_columns(int64_t n, int64_t nnz, const
         atomicAdd(&counts[(blockIdx.x & (copies - 1)) * n + v], (unsigned)t.all);
 }
 
-// a vertex has the entries of its row and of its column; starts, if given: entries of the columns before each
-__global__ __launch_bounds__(256) void tri_rank_keys(int64_t n, const int64_t *__restrict__ pos, unsigned copies,
-                                                     const unsigned *__restrict__ counts, const int64_t *__restrict__ starts,
-                                                     uint64_t *__restrict__ keys, uint32_t *__restrict__ idx)
+__global__ __launch_bounds__(256) void tri_column_keys(int64_t nnz, const int32_t *__restrict__ crd, uint64_t *__restrict__ keys)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n)
-        return;
-    unsigned degree = (unsigned)(pos[i + 1] - pos[i]);
-    if (starts)
-        degree += (unsigned)(starts[i + 1] - starts[i]);
-    for (unsigned c = 0; c < copies; ++c)
-        degree += counts[c * n + i];
-    keys[i] = 0xffffffffu - degree;
-    idx[i] = (uint32_t)i;
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p < nnz)
+        keys[p] = (uint64_t)crd[p];
 }
 
-__global__ __launch_bounds__(256) void tri_ranks(int64_t n, const uint32_t *__restrict__ by_degree, uint32_t *__restrict__ rank)
+// The vertices by their edges, most first, of equally many those first that were: places for each by counting, TRI_UNIT
+// vertices to a wavefront.  Up to 511 edges every number is a class of its own, above there are 32 to a factor of two.  (A
+// sort of so few keys takes up to 24 launches, 230 us for 2^20 vertices; this takes five.)
+constexpr int TRI_UNIT = 1024, TRI_CLASSES = 1024;
+__device__ __forceinline__ int tri_class(unsigned edges)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n)
-        rank[by_degree[i]] = (uint32_t)i;
+    const int log = 31 - __clz((int)edges);
+    return TRI_CLASSES - 1 - (edges < 512 ? (int)edges : 512 + (log - 9) * 32 + (int)(edges >> (log - 5) & 31u));
+}
+
+// An edge is an entry of the vertex' row or of its column: starts (if given) says how many the columns before each have,
+// otherwise counts does, copy by copy.  classes[v], and held[c * units + unit]: vertices of class c.
+constexpr unsigned TRI_COPIES = 16;          // at most
+__global__ __launch_bounds__(256) void tri_degrees(int64_t n, const int64_t *__restrict__ pos, unsigned copies,
+                                                   const unsigned *__restrict__ counts, const int64_t *__restrict__ starts,
+                                                   uint32_t *__restrict__ classes, int64_t *__restrict__ held)
+{
+    __shared__ unsigned here[TRI_CLASSES];
+    for (int c = threadIdx.x; c < TRI_CLASSES; c += 256)
+        here[c] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < TRI_UNIT; t += 256) {
+        const int64_t v = (int64_t)blockIdx.x * TRI_UNIT + t + threadIdx.x;
+        if (v < n) {
+            unsigned edges = (unsigned)(pos[v + 1] - pos[v]);
+            if (starts) {
+                edges += (unsigned)(starts[v + 1] - starts[v]);
+            } else {
+#pragma unroll
+                for (unsigned c = 0; c < TRI_COPIES; ++c) {          // all loads at once
+                    const unsigned held_there = counts[(c < copies ? c : 0u) * n + v];
+                    edges += c < copies ? held_there : 0u;
+                }
+            }
+            const int k = tri_class(edges);
+            classes[v] = (uint32_t)k;
+            atomicAdd(&here[k], 1u);
+        }
+    }
+    __syncthreads();
+    for (int c = threadIdx.x; c < TRI_CLASSES; c += 256)
+        held[(int64_t)c * gridDim.x + blockIdx.x] = here[c];
+}
+
+// rank[v]: v's new number; before[c * units + unit]: vertices of the classes before c, and of c in the units before
+__global__ __launch_bounds__(64) void tri_ranks(int64_t n, const uint32_t *__restrict__ classes,
+                                                const int64_t *__restrict__ before, uint32_t *__restrict__ rank)
+{
+    __shared__ unsigned next[TRI_CLASSES];
+    for (int c = threadIdx.x; c < TRI_CLASSES; c += 64)
+        next[c] = (unsigned)before[(int64_t)c * gridDim.x + blockIdx.x];
+    __syncthreads();
+    const int lane = threadIdx.x;
+    const int64_t first = (int64_t)blockIdx.x * TRI_UNIT + lane;
+    int ks[TRI_UNIT / 64];
+#pragma unroll
+    for (int t = 0; t < TRI_UNIT / 64; ++t)
+        ks[t] = first + 64 * t < n ? (int)classes[first + 64 * t] : -1;
+#pragma unroll
+    for (int t = 0; t < TRI_UNIT / 64; ++t) {
+        const int k = ks[t];
+        const TriAlike a = tri_alike(k, lane);
+        if (k >= 0)
+            rank[first + 64 * t] = next[k] + (unsigned)a.before;
+        __syncthreads();
+        if (k >= 0 && a.first == lane)
+            next[k] += (unsigned)a.all;
+        __syncthreads();
+    }
 }
 
 // keys[p] = larger new number << bits | smaller one, whatever rows the entries are of (a wavefront per row: 0.49 ms for
-// 15.7 M entries, most of it the longest row's)
+// 15.7 M entries, most of it the longest row's).  Without rank the numbers stay, or for an upper triangle are counted from
+// the last vertex, and the keys are in order.
 __global__ __launch_bounds__(256) void tri_edge_keys(int64_t n, int64_t nnz, const int64_t *__restrict__ pos,
                                                      const int32_t *__restrict__ crd, const uint32_t *__restrict__ rank,
-                                                     int bits, uint64_t *__restrict__ keys)
+                                                     bool upper, int bits, uint64_t *__restrict__ keys)
 {
     const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t first = uniform_i64_sg(p - (threadIdx.x & 63));
@@ -102,9 +161,16 @@ __global__ __launch_bounds__(256) void tri_edge_keys(int64_t n, int64_t nnz, con
     };
     const int64_t last = first + 63 < nnz ? first + 63 : nnz - 1;
     const int64_t lo = row_of(first, 0, n - 1), hi = row_of(last, lo, n - 1);
-    if (p < nnz) {
-        const uint64_t a = rank[row_of(p, lo, hi)], b = rank[crd[p]];
+    if (p >= nnz)
+        return;
+    const int64_t row = row_of(p, lo, hi);
+    if (rank) {
+        const uint64_t a = rank[row], b = rank[crd[p]];
         keys[p] = a > b ? a << bits | b : b << bits | a;
+    } else if (upper) {
+        keys[nnz - 1 - p] = (uint64_t)(n - 1 - row) << bits | (uint64_t)(n - 1 - crd[p]);
+    } else {
+        keys[p] = (uint64_t)row << bits | (uint64_t)crd[p];
     }
 }
 
@@ -117,8 +183,7 @@ __global__ __launch_bounds__(256) void tri_opens(int64_t nnz, const uint64_t *__
 }
 
 // at[r] = first p with keys[p] >> bits >= r, for r in [0, n]
-template <typename KEY>
-__global__ __launch_bounds__(256) void tri_row_starts(int64_t n, int64_t nnz, const KEY *__restrict__ keys, int bits,
+__global__ __launch_bounds__(256) void tri_row_starts(int64_t n, int64_t nnz, const uint64_t *__restrict__ keys, int bits,
                                                       int64_t *__restrict__ at)
 {
     const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -553,7 +618,7 @@ static int tri_plan(Csr *a, int only)
     // Scratch: three arrays of a 64-bit and two of a 32-bit word for every entry, two of a 64-bit word for every row, in one
     // allocation (each costs about as much as a small count).
     char *scratch = nullptr;
-    const size_t entries = ((size_t)std::max(nnz, n) + 64) & ~(size_t)63, rows = ((size_t)n + 65) & ~(size_t)63;
+    const size_t entries = ((size_t)std::max(nnz, n + TRI_UNIT) + 64) & ~(size_t)63, rows = ((size_t)n + 65) & ~(size_t)63;
     const int64_t quads_most = nnz / 4 + n + 2;
     const bool room =
         dev_malloc((void **)&scratch, 32 * entries + 16 * rows) == hipSuccess &&
@@ -565,31 +630,40 @@ static int tri_plan(Csr *a, int only)
     uint32_t *i0 = (uint32_t *)(r1 + rows), *i1 = i0 + entries;
     const auto run = [&]() -> int {
         KernelTimer t("triangle_plan");
-        uint32_t *rank = i0;
-        // ---- the vertices by their number of edges
-        if (nnz <= TRI_COUNTED) {
-            unsigned copies = 16, *counts = (unsigned *)k1;
-            while (sizeof(unsigned) * copies * (size_t)n > 8 * entries)
-                copies /= 2;
-            COMET_HIPCHK(hipMemsetAsync(counts, 0, sizeof(unsigned) * copies * (size_t)n, stream()));
-            tri_columns<<<per_entry, block, 0, stream()>>>(n, nnz, a->crd, copies, counts);
-            tri_rank_keys<<<per_row, block, 0, stream()>>>(n, a->pos, copies, counts, nullptr, k0, i0);
+        uint32_t *rank = i0, *classes = i1;
+        // ---- the edges in order of their rows, the vertices by their number of edges where that pays
+        if (a->uneven) {
+            unsigned copies = 0, *counts = nullptr;
+            int64_t *starts = nullptr;
+            if (nnz <= TRI_COUNTED) {
+                copies = TRI_COPIES, counts = (unsigned *)k1;
+                while (sizeof(unsigned) * copies * (size_t)n > 8 * entries)
+                    copies /= 2;
+                COMET_HIPCHK(hipMemsetAsync(counts, 0, sizeof(unsigned) * copies * (size_t)n, stream()));
+                tri_columns<<<per_entry, block, 0, stream()>>>(n, nnz, a->crd, copies, counts);
+            } else {
+                starts = r0;
+                tri_column_keys<<<per_entry, block, 0, stream()>>>(nnz, a->crd, k0);
+                COMET_CHK(sort_pairs_u64_u32(k0, k1, i0, i1, nnz, bits));          // (of the keys alone, see below)
+                tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, k1, 0, starts);
+            }
+            const unsigned units = (unsigned)ceil_div(n, TRI_UNIT);
+            tri_degrees<<<dim3(units), block, 0, stream()>>>(n, a->pos, copies, counts, starts, classes, w0);
+            COMET_CHK(exclusive_scan_i64(w0, (int64_t)units * TRI_CLASSES, (int64_t *)k0));
+            tri_ranks<<<dim3(units), dim3(64), 0, stream()>>>(n, classes, (const int64_t *)k0, rank);
+            tri_edge_keys<<<per_entry, block, 0, stream()>>>(n, nnz, a->pos, a->crd, rank, false, bits, k0);
+            // As far as the group of the smaller number: the order of the entries of a word does not matter.  What goes along is
+            // read by nobody; a sort of keys alone is a fifth quicker (3880 us for the first count of 2^20 vertices, this way
+            // 4240), but its code takes 4 ms to come to the device, once for every program that counts triangles.
+            COMET_CHK(sort_pairs_u64_u32(k0, k1, i0, i1, nnz, 2 * bits, TRI_GROUP_LOG));
         } else {
-            uint32_t *columns = (uint32_t *)k0;
-            COMET_CHK(sort_keys((const uint32_t *)a->crd, columns, nnz, 0, bits));
-            tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, (const uint32_t *)columns, 0, r0);
-            tri_rank_keys<<<per_row, block, 0, stream()>>>(n, a->pos, 0, nullptr, r0, k0, i0);
+            tri_edge_keys<<<per_entry, block, 0, stream()>>>(n, nnz, a->pos, a->crd, nullptr, a->sides == 1, bits, k1);
         }
-        COMET_CHK(sort_pairs_u64_u32(k0, k1, i0, i1, n, 32));
-        tri_ranks<<<per_row, block, 0, stream()>>>(n, i1, rank);
-        // ---- their rows
-        tri_edge_keys<<<per_entry, block, 0, stream()>>>(n, nnz, a->pos, a->crd, rank, bits, k0);
-        // (as far as the group of the smaller number: the order of the entries of a word does not matter)
-        COMET_CHK(sort_keys((const uint64_t *)k0, k1, nnz, TRI_GROUP_LOG, 2 * bits));
+        // ---- the rows
         int64_t *opens = (int64_t *)k0;
         tri_opens<<<per_entry, block, 0, stream()>>>(nnz, k1, opens);
         COMET_CHK(exclusive_scan_i64(opens, nnz, w0));
-        tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, (const uint64_t *)k1, bits, r0);
+        tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, k1, bits, r0);
         tri_row_quads<<<per_row, block, 0, stream()>>>(n, r0, w0, r1);
         COMET_CHK(exclusive_scan_i64(r1, n, side.kpos));
         tri_word_starts<<<per_row, block, 0, stream()>>>(n, side.kpos, plan.tpos);
@@ -607,7 +681,7 @@ static int tri_plan(Csr *a, int only)
         } else {
             tri_pairs<<<per_entry, block, 0, stream()>>>(n, nnz, k1, bits, plan.tpos, k0, i0, nullptr);
             COMET_CHK(sort_pairs_u64_u32(k0, k1, i0, i1, nnz, bits + 1));          // n is among the keys
-            tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, (const uint64_t *)k1, 0, side.kpos);
+            tri_row_starts<<<per_row, block, 0, stream()>>>(n, nnz, k1, 0, side.kpos);
             tri_entries<<<per_entry, block, 0, stream()>>>(n, nnz, k1, i1, plan.tpos, (PairEnt *)side.ent, work);
         }
         COMET_CHK(exclusive_scan_i64(work, nnz, w0));

@@ -542,8 +542,8 @@ def _edges(kind, rng):
         u = np.concatenate([np.arange(1, n), np.arange(2, n), [n - 1]])
         v = np.concatenate([np.zeros(n - 1, np.int64), np.arange(1, n - 1), [1]])
     else:
-        n, m = kind
-        u, v = rng.integers(0, n, (2, m)) if m else np.zeros((2, 0), np.int64)
+        n, m, hubs = (*kind, 1)[:3]          # hubs > 1: vertices with many edges, rows much longer than the mean
+        u, v = (n * rng.random((2, m)) ** hubs).astype(np.int64) if m else np.zeros((2, 0), np.int64)
         u, v = np.maximum(u, v)[u != v], np.minimum(u, v)[u != v]
     key = np.unique(np.asarray(u, np.int64) * n + v)
     return n, key // n, key % n
@@ -552,7 +552,8 @@ def _edges(kind, rng):
 @pytest.mark.parametrize("only", [None, "workgroup", "wavefront"])
 @pytest.mark.parametrize("upper", [False, True])
 @pytest.mark.parametrize("kind", ["complete", "dense", "star", "wheel", (1, 0), (2, 1), (15, 60), (16, 90), (17, 100), (33, 300),
-                                  (4097, 60_000), (100_003, 900_000), (1 << 20, 2_000_000), ((1 << 20) + 1, 500_000)])
+                                  (4097, 60_000), (100_003, 900_000), (1 << 20, 2_000_000), ((1 << 20) + 1, 500_000),
+                                  (511, 4000, 4), (1025, 30_000, 3), (20_001, 300_000, 4), (1 << 20, 2_000_000, 3)])
 def test_triangle_counts_of_every_kind_of_graph(kind, upper, only, monkeypatch):
     # both triangles of the matrix, rows through either kernel, numbers of vertices around a word's and the most that are
     # named in 16 + 4 bits; counts of one handle walk the vertices by their number of edges, a mask of its own walks L as it is
