@@ -1684,7 +1684,7 @@ static int spmv_run(Csr *a, int64_t x_dptr, int64_t y_dptr, int accumulate)
     // is made when it is multiplied again.
     const bool plan_now = a->spmv_uses > 0 || plan_at_once();
     a->spmv_uses = a->spmv_uses < 2 ? a->spmv_uses + 1 : 2;
-    if (plan_now && !plan_made([&] { return spmv_plan(a); }))
+    if (plan_now && a->spmv_nb == 0 && !plan_made([&] { return spmv_plan(a); }))
         a->spmv_nb = 1;
     const int nb = a->spmv_nb > 0 ? a->spmv_nb : 1;
     const unsigned blocks = (unsigned)ceil_div(a->nrows, SPMV_T);
@@ -1769,7 +1769,7 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
     // once goes through the chunk kernel whole, the plan is made when it is multiplied again.
     const bool plan_now = a->spmm_uses > 0 || plan_at_once();
     a->spmm_uses = a->spmm_uses < 2 ? a->spmm_uses + 1 : 2;
-    if (sweep_fits && plan_now)
+    if (sweep_fits && plan_now && a->heavy_state == 0)
         (void)plan_made([&] { return spmm_heavy_plan(a); });          // or the chunk kernel goes on taking all rows
     if (a->heavy_state != 2 || !sweep_fits)
         return spmm_chunks(a, K, B, ldb, C, ldc, accumulate);
