@@ -153,8 +153,8 @@ __device__ __forceinline__ void dot_walk(DotLists &lists, const PairSide &s, uin
 
 // ---------------------------------------------------------------------------
 // Rows of long tables: a workgroup per part of a row.  Large graphs are bound by the lists' way from the memory-side cache
-// (33 GB a call of 200003 vertices, edge factor 16, at 7.7 TB/s; a part of the lists for every XCD found more of them in
-// its L2 but built eight times the tables: 4.0 ms instead of 3.3), smaller ones, whose lists the L2 holds, by the vector
+// (200003 vertices, edge factor 16: 23.5 GB past the L2s in 3.2 ms, 7.3 TB/s, and 1.1 GB for the short rows beside it; a part
+// of the lists for every XCD found more of them in its L2 but built eight times the tables: 4.0 ms instead of 3.3), smaller ones, whose lists the L2 holds, by the vector
 // unit, busy two thirds of the time.  The first item of a workgroup is its own, not drawn: with one word to draw from, the
 // last of 256 began 3 us after the first.  Whole product: n = 200003 21.7 -> 3.6 ms, 20351 0.70 -> 0.24.  With values
 // read from LDS rather than by flat loads, sums over the lanes of a list by scalar masks, and two workgroups to a CU, us:

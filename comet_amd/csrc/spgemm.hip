@@ -2637,7 +2637,8 @@ struct CsrTraits {
 };
 // crd or val null: that part is not looked at.  A lane to every entry and to every row: of the few entries whose right
 // neighbour has the same column it is looked up whether a row ends between them.  (A wavefront to a row took 293 us for the
-// 15.7 M entries of the scale-20 R-MAT graph's lower triangle, the longest rows' way from turn to turn; 40 us now.)
+// 15.7 M entries of the scale-20 R-MAT graph's lower triangle, the longest rows' way from turn to turn; now 60 us with the
+// values.)
 __global__ __launch_bounds__(256) void csr_traits(int64_t nrows, int64_t nnz, const int64_t *__restrict__ pos,
                                                   const int32_t *__restrict__ crd, const double *__restrict__ val,
                                                   int64_t even, CsrTraits *__restrict__ out)

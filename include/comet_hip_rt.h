@@ -123,7 +123,8 @@ int comet_hip_spmv_csr_f64(int64_t csr, int64_t x_dptr, int64_t y_dptr, int accu
  * (elements).  accumulate as for SpMV.
  * Both products keep a plan in the handle (a re-ordered copy of parts of the
  * matrix) that costs tens of products to build: it is built when a handle is
- * multiplied for the second time, the first product runs without it.
+ * multiplied for the second time, the first product runs without it, and so
+ * does every product where there is no memory for it.
  * Rounding: a row that lies inside one 256-nonzero chunk is summed in nonzero
  * order with separate multiply and add, bit for bit as the reference's nest
  * (IndexTreeToSCF.cpp:203-205); a row cut by a chunk boundary adds its pieces
@@ -360,6 +361,9 @@ int64_t comet_hip_csr_transpose(int64_t csr);
  * kept in a's handle for four (b, mask) at most (8 bytes per entry of a, and a
  * copy of a's values in the plan's order where they are not all one number, so a
  * caller that writes into a's arrays calls comet_hip_csr_invalidate here too).
+ * Where a, b and mask are one strictly triangular pattern matrix of at most 2^20
+ * rows without repeated columns, the plan is the graph with its vertices in order
+ * of their edges instead (12 bytes per entry and 32 per row).
  * COMET_HIP_MASKED_SUM_ONLY=workgroup|wavefront in the environment
  * sends every row through one of the two kernels (a diagnostic: the tests use it). */
 int comet_hip_spgemm_masked_sum(int64_t a, int64_t b, int64_t mask, double *out);
