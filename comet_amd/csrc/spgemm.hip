@@ -2090,7 +2090,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_span_kernel(
     // a row's slices can be fetched ahead - the bounds of 64 rows at a time, a row's first entries of A two rows ahead and
     // their slices one.
     int64_t l_as = 0, l_coff = 0;
-    int l_cnt = 0;
+    int l_cnt = 0, l_out = 0;
     const auto load_entry = [&](int r, int base, int &k, double &a) {
         k = -1;
         a = 0.0;
@@ -2122,6 +2122,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_span_kernel(
         l_as = Apos[i];
         l_cnt = (int)(Apos[i + 1] - l_as);               // (the host sends matrices of under 2^30 entries here)
         l_coff = Cpos[i] - out0;
+        l_out = (int)(Cpos[i + 1] - Cpos[i]);
     }
     const int64_t left = (t_end - 1 - t0) / gridDim.x + 1;
     const int nr = __builtin_amdgcn_readfirstlane((int)(left < 64 ? left : 64));
@@ -2139,7 +2140,12 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_span_kernel(
         load_entry(r + 2, 0, k2, a2);
         const int64_t as = readlane_i64(l_as, r), coff = readlane_i64(l_coff, r);
         const int cnt = __builtin_amdgcn_readlane(l_cnt, r);
-        if (cnt == 1) {
+        bool copy = false;
+        if (cnt == 1) {          // and the row of B holds no column twice
+            const int64_t *bp = blkptr + (int64_t)Acrd[as] * (nblk + 1);
+            copy = __builtin_amdgcn_readfirstlane((int)(bp[nblk] - bp[0])) == __builtin_amdgcn_readlane(l_out, r);
+        }
+        if (copy) {
             // one entry of A: the row of C is that row of B times the entry (0 + a * b, as an accumulator that
             // starts at zero gives it).  70,000 rows of the R-MAT product at scale 20 are like that, each the
             // copy of a hub's row.
@@ -2157,7 +2163,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_span_kernel(
                     store_streaming(&Cval[off + q], 0.0 + a * Bval[bs + q]);
                 }
             }
-        } else if (cnt > 1) {
+        } else if (cnt > 0) {
             int64_t off = coff;
             int cb = 0;
             while (cb < nblk) {

@@ -487,6 +487,24 @@ def test_spgemm_keeps_entries_whose_products_underflow(wide, monkeypatch):
     assert not v.any() and not np.any(np.signbit(v))
 
 
+@pytest.mark.parametrize("semiring", [None, ("min", "plus"), ("max", "times"), ("any", "pair")])
+def test_spgemm_of_one_entry_and_a_row_with_repeated_columns(semiring, monkeypatch):
+    # a row of A with one entry copies its row of B where that is right: columns stored more than once are added up
+    monkeypatch.setenv("COMET_HIP_SPGEMM_WIDE", str(1 << 40))
+    rng = np.random.default_rng(5)
+    m, lens, repeats = 40_000, [600, 9000, 2500, 5000], [16, 1, 2, 1]
+    rows = [np.sort(rng.choice(m, l, replace=False)) for l in lens]
+    bcrd = np.concatenate([np.repeat(c, r) for c, r in zip(rows, repeats)]).astype(np.int64)
+    bpos = np.concatenate([[0], np.cumsum(np.multiply(lens, repeats))]).astype(np.int64)
+    apos, acrd = np.array([0, 1, 2, 3, 4, 6, 7]).astype(np.int64), np.array([0, 1, 2, 3, 0, 3, 0]).astype(np.int64)
+    pick = np.array([-3.0, -1.0, -0.0, 0.0, 1.0, 2.0])
+    aval, bval = rng.choice(pick, len(acrd)), rng.choice(pick, len(bcrd))
+    A, B = rt.CsrMatrix.from_arrays((6, 4), apos, acrd, aval), rt.CsrMatrix.from_arrays((4, m), bpos, bcrd, bval)
+    want = orc.spgemm(apos, acrd, aval, bpos, bcrd, bval, m, semiring=semiring)
+    p, c, v = rt.spgemm(A, B, semiring=semiring).to_arrays()
+    assert np.array_equal(p, want[0]) and np.array_equal(c, want[1]) and np.array_equal(v, want[2])
+
+
 @pytest.mark.parametrize("medium", [False, True])
 @pytest.mark.parametrize("K,ldb,ldc,shift,accumulate", [(63, 63, 63, 0, False), (63, 63, 63, 0, True), (17, 53, 40, 0, True),
                                                         (64, 64, 64, 1, False), (64, 65, 67, 0, True), (99, 99, 100, 1, False)])
