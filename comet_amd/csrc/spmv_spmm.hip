@@ -679,7 +679,7 @@ constexpr int spmm_hrows(int g) { return g * (SPMM_HW - 1) * SPMM_HR; }    // lo
 #define COMET_SPMM_MED_MIN 32
 #endif
 constexpr int SPMM_MED_MIN_LEN = COMET_SPMM_MED_MIN;   // such a row has at least this many nonzeros
-constexpr int SPMM_MSLOTS = 288;                        // sums a workgroup keeps in LDS: 144 KiB
+constexpr int SPMM_MSLOTS = 287;                        // sums a workgroup keeps in LDS, beside the entries of its lists (SWEEP_LDS)
 constexpr int SPMM_HEAVY_MIN_LEN = COMET_SPMM_HEAVY_MIN;              // a long row has at least this many nonzeros
 constexpr int64_t SPMM_UNEVEN_SWEEP = 24 << 20;         // bytes of B from which on rows of any alignment are swept
 constexpr int SPMM_HCB = 32;                         // column blocks a wavefront's list is cut into
@@ -919,6 +919,10 @@ __device__ inline void single_rows(const spmm_v4i *__restrict__ list, int64_t n,
         turn(std::integral_constant<int, 32>(), k + 1);
     }
 }
+
+// the sweep's LDS without the sums of the rows of middling length: 64 entries and a place of every wavefront
+constexpr size_t SWEEP_LDS = SPMM_HW * (64 * sizeof(spmm_v4i) + sizeof(int));
+static_assert(SWEEP_LDS + SPMM_MSLOTS * 64 * sizeof(double) <= 160 * 1024, "as many sums as a plan hands out fit a CU's LDS");
 
 template <bool SMALL, bool ACC>
 __global__ __launch_bounds__(SPMM_HW * 64) void spmm_heavy_sweep(
@@ -1336,12 +1340,13 @@ static Workspace g_heavy_partial, g_medium_partial;
 
 // Launches the sweep with `lds` bytes of dynamic LDS, asking for more than the 64 KiB a kernel gets by default.
 template <typename Kern, typename... Args>
-static void sweep_launch(Kern kernel, dim3 grid, dim3 block, size_t lds, Args... args)
+static int sweep_launch(Kern kernel, dim3 grid, dim3 block, size_t lds, Args... args)
 {
     if (lds > 64 * 1024)
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)lds);
+        COMET_HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         (int)lds));
     kernel<<<grid, block, lds, stream()>>>(args...);
+    return COMET_HIP_OK;
 }
 
 static int spmm_heavy_plan(Csr *a)
@@ -1806,18 +1811,14 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
         const bool small_b = a->ncols < (1 << 24) && ldb * 8 < (1 << 24) && a->ncols * ldb * 8 < (1ll << 32);
         const dim3 grid(8 * G, tiles), block(SPMM_HW * 64);
         const int slack = sweep_slack(ceil_div(a->ncols, 8), K);
-        if (small_b && accumulate)
-            sweep_launch(spmm_heavy_sweep<true, true>, grid, block, medium_lds, a->heavy_seg, a->heavy_ent, B, ldb, K, partial, C, ldc,
-                         G, ceil_div(a->ncols, 8), nslots, partial_medium, slack);
-        else if (small_b)
-            sweep_launch(spmm_heavy_sweep<true, false>, grid, block, medium_lds, a->heavy_seg, a->heavy_ent, B, ldb, K, partial, C, ldc,
-                         G, ceil_div(a->ncols, 8), nslots, partial_medium, slack);
-        else if (accumulate)
-            sweep_launch(spmm_heavy_sweep<false, true>, grid, block, medium_lds, a->heavy_seg, a->heavy_ent, B, ldb, K, partial, C, ldc,
-                         G, ceil_div(a->ncols, 8), nslots, partial_medium, slack);
+        const auto launch = [&](auto kernel) {
+            return sweep_launch(kernel, grid, block, medium_lds, a->heavy_seg, a->heavy_ent, B, ldb, K, partial, C, ldc, G,
+                                ceil_div(a->ncols, 8), nslots, partial_medium, slack);
+        };
+        if (small_b)
+            COMET_CHK(accumulate ? launch(spmm_heavy_sweep<true, true>) : launch(spmm_heavy_sweep<true, false>));
         else
-            sweep_launch(spmm_heavy_sweep<false, false>, grid, block, medium_lds, a->heavy_seg, a->heavy_ent, B, ldb, K, partial, C, ldc,
-                         G, ceil_div(a->ncols, 8), nslots, partial_medium, slack);
+            COMET_CHK(accumulate ? launch(spmm_heavy_sweep<false, true>) : launch(spmm_heavy_sweep<false, false>));
     }
     if (overlap) {      // the rows in between, on the CUs the sweep leaves free
         COMET_CHK(spmm_chunks(a->light, K, B, ldb, C, ldc, accumulate, aux_stream()));

@@ -237,7 +237,7 @@ def test_spmm_golden(golden, golden_dir):
 
 def _swept_rows(pos, K):
     """The rows the library hands to the column sweep (its rule restated), as (long, middling).  Middling: the rows
-    of 32 to 127 nonzeros and the long rows the sweep has no register for, longest first, at most 288 x g; their
+    of 32 to 127 nonzeros and the long rows the sweep has no register for, longest first, at most 287 x g; their
     sums are kept in LDS.  Long: at least 128 nonzeros, at most the
     120 x g longest (ties: lower row first) with g = 32 workgroups of the sweep per XCD - or 24, leaving CUs to
     the chunk kernel beside it, when the rows that are neither long (at g = 32) nor single hold a sixteenth of
@@ -256,7 +256,7 @@ def _swept_rows(pos, K):
     rows = rows[:120 * groups]
     if not (16 <= K <= 2048) or pos[-1] < (1 << 19) or 4 * lens[rows].sum() < pos[-1]:
         return rows[:0], rows[:0]
-    return rows, medium[:288 * groups]
+    return rows, medium[:287 * groups]
 
 
 def _by_length(lens, rows):
@@ -1471,6 +1471,23 @@ def test_spmm_more_long_rows_than_the_sweep_holds(groups, held, monkeypatch):
     crd = np.concatenate([np.sort(rng.choice(m, l, replace=False)) for l in lens]).astype(np.int64)
     val = rng.uniform(-1, 1, len(crd))
     assert _sweep_check(pos, crd, val, gen.dense((m, 64), seed=2)) == held
+
+
+@pytest.mark.parametrize("groups", [1, 2])
+def test_spmm_more_middling_rows_than_the_sweep_holds(groups, monkeypatch):
+    """900 rows of 100 nonzeros and long ones without a register: the LDS of one or two workgroups is full of sums, and the rows
+    that find no place there stay on the chunk kernel."""
+    monkeypatch.setenv("COMET_HIP_SPMM_GROUPS", str(groups))
+    monkeypatch.setenv("COMET_HIP_SPMM_MEDIUM", "1")
+    rng = np.random.default_rng(32)
+    n, m = 2000, 6000
+    lens = np.full(n, 3); lens[rng.choice(n, 1200, replace=False)] = np.repeat([1500, 100], [300, 900])
+    pos = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    assert pos[-1] >= 1 << 19
+    crd = np.concatenate([np.sort(rng.choice(m, l, replace=False)) for l in lens]).astype(np.int64)
+    val = rng.uniform(-1, 1, len(crd))
+    assert len(_swept_rows(pos, 64)[1]) == 287 * groups
+    assert _sweep_check(pos, crd, val, gen.dense((m, 64), seed=2)) == 120 * groups
 
 
 @pytest.mark.parametrize("acc", [False, True])
