@@ -4286,6 +4286,11 @@ extern "C" int comet_hip_debug_masked_sum_registers(int *workgroup_kernel, int *
 
 // Diagnostic: where the fp64 sums of the dot-product kernel begin in its LDS, in 32-bit words, for a bitmap of
 // `words` words (the counts beside it included); lets a CPU-side test sweep the invariant "even".
+extern "C" int comet_hip_debug_tri_bucket(int group, int attempt, int log_buckets)
+{
+    return tri_bucket((uint32_t)group << 16, tri_multiplier(attempt), log_buckets);
+}
+
 extern "C" int comet_hip_debug_dot_table_words(int words)
 {
     return dot_table_words(32 * (int64_t)(words < 1 ? 1 : words));

@@ -354,13 +354,31 @@ struct TriBitsProbe {
     }
 };
 // of a short one: its words in buckets of four
+// (The bucket of a word's group: the upper of the low 24 bits of its product with 0.618 x 2^24, or what is tried after that,
+// so that groups next to each other, as most are, come far apart.  The upper of 32 bits, as for the pairs of columns, put
+// six neighbours into one bucket of four and such rows were looked up by bisection: us a count, that way / this, R-MAT with
+// 16 edges a vertex, n = 200003 253 / 158, 60000 100 / 76, 20351 64 / 49, 5000 40 / 27, 1000 22 / 18; uniform edges, 5000 and
+// 40 a vertex 60 / 43, 3000 and 30 46 / 28, 1000 and 40 45 / 27.)
+constexpr int TRI_TRIES = 4;
+__host__ __device__ __forceinline__ uint32_t tri_multiplier(int attempt)
+{
+    return attempt == 0 ? 0x9E3779u : attempt == 1 ? 0x85EBCBu : attempt == 2 ? 0xC2B2AFu : 0x27D4EBu;
+}
+__host__ __device__ __forceinline__ int tri_bucket(uint32_t w, uint32_t mult, int log_nb)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return (int)__builtin_amdgcn_ubfe(__umul24(w >> 16, mult), 24 - log_nb, log_nb);
+#else
+    return (int)(((uint64_t)(w >> 16) * mult & 0xffffffu) >> (24 - log_nb));
+#endif
+}
 struct TriBucketProbe {
     const int *tab;
     uint32_t mult;
-    int shift;               // 32 - log2 of the buckets
+    int log_nb;              // log2 of the buckets
     __device__ __forceinline__ uint32_t common(uint32_t w) const
     {
-        const si_bucket b = *reinterpret_cast<const si_bucket *>(tab + 4 * BucketProbe::bucket((int)(w >> 16), mult, shift));
+        const si_bucket b = *reinterpret_cast<const si_bucket *>(tab + 4 * tri_bucket(w, mult, log_nb));
         const uint32_t x[4] = {(uint32_t)b.x ^ w, (uint32_t)b.y ^ w, (uint32_t)b.z ^ w, (uint32_t)b.w ^ w};
         uint32_t same = 0;           // where the group is the same: the bits that differ, turned over
 #pragma unroll
@@ -544,16 +562,15 @@ __global__ __launch_bounds__(PAIR_LIGHT_WAVES * 64, PAIR_LIGHT_OCC) void tri_lig
             int log_nb = 6;
             while (log_nb < PAIR_LIGHT_LOG && tlen > (1 << log_nb) * 3 / 4)
                 ++log_nb;
-            const int shift = 32 - log_nb;
             if (tlen <= PAIR_LIGHT_MAX) {
-                for (int attempt = 0; attempt < 4 && !hashed; ++attempt) {
-                    mult = attempt == 0 ? 0x9E3779u : attempt == 1 ? 0x85EBCBu : attempt == 2 ? 0xC2B2AFu : 0x27D4EBu;
+                for (int attempt = 0; attempt < TRI_TRIES && !hashed; ++attempt) {
+                    mult = tri_multiplier(attempt);
                     bool placed = true;
 #pragma unroll
                     for (int u = 0; u < PER; ++u) {
                         bool in = w[u] == 0;
                         if (!in) {
-                            int *bk = tab + 4 * BucketProbe::bucket((int)(w[u] >> 16), mult, shift);
+                            int *bk = tab + 4 * tri_bucket(w[u], mult, log_nb);
 #pragma unroll
                             for (int x = 0; x < 4; ++x)
                                 if (!in)
@@ -580,7 +597,7 @@ __global__ __launch_bounds__(PAIR_LIGHT_WAVES * 64, PAIR_LIGHT_OCC) void tri_lig
                 tri_sum(pend, probe, hits);
             };
             if (hashed)
-                walk(TriBucketProbe{tab, mult, shift});
+                walk(TriBucketProbe{tab, mult, log_nb});
             else
                 walk(TriBisectProbe{words + ts, tlen});
             all_hits += hits;

@@ -129,6 +129,7 @@ SIGNATURES = {
     "comet_hip_debug_masked_sum_registers": (_int, [C.POINTER(_int), C.POINTER(_int)]),
     "comet_hip_debug_fail_allocations": (None, [_i64, _i64]),
     "comet_hip_debug_sweep_slack": (_int, [_i64, _i64]),
+    "comet_hip_debug_tri_bucket": (_int, [_int, _int, _int]),
     "comet_hip_stream_create": (_i64, []),
     "comet_hip_stream_sync": (_int, [_i64]),
     "comet_hip_stream_destroy": (_int, [_i64]),

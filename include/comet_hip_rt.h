@@ -472,6 +472,10 @@ void comet_hip_debug_fail_allocations(int64_t after, int64_t count);
 /* Diagnostic: how far apart, in steps of 1024 columns, the wavefronts of the SpMM
  * column sweep may be in a matrix of ncols columns.  Runs on the host. */
 int comet_hip_debug_sweep_slack(int64_t ncols, int64_t K);
+/* Diagnostic: which of 2^log_buckets buckets of a short row's table in a triangle
+ * count a group of vertices goes to, at the attempt's (from 0) multiplier.  Runs
+ * on the host. */
+int comet_hip_debug_tri_bucket(int group, int attempt, int log_buckets);
 int comet_hip_gather_rows_bench(int64_t workgroups, int64_t per_wave, int64_t idx_dptr,
                                 int64_t table_dptr, int64_t table_rows, int64_t out_dptr);
 

@@ -181,3 +181,15 @@ def test_wavefronts_of_one_column_block_do_not_wait_for_each_other(ncols):
     for K in (16, 33, 48, 64, 130):
         slack = rt.lib().comet_hip_debug_sweep_slack(ncols, K)
         assert max(span, 2) <= slack <= max(span + 1, 3), K
+
+
+@pytest.mark.parametrize("log_buckets", [6, 7, 8])
+def test_groups_next_to_each_other_fit_the_buckets_of_a_triangle_count(log_buckets):
+    """A short row's table has buckets of four words and at most three words to four buckets: runs of groups, whole or with
+    gaps, have to go in at the first attempt (rows that do not are looked up by bisection)."""
+    L = rt.lib()
+    buckets = 1 << log_buckets
+    for step in (1, 2, 3):
+        for first in (0, 1, 37, 300, 5000, 65_535 - step * buckets):
+            run = [L.comet_hip_debug_tri_bucket(first + step * k, 0, log_buckets) for k in range(buckets * 3 // 4)]
+            assert min(run) >= 0 and np.bincount(run, minlength=buckets).max() <= 4 and max(run) < buckets, (step, first)
