@@ -236,9 +236,11 @@ __global__ __launch_bounds__(256) void pair_turn(int64_t nrows, const int64_t *_
 }
 
 // How a row is taken: parts of a heavy row in the low half, 1 for a light one in the high half.  only: 0 by the
-// table's length, 1 every row by workgroups, 2 every row by wavefronts.
+// table's length, 1 every row by workgroups, 2 every row by wavefronts.  A short table's row is light up to light_work
+// look-ups whatever a part of a heavy one has.
 __global__ void pair_parts(int64_t first, int64_t n, const int64_t *__restrict__ Tpos, const int64_t *__restrict__ kpos,
-                           const int64_t *__restrict__ wpos, int only, int light_max, int64_t *__restrict__ packed)
+                           const int64_t *__restrict__ wpos, int only, int light_max, int64_t light_work,
+                           int64_t *__restrict__ packed)
 {
     const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (x >= n)
@@ -248,7 +250,8 @@ __global__ void pair_parts(int64_t first, int64_t n, const int64_t *__restrict__
     int64_t v = 0;
     const int64_t share = wpos[n] / 2048, target = share > PAIR_ITEM_MIN ? share : PAIR_ITEM_MIN;
     // a short table may be paired with a hundred thousand lists: no wavefront gets more than a fraction of a part
-    const int64_t most_light = target / 8 < PAIR_LIGHT_WORK ? target / 8 : PAIR_LIGHT_WORK;
+    const int64_t fraction = target / 8 < PAIR_LIGHT_WORK ? target / 8 : PAIR_LIGHT_WORK;
+    const int64_t most_light = fraction > light_work ? fraction : light_work;
     if (kept > 0 && (only == 2 || (only == 0 && tlen <= light_max && work <= most_light))) {
         v = 1ll << 32;
     } else if (kept > 0) {
@@ -888,7 +891,7 @@ static int pair_side_plan(const Csr *T, const Csr *P, const Csr *L, int64_t firs
     pair_pass<true><<<grid, block, 0, stream()>>>(first, last, T->pos, P->pos, P->crd, L->pos, strict, xlo, xhi, kept_before,
                                                   work_before, plan->kpos, wpos, (PairEnt *)plan->ent, P->val, scale,
                                                   plan->weight, perm, out0, plan->place);
-    pair_parts<<<rows, block, 0, stream()>>>(first, n, T->pos, plan->kpos, wpos, only, light_max, parts);
+    pair_parts<<<rows, block, 0, stream()>>>(first, n, T->pos, plan->kpos, wpos, only, light_max, 0, parts);
     COMET_CHK(exclusive_scan_i64(parts, n, wpos));
     COMET_HIPCHK(hipMemcpyAsync(word, wpos + n, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
     COMET_CHK(stream_wait());

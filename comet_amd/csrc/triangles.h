@@ -9,12 +9,11 @@
 // A graph whose rows of L are about equally long keeps its numbers: there are no hubs to bring together, its rows are as
 // short as they would be, and neighbours that lie next to each other stay there.
 // The plan is made at the first count, in the place of the plan of L's pairs, which costs as much or more: us of a first
-// count / of each one after it, this form | the pairs of L as it is, R-MAT with 16 edges a vertex: n = 2^20 4190 / 900 | 4650 /
-// 1560, 200003 1170 / 248 | 1220 / 339, 60000 640 / 101 | 725 / 158, 20351 455 / 66 | 535 / 79, 1000 200 / 23 | 235 / 40; rows
-// about equally long, uniform edges, 300000 vertices and 16 a vertex 820 / 166 | 1296 / 212, 30000 and 3 159 / 27 | 280 / 28, a
-// triangulated mesh of 10^6 947 / 430 | 1290 / 423, a band of 32 diagonals, 300000 1280 / 153 | 2730 / 1180.  Uniform graphs of
-// 30 to 100 edges a vertex and up to 20000 vertices have rows just above what a wavefront takes: 5000 and 40 184 / 58 |
-// 280 / 45.
+// count / of each one after it, this form | the pairs of L as it is, R-MAT with 16 edges a vertex: n = 2^20 4140 / 792 | 4430 /
+// 1555, 200003 1120 / 161 | 1165 / 324, 60000 605 / 72 | 685 / 161, 20351 440 / 46 | 500 / 81, 1000 190 / 18 | 205 / 40; rows
+// about equally long, uniform edges, 300000 vertices and 16 a vertex 865 / 166 | 1290 / 208, 30000 and 3 153 / 26 | 230 / 28,
+// 5000 and 40 158 / 38 | 235 / 45, 1000 and 10 114 / 18 | 170 / 18, a triangulated mesh of 10^6 1000 / 428 | 1230 / 420, a
+// band of 32 diagonals, 300000 1330 / 148 | 2800 / 1185.
 // Bound by the rows' way from the memory-side cache for large graphs (5 TB/s), by the chain of a wavefront - bounds of a
 // row, its table, its lists - for small ones.
 
@@ -610,6 +609,12 @@ __global__ __launch_bounds__(PAIR_LIGHT_WAVES * 64, PAIR_LIGHT_OCC) void tri_lig
     pair_block_hits(wave_hits, all_hits, PAIR_LIGHT_WAVES, block_hits);
 }
 
+// A wavefront's row may have this many look-ups in a small graph too, whose parts of PAIR_ITEM_MIN would make it 2048: rows
+// of a hundred words are too little for a workgroup.  us a count, 2048 / 3072: uniform edges, 20000 vertices and 30 each
+// 61 / 43, 10000 and 40 64 / 48, 5000 and 40 43 / 38; R-MAT, 16 a vertex, 60000 76 / 71, 20351 49 / 46.  (4096 and more
+// are faster still for these, but take every row of some graphs from the workgroups.)
+constexpr int TRI_LIGHT_WORK = 3072;
+
 // ---------------------------------------------------------------------------
 // The plan, kept in the handle as tri (its side holds the pairs) with tri_state 2; 1: the matrix is not of the kind, or the
 // plan could not be made, and the pairs of L as it is serve all its counts.
@@ -703,7 +708,7 @@ static int tri_plan(Csr *a, int only)
         }
         COMET_CHK(exclusive_scan_i64(work, nnz, w0));
         tri_row_work<<<per_row, block, 0, stream()>>>(n, side.kpos, w0, r0);
-        pair_parts<<<per_row, block, 0, stream()>>>(0, n, plan.tpos, side.kpos, r0, only, PAIR_LIGHT_MAX, r1);
+        pair_parts<<<per_row, block, 0, stream()>>>(0, n, plan.tpos, side.kpos, r0, only, PAIR_LIGHT_MAX, TRI_LIGHT_WORK, r1);
         COMET_CHK(exclusive_scan_i64(r1, n, r0, word));
         COMET_CHK(stream_wait());
         const int64_t packed = *(volatile int64_t *)word;
