@@ -115,10 +115,10 @@ struct HeavyEnt {
 // the thresholds, so the seven lists a product of the benchmark takes are built once, not once per product.
 struct RowListEntry {
     uint64_t b_uid = 0, mask_uid = 0;
-    int64_t rb = 0, re = 0, dense_threshold = 0, wide_threshold = 0, mid_threshold = 0, mask_fill = 0;
+    int64_t rb = 0, re = 0, dense_threshold = 0, wide_threshold = 0, mid_threshold = 0, few_threshold = 0, mask_fill = 0;
     int32_t *rows = nullptr;     // device, re - rb entries
-    int64_t *bounds = nullptr;   // device, 4 entries
-    int64_t counts[4] = {-1, -1, -1, -1};          // the same, where the host has asked for them
+    int64_t *bounds = nullptr;   // device, 5 entries
+    int64_t counts[5] = {-1, -1, -1, -1, -1};          // the same, where the host has asked for them
 };
 uint64_t next_csr_uid();
 

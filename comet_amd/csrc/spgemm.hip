@@ -381,8 +381,9 @@ struct RowList {
     const int32_t *rows;       // row - row_begin, by descending number of products
     const int64_t *bounds;     // [0] rows with >= dense_threshold products, [1] rows with any product,
                                // [2] rows with >= wide_threshold products (a prefix of [0]),
-                               // [3] rows with >= mid_threshold products ([0] is a prefix of it)
-    int64_t counts[4];         // the same on the host where it has them, else -1
+                               // [3] rows with >= mid_threshold products ([0] is a prefix of it),
+                               // [4] rows with >= few_threshold products ([3] is a prefix of it)
+    int64_t counts[5];         // the same on the host where it has them, else -1
     // whether the host knows that there are none such (unknown counts are all -1, hence equal)
     bool only_heavy() const { return counts[1] >= 0 && counts[1] == counts[0]; }
     bool none_small() const { return counts[1] >= 0 && counts[1] == counts[3]; }
@@ -392,9 +393,11 @@ __device__ inline void list_range(const RowList &l, int part, int64_t *first, in
 {
     // part 0: the heavy rows, 1: the others that have products, 2: both, 3: the widest of the heavy rows,
     // 4: the heavy rows that are not among the widest, 5: the small rows, 6: those between the small and the heavy ones,
-    // 7: all but the small ones
-    *first = part == 1 || part == 6 ? l.bounds[0] : part == 4 ? l.bounds[2] : part == 5 ? l.bounds[3] : 0;
-    *end = part == 0 || part == 4 ? l.bounds[0] : part == 3 ? l.bounds[2] : part == 6 || part == 7 ? l.bounds[3] : l.bounds[1];
+    // 7: all but the small ones, 8: the small rows without, 9: those with the fewest products
+    *first = part == 1 || part == 6 ? l.bounds[0] : part == 4 ? l.bounds[2] : part == 5 || part == 8 ? l.bounds[3]
+             : part == 9 ? l.bounds[4] : 0;
+    *end = part == 0 || part == 4 ? l.bounds[0] : part == 3 ? l.bounds[2] : part == 6 || part == 7 ? l.bounds[3]
+           : part == 8 ? l.bounds[4] : l.bounds[1];
 }
 // A workgroup barrier that orders LDS traffic only.  __syncthreads() also makes every wavefront wait until its
 // global stores have been acknowledged, a microsecond that a kernel whose stores nobody reads back (the rows
@@ -2703,54 +2706,119 @@ __global__ void fill_iota_f64(int64_t n, double *__restrict__ out)
 // lanes to an entry a row of two hundred entries was thirteen times three loads one after the other, twice.)  us, structure
 // and values: A*A of R-MAT graphs of 65536 vertices, edge factor 16 96 + 379 -> 56 + 95, 30000 and 10 47 + 156 -> 26 + 48,
 // 16000 and 8 24 + 84 -> 17 + 34, 5000 and 12 17 + 36 -> 10 + 21.
+// Rows of a product a lane at most - all there are in products of meshes, bands and other graphs of a few edges a vertex -
+// are bound by instructions and barriers.  Up to 64 entries of A are therefore held by every wavefront, which finds its
+// products' entries by itself; the structure counts the columns that found their bit clear instead of going over the bitmap;
+// and where there are enough of them their values have a launch of their own, with half the registers.  us, structure and
+// values, sixteen lanes to an entry / eight products a lane / so: 65536 rows of 8 uniform entries 129 + 246 / 210 + 282 / 59 +
+// 194, 60000 rows of a band of 9 125 + 230 / 199 + 260 / 63 + 181, a mesh of 22500 18 + 48 / 44 + 70 / 22 + 35, 20000 rows of
+// a band of 15 32 + 63 / 54 + 74 / 31 + 48.
 // ---------------------------------------------------------------------------
 constexpr int SM_PER = 8;                           // products of a lane
 constexpr int SM_T = 256, SM_COLS = 1 << 16;
 constexpr int SM_MID_T = 512;                       // the lanes of a workgroup for twice as many
-constexpr int SM_PRODUCTS = SM_PER * SM_T, SM_MID_PRODUCTS = SM_PER * SM_MID_T;
+constexpr int64_t SM_FEW_ROWS = 2048;               // rows of few products that are worth a launch beside others' (4 us)
+constexpr int SM_FEW_PRODUCTS = SM_T, SM_PRODUCTS = SM_PER * SM_T, SM_MID_PRODUCTS = SM_PER * SM_MID_T;
 template <int T>
 struct SmallStage {
     int64_t start[T];                    // of the entries of A that have any: where their products begin in B, less their
     double a[T];                         // place among the products; A's value; the entry's place in the row
     int place[T];
     unsigned long long marks[SM_PER * T / 64];       // a bit where an entry's products begin; zero between passes
+    uint32_t own_marks[T / 64][2];       // the same for a wavefront that works by itself
     int tot[2][T / 64];
 };
-template <int T>
+template <int T, int PER>
 struct SmallRowLds {                     // behind the bitmap
-    double val[SM_PER * T];
+    double val[PER * T];
     SmallStage<T> stage;
-    uint16_t col[SM_PER * T];
+    uint16_t col[PER * T];
     int wave_tot[T / 64];
 };
-template <bool VALUES>
+template <bool VALUES, int PER>
 struct SmallProducts {
-    int col[SM_PER];                     // -1: none
-    double a[VALUES ? SM_PER : 1], b[VALUES ? SM_PER : 1];
-    int place[VALUES ? SM_PER : 1];
-    int64_t q[VALUES ? SM_PER : 1];      // the place in B
+    int col[PER];                        // -1: none
+    double a[VALUES ? PER : 1], b[VALUES ? PER : 1];
+    int place[VALUES ? PER : 1];
+    int64_t q[VALUES ? PER : 1];         // the place in B
 };
 
-// The lane's products of the entries [p0, ae) of a row of A, T of them at most.  The marks are left set: small_clear
-// behind the next barrier.
-template <bool VALUES, int T>
-__device__ __forceinline__ void small_products(SmallStage<T> &st, int64_t as, int64_t p0, int64_t ae,
-                                               const int32_t *__restrict__ Acrd, const double *__restrict__ Aval,
-                                               const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd,
-                                               const double *__restrict__ Bval, SmallProducts<VALUES> &out)
-{
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t p = p0 + tid;
-    int64_t bs = 0;
-    int len = 0;
+// A lane's entry of A: its row of B, or no products.
+struct SmallEntry {
+    int64_t start = 0;                   // in B
+    int len = 0, place = 0;              // products; the entry's place in its row, from 1 on
     double a = 0.0;
+};
+template <bool VALUES>
+__device__ __forceinline__ SmallEntry small_entry(int64_t as, int64_t p, int64_t ae, const int32_t *__restrict__ Acrd,
+                                                  const double *__restrict__ Aval, const int64_t *__restrict__ Bpos)
+{
+    SmallEntry e;
     if (p < ae) {
         const int k = Acrd[p];
-        bs = Bpos[k];
-        len = (int)(Bpos[k + 1] - bs);
-        if constexpr (VALUES)
-            a = Aval[p];
+        e.start = Bpos[k];
+        e.len = (int)(Bpos[k + 1] - e.start);
+        if constexpr (VALUES) {
+            e.a = Aval[p];
+            e.place = (int)(p - as) + 1;
+        }
     }
+    return e;
+}
+
+// Of a row whose entries of A every wavefront holds, lane by lane, and of T products at most: the lane's one.  No wavefront
+// waits for another.
+template <bool VALUES, int T, int PER>
+__device__ __forceinline__ void small_few(SmallStage<T> &st, const SmallEntry &e, const int32_t *__restrict__ Bcrd,
+                                          const double *__restrict__ Bval, SmallProducts<VALUES, PER> &out)
+{
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), base = 64 * wave;
+    const int inc = wave_inclusive_scan(e.len), total = __builtin_amdgcn_readlane(inc, 63);
+    out.col[0] = -1;
+    if (base >= total)
+        return;
+    const int off = inc - e.len;
+    const unsigned long long has = __ballot(e.len > 0);
+    const int below = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(has >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)has, 0));
+    // entry number x of those with products is that of lane by_rank[x]
+    const int by_rank = __builtin_amdgcn_ds_permute((e.len > 0 ? below : (int)__popcll(has) + lane - below) << 2, lane);
+    // an entry that begins at product s > base sets bit s - 1 - base: the bits below a lane are the entries up to its own
+    uint32_t *marks = st.own_marks[wave];
+    const uint32_t bit = (uint32_t)(off - 1 - base);
+    if (e.len > 0 && bit < 64u)
+        atomicOr(&marks[bit >> 5], 1u << (bit & 31u));
+    const int before = __popcll(__ballot(e.len > 0 && off <= base)) - 1;
+    wave_lds_order();
+    const uint2 m = *reinterpret_cast<const uint2 *>(marks);
+    wave_lds_order();
+    if (lane < 2)
+        marks[lane] = 0;
+    const int owner = lane_value(by_rank, (int)__builtin_amdgcn_mbcnt_hi(m.y, __builtin_amdgcn_mbcnt_lo(m.x, (uint32_t)before)));
+    const int64_t start = e.start - off;
+    const int64_t q = ((int64_t)lane_value((int)(start >> 32), owner) << 32 | (uint32_t)lane_value((int)start, owner)) + base + lane;
+    double a = 0.0;
+    int place = 0;
+    if constexpr (VALUES) {
+        a = __hiloint2double(lane_value(__double2hiint(e.a), owner), lane_value(__double2loint(e.a), owner));
+        place = lane_value(e.place, owner);
+    }
+    if (base + lane < total) {
+        out.col[0] = Bcrd[q];
+        if constexpr (VALUES) {
+            out.q[0] = q;
+            out.b[0] = Bval[q];
+            out.a[0] = a;
+            out.place[0] = place;
+        }
+    }
+}
+
+// Lays out the products of T entries of a row of A, one to a lane, and returns how many there are.  The marks are left set:
+// small_clear behind the next barrier.
+template <bool VALUES, int T>
+__device__ __forceinline__ int small_stage(SmallStage<T> &st, const SmallEntry &e)
+{
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), len = e.len;
     const int inc = wave_inclusive_scan(len);
     const unsigned long long has = __ballot(len > 0);
     if (lane == 63) {
@@ -2767,19 +2835,27 @@ __device__ __forceinline__ void small_products(SmallStage<T> &st, int64_t as, in
         total += st.tot[0][w];
     }
     if (len > 0) {
-        st.start[slot] = bs - off;
+        st.start[slot] = e.start - off;
         if constexpr (VALUES) {
-            st.a[slot] = a;
-            st.place[slot] = (int)(p - as) + 1;
+            st.a[slot] = e.a;
+            st.place[slot] = e.place;
         }
         atomicOr(&st.marks[off >> 6], 1ull << (off & 63));
     }
     lds_barrier();
-    static_assert(SM_PER * T / 64 <= 64, "a word of marks to a lane");
-    const unsigned long long word = lane < SM_PER * T / 64 ? st.marks[lane] : 0;
+    return __builtin_amdgcn_readfirstlane(total);
+}
+// The lane's products of those laid out, PER at most.
+template <bool VALUES, int T, int PER>
+__device__ __forceinline__ void small_products(SmallStage<T> &st, int total, const int32_t *__restrict__ Bcrd,
+                                               const double *__restrict__ Bval, SmallProducts<VALUES, PER> &out)
+{
+    const int tid = threadIdx.x, lane = tid & 63;
+    static_assert(PER * T / 64 <= 64, "a word of marks to a lane");
+    const unsigned long long word = lane < PER * T / 64 ? st.marks[lane] : 0;
     const int before = wave_inclusive_scan(__popcll(word)) - __popcll(word);
 #pragma unroll
-    for (int x = 0; x < SM_PER; ++x) {
+    for (int x = 0; x < PER; ++x) {
         const int t = tid + T * x, w = t >> 6;
         const unsigned lo = (unsigned)lane_value((int)word, w), hi = (unsigned)lane_value((int)(word >> 32), w);
         const int c = lane_value(before, w);
@@ -2858,6 +2934,8 @@ __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
     for (int w = threadIdx.x; w < words; w += SM_T)
         bm[w] = 0;
     small_clear(stage);
+    if ((threadIdx.x & 63) < 2)
+        stage.own_marks[threadIdx.x >> 6][threadIdx.x & 63] = 0;
     lds_barrier();
     SmallRows rows(list, 5, Apos, row_begin);
     while (rows.more()) {
@@ -2867,9 +2945,40 @@ __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
         rows.as = Apos[row_begin + rows.rn];
         rows.ae = Apos[row_begin + rows.rn + 1];
         rows.rn = rows.t + gridDim.x < rows.t_end ? list.rows[rows.t + gridDim.x] : rows.rn;
+        const bool held = ae - as <= 64;          // by every wavefront
+        SmallEntry e = small_entry<false>(as, as + (held ? threadIdx.x & 63 : threadIdx.x), ae, Acrd, nullptr, Bpos);
+        if (held && __builtin_amdgcn_readlane(wave_inclusive_scan(e.len), 63) <= SM_T) {
+            // a product to a lane: the columns are those that found their bit clear
+            SmallProducts<false, 1> it;
+            small_few<false, SM_T>(stage, e, Bcrd, nullptr, it);
+            const int j = it.col[0];
+            const uint32_t bit = 1u << (j & 31);
+            bool fresh = false;
+            if (j >= 0)
+                fresh = !(atomicOr(&bm[j >> 5], bit) & bit);
+            const int n = (int)__popcll(__ballot(fresh));
+            if ((threadIdx.x & 63) == 0)
+                wave_tot[threadIdx.x >> 6] = n;
+            lds_barrier();
+            if (threadIdx.x == 0) {
+                int all = 0;
+                for (int w = 0; w < SM_T / 64; ++w)
+                    all += wave_tot[w];
+                rowcount[r] = all;
+            }
+            if (j >= 0)
+                bm[j >> 5] = 0;
+            lds_barrier();
+            continue;
+        }
+        if (held && threadIdx.x >= 64)
+            e.len = 0;
         for (int64_t p0 = as; p0 < ae; p0 += SM_T) {
-            SmallProducts<false> it;
-            small_products<false, SM_T>(stage, as, p0, ae, Acrd, nullptr, Bpos, Bcrd, nullptr, it);
+            if (p0 > as)
+                e = small_entry<false>(as, p0 + threadIdx.x, ae, Acrd, nullptr, Bpos);
+            const int products = small_stage<false, SM_T>(stage, e);
+            SmallProducts<false, SM_PER> it;
+            small_products<false, SM_T, SM_PER>(stage, products, Bcrd, nullptr, it);
 #pragma unroll
             for (int x = 0; x < SM_PER; ++x)
                 if (it.col[x] >= 0)
@@ -3078,21 +3187,22 @@ __global__ __launch_bounds__(SMID_T, 8) void spgemm_symbolic_rows_kernel(
     }
 }
 
-template <bool SEMI, int T>
+// PER: products of a lane; part: the list's rows that are taken (PER = 1: of at most T products)
+template <bool SEMI, int T, int PER>
 __global__ __launch_bounds__(T) void spgemm_numeric_small_kernel(
-    int64_t row_begin, RowList list, int words, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
+    int64_t row_begin, RowList list, int part, int words, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
     const double *__restrict__ Aval, const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd,
     const double *__restrict__ Bval, const int64_t *__restrict__ Cpos, int32_t *__restrict__ Ccrd,
     double *__restrict__ Cval, int reduce_op, int mult_op)
 {
     uint32_t *bm = sg_dyn_lds;
     uint16_t *before = reinterpret_cast<uint16_t *>(bm + words);
-    SmallRowLds<T> &sh = *reinterpret_cast<SmallRowLds<T> *>(bm + words + words / 2);
+    SmallRowLds<T, PER> &sh = *reinterpret_cast<SmallRowLds<T, PER> *>(bm + words + words / 2);
     for (int w = threadIdx.x; w < words + words / 2 + (int)(sizeof sh / 4); w += T)
         bm[w] = 0;
     lds_barrier();
     const int64_t c0 = Cpos[row_begin];
-    SmallRows rows(list, T == SM_T ? 5 : 6, Apos, row_begin);
+    SmallRows rows(list, part, Apos, row_begin);
     while (rows.more()) {
         const int64_t as = rows.as, ae = rows.ae, coff = Cpos[row_begin + rows.r] - c0;
         rows.t += gridDim.x;
@@ -3100,11 +3210,20 @@ __global__ __launch_bounds__(T) void spgemm_numeric_small_kernel(
         rows.as = Apos[row_begin + rows.rn];
         rows.ae = Apos[row_begin + rows.rn + 1];
         rows.rn = rows.t + gridDim.x < rows.t_end ? list.rows[rows.t + gridDim.x] : rows.rn;
-        SmallProducts<true> it;
+        SmallProducts<true, PER> it;
+        const auto products = [&](int64_t p0) {
+            if (PER == 1 && ae - as <= 64) {
+                const SmallEntry e = small_entry<true>(as, as + (threadIdx.x & 63), ae, Acrd, Aval, Bpos);
+                small_few<true, T>(sh.stage, e, Bcrd, Bval, it);
+            } else {
+                const int n = small_stage<true, T>(sh.stage, small_entry<true>(as, p0 + threadIdx.x, ae, Acrd, Aval, Bpos));
+                small_products<true, T, PER>(sh.stage, n, Bcrd, Bval, it);
+            }
+        };
         for (int64_t p0 = as; p0 < ae; p0 += T) {
-            small_products<true, T>(sh.stage, as, p0, ae, Acrd, Aval, Bpos, Bcrd, Bval, it);
+            products(p0);
 #pragma unroll
-            for (int x = 0; x < SM_PER; ++x)
+            for (int x = 0; x < PER; ++x)
                 if (it.col[x] >= 0)
                     atomicOr(&bm[it.col[x] >> 5], 1u << (it.col[x] & 31));
             lds_barrier();
@@ -3114,12 +3233,12 @@ __global__ __launch_bounds__(T) void spgemm_numeric_small_kernel(
         lds_barrier();
         for (int64_t p0 = as; p0 < ae; p0 += T) {
             if (ae - as > T) {          // more entries than lanes: their products once more
-                small_products<true, T>(sh.stage, as, p0, ae, Acrd, Aval, Bpos, Bcrd, Bval, it);
+                products(p0);
                 lds_barrier();
                 small_clear(sh.stage);
             }
 #pragma unroll
-            for (int x = 0; x < SM_PER; ++x)
+            for (int x = 0; x < PER; ++x)
                 if (it.col[x] >= 0) {
                     const int j = it.col[x], r = before[j >> 5] + __popc(bm[j >> 5] & ((1u << (j & 31)) - 1u));
                     sh.col[r] = (uint16_t)j;
@@ -3235,15 +3354,16 @@ __global__ void sg_row_keys(int64_t n, const int64_t *__restrict__ rowprod, cons
 // bounds[0] = rows with >= threshold products, bounds[1] = rows with any, bounds[2] = rows with >= wide products,
 // in the sorted key array
 __global__ void sg_row_bounds(int64_t n, const uint64_t *__restrict__ keys, int64_t threshold, int64_t wide, int64_t middle,
-                              int64_t *__restrict__ bounds)
+                              int64_t few, int64_t *__restrict__ bounds)
 {
-    if (threadIdx.x > 3 || blockIdx.x > 0)
+    if (threadIdx.x > 4 || blockIdx.x > 0)
         return;
     // first key that is larger than the limit: keys ascend as products descend
     const uint64_t limit = threadIdx.x == 1 ? (uint64_t)((1ll << 62) - 1)
                                             : (uint64_t)((1ll << 62) - (threadIdx.x == 0   ? threshold
                                                                         : threadIdx.x == 2 ? wide
-                                                                                           : middle));
+                                                                        : threadIdx.x == 3 ? middle
+                                                                                           : few));
     int64_t lo = 0, hi = n;
     while (lo < hi) {
         const int64_t mid = (lo + hi) >> 1;
@@ -3268,12 +3388,14 @@ static SgRowLists g_rl;
 constexpr size_t SG_ROW_LISTS_KEPT = 24;
 static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64_t dense_threshold,
                        int64_t wide_threshold, RowList *out, const Csr *long_mask = nullptr,
-                       int64_t mask_fill = 0, bool want_counts = false, int64_t mid_threshold = -1)
+                       int64_t mask_fill = 0, bool want_counts = false, int64_t mid_threshold = -1, int64_t few_threshold = -1)
 {
     for (int64_t &c : out->counts)
         c = -1;
     if (mid_threshold < 0)
         mid_threshold = dense_threshold;
+    if (few_threshold < 0)
+        few_threshold = mid_threshold;
     const int64_t n = re - rb;
     const bool keep = getenv("COMET_HIP_SPGEMM_NO_LIST_CACHE") == nullptr;
     Csr *owner = const_cast<Csr *>(a);
@@ -3285,15 +3407,16 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
     key.dense_threshold = dense_threshold;
     key.wide_threshold = wide_threshold;
     key.mid_threshold = mid_threshold;
+    key.few_threshold = few_threshold;
     key.mask_fill = mask_fill;
     if (keep)
         for (const RowListEntry &e : owner->row_lists)
             if (e.b_uid == key.b_uid && e.mask_uid == key.mask_uid && e.rb == rb && e.re == re &&
                 e.dense_threshold == dense_threshold && e.wide_threshold == wide_threshold &&
-                e.mid_threshold == mid_threshold && e.mask_fill == mask_fill) {
+                e.mid_threshold == mid_threshold && e.few_threshold == few_threshold && e.mask_fill == mask_fill) {
                 out->rows = e.rows;
                 out->bounds = e.bounds;
-                std::copy(e.counts, e.counts + 4, out->counts);
+                std::copy(e.counts, e.counts + 5, out->counts);
                 return COMET_HIP_OK;
             }
     COMET_CHK(g_rl.rowprod.ensure(sizeof(int64_t) * (size_t)n, false));
@@ -3301,7 +3424,7 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
     COMET_CHK(g_rl.keys_out.ensure(8 * (size_t)n, false));
     COMET_CHK(g_rl.idx_in.ensure(4 * (size_t)n, false));
     COMET_CHK(g_rl.idx_out.ensure(4 * (size_t)n, false));
-    COMET_CHK(g_rl.bounds.ensure(32, false));
+    COMET_CHK(g_rl.bounds.ensure(40, false));
     int64_t *rowprod = (int64_t *)g_rl.rowprod.ptr;
     {
         KernelTimer t("spgemm_row_products");
@@ -3315,7 +3438,7 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
     COMET_CHK(sort_pairs_u64_u32((const uint64_t *)g_rl.keys_in.ptr, (uint64_t *)g_rl.keys_out.ptr,
                                  (const uint32_t *)g_rl.idx_in.ptr, (uint32_t *)g_rl.idx_out.ptr, n, 63));
     sg_row_bounds<<<dim3(1), dim3(64), 0, stream()>>>(n, (const uint64_t *)g_rl.keys_out.ptr, dense_threshold,
-                                                      wide_threshold, mid_threshold, (int64_t *)g_rl.bounds.ptr);
+                                                      wide_threshold, mid_threshold, few_threshold, (int64_t *)g_rl.bounds.ptr);
     COMET_HIPCHK(hipGetLastError());
     out->rows = (const int32_t *)g_rl.idx_out.ptr;
     out->bounds = (const int64_t *)g_rl.bounds.ptr;
@@ -3328,20 +3451,20 @@ static int sg_row_list(const Csr *a, const Csr *b, int64_t rb, int64_t re, int64
             owner->row_lists.erase(owner->row_lists.begin());
         }
         if (dev_malloc((void **)&key.rows, 4 * (size_t)n) != hipSuccess ||
-            dev_malloc((void **)&key.bounds, 32) != hipSuccess) {
+            dev_malloc((void **)&key.bounds, 40) != hipSuccess) {
             (void)hipGetLastError();
             (void)dev_free(key.rows);
             return COMET_HIP_OK;
         }
         COMET_HIPCHK(hipMemcpyAsync(key.rows, g_rl.idx_out.ptr, 4 * (size_t)n, hipMemcpyDeviceToDevice, stream()));
-        COMET_HIPCHK(hipMemcpyAsync(key.bounds, g_rl.bounds.ptr, 32, hipMemcpyDeviceToDevice, stream()));
+        COMET_HIPCHK(hipMemcpyAsync(key.bounds, g_rl.bounds.ptr, 40, hipMemcpyDeviceToDevice, stream()));
         if (want_counts) {          // once per list instead of once per product
             int64_t *word = nullptr;
             COMET_CHK(mailbox((void **)&word));
-            COMET_HIPCHK(hipMemcpyAsync(word, key.bounds, 32, hipMemcpyDeviceToHost, stream()));
+            COMET_HIPCHK(hipMemcpyAsync(word, key.bounds, 40, hipMemcpyDeviceToHost, stream()));
             COMET_CHK(stream_wait());
-            std::copy(word, word + 4, key.counts);
-            std::copy(word, word + 4, out->counts);
+            std::copy(word, word + 5, key.counts);
+            std::copy(word, word + 5, out->counts);
         }
         owner->row_lists.push_back(key);
         out->rows = key.rows;
@@ -3385,13 +3508,14 @@ static int64_t sg_wide_threshold(int64_t ncols, int nblk)
 // for a workgroup of 256 lanes.  Rows of mid up to dense products go to one of 512 lanes: 7000 of the rows of a product of
 // 65536 rows (R-MAT, 16 edges a row), 74 us there and 127 less in the kernel that visits the blocks, 12 and 40 of 980 us
 // in all with 30000 rows.  A matrix of half a block has no such rows: the kernel of whole blocks visits it once.
-struct SgClasses { int64_t mid, dense, wide; };
+struct SgClasses { int64_t few, mid, dense, wide; };
 static SgClasses sg_row_classes(int64_t ncols, bool small)
 {
     const int nblk = (int)ceil_div(ncols > 0 ? ncols : 1, SG_CB);
     SgClasses c;
     c.dense = !small ? SG_DENSE_PER_BLOCK * nblk : ncols <= SG_NARROW ? SM_PRODUCTS + 1 : SM_MID_PRODUCTS + 1;
     c.mid = small ? SM_PRODUCTS + 1 : c.dense;
+    c.few = small ? SM_FEW_PRODUCTS + 1 : c.mid;
     c.wide = std::max(sg_wide_threshold(ncols, nblk), c.dense);
     return c;
 }
@@ -3466,7 +3590,7 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
     const bool small = !m && b->ncols <= SM_COLS;
     const SgClasses classes = sg_row_classes(b->ncols, small);
     if (small)          // the list the numeric phase takes
-        COMET_CHK(sg_row_list(a, b, 0, a->nrows, classes.dense, classes.wide, &list, nullptr, 0, true, classes.mid));
+        COMET_CHK(sg_row_list(a, b, 0, a->nrows, classes.dense, classes.wide, &list, nullptr, 0, true, classes.mid, classes.few));
     else
         COMET_CHK(sg_row_list(a, b, 0, a->nrows, SG_NO_DENSE, SG_NO_DENSE, &list));
     COMET_CHK(g_sg.ticket.ensure(SG_TICKETS * sizeof(unsigned long long), false));
@@ -3719,7 +3843,7 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         COMET_CHK(sg_row_list(a, b, rb, re, 1ll << 61, 1ll << 61, &list, m, SG_HASH_FILL));
     else
         COMET_CHK(sg_row_list(a, b, rb, re, dense ? classes.dense : SG_NO_DENSE, dense ? classes.wide : SG_NO_DENSE, &list, nullptr,
-                              0, dense, dense ? classes.mid : -1));
+                              0, dense, dense ? classes.mid : -1, dense ? classes.few : -1));
     uint32_t *gbm = nullptr, *gmask = nullptr;
     if (!small) {
         if (!g.lds || m) {          // the output row's bitmap is in HBM when LDS holds the mask row instead
@@ -3751,20 +3875,27 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
     if (small) {
         const int words = sm_words(b->ncols);
         const bool known = list.counts[0] >= 0;
-        const auto launch = [&](auto kernel, int lanes, size_t behind, int64_t rows, int per_cu) -> int {
+        const auto launch = [&](auto kernel, int part, int lanes, size_t behind, int64_t rows, int per_cu) -> int {
             const size_t lds = sizeof(uint32_t) * (size_t)(words + words / 2) + behind;
             KernelTimer t(semi ? "spgemm_numeric_semiring" : "spgemm_numeric");
             COMET_CHK(sg_allow_lds(kernel, lds));
             kernel<<<sm_grid(known ? rows : -1, per_cu), dim3(lanes), lds, stream()>>>(
-                rb, list, words, a->pos, a->crd, a->val, b->pos, b->crd, b->val, Cpos, Ccrd, Cval, reduce_op, mult_op);
+                rb, list, part, words, a->pos, a->crd, a->val, b->pos, b->crd, b->val, Cpos, Ccrd, Cval, reduce_op, mult_op);
             return COMET_HIP_OK;
         };
-        if (!list.none_small())
-            COMET_CHK(launch(semi ? spgemm_numeric_small_kernel<true, SM_T> : spgemm_numeric_small_kernel<false, SM_T>, SM_T,
-                             sizeof(SmallRowLds<SM_T>), list.counts[1] - list.counts[3], 7));
+        // rows of few products by a launch of their own, unless they are too few beside others to be worth it
+        const int64_t few = known ? list.counts[1] - list.counts[4] : 0;
+        const bool apart = few >= SM_FEW_ROWS || (few > 0 && list.counts[4] == list.counts[3]);
+        if (apart)
+            COMET_CHK(launch(semi ? spgemm_numeric_small_kernel<true, SM_T, 1> : spgemm_numeric_small_kernel<false, SM_T, 1>, 9, SM_T,
+                             sizeof(SmallRowLds<SM_T, 1>), few, 7));
+        if (!list.none_small() && !(apart && list.counts[4] == list.counts[3]))
+            COMET_CHK(launch(semi ? spgemm_numeric_small_kernel<true, SM_T, SM_PER> : spgemm_numeric_small_kernel<false, SM_T, SM_PER>,
+                             apart ? 8 : 5, SM_T, sizeof(SmallRowLds<SM_T, SM_PER>),
+                             list.counts[apart ? 4 : 1] - list.counts[3], 7));
         if (classes.mid < classes.dense && !list.none_mid())
-            COMET_CHK(launch(semi ? spgemm_numeric_small_kernel<true, SM_MID_T> : spgemm_numeric_small_kernel<false, SM_MID_T>,
-                             SM_MID_T, sizeof(SmallRowLds<SM_MID_T>), list.counts[3] - list.counts[0], 2));
+            COMET_CHK(launch(semi ? spgemm_numeric_small_kernel<true, SM_MID_T, SM_PER> : spgemm_numeric_small_kernel<false, SM_MID_T, SM_PER>,
+                             6, SM_MID_T, sizeof(SmallRowLds<SM_MID_T, SM_PER>), list.counts[3] - list.counts[0], 2));
     } else if (list.only_heavy()) {
         // nothing for these kernels
     } else if (g.lds) {

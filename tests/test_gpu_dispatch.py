@@ -487,6 +487,39 @@ def test_spgemm_keeps_entries_whose_products_underflow(wide, monkeypatch):
     assert not v.any() and not np.any(np.signbit(v))
 
 
+@pytest.mark.parametrize("semiring", [None, ("min", "plus"), ("any", "second")])
+@pytest.mark.parametrize("ncols", [40, 9000, 65_536])
+@pytest.mark.parametrize("times,others", [(1, True), (1, False), (70, True), (70, False)])
+def test_spgemm_rows_of_a_product_a_lane(times, others, ncols, semiring):
+    # rows around 64 entries and 256 products, entries without products among them, columns that meet and that are stored
+    # twice; few and many such rows, alone and beside rows with more products
+    rng = np.random.default_rng(ncols + times)
+    blens = np.array([0, 0, 1, 1, 1, 2, 3, 4, 5, 8, 17, 33] * 12)
+    bcrd = np.concatenate([np.sort(rng.integers(0, ncols, l)) for l in blens]).astype(np.int64)
+    bpos = np.concatenate([[0], np.cumsum(blens)]).astype(np.int64)
+    k, ones = len(blens), np.flatnonzero(blens == 1)
+    rows = [[], [0], [2], [11]]
+    for entries in (1, 2, 15, 16, 17, 63, 64, 65, 100):
+        rows.append(np.sort(rng.choice(k, entries, replace=False)))
+    for products in (63, 64, 65, 127, 128, 129, 255, 256, 257):          # as few entries as make them up, and single ones
+        row, left = [], products
+        for r in np.argsort(-blens, kind="stable"):
+            if 0 < blens[r] <= left and blens[r] > 1:
+                row.append(r)
+                left -= blens[r]
+        rows.append(np.sort(np.concatenate([row, ones[:left]]).astype(np.int64)))
+    rows = [r for r in rows if others or blens[np.asarray(r, int)].sum() <= 256] * times
+    apos = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int64)
+    acrd = np.concatenate(rows).astype(np.int64)
+    pick = np.array([-3.0, -1.0, 0.5, 1.0, 2.0])
+    aval, bval = rng.choice(pick, len(acrd)), rng.choice(pick, len(bcrd))
+    A, B = rt.CsrMatrix.from_arrays((len(rows), k), apos, acrd, aval), rt.CsrMatrix.from_arrays((k, ncols), bpos, bcrd, bval)
+    want = orc.spgemm(apos, acrd, aval, bpos, bcrd, bval, ncols, semiring=semiring)
+    p, c, v = rt.spgemm(A, B, semiring=semiring).to_arrays()
+    assert np.array_equal(p, want[0]) and np.array_equal(c, want[1])
+    assert np.array_equal(v, want[2])          # quarters of whole numbers: sums are exact
+
+
 @pytest.mark.parametrize("semiring", [None, ("min", "plus"), ("max", "times"), ("any", "pair")])
 def test_spgemm_of_one_entry_and_a_row_with_repeated_columns(semiring, monkeypatch):
     # a row of A with one entry copies its row of B where that is right: columns stored more than once are added up
