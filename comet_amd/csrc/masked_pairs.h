@@ -779,30 +779,36 @@ __global__ __launch_bounds__(256) void pair_sum_partial(PairSide s0, PairSide s1
         partial[blockIdx.x] = lds[0];
 }
 
-// The result to the host's word, the ticket back to zero for the next call.  partial: n sums, or null: block_hits, n counts.
+// The result to the host's word, the ticket back to zero for the next call: of 256 sums, and of n workgroups' hits, whose
+// wavefronts add them up by themselves (a tree over 256 lanes with a barrier to each step took up to 1 us more).
 __global__ __launch_bounds__(256) void pair_sum_finish(unsigned long long *__restrict__ tickets,
-                                                       const double *__restrict__ partial,
-                                                       const unsigned long long *__restrict__ block_hits, int n, double each,
-                                                       double *__restrict__ result)
+                                                       const double *__restrict__ partial, double *__restrict__ result)
 {
     __shared__ double lds[256];
-    __shared__ unsigned long long counts[256];
-    unsigned long long mine = 0;
-    if (!partial)
-        for (int i = threadIdx.x; i < n; i += 256)
-            mine += block_hits[i];
-    counts[threadIdx.x] = mine;
-    lds[threadIdx.x] = partial && (int)threadIdx.x < n ? partial[threadIdx.x] : 0.0;
+    lds[threadIdx.x] = partial[threadIdx.x];
     __syncthreads();
     for (int d = 128; d > 0; d >>= 1) {
-        if ((int)threadIdx.x < d) {
+        if ((int)threadIdx.x < d)
             lds[threadIdx.x] += lds[threadIdx.x + d];
-            counts[threadIdx.x] += counts[threadIdx.x + d];
-        }
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        *result = partial ? lds[0] * each : counts[0] ? (double)counts[0] * each : 0.0;
+        *result = lds[0];
+        tickets[0] = 0;
+    }
+}
+constexpr int PAIR_HITS_T = 1024;
+__global__ __launch_bounds__(PAIR_HITS_T) void pair_hits_finish(unsigned long long *__restrict__ tickets,
+                                                                const unsigned long long *__restrict__ block_hits, int n,
+                                                                double each, double *__restrict__ result)
+{
+    __shared__ unsigned long long wave_hits[PAIR_HITS_T / 64], all;
+    unsigned long long mine = 0;
+    for (int i = threadIdx.x; i < n; i += PAIR_HITS_T)
+        mine += block_hits[i];
+    pair_block_hits(wave_hits, mine, PAIR_HITS_T / 64, &all);
+    if (threadIdx.x == 0) {
+        *result = all ? (double)all * each : 0.0;
         tickets[0] = 0;
     }
 }
@@ -1114,8 +1120,11 @@ static int pair_masked_sum(Csr *a, Csr *b, Csr *m, double *result)
         KernelTimer t("spgemm_masked_sum_reduce");
         pair_sum_partial<<<dim3(256), dim3(256), 0, stream()>>>(s0, s1, out, partial);
     }
-    pair_sum_finish<<<dim3(1), dim3(256), 0, stream()>>>(tickets, partial, hits, one ? (int)(grids.heavy + grids.light) : 256,
-                                                         one ? a->iso_value * b->iso_value : 1.0, word);
+    if (one)
+        pair_hits_finish<<<dim3(1), dim3(PAIR_HITS_T), 0, stream()>>>(tickets, hits, (int)(grids.heavy + grids.light),
+                                                                      a->iso_value * b->iso_value, word);
+    else
+        pair_sum_finish<<<dim3(1), dim3(256), 0, stream()>>>(tickets, partial, word);
     COMET_HIPCHK(hipGetLastError());
     COMET_CHK(stream_wait());
     *result = *(volatile double *)word;

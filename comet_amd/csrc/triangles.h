@@ -752,7 +752,8 @@ static int tri_count(Csr *a, double *result)
         KernelTimer t("spgemm_masked_sum_small");
         tri_light_kernel<<<dim3(grids.light), dim3(PAIR_LIGHT_WAVES * 64), 0, stream()>>>(s, hits + grids.heavy);
     }
-    pair_sum_finish<<<dim3(1), dim3(256), 0, stream()>>>(tickets, nullptr, hits, (int)(grids.heavy + grids.light), a->iso_value * a->iso_value, word);
+    pair_hits_finish<<<dim3(1), dim3(PAIR_HITS_T), 0, stream()>>>(tickets, hits, (int)(grids.heavy + grids.light),
+                                                                  a->iso_value * a->iso_value, word);
     COMET_HIPCHK(hipGetLastError());
     COMET_CHK(stream_wait());
     *result = *(volatile double *)word;
