@@ -2123,7 +2123,8 @@ extern "C" int comet_hip_densemat_csr_f64(int64_t csr, int64_t M, int64_t a_dptr
 // A wavefront takes 64 stored entries, KT = 16 columns of C and of the transposed D at a time: a group of eight lanes has
 // eight entries next to each other, and loads 128 bytes of each one's row of D, 16 a lane - the row of C only where it
 // is not that of the entry before, and entries of one row lie together.  The products go to LDS, and lane e adds those
-// of entry e in ascending k while the next 16 columns are on their way.  (Sixteen entries and 64 columns at a time read C
+// of entry e in ascending k while the next 16 columns are on their way.  (Other numbers of entries and columns at a time: where
+// they are chosen.)  (Sixteen entries and 64 columns at a time read C
 // for every entry and left three quarters of the lanes idle in the sums: whole call, 250000 rows of 16 entries, K = 64
 // 301 -> 227 us, K = 48 217 -> 140, K = 33 213 -> 170; 500000 rows, K = 15 217 -> 199, K = 3 150 -> 137.)  Bound by the
 // way of D's rows from the L2s: 16 of the 18.6 M lines that the CUs ask for at K = 64, 80 of them under way a CU, a third
@@ -2194,60 +2195,71 @@ __global__ __launch_bounds__(SDDMM_W * 64, 4) void sddmm_kernel(int64_t nnz, con
         if (n & 1)
             t = t + mine[q].x;
     };
-    int64_t kc = 0;
-    if (K >= KT) {
+    // Pieces of KT columns, a last one of more than half as many like them, the lanes behind its end idle; a shorter rest
+    // takes as many lanes to an entry as it has columns for, two a lane.  The next piece is on its way while one is added (the
+    // rest too took more registers than there are).
+    const int64_t whole = K / KT;
+    const int rest = (int)(K - whole * KT);
+    const int64_t pieces = whole + (rest > KT / 2 ? 1 : 0);
+    const int rn = pieces > whole ? 0 : rest;
+    spmm_pair c[R], d[R];
+    if (pieces > 0) {
         const int g = lane / LANES, sub = lane % LANES;
         const unsigned kept = (unsigned)(again >> (R * g)) & ~1u;      // bit u: the row of C is there already
+        // in a last piece: one column back where the lane has one only, to the first where it has none
+        const bool half = rest - 1 == 2 * sub;
+        const int back = half ? 1 : 2 * sub < rest ? 0 : 2 * sub;
         typename At::Off co[R], dO[R];
 #pragma unroll
         for (int u = 0; u < R; ++u) {
             co[u] = At::row(__shfl(my_row, R * g + u, 64), ldc, 2 * sub);
             dO[u] = At::row(__shfl(my_col, R * g + u, 64), ldt, 2 * sub);
         }
-        spmm_pair c[R], d[R];
-        const auto load = [&](int64_t k) {
-            const double *Ck = C + k, *Dk = Dt + k;
+        const auto load = [&](int64_t i) {
+            const double *Ck = C + i * KT, *Dk = Dt + i * KT;
+            const typename At::Off less = i == whole ? (typename At::Off)back * 8 : 0;
 #pragma unroll
             for (int u = 0; u < R; ++u) {
                 if (!(kept >> u & 1u))
-                    c[u] = *reinterpret_cast<const spmm_pair *>(At::at(Ck, co[u]));
-                d[u] = *reinterpret_cast<const spmm_pair *>(At::at(Dk, dO[u]));
+                    c[u] = *reinterpret_cast<const spmm_pair *>(At::at(Ck, co[u] - less));
+                d[u] = *reinterpret_cast<const spmm_pair *>(At::at(Dk, dO[u] - less));
             }
         };
         load(0);
-        for (; kc + KT <= K; kc += KT) {
+        for (int64_t i = 0; i < pieces; ++i) {
+            const bool one = half && i == whole;
             spmm_pair cur = c[0];
 #pragma unroll
             for (int u = 0; u < R; ++u) {
                 cur.x = kept >> u & 1u ? cur.x : c[u].x;
                 cur.y = kept >> u & 1u ? cur.y : c[u].y;
-                *reinterpret_cast<double2 *>(tile + (R * g + u) * LD + 2 * sub) =
-                    make_double2(cur.x * d[u].x, cur.y * d[u].y);
+                double2 q = make_double2(cur.x * d[u].x, cur.y * d[u].y);
+                if (one)
+                    q.x = q.y;
+                *reinterpret_cast<double2 *>(tile + (R * g + u) * LD + 2 * sub) = q;
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-            if (kc + 2 * KT <= K)
-                load(kc + KT);
-            sum(KT);
+            if (i + 1 < pieces)
+                load(i + 1);
+            sum(i < whole ? KT : rest);
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
         }
     }
-    if (kc < K) {                        // fewer than 16 columns: as many lanes to an entry as they take, two columns a lane
-        const int kn = (int)(K - kc), L = (kn + 1) / 2, G = 64 / L, rounds = (E + G - 1) / G;
-        const int g = lane / L, sub = lane - g * L;
-        // the last lane of an odd kn has one column, and reads the one before it as well, if there is one
-        const bool half = sub == L - 1 && (kn & 1);
-        const int64_t from = kc + 2 * sub - (half && kc + 2 * sub > 0 ? 1 : 0);
-        const int e0 = g * rounds;
-        const unsigned kept = (unsigned)(again >> (e0 & 63)) & ~1u;
-        spmm_pair c[R], d[R];
+    if (rn > 0) {
+        const int rL = (rn + 1) / 2, rG = 64 / rL, rounds = (E + rG - 1) / rG;
+        const int rg = lane / rL, rsub = lane - rg * rL, e0 = rg * rounds;
+        // the last lane of an odd number has one column, and reads the one before it as well, if there is one
+        const bool rhalf = rsub == rL - 1 && (rn & 1);
+        const unsigned rkept = (unsigned)(again >> (e0 & 63)) & ~1u;
+        const int64_t from = K - rn + 2 * rsub, at = from - (rhalf && from > 0 ? 1 : 0);
 #pragma unroll
         for (int u = 0; u < R; ++u) {
             if (u < rounds) {
                 const int e = e0 + u < E ? e0 + u : E - 1;
                 const int r = __shfl(my_row, e, 64), j = __shfl(my_col, e, 64);
-                const double *cp = At::at(C, At::row(r, ldc, from)), *dp = At::at(Dt, At::row(j, ldt, from));
+                const double *cp = At::at(C, At::row(r, ldc, at)), *dp = At::at(Dt, At::row(j, ldt, at));
                 if (K > 1) {
-                    if (!(kept >> u & 1u))
+                    if (!(rkept >> u & 1u))
                         c[u] = *reinterpret_cast<const spmm_pair *>(cp);
                     d[u] = *reinterpret_cast<const spmm_pair *>(dp);
                 } else {
@@ -2260,17 +2272,17 @@ __global__ __launch_bounds__(SDDMM_W * 64, 4) void sddmm_kernel(int64_t nnz, con
 #pragma unroll
         for (int u = 0; u < R; ++u) {
             const int e = e0 + u;
-            if (u < rounds && g < G && e < E) {
-                cur.x = K > 1 && (kept >> u & 1u) ? cur.x : c[u].x;
-                cur.y = K > 1 && (kept >> u & 1u) ? cur.y : c[u].y;
+            if (u < rounds && rg < rG && e < E) {
+                cur.x = K > 1 && (rkept >> u & 1u) ? cur.x : c[u].x;
+                cur.y = K > 1 && (rkept >> u & 1u) ? cur.y : c[u].y;
                 double2 q = make_double2(cur.x * d[u].x, cur.y * d[u].y);
-                if (half)
+                if (rhalf)
                     q.x = q.y;
-                *reinterpret_cast<double2 *>(tile + e * LD + 2 * sub) = q;
+                *reinterpret_cast<double2 *>(tile + e * LD + 2 * rsub) = q;
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-        sum(kn);
+        sum(rn);
     }
     if (lane < cnt)
         out[p] = v * t;
@@ -2550,12 +2562,17 @@ static int sddmm_values(Csr *b, int64_t K, int64_t c_dptr, int64_t ldc, int64_t 
             longest = x > 0 ? std::max(longest, start.v[x] - start.v[x - 1]) : 0;
         }
         // 64 entries to a wavefront, 32 where there are too few to keep every CU in wavefronts that way (us, 64 / 32: 3.9 M
-        // entries K = 64 228 / 231, 8 M K = 15 198 / 207; 0.64 M K = 33 32.9 / 32.7; 0.32 M K = 50 30.6 / 28.5, K = 10 13.3 / 11.9).
-        // 32 with 32 columns at a time where a row of D comes from beyond the L2s, which give two lines next to each other
-        // quicker than one now and one later (3.7 M entries as stored, 16 / 32 columns: K = 24 135 / 143, 32 142 / 137, 48
-        // 214 / 204, 64 285 / 271, 128 570 / 533, 256 1161 / 1077; in order K = 48 140 / 170, 64 178 / 184).
-        const bool wide = !order && large && K >= 32;
-        const int per_group = SDDMM_W * (wide || b->nnz < SDDMM_ORDER_NNZ ? 32 : 64);
+        // entries K = 64 228 / 231; 0.64 M K = 33 32.9 / 32.7; 0.32 M K = 50 30.6 / 28.5; 0.43 M K = 9 10.9 / 11.8, 16 10.9 /
+        // 11.7).
+        // Where rows of D come from beyond the L2s, these give two lines next to each other quicker than one now and one later:
+        // 32 entries with 32 columns at a time (3.7 M entries as stored, 16 / 32 columns: K = 32 142 / 137, 48 214 / 204, 64
+        // 285 / 271, 128 570 / 533, 256 1161 / 1077; in order K = 48 140 / 170, 64 178 / 184), and 32 entries where a row is one
+        // line and a rest (64 / 32, 300000 rows of 4 uniform entries K = 17 76 / 67, 24 77 / 74, 150000 of 30 173 / 155, 178 / 172).
+        // Up to 8 columns, 8 at a time: more workgroups fit a CU (16 / 8 columns: 100000 rows of a band of 27 K = 1 28 / 23, 5
+        // 35 / 26, 8 35 / 28, 300000 of 4 uniform ones 25.0 / 23.0, 40.4 / 39.7, 38.7 / 37.8).
+        const bool far = !order && large, narrow = K <= 8, wide = far && K >= 32;
+        const bool most = K <= 16 || (b->nnz >= SDDMM_ORDER_NNZ && !far);
+        const int per_group = SDDMM_W * (most ? 64 : 32);
         const dim3 grid((unsigned)(order ? 8 * ceil_div(longest, per_group) : ceil_div(b->nnz, per_group)));
         const dim3 block(SDDMM_W * 64);
         const int32_t *by_row = order ? order + b->nnz : rows, *by_col = order ? order + 2 * b->nnz : b->crd;
@@ -2566,9 +2583,11 @@ static int sddmm_values(Csr *b, int64_t K, int64_t c_dptr, int64_t ldc, int64_t 
         const auto launch = [&](auto kernel) {
             kernel<<<grid, block, 0, stream()>>>(b->nnz, order, start, by_row, by_col, b->val, C, ldc, Dt, ldt, K, out);
         };
-        if (wide)
+        if (narrow)
+            small ? launch(sddmm_kernel<true, 8, 4>) : launch(sddmm_kernel<false, 8, 4>);
+        else if (wide)
             small ? launch(sddmm_kernel<true, 32, 8>) : launch(sddmm_kernel<false, 32, 8>);
-        else if (b->nnz >= SDDMM_ORDER_NNZ)
+        else if (most)
             small ? launch(sddmm_kernel<true, 16, 8>) : launch(sddmm_kernel<false, 16, 8>);
         else
             small ? launch(sddmm_kernel<true, 16, 4>) : launch(sddmm_kernel<false, 16, 4>);

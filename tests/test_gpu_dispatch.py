@@ -330,6 +330,42 @@ def test_sddmm_of_many_entries(nnz, K):
     assert np.array_equal(got[:nnz], orc.sddmm(pos, crd, val, C, D)) and got[nnz] == 7.0
 
 
+@pytest.mark.parametrize("wide", [False, True])
+def test_sddmm_of_every_piece_and_rest(wide):
+    # every number of columns up to three pieces: whole ones, a last one with lanes behind its end, a rest of one or two a lane;
+    # wide: rows of C so far apart that an address is no 24-bit product
+    rng = np.random.default_rng(9)
+    n, m, nnz = 13, 40, 200
+    cells = np.sort(rng.choice(n * m, nnz, replace=False))
+    pos = np.concatenate([[0], np.cumsum(np.bincount(cells // m, minlength=n))]).astype(np.int64)
+    crd, val = (cells % m).astype(np.int32), rng.uniform(-1, 1, nnz)
+    S = rt.CsrMatrix.from_arrays((n, m), pos, crd, val)
+    for K in range(1, 49):
+        C, D = rng.uniform(-1, 1, (n, K)), rng.uniform(-1, 1, (K, m))
+        ldc = (1 << 21) + 5 if wide else K
+        flat = np.full((n - 1) * ldc + K, np.inf)          # what lies between the rows is nobody's
+        np.lib.stride_tricks.as_strided(flat, (n, K), (8 * ldc, 8))[:] = C
+        dC, dD, out = rt.DeviceArray.from_numpy(flat), rt.DeviceArray.from_numpy(D), rt.DeviceArray.from_numpy(np.full(nnz + 1, 7.0))
+        rt._check(rt.lib().comet_hip_sddmm_csr_values_f64(S.handle, K, dC.ptr, ldc, dD.ptr, m, out.ptr), "sddmm")
+        got = out.to_numpy()
+        assert np.array_equal(got[:nnz], orc.sddmm(pos, crd, val, C, D)) and got[nnz] == 7.0, K
+
+
+@pytest.mark.parametrize("K", [16, 17, 18, 24, 25, 31, 32])
+def test_sddmm_of_rows_from_beyond_the_l2(K):
+    # many entries as stored and a large D: 32 entries a wavefront
+    rng = np.random.default_rng(K)
+    n = 80_000
+    pos = np.arange(0, 7 * n + 1, 7).astype(np.int64)
+    crd = np.sort(rng.integers(0, n // 7, (n, 7)) + np.arange(7) * (n // 7), axis=1).ravel().astype(np.int32)
+    val, C, D = rng.uniform(-1, 1, len(crd)), rng.uniform(-1, 1, (n, K)), rng.uniform(-1, 1, (K, n))
+    assert len(crd) >= 1 << 19 and n * K * 8 >= 8 << 20
+    out = rt.DeviceArray(len(crd))
+    S = rt.CsrMatrix.from_arrays((n, n), pos, crd, val)
+    rt.sddmm(S, rt.DeviceArray.from_numpy(C), rt.DeviceArray.from_numpy(D), out_values=out)
+    assert np.array_equal(out.to_numpy(), orc.sddmm(pos, crd, val, C, D))
+
+
 @pytest.mark.parametrize("K", [27, 31, 32, 33, 64, 65])
 @pytest.mark.parametrize("hub", [False, True])
 def test_sddmm_in_an_order_that_keeps_columns_close(K, hub):
