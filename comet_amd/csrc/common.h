@@ -186,7 +186,7 @@ struct Csr {
     // SpMM plan for long rows (heavy_state: 0 undecided, 1 not worth it, 2 in use): the long rows re-stored as
     // per-(XCD, wavefront) lists ordered by column for spmm_heavy_sweep, and the rest of the matrix as `light`.
     int heavy_state = 0;
-    int64_t heavy_nnz = 0;
+    int64_t heavy_nnz = -1;                  // entries of the long rows; -1: not looked at
     int64_t *heavy_seg = nullptr;            // [8 * 512 + 1] list boundaries
     HeavyEnt *heavy_ent = nullptr;           // the lists, runs padded to even length
     int64_t heavy_rows = 0;

@@ -437,7 +437,8 @@ static void csr_drop_plans(Csr *c)
     (void)dev_free(c->sddmm_order);
     c->sddmm_order = nullptr;
     c->sddmm_state = 0;
-    c->heavy_nnz = c->heavy_rows = 0;
+    c->heavy_nnz = -1;
+    c->heavy_rows = 0;
     (void)dev_free(c->spmm_chunk_row);
     c->spmm_chunk_row = nullptr;
     c->spmm_nchunks = 0;

@@ -1349,7 +1349,19 @@ static int sweep_launch(Kern kernel, dim3 grid, dim3 block, size_t lds, Args... 
     return COMET_HIP_OK;
 }
 
-static int spmm_heavy_plan(Csr *a)
+// Whether rows of B and C that are no multiple of 16 bytes are swept: most of the matrix has to be in the long rows, and a
+// row of B in several of them.  us, chunks / sweep at K = 17, 33, 63, and of the entries the share in long rows and how many
+// of them there are a column: zipf, 200000 rows of 4 (0.69, 2.7) 62 / 124, 77 / 131, 113 / 113, of 8 (0.81, 6.5) 87 / 100, 115 /
+// 107, 177 / 106, 100000 of 16 (0.86, 14) K = 33 101 / 78, 63 159 / 83; R-MAT scale 17, 4 edges a vertex (0.37, 2.8) K = 33
+// 105 / 145, 16 (0.54, 15) 144 / 332.
+static bool sweep_uneven(const Csr *a, int64_t K)
+{
+    return a->heavy_nnz * 4 >= a->nnz * 3 && a->heavy_nnz >= (K < 32 ? 8 : 4) * a->ncols;
+}
+
+// even: the call's rows are multiples of 16 bytes; if not, the plan is made only if the sweep is worth it for such, and is
+// left to a call with even ones otherwise
+static int spmm_heavy_plan(Csr *a, bool even, int64_t K)
 {
     if (a->heavy_state != 0)
         return COMET_HIP_OK;
@@ -1415,6 +1427,11 @@ static int spmm_heavy_plan(Csr *a)
     int64_t hnnz = 0;
     for (auto &c : cand)
         hnnz -= c.first;
+    a->heavy_nnz = hnnz;
+    if (!even && !sweep_uneven(a, K)) {
+        a->heavy_state = 0;
+        return COMET_HIP_OK;
+    }
     if (H == 0 || hnnz * 4 < a->nnz)
         return COMET_HIP_OK;        // the long rows hold too little of the matrix to pay for a second kernel
     std::vector<int32_t> hrow((size_t)H), hcode((size_t)(8 * H)), cnt((size_t)(8 * H));
@@ -1623,7 +1640,6 @@ static int spmm_heavy_plan(Csr *a)
     cleanup(false);
     light->heavy_state = 1;
     a->light = light;
-    a->heavy_nnz = hnnz;
     a->heavy_rows = H;
     a->heavy_groups = G;
     a->medium_rows = M;
@@ -1765,17 +1781,17 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
     // long rows: column sweep with the sums on chip; everything else: one wavefront per 256 nonzeros
     // Rows of B and C that are no multiple of 16 bytes are swept where B is so large that its gathers come from far away
     // (chunks / sweep, us: K = 33 40000 rows 51 / 65, 60001 69 / 68, 120000 121 / 87, 250000 242 / 153, 500000 477 / 277;
-    // K = 63 40000 71 / 74, 60001 102 / 77, 500000 758 / 358; K = 17 60001 52 / 60, 500000 348 / 230), and where no tile of
-    // columns holds a single one.
+    // K = 63 40000 71 / 74, 60001 102 / 77, 500000 758 / 358; K = 17 60001 52 / 60, 500000 348 / 230: zipf, 16 entries a row),
+    // where the matrix is right for it (sweep_uneven), and where no tile of columns holds a single one.
     const bool even = (K & 1) == 0 && (ldb & 1) == 0 && (b_dptr & 15) == 0 && (ldc & 1) == 0 && (c_dptr & 15) == 0;
-    const bool uneven_pays = K % 64 != 1 && a->ncols * ldb * 8 >= SPMM_UNEVEN_SWEEP;
+    const bool uneven_pays = K % 64 != 1 && a->ncols * ldb * 8 >= SPMM_UNEVEN_SWEEP && (a->heavy_nnz < 0 || sweep_uneven(a, K));
     const bool sweep_fits = K >= 16 && K <= 2048 && (even || uneven_pays) && getenv("COMET_SPMM_NO_SWEEP") == nullptr;
     // The plan (the long rows as per-XCD lists, the rest re-packed) costs some forty products: a matrix multiplied
     // once goes through the chunk kernel whole, the plan is made when it is multiplied again.
     const bool plan_now = a->spmm_uses > 0 || plan_at_once();
     a->spmm_uses = a->spmm_uses < 2 ? a->spmm_uses + 1 : 2;
     if (sweep_fits && plan_now && a->heavy_state == 0)
-        (void)plan_made([&] { return spmm_heavy_plan(a); });          // or the chunk kernel goes on taking all rows
+        (void)plan_made([&] { return spmm_heavy_plan(a, even, K); });          // or the chunk kernel goes on taking all rows
     if (a->heavy_state != 2 || !sweep_fits)
         return spmm_chunks(a, K, B, ldb, C, ldc, accumulate);
     const int G = a->heavy_groups;

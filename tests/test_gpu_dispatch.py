@@ -611,6 +611,27 @@ def test_spmm_sweep_of_rows_that_are_no_multiple_of_16_bytes(K, ldb, ldc, shift,
     assert np.all(out == 7.0)
 
 
+@pytest.mark.parametrize("mean,widths", [(4.0, {17: False, 33: False, 63: False, 64: True}), (8.0, {17: False, 33: True, 63: True, 64: True}),
+                                         (16.0, {17: True, 63: True, 64: True})])
+def test_spmm_sweeps_odd_widths_where_long_rows_hold_the_matrix(mean, widths):
+    # the plan of a matrix is made by the first call it is right for, whatever calls came before
+    n = 200_000
+    pos, crd, val = gen.zipf_csr(n=n, mean=mean, cap=4096, seed=7)
+    A = rt.CsrMatrix.from_arrays((n, n), pos, crd, val)
+    rng = np.random.default_rng(int(mean))
+    for K, swept in widths.items():
+        B = rng.uniform(-1, 1, (n, K))
+        dB, dC = rt.DeviceArray.from_numpy(B), rt.DeviceArray((n, K))
+        rt.profile_reset()
+        rt.profile_enable(True)
+        rt.spmm(A, dB, dC, accumulate=False)
+        rt.sync()
+        assert ("spmm_heavy_sweep" in rt.profile_report()) == swept, K
+        rt.profile_enable(False)
+        bound = orc.spmm(pos, crd, np.abs(val), np.abs(B))
+        assert np.all(np.abs(dC.to_numpy() - orc.spmm(pos, crd, val, B)) <= 1e-12 * bound)
+
+
 def _edges(kind, rng):
     """Pairs of vertices (u > v) and the number of vertices."""
     if kind == "complete":
