@@ -2945,9 +2945,10 @@ __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
         rows.as = Apos[row_begin + rows.rn];
         rows.ae = Apos[row_begin + rows.rn + 1];
         rows.rn = rows.t + gridDim.x < rows.t_end ? list.rows[rows.t + gridDim.x] : rows.rn;
-        const bool held = ae - as <= 64;          // by every wavefront
+        const int held = __builtin_amdgcn_readfirstlane((int)(ae - as <= 64));          // by every wavefront
         SmallEntry e = small_entry<false>(as, as + (held ? threadIdx.x & 63 : threadIdx.x), ae, Acrd, nullptr, Bpos);
-        if (held && __builtin_amdgcn_readlane(wave_inclusive_scan(e.len), 63) <= SM_T) {
+        const int products = __builtin_amdgcn_readlane(wave_inclusive_scan(e.len), 63);
+        if (held && products <= SM_T) {
             // a product to a lane: the columns are those that found their bit clear
             SmallProducts<false, 1> it;
             small_few<false, SM_T>(stage, e, Bcrd, nullptr, it);
@@ -2968,30 +2969,28 @@ __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
             }
             if (j >= 0)
                 bm[j >> 5] = 0;
-            lds_barrier();
-            continue;
-        }
-        if (held && threadIdx.x >= 64)
-            e.len = 0;
-        for (int64_t p0 = as; p0 < ae; p0 += SM_T) {
-            if (p0 > as)
-                e = small_entry<false>(as, p0 + threadIdx.x, ae, Acrd, nullptr, Bpos);
-            const int products = small_stage<false, SM_T>(stage, e);
-            SmallProducts<false, SM_PER> it;
-            small_products<false, SM_T, SM_PER>(stage, products, Bcrd, nullptr, it);
+        } else {
+            if (held && threadIdx.x >= 64)
+                e.len = 0;
+            for (int64_t p0 = as; p0 < ae; p0 += SM_T) {
+                if (p0 > as)
+                    e = small_entry<false>(as, p0 + threadIdx.x, ae, Acrd, nullptr, Bpos);
+                SmallProducts<false, SM_PER> it;
+                small_products<false, SM_T, SM_PER>(stage, small_stage<false, SM_T>(stage, e), Bcrd, nullptr, it);
 #pragma unroll
-            for (int x = 0; x < SM_PER; ++x)
-                if (it.col[x] >= 0)
-                    atomicOr(&bm[it.col[x] >> 5], 1u << (it.col[x] & 31));
-            lds_barrier();
-            small_clear(stage);
+                for (int x = 0; x < SM_PER; ++x)
+                    if (it.col[x] >= 0)
+                        atomicOr(&bm[it.col[x] >> 5], 1u << (it.col[x] & 31));
+                lds_barrier();
+                small_clear(stage);
+            }
+            const int n = small_row_ranks<SM_T>(bm, nullptr, words, wave_tot);
+            if (threadIdx.x == 0)
+                rowcount[r] = n;
+            const int per = (words + SM_T - 1) / SM_T;
+            for (int w = threadIdx.x * per; w < (int)(threadIdx.x + 1) * per && w < words; ++w)          // its own words
+                bm[w] = 0;
         }
-        const int n = small_row_ranks<SM_T>(bm, nullptr, words, wave_tot);
-        if (threadIdx.x == 0)
-            rowcount[r] = n;
-        const int per = (words + SM_T - 1) / SM_T;
-        for (int w = threadIdx.x * per; w < (int)(threadIdx.x + 1) * per && w < words; ++w)          // its own words
-            bm[w] = 0;
         lds_barrier();
     }
 }
@@ -3211,8 +3210,9 @@ __global__ __launch_bounds__(T) void spgemm_numeric_small_kernel(
         rows.ae = Apos[row_begin + rows.rn + 1];
         rows.rn = rows.t + gridDim.x < rows.t_end ? list.rows[rows.t + gridDim.x] : rows.rn;
         SmallProducts<true, PER> it;
+        const int held = PER == 1 ? __builtin_amdgcn_readfirstlane((int)(ae - as <= 64)) : 0;          // by every wavefront
         const auto products = [&](int64_t p0) {
-            if (PER == 1 && ae - as <= 64) {
+            if (held) {
                 const SmallEntry e = small_entry<true>(as, as + (threadIdx.x & 63), ae, Acrd, Aval, Bpos);
                 small_few<true, T>(sh.stage, e, Bcrd, Bval, it);
             } else {

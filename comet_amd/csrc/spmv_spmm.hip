@@ -715,11 +715,12 @@ constexpr int SPMM_HCB = 32;                         // column blocks a wavefron
 // of every pair took 23 instructions a pair, these 14.)  The
 // gathers go out in batches of 8 pairs (16 rows of B) and the batch is added
 // before the next one is issued: with sixteen wavefronts per CU the memory path
-// is kept busy by the other wavefronts, and more requests queued per wavefront
-// only lengthen the queues (batches of 4 or 16 pairs: 0.25 ms for the long rows
-// alone instead of 0.19).  What bounds it is that path: 29 M lines a product of
-// 500000 rows and K = 64, 60 of them under way a CU, back in 257 clocks on
-// average - 1.5 times as long as where every line comes from the L2.
+// is kept busy by the other wavefronts (batches of 4 or 16 pairs, before the
+// wavefronts were kept together: 0.25 ms for the long rows alone instead of
+// 0.19).  What bounds it is not settled: 29 M lines a product of 500000 rows and
+// K = 64, 60 of them under way a CU, back in 257 clocks on average - 1.5 times
+// as long as where every line comes from the L2; but the chunk kernel beside it
+// keeps 140 to 160 under way.
 // Entry = column - first column of the XCD's range (the low 24 bits, so that the byte offset of the row of B is one
 // 24-bit multiply-add on the entry as it is) | real, first-of-run, kept-in-LDS | owned row << SPMM_E_ROW | partner-is-a-pad.  The slot of
 // a row kept in LDS is the entry's second word.
@@ -2141,8 +2142,9 @@ extern "C" int comet_hip_densemat_csr_f64(int64_t csr, int64_t M, int64_t a_dptr
 // is not that of the entry before, and entries of one row lie together.  The products go to LDS, and lane e adds those
 // of entry e in ascending k while the next 16 columns are on their way.  (Other numbers of entries and columns at a time: where
 // they are chosen.)  (Sixteen entries and 64 columns at a time read C
-// for every entry and left three quarters of the lanes idle in the sums: whole call, 250000 rows of 16 entries, K = 64
-// 301 -> 227 us, K = 48 217 -> 140, K = 33 213 -> 170; 500000 rows, K = 15 217 -> 199, K = 3 150 -> 137.)  Bound by the
+// for every entry and left three quarters of the lanes idle in the sums: whole call, zipf, 16 entries a row, 250000 rows K = 64
+// 304 -> 228 us, 48 270 -> 179, 33 259 -> 195, 17 124 -> 109, 9 83 -> 67, 5 66 -> 58; 500000 rows K = 15 216 -> 166, 3 121 ->
+// 98.)  Bound by the
 // way of D's rows from the L2s: 16 of the 18.6 M lines that the CUs ask for at K = 64, 80 of them under way a CU, a third
 // of them beyond the L2.  D is transposed first, so that its "row" for a
 // column j is contiguous; the row of every entry comes from a list kept in B's handle (searching pos per entry cost
