@@ -1360,6 +1360,22 @@ static bool sweep_uneven(const Csr *a, int64_t K)
     return a->heavy_nnz * 4 >= a->nnz * 3 && a->heavy_nnz >= (K < 32 ? 8 : 4) * a->ncols;
 }
 
+// *held += entries of the rows of min_len entries and more
+__global__ __launch_bounds__(256) void spmm_long_entries(int64_t nrows, const int64_t *__restrict__ pos, int64_t min_len,
+                                                         unsigned long long *__restrict__ held)
+{
+    int64_t mine = 0;
+    for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < nrows; r += (int64_t)gridDim.x * 256) {
+        const int64_t len = pos[r + 1] - pos[r];
+        mine += len >= min_len ? len : 0;
+    }
+    for (int d = 32; d > 0; d >>= 1)
+        mine += ((int64_t)__shfl_down((int)(mine >> 32), d, 64) << 32) + (int64_t)(uint32_t)__shfl_down((int)mine, d, 64);
+    if ((threadIdx.x & 63) == 0 && mine > 0)
+        atomicAdd(held, (unsigned long long)mine);
+}
+static Workspace g_long_entries;
+
 // even: the call's rows are multiples of 16 bytes; if not, the plan is made only if the sweep is worth it for such, and is
 // left to a call with even ones otherwise
 static int spmm_heavy_plan(Csr *a, bool even, int64_t K)
@@ -1370,6 +1386,25 @@ static int spmm_heavy_plan(Csr *a, bool even, int64_t K)
     if (a->nnz < (1 << 19) || a->nnz >= (1ll << 32) || ceil_div(a->ncols, 8) >= (1ll << SPMM_HCOLB))
         return COMET_HIP_OK;        // a list entry has SPMM_HCOLB bits for the column inside an XCD's eighth
     const int64_t n = a->nrows;
+    {   // The long rows may hold too little for the sweep: asked of the device, 15 us, before the row pointers are fetched and
+        // gone through here (300000 rows: 540).  Those that are long may be more than the sweep holds.
+        unsigned long long *held = nullptr;
+        COMET_CHK(mailbox((void **)&held));
+        COMET_CHK(g_long_entries.ensure(sizeof *held, false));
+        COMET_HIPCHK(hipMemsetAsync(g_long_entries.ptr, 0, sizeof *held, stream()));
+        spmm_long_entries<<<dim3((unsigned)std::min<int64_t>(ceil_div(n, 256), 2 * (int64_t)num_cus())), dim3(256), 0, stream()>>>(
+            n, a->pos, SPMM_HEAVY_MIN_LEN, (unsigned long long *)g_long_entries.ptr);
+        COMET_HIPCHK(hipGetLastError());
+        COMET_HIPCHK(hipMemcpyAsync(held, g_long_entries.ptr, sizeof *held, hipMemcpyDeviceToHost, stream()));
+        COMET_CHK(stream_wait());
+        a->heavy_nnz = (int64_t)*(volatile unsigned long long *)held;
+        if (!even && !sweep_uneven(a, K)) {
+            a->heavy_state = 0;
+            return COMET_HIP_OK;
+        }
+        if (a->heavy_nnz == 0 || a->heavy_nnz * 4 < a->nnz)
+            return COMET_HIP_OK;
+    }
     std::vector<int64_t> pos((size_t)n + 1);
     COMET_HIPCHK(hipMemcpyAsync(pos.data(), a->pos, sizeof(int64_t) * (size_t)(n + 1), hipMemcpyDeviceToHost,
                                 stream()));
@@ -1428,7 +1463,7 @@ static int spmm_heavy_plan(Csr *a, bool even, int64_t K)
     int64_t hnnz = 0;
     for (auto &c : cand)
         hnnz -= c.first;
-    a->heavy_nnz = hnnz;
+    a->heavy_nnz = hnnz;          // of those the sweep holds
     if (!even && !sweep_uneven(a, K)) {
         a->heavy_state = 0;
         return COMET_HIP_OK;
