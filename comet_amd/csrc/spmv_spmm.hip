@@ -359,26 +359,32 @@ static int spmv_plan(Csr *a)
 // tile of kt columns takes kt / 2 lanes and a wavefront holds 64 / (kt / 2)
 // groups of them, each with a run of the chunk's nonzeros of its own, SPMM_U
 // gathers of B deep.  Which row a nonzero is of is worked out once per chunk in
-// LDS.  A row that lies inside one block of SPMM_CH nonzeros is summed by one
-// group, in nonzero order: where a boundary of a chunk or run would cut it, it
-// goes to the one it begins in.  The other rows are cut wherever that happens;
-// the pieces of a chunk are added in LDS, and what the chunk has of them goes to
-// `carry` (two 64-wide slots per chunk: [0] a piece whose row began in an
-// earlier chunk, [1] a piece whose row goes on into the next), from where the
-// wavefront that leaves the last piece of a row (`arrived` counts them, by the
-// chunk the row begins in, from zero) adds them in chunk order.
-// Bound by the gathers' way from the memory-side cache where B is larger than
-// an L2.  A lane per column and one nonzero at a time (K of 64 lanes busy, 8
-// bytes each) took 84 us for 60001 rows of 16 nonzeros and K = 33, this 69; 81 and 47 for
-// K = 14, 349 and 175 for 500000 rows and K = 3, 49 and 22 for 2000 rows.
+// LDS.  A row of fewer than SPMM_WHOLE nonzeros, or one that lies inside one
+// block of SPMM_CH, is summed in nonzero order: where a boundary of a chunk would
+// cut it, it goes to the one it begins in.  The other rows are cut wherever that
+// happens; the pieces of a chunk are added in LDS, and what the chunk has of them
+// goes to `carry` (two slots of a tile's columns per chunk: [0] a piece whose row
+// began in an earlier chunk, [1] a piece whose row goes on into the next), from
+// where the wavefront that leaves the last piece of a row (`arrived` counts them,
+// by the chunk the row begins in, from zero) adds them in chunk order.
+// The groups' runs end with rows, so one run may be much longer than the others:
+// then every group gathers the same number of nonzeros, and the sum of a row goes
+// from group to group.  Until that was so, one group went through a row of up to
+// 255 nonzeros by itself, 22 of the 24 us that a matrix of 2000 rows took (zipf, 12
+// nonzeros a row; 14 now); 20000 rows and K = 8 30 -> 20, 500000 and K = 3 175 -> 152.
+// Bound by the latency of that where the matrix is small, by the gathers' way from
+// the memory-side cache where B is larger than an L2.
 // ============================================================================
 #ifndef COMET_SPMM_U
 #define COMET_SPMM_U 8
 #endif
-constexpr int SPMM_CH = 256;                  // nonzeros per wavefront, at most
+constexpr int SPMM_CH = 256;                  // nonzeros per wavefront, at most, but for the end of a row that is not cut
+constexpr int SPMM_WHOLE = 128;               // a row of fewer nonzeros is never cut
+constexpr int SPMM_HELD = SPMM_CH + SPMM_WHOLE;
 constexpr int SPMM_GRAIN = 64;                // the row of every so many'th nonzero is kept
 constexpr int SPMM_U = COMET_SPMM_U;          // B-row loads in flight per lane
 constexpr int SPMM_WAVES = 4;                 // wavefronts per workgroup
+constexpr int SPMM_TURNS = 4;                 // sums handed from group to group in the time of a round of gathers
 
 // chunk_row[c] = the row r with pos[r] <= c*grain < pos[r+1]; arrived[0 .. counts) = 0 (counts 0: not asked for)
 __global__ void spmm_chunk_rows(const int64_t *__restrict__ pos, int64_t nrows, int64_t nchunks, int grain,
@@ -406,20 +412,20 @@ typedef double spmm_pair __attribute__((ext_vector_type(2), aligned(8)));
 struct SpmmChunkLds {
     union {
         struct {
-            double val[SPMM_CH];
-            int32_t crd[SPMM_CH];
+            double val[SPMM_HELD];
+            int32_t crd[SPMM_HELD];
         };
         double piece[2][128];            // of every group: its head and its tail, over the entries
     };
-    int32_t row[SPMM_CH + 4];            // the last one: whose row goes on past the chunk
+    int32_t row[SPMM_HELD + 4];            // the last one: whose row goes on past the chunk
 };
 
 // W: columns of a lane, 2 unless K is 1.  SMALL: B is within 4 GiB.
 template <bool ACC, int W, bool SMALL>
-__global__ __launch_bounds__(SPMM_WAVES * 64) void spmm_csr_nnzsplit(
+__global__ __launch_bounds__(SPMM_WAVES * 64, ACC ? 4 : 6) void spmm_csr_nnzsplit(
     const int64_t *__restrict__ pos, const int32_t *__restrict__ crd, const double *__restrict__ val,
     int64_t nnz, int64_t nrows, const int32_t *__restrict__ chunk_row, int grain, int chunk_len, int64_t nchunks,
-    const double *__restrict__ B, int64_t ldb, double *__restrict__ C, int64_t ldc, int64_t K,
+    const double *__restrict__ B, int64_t ldb, double *__restrict__ C, int64_t ldc, int64_t K, int tile_cols,
     double *__restrict__ carry, unsigned *__restrict__ arrived, const int32_t *__restrict__ rowmap)
 {
     __shared__ __align__(16) SpmmChunkLds all[SPMM_WAVES];
@@ -431,8 +437,8 @@ __global__ __launch_bounds__(SPMM_WAVES * 64) void spmm_csr_nnzsplit(
     if (chunk >= nchunks)
         return;
     SpmmChunkLds &sh = all[wave];
-    const int64_t tile = (int64_t)blockIdx.y * 64;
-    const int kt = (int)(K - tile < 64 ? K - tile : 64);
+    const int64_t tile = (int64_t)blockIdx.y * tile_cols;
+    const int kt = (int)(K - tile < tile_cols ? K - tile : tile_cols);
     const int L = (kt + W - 1) / W, G = 64 / L;               // lanes of a group, groups
     const int g = lane / L, sub = lane - g * L;
     // the last lane of an odd tile has one column, and reads the one before it as well
@@ -445,14 +451,15 @@ __global__ __launch_bounds__(SPMM_WAVES * 64) void spmm_csr_nnzsplit(
     const int64_t rn = e_cut < nnz ? (int64_t)__builtin_amdgcn_readfirstlane(chunk_row[e_cut / grain]) : nrows;
     int64_t s = s_cut, e = e_cut;
     const int64_t p0 = pos[r0], q0 = pos[r0 + 1];
-    const bool head = p0 < s_cut && (p0 < block || q0 > block + SPMM_CH);          // the first row is a piece of one
+    const auto whole = [&](int64_t p, int64_t q) { return q - p < SPMM_WHOLE || (p >= block && q <= block + SPMM_CH); };
+    const bool head = p0 < s_cut && !whole(p0, q0);          // the first row is a piece of one
     if (p0 < s_cut && !head)                             // an earlier chunk's
         s = q0;
     bool tail = false;                                   // the last row goes on into the next block
     if (rn < nrows) {
         const int64_t pn = pos[rn], qn = pos[rn + 1];
         if (pn < e_cut) {
-            tail = pn < block || qn > block + SPMM_CH;
+            tail = !whole(pn, qn);
             e = tail ? e_cut : qn;
         }
     }
@@ -516,7 +523,7 @@ __global__ __launch_bounds__(SPMM_WAVES * 64) void spmm_csr_nnzsplit(
         return sh.row[t - 1] != r || cut(r) ? t : (int)(pos[r0 + r + 1] - s);
     };
     const int a = begin(g), z = g < G ? begin(g + 1) : n;
-    const int longest = g < G ? z - a : 0;
+    int longest = g < G ? z - a : 0, until = z;
     double ax = 0.0, ay = 0.0, hx = 0.0, hy = 0.0;          // hx, hy: the piece of a row that began before
     auto store = [&](int32_t r, double x, double y) {
         double *to = C + crow(r0 + r) * ldc + col;
@@ -529,67 +536,170 @@ __global__ __launch_bounds__(SPMM_WAVES * 64) void spmm_csr_nnzsplit(
             __builtin_nontemporal_store(x, to);
         }
     };
-    for (int t0 = 0; __any(t0 < longest); t0 += SPMM_U) {
-        spmm_pair b[SPMM_U], c[ACC ? SPMM_U : 1];
-        double v[SPMM_U];
-        // bit u: the row of the batch's nonzero u ends with it (all of this read before the first is used: the adds of a
-        // long row are one chain, and a look into LDS in it costs more than the rest)
-        unsigned ends = 0;
-        int32_t r = sh.row[a + t0 < n ? a + t0 : n - 1];
-        const bool fresh = t0 == 0 || sh.row[a + t0 - 1 < n ? a + t0 - 1 : n - 1] != r;
-#pragma unroll
-        for (int u = 0; u < SPMM_U; ++u) {
-            const int t = a + t0 + u < n ? a + t0 + u : n - 1;
-            const uint32_t j = (uint32_t)sh.crd[t];
-            v[u] = sh.val[t];
-            const double *at = SMALL ? reinterpret_cast<const double *>(reinterpret_cast<const char *>(B) +
-                                                                        (j * (uint32_t)ldb + (uint32_t)from) * 8u)
-                                     : B + (int64_t)j * ldb + from;
-            if constexpr (W == 2)
-                b[u] = *reinterpret_cast<const spmm_pair *>(at);
-            else
-                b[u].x = *at;
-            const int32_t next = sh.row[t + 1];
-            if constexpr (ACC) {         // where a row begins; the value of a row in pieces is added with them
-                if (t0 + u < longest && (u == 0 ? fresh : (ends >> (u - 1) & 1u) != 0) && !cut(r)) {
-                    const double *to = C + crow(r0 + r) * ldc + from;
-                    if constexpr (W == 2)
-                        c[u] = *reinterpret_cast<const spmm_pair *>(to);
-                    else
-                        c[u].x = *to;
+    // rounds of gathers with every group on its run, and with the nonzeros dealt evenly
+    const int even = (run + SPMM_U - 1) / SPMM_U;
+    bool in_turn = __any(longest > SPMM_U * (even + 1));
+    if (in_turn) {
+        const int most = __builtin_amdgcn_readlane(wave_inclusive_max(longest), 63);
+        const int next = SPMM_U * (lane + 1), at = next < n ? next : 1;
+        in_turn = ((most + SPMM_U - 1) / SPMM_U - even) * SPMM_TURNS > __popcll(__ballot(next < n && sh.row[at - 1] == sh.row[at]));
+    }
+    if (!in_turn) {
+        for (int t0 = 0; __any(t0 < longest); t0 += SPMM_U) {
+            spmm_pair b[SPMM_U], c[ACC ? SPMM_U : 1];
+            double v[SPMM_U];
+            // bit u: the row of the batch's nonzero u ends with it (all of this read before the first is used: the adds of a
+            // long row are one chain, and a look into LDS in it costs more than the rest)
+            unsigned ends = 0;
+            int32_t r = sh.row[a + t0 < n ? a + t0 : n - 1];
+            const bool fresh = t0 == 0 || sh.row[a + t0 - 1 < n ? a + t0 - 1 : n - 1] != r;
+    #pragma unroll
+            for (int u = 0; u < SPMM_U; ++u) {
+                const int t = a + t0 + u < n ? a + t0 + u : n - 1;
+                const uint32_t j = (uint32_t)sh.crd[t];
+                v[u] = sh.val[t];
+                const double *at = SMALL ? reinterpret_cast<const double *>(reinterpret_cast<const char *>(B) +
+                                                                            (j * (uint32_t)ldb + (uint32_t)from) * 8u)
+                                         : B + (int64_t)j * ldb + from;
+                if constexpr (W == 2)
+                    b[u] = *reinterpret_cast<const spmm_pair *>(at);
+                else
+                    b[u].x = *at;
+                const int32_t next = sh.row[t + 1];
+                if constexpr (ACC) {         // where a row begins; the value of a row in pieces is added with them
+                    if (t0 + u < longest && (u == 0 ? fresh : (ends >> (u - 1) & 1u) != 0) && !cut(r)) {
+                        const double *to = C + crow(r0 + r) * ldc + from;
+                        if constexpr (W == 2)
+                            c[u] = *reinterpret_cast<const spmm_pair *>(to);
+                        else
+                            c[u].x = *to;
+                    }
+                }
+                ends |= (unsigned)(next != r && t0 + u < longest) << u;
+                r = next;
+            }
+            bool begins = fresh;
+    #pragma unroll
+            for (int u = 0; u < SPMM_U; ++u) {
+                if constexpr (ACC)
+                    if (begins && t0 + u < longest && !cut(sh.row[a + t0 + u])) {
+                        ax = half ? c[u].y : c[u].x;
+                        ay = W == 2 ? c[u].y : 0.0;
+                    }
+                const double x = ax + v[u] * (half ? b[u].y : b[u].x), y = W == 2 ? ay + v[u] * b[u].y : 0.0;
+                ax = t0 + u < longest ? x : ax;
+                ay = t0 + u < longest ? y : ay;
+                begins = (ends >> u & 1u) != 0;
+                if (begins) {
+                    const int32_t mine = sh.row[a + t0 + u];
+                    if (head && mine == 0) {
+                        hx = ax;
+                        hy = ay;
+                    } else {
+                        store(mine, ax, ay);
+                    }
+                    ax = ay = 0.0;
                 }
             }
-            ends |= (unsigned)(next != r && t0 + u < longest) << u;
-            r = next;
         }
-        bool begins = fresh;
+    } else {
+        // all groups gather, SPMM_U nonzeros each.  Rows that begin in a group's nonzeros are summed there; the sum of one
+        // that goes on is handed from group to group, each adding its products in order.
+        double ox = 0.0, oy = 0.0;           // what is open at the end of a batch
+        const auto ended = [&](int32_t row, double x, double y) {
+            if (head && row == 0) {
+                hx = x;
+                hy = y;
+            } else {
+                store(row, x, y);
+            }
+        };
+        for (int t0 = 0; t0 < n; t0 += G * SPMM_U) {
+            spmm_pair p[SPMM_U], c[ACC ? SPMM_U : 1];
+            const int first = t0 + g * SPMM_U, mine = g < G ? n - first : 0;          // of the batch's nonzeros, the first mine
+            unsigned ends = 0;
+            int32_t r = sh.row[first < n ? first : n - 1];
+            const bool fresh = first == 0 || sh.row[first - 1 < n ? first - 1 : n - 1] != r;
 #pragma unroll
-        for (int u = 0; u < SPMM_U; ++u) {
-            if constexpr (ACC)
-                if (begins && t0 + u < longest && !cut(sh.row[a + t0 + u])) {
-                    ax = half ? c[u].y : c[u].x;
-                    ay = W == 2 ? c[u].y : 0.0;
+            for (int u = 0; u < SPMM_U; ++u) {
+                const int t = first + u < n ? first + u : n - 1;
+                const uint32_t j = (uint32_t)sh.crd[t];
+                const double *at = SMALL ? reinterpret_cast<const double *>(reinterpret_cast<const char *>(B) +
+                                                                            (j * (uint32_t)ldb + (uint32_t)from) * 8u)
+                                         : B + (int64_t)j * ldb + from;
+                if constexpr (W == 2)
+                    p[u] = *reinterpret_cast<const spmm_pair *>(at);
+                else
+                    p[u].x = *at;
+                const int32_t next = sh.row[t + 1];
+                if constexpr (ACC) {
+                    if (u < mine && (u == 0 ? fresh : (ends >> (u - 1) & 1u) != 0) && !cut(r)) {
+                        const double *to = C + crow(r0 + r) * ldc + from;
+                        if constexpr (W == 2)
+                            c[u] = *reinterpret_cast<const spmm_pair *>(to);
+                        else
+                            c[u].x = *to;
+                    }
                 }
-            const double x = ax + v[u] * (half ? b[u].y : b[u].x), y = W == 2 ? ay + v[u] * b[u].y : 0.0;
-            ax = t0 + u < longest ? x : ax;
-            ay = t0 + u < longest ? y : ay;
-            begins = (ends >> u & 1u) != 0;
-            if (begins) {
-                const int32_t mine = sh.row[a + t0 + u];
-                if (head && mine == 0) {
-                    hx = ax;
-                    hy = ay;
-                } else {
-                    store(mine, ax, ay);
+                ends |= (unsigned)(next != r && u < mine) << u;
+                r = next;
+            }
+            // the first `lead` go on with a row of the nonzeros before
+            const int own = mine < SPMM_U ? (mine > 0 ? mine : 0) : SPMM_U;
+            const int lead = fresh ? 0 : ends != 0 && __builtin_ctz(ends) < own ? __builtin_ctz(ends) + 1 : own;
+            bool begins = true;
+            ax = ay = 0.0;
+#pragma unroll
+            for (int u = 0; u < SPMM_U; ++u) {
+                const double v = sh.val[first + u < n ? first + u : n - 1];
+                p[u].x = v * (half ? p[u].y : p[u].x);
+                p[u].y = W == 2 ? v * p[u].y : 0.0;
+                if (u >= lead && u < own) {
+                    if constexpr (ACC)
+                        if (begins && !cut(sh.row[first + u])) {
+                            ax = half ? c[u].y : c[u].x;
+                            ay = W == 2 ? c[u].y : 0.0;
+                        }
+                    ax += p[u].x;
+                    ay += p[u].y;
+                    begins = (ends >> u & 1u) != 0;
+                    if (begins) {
+                        ended(sh.row[first + u], ax, ay);
+                        ax = ay = 0.0;
+                    }
                 }
+            }
+            unsigned long long on = __ballot(lead > 0 && sub == 0);
+            while (on) {
+                const int at = __builtin_ctzll(on);          // the first lane of group x
+                on &= on - 1;
+                const int before = (at > 0 ? at - L : (G - 1) * L) + sub;
+                double sx = __shfl(at > 0 ? ax : ox, before & 63, 64), sy = W == 2 ? __shfl(at > 0 ? ay : oy, before & 63, 64) : 0.0;
+                if (lane - sub == at) {
+#pragma unroll
+                    for (int u = 0; u < SPMM_U; ++u) {
+                        sx = u < lead ? sx + p[u].x : sx;
+                        sy = u < lead ? sy + p[u].y : sy;
+                    }
+                    if (ends >> (lead - 1) & 1u) {
+                        ended(sh.row[first + lead - 1], sx, sy);
+                    } else {
+                        ax = sx;
+                        ay = sy;
+                    }
+                }
+            }
+            ox = ax;
+            oy = ay;
+            if (t0 + G * SPMM_U >= n && g != (n - 1 - t0) / SPMM_U)          // the rest has been handed on
                 ax = ay = 0.0;
-            }
         }
+        longest = until = n;
     }
     if (!head && !tail)
         return;
     // ---- the pieces, a lane per column; what a group's run ends inside of is a piece of the first row or of the last
-    if (longest > 0 && head && sh.row[z - 1] == 0 && sh.row[z] == 0) {
+    if (longest > 0 && head && sh.row[until - 1] == 0 && sh.row[until] == 0) {
         hx = ax;
         hy = ay;
         ax = ay = 0.0;
@@ -609,7 +719,8 @@ __global__ __launch_bounds__(SPMM_WAVES * 64) void spmm_csr_nnzsplit(
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
     if (lane >= kt)
         return;
-    double *slots = carry + (int64_t)blockIdx.y * nchunks * 128 + lane;
+    const int slot = 2 * tile_cols;
+    double *slots = carry + (int64_t)blockIdx.y * nchunks * slot + lane;
     double began = 0.0, goes_on = 0.0;
     for (int x = 0; x < G; ++x) {
         began += sh.piece[0][x * kt + lane];
@@ -617,9 +728,9 @@ __global__ __launch_bounds__(SPMM_WAVES * 64) void spmm_csr_nnzsplit(
     }
     const bool both = head && tail && last == 0;          // one row, through the chunk
     if (head)
-        __hip_atomic_store(slots + chunk * 128, began, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(slots + chunk * slot, began, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (tail && !both)
-        __hip_atomic_store(slots + chunk * 128 + 64, goes_on, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(slots + chunk * slot + tile_cols, goes_on, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // Whoever leaves the last piece of a row adds all of them, in order.  The pieces are written and read past the L2s
     // (agent scope), and this wavefront's have arrived before it counts itself in.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -634,12 +745,12 @@ __global__ __launch_bounds__(SPMM_WAVES * 64) void spmm_csr_nnzsplit(
         if (lane == 0)
             __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);          // for the next call on the workspace
         double *to = C + crow(r) * ldc + tile + lane;
-        double sum = __hip_atomic_load(slots + c0 * 128 + 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        double sum = __hip_atomic_load(slots + c0 * slot + tile_cols, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (ACC)
             sum = *to + sum;
 #pragma unroll 8
         for (int64_t c = c0 + 1; c <= c1; ++c)
-            sum += __hip_atomic_load(slots + c * 128, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            sum += __hip_atomic_load(slots + c * slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         *to = sum;
     };
     if (head)
@@ -1064,6 +1175,11 @@ static Workspace g_spmm_carry, g_spmm_arrived;
 // Nonzeros of a chunk: a half or a quarter of SPMM_CH where that makes 8192 wavefronts at most, 32 for every CU.  (The
 // number is also what the scratch of the form without allocations holds, which cuts rows in the same places.)
 constexpr int64_t SPMM_SHORT_CHUNKS = 8192;
+// Tiles narrower than 64 columns where that makes 4096 wavefronts at most: more groups for the same nonzeros.  Only for a B
+// that an L2 holds, since a tile's part of a row of B is lines of its own.  us with tiles of 64 / narrow ones, zipf, 16
+// nonzeros a row: 2000 rows K = 64 22.4 / 15.6, 4000 rows K = 48 23.7 / 15.5, 8000 rows K = 64 28.6 / 22.3; with 8192
+// wavefronts at most 16000 rows and K = 17 took 24.9 in place of 20.7; 120000 rows and K = 33, B 32 MB, 102 in place of 87.
+constexpr int64_t SPMM_NARROW_B = 4 << 20, SPMM_NARROW_WAVES = 4096;
 static int spmm_chunk_len(int64_t nnz, int64_t tiles)
 {
     for (int len = SPMM_CH / 4; len < SPMM_CH; len *= 2)
@@ -1072,11 +1188,33 @@ static int spmm_chunk_len(int64_t nnz, int64_t tiles)
     return SPMM_CH;
 }
 
-static int spmm_chunk_scratch(const Csr *a, int64_t K)
+// How a product is cut: chunks of len nonzeros, tiles of `cols` columns.
+struct SpmmShape {
+    int len, cols;
+    int64_t chunks, tiles;
+};
+static SpmmShape spmm_shape(const Csr *a, int64_t K)
 {
-    const int64_t tiles = ceil_div(K, 64), slots = tiles * ceil_div(a->nnz, spmm_chunk_len(a->nnz, tiles));
-    COMET_CHK(g_spmm_carry.ensure(sizeof(double) * 128 * (size_t)slots, false));
-    return g_spmm_arrived.ensure(sizeof(unsigned) * (size_t)slots, true);
+    SpmmShape h;
+    h.cols = 64;
+    if (a->ncols * K * 8 <= SPMM_NARROW_B)
+        for (int w = 16; w < 64; w += 8) {
+            const int64_t tiles = ceil_div(K, w);
+            if (tiles * ceil_div(a->nnz, SPMM_CH / 4) <= SPMM_NARROW_WAVES) {
+                h.cols = 2 * (int)ceil_div(K, 2 * tiles);
+                break;
+            }
+        }
+    h.tiles = ceil_div(K, h.cols);
+    h.len = spmm_chunk_len(a->nnz, h.tiles);
+    h.chunks = ceil_div(a->nnz, h.len);
+    return h;
+}
+
+static int spmm_chunk_scratch(const SpmmShape &h)
+{
+    COMET_CHK(g_spmm_carry.ensure(sizeof(double) * 2 * (size_t)h.cols * (size_t)(h.tiles * h.chunks), false));
+    return g_spmm_arrived.ensure(sizeof(unsigned) * (size_t)(h.tiles * h.chunks), true);
 }
 
 static int spmm_plan(Csr *a)
@@ -1688,7 +1826,7 @@ static int spmm_heavy_plan(Csr *a, bool even, int64_t K)
 
 using namespace comet;
 
-static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate,
+static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate, const SpmmShape &h,
                        hipStream_t on = nullptr);
 static int spmv_run(Csr *a, int64_t x_dptr, int64_t y_dptr, int accumulate);
 static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dptr, int64_t ldc, int accumulate);
@@ -1826,22 +1964,24 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
     // once goes through the chunk kernel whole, the plan is made when it is multiplied again.
     const bool plan_now = a->spmm_uses > 0 || plan_at_once();
     a->spmm_uses = a->spmm_uses < 2 ? a->spmm_uses + 1 : 2;
+    const SpmmShape h = spmm_shape(a, K);
     if (sweep_fits && plan_now && a->heavy_state == 0)
         (void)plan_made([&] { return spmm_heavy_plan(a, even, K); });          // or the chunk kernel goes on taking all rows
     if (a->heavy_state != 2 || !sweep_fits)
-        return spmm_chunks(a, K, B, ldb, C, ldc, accumulate);
+        return spmm_chunks(a, K, B, ldb, C, ldc, accumulate, h);
     const int G = a->heavy_groups;
     // rows of middling length: ceil(rows / G) sums of 64 doubles in the LDS of every workgroup
     const int nslots = (int)ceil_div(a->medium_rows, G);
     const size_t medium_lds = sizeof(double) * 64 * (size_t)nslots;
     // what the kernels leave sums in; without room for it the chunk kernel takes all rows
+    const SpmmShape light = spmm_shape(a->light, K);
     const auto scratch = [&]() -> int {
         COMET_CHK(g_heavy_partial.ensure(sizeof(double) * 8 * (size_t)spmm_hslots(G) * (size_t)K, false));
         COMET_CHK(g_medium_partial.ensure(sizeof(double) * 8 * (size_t)G * (size_t)(nslots > 0 ? nslots : 1) * (size_t)K, false));
-        return a->light->nnz > 0 ? spmm_chunk_scratch(a->light, K) : COMET_HIP_OK;
+        return a->light->nnz > 0 ? spmm_chunk_scratch(light) : COMET_HIP_OK;
     };
     if (!plan_made(scratch))
-        return spmm_chunks(a, K, B, ldb, C, ldc, accumulate);
+        return spmm_chunks(a, K, B, ldb, C, ldc, accumulate, h);
     double *partial = (double *)g_heavy_partial.ptr, *partial_medium = (double *)g_medium_partial.ptr;
     // rows of two and more nonzeros that are not long: one wavefront per 256 nonzeros
     // with CUs left free by the sweep, the chunk kernel of the rows in between runs beside it on a second stream
@@ -1850,7 +1990,7 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
         // (what it needs from stream() - its chunk table, its scratch - is in place before the fork)
         COMET_CHK(aux_fork());
     } else if (a->light->nnz > 0)
-        COMET_CHK(spmm_chunks(a->light, K, B, ldb, C, ldc, accumulate));
+        COMET_CHK(spmm_chunks(a->light, K, B, ldb, C, ldc, accumulate, light));
     const unsigned tiles = (unsigned)ceil_div(K, 64);
     if (!accumulate && a->nempty > 0) {
         KernelTimer t("zero_listed_rows_f64");
@@ -1873,7 +2013,7 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
             COMET_CHK(accumulate ? launch(spmm_heavy_sweep<false, true>) : launch(spmm_heavy_sweep<false, false>));
     }
     if (overlap) {      // the rows in between, on the CUs the sweep leaves free
-        COMET_CHK(spmm_chunks(a->light, K, B, ldb, C, ldc, accumulate, aux_stream()));
+        COMET_CHK(spmm_chunks(a->light, K, B, ldb, C, ldc, accumulate, light, aux_stream()));
         COMET_CHK(aux_join());
     }
     {
@@ -1892,17 +2032,17 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
     return COMET_HIP_OK;
 }
 
-// The chunk kernel: the row of every grain'th nonzero in chunk_row, chunks of len nonzeros (a multiple of grain), two
-// slots for each of them and column tile in carry and a zero in arrived.  timed: events may be recorded (not where the stream is being captured).
+// The chunk kernel: the row of every grain'th nonzero in chunk_row, chunks of h.len nonzeros (a multiple of grain), two
+// slots for each of them and column tile in carry and a zero in arrived.  name: what events are recorded under (null: none, where the stream is being captured).
 static void spmm_chunk_launch(const Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate,
-                              const int32_t *chunk_row, int grain, int len, double *carry, unsigned *arrived, hipStream_t on, bool timed)
+                              const int32_t *chunk_row, int grain, const SpmmShape &h, double *carry,
+                              unsigned *arrived, hipStream_t on, const char *name)
 {
-    const int64_t nchunks = ceil_div(a->nnz, len);
-    const dim3 grid((unsigned)ceil_div(nchunks, SPMM_WAVES), (unsigned)ceil_div(K, 64)), block(SPMM_WAVES * 64);
+    const dim3 grid((unsigned)ceil_div(h.chunks, SPMM_WAVES), (unsigned)h.tiles), block(SPMM_WAVES * 64);
     const auto split = [&](auto kernel) {
-        std::unique_ptr<KernelTimer> t(timed ? new KernelTimer("spmm_csr_nnzsplit", on) : nullptr);
-        kernel<<<grid, block, 0, on>>>(a->pos, a->crd, a->val, a->nnz, a->nrows, chunk_row, grain, len, nchunks, B, ldb, C, ldc,
-                                       K, carry, arrived, a->rowmap);
+        std::unique_ptr<KernelTimer> t(name ? new KernelTimer(name, on) : nullptr);
+        kernel<<<grid, block, 0, on>>>(a->pos, a->crd, a->val, a->nnz, a->nrows, chunk_row, grain, h.len, h.chunks, B, ldb, C,
+                                       ldc, K, h.cols, carry, arrived, a->rowmap);
     };
     const bool small_b = K > 1 && a->ncols * ldb * 8 < (1ll << 32);
     if (K == 1)
@@ -1913,7 +2053,7 @@ static void spmm_chunk_launch(const Csr *a, int64_t K, const double *B, int64_t 
         accumulate ? split(spmm_csr_nnzsplit<true, 2, false>) : split(spmm_csr_nnzsplit<false, 2, false>);
 }
 
-static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate,
+static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate, const SpmmShape &h,
                        hipStream_t on)
 {
     if (!on)
@@ -1928,10 +2068,9 @@ static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *
         return COMET_HIP_OK;
     }
     COMET_CHK(spmm_plan(a));
-    const int64_t tiles = ceil_div(K, 64);
-    COMET_CHK(spmm_chunk_scratch(a, K));
-    spmm_chunk_launch(a, K, B, ldb, C, ldc, accumulate, a->spmm_chunk_row, SPMM_GRAIN, spmm_chunk_len(a->nnz, tiles), (double *)g_spmm_carry.ptr,
-                      (unsigned *)g_spmm_arrived.ptr, on, true);
+    COMET_CHK(spmm_chunk_scratch(h));
+    spmm_chunk_launch(a, K, B, ldb, C, ldc, accumulate, a->spmm_chunk_row, SPMM_GRAIN, h, (double *)g_spmm_carry.ptr,
+                      (unsigned *)g_spmm_arrived.ptr, on, "spmm_csr_nnzsplit");
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
 }
@@ -2039,7 +2178,8 @@ extern "C" int comet_hip_spmm_csr_f64_noalloc(int64_t csr, int64_t K, int64_t b_
         return COMET_HIP_OK;
     if (!c_dptr || (a->nnz > 0 && !b_dptr))
         return set_error(COMET_HIP_ERR_ARG, "null matrix passed to a sparse-dense matrix product");
-    const int64_t tiles = ceil_div(K, 64), nchunks = ceil_div(a->nnz, SPMM_CH);
+    const int64_t tiles = ceil_div(K, 64);
+    const int64_t nchunks = ceil_div(a->nnz, SPMM_CH);
     if (tiles > 65535 || tiles * nchunks > SPMM_STATIC_SLOTS)
         return set_error(COMET_HIP_ERR_SIZE,
                          "comet_hip_spmm_csr_f64_noalloc: ceil(K/64) * ceil(nnz/%d) = %lld exceeds the %lld slots of the "
@@ -2065,12 +2205,11 @@ extern "C" int comet_hip_spmm_csr_f64_noalloc(int64_t csr, int64_t K, int64_t b_
     // holds when a call begins - calls that overlapped may leave anything - does not matter.
     int32_t *chunk_row = reinterpret_cast<int32_t *>(scratch);
     double *carry = reinterpret_cast<double *>(scratch + SPMM_STATIC_TABLE_BYTES);
-    const int len = spmm_chunk_len(a->nnz, tiles);
-    const int64_t rows = ceil_div(a->nnz, len);
+    const SpmmShape h = spmm_shape(a, K);
     unsigned *arrived = reinterpret_cast<unsigned *>(scratch + SPMM_STATIC_TABLE_BYTES + SPMM_STATIC_CARRY_BYTES);
-    spmm_chunk_rows<<<dim3((unsigned)ceil_div(rows, 256)), dim3(256), 0, on>>>(a->pos, a->nrows, rows, len, chunk_row, arrived,
-                                                                               tiles * rows);
-    spmm_chunk_launch(a, K, (const double *)b_dptr, ldb, C, ldc, accumulate, chunk_row, len, len, carry, arrived, on, false);
+    spmm_chunk_rows<<<dim3((unsigned)ceil_div(h.chunks, 256)), dim3(256), 0, on>>>(a->pos, a->nrows, h.chunks, h.len, chunk_row, arrived,
+                                                                                   h.tiles * h.chunks);
+    spmm_chunk_launch(a, K, (const double *)b_dptr, ldb, C, ldc, accumulate, chunk_row, h.len, h, carry, arrived, on, nullptr);
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
 }

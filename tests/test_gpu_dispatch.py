@@ -297,6 +297,21 @@ def test_spmm_chunks_of_every_length_and_width(nrows, K, accumulate):
             assert np.array_equal(got[whole], want[whole])
 
 
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("K", [1, 3, 16, 17, 33, 64, 70])
+@pytest.mark.parametrize("nrows", [130, 3000, 26_000])
+def test_spmm_rows_that_are_not_cut(nrows, K, accumulate):
+    # rows below 128 nonzeros across the blocks of 256, alone in their chunk or with many short ones; chunks of 64, 128 and 256
+    rng = np.random.default_rng(nrows + K)
+    lens = np.resize([1, 1, 127, 1, 2, 1, 96, 3, 120, 5, 1, 1, 40], nrows)
+    pos = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    crd = np.concatenate([np.sort(rng.choice(500, l, replace=False)) for l in lens]).astype(np.int32)
+    val, B, C0 = rng.uniform(-1, 1, pos[-1]), rng.uniform(-1, 1, (500, K)), rng.uniform(-1, 1, (nrows, K))
+    dC = rt.DeviceArray.from_numpy(C0)
+    rt.spmm(rt.CsrMatrix.from_arrays((nrows, 500), pos, crd, val), rt.DeviceArray.from_numpy(B), dC, accumulate=accumulate)
+    assert np.array_equal(dC.to_numpy(), orc.spmm(pos, crd, val, B, C0 if accumulate else None))
+
+
 @pytest.mark.parametrize("K", [1, 2, 3, 5, 16, 17, 31, 32, 33, 63, 64, 65, 66, 130])
 @pytest.mark.parametrize("nnz", [1, 15, 17, 63, 65, 4097])
 def test_sddmm_of_every_tile_and_width(nnz, K):
