@@ -148,6 +148,7 @@ struct TriPlan {
 };
 void tri_plan_free(TriPlan &p);
 
+constexpr int SPMM_LONG_KINDS = 4;
 struct Csr {
     // names this state of the matrix: new for every matrix and again whenever its arrays may have changed
     // (comet_hip_csr_invalidate), so that what other handles keep about it can tell that it is stale
@@ -163,6 +164,9 @@ struct Csr {
     // SpMM plan: row that holds the first nonzero of every fixed-size chunk.
     int32_t *spmm_chunk_row = nullptr;
     int64_t spmm_nchunks = 0;
+    uint32_t *spmm_order[3] = {};            // the chunks by columns, for chunks of 64, 128 and 256
+    // entries of the rows of 128, 256, 512 and 1024 entries and more; -1: not looked at
+    int64_t long_nnz[SPMM_LONG_KINDS] = {-1, -1, -1, -1};
     // SpMV plan: the matrix re-stored as `spmv_nb` column blocks (block-major copy of crd/val, one row
     // pointer array per block) so that the slice of x a pass gathers from stays inside one L2.
     // spmv_nb == 0: not decided yet; 1: run on the original arrays.

@@ -438,9 +438,14 @@ static void csr_drop_plans(Csr *c)
     c->sddmm_order = nullptr;
     c->sddmm_state = 0;
     c->heavy_nnz = -1;
+    c->long_nnz[0] = -1;
     c->heavy_rows = 0;
     (void)dev_free(c->spmm_chunk_row);
     c->spmm_chunk_row = nullptr;
+    for (uint32_t *&order : c->spmm_order) {
+        (void)dev_free(order);
+        order = nullptr;
+    }
     c->spmm_nchunks = 0;
     (void)dev_free(c->sg_blkptr);
     (void)dev_free(c->sg_crd16);

@@ -424,7 +424,7 @@ struct SpmmChunkLds {
 template <bool ACC, int W, bool SMALL>
 __global__ __launch_bounds__(SPMM_WAVES * 64, ACC ? 4 : 6) void spmm_csr_nnzsplit(
     const int64_t *__restrict__ pos, const int32_t *__restrict__ crd, const double *__restrict__ val,
-    int64_t nnz, int64_t nrows, const int32_t *__restrict__ chunk_row, int grain, int chunk_len, int64_t nchunks,
+    int64_t nnz, int64_t nrows, const int32_t *__restrict__ chunk_row, int grain, int chunk_len, int64_t nchunks, const uint32_t *__restrict__ order,
     const double *__restrict__ B, int64_t ldb, double *__restrict__ C, int64_t ldc, int64_t K, int tile_cols,
     double *__restrict__ carry, unsigned *__restrict__ arrived, const int32_t *__restrict__ rowmap)
 {
@@ -433,7 +433,12 @@ __global__ __launch_bounds__(SPMM_WAVES * 64, ACC ? 4 : 6) void spmm_csr_nnzspli
     auto crow = [&](int64_t r) -> int64_t { return rowmap ? (int64_t)rowmap[r] : r; };
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int64_t chunk = (int64_t)blockIdx.x * SPMM_WAVES + wave;
+    // the order's eighths, one to an XCD (workgroup w runs on XCD w % 8, and the grid is a multiple of eight wide)
+    int64_t chunk = (int64_t)(order ? blockIdx.x >> 3 : blockIdx.x) * SPMM_WAVES + wave;
+    if (order) {
+        const int64_t eighth = (nchunks + 7) / 8, at = (blockIdx.x & 7) * eighth + chunk;
+        chunk = chunk < eighth && at < nchunks ? (int64_t)__builtin_amdgcn_readfirstlane((int)order[at]) : nchunks;
+    }
     if (chunk >= nchunks)
         return;
     SpmmChunkLds &sh = all[wave];
@@ -792,6 +797,7 @@ constexpr int spmm_hrows(int g) { return g * (SPMM_HW - 1) * SPMM_HR; }    // lo
 constexpr int SPMM_MED_MIN_LEN = COMET_SPMM_MED_MIN;   // such a row has at least this many nonzeros
 constexpr int SPMM_MSLOTS = 287;                        // sums a workgroup keeps in LDS, beside the entries of its lists (SWEEP_LDS)
 constexpr int SPMM_HEAVY_MIN_LEN = COMET_SPMM_HEAVY_MIN;              // a long row has at least this many nonzeros
+constexpr int64_t SPMM_SWEEP_NNZ = 1 << 19;             // a matrix of fewer nonzeros is not swept
 constexpr int64_t SPMM_UNEVEN_SWEEP = 24 << 20;         // bytes of B from which on rows of any alignment are swept
 constexpr int SPMM_HCB = 32;                         // column blocks a wavefront's list is cut into
 
@@ -1217,6 +1223,125 @@ static int spmm_chunk_scratch(const SpmmShape &h)
     return g_spmm_arrived.ensure(sizeof(unsigned) * (size_t)(h.tiles * h.chunks), true);
 }
 
+// ---------------------------------------------------------------------------
+// Chunks by columns.  A chunk of a row of many chunks has its columns in a short
+// range, and taken in the order of the matrix every chunk's rows of B come from
+// somewhere else.  So, from a matrix's second product on, the chunks are taken in
+// the order of their columns, an eighth of them by every XCD: an L2 then sees an
+// eighth of B, ascending, in place of all of it (workgroup w runs on XCD w % 8).
+// The sums do not change: pieces of rows are added in the order of the chunks'
+// numbers.  It pays where rows of four chunks and more hold half of the matrix;
+// graphs whose columns are as uneven as their rows (R-MAT scale 13 to 18: 7 to 48 %
+// in such rows) have the rows of B that count in every L2 as it is, and lose up to 15 %.
+// us, zipf, 16 nonzeros a row, as stored / by columns: 30000 rows K = 64 51 / 38, 60001 rows K = 33 61 / 45, 250000 rows
+// K = 15 146 / 99, 500000 rows K = 3 153 / 121, K = 15 298 / 182, 1000000 rows K = 8 343 / 249.
+// Chunks of half the length keep a window of a larger B in the L2: 120000 rows K = 33 83 / 75, 250000 rows K = 32 131 / 105;
+// below 28 MiB of B, or 48 with 16 columns and less, they only cost (120000 rows K = 8 38 / 39, 500000 rows K = 8 119 / 128).
+// The sweep takes over where B is larger than 56 MiB, or 80 with 32 columns and less; by columns / sweep: 150000 rows K = 48
+// 93 / 95, K = 56 114 / 104, 250000 rows K = 32 105 / 127, 500000 rows K = 17 206 / 225, K = 21 245 / 229.
+// ---------------------------------------------------------------------------
+constexpr int64_t SPMM_ORDER_B = 1 << 20;               // bytes of B from which on chunks go by columns
+
+// keys[c]: where chunk c has its columns, in 65536ths of the matrix; a chunk of several rows, which has them everywhere, goes
+// where its number puts it
+__global__ __launch_bounds__(256) void spmm_order_keys(const int32_t *__restrict__ crd, int64_t nnz, int64_t ncols,
+                                                       const int32_t *__restrict__ chunk_row, int chunk_len, int64_t nchunks, uint64_t *__restrict__ keys, uint32_t *__restrict__ idx)
+{
+    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (c >= nchunks)
+        return;
+    const int64_t s = c * chunk_len, e = s + chunk_len;
+    uint64_t key = (uint64_t)(c * 65536 / nchunks);
+    if (e < nnz && chunk_row[s / SPMM_GRAIN] == chunk_row[e / SPMM_GRAIN])
+        key = (uint64_t)((int64_t)crd[s + chunk_len / 2] * 65536 / ncols);
+    keys[c] = key;
+    idx[c] = (uint32_t)c;
+}
+
+static Workspace g_spmm_order, g_long_entries;
+static int spmm_plan(Csr *a);
+
+static int spmm_order(Csr *a, const SpmmShape &h)
+{
+    uint32_t *&kept = a->spmm_order[h.len / SPMM_GRAIN / 2];
+    if (kept)
+        return COMET_HIP_OK;
+    COMET_CHK(spmm_plan(a));
+    COMET_CHK(g_spmm_order.ensure((2 * sizeof(uint64_t) + sizeof(uint32_t)) * (size_t)h.chunks, false));
+    uint64_t *keys = (uint64_t *)g_spmm_order.ptr, *sorted = keys + h.chunks;
+    uint32_t *idx = (uint32_t *)(sorted + h.chunks), *order = nullptr;
+    COMET_HIPCHK(dev_malloc((void **)&order, sizeof(uint32_t) * (size_t)h.chunks));
+    spmm_order_keys<<<dim3((unsigned)ceil_div(h.chunks, 256)), dim3(256), 0, stream()>>>(
+        a->crd, a->nnz, a->ncols, a->spmm_chunk_row, h.len, h.chunks, keys, idx);
+    const int rc = sort_pairs_u64_u32(keys, sorted, idx, order, h.chunks, 16);
+    if (rc != COMET_HIP_OK) {
+        (void)dev_free(order);
+        return rc;
+    }
+    kept = order;
+    return COMET_HIP_OK;
+}
+
+// held[i] += entries of the rows of 128 << i entries and more
+__global__ __launch_bounds__(256) void spmm_long_entries(int64_t nrows, const int64_t *__restrict__ pos,
+                                                         unsigned long long *__restrict__ held)
+{
+    int64_t mine[SPMM_LONG_KINDS] = {};
+    for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < nrows; r += (int64_t)gridDim.x * 256) {
+        const int64_t len = pos[r + 1] - pos[r];
+#pragma unroll
+        for (int i = 0; i < SPMM_LONG_KINDS; ++i)
+            mine[i] += len >= (SPMM_HEAVY_MIN_LEN << i) ? len : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < SPMM_LONG_KINDS; ++i) {
+        for (int d = 32; d > 0; d >>= 1)
+            mine[i] += ((int64_t)__shfl_down((int)(mine[i] >> 32), d, 64) << 32) + (int64_t)(uint32_t)__shfl_down((int)mine[i], d, 64);
+        if ((threadIdx.x & 63) == 0 && mine[i] > 0)
+            atomicAdd(&held[i], (unsigned long long)mine[i]);
+    }
+}
+
+// a->long_nnz: asked of the device once, 20 us
+static int spmm_long_rows(Csr *a)
+{
+    if (a->long_nnz[0] >= 0)
+        return COMET_HIP_OK;
+    unsigned long long *held = nullptr;
+    const size_t bytes = SPMM_LONG_KINDS * sizeof *held;
+    COMET_CHK(mailbox((void **)&held));
+    COMET_CHK(g_long_entries.ensure(bytes, false));
+    COMET_HIPCHK(hipMemsetAsync(g_long_entries.ptr, 0, bytes, stream()));
+    spmm_long_entries<<<dim3((unsigned)std::min<int64_t>(ceil_div(a->nrows, 256), 2 * (int64_t)num_cus())), dim3(256), 0, stream()>>>(
+        a->nrows, a->pos, (unsigned long long *)g_long_entries.ptr);
+    COMET_HIPCHK(hipGetLastError());
+    COMET_HIPCHK(hipMemcpyAsync(held, g_long_entries.ptr, bytes, hipMemcpyDeviceToHost, stream()));
+    COMET_CHK(stream_wait());
+    for (int i = 0; i < SPMM_LONG_KINDS; ++i)
+        a->long_nnz[i] = (int64_t)((volatile unsigned long long *)held)[i];
+    a->heavy_nnz = a->long_nnz[0];
+    return COMET_HIP_OK;
+}
+
+// Whether a product of a matrix that has been multiplied before goes through its chunks by columns (*h: cut as it is then).
+static bool spmm_by_columns(Csr *a, int64_t K, SpmmShape *h)
+{
+    const int64_t bytes = a->ncols * K * 8, most = K < 16 ? INT64_MAX : (K > 32 ? 56 : 80) << 20;
+    if (bytes < SPMM_ORDER_B || bytes > most || a->rowmap || getenv("COMET_HIP_SPMM_GROUPS") || getenv("COMET_HIP_SPMM_MEDIUM"))
+        return false;           // the two switches shape the sweep, and ask for it
+    SpmmShape cut = *h;
+    if (cut.len == SPMM_CH && bytes > (K > 16 ? 28 << 20 : 48 << 20)) {
+        cut.len = SPMM_CH / 2;
+        cut.chunks = ceil_div(a->nnz, cut.len);
+    }
+    if (cut.chunks >= 1ll << 31 || (a->long_nnz[0] < 0 && !plan_made([&] { return spmm_long_rows(a); })))
+        return false;
+    if (a->long_nnz[1 + cut.len / SPMM_GRAIN / 2] * 2 < a->nnz || !plan_made([&] { return spmm_order(a, cut); }))
+        return false;
+    *h = cut;
+    return true;
+}
+
 static int spmm_plan(Csr *a)
 {
     const int64_t nchunks = ceil_div(a->nnz, SPMM_GRAIN);
@@ -1498,22 +1623,6 @@ static bool sweep_uneven(const Csr *a, int64_t K)
     return a->heavy_nnz * 4 >= a->nnz * 3 && a->heavy_nnz >= (K < 32 ? 8 : 4) * a->ncols;
 }
 
-// *held += entries of the rows of min_len entries and more
-__global__ __launch_bounds__(256) void spmm_long_entries(int64_t nrows, const int64_t *__restrict__ pos, int64_t min_len,
-                                                         unsigned long long *__restrict__ held)
-{
-    int64_t mine = 0;
-    for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < nrows; r += (int64_t)gridDim.x * 256) {
-        const int64_t len = pos[r + 1] - pos[r];
-        mine += len >= min_len ? len : 0;
-    }
-    for (int d = 32; d > 0; d >>= 1)
-        mine += ((int64_t)__shfl_down((int)(mine >> 32), d, 64) << 32) + (int64_t)(uint32_t)__shfl_down((int)mine, d, 64);
-    if ((threadIdx.x & 63) == 0 && mine > 0)
-        atomicAdd(held, (unsigned long long)mine);
-}
-static Workspace g_long_entries;
-
 // even: the call's rows are multiples of 16 bytes; if not, the plan is made only if the sweep is worth it for such, and is
 // left to a call with even ones otherwise
 static int spmm_heavy_plan(Csr *a, bool even, int64_t K)
@@ -1521,28 +1630,18 @@ static int spmm_heavy_plan(Csr *a, bool even, int64_t K)
     if (a->heavy_state != 0)
         return COMET_HIP_OK;
     a->heavy_state = 1;
-    if (a->nnz < (1 << 19) || a->nnz >= (1ll << 32) || ceil_div(a->ncols, 8) >= (1ll << SPMM_HCOLB))
+    if (a->nnz < SPMM_SWEEP_NNZ || a->nnz >= (1ll << 32) || ceil_div(a->ncols, 8) >= (1ll << SPMM_HCOLB))
         return COMET_HIP_OK;        // a list entry has SPMM_HCOLB bits for the column inside an XCD's eighth
     const int64_t n = a->nrows;
-    {   // The long rows may hold too little for the sweep: asked of the device, 15 us, before the row pointers are fetched and
-        // gone through here (300000 rows: 540).  Those that are long may be more than the sweep holds.
-        unsigned long long *held = nullptr;
-        COMET_CHK(mailbox((void **)&held));
-        COMET_CHK(g_long_entries.ensure(sizeof *held, false));
-        COMET_HIPCHK(hipMemsetAsync(g_long_entries.ptr, 0, sizeof *held, stream()));
-        spmm_long_entries<<<dim3((unsigned)std::min<int64_t>(ceil_div(n, 256), 2 * (int64_t)num_cus())), dim3(256), 0, stream()>>>(
-            n, a->pos, SPMM_HEAVY_MIN_LEN, (unsigned long long *)g_long_entries.ptr);
-        COMET_HIPCHK(hipGetLastError());
-        COMET_HIPCHK(hipMemcpyAsync(held, g_long_entries.ptr, sizeof *held, hipMemcpyDeviceToHost, stream()));
-        COMET_CHK(stream_wait());
-        a->heavy_nnz = (int64_t)*(volatile unsigned long long *)held;
-        if (!even && !sweep_uneven(a, K)) {
-            a->heavy_state = 0;
-            return COMET_HIP_OK;
-        }
-        if (a->heavy_nnz == 0 || a->heavy_nnz * 4 < a->nnz)
-            return COMET_HIP_OK;
+    // The long rows may hold too little for the sweep: looked at before the row pointers are fetched and gone through here
+    // (300000 rows: 540 us).  Those that are long may be more than the sweep holds.
+    COMET_CHK(spmm_long_rows(a));
+    if (!even && !sweep_uneven(a, K)) {
+        a->heavy_state = 0;
+        return COMET_HIP_OK;
     }
+    if (a->heavy_nnz == 0 || a->heavy_nnz * 4 < a->nnz)
+        return COMET_HIP_OK;
     std::vector<int64_t> pos((size_t)n + 1);
     COMET_HIPCHK(hipMemcpyAsync(pos.data(), a->pos, sizeof(int64_t) * (size_t)(n + 1), hipMemcpyDeviceToHost,
                                 stream()));
@@ -1827,7 +1926,7 @@ static int spmm_heavy_plan(Csr *a, bool even, int64_t K)
 using namespace comet;
 
 static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate, const SpmmShape &h,
-                       hipStream_t on = nullptr);
+                       bool ordered = false, const char *name = "spmm_csr_nnzsplit", hipStream_t on = nullptr);
 static int spmv_run(Csr *a, int64_t x_dptr, int64_t y_dptr, int accumulate);
 static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dptr, int64_t ldc, int accumulate);
 
@@ -1964,7 +2063,12 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
     // once goes through the chunk kernel whole, the plan is made when it is multiplied again.
     const bool plan_now = a->spmm_uses > 0 || plan_at_once();
     a->spmm_uses = a->spmm_uses < 2 ? a->spmm_uses + 1 : 2;
-    const SpmmShape h = spmm_shape(a, K);
+    SpmmShape h = spmm_shape(a, K);
+    if (plan_now && spmm_by_columns(a, K, &h)) {
+        // what would be swept with the sums in registers is a sweep in this form too, and listed as one by the profile
+        const bool sweep = sweep_fits && a->nnz >= SPMM_SWEEP_NNZ && a->long_nnz[0] * 4 >= a->nnz && (even || sweep_uneven(a, K));
+        return spmm_chunks(a, K, B, ldb, C, ldc, accumulate, h, true, sweep ? "spmm_heavy_sweep" : "spmm_csr_nnzsplit");
+    }
     if (sweep_fits && plan_now && a->heavy_state == 0)
         (void)plan_made([&] { return spmm_heavy_plan(a, even, K); });          // or the chunk kernel goes on taking all rows
     if (a->heavy_state != 2 || !sweep_fits)
@@ -2013,7 +2117,7 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
             COMET_CHK(accumulate ? launch(spmm_heavy_sweep<false, true>) : launch(spmm_heavy_sweep<false, false>));
     }
     if (overlap) {      // the rows in between, on the CUs the sweep leaves free
-        COMET_CHK(spmm_chunks(a->light, K, B, ldb, C, ldc, accumulate, light, aux_stream()));
+        COMET_CHK(spmm_chunks(a->light, K, B, ldb, C, ldc, accumulate, light, false, "spmm_csr_nnzsplit", aux_stream()));
         COMET_CHK(aux_join());
     }
     {
@@ -2033,15 +2137,17 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
 }
 
 // The chunk kernel: the row of every grain'th nonzero in chunk_row, chunks of h.len nonzeros (a multiple of grain), two
-// slots for each of them and column tile in carry and a zero in arrived.  name: what events are recorded under (null: none, where the stream is being captured).
+// slots for each of them and column tile in carry and a zero in arrived; order: the chunks in the order they are taken in, or
+// null.  name: what events are recorded under (null: none, where the stream is being captured).
 static void spmm_chunk_launch(const Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate,
-                              const int32_t *chunk_row, int grain, const SpmmShape &h, double *carry,
+                              const int32_t *chunk_row, int grain, const SpmmShape &h, const uint32_t *order, double *carry,
                               unsigned *arrived, hipStream_t on, const char *name)
 {
-    const dim3 grid((unsigned)ceil_div(h.chunks, SPMM_WAVES), (unsigned)h.tiles), block(SPMM_WAVES * 64);
+    const int64_t wide = order ? 8 * ceil_div(ceil_div(h.chunks, 8), SPMM_WAVES) : ceil_div(h.chunks, SPMM_WAVES);
+    const dim3 grid((unsigned)wide, (unsigned)h.tiles), block(SPMM_WAVES * 64);
     const auto split = [&](auto kernel) {
         std::unique_ptr<KernelTimer> t(name ? new KernelTimer(name, on) : nullptr);
-        kernel<<<grid, block, 0, on>>>(a->pos, a->crd, a->val, a->nnz, a->nrows, chunk_row, grain, h.len, h.chunks, B, ldb, C,
+        kernel<<<grid, block, 0, on>>>(a->pos, a->crd, a->val, a->nnz, a->nrows, chunk_row, grain, h.len, h.chunks, order, B, ldb, C,
                                        ldc, K, h.cols, carry, arrived, a->rowmap);
     };
     const bool small_b = K > 1 && a->ncols * ldb * 8 < (1ll << 32);
@@ -2053,8 +2159,9 @@ static void spmm_chunk_launch(const Csr *a, int64_t K, const double *B, int64_t 
         accumulate ? split(spmm_csr_nnzsplit<true, 2, false>) : split(spmm_csr_nnzsplit<false, 2, false>);
 }
 
+// ordered: h is how spmm_by_columns cut the product
 static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate, const SpmmShape &h,
-                       hipStream_t on)
+                       bool ordered, const char *name, hipStream_t on)
 {
     if (!on)
         on = stream();
@@ -2069,8 +2176,9 @@ static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *
     }
     COMET_CHK(spmm_plan(a));
     COMET_CHK(spmm_chunk_scratch(h));
-    spmm_chunk_launch(a, K, B, ldb, C, ldc, accumulate, a->spmm_chunk_row, SPMM_GRAIN, h, (double *)g_spmm_carry.ptr,
-                      (unsigned *)g_spmm_arrived.ptr, on, "spmm_csr_nnzsplit");
+    spmm_chunk_launch(a, K, B, ldb, C, ldc, accumulate, a->spmm_chunk_row, SPMM_GRAIN, h,
+                      ordered ? a->spmm_order[h.len / SPMM_GRAIN / 2] : nullptr, (double *)g_spmm_carry.ptr,
+                      (unsigned *)g_spmm_arrived.ptr, on, name);
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
 }
@@ -2209,7 +2317,7 @@ extern "C" int comet_hip_spmm_csr_f64_noalloc(int64_t csr, int64_t K, int64_t b_
     unsigned *arrived = reinterpret_cast<unsigned *>(scratch + SPMM_STATIC_TABLE_BYTES + SPMM_STATIC_CARRY_BYTES);
     spmm_chunk_rows<<<dim3((unsigned)ceil_div(h.chunks, 256)), dim3(256), 0, on>>>(a->pos, a->nrows, h.chunks, h.len, chunk_row, arrived,
                                                                                    h.tiles * h.chunks);
-    spmm_chunk_launch(a, K, (const double *)b_dptr, ldb, C, ldc, accumulate, chunk_row, h.len, h, carry, arrived, on, nullptr);
+    spmm_chunk_launch(a, K, (const double *)b_dptr, ldb, C, ldc, accumulate, chunk_row, h.len, h, nullptr, carry, arrived, on, nullptr);
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
 }

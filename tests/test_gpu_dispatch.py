@@ -312,6 +312,41 @@ def test_spmm_rows_that_are_not_cut(nrows, K, accumulate):
     assert np.array_equal(dC.to_numpy(), orc.spmm(pos, crd, val, B, C0 if accumulate else None))
 
 
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("nlong,ncols,K", [(40, 20_000, 7), (40, 9_000, 16), (300, 9_000, 21), (300, 4_100, 64), (700, 9_000, 33),
+                                           (700, 120_000, 32), (700, 120_001, 31)])
+def test_spmm_chunks_by_columns(nlong, ncols, K, accumulate, monkeypatch):
+    # from the second product on; chunks of 64, 128 and 256 nonzeros, and 128 in place of 256 for a large B; rows below 128
+    # nonzeros across the blocks of 256, empty rows in front, between and behind
+    monkeypatch.delenv("COMET_HIP_PLAN_AT_ONCE")
+    rng = np.random.default_rng(nlong + K)
+    lens = np.resize([0, 0, 60, 4, 127, 0, 128, 1, 256, 1, 3, 100, 511], 13 * nlong)
+    lens[rng.choice(len(lens) - 1, nlong, replace=False)] = 3000
+    pos = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    crd = np.concatenate([np.sort(rng.choice(ncols, l, replace=False)) for l in lens]).astype(np.int32)
+    val, B, C0 = rng.uniform(-1, 1, pos[-1]), rng.uniform(-1, 1, (ncols, K)), rng.uniform(-1, 1, (len(lens), K))
+    A, dB = rt.CsrMatrix.from_arrays((len(lens), ncols), pos, crd, val), rt.DeviceArray.from_numpy(B)
+    want = orc.spmm(pos, crd, val, B, C0 if accumulate else None)
+    bound = orc.spmm(pos, crd, np.abs(val), np.abs(B), np.abs(C0))
+    whole = (lens < 128) | (pos[:-1] // 256 == (pos[1:] - 1) // 256)
+    first, sorted_at = None, []
+    for _ in range(3):
+        dC = rt.DeviceArray.from_numpy(C0)
+        rt.profile_reset()
+        rt.profile_enable(True)
+        rt.spmm(A, dB, dC, accumulate=accumulate)
+        rt.sync()
+        sorted_at.append("radix_sort_pairs" in rt.profile_report())
+        rt.profile_enable(False)
+        got = dC.to_numpy()
+        assert np.all(np.abs(got - want) <= 1e-12 * bound)
+        assert np.array_equal(got[whole], want[whole])
+        first = got if first is None else first
+        if ncols < 100_000:          # the same chunks: the same sums
+            assert np.array_equal(got, first)
+    assert sorted_at == [False, True, False]
+
+
 @pytest.mark.parametrize("K", [1, 2, 3, 5, 16, 17, 31, 32, 33, 63, 64, 65, 66, 130])
 @pytest.mark.parametrize("nnz", [1, 15, 17, 63, 65, 4097])
 def test_sddmm_of_every_tile_and_width(nnz, K):
