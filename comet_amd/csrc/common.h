@@ -234,6 +234,10 @@ struct Csr {
     int sddmm_state = 0;
     int32_t *sddmm_order = nullptr;
     int64_t sddmm_start[9] = {};
+    int sddmm_tile_state = 0, sddmm_width = 0;
+    int64_t sddmm_nitems = 0;
+    int32_t *sddmm_tile_order = nullptr;
+    void *sddmm_items = nullptr;
 };
 
 // host arrays -> a new matrix (checked, registered by the caller), `more` going up in the same transfer; nullptr on failure

@@ -437,6 +437,11 @@ static void csr_drop_plans(Csr *c)
     (void)dev_free(c->sddmm_order);
     c->sddmm_order = nullptr;
     c->sddmm_state = 0;
+    (void)dev_free(c->sddmm_tile_order);
+    (void)dev_free(c->sddmm_items);
+    c->sddmm_tile_order = nullptr;
+    c->sddmm_items = nullptr;
+    c->sddmm_tile_state = 0;
     c->heavy_nnz = -1;
     c->long_nnz[0] = -1;
     c->heavy_rows = 0;

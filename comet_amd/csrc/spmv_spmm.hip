@@ -2823,7 +2823,291 @@ static int sddmm_order(Csr *b, const int32_t *rows)
     return COMET_HIP_OK;
 }
 
+// ---------------------------------------------------------------------------
+// Entries by tiles of columns, D as it is: a workgroup has a tile of up to 512
+// columns and the entries in it, by rows, up to ten a lane; sixteen rows of the
+// tile of D are in LDS while the next sixteen are on their way, a lane reads its
+// column there and its row of C from memory, sixteen bytes at a time, and adds in
+// ascending k in a register.  D is read once, and neither turned over nor gathered;
+// no product goes through LDS.  What is left is the lines of C: one for every run
+// of entries of one row in a tile, looked up eight times, since a lane takes
+// sixteen bytes of it - two thirds of the time of the CUs' address units, and the
+// reason why runs have to be long (sddmm_tiles).  Rows of C staged in LDS, loaded
+// a line at a time, were slower (250000 rows K = 64 279 us against 234).
+// ---------------------------------------------------------------------------
+constexpr int SDDMM_TILE_T = 1024, SDDMM_TILE_COLS = 512, SDDMM_TILE_K = 16, SDDMM_TILE_BATCHES = 10;
+constexpr int SDDMM_TILE_ENTRIES = SDDMM_TILE_T * SDDMM_TILE_BATCHES;          // what the registers hold of a tile
+constexpr size_t SDDMM_TILE_LDS = sizeof(double) * 2 * SDDMM_TILE_K * SDDMM_TILE_COLS;
+static_assert(SDDMM_TILE_K == SDDMM_TILE_T / 64, "a wavefront fetches a row of the tile");
+
+// begin, count: entries in the order; col: first column of the tile
+struct SddmmItem { int64_t begin; int32_t count, col; };
+
+extern __shared__ __align__(16) double sddmm_lds[];
+
+template <bool SMALL>
+__global__ __launch_bounds__(SDDMM_TILE_T) void sddmm_tile_kernel(const SddmmItem *__restrict__ items, const int32_t *__restrict__ order,
+                                                                const int32_t *__restrict__ rows, const int32_t *__restrict__ cols,
+                                                                const double *__restrict__ val, const double *__restrict__ C,
+                                                                int64_t ldc, const double *__restrict__ D, int64_t ldd,
+                                                                int64_t ncols, int64_t K, int width, double *__restrict__ out)
+{
+    using At = SddmmAt<SMALL>;
+    constexpr int KT = SDDMM_TILE_K, NB = SDDMM_TILE_BATCHES, ROW = SDDMM_TILE_COLS;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const SddmmItem it = items[blockIdx.x];
+    const int count = it.count, nb = (count + SDDMM_TILE_T - 1) / SDDMM_TILE_T;
+    const int w = (int)(ncols - it.col < width ? ncols - it.col : width);
+    typename At::Off row[NB];
+    int col[NB];
+    double t[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const int e = b * SDDMM_TILE_T + (int)threadIdx.x;
+        const int64_t at = it.begin + (e < count ? e : count - 1);
+        row[b] = At::row(rows[at], ldc, 0);
+        col[b] = b < nb ? cols[at] - it.col : 0;
+        t[b] = 0.0;
+    }
+    double next[ROW / 64];
+    const auto fetch = [&](int64_t i) {
+        const int64_t k = i * KT + wave;
+#pragma unroll
+        for (int q = 0; q < ROW / 64; ++q)
+            if (k < K && 64 * q + lane < w)
+                next[q] = D[k * ldd + it.col + 64 * q + lane];
+    };
+    const auto put = [&](double *buf) {
+#pragma unroll
+        for (int q = 0; q < ROW / 64; ++q)
+            if (64 * q + lane < w)
+                buf[wave * ROW + 64 * q + lane] = next[q];
+    };
+    const int64_t pieces = K / KT;
+    const int rest = (int)(K - pieces * KT);
+    fetch(0);
+    put(sddmm_lds);
+    __syncthreads();
+    // Sixteen columns from Ck on, or a last piece of kp: half of a batch's are on their way while the other half is added.
+    // MANY: of more than four columns; no load and no sum on a condition then, which would make every sum wait for all loads,
+    // but the last two columns in the place of those behind them, and sums that are dropped.
+    enum { ALL, MANY, FEW };
+    const auto piece = [&](const double *buf, const double *Ck, auto kind, int kp) {
+        constexpr int KIND = decltype(kind)::value;
+        spmm_pair c[2][KT / 4];
+        const auto load = [&](int h, typename At::Off r) {
+#pragma unroll
+            for (int q = 0; q < KT / 4; ++q) {
+                const int k = h * (KT / 2) + 2 * q;
+                if (KIND == ALL || (KIND == FEW && k + 1 < kp))
+                    c[h][q] = *reinterpret_cast<const spmm_pair *>(At::at(Ck + k, r));
+                else if (KIND == MANY)
+                    c[h][q] = *reinterpret_cast<const spmm_pair *>(At::at(Ck + (k + 1 < kp ? k : kp - 2), r));
+                else if (k < kp)
+                    c[h][q].x = *At::at(Ck + k, r);
+            }
+        };
+        const auto add = [&](int h, double &t, const double *d) {
+#pragma unroll
+            for (int q = 0; q < KT / 4; ++q) {
+                const int k = h * (KT / 2) + 2 * q;
+                if constexpr (KIND == MANY) {
+                    const double x = t + (k + 1 < kp ? c[h][q].x : c[h][q].y) * d[k * ROW];
+                    t = k < kp ? x : t;
+                    const double y = t + c[h][q].y * d[(k + 1) * ROW];
+                    t = k + 1 < kp ? y : t;
+                } else {
+                    if (KIND == ALL || k < kp)
+                        t = t + c[h][q].x * d[k * ROW];
+                    if (KIND == ALL || k + 1 < kp)
+                        t = t + c[h][q].y * d[(k + 1) * ROW];
+                }
+            }
+        };
+        const bool both = KIND == ALL || (KIND == MANY && kp > KT / 2);
+        load(0, row[0]);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            if (b < nb) {
+                const double *d = buf + col[b];
+                if (both)
+                    load(1, row[b]);
+                add(0, t[b], d);
+                if (b + 1 < NB)
+                    load(0, row[b + 1 < NB ? b + 1 : b]);
+                if (both)
+                    add(1, t[b], d);
+            }
+        }
+    };
+    for (int64_t i = 0; i < pieces; ++i) {
+        fetch(i + 1);
+        piece(sddmm_lds + (i & 1) * KT * ROW, C + i * KT, std::integral_constant<int, ALL>(), KT);
+        put(sddmm_lds + ((i + 1) & 1) * KT * ROW);
+        __syncthreads();
+    }
+    if (rest > 4)
+        piece(sddmm_lds + (pieces & 1) * KT * ROW, C + pieces * KT, std::integral_constant<int, MANY>(), rest);
+    else if (rest > 0)
+        piece(sddmm_lds + (pieces & 1) * KT * ROW, C + pieces * KT, std::integral_constant<int, FEW>(), rest);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const int e = b * SDDMM_TILE_T + (int)threadIdx.x;
+        if (e < count) {
+            const int64_t p = order[it.begin + e];
+            out[p] = val[p] * t[b];
+        }
+    }
+}
+
+// keys[p]: the tile of entry p
+__global__ __launch_bounds__(256) void sddmm_tile_keys(int64_t nnz, const int32_t *__restrict__ crd, int width,
+                                                       uint64_t *__restrict__ keys, uint32_t *__restrict__ idx)
+{
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p >= nnz)
+        return;
+    keys[p] = (uint64_t)(crd[p] / width);
+    idx[p] = (uint32_t)p;
+}
+
+// start[x] = first entry of tile x or a later one, x = 0 .. ntiles
+__global__ __launch_bounds__(256) void sddmm_tile_starts(int64_t nnz, const uint64_t *__restrict__ keys, int64_t ntiles,
+                                                         int64_t *__restrict__ start)
+{
+    const int64_t x = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (x > ntiles)
+        return;
+    int64_t lo = 0, hi = nnz;
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if ((int64_t)keys[mid] < x)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    start[x] = lo;
+}
+
+// *runs += entries that are not of the row and tile of the one before
+__global__ __launch_bounds__(256) void sddmm_tile_runs(int64_t nnz, const int32_t *__restrict__ rows, const int32_t *__restrict__ crd,
+                                                       int width, unsigned long long *__restrict__ runs)
+{
+    unsigned long long mine = 0;
+    for (int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x; p < nnz; p += (int64_t)gridDim.x * 256)
+        mine += p == 0 || rows[p] != rows[p - 1] || crd[p] / width != crd[p - 1] / width;
+    for (int d = 32; d > 0; d >>= 1)
+        mine += (unsigned long long)__shfl_down((int)mine, d, 64);
+    if ((threadIdx.x & 63) == 0)
+        atomicAdd(runs, mine);
+}
+
+// How a matrix is cut into tiles: every CU the same number of them (rounds), of as few columns as the entries allow.  (One
+// workgroup is on a CU at a time: 250000 columns, K = 64, in 489 tiles 214 us, in 559 275.)
+static int64_t sddmm_tile_width(const Csr *b, int64_t *rounds)
+{
+    const double most = 0.9 * SDDMM_TILE_ENTRIES * (double)b->ncols / (double)b->nnz;
+    const int64_t width = most < SDDMM_TILE_COLS ? std::max<int64_t>(1, (int64_t)most) : SDDMM_TILE_COLS;
+    *rounds = ceil_div(b->ncols, num_cus() * width);
+    return std::max<int64_t>(16, ceil_div(b->ncols, num_cus() * *rounds));
+}
+
+// The plan: worth it where a run of entries of one row in one tile is two and a half entries long.  us, whole call, gathered / by
+// tiles, and entries a run: zipf 20000 rows of 15 (3.7) K = 33 23.2 / 14.5, 250000 of 16 (2.7) 196 / 149, band of 15 in 100000 rows (15) K = 64 78.8 / 60.6;
+// R-MAT scale 15 (2.2) K = 33 38.8 / 44.1, scale 17 (2.1) K = 64 129 / 151; 100000 rows of 16 uniform entries (1.03) K = 64
+// 140 / 158, 60000 of 40 K = 16 46 / 102.
+constexpr double SDDMM_TILE_RUN = 2.5;
+static int sddmm_tiles(Csr *b, const int32_t *rows)
+{
+    b->sddmm_tile_state = 1;
+    int64_t rounds = 0;
+    const int64_t width = sddmm_tile_width(b, &rounds);
+    {
+        unsigned long long *held = nullptr;
+        COMET_CHK(mailbox((void **)&held));
+        COMET_CHK(g_sddmm_plan.ensure(sizeof *held, false));
+        COMET_HIPCHK(hipMemsetAsync(g_sddmm_plan.ptr, 0, sizeof *held, stream()));
+        sddmm_tile_runs<<<dim3((unsigned)std::min<int64_t>(ceil_div(b->nnz, 256), 4 * (int64_t)num_cus())), dim3(256), 0, stream()>>>(
+            b->nnz, rows, b->crd, (int)width, (unsigned long long *)g_sddmm_plan.ptr);
+        COMET_HIPCHK(hipGetLastError());
+        COMET_HIPCHK(hipMemcpyAsync(held, g_sddmm_plan.ptr, sizeof *held, hipMemcpyDeviceToHost, stream()));
+        COMET_CHK(stream_wait());
+        const int64_t runs = (int64_t)*(volatile unsigned long long *)held;
+        if ((double)b->nnz < SDDMM_TILE_RUN * (double)runs)
+            return COMET_HIP_OK;
+    }
+    // a tile of more entries than its share is taken in parts
+    const int64_t share = ceil_div(5 * b->nnz, 4 * num_cus() * rounds);
+    const int64_t most = std::min<int64_t>(SDDMM_TILE_ENTRIES, ceil_div(share, SDDMM_TILE_T) * SDDMM_TILE_T);
+    const int64_t ntiles = ceil_div(b->ncols, width);
+    int end_bit = 1;
+    while ((1ll << end_bit) <= ntiles)
+        ++end_bit;
+    const size_t n = (size_t)b->nnz;
+    uint64_t *keys = nullptr;
+    uint32_t *idx = nullptr, *order = nullptr;
+    int64_t *d_start = nullptr;
+    SddmmItem *d_items = nullptr;
+    std::vector<SddmmItem> items;
+    const auto run = [&]() -> int {
+        COMET_HIPCHK(dev_malloc((void **)&keys, 16 * n));
+        COMET_HIPCHK(dev_malloc((void **)&idx, 4 * n));
+        COMET_HIPCHK(dev_malloc((void **)&order, 12 * n));
+        COMET_HIPCHK(dev_malloc((void **)&d_start, sizeof(int64_t) * (size_t)(ntiles + 1)));
+        const dim3 grid((unsigned)ceil_div(b->nnz, 256)), block(256);
+        sddmm_tile_keys<<<grid, block, 0, stream()>>>(b->nnz, b->crd, (int)width, keys, idx);
+        COMET_CHK(sort_pairs_u64_u32(keys, keys + n, idx, order, b->nnz, end_bit));
+        sddmm_gather<<<grid, block, 0, stream()>>>(b->nnz, (const int32_t *)order, rows, b->crd, (int32_t *)order + n,
+                                                   (int32_t *)order + 2 * n);
+        sddmm_tile_starts<<<dim3((unsigned)ceil_div(ntiles + 1, 256)), block, 0, stream()>>>(b->nnz, keys + n, ntiles, d_start);
+        std::vector<int64_t> start((size_t)ntiles + 1);
+        COMET_HIPCHK(hipMemcpyAsync(start.data(), d_start, sizeof(int64_t) * start.size(), hipMemcpyDeviceToHost, stream()));
+        COMET_CHK(stream_wait());
+        for (int64_t x = 0; x < ntiles; ++x) {
+            const int64_t held = start[(size_t)x + 1] - start[(size_t)x], parts = ceil_div(held, most);
+            for (int64_t q = 0; q < parts; ++q) {
+                const int64_t from = start[(size_t)x] + held * q / parts, to = start[(size_t)x] + held * (q + 1) / parts;
+                items.push_back({from, (int32_t)(to - from), (int32_t)(x * width)});
+            }
+        }
+        std::stable_sort(items.begin(), items.end(), [](const SddmmItem &a, const SddmmItem &c) { return a.count > c.count; });
+        COMET_HIPCHK(dev_malloc((void **)&d_items, sizeof(SddmmItem) * items.size()));
+        COMET_HIPCHK(hipMemcpyAsync(d_items, items.data(), sizeof(SddmmItem) * items.size(), hipMemcpyHostToDevice, stream()));
+        return stream_wait();
+    };
+    const int rc = run();
+    (void)dev_free(keys);
+    (void)dev_free(idx);
+    (void)dev_free(d_start);
+    if (rc != COMET_HIP_OK) {
+        (void)dev_free(order);
+        (void)dev_free(d_items);
+        return rc;
+    }
+    b->sddmm_tile_order = (int32_t *)order;
+    b->sddmm_items = d_items;
+    b->sddmm_nitems = (int64_t)items.size();
+    b->sddmm_width = (int)width;
+    b->sddmm_tile_state = 2;
+    return COMET_HIP_OK;
+}
+
 static Workspace g_sddmm_dt;
+
+// Whether a matrix that is sampled at again is to go by tiles for these K columns.  us, zipf, 16 entries a row, gathered /
+// by tiles: one tile a CU 10000 rows K = 9 10.6 / 7.6, K = 64 17.4 / 14.6, 35000 K = 24 26 / 16.5, 60000 K = 17 39 / 20, 100000
+// K = 3 22.5 / 21.2, K = 33 79 / 52, K = 64 96 / 78 - but 5000 rows K = 64 11.8 / 13.0, a chain of four loads and barriers -;
+// two tiles a CU, one after the other, 160000 K = 15 56 / 69, K = 24 81 / 73, 250000 K = 33 196 / 149, K = 64 228 / 207,
+// 260000 K = 47 189 / 191 (a last piece of 15 columns costs more than a whole one); three
+// 350000 K = 24 176 / 186, K = 64 326 / 329.
+static bool sddmm_tiled(const Csr *b, int64_t K)
+{
+    if (K < 1 || b->nnz < (K > 40 ? 1 << 17 : 1 << 15) || b->nnz >= 1ll << 31)
+        return false;
+    int64_t rounds = 0;
+    (void)sddmm_tile_width(b, &rounds);
+    return rounds == 1 || (rounds == 2 && K > 16 && K % 16 <= 12);
+}
 
 static int sddmm_values(Csr *b, int64_t K, int64_t c_dptr, int64_t ldc, int64_t d_dptr, int64_t ldd, double *out)
 {
@@ -2832,6 +3116,30 @@ static int sddmm_values(Csr *b, int64_t K, int64_t c_dptr, int64_t ldc, int64_t 
                          (long long)K, (long long)ldc, (long long)ldd);
     if (b->nnz == 0)
         return COMET_HIP_OK;
+    const int32_t *rows = nullptr;
+    // ordering the entries costs some five products: made when the matrix is sampled at again
+    const bool plan_now = b->sddmm_uses > 0 || plan_at_once();
+    b->sddmm_uses = 1;
+    if (plan_now && sddmm_tiled(b, K)) {
+        COMET_CHK(csr_entry_rows(b, &rows));
+        if (b->sddmm_tile_state == 0)
+            (void)plan_made([&] { return sddmm_tiles(b, rows); });
+        if (b->sddmm_tile_state == 2) {
+            KernelTimer t("sddmm_tile_kernel");
+            const bool small = b->nrows <= 1 << 24 && ldc * 8 < 1 << 24 && b->nrows * ldc * 8 < (1ll << 32);
+            const int32_t *order = b->sddmm_tile_order;
+            const auto launch = [&](auto kernel) -> int {
+                COMET_HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 (int)SDDMM_TILE_LDS));
+                kernel<<<dim3((unsigned)b->sddmm_nitems), dim3(SDDMM_TILE_T), SDDMM_TILE_LDS, stream()>>>(
+                    (const SddmmItem *)b->sddmm_items, order, order + b->nnz, order + 2 * b->nnz, b->val, (const double *)c_dptr, ldc,
+                    (const double *)d_dptr, ldd, b->ncols, K, b->sddmm_width, out);
+                COMET_HIPCHK(hipGetLastError());
+                return COMET_HIP_OK;
+            };
+            return small ? launch(sddmm_tile_kernel<true>) : launch(sddmm_tile_kernel<false>);
+        }
+    }
     // Rows of D begin at a line of 128 bytes, 16 columns are one line then, unless that makes them nearly twice as long
     // (200000 rows, 3.7 M entries, us, packed / so: K = 3 50 / 71, 9 69 / 65, 15 80 / 73, 17 86 / 91, 18 85 / 79, 28 117 /
     // 105, 50 219 / 179, 61 253 / 197, 100 390 / 317), D very large, or no room for it.
@@ -2844,11 +3152,7 @@ static int sddmm_values(Csr *b, int64_t K, int64_t c_dptr, int64_t ldc, int64_t 
         COMET_CHK(room());
         COMET_CHK(transpose2d((const double *)d_dptr, ldd, K, b->ncols, (double *)g_sddmm_dt.ptr, ldt));
     }
-    const int32_t *rows = nullptr;
     COMET_CHK(csr_entry_rows(b, &rows));
-    // ordering the entries costs some five products: made when the matrix is sampled at again
-    const bool plan_now = b->sddmm_uses > 0 || plan_at_once();
-    b->sddmm_uses = 1;
     const bool large = b->nnz >= SDDMM_ORDER_NNZ && b->ncols * K * 8 >= SDDMM_ORDER_D;
     if (large && plan_now && b->sddmm_state == 0)
         (void)plan_made([&] { return sddmm_order(b, rows); });

@@ -380,6 +380,46 @@ def test_sddmm_of_many_entries(nnz, K):
     assert np.array_equal(got[:nnz], orc.sddmm(pos, crd, val, C, D)) and got[nnz] == 7.0
 
 
+@pytest.mark.parametrize("kind", ["band", "one tile", "hub", "two rounds", "widest tile"])
+@pytest.mark.parametrize("K", [1, 2, 7, 15, 16, 17, 31, 33, 48, 70])
+def test_sddmm_by_tiles_of_columns(kind, K, monkeypatch):
+    # runs of entries of one row in tiles of 16 columns to 512, entries of a tile in one part or several, the last one of a
+    # wavefront or two; pieces of sixteen columns of C and every kind of rest; operands wider than they need be
+    monkeypatch.delenv("COMET_HIP_PLAN_AT_ONCE")
+    rng = np.random.default_rng(K)
+    n, m, run = {"band": (2500, 2600, 70), "one tile": (9000, 16, 15), "hub": (20_000, 5000, 12), "two rounds": (4600, 131_073, 40),
+                 "widest tile": (5000, 131_072, 40)}[kind]
+    first = rng.integers(0, m - run + 1, n)
+    if kind == "hub":
+        first[:15_000] = rng.integers(0, 4, 15_000)
+    crd = (first[:, None] + np.arange(run)).ravel()
+    lens = np.full(n, run)
+    drop = rng.choice(n, n // 50, replace=False)
+    keep = np.ones((n, run), bool)
+    keep[drop] = False                    # empty rows
+    lens[drop] = 0
+    crd = crd[keep.ravel()].astype(np.int32)
+    pos = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    assert pos[-1] >= 1 << 15
+    val, C, D = rng.uniform(-1, 1, pos[-1]), rng.uniform(-1, 1, (n, K + 3)), rng.uniform(-1, 1, (K, m + 5))
+    S, out = rt.CsrMatrix.from_arrays((n, m), pos, crd, val), rt.DeviceArray.from_numpy(np.full(pos[-1] + 1, 7.0))
+    dC, dD = rt.DeviceArray.from_numpy(C), rt.DeviceArray.from_numpy(D)
+    want = orc.sddmm(pos, crd, val, np.ascontiguousarray(C[:, :K]), np.ascontiguousarray(D[:, :m]))
+    tiled = []
+    for _ in range(3):
+        rt._check(rt.lib().comet_hip_memcpy(out.ptr, rt._vptr(np.full(pos[-1] + 1, 7.0)), 8 * (int(pos[-1]) + 1), 0))
+        rt.profile_reset()
+        rt.profile_enable(True)
+        rt._check(rt.lib().comet_hip_sddmm_csr_values_f64(S.handle, K, dC.ptr, K + 3, dD.ptr, m + 5, out.ptr), "sddmm")
+        rt.sync()
+        tiled.append("sddmm_tile_kernel" in rt.profile_report())
+        rt.profile_enable(False)
+        got = out.to_numpy()
+        assert np.array_equal(got[:-1], want) and got[-1] == 7.0
+    by_tiles = (kind != "two rounds" or (K > 16 and K % 16 <= 12)) and (K <= 40 or pos[-1] >= 1 << 17)
+    assert tiled == [False, by_tiles, by_tiles]
+
+
 @pytest.mark.parametrize("wide", [False, True])
 def test_sddmm_of_every_piece_and_rest(wide):
     # every number of columns up to three pieces: whole ones, a last one with lanes behind its end, a rest of one or two a lane;
