@@ -221,7 +221,7 @@ static int transpose_device(int rank, const int64_t *in_shape, const int32_t *pe
 // TM x TN MFMA tiles of 16 x 16.  K advances 16 at a time through
 // double-buffered LDS, both operands stored k-major (a 16 x 4 operand is one
 // ds_read_b64 per lane).  Offsets of the rows and columns are worked out once
-// per tile of C, those of the 16 k of a turn by sixteen lanes two turns ahead.
+// per tile of C, those of the 16 k of a turn sixteen turns at a time, one to a lane.
 // A thread takes its elements along whichever index is contiguous in memory
 // (A_M / B_N: the outer one, else along k).  Operand layout of
 // v_mfma_f64_16x16x4_f64: lane l supplies A[l%16][l/16] and B[l/16][l%16] and
@@ -301,8 +301,8 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
     constexpr int KSA = 256 / BM, KSB = 256 / BN;
     __shared__ double As[2][GM_BK][LDA];
     __shared__ double Bs[2][GM_BK][LDB];
-    // offsets in bytes of the rows (A), the columns (B) and, unless they are regular, of the k of two turns
-    __shared__ uint32_t rowA[BM], colB[BN], kA[2][GM_BK], kB[2][GM_BK];
+    // offsets in bytes of the rows (A), the columns (B) and, unless they are regular, of the k of sixteen turns, twice
+    __shared__ uint32_t rowA[BM], colB[BN], kA[REG ? 1 : 2][REG ? 1 : 256], kB[REG ? 1 : 2][REG ? 1 : 256];
     __shared__ int64_t rowC[BM], colC[BN];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WN, wn = wave % WN;
@@ -312,13 +312,14 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
     const uint32_t k_end = k_begin + g.turns * GM_BK < g.K ? k_begin + g.turns * GM_BK : g.K;
     const int nt = (int)((k_end - k_begin + GM_BK - 1) / GM_BK);
 
-    const auto k_offsets = [&](int t) {          // the offsets of turn t's k, by the first sixteen lanes
-        if (!REG && tid < GM_BK) {
-            const uint32_t k = k_begin + (uint32_t)t * GM_BK + tid;
+    // the offsets of the k of sixteen turns, one to a lane (by sixteen lanes a turn they were the longest chain of every turn)
+    const auto k_offsets = [&](int chunk) {
+        if constexpr (!REG) {
+            const uint32_t k = k_begin + 256u * (uint32_t)chunk + tid;
             uint32_t a, b;
             gett_offsets(g.k, k < k_end ? k : k_end - 1, &a, &b);
-            kA[t & 1][tid] = a * 8;
-            kB[t & 1][tid] = b * 8;
+            kA[chunk & 1][tid] = a * 8;
+            kB[chunk & 1][tid] = b * 8;
         }
     };
     for (int r = tid; r < BM; r += 256) {
@@ -334,8 +335,6 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
         colC[c] = d;
     }
     k_offsets(0);
-    if (nt > 1)
-        k_offsets(1);
     __syncthreads();
 
     // thread -> elements of a turn's tiles: along the outer index (one row, E values of k) or along k (one k, E rows).
@@ -427,7 +426,7 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
             k_next += GM_BK;
             --run;
         } else {
-            const uint32_t *ka = kA[t & 1], *kb = kB[t & 1];
+            const uint32_t *ka = kA[t >> 4 & 1] + (t & 15) * GM_BK, *kb = kB[t >> 4 & 1] + (t & 15) * GM_BK;
 #pragma unroll
             for (int e = 0; e < EA; ++e)
                 ra[e] = gett_load(A, A_M ? ao[0] + ka[a_k + KSA * e] : ao[A_M ? 0 : e] + ka[a_k]);
@@ -487,8 +486,8 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
         fragments(0);
         if (t + 1 < nt)
             load_tiles(t + 1);
-        if (!REG && t + 2 < nt)
-            k_offsets(t + 2);           // the slot turn t was loaded through
+        if (!REG && (t + 2) % 16 == 0 && t + 2 < nt)
+            k_offsets((t + 2) / 16);           // for the loads of the next turn
 #pragma unroll
         for (int ks = 0; ks < GM_BK; ks += 4) {
             if (ks + 4 < GM_BK)
@@ -531,35 +530,40 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
         }
 }
 
-// C[m,n] (+)= the partial tiles in order of their k.  `group` threads of a workgroup share an output: each adds
-// every group-th partial, then the first adds what the others have.
-__global__ __launch_bounds__(256) void gett_reduce(GettArgs g, int splits, int group, const double *__restrict__ partial,
-                                                   double *__restrict__ C, int use_c)
+// C[m,n] (+)= the partial tiles.  `group` threads of a workgroup share an output: each adds every group-th partial in order of
+// k, up to eight of them on their way at once, then those sums are added by halves, a step of a fixed tree at a time.
+// Bound by the trips to memory one after the other: 491 shares of 1830 outputs, 31 to a thread and four at once, took 6.5 us,
+// now 5.7, 3 of them the launch.
+constexpr int GETT_REDUCE_T = 1024, GETT_REDUCE_U = 8;
+__global__ __launch_bounds__(GETT_REDUCE_T) void gett_reduce(GettArgs g, int splits, int group, const double *__restrict__ partial,
+                                                             double *__restrict__ C, int use_c)
 {
-    __shared__ double lds[256];
-    const int per = 256 / group, o = threadIdx.x % per, share = threadIdx.x / per;
+    __shared__ double lds[GETT_REDUCE_T];
+    const int per = GETT_REDUCE_T / group, o = threadIdx.x % per, share = threadIdx.x / per;
     const uint64_t total = (uint64_t)g.M * g.N, i = (uint64_t)blockIdx.x * per + o;
     double s = 0.0;
     if (i < total) {
-        int z = share;
-        for (; z + 3 * group < splits; z += 4 * group) {
-            const double p0 = partial[(uint64_t)z * total + i], p1 = partial[(uint64_t)(z + group) * total + i],
-                         p2 = partial[(uint64_t)(z + 2 * group) * total + i],
-                         p3 = partial[(uint64_t)(z + 3 * group) * total + i];
-            s = s + p0;
-            s = s + p1;
-            s = s + p2;
-            s = s + p3;
+        const double *at = partial + i;
+        for (int z = share; z < splits; z += GETT_REDUCE_U * group) {
+            double p[GETT_REDUCE_U];
+#pragma unroll
+            for (int u = 0; u < GETT_REDUCE_U; ++u)
+                p[u] = z + u * group < splits ? at[(uint64_t)(z + u * group) * total] : 0.0;
+#pragma unroll
+            for (int u = 0; u < GETT_REDUCE_U; ++u)
+                s = z + u * group < splits ? s + p[u] : s;
         }
-        for (; z < splits; z += group)
-            s = s + partial[(uint64_t)z * total + i];
     }
-    lds[threadIdx.x] = s;
-    __syncthreads();
+    for (int half = group / 2; half > 0; half /= 2) {
+        if (share >= half && share < 2 * half)
+            lds[threadIdx.x - half * per] = s;
+        __syncthreads();
+        if (share < half)
+            s = s + lds[threadIdx.x];
+        __syncthreads();
+    }
     if (share != 0 || i >= total)
         return;
-    for (int q = 1; q < group; ++q)
-        s = s + lds[q * per + o];
     int64_t ma, mc, nb, nc;
     gett_offsets(g.m, (uint32_t)(i / g.N), &ma, &mc);
     gett_offsets(g.n, (uint32_t)(i % g.N), &nb, &nc);
@@ -576,6 +580,9 @@ struct GettShape {
     double turn_us, alone_us;
 };
 constexpr GettShape GETT_SHAPES[] = {{128, 128, 2, 1.86, 2.65}, {64, 64, 4, 0.52, 1.2}, {64, 32, 6, 0.30, 0.71}, {128, 16, 4, 0.38, 0.83}};
+// What adding the shares up costs besides reading them, a launch: 10 x 60 x 12 x 40 over 120 products take 13.7 us in eight
+// shares, 10.9 in one.
+constexpr double GETT_REDUCE_US = 5.0;
 constexpr int GETT_NSHAPES = sizeof(GETT_SHAPES) / sizeof(GETT_SHAPES[0]);
 
 static Workspace g_gett_partial;
@@ -657,7 +664,7 @@ static int gett_run(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t N,
             const double per_cu = (double)std::min<int64_t>(sh.resident, ceil_div(groups, cus));
             const double turn = std::max(sh.alone_us, per_cu * sh.turn_us);
             const double us = (double)rounds * ((double)turns * turn + 2.5) +
-                              (s > 1 ? 3.0 + (double)ceil_div(nk, turns) * (double)(M * N) * 16.0 / 3.0e6 : 0.0);
+                              (s > 1 ? GETT_REDUCE_US + (double)ceil_div(nk, turns) * (double)(M * N) * 16.0 / 3.0e6 : 0.0);
             if (best_us == 0.0 || us < best_us) {
                 best_us = us;
                 best = c;
@@ -725,11 +732,11 @@ static int gett_run(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t N,
     }
     if (splits > 1) {
         int group = 1;
-        while (group < 16 && group * 8 <= splits)
+        while (group < GETT_REDUCE_T / 16 && group * 4 < splits)
             group *= 2;
         KernelTimer t("gett_reduce");
-        gett_reduce<<<dim3((unsigned)ceil_div(M * N, 256 / group)), dim3(256), 0, stream()>>>(g, (int)splits, group,
-                                                                                             partial, C, use_c);
+        gett_reduce<<<dim3((unsigned)ceil_div(M * N, GETT_REDUCE_T / group)), dim3(GETT_REDUCE_T), 0, stream()>>>(
+            g, (int)splits, group, partial, C, use_c);
     }
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
