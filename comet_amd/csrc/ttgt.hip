@@ -583,6 +583,9 @@ constexpr GettShape GETT_SHAPES[] = {{128, 128, 2, 1.86, 2.65}, {64, 64, 4, 0.52
 // What adding the shares up costs besides reading them, a launch: 10 x 60 x 12 x 40 over 120 products take 13.7 us in eight
 // shares, 10.9 in one.
 constexpr double GETT_REDUCE_US = 5.0;
+// bytes a us that partial tiles are written and read at: few and large, many and small (62 x 62 outputs 97 shares 12.3 us, 194
+// 14.4; 300 x 650 over 225 products one share 18.4, four 16.5)
+constexpr double GETT_REDUCE_FEW = 6.0e6, GETT_REDUCE_MANY = 3.0e6;
 constexpr int GETT_NSHAPES = sizeof(GETT_SHAPES) / sizeof(GETT_SHAPES[0]);
 
 static Workspace g_gett_partial;
@@ -664,7 +667,9 @@ static int gett_run(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t N,
             const double per_cu = (double)std::min<int64_t>(sh.resident, ceil_div(groups, cus));
             const double turn = std::max(sh.alone_us, per_cu * sh.turn_us);
             const double us = (double)rounds * ((double)turns * turn + 2.5) +
-                              (s > 1 ? GETT_REDUCE_US + (double)ceil_div(nk, turns) * (double)(M * N) * 16.0 / 3.0e6 : 0.0);
+                              (s > 1 ? GETT_REDUCE_US + (double)ceil_div(nk, turns) * (double)(M * N) * 16.0 /
+                                                            (s <= 4 ? GETT_REDUCE_FEW : GETT_REDUCE_MANY)
+                                     : 0.0);
             if (best_us == 0.0 || us < best_us) {
                 best_us = us;
                 best = c;
@@ -868,25 +873,19 @@ static int make_plan(int32_t rankA, const int32_t *a_lab, int32_t rankB, const i
                     cur.rankA = rankA;
                     cur.rankB = rankB;
                     cur.rankC = rankC;
-                    std::vector<int32_t> ai, bi, ci;
-                    if (sw) {
-                        ai = k; ai.insert(ai.end(), m.begin(), m.end());
-                        bi = n; bi.insert(bi.end(), k.begin(), k.end());
-                        ci = n; ci.insert(ci.end(), m.begin(), m.end());
-                    } else {
-                        ai = m; ai.insert(ai.end(), k.begin(), k.end());
-                        bi = k; bi.insert(bi.end(), n.begin(), n.end());
-                        ci = m; ci.insert(ci.end(), n.begin(), n.end());
-                    }
-                    std::copy(ai.begin(), ai.end(), cur.a_idx);
-                    std::copy(bi.begin(), bi.end(), cur.b_idx);
-                    std::copy(ci.begin(), ci.end(), cur.c_idx);
+                    // (written in place: a candidate's three lists in vectors were most of what a plan takes)
+                    const auto join = [](const std::vector<int32_t> &x, const std::vector<int32_t> &y, int32_t *to) {
+                        std::copy(y.begin(), y.end(), std::copy(x.begin(), x.end(), to));
+                    };
+                    join(sw ? k : m, sw ? m : k, cur.a_idx);
+                    join(sw ? n : k, sw ? k : n, cur.b_idx);
+                    join(sw ? n : m, sw ? m : n, cur.c_idx);
                     positions_of(a_lab, cur.a_idx, rankA, cur.permA);
                     positions_of(b_lab, cur.b_idx, rankB, cur.permB);
                     positions_of(c_lab, cur.c_idx, rankC, cur.permC);
-                    cur.transA = !std::equal(ai.begin(), ai.end(), a_lab);
-                    cur.transB = !std::equal(bi.begin(), bi.end(), b_lab);
-                    cur.transC = !std::equal(ci.begin(), ci.end(), c_lab);
+                    cur.transA = !std::equal(cur.a_idx, cur.a_idx + rankA, a_lab);
+                    cur.transB = !std::equal(cur.b_idx, cur.b_idx + rankB, b_lab);
+                    cur.transC = !std::equal(cur.c_idx, cur.c_idx + rankC, c_lab);
                     cur.swapAB = sw;
                     cur.M = M;
                     cur.N = N;

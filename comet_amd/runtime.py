@@ -7,6 +7,7 @@ tensors: dense tensors as contiguous row-major float64, sparse matrices as the
 There is no CPU fallback: if the shared library has not been built, or no
 MI355X is present, every entry point raises.
 """
+import array
 import ctypes as C
 import os
 
@@ -615,14 +616,26 @@ def label_ids(a, b, c):
     return ids, conv(a), conv(b), conv(c)
 
 
+def _ints(code, values):
+    """A few integers for a call: (what holds them, their address).  An array of numpy's and a pointer to it take 3 us, which
+    is what a small contraction takes on the device; one element more, so that there is an address without any."""
+    held = array.array(code, values)
+    held.append(0)
+    return held, held.buffer_info()[0]
+
+
 def ttgt_plan(a, b, c, extent, which=-1):
-    ids, al, bl, cl = label_ids(a, b, c)
-    ext = np.zeros(len(ids), dtype=np.int64)
-    for ch, i in ids.items():
-        ext[i] = extent[ch]
+    ids = {}
+    for s in (a, b, c):
+        for ch in s:
+            ids.setdefault(ch, len(ids))
+    al, al_at = _ints("i", [ids[ch] for ch in a])
+    bl, bl_at = _ints("i", [ids[ch] for ch in b])
+    cl, cl_at = _ints("i", [ids[ch] for ch in c])
+    ext, ext_at = _ints("q", [int(extent[ch]) for ch in ids])
     plan = TtgtPlan()
-    _check(lib().comet_hip_ttgt_plan(len(al), _vptr(al), len(bl), _vptr(bl), len(cl), _vptr(cl), _vptr(ext), which,
-                                     C.byref(plan)), "comet_hip_ttgt_plan")
+    _check(lib().comet_hip_ttgt_plan(len(a), al_at, len(b), bl_at, len(c), cl_at, ext_at, which, C.byref(plan)),
+           "comet_hip_ttgt_plan")
     return plan
 
 
@@ -638,8 +651,8 @@ def ttgt_contract(a, b, c, A, B, Cm=None, beta=0.0, which=-1, plan=None):
     cshape = [extent[ch] for ch in c]
     if Cm is None:
         Cm = DeviceArray(cshape, zero=True)
-    ash, bsh, csh = (np.array(s, dtype=np.int64) for s in (A.shape, B.shape, cshape))
-    _check(lib().comet_hip_ttgt_contract(C.byref(plan), _vptr(ash), _vptr(bsh), _vptr(csh), A.ptr, B.ptr, Cm.ptr, beta),
+    (ash, ash_at), (bsh, bsh_at), (csh, csh_at) = _ints("q", A.shape), _ints("q", B.shape), _ints("q", cshape)
+    _check(lib().comet_hip_ttgt_contract(C.byref(plan), ash_at, bsh_at, csh_at, A.ptr, B.ptr, Cm.ptr, beta),
            "comet_hip_ttgt_contract")
     return Cm, plan
 

@@ -272,6 +272,20 @@ def test_masked_product_gathers_its_result_by_chunks(nnz):
     assert all(np.array_equal(g, w) for g, w in zip(rt.spgemm(A, B, M).to_arrays(), want))
 
 
+@pytest.mark.parametrize("shape", [0, 1, 2, 3])
+@pytest.mark.parametrize("c,n,shares", [(17, 15, 1), (19, 27, 1), (31, 33, 1), (61, 47, 1), (61, 47, 2), (61, 47, 3), (61, 47, 17),
+                                        (61, 47, 64), (61, 47, 180)])
+def test_contractions_over_irregular_k(shape, c, n, shares, monkeypatch):
+    # k in two dimensions that no sixteen divide: sixteen turns of offsets at a time, less, more, up to eleven times; shares of
+    # one turn and more, added by one thread an output and by several with steps left over
+    monkeypatch.setenv("COMET_HIP_GETT", "%d,%d" % (shape, shares))
+    rng = np.random.default_rng(c + shares)
+    A, B = rng.uniform(-1, 1, (13, c, n)), rng.uniform(-1, 1, (n, c, 21))
+    got = rt.ttgt_contract("icn", "nca", "ia", rt.DeviceArray.from_numpy(A), rt.DeviceArray.from_numpy(B))[0].to_numpy()
+    want, bound = np.einsum("icn,nca->ia", A, B), np.einsum("icn,nca->ia", np.abs(A), np.abs(B))
+    assert np.all(np.abs(got - want) <= 2 * c * n * 2.0 ** -53 * bound)          # two sums of c * n products in any order
+
+
 @pytest.mark.parametrize("accumulate", [False, True])
 @pytest.mark.parametrize("K", [1, 2, 3, 5, 21, 22, 33, 63, 64, 65, 130])
 @pytest.mark.parametrize("nrows", [1, 40, 4000, 14_000])
