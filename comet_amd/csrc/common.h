@@ -128,7 +128,7 @@ struct PairSidePlan {
     int64_t first = 0, pairs = 0, nheavy = 0, nlight = 0;
     int64_t *kpos = nullptr, *counts = nullptr;
     uint32_t *place = nullptr;
-    void *ent = nullptr, *heavy = nullptr;
+    void *ent = nullptr, *heavy = nullptr, *ranged = nullptr;
     double *weight = nullptr, *padded = nullptr;
     int32_t *light = nullptr;
 };

@@ -152,9 +152,14 @@ __device__ __forceinline__ void dot_walk(DotLists &lists, const PairSide &s, uin
 }
 
 // ---------------------------------------------------------------------------
-// Rows of long tables: a workgroup per part of a row.  Large graphs are bound by the lists' way from the memory-side cache
-// (200003 vertices, edge factor 16: 23.5 GB past the L2s in 3.2 ms, 7.3 TB/s, and 1.1 GB for the short rows beside it; a part
-// of the lists for every XCD found more of them in its L2 but built eight times the tables: 4.0 ms instead of 3.3), smaller ones, whose lists the L2 holds, by the vector
+// Rows of long tables: a workgroup per part of a row.  Large graphs are bound by the lists' way from the memory-side cache:
+// 200003 vertices, edge factor 16, 23.5 GB past the L2s in 3.2 ms, 7.3 TB/s, while parts took every so many'th list of a row.
+// A part has the lists of a stretch of memory now (pair_ranges), and the parts are taken in the order of their stretches, an
+// eighth of them by every XCD, so that its workgroups read about the same lists at about the same time: 36 % of the lines are
+// in the L2 where 13 % were, 17.8 GB in 2.67 ms, the vector unit busy in three quarters of it.  Whole product, us, every
+// so many'th list / by stretches: 200003 and 16 3505 / 2930, 260000 and 14 3085 / 2650, 120000 and 16 1565 / 1250, 90000 and 16
+// 1295 / 1020, 260000 and 5 757 / 712, 60000 and 12 467 / 455.  (Without the order, a part of the lists for every XCD: eight
+// times the tables, 4.0 ms.)  Smaller ones, whose lists the L2 holds, by the vector
 // unit, busy two thirds of the time.  The first item of a workgroup is its own, not drawn: with one word to draw from, the
 // last of 256 began 3 us after the first.  Whole product: n = 200003 21.7 -> 3.6 ms, 20351 0.70 -> 0.24.  With values
 // read from LDS rather than by flat loads, sums over the lanes of a list by scalar masks, and two workgroups to a CU, us:
@@ -246,7 +251,7 @@ static_assert(dot_table_words(1 << 20) * sizeof(uint32_t) + sizeof(DotHeavyShare
 // rows, two / one: 100000 vertices, edge factor 8 394 / 433, 60000 and 16 524 / 555, 30000 and 8 110 / 128, 16000 and 16
 // 128 / 150; 140000 and 10 1233 / 1088, 200003 and 16 3922 / 3192; few items: 8000 and 6 34 / 29, 5000 and 12 45 / 43.
 constexpr int DOT_TWO_T = 512;
-constexpr int64_t DOT_TWO_COLS = 1 << 17;
+constexpr int64_t DOT_TWO_COLS = PAIR_RANGED_COLS;
 constexpr size_t DOT_TWO_LDS_MOST = 80 * 1024 - 256;
 static_assert(dot_table_words(DOT_TWO_COLS) * sizeof(uint32_t) + sizeof(DotHeavyShared<DOT_TWO_T>) <= DOT_TWO_LDS_MOST / 2,
               "half of a workgroup's LDS is left for values");
@@ -255,7 +260,7 @@ static_assert(dot_table_words(DOT_TWO_COLS) * sizeof(uint32_t) + sizeof(DotHeavy
 // nvals: values of a row that fit LDS behind the shared part
 template <int T, bool BIG, bool SEMI>
 __global__ __launch_bounds__(T, 4) void pair_dot_heavy_kernel(PairSide s0, PairSide s1, int table_words, int before_at, int nvals,
-                                                              unsigned long long *__restrict__ tickets,
+                                                              unsigned queues, unsigned long long *__restrict__ tickets,
                                                               double *__restrict__ pair_val,
                                                               uint8_t *__restrict__ pair_hit, DotSemiring op)
 {
@@ -271,8 +276,24 @@ __global__ __launch_bounds__(T, 4) void pair_dot_heavy_kernel(PairSide s0, PairS
         sg_dyn_lds[w] = 0;
     __syncthreads();
     const uint32_t n0 = (uint32_t)(s0.counts[0] & 0xffffffff), n1 = (uint32_t)(s1.counts[0] & 0xffffffff);
-    if (threadIdx.x == 0)
-        sh.slot[0] = pair_item(s0, s1, n0, n1, blockIdx.x);
+    // the items in eighths, one to an XCD, whose workgroups draw from the others' when theirs are gone
+    const unsigned long long items = (unsigned long long)n0 + n1;
+    unsigned queue = blockIdx.x % queues;
+    const auto begin = [&](unsigned q) { return items * q / queues; };
+    const auto draw = [&]() -> PairItem {
+        for (unsigned tries = 0; tries < queues; ++tries) {
+            const unsigned long long own = (gridDim.x + queues - 1u - queue) / queues;
+            const unsigned long long at = begin(queue) + own + atomicAdd(&tickets[queue], 1ull);
+            if (at < begin(queue + 1))
+                return pair_item<true>(s0, s1, n0, n1, at);
+            queue = (queue + 1u) % queues;
+        }
+        return pair_item<true>(s0, s1, n0, n1, items);
+    };
+    if (threadIdx.x == 0) {
+        const unsigned long long at = begin(queue) + blockIdx.x / queues;
+        sh.slot[0] = at < begin(queue + 1) ? pair_item<true>(s0, s1, n0, n1, at) : draw();
+    }
     __syncthreads();
     PairItem it = pair_item_read(sh.slot[0]);
     int cur = 0;
@@ -298,7 +319,7 @@ __global__ __launch_bounds__(T, 4) void pair_dot_heavy_kernel(PairSide s0, PairS
             sh.batch_next = T / 64;
         lds_barrier();
         if (threadIdx.x == 0)
-            sh.slot[cur ^ 1] = pair_item(s0, s1, n0, n1, gridDim.x + atomicAdd(&tickets[0], 1ull));
+            sh.slot[cur ^ 1] = draw();
         const int mine = (it.kn + it.parts - 1) / it.parts;          // pairs of a part, about
         int B = mine / (4 * (T / 64));
         B = B > 64 ? 64 : B < 4 ? 4 : B;          // four lists fill a turn or two
@@ -337,7 +358,8 @@ __global__ __launch_bounds__(T, 4) void pair_dot_heavy_kernel(PairSide s0, PairS
             }
         };
         const uint32_t vals_at = (uint32_t)sizeof(uint32_t) * (uint32_t)table_words + (uint32_t)sizeof sh;
-        if (in_lds)
+        if (it.kn == 0) {          // no list of the row begins there
+        } else if (in_lds)
             walk(RankProbe<BIG, true>{before, vals_at, nullptr});
         else
             walk(RankProbe<BIG, false>{before, 0, s.Tval + it.ts});
@@ -588,11 +610,12 @@ static int pair_dot_values(Csr *a, Csr *b, Csr *m, int64_t rb, int64_t re, doubl
         const int nvals = (int)(((two ? DOT_TWO_LDS_MOST : DOT_LDS_MOST) - fixed) / sizeof(double)) & ~1;
         const size_t lds = fixed + sizeof(double) * (size_t)nvals;
         const dim3 grid((unsigned)std::min<int64_t>(nheavy, (int64_t)num_cus() * (two ? 2 : 1))), block(two ? DOT_TWO_T : SG_T);
+        const unsigned queues = s0.ranged || s1.ranged ? 8 : 1;
         KernelTimer t("spgemm_numeric_dot");
 #define LAUNCH_DOT(T, BIG, SEMI)                                                                                       \
     do {                                                                                                               \
         COMET_CHK(sg_allow_lds(pair_dot_heavy_kernel<T, BIG, SEMI>, lds));                                             \
-        pair_dot_heavy_kernel<T, BIG, SEMI><<<grid, block, lds, stream()>>>(s0, s1, words, before_at, nvals, tickets,  \
+        pair_dot_heavy_kernel<T, BIG, SEMI><<<grid, block, lds, stream()>>>(s0, s1, words, before_at, nvals, queues, tickets,  \
                                                                             *pair_val, *pair_hit, op);                 \
     } while (0)
         if (two && semi)
@@ -608,7 +631,7 @@ static int pair_dot_values(Csr *a, Csr *b, Csr *m, int64_t rb, int64_t re, doubl
         else
             LAUNCH_DOT(SG_T, false, false);
 #undef LAUNCH_DOT
-        COMET_HIPCHK(hipMemsetAsync(tickets, 0, sizeof *tickets, stream()));
+        COMET_HIPCHK(hipMemsetAsync(tickets, 0, 8 * sizeof *tickets, stream()));
     }
     if (nlight > 0) {
         const dim3 grid((unsigned)std::min<int64_t>(ceil_div(nlight, DOT_LIGHT_WAVES), (int64_t)num_cus() * DOT_LIGHT_OCC)),

@@ -33,6 +33,7 @@ struct PairSide {
     const double *Lval;
     uint32_t Lnnz;               // at least 4: a lane reads four columns at a time
     const uint2 *heavy;          // rows a workgroup takes, in parts: row, part | parts << 16
+    const uint4 *ranged;         // product: the same as row and pairs [y, z) of the row; or null
     const int32_t *light;        // rows a wavefront takes
     const int64_t *counts;       // [0]: entries of heavy | entries of light << 32
 };
@@ -42,7 +43,16 @@ constexpr int PAIR_LIGHT_LOG = 8;                 // log2 of the buckets of four
 constexpr int PAIR_LIGHT_MAX = (1 << PAIR_LIGHT_LOG) * 3 / 4;        // three quarters of a column per bucket
 constexpr int PAIR_LIGHT_WORK = 8192;               // and of at most this many look-ups
 constexpr int PAIR_LIST_COST = 8;                                    // what taking a list up costs, in look-ups
-constexpr int PAIR_ITEM_MIN = 16384;                                 // look-ups a part of a row is worth at least
+constexpr int64_t PAIR_ITEM_MIN = 16384;                             // look-ups a part of a row is worth at least
+constexpr int64_t PAIR_SHARES = 2048;                                // parts that all the work would make, at most
+// Products whose lists, columns and values, take more than this: parts by stretches of the lists.  Smaller lists are in the
+// L2s by themselves (30000 vertices, edge factor 16, 10 MB 316 us, by stretches 344; 60000 and 12, 17 MB 467 / 455).  A part is
+// worth 200,000 look-ups then, 140,000 where two workgroups share a CU (up to PAIR_RANGED_COLS columns) - a table is built
+// and cleared for it -, us at 60,000 / 100,000 / 140,000 / 200,000: 160000 and 8 1091 / 1023 / 976 / 947, 260000 and 8 1309 / 1279
+// / 1219 / 1184, 90000 and 16 1080 / 1063 / 1022 / 1041; and a 4096th of all at least (2048th, 8192th: 200003 and 16 3046,
+// 3177 against 2935).
+constexpr int64_t PAIR_RANGED_LISTS = 14 << 20, PAIR_RANGED_COLS = 1 << 17, PAIR_RANGED_TWO = 140000, PAIR_RANGED_ONE = 200000;
+constexpr int64_t PAIR_RANGED_SHARES = 4096;
 
 // strict 0: lists not longer than the table's row, 1: shorter ones, 2: all of them (no second side)
 __device__ __forceinline__ bool pair_kept(int strict, int64_t len, int64_t tlen)
@@ -240,7 +250,7 @@ __global__ __launch_bounds__(256) void pair_turn(int64_t nrows, const int64_t *_
 // look-ups whatever a part of a heavy one has.
 __global__ void pair_parts(int64_t first, int64_t n, const int64_t *__restrict__ Tpos, const int64_t *__restrict__ kpos,
                            const int64_t *__restrict__ wpos, int only, int light_max, int64_t light_work,
-                           int64_t *__restrict__ packed)
+                           int64_t shares, int64_t item_min, int64_t *__restrict__ packed)
 {
     const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (x >= n)
@@ -248,7 +258,7 @@ __global__ void pair_parts(int64_t first, int64_t n, const int64_t *__restrict__
     const int64_t kept = kpos[x + 1] - kpos[x], tlen = Tpos[first + x + 1] - Tpos[first + x];
     const int64_t work = wpos[x + 1] - wpos[x];
     int64_t v = 0;
-    const int64_t share = wpos[n] / 2048, target = share > PAIR_ITEM_MIN ? share : PAIR_ITEM_MIN;
+    const int64_t share = wpos[n] / shares, target = share > item_min ? share : item_min;
     // a short table may be paired with a hundred thousand lists: no wavefront gets more than a fraction of a part
     const int64_t fraction = target / 8 < PAIR_LIGHT_WORK ? target / 8 : PAIR_LIGHT_WORK;
     const int64_t most_light = fraction > light_work ? fraction : light_work;
@@ -279,6 +289,48 @@ __global__ void pair_items(int64_t first, int64_t n, const int64_t *__restrict__
         for (int64_t q = 0; q < v; ++q)
             heavy[(o & 0xffffffff) + q] = make_uint2((unsigned)(first + x), (unsigned)q | (unsigned)(v << 16));
     }
+}
+
+// The parts of heavy rows cut where their lists lie: part q of v has the pairs whose lists begin in the q-th v-th of the lists'
+// entries.  keys: the middle of that, in 2^20ths; a row in one part goes anywhere.
+__global__ void pair_ranges(int64_t first, int64_t n, const int64_t *__restrict__ packed, const int64_t *__restrict__ off,
+                            const int64_t *__restrict__ kpos, const PairEnt *__restrict__ ent, uint32_t Lnnz,
+                            uint4 *__restrict__ ranged, uint64_t *__restrict__ keys, uint32_t *__restrict__ idx)
+{
+    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (x >= n)
+        return;
+    const int64_t v = packed[x], ks = kpos[x], kn = kpos[x + 1] - ks;
+    if (v >> 32)
+        return;
+    int64_t from = 0;
+    for (int64_t q = 0; q < v; ++q) {
+        int64_t to = kn;
+        if (q + 1 < v) {          // first pair whose list begins at the bound or behind it
+            const uint32_t bound = (uint32_t)((uint64_t)Lnnz * (uint64_t)(q + 1) / (uint64_t)v);
+            int64_t lo = from;
+            while (lo < to) {
+                const int64_t mid = (lo + to) >> 1;
+                if (ent[ks + mid].start < bound)
+                    lo = mid + 1;
+                else
+                    to = mid;
+            }
+        }
+        const int64_t at = (off[x] & 0xffffffff) + q;
+        ranged[at] = make_uint4((unsigned)(first + x), (unsigned)from, (unsigned)to, 0);
+        keys[at] = v > 1 ? (uint64_t)((2 * q + 1) * (1ll << 19) / v) : (uint64_t)((uint32_t)x * 0x9E3779B1u >> 12);
+        idx[at] = (uint32_t)at;
+        from = to;
+    }
+}
+
+__global__ void pair_ranges_sorted(int64_t n, const uint4 *__restrict__ ranged, const uint32_t *__restrict__ idx,
+                                   uint4 *__restrict__ sorted)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n)
+        sorted[i] = ranged[idx[i]];
 }
 
 // ---------------------------------------------------------------------------
@@ -436,6 +488,8 @@ struct PairItem {
     int64_t ts, ks;
     int tlen, kn, part, parts, side, index;          // index < 0: nothing left
 };
+// RANGED: the sides may have their parts by stretches of the lists
+template <bool RANGED>
 __device__ __forceinline__ PairItem pair_item(const PairSide &s0, const PairSide &s1, uint32_t n0, uint32_t n1,
                                               unsigned long long tk)
 {
@@ -444,15 +498,28 @@ __device__ __forceinline__ PairItem pair_item(const PairSide &s0, const PairSide
     if (tk < (unsigned long long)n0 + n1) {
         const bool one = tk >= n0;
         const int64_t *Tpos = one ? s1.Tpos : s0.Tpos, *kpos = one ? s1.kpos : s0.kpos;
-        const uint2 h = (one ? s1.heavy : s0.heavy)[one ? tk - n0 : tk];
+        const unsigned long long at = one ? tk - n0 : tk;
+        const uint4 *ranged = !RANGED ? nullptr : one ? s1.ranged : s0.ranged;
         it.side = one;
         it.index = (int)tk;
-        it.part = (int)(h.y & 0xffffu);
-        it.parts = (int)(h.y >> 16);
-        it.ts = Tpos[h.x];
-        it.tlen = (int)(Tpos[h.x + 1] - it.ts);
-        it.ks = kpos[h.x];
-        it.kn = (int)(kpos[h.x + 1] - it.ks);
+        uint32_t x;
+        if (ranged) {
+            const uint4 h = ranged[at];
+            x = h.x;
+            it.part = 0;
+            it.parts = 1;
+            it.ks = kpos[x] + h.y;
+            it.kn = (int)(h.z - h.y);
+        } else {
+            const uint2 h = (one ? s1.heavy : s0.heavy)[at];
+            x = h.x;
+            it.part = (int)(h.y & 0xffffu);
+            it.parts = (int)(h.y >> 16);
+            it.ks = kpos[x];
+            it.kn = (int)(kpos[x + 1] - it.ks);
+        }
+        it.ts = Tpos[x];
+        it.tlen = (int)(Tpos[x + 1] - it.ts);
     }
     return it;
 }
@@ -519,7 +586,7 @@ __global__ __launch_bounds__(SG_T) void pair_sum_heavy_kernel(PairSide s0, PairS
     __syncthreads();
     const uint32_t n0 = (uint32_t)(s0.counts[0] & 0xffffffff), n1 = (uint32_t)(s1.counts[0] & 0xffffffff);
     if (threadIdx.x == 0)
-        sh.slot[0] = pair_item(s0, s1, n0, n1, blockIdx.x);
+        sh.slot[0] = pair_item<false>(s0, s1, n0, n1, blockIdx.x);
     __syncthreads();
     PairItem it = pair_item_read(sh.slot[0]);
     int cur = 0;
@@ -536,7 +603,7 @@ __global__ __launch_bounds__(SG_T) void pair_sum_heavy_kernel(PairSide s0, PairS
             sh.batch_next = SG_WAVES;
         lds_barrier();
         if (threadIdx.x == 0)
-            sh.slot[cur ^ 1] = pair_item(s0, s1, n0, n1, gridDim.x + atomicAdd(&tickets[0], 1ull));
+            sh.slot[cur ^ 1] = pair_item<false>(s0, s1, n0, n1, gridDim.x + atomicAdd(&tickets[0], 1ull));
         // batches of 64 pairs, or fewer where that leaves the wavefronts less than four each
         const int mine = (it.kn + it.parts - 1) / it.parts;          // pairs of a part, about
         int B = mine / (4 * SG_WAVES);
@@ -816,7 +883,7 @@ __global__ __launch_bounds__(PAIR_HITS_T) void pair_hits_finish(unsigned long lo
 // ---------------------------------------------------------------------------
 // Plans
 // ---------------------------------------------------------------------------
-static Workspace g_pair_chunk, g_pair_row, g_pair_turn, g_pair_tickets, g_pair_out, g_pair_partial, g_pair_hits;
+static Workspace g_pair_range, g_pair_chunk, g_pair_row, g_pair_turn, g_pair_tickets, g_pair_out, g_pair_partial, g_pair_hits;
 
 // pos[first] and pos[last] of x
 static int pair_ends(const Csr *x, int64_t first, int64_t last, int64_t *word, int64_t *ends)
@@ -897,7 +964,10 @@ static int pair_side_plan(const Csr *T, const Csr *P, const Csr *L, int64_t firs
     pair_pass<true><<<grid, block, 0, stream()>>>(first, last, T->pos, P->pos, P->crd, L->pos, strict, xlo, xhi, kept_before,
                                                   work_before, plan->kpos, wpos, (PairEnt *)plan->ent, P->val, scale,
                                                   plan->weight, perm, out0, plan->place);
-    pair_parts<<<rows, block, 0, stream()>>>(first, n, T->pos, plan->kpos, wpos, only, light_max, 0, parts);
+    const bool ranged = places && L->nnz * (int64_t)(sizeof(int32_t) + sizeof(double)) > PAIR_RANGED_LISTS;
+    const int64_t item_min = !ranged ? PAIR_ITEM_MIN : T->ncols <= PAIR_RANGED_COLS ? PAIR_RANGED_TWO : PAIR_RANGED_ONE;
+    pair_parts<<<rows, block, 0, stream()>>>(first, n, T->pos, plan->kpos, wpos, only, light_max, 0,
+                                             ranged ? PAIR_RANGED_SHARES : PAIR_SHARES, item_min, parts);
     COMET_CHK(exclusive_scan_i64(parts, n, wpos));
     COMET_HIPCHK(hipMemcpyAsync(word, wpos + n, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
     COMET_CHK(stream_wait());
@@ -907,6 +977,19 @@ static int pair_side_plan(const Csr *T, const Csr *P, const Csr *L, int64_t firs
     COMET_HIPCHK(dev_malloc((void **)&plan->heavy, sizeof(uint2) * (size_t)(plan->nheavy > 0 ? plan->nheavy : 1)));
     COMET_HIPCHK(dev_malloc((void **)&plan->light, sizeof(int32_t) * (size_t)(plan->nlight > 0 ? plan->nlight : 1)));
     pair_items<<<rows, block, 0, stream()>>>(first, n, parts, wpos, (uint2 *)plan->heavy, plan->light, plan->counts);
+    if (ranged && plan->nheavy > 0) {
+        const size_t items = (size_t)plan->nheavy;
+        COMET_HIPCHK(dev_malloc((void **)&plan->ranged, sizeof(uint4) * items));
+        COMET_CHK(g_pair_range.ensure((sizeof(uint4) + 2 * sizeof(uint64_t) + 2 * sizeof(uint32_t)) * items, false));
+        uint4 *list = (uint4 *)g_pair_range.ptr;
+        uint64_t *keys = (uint64_t *)(list + items);
+        uint32_t *idx = (uint32_t *)(keys + 2 * items);
+        pair_ranges<<<rows, block, 0, stream()>>>(first, n, parts, wpos, plan->kpos, (const PairEnt *)plan->ent, (uint32_t)L->nnz, list,
+                                                  keys, idx);
+        COMET_CHK(sort_pairs_u64_u32(keys, keys + items, idx, idx + items, plan->nheavy, 20));
+        pair_ranges_sorted<<<dim3((unsigned)ceil_div(plan->nheavy, 256)), block, 0, stream()>>>(plan->nheavy, list, idx + items,
+                                                                                               (uint4 *)plan->ranged);
+    }
     if (L->nnz < 4) {          // a lane reads four columns at a time
         constexpr size_t room = 4 * (sizeof(double) + sizeof(int32_t));
         COMET_HIPCHK(dev_malloc((void **)&plan->padded, room));
@@ -933,6 +1016,7 @@ static PairSide pair_side(const PairSidePlan &p, const Csr *T, const Csr *L)
     s.Lval = p.padded ? p.padded : L->val;
     s.Lnnz = p.padded ? 4u : (uint32_t)L->nnz;
     s.heavy = (const uint2 *)p.heavy;
+    s.ranged = (const uint4 *)p.ranged;
     s.light = p.light;
     s.counts = p.counts;
     return s;

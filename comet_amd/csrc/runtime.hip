@@ -375,7 +375,7 @@ uint64_t next_csr_uid()
 
 static void pair_side_free(PairSidePlan &s)
 {
-    for (void *q : {(void *)s.kpos, (void *)s.place, (void *)s.counts, s.ent, s.heavy, (void *)s.weight,
+    for (void *q : {(void *)s.kpos, (void *)s.place, (void *)s.counts, s.ent, s.heavy, s.ranged, (void *)s.weight,
                     (void *)s.light, (void *)s.padded})
         (void)dev_free(q);
     s = PairSidePlan();

@@ -433,7 +433,7 @@ __global__ __launch_bounds__(SG_T) void tri_heavy_kernel(PairSide s, int nwords,
     __syncthreads();
     const uint32_t n = (uint32_t)(s.counts[0] & 0xffffffff);
     if (threadIdx.x == 0)
-        sh.slot[0] = pair_item(s, s, n, 0, blockIdx.x);
+        sh.slot[0] = pair_item<false>(s, s, n, 0, blockIdx.x);
     __syncthreads();
     PairItem it = pair_item_read(sh.slot[0]);
     int cur = 0;
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(SG_T) void tri_heavy_kernel(PairSide s, int nwords,
             sh.batch_next = SG_WAVES;
         lds_barrier();
         if (threadIdx.x == 0)
-            sh.slot[cur ^ 1] = pair_item(s, s, n, 0, gridDim.x + atomicAdd(&tickets[0], 1ull));
+            sh.slot[cur ^ 1] = pair_item<false>(s, s, n, 0, gridDim.x + atomicAdd(&tickets[0], 1ull));
         const int mine = (it.kn + it.parts - 1) / it.parts;          // pairs of a part, about
         int B = mine / (4 * SG_WAVES);
         B = B > 64 ? 64 : B < 2 ? 2 : B;
@@ -708,7 +708,8 @@ static int tri_plan(Csr *a, int only)
         }
         COMET_CHK(exclusive_scan_i64(work, nnz, w0));
         tri_row_work<<<per_row, block, 0, stream()>>>(n, side.kpos, w0, r0);
-        pair_parts<<<per_row, block, 0, stream()>>>(0, n, plan.tpos, side.kpos, r0, only, PAIR_LIGHT_MAX, TRI_LIGHT_WORK, r1);
+        pair_parts<<<per_row, block, 0, stream()>>>(0, n, plan.tpos, side.kpos, r0, only, PAIR_LIGHT_MAX, TRI_LIGHT_WORK, PAIR_SHARES,
+                                                    PAIR_ITEM_MIN, r1);
         COMET_CHK(exclusive_scan_i64(r1, n, r0, word));
         COMET_CHK(stream_wait());
         const int64_t packed = *(volatile int64_t *)word;

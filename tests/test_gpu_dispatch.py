@@ -257,6 +257,32 @@ def test_masked_product_of_every_list_and_table_length(k, semiring):
             assert np.all(np.abs(v - wv) <= 1e-12 * bound)
 
 
+@pytest.mark.parametrize("semiring", [None, ("min", "plus")])
+def test_masked_product_by_stretches_of_its_lists(semiring):
+    # lists of more than 14 MiB; long rows in several parts, some of which have no list; short rows beside them
+    n = 16_000
+    rng = np.random.default_rng(5)
+    lens = np.full(n, 82)
+    lens[[0, 77, 8000, 15_999]] = 8000, 15_000, 3000, 9000
+
+    def matrix(columns):
+        crd = np.concatenate([np.sort(rng.permutation(columns[i])[:l]) if l > 82 else np.unique(rng.integers(0, n, l))
+                              for i, l in enumerate(lens)])
+        pos = np.concatenate([[0], np.cumsum([len(r) for r in np.split(crd, np.flatnonzero(np.diff(crd) < 0) + 1)])])
+        return pos.astype(np.int64), crd.astype(np.int32), rng.uniform(1, 2, len(crd))
+
+    low = {i: n for i in range(n)}
+    low[8000] = 3500                       # all of its columns are in front: the last parts of the row are empty
+    a, b, m = matrix(low), matrix(low), matrix(low)
+    assert all(len(x[1]) * 12 > 14 << 20 and len(x[0]) == n + 1 for x in (a, b, m))
+    A, B, M = (rt.CsrMatrix.from_arrays((n, n), *x) for x in (a, b, m))
+    want = orc.spgemm(*a, *b, n, mask=m[:2], **({"semiring": semiring} if semiring else {}))
+    for _ in range(2):
+        p, c, v = rt.spgemm(A, B, M, semiring=semiring).to_arrays()
+        assert np.array_equal(p, want[0]) and np.array_equal(c, want[1])
+        assert np.array_equal(v, want[2]) if semiring else np.all(np.abs(v - want[2]) <= 1e-12 * np.abs(want[2]))
+
+
 @pytest.mark.parametrize("nnz", [1, 2047, 2048, 2049, 6144])
 def test_masked_product_gathers_its_result_by_chunks(nnz):
     # a diagonal A keeps every second row's mask entries; rows of one entry, empty rows, a row longer than a chunk
