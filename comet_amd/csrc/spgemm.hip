@@ -389,15 +389,18 @@ struct RowList {
     bool none_small() const { return counts[1] >= 0 && counts[1] == counts[3]; }
     bool none_mid() const { return counts[0] >= 0 && counts[0] == counts[3]; }
 };
+// Which of a list's rows a kernel takes: from one of the bounds (-1: the list's begin) to another.  A number of both, so
+// that a kernel reads two words in place of a chain of branches (values of 60000 rows of 20 entries, us: 316, now 296).
+constexpr int list_part(int first, int end) { return (first + 1) | end << 4; }
+constexpr int LIST_LIGHT = list_part(0, 1), LIST_ALL = list_part(-1, 1);
+constexpr int LIST_WIDEST = list_part(-1, 2), LIST_SPAN = list_part(2, 0);                // the heavy rows
+constexpr int LIST_MID = list_part(0, 3), LIST_SMALL = list_part(3, 1);                   // the light ones
+constexpr int LIST_SMALL_MORE = list_part(3, 4), LIST_FEW = list_part(4, 1);              // the small ones
+constexpr int LIST_NOT_FEW = list_part(-1, 4);
 __device__ inline void list_range(const RowList &l, int part, int64_t *first, int64_t *end)
 {
-    // part 0: the heavy rows, 1: the others that have products, 2: both, 3: the widest of the heavy rows,
-    // 4: the heavy rows that are not among the widest, 5: the small rows, 6: those between the small and the heavy ones,
-    // 7: all but the small ones, 8: the small rows without, 9: those with the fewest products
-    *first = part == 1 || part == 6 ? l.bounds[0] : part == 4 ? l.bounds[2] : part == 5 || part == 8 ? l.bounds[3]
-             : part == 9 ? l.bounds[4] : 0;
-    *end = part == 0 || part == 4 ? l.bounds[0] : part == 3 ? l.bounds[2] : part == 6 || part == 7 ? l.bounds[3]
-           : part == 8 ? l.bounds[4] : l.bounds[1];
+    *first = (part & 15) ? l.bounds[(part & 15) - 1] : 0;
+    *end = l.bounds[part >> 4];
 }
 // A workgroup barrier that orders LDS traffic only.  __syncthreads() also makes every wavefront wait until its
 // global stores have been acknowledged, a microsecond that a kernel whose stores nobody reads back (the rows
@@ -1457,7 +1460,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_kernel(
     int visit = 0;
     const int64_t out0 = Cpos[row_begin];
     int64_t t_first, t_end;
-    list_range(list, 3, &t_first, &t_end);     // the other heavy rows go to spgemm_numeric_span_kernel
+    list_range(list, LIST_WIDEST, &t_first, &t_end);     // the other heavy rows go to spgemm_numeric_span_kernel
     int64_t t = draw_row<true>(ticket, t_first, &row_slot);
     while (t < t_end) {
         const int64_t i = row_begin + list.rows[t];
@@ -2088,7 +2091,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_span_kernel(
     lds_barrier();
     const int64_t out0 = Cpos[row_begin];
     int64_t t_first, t_end;
-    list_range(list, 4, &t_first, &t_end);
+    list_range(list, LIST_SPAN, &t_first, &t_end);
     // Rows dealt out in advance: the list goes down by products, so every workgroup gets about the same, and what leads to
     // a row's slices can be fetched ahead - the bounds of 64 rows at a time, a row's first entries of A two rows ahead and
     // their slices one.
@@ -2340,7 +2343,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_masked_sum_kernel(
     }
     __syncthreads();
     int64_t t_first, t_end;
-    list_range(list, 2, &t_first, &t_end);
+    list_range(list, LIST_ALL, &t_first, &t_end);
     int64_t tk = draw_front(ticket, t_end, &row_slot);
     while (tk < t_end) {
         const int64_t i = list.rows[tk];      // rows outside the list keep the zero the host put there
@@ -2414,7 +2417,7 @@ __global__ __launch_bounds__(SM_WAVES * 64) void spgemm_masked_sum_small_kernel(
     for (int s = lane; s < SM_SLOTS; s += 64)
         tab[s] = -1;
     int64_t t_first, t_end;
-    list_range(list, 2, &t_first, &t_end);
+    list_range(list, LIST_ALL, &t_first, &t_end);
     int take = SM_BATCH;
     int64_t mine_next = 0, mine_end = 0;     // the rows t_end - 1 - b, b in [mine_next, mine_end), are this wavefront's
     for (;;) {
@@ -2712,7 +2715,7 @@ __global__ void fill_iota_f64(int64_t n, double *__restrict__ out)
 // and where there are enough of them their values have a launch of their own, with half the registers.  us, structure and
 // values, sixteen lanes to an entry / eight products a lane / so: 65536 rows of 8 uniform entries 129 + 246 / 210 + 282 / 59 +
 // 194, 60000 rows of a band of 9 125 + 230 / 199 + 260 / 63 + 181, a mesh of 22500 18 + 48 / 44 + 70 / 22 + 35, 20000 rows of
-// a band of 15 32 + 63 / 54 + 74 / 31 + 48.
+// a band of 15 32 + 63 / 54 + 74 / 31 + 48.  (Only these rows have their structure found here: SG_FEW_TOGETHER.)
 // ---------------------------------------------------------------------------
 constexpr int SM_PER = 8;                           // products of a lane
 constexpr int SM_T = 256, SM_COLS = 1 << 16;
@@ -2924,10 +2927,29 @@ struct SmallRows {
     __device__ __forceinline__ bool more() const { return t < t_end; }
 };
 
+// The row counters of a phase's kernels, one each.  0-3: a phase's own, which clears them; 4-7: the numeric phase's where the
+// symbolic one of the same call has cleared them.
+constexpr int SG_TICKETS = 8;
+// What the symbolic phase's first kernel over a row list clears for the ones behind it: those counters, and the counts of the
+// rows without products, which the list has at its end and no kernel takes.
+__device__ __forceinline__ void sg_clear_rest(const RowList &list, int64_t nrows, unsigned long long *__restrict__ tickets,
+                                              int64_t *__restrict__ rowcount)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < SG_TICKETS)
+        tickets[i] = 0;
+    for (int64_t t = list.bounds[1] + i; t < nrows; t += (int64_t)gridDim.x * blockDim.x)
+        rowcount[list.rows[t]] = 0;
+}
+
+// tickets: null, or what it clears first (sg_clear_rest)
 __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
     int64_t row_begin, RowList list, int words, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
-    const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd, int64_t *__restrict__ rowcount)
+    const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd, int64_t nrows, unsigned long long *__restrict__ tickets,
+    int64_t *__restrict__ rowcount)
 {
+    if (tickets)
+        sg_clear_rest(list, nrows, tickets, rowcount);
     uint32_t *bm = sg_dyn_lds;
     __shared__ SmallStage<SM_T> stage;
     __shared__ int wave_tot[SM_T / 64];
@@ -2937,7 +2959,7 @@ __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
     if ((threadIdx.x & 63) < 2)
         stage.own_marks[threadIdx.x >> 6][threadIdx.x & 63] = 0;
     lds_barrier();
-    SmallRows rows(list, 5, Apos, row_begin);
+    SmallRows rows(list, LIST_FEW, Apos, row_begin);
     while (rows.more()) {
         const int64_t r = rows.r, as = rows.as, ae = rows.ae;
         rows.t += gridDim.x;
@@ -2975,12 +2997,10 @@ __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
             for (int64_t p0 = as; p0 < ae; p0 += SM_T) {
                 if (p0 > as)
                     e = small_entry<false>(as, p0 + threadIdx.x, ae, Acrd, nullptr, Bpos);
-                SmallProducts<false, SM_PER> it;
-                small_products<false, SM_T, SM_PER>(stage, small_stage<false, SM_T>(stage, e), Bcrd, nullptr, it);
-#pragma unroll
-                for (int x = 0; x < SM_PER; ++x)
-                    if (it.col[x] >= 0)
-                        atomicOr(&bm[it.col[x] >> 5], 1u << (it.col[x] & 31));
+                SmallProducts<false, 1> it;
+                small_products<false, SM_T, 1>(stage, small_stage<false, SM_T>(stage, e), Bcrd, nullptr, it);
+                if (it.col[0] >= 0)
+                    atomicOr(&bm[it.col[0] >> 5], 1u << (it.col[0] & 31));
                 lds_barrier();
                 small_clear(stage);
             }
@@ -2995,7 +3015,7 @@ __global__ __launch_bounds__(SM_T) void spgemm_symbolic_small_kernel(
     }
 }
 
-// The structure of the other rows of such a matrix: eight wavefronts to a row, its rows of B streamed as staged slices, and
+// The structure of the other rows of such a matrix, of more than a product a lane there: eight wavefronts to a row, its rows of B streamed as staged slices, and
 // as many workgroups as make 32 wavefronts a CU.  (Sixteen wavefronts, all that a
 // CU then held, a row of B at a time took, us, A*A of 65536 vertices, edge factor 16 971, 30000 and 10 240, 16000 and 8 86,
 // 5000 and 12 48, so 739, 168, 66, 38.)
@@ -3040,14 +3060,17 @@ __global__ __launch_bounds__(256) void spgemm_hub_bits(const int64_t *__restrict
     }
 }
 
-// HUBS: with such bitmaps (hub_slot, hub_bits; else null)
+// HUBS: with such bitmaps (hub_slot, hub_bits; else null).  part: the list's rows that are taken; tickets: null, or what it
+// clears first (sg_clear_rest)
 template <bool HUBS>
 __global__ __launch_bounds__(SMID_T, 8) void spgemm_symbolic_rows_kernel(
-    int64_t row_begin, RowList list, int words, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
+    int64_t row_begin, RowList list, int part, int words, const int64_t *__restrict__ Apos, const int32_t *__restrict__ Acrd,
     const int64_t *__restrict__ Bpos, const int32_t *__restrict__ Bcrd, int64_t Bnnz, const int32_t *__restrict__ hub_slot,
-    const uint4 *__restrict__ hub_bits, int64_t *__restrict__ rowcount)
+    const uint4 *__restrict__ hub_bits, int64_t nrows, unsigned long long *__restrict__ tickets, int64_t *__restrict__ rowcount)
 {
     uint32_t *bm = sg_dyn_lds;
+    if (tickets)
+        sg_clear_rest(list, nrows, tickets, rowcount);
     __shared__ RowStage st;
     __shared__ int wave_cnt[SMID_WAVES], hub[HUBS ? SMID_T : 1], hubs[2];
     const bool mine = (int)threadIdx.x < words / 4;          // four words of a bitmap
@@ -3062,7 +3085,7 @@ __global__ __launch_bounds__(SMID_T, 8) void spgemm_symbolic_rows_kernel(
         st.marks[wave][lane] = 0;
     lds_barrier();          // the first pass counts its hubs before its own
     int64_t t_first, t_end;
-    list_range(list, 7, &t_first, &t_end);
+    list_range(list, part, &t_first, &t_end);
     // rows dealt out in advance, heaviest first; the bounds of 64 at a time, entries of A and their rows of B ahead
     for (int64_t t0 = t_first + blockIdx.x; t0 < t_end; t0 += 64 * (int64_t)gridDim.x) {
         const int64_t t = t0 + lane * (int64_t)gridDim.x;
@@ -3304,9 +3327,6 @@ static int sg_allow_lds(K kernel, size_t bytes)
     return COMET_HIP_OK;
 }
 
-// the row counters of a phase's kernels, one each
-// 0-3: a phase's own, which clears them; 4-7: the numeric phase's where the symbolic one of the same call has cleared them
-constexpr int SG_TICKETS = 8;
 __global__ __launch_bounds__(256) void sg_clear(unsigned long long *__restrict__ tickets, int64_t *__restrict__ rowcount, int64_t n)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -3568,6 +3588,13 @@ static int sg_plan_hubs(Csr *b, int words)
     return rc;
 }
 
+// Rows of at most SM_FEW_PRODUCTS products go to a kernel of 256 lanes a row, the others to one of 512 that streams slices of
+// B; so few of the former join the latter instead, since a launch (4 us) costs more.  us, A*A, R-MAT graphs, apart / together:
+// 1024 vertices, edge factor 8 65 / 62, 4000 and 10 126 / 122, 8000 and 5 123 / 120, 65000 and 4 832 / 837 with 16384 rows;
+// 20000 rows of 8 entries and 8 hubs 179 / 191, 60000 of 4 326 / 392.  (Rows of up to 2048 products to the first: 60000 rows
+// of 20 entries 504 in place of 454, a band of 27 697 in place of 548; the counters and counts cleared by a launch of their
+// own: 2.2 more for every product.)
+constexpr int64_t SG_FEW_TOGETHER = 4096;
 static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *rowcount)
 {
     bool dots = false;
@@ -3594,30 +3621,40 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
     else
         COMET_CHK(sg_row_list(a, b, 0, a->nrows, SG_NO_DENSE, SG_NO_DENSE, &list));
     COMET_CHK(g_sg.ticket.ensure(SG_TICKETS * sizeof(unsigned long long), false));
-    const int64_t words = std::max<int64_t>(a->nrows, SG_TICKETS);
-    sg_clear<<<dim3((unsigned)ceil_div(words, 256)), dim3(256), 0, stream()>>>(sg_ticket(0), rowcount, a->nrows);
     const bool known = list.counts[0] >= 0;
-    if (small && !list.none_small()) {
+    const bool rows_fit = small && b->nnz >= 4 && b->nnz < SLICE_NNZ_MOST && a->nnz < (1ll << 30);
+    const int64_t few = known ? list.counts[1] - list.counts[4] : -1;
+    const bool together = rows_fit && known && list.counts[4] > 0 && few <= SG_FEW_TOGETHER;
+    const bool small_rows = small && !together && few != 0, other_rows = rows_fit && list.counts[4] != 0;
+    // the first of these launches clears for itself and the others
+    unsigned long long *clears = small_rows || other_rows ? sg_ticket(0) : nullptr;
+    if (!clears) {
+        const int64_t words = std::max<int64_t>(a->nrows, SG_TICKETS);
+        sg_clear<<<dim3((unsigned)ceil_div(words, 256)), dim3(256), 0, stream()>>>(sg_ticket(0), rowcount, a->nrows);
+    }
+    if (small_rows) {
         const int words = sm_words(b->ncols);
         KernelTimer t("spgemm_symbolic_small");
-        const dim3 grid = sm_grid(known ? list.counts[1] - list.counts[3] : -1, 7);
+        const dim3 grid = sm_grid(few, 7);
         spgemm_symbolic_small_kernel<<<grid, dim3(SM_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
-            0, list, words, a->pos, a->crd, b->pos, b->crd, rowcount);
+            0, list, words, a->pos, a->crd, b->pos, b->crd, a->nrows, clears, rowcount);
+        clears = nullptr;
     }
-    if (small && b->nnz >= 4 && b->nnz < SLICE_NNZ_MOST && a->nnz < (1ll << 30)) {
-        if (list.counts[3] != 0) {
+    if (rows_fit) {
+        if (other_rows) {
             const int words = sm_words(b->ncols);
             Csr *right = const_cast<Csr *>(b);           // what is kept in a handle is not part of the matrix
             (void)plan_made([&] { return sg_plan_hubs(right, words); });
             KernelTimer t("spgemm_symbolic");
             const auto kernel = b->sg_hub_bits ? spgemm_symbolic_rows_kernel<true> : spgemm_symbolic_rows_kernel<false>;
-            kernel<<<sm_grid(list.counts[3], 4), dim3(SMID_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
-                0, list, words, a->pos, a->crd, b->pos, b->crd, b->nnz, b->sg_hub_slot, (const uint4 *)b->sg_hub_bits, rowcount);
+            kernel<<<sm_grid(list.counts[together ? 1 : 4], 4), dim3(SMID_T), sizeof(uint32_t) * (size_t)words, stream()>>>(
+                0, list, together ? LIST_ALL : LIST_NOT_FEW, words, a->pos, a->crd, b->pos, b->crd, b->nnz, b->sg_hub_slot,
+                (const uint4 *)b->sg_hub_bits, a->nrows, clears, rowcount);
         }
         COMET_HIPCHK(hipGetLastError());
         return COMET_HIP_OK;
     }
-    if (small && list.counts[3] == 0) {
+    if (small && list.counts[4] == 0) {
         COMET_HIPCHK(hipGetLastError());
         return COMET_HIP_OK;
     }
@@ -3633,7 +3670,7 @@ static int symbolic_counts(const Csr *a, const Csr *b, const Csr *m, int64_t *ro
         KernelTimer t(M ? "spgemm_symbolic_masked" : "spgemm_symbolic");                                   \
         spgemm_symbolic_kernel<L, M><<<grid, block, g.lds_bytes, stream()>>>(                              \
             a->nrows, a->pos, a->crd, b->pos, b->crd, m ? m->pos : nullptr, m ? m->crd : nullptr, g.logW,  \
-            gbm, (unsigned long long *)g_sg.ticket.ptr, list, small ? 7 : 2, rowcount);                    \
+            gbm, (unsigned long long *)g_sg.ticket.ptr, list, small ? LIST_NOT_FEW : LIST_ALL, rowcount);              \
     } while (0)
     if (g.lds) {
         if (m) LAUNCH_SYM(true, true); else LAUNCH_SYM(true, false);
@@ -3866,7 +3903,7 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         spgemm_numeric_kernel<L, M, S><<<grid, block, num_lds, stream()>>>(                                \
             rb, re, b->ncols, a->pos, a->crd, a->val, b->pos, b->crd, b->val, m ? m->pos : nullptr,        \
             m ? m->crd : nullptr, g.logW, gbm, gmask, (double *)g_sg.slabs.ptr,                            \
-            tickets, list, 1, reduce_op, mult_op, Cpos, Ccrd, Cval);         \
+            tickets, list, LIST_LIGHT, reduce_op, mult_op, Cpos, Ccrd, Cval);                               \
     } while (0)
 #define LAUNCH_NUM_S(L, M)                                                                                 \
     do {                                                                                                   \
@@ -3887,15 +3924,15 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
         const int64_t few = known ? list.counts[1] - list.counts[4] : 0;
         const bool apart = few >= SM_FEW_ROWS || (few > 0 && list.counts[4] == list.counts[3]);
         if (apart)
-            COMET_CHK(launch(semi ? spgemm_numeric_small_kernel<true, SM_T, 1> : spgemm_numeric_small_kernel<false, SM_T, 1>, 9, SM_T,
-                             sizeof(SmallRowLds<SM_T, 1>), few, 7));
+            COMET_CHK(launch(semi ? spgemm_numeric_small_kernel<true, SM_T, 1> : spgemm_numeric_small_kernel<false, SM_T, 1>,
+                             LIST_FEW, SM_T, sizeof(SmallRowLds<SM_T, 1>), few, 7));
         if (!list.none_small() && !(apart && list.counts[4] == list.counts[3]))
             COMET_CHK(launch(semi ? spgemm_numeric_small_kernel<true, SM_T, SM_PER> : spgemm_numeric_small_kernel<false, SM_T, SM_PER>,
-                             apart ? 8 : 5, SM_T, sizeof(SmallRowLds<SM_T, SM_PER>),
+                             apart ? LIST_SMALL_MORE : LIST_SMALL, SM_T, sizeof(SmallRowLds<SM_T, SM_PER>),
                              list.counts[apart ? 4 : 1] - list.counts[3], 7));
         if (classes.mid < classes.dense && !list.none_mid())
             COMET_CHK(launch(semi ? spgemm_numeric_small_kernel<true, SM_MID_T, SM_PER> : spgemm_numeric_small_kernel<false, SM_MID_T, SM_PER>,
-                             6, SM_MID_T, sizeof(SmallRowLds<SM_MID_T, SM_PER>), list.counts[3] - list.counts[0], 2));
+                             LIST_MID, SM_MID_T, sizeof(SmallRowLds<SM_MID_T, SM_PER>), list.counts[3] - list.counts[0], 2));
     } else if (list.only_heavy()) {
         // nothing for these kernels
     } else if (g.lds) {

@@ -283,6 +283,33 @@ def test_masked_product_by_stretches_of_its_lists(semiring):
         assert np.array_equal(v, want[2]) if semiring else np.all(np.abs(v - want[2]) <= 1e-12 * np.abs(want[2]))
 
 
+@pytest.mark.parametrize("counted", [True, False])
+@pytest.mark.parametrize("rows,long_row,b_entries", [(60, 120, 900), (10_240, 120, 900), (10_242, 120, 900), (60, 2, 900),
+                                                     (9000, 2, 900), (60, 120, 3), (7, 0, 900)])
+def test_the_structure_of_rows_of_few_products(rows, long_row, b_entries, counted, monkeypatch):
+    # by turns rows of no entry, of two, of a hundred that mostly meet empty rows of B, of entries without a product and (of
+    # 120) of more products than a workgroup has lanes; up to 4096 rows of few products join the last kind
+    if not counted:
+        monkeypatch.setenv("COMET_HIP_SPGEMM_NO_LIST_CACHE", "1")
+    k, n = 600, 777
+    rng = np.random.default_rng(rows)
+    full = 300 if b_entries == 900 else 1          # rows of B that have entries, the others are empty
+    b = (np.minimum(np.arange(k + 1), full).astype(np.int64) * 3, np.sort(rng.random((full, n)).argsort(1)[:, :3]).ravel().astype(np.int32),
+         rng.integers(1, 9, b_entries).astype(np.float64))
+    empty = np.arange(full, k)
+    kinds = [np.zeros(0, int), np.arange(min(full, 2)), np.concatenate([np.arange(min(full, 20)), empty[:80]]), empty[:3],
+             np.arange(min(full, long_row))]
+    picked = [kinds[i % 5] for i in range(rows)] if long_row else [kinds[0]] * rows
+    pos = np.concatenate([[0], np.cumsum([len(r) for r in picked])]).astype(np.int64)
+    crd = np.concatenate(picked).astype(np.int32)
+    a = (pos, crd, rng.integers(1, 9, len(crd)).astype(np.float64))
+    want = orc.spgemm(*a, *b, n)
+    A, B = rt.CsrMatrix.from_arrays((rows, k), *a), rt.CsrMatrix.from_arrays((k, n), *b)
+    for _ in range(2):
+        for g, w in zip(rt.spgemm(A, B).to_arrays(), want):
+            assert np.array_equal(g, w)
+
+
 @pytest.mark.parametrize("nnz", [1, 2047, 2048, 2049, 6144])
 def test_masked_product_gathers_its_result_by_chunks(nnz):
     # a diagonal A keeps every second row's mask entries; rows of one entry, empty rows, a row longer than a chunk
