@@ -438,10 +438,14 @@ struct DotLightShared {
     int hit[64];
 };
 
+// tickets: null, or those of the long rows' launch in front of this one, which it clears
 template <bool SEMI>
 __global__ __launch_bounds__(DOT_LIGHT_WAVES * 64, DOT_LIGHT_OCC) void pair_dot_light_kernel(
-    PairSide s0, PairSide s1, double *__restrict__ pair_val, uint8_t *__restrict__ pair_hit, DotSemiring op)
+    PairSide s0, PairSide s1, unsigned long long *__restrict__ tickets, double *__restrict__ pair_val,
+    uint8_t *__restrict__ pair_hit, DotSemiring op)
 {
+    if (tickets && blockIdx.x == 0 && threadIdx.x < 8)
+        tickets[threadIdx.x] = 0;
     __shared__ __align__(16) DotLightShared all[DOT_LIGHT_WAVES];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     DotLightShared &sh = all[wv];
@@ -592,15 +596,16 @@ static int pair_dot_values(Csr *a, Csr *b, Csr *m, int64_t rb, int64_t re, doubl
     *pair_val = (double *)g_dot_val.ptr;
     if (plan->outs == 0)
         return COMET_HIP_OK;
-    COMET_HIPCHK(hipMemsetAsync(*pair_hit, 0, outs, stream()));          // pairs of an empty row or column are of no side
+    if (plan->side[0].pairs + plan->side[1].pairs < plan->outs)          // pairs of an empty row or column are of no side
+        COMET_HIPCHK(hipMemsetAsync(*pair_hit, 0, outs, stream()));
     const PairSide s0 = pair_side(plan->side[0], a, bt), s1 = pair_side(plan->side[1], bt, a);
     const int64_t nheavy = plan->side[0].nheavy + plan->side[1].nheavy, nlight = plan->side[0].nlight + plan->side[1].nlight;
     const DotSemiring op{reduce_op, mult_op};
     const bool beside = nheavy > 0 && nlight > 0 && plan->side[0].pairs + plan->side[1].pairs >= PAIR_BESIDE;
     if (beside)
         COMET_CHK(aux_fork());
+    unsigned long long *tickets = nullptr;
     if (nheavy > 0) {
-        unsigned long long *tickets = nullptr;
         COMET_CHK(pair_tickets(&tickets));
         const bool big = dot_table_big(a->ncols);
         const int words = dot_table_words(a->ncols);
@@ -631,7 +636,10 @@ static int pair_dot_values(Csr *a, Csr *b, Csr *m, int64_t rb, int64_t re, doubl
         else
             LAUNCH_DOT(SG_T, false, false);
 #undef LAUNCH_DOT
-        COMET_HIPCHK(hipMemsetAsync(tickets, 0, 8 * sizeof *tickets, stream()));
+        if (nlight == 0 || beside) {          // else the launch behind this one clears them
+            COMET_HIPCHK(hipMemsetAsync(tickets, 0, 8 * sizeof *tickets, stream()));
+            tickets = nullptr;
+        }
     }
     if (nlight > 0) {
         const dim3 grid((unsigned)std::min<int64_t>(ceil_div(nlight, DOT_LIGHT_WAVES), (int64_t)num_cus() * DOT_LIGHT_OCC)),
@@ -639,9 +647,9 @@ static int pair_dot_values(Csr *a, Csr *b, Csr *m, int64_t rb, int64_t re, doubl
         const hipStream_t on = beside ? aux_stream() : stream();
         KernelTimer t("spgemm_numeric_dot_small", on);
         if (semi)
-            pair_dot_light_kernel<true><<<grid, block, 0, on>>>(s0, s1, *pair_val, *pair_hit, op);
+            pair_dot_light_kernel<true><<<grid, block, 0, on>>>(s0, s1, tickets, *pair_val, *pair_hit, op);
         else
-            pair_dot_light_kernel<false><<<grid, block, 0, on>>>(s0, s1, *pair_val, *pair_hit, op);
+            pair_dot_light_kernel<false><<<grid, block, 0, on>>>(s0, s1, tickets, *pair_val, *pair_hit, op);
     }
     if (beside)
         COMET_CHK(aux_join());
@@ -670,6 +678,55 @@ __global__ __launch_bounds__(256) void dot_chunk_count(int64_t n, const uint8_t 
     __syncthreads();
     if (threadIdx.x == 0)
         chunk_kept[blockIdx.x] = wave_count[0] + wave_count[1] + wave_count[2] + wave_count[3];
+}
+
+// The same and where the chunks' pairs go, by one workgroup, four chunks to a wavefront: a launch in place of two.  us of a
+// masked product with three launches behind its pairs / two, R-MAT: 500 vertices, edge factor 4 50.3 / 45.9, 2000 and 8 51.6 /
+// 50.3, 5000 and 6 67.2 / 65.2; with 128 chunks, the workgroup's loads in two turns, 5000 and 16 89.1 / 90.2, with 256 20000
+// and 8 140.6 / 145.7.
+constexpr int DOT_PLACES_T = 1024, DOT_PLACES_U = 4, DOT_PLACES_MOST = DOT_PLACES_T / 64 * DOT_PLACES_U;
+__global__ __launch_bounds__(DOT_PLACES_T) void dot_chunk_places(int64_t n, const uint8_t *__restrict__ pair_hit,
+                                                                 int64_t *__restrict__ chunk_before, int64_t *total)
+{
+    __shared__ int kept[DOT_PLACES_MOST];
+    static_assert(PAIR_CHUNK == 2 * 64 * sizeof(uint4) && DOT_PLACES_MOST == 64, "two loads of a lane to a chunk, a lane to a count");
+    const int lane = threadIdx.x & 63, c0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * DOT_PLACES_U;
+    const int full = (int)(n / PAIR_CHUNK), chunks = (int)((n + PAIR_CHUNK - 1) / PAIR_CHUNK);
+    const uint4 *quads = reinterpret_cast<const uint4 *>(pair_hit);
+    uint4 q[DOT_PLACES_U][2];
+#pragma unroll
+    for (int u = 0; u < DOT_PLACES_U; ++u)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            q[u][h] = c0 + u < full ? quads[(c0 + u) * 128 + 64 * h + lane] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < DOT_PLACES_U; ++u) {
+        int k = 0;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            k += __popc(q[u][h].x) + __popc(q[u][h].y) + __popc(q[u][h].z) + __popc(q[u][h].w);          // bytes of 0 and 1
+        if (c0 + u == full)          // what is left behind the last whole chunk
+            for (int64_t at = (int64_t)full * PAIR_CHUNK + 8 * lane; at < n; at += 8 * 64)
+                if (at + 8 <= n)
+                    k += __popcll(*reinterpret_cast<const unsigned long long *>(pair_hit + at));
+                else
+                    for (int64_t p = at; p < n; ++p)
+                        k += pair_hit[p];
+        k = wave_sum_i32(k);
+        if (lane == 0)
+            kept[c0 + u] = k;
+    }
+    __syncthreads();
+    if (c0 == 0) {
+        const int k = kept[lane], inc = wave_inclusive_scan(k);
+        if (lane < chunks)
+            chunk_before[lane] = inc - k;
+        if (lane == 63) {
+            chunk_before[chunks] = inc;
+            if (total)
+                *total = inc;
+        }
+    }
 }
 
 // Cpos (or null): where the rows begin.
@@ -739,6 +796,12 @@ static int dot_chunks(int64_t n, const uint8_t *pair_hit, int64_t **chunk_before
     COMET_CHK(g_pair_chunk.ensure(sizeof(int64_t) * 2 * (size_t)(*chunks + 1), false));
     int64_t *kept = (int64_t *)g_pair_chunk.ptr;
     *chunk_before = kept + *chunks + 1;
+    if (*chunks > 0 && *chunks <= DOT_PLACES_MOST) {
+        KernelTimer t("spgemm_symbolic_dot_count");
+        dot_chunk_places<<<dim3(1), dim3(DOT_PLACES_T), 0, stream()>>>(n, pair_hit, *chunk_before, total);
+        COMET_HIPCHK(hipGetLastError());
+        return COMET_HIP_OK;
+    }
     if (*chunks > 0) {
         KernelTimer t("spgemm_symbolic_dot_count");
         dot_chunk_count<<<dim3((unsigned)*chunks), dim3(256), 0, stream()>>>(n, pair_hit, kept);

@@ -970,8 +970,12 @@ static int pair_side_plan(const Csr *T, const Csr *P, const Csr *L, int64_t firs
                                              ranged ? PAIR_RANGED_SHARES : PAIR_SHARES, item_min, parts);
     COMET_CHK(exclusive_scan_i64(parts, n, wpos));
     COMET_HIPCHK(hipMemcpyAsync(word, wpos + n, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
+    if (npairs == entries)          // what was room is a number
+        COMET_HIPCHK(hipMemcpyAsync((int64_t *)word + 1, kept_before + chunks, sizeof(int64_t), hipMemcpyDeviceToHost, stream()));
     COMET_CHK(stream_wait());
     const int64_t packed = *(volatile int64_t *)word;
+    if (npairs == entries)
+        plan->pairs = *((volatile int64_t *)word + 1);
     plan->nheavy = packed & 0xffffffff;
     plan->nlight = packed >> 32;
     COMET_HIPCHK(dev_malloc((void **)&plan->heavy, sizeof(uint2) * (size_t)(plan->nheavy > 0 ? plan->nheavy : 1)));

@@ -325,6 +325,34 @@ def test_masked_product_gathers_its_result_by_chunks(nnz):
     assert all(np.array_equal(g, w) for g, w in zip(rt.spgemm(A, B, M).to_arrays(), want))
 
 
+@pytest.mark.parametrize("empty", [None, "row", "column"])
+@pytest.mark.parametrize("pairs", [64 * 2048 - 1, 64 * 2048, 64 * 2048 + 1, 2048, 7])
+def test_masked_product_with_and_without_pairs_of_no_side(pairs, empty):
+    # up to 64 chunks of 2048 pairs are counted and placed by one launch; the marks are cleared first only where a pair's
+    # row of A or column of B is empty; the same handles with another mask in between leave marks behind
+    rows, k, n = 40, 3, 5000
+    rng = np.random.default_rng(pairs)
+    cells = np.sort(rng.permutation(rows * n)[:pairs])
+    mask = (np.searchsorted(cells, np.arange(rows + 1) * n).astype(np.int64), (cells % n).astype(np.int32), np.ones(pairs))
+    full = (np.arange(rows + 1, dtype=np.int64) * 4000, np.tile(np.arange(4000, dtype=np.int32), rows), np.ones(rows * 4000))
+    a_full, b_full = rng.integers(1, 9, (rows, k)).astype(float), rng.integers(1, 9, (k, n)).astype(float)
+    a_full[::3, 1:] = 0.0                        # those rows do not meet the columns without an entry in the first row of B
+    b_full[0, ::2] = 0.0
+    if empty == "row":
+        a_full[[0, 17, rows - 1]] = 0.0
+    if empty == "column":
+        b_full[:, n // 2:] = 0.0
+
+    def csr(x):
+        return np.concatenate([[0], np.cumsum((x != 0).sum(1))]).astype(np.int64), np.nonzero(x)[1].astype(np.int32), x[x != 0]
+
+    a, b = csr(a_full), csr(b_full)
+    A, B, M, F = (rt.CsrMatrix.from_arrays(shape, *x) for shape, x in (((rows, k), a), ((k, n), b), ((rows, n), mask), ((rows, n), full)))
+    want, between = (orc.spgemm(*a, *b, n, mask=m[:2]) for m in (mask, full))
+    for handle, w in ((F, between), (M, want), (F, between), (M, want)):
+        assert all(np.array_equal(g, x) for g, x in zip(rt.spgemm(A, B, handle).to_arrays(), w))
+
+
 @pytest.mark.parametrize("shape", [0, 1, 2, 3])
 @pytest.mark.parametrize("c,n,shares", [(17, 15, 1), (19, 27, 1), (31, 33, 1), (61, 47, 1), (61, 47, 2), (61, 47, 3), (61, 47, 17),
                                         (61, 47, 64), (61, 47, 180)])
