@@ -418,8 +418,8 @@ __device__ __forceinline__ void tri_sum(const TriTurn<ROWS> &t, const PROBE &pro
 }
 
 // As pair_sum_heavy_kernel.  nwords: 32-bit words of the table.
-__global__ __launch_bounds__(SG_T) void tri_heavy_kernel(PairSide s, int nwords, unsigned long long *__restrict__ tickets,
-                                                         unsigned long long *__restrict__ block_hits)
+__global__ __launch_bounds__(SG_T) void tri_heavy_kernel(PairSide s, int nwords, unsigned long long *tickets,
+                                                         PairTotal total)
 {
     uint16_t *bits = reinterpret_cast<uint16_t *>(sg_dyn_lds);
     PairHeavyShared &sh = *reinterpret_cast<PairHeavyShared *>(sg_dyn_lds + nwords);
@@ -485,12 +485,12 @@ __global__ __launch_bounds__(SG_T) void tri_heavy_kernel(PairSide s, int nwords,
         it = pair_item_read(sh.slot[cur]);
         lds_barrier();
     }
-    pair_block_hits(sh.wave_hits, all_hits, SG_WAVES, block_hits);
+    pair_block_hits(sh.wave_hits, all_hits, SG_WAVES, total);
 }
 
 // As pair_sum_light_kernel.
 __global__ __launch_bounds__(PAIR_LIGHT_WAVES * 64, PAIR_LIGHT_OCC) void tri_light_kernel(
-    PairSide s, unsigned long long *__restrict__ block_hits)
+    PairSide s, PairTotal total)
 {
     constexpr int NB = 1 << PAIR_LIGHT_LOG;
     __shared__ __align__(16) int table[PAIR_LIGHT_WAVES][NB * 4];
@@ -606,7 +606,7 @@ __global__ __launch_bounds__(PAIR_LIGHT_WAVES * 64, PAIR_LIGHT_OCC) void tri_lig
             wave_lds_order();
         }
     }
-    pair_block_hits(wave_hits, all_hits, PAIR_LIGHT_WAVES, block_hits);
+    pair_block_hits(wave_hits, all_hits, PAIR_LIGHT_WAVES, total);
 }
 
 // A wavefront's row may have this many look-ups in a small graph too, whose parts of PAIR_ITEM_MIN would make it 2048: rows
@@ -742,20 +742,22 @@ static int tri_count(Csr *a, double *result)
     COMET_CHK(pair_tickets(&tickets));
     COMET_CHK(mailbox((void **)&word));
     const PairGrids grids = pair_grids(nheavy, nlight, a->ncols);
-    COMET_CHK(g_pair_hits.ensure(sizeof(unsigned long long) * (size_t)(grids.heavy + grids.light + 1), false));
-    unsigned long long *hits = (unsigned long long *)g_pair_hits.ptr;
+    PairTotal total{tickets, grids.heavy + grids.light, 0, a->iso_value * a->iso_value, word};
+    if (total.blocks == 0) {
+        *result = 0.0;
+        return COMET_HIP_OK;
+    }
     if (nheavy > 0) {
         COMET_CHK(sg_allow_lds(tri_heavy_kernel, grids.lds));
         KernelTimer t("spgemm_masked_sum");
-        tri_heavy_kernel<<<dim3(grids.heavy), dim3(SG_T), grids.lds, stream()>>>(s, grids.nwords, tickets, hits);
+        tri_heavy_kernel<<<dim3(grids.heavy), dim3(SG_T), grids.lds, stream()>>>(s, grids.nwords, tickets, total);
     }
     if (nlight > 0) {
         KernelTimer t("spgemm_masked_sum_small");
-        tri_light_kernel<<<dim3(grids.light), dim3(PAIR_LIGHT_WAVES * 64), 0, stream()>>>(s, hits + grids.heavy);
+        total.first = grids.heavy;
+        tri_light_kernel<<<dim3(grids.light), dim3(PAIR_LIGHT_WAVES * 64), 0, stream()>>>(s, total);
     }
-    pair_hits_finish<<<dim3(1), dim3(PAIR_HITS_T), 0, stream()>>>(tickets, hits, (int)(grids.heavy + grids.light),
-                                                                  a->iso_value * a->iso_value, word);
-    COMET_HIPCHK(hipGetLastError());
+    COMET_CHK(pair_launched(tickets));
     COMET_CHK(stream_wait());
     *result = *(volatile double *)word;
     return COMET_HIP_OK;

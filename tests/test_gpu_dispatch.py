@@ -874,6 +874,20 @@ def test_triangle_counts_of_every_kind_of_graph(kind, upper, only, monkeypatch):
     assert [rt.spgemm_masked_sum(L, L, mask) for _ in range(2)] == [0.25 * want] * 2
 
 
+@pytest.mark.parametrize("only", [None, "workgroup", "wavefront"])
+def test_sums_of_hits_of_any_number_of_workgroups(only, monkeypatch):
+    # bands of three: from no workgroup over fewer than eight and remainders to those of a full chip and more rows than that
+    if only:
+        monkeypatch.setenv("COMET_HIP_MASKED_SUM_ONLY", only)
+    for n in [2, 3, 4, 7, 9, 10, 11, 30, 33, 66, 257, 1030, 2051, 9000]:
+        u = np.repeat(np.arange(n), 2)
+        v = u - np.tile([2, 1], n)
+        u, v = u[v >= 0], v[v >= 0]
+        pos = np.concatenate([[0], np.cumsum(np.bincount(u, minlength=n))]).astype(np.int64)
+        L, M = (rt.CsrMatrix.from_arrays((n, n), pos, v.astype(np.int64), np.full(len(u), x)) for x in (0.5, 2.0))
+        assert [rt.triangle_count(L), rt.spgemm_masked_sum(L, L, M), rt.triangle_count(L)] == [0.25 * (n - 2)] * 3, n
+
+
 def test_the_plan_of_triangle_counts_is_made_once_and_where_it_serves(monkeypatch):
     # at the first count and never again, for matrices that are strictly on one side and hold no column twice - the last
     # column of a row and the first of the next may be the same -; the others' sums take the pairs as they are
