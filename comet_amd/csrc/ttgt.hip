@@ -221,7 +221,7 @@ static int transpose_device(int rank, const int64_t *in_shape, const int32_t *pe
 // TM x TN MFMA tiles of 16 x 16.  K advances 16 at a time through
 // double-buffered LDS, both operands stored k-major (a 16 x 4 operand is one
 // ds_read_b64 per lane).  Offsets of the rows and columns are worked out once
-// per tile of C, those of the 16 k of a turn sixteen turns at a time, one to a lane.
+// per tile of C, those of the k of some turns at a time, one to a lane.
 // A thread takes its elements along whichever index is contiguous in memory
 // (A_M / B_N: the outer one, else along k).  Operand layout of
 // v_mfma_f64_16x16x4_f64: lane l supplies A[l%16][l/16] and B[l/16][l%16] and
@@ -290,6 +290,31 @@ __device__ __forceinline__ void gett_offsets(const GettDims &g, uint32_t i, OFF 
     *o1 = b + (OFF)i * (OFF)g.s1[0];
 }
 
+// Which tile and share of k a workgroup takes.  Workgroup i runs on XCD i mod 8: an XCD takes an eighth of the list of tiles,
+// band by band of GETT_BAND rows of tiles, down the columns of a band, so that the workgroups of its CUs share few rows and
+// columns of the operands in its L2.  (Tile i to workgroup i spreads the tiles of a row over the XCDs unless a row has a
+// multiple of eight.)  us, tile i to workgroup i / in bands of 4 / 8 / 16 / 32, aebf,dfce->abcd: 77 x 1665 outputs of 532
+// products 31.5 / 22.2 / 22.2 / 22.2 / 22.2, 20^6 18.5 / 17.6 / 17.3 / 17.1 / 17.1, 24^6 25.9 / 27.6 / 27.4 / 26.8 / 26.9, 26^6
+// 32.1 / 34.5 / 34.1 / 33.8 / 33.7, 28^6 41.8 / 40.8 / 40.7 / 40.0 / 39.9, 36^6 128.2 / 124.0 / 124.5 / 124.5 / 124.3, 61^6
+// 1996 / 1912 / 1914 / 1930 / 1974, 62^6 2187 / 2114 / 2118 / 2137 / 2177, 64^6 1980 / 1974 / 1979 / 1982 / 1985.
+constexpr uint32_t GETT_XCDS = 8, GETT_BAND = 16;
+struct GettPlace {
+    uint32_t m, n, share;
+};
+__device__ __forceinline__ GettPlace gett_place(uint32_t tiles_m, uint32_t tiles_n)
+{
+    const uint32_t all = gridDim.x * gridDim.y, id = blockIdx.y * gridDim.x + blockIdx.x;
+    const uint32_t xcd = id % GETT_XCDS, each = all / GETT_XCDS, more = all % GETT_XCDS;
+    const uint32_t i = xcd * each + (xcd < more ? xcd : more) + id / GETT_XCDS;
+    GettPlace p;
+    p.share = i / gridDim.x;
+    const uint32_t t = i - p.share * gridDim.x, band = t / (GETT_BAND * tiles_n), first = band * GETT_BAND;
+    const uint32_t rows = tiles_m - first < GETT_BAND ? tiles_m - first : GETT_BAND, in = t - first * tiles_n;
+    p.n = in / rows;
+    p.m = first + (in - p.n * rows);
+    return p;
+}
+
 template <int BM, int BN, int WM, int OCC, bool A_M, bool B_N, bool REG, bool RUN>
 __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const double *__restrict__ A,
                                                              const double *__restrict__ B, double *__restrict__ C,
@@ -301,21 +326,23 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
     constexpr int KSA = 256 / BM, KSB = 256 / BN;
     __shared__ double As[2][GM_BK][LDA];
     __shared__ double Bs[2][GM_BK][LDB];
-    // offsets in bytes of the rows (A), the columns (B) and, unless they are regular, of the k of sixteen turns, twice
-    __shared__ uint32_t rowA[BM], colB[BN], kA[REG ? 1 : 2][REG ? 1 : 256], kB[REG ? 1 : 2][REG ? 1 : 256];
+    // offsets in bytes of the rows (A), the columns (B) and, unless they are regular, of the k of KT turns, twice: sixteen,
+    // but one where sixteen would take the fourth workgroup its LDS (3844 sums of 3844 products 37.4 us, with one 33.8)
+    constexpr int KT = BN == 16 ? 1 : 16, KN = REG ? 1 : KT * GM_BK;
+    __shared__ uint32_t rowA[BM], colB[BN], kA[REG ? 1 : 2][KN], kB[REG ? 1 : 2][KN];
     __shared__ int64_t rowC[BM], colC[BN];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WN, wn = wave % WN;
-    const uint32_t tiles_n = (g.N + BN - 1) / BN;
-    const uint32_t m0 = blockIdx.x / tiles_n * BM, n0 = blockIdx.x % tiles_n * BN;
-    const uint32_t k_begin = blockIdx.y * g.turns * GM_BK;
+    const GettPlace place = gett_place((g.M + BM - 1) / BM, (g.N + BN - 1) / BN);
+    const uint32_t m0 = place.m * BM, n0 = place.n * BN;
+    const uint32_t k_begin = place.share * g.turns * GM_BK;
     const uint32_t k_end = k_begin + g.turns * GM_BK < g.K ? k_begin + g.turns * GM_BK : g.K;
     const int nt = (int)((k_end - k_begin + GM_BK - 1) / GM_BK);
 
-    // the offsets of the k of sixteen turns, one to a lane (by sixteen lanes a turn they were the longest chain of every turn)
+    // the offsets of the k of KT turns, one to a lane (by sixteen lanes a turn they were the longest chain of every turn)
     const auto k_offsets = [&](int chunk) {
-        if constexpr (!REG) {
-            const uint32_t k = k_begin + 256u * (uint32_t)chunk + tid;
+        if (!REG && tid < KN) {
+            const uint32_t k = k_begin + (uint32_t)(KN * chunk) + tid;
             uint32_t a, b;
             gett_offsets(g.k, k < k_end ? k : k_end - 1, &a, &b);
             kA[chunk & 1][tid] = a * 8;
@@ -335,6 +362,8 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
         colC[c] = d;
     }
     k_offsets(0);
+    if (KT == 1 && nt > 1)
+        k_offsets(1);
     __syncthreads();
 
     // thread -> elements of a turn's tiles: along the outer index (one row, E values of k) or along k (one k, E rows).
@@ -426,7 +455,7 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
             k_next += GM_BK;
             --run;
         } else {
-            const uint32_t *ka = kA[t >> 4 & 1] + (t & 15) * GM_BK, *kb = kB[t >> 4 & 1] + (t & 15) * GM_BK;
+            const uint32_t *ka = kA[t / KT & 1] + t % KT * GM_BK, *kb = kB[t / KT & 1] + t % KT * GM_BK;
 #pragma unroll
             for (int e = 0; e < EA; ++e)
                 ra[e] = gett_load(A, A_M ? ao[0] + ka[a_k + KSA * e] : ao[A_M ? 0 : e] + ka[a_k]);
@@ -486,8 +515,8 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
         fragments(0);
         if (t + 1 < nt)
             load_tiles(t + 1);
-        if (!REG && (t + 2) % 16 == 0 && t + 2 < nt)
-            k_offsets((t + 2) / 16);           // for the loads of the next turn
+        if (!REG && (t + 2) % KT == 0 && t + 2 < nt)
+            k_offsets((t + 2) / KT);           // for the loads of the next turn
 #pragma unroll
         for (int ks = 0; ks < GM_BK; ks += 4) {
             if (ks + 4 < GM_BK)
@@ -504,7 +533,7 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
     }
 
     const bool whole = gridDim.y == 1, inside = m0 + BM <= g.M && n0 + BN <= g.N;
-    double *out = whole ? C : partial + (uint64_t)blockIdx.y * g.M * g.N;
+    double *out = whole ? C : partial + (uint64_t)place.share * g.M * g.N;
     int64_t cols[TN];
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
@@ -573,7 +602,8 @@ __global__ __launch_bounds__(GETT_REDUCE_T) void gett_reduce(GettArgs g, int spl
 // The tile shapes: workgroups a CU holds, the time of a turn of 16 k divided by them on a full CU, and the time of a
 // turn of a workgroup that has its CU to itself (measured, us; 4096^3 takes 1908 / 2125 / 2440 / 3109 us with the four
 // shapes, the first at 92 % of the matrix cores' rate).  The launch takes the shape and the number of shares of k that
-// these figures make cheapest: small tiles and many shares where the outputs are few, the large tile where they are
+// these figures make cheapest, a last round that fills no more than some of the workgroups' places by what it leaves to a
+// CU: small tiles and many shares where the outputs are few, the large tile where they are
 // not, and the narrow ones where one side of C is short.
 struct GettShape {
     int bm, bn, resident;
@@ -586,6 +616,9 @@ constexpr double GETT_REDUCE_US = 5.0;
 // bytes a us that partial tiles are written and read at: few and large, many and small (62 x 62 outputs 97 shares 12.3 us, 194
 // 14.4; 300 x 650 over 225 products one share 18.4, four 16.5)
 constexpr double GETT_REDUCE_FEW = 6.0e6, GETT_REDUCE_MANY = 3.0e6;
+// The large tile loses more where the k have to be looked up: 52^6 in the large tile 790, in the next 812, 62^6 2170 and 2190 to
+// 2275, which without this come out as 632 / 708 and 1798 / 1890 (and 64^6, regular, as 1910 / 2130).
+constexpr double GETT_IRREGULAR = 1.06;
 constexpr int GETT_NSHAPES = sizeof(GETT_SHAPES) / sizeof(GETT_SHAPES[0]);
 
 static Workspace g_gett_partial;
@@ -654,6 +687,7 @@ static int gett_run(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t N,
     g.N = (uint32_t)N;
     g.K = (uint32_t)K;
     const int64_t nk = ceil_div(K, GM_BK);
+    const bool reg = k.nd == 1 || k.ext[k.nd - 1] % GM_BK == 0;
     const int64_t cus = num_cus() > 0 ? num_cus() : 256;
     int best = 0;
     int64_t splits = 1;
@@ -661,12 +695,15 @@ static int gett_run(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t N,
     for (int c = 0; c < GETT_NSHAPES; ++c) {
         const GettShape &sh = GETT_SHAPES[c];
         const int64_t tiles = ceil_div(M, sh.bm) * ceil_div(N, sh.bn);
-        for (int64_t s = 1; s <= nk && s <= 1024; s *= 2) {
+        // (shares by powers of two only: 48^6 490 us, now in three 437; 60^6 1900, now 1805; 28^6 45.4, 41.8)
+        for (int64_t s = 1; s <= nk && s <= 1024; s += s < 8 ? 1 : s) {
             const int64_t turns = ceil_div(nk, s), groups = tiles * ceil_div(nk, turns);
-            const int64_t rounds = ceil_div(groups, cus * sh.resident);
-            const double per_cu = (double)std::min<int64_t>(sh.resident, ceil_div(groups, cus));
-            const double turn = std::max(sh.alone_us, per_cu * sh.turn_us);
-            const double us = (double)rounds * ((double)turns * turn + 2.5) +
+            const int64_t full = groups / (cus * sh.resident), rest = groups % (cus * sh.resident);
+            const double slower = c == 0 && !reg ? GETT_IRREGULAR : 1.0;
+            const auto round_us = [&](int64_t a_cu) {
+                return (double)turns * std::max(sh.alone_us, (double)a_cu * sh.turn_us) * slower + 2.5;
+            };
+            const double us = (double)full * round_us(sh.resident) + (rest > 0 ? round_us(ceil_div(rest, cus)) : 0.0) +
                               (s > 1 ? GETT_REDUCE_US + (double)ceil_div(nk, turns) * (double)(M * N) * 16.0 /
                                                             (s <= 4 ? GETT_REDUCE_FEW : GETT_REDUCE_MANY)
                                      : 0.0);
@@ -702,7 +739,6 @@ static int gett_run(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t N,
     const int use_c = beta != 0.0;
     {
         KernelTimer t("gett_mfma_kernel");
-        const bool reg = k.nd == 1 || k.ext[k.nd - 1] % GM_BK == 0;
         // sixteen bytes at a time: a thread's run along the contiguous index is unbroken and aligned
         const auto runs = [](const GettIndex &x, const int64_t *s, bool along, int run) {
             for (int d = 0; d < x.nd; ++d)

@@ -55,6 +55,20 @@ def test_contraction_every_tile_shape_and_layout(a, b, c, forced, monkeypatch):
             assert np.all(np.abs(dC.to_numpy() - want - beta * C0) <= 1e-13 * (bound + 1.0)), (extent, beta)
 
 
+@pytest.mark.parametrize("forced", ["0,1", "1,1", "1,3", "2,1", "2,5", "3,1", "3,2"])
+@pytest.mark.parametrize("m,n,k", [(1100, 200, 40), (2200, 33, 33), (70, 2100, 96), (1030, 1030, 17), (129, 16, 130)])
+def test_contraction_takes_every_tile_once(m, n, k, forced, monkeypatch):
+    # tiles by bands of sixteen rows, an eighth of the list to an XCD: last bands of few rows, lists of no multiple of eight
+    monkeypatch.setenv("COMET_HIP_GETT", forced)
+    rng = np.random.default_rng(m)
+    A, B, C0 = rng.uniform(-1, 1, (m, k)), rng.uniform(-1, 1, (k, n)), rng.uniform(-1, 1, (m, n))
+    want, bound = A @ B, np.abs(A) @ np.abs(B)
+    for beta in (0.0, 1.0):
+        dC = rt.DeviceArray.from_numpy(C0)
+        rt.ttgt_contract("ef", "fc", "ec", rt.DeviceArray.from_numpy(A), rt.DeviceArray.from_numpy(B), dC, beta=beta)
+        assert np.all(np.abs(dC.to_numpy() - want - beta * C0) <= 1e-13 * (bound + 1.0))
+
+
 @pytest.mark.parametrize("pieces", [2, 3, 7])
 @pytest.mark.parametrize("a,b,c", [("ef", "fc", "ec"), ("aebf", "dfce", "abcd"), ("aebf", "efcd", "abcd"), ("feab", "efcd", "dcba"),
                                    ("abef", "ef", "ab"), ("ab", "cd", "acbd"), ("f", "fa", "a")])
