@@ -50,7 +50,10 @@ constexpr int64_t PAIR_SHARES = 2048;                                // parts th
 // worth 200,000 look-ups then, 140,000 where two workgroups share a CU (up to PAIR_RANGED_COLS columns) - a table is built
 // and cleared for it -, us at 60,000 / 100,000 / 140,000 / 200,000: 160000 and 8 1091 / 1023 / 976 / 947, 260000 and 8 1309 / 1279
 // / 1219 / 1184, 90000 and 16 1080 / 1063 / 1022 / 1041; and a 4096th of all at least (2048th, 8192th: 200003 and 16 3046,
-// 3177 against 2935).
+// 3177 against 2935).  Beyond PAIR_RANGED_MOST columns the larger tables of more parts cost what the L2s save, ms without / by
+// stretches, edge factor 16: 262144 3.92 / 3.45, 500000 10.6 / 10.1, 700000 35.3 / 34.2, 2^20 39.9 / 40.0; 2^20 and 8 12.2 / 12.3;
+// a permuted graph of 2^20 34.2 / 35.6.
+constexpr int64_t PAIR_RANGED_MOST = 3 << 18;
 constexpr int64_t PAIR_RANGED_LISTS = 14 << 20, PAIR_RANGED_COLS = 1 << 17, PAIR_RANGED_TWO = 140000, PAIR_RANGED_ONE = 200000;
 constexpr int64_t PAIR_RANGED_SHARES = 4096;
 
@@ -976,7 +979,7 @@ static int pair_side_plan(const Csr *T, const Csr *P, const Csr *L, int64_t firs
     pair_pass<true><<<grid, block, 0, stream()>>>(first, last, T->pos, P->pos, P->crd, L->pos, strict, xlo, xhi, kept_before,
                                                   work_before, plan->kpos, wpos, (PairEnt *)plan->ent, P->val, scale,
                                                   plan->weight, perm, out0, plan->place);
-    const bool ranged = places && L->nnz * (int64_t)(sizeof(int32_t) + sizeof(double)) > PAIR_RANGED_LISTS;
+    const bool ranged = places && T->ncols <= PAIR_RANGED_MOST && L->nnz * (int64_t)(sizeof(int32_t) + sizeof(double)) > PAIR_RANGED_LISTS;
     const int64_t item_min = !ranged ? PAIR_ITEM_MIN : T->ncols <= PAIR_RANGED_COLS ? PAIR_RANGED_TWO : PAIR_RANGED_ONE;
     pair_parts<<<rows, block, 0, stream()>>>(first, n, T->pos, plan->kpos, wpos, only, light_max, 0,
                                              ranged ? PAIR_RANGED_SHARES : PAIR_SHARES, item_min, parts);
