@@ -1614,7 +1614,7 @@ static int sweep_launch(Kern kernel, dim3 grid, dim3 block, size_t lds, Args... 
 }
 
 // Whether rows of B and C that are no multiple of 16 bytes are swept: most of the matrix has to be in the long rows, and a
-// row of B in several of them.  us, chunks / sweep at K = 17, 33, 63, and of the entries the share in long rows and how many
+// row of B in several of them.  us, chunks as stored / sweep at K = 17, 33, 63, and of the entries the share in long rows and how many
 // of them there are a column: zipf, 200000 rows of 4 (0.69, 2.7) 62 / 124, 77 / 131, 113 / 113, of 8 (0.81, 6.5) 87 / 100, 115 /
 // 107, 177 / 106, 100000 of 16 (0.86, 14) K = 33 101 / 78, 63 159 / 83; R-MAT scale 17, 4 edges a vertex (0.37, 2.8) K = 33
 // 105 / 145, 16 (0.54, 15) 144 / 332.
@@ -2053,7 +2053,7 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
         return set_error(COMET_HIP_ERR_SIZE, "K = %lld needs more than 65535 column tiles", (long long)K);
     // long rows: column sweep with the sums on chip; everything else: one wavefront per 256 nonzeros
     // Rows of B and C that are no multiple of 16 bytes are swept where B is so large that its gathers come from far away
-    // (chunks / sweep, us: K = 33 40000 rows 51 / 65, 60001 69 / 68, 120000 121 / 87, 250000 242 / 153, 500000 477 / 277;
+    // (chunks as stored / sweep, us: K = 33 40000 rows 51 / 65, 60001 69 / 68, 120000 121 / 87, 250000 242 / 153, 500000 477 / 277;
     // K = 63 40000 71 / 74, 60001 102 / 77, 500000 758 / 358; K = 17 60001 52 / 60, 500000 348 / 230: zipf, 16 entries a row),
     // where the matrix is right for it (sweep_uneven), and where no tile of columns holds a single one.
     const bool even = (K & 1) == 0 && (ldb & 1) == 0 && (b_dptr & 15) == 0 && (ldc & 1) == 0 && (c_dptr & 15) == 0;
