@@ -1581,6 +1581,13 @@ struct DenseRow {
     int32_t pad;
 };
 constexpr int DB_ROWS = 8;
+// A matrix of fewer columns than a block.  The columns there are are shared out to the wavefronts, or one writes out what all
+// have added; and where there are rows enough (nine to two CUs) two workgroups of half the lanes share a CU, one adding while
+// the other starts on a row or writes it out.  us, A*A, R-MAT, a block of 16384 columns / its own / two workgroups, and the rows
+// here: 1024 vertices, edge factor 8, min-plus 61.9 / 57.8 / 60.5 (114), 2048 and 16 95.0 / 85.7 / 94.7 (724), 4000 and 10 122 /
+// 112 / 120 (1105); plus-times 3000 and 12 107 / 99 / 98 (1121), 8000 and 5 119 / 115 / 111 (1171), 4096 and 16 136 / 126 / 120
+// (1766), 8000 and 10 177 / 168 / 158 (2639), 6000 and 16 236 / 232 / 184 (3096), 8192 and 16 268 / 264 / 218 (3776).
+constexpr int64_t DB_TWO_ROWS = 9;
 constexpr int DB_PATIENCE = 1 << 24;
 
 // Where the rows come from: the first of the list, as rows of A and C.
@@ -1635,9 +1642,13 @@ struct SliceStage {
     uint32_t marks[WAVES][2];        // zero between turns
     int turns[ENTRIES / 64];         // of each batch
 };
-typedef SliceStage<SG_T, SG_CB, 21> BlockStage;
-constexpr size_t DB_LDS = (size_t)SG_CB * 8 + sizeof(BlockStage);
-static_assert(DB_LDS + 256 <= 160 * 1024, "accumulators and slices fit LDS");
+template <int T>
+using BlockStage = SliceStage<T, SG_CB, 21, T / 64>;
+// of workgroups of T lanes whose wavefronts each have 64 * ROWS columns
+template <int T, int ROWS>
+constexpr size_t DB_LDS = (size_t)T * ROWS * 8 + sizeof(BlockStage<T>);
+static_assert(DB_LDS<SG_T, 16> + 256 <= 160 * 1024, "accumulators and slices fit LDS");
+static_assert(512 * 16 == SG_CB / 2 && 2 * (DB_LDS<512, 16> + 256) <= 160 * 1024, "so do two workgroups' of a matrix of half a block");
 
 template <typename COL>
 struct SliceTurn {
@@ -1798,11 +1809,11 @@ __device__ __forceinline__ void block_add(double *slot, double a, double b, int 
 // Writes out what the accumulators of a block hold, in order of the columns, and leaves them empty; place(total) as in
 // dense_emit_block.  A wavefront has 1024 columns to itself: it takes them into registers, and its part of acc becomes
 // the list, half of the columns at a time, from which every lane writes the entry at its own place.
-template <bool SEMI, typename VALUE, typename PLACE>
+template <bool SEMI, int WAVES, int ROWS, typename VALUE, typename PLACE>
 __device__ __forceinline__ void block_emit(double *acc, int *wave_tot, int lane, int wave, int col0, int reduce_op,
                                            int32_t *__restrict__ Ccrd, double *__restrict__ Cval, VALUE value, PLACE place)
 {
-    constexpr int MINE = SG_CB / SG_WAVES, ROWS = MINE / 64, HALF = ROWS / 2;
+    constexpr int MINE = 64 * ROWS, HALF = ROWS / 2;
     static_assert(MINE / 2 * (8 + 2) <= MINE * 8, "the list of half the columns fits their accumulators");
     const unsigned long long empty = block_empty(SEMI ? reduce_op : SR_PLUS);
     unsigned long long *own = reinterpret_cast<unsigned long long *>(acc) + wave * MINE;
@@ -1820,8 +1831,8 @@ __device__ __forceinline__ void block_emit(double *acc, int *wave_tot, int lane,
     if (lane == 0)
         wave_tot[wave] = cnt;
     lds_barrier();
-    const int tots = wave_inclusive_scan(lane < SG_WAVES ? wave_tot[lane] : 0);
-    const int total = __builtin_amdgcn_readlane(tots, SG_WAVES - 1);
+    const int tots = wave_inclusive_scan(lane < WAVES ? wave_tot[lane] : 0);
+    const int total = __builtin_amdgcn_readlane(tots, WAVES - 1);
     int64_t off = place(total) + (wave ? __builtin_amdgcn_readlane(tots, wave - 1) : 0);
     const int first = col0 + wave * MINE;
 #pragma unroll
@@ -1852,21 +1863,22 @@ __device__ __forceinline__ void block_emit(double *acc, int *wave_tot, int lane,
 }
 
 // ALONE: the matrix is one block wide, a row's entries leave at once; nobody has listed the rows (rows is null then).
-template <bool SEMI, typename COL, bool ALONE>
-__global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
+// T lanes, 64 * ROWS columns to a wavefront.
+template <bool SEMI, typename COL, bool ALONE, int T, int ROWS>
+__global__ __launch_bounds__(T, 4) void spgemm_numeric_dense_blocks_kernel(
     const DenseRow *__restrict__ rows, RowSource source, int64_t nd, const int32_t *__restrict__ Acrd, const double *__restrict__ Aval,
     const COL *__restrict__ Bcrd, const double *__restrict__ Bval, int64_t Bnnz, const int64_t *__restrict__ blkptr, int nblk,
     unsigned long long *ticket, int32_t *before, int rows_each, int patience, int *gave_up, int32_t *__restrict__ Ccrd,
     double *__restrict__ Cval, int reduce_op, int mult_op)
 {
     __shared__ int64_t row_slot;
-    __shared__ int wave_tot[SG_WAVES];
+    __shared__ int wave_tot[T / 64];
     __shared__ int ahead_slot;                  // the row's entries ahead of the block
     double *acc = reinterpret_cast<double *>(sg_dyn_lds);
-    BlockStage &st = *reinterpret_cast<BlockStage *>(acc + SG_CB);
+    BlockStage<T> &st = *reinterpret_cast<BlockStage<T> *>(acc + T * ROWS);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    for (int j = threadIdx.x; j < SG_CB; j += SG_T)
+    for (int j = threadIdx.x; j < T * ROWS; j += T)
         reinterpret_cast<unsigned long long *>(acc)[j] = block_empty(SEMI ? reduce_op : SR_PLUS);
     if (lane < 2)
         st.marks[wave][lane] = 0;
@@ -1890,7 +1902,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
             else
                 mine = rows[r0 + lane];
         }
-        // the entry of A a lane holds of row x of the ticket (of its first SG_T entries: a longer row loads the others
+        // the entry of A a lane holds of row x of the ticket (of its first T entries: a longer row loads the others
         // as it goes), and the slice of its row of B inside the block
         const auto load_entry = [&](int x, int &k, double &a) {
             k = -1;
@@ -1941,7 +1953,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
                         if (t.mask >> x & 1u)
                             block_add<SEMI>(&acc[j[x] - from0], t.a, b[x], pa0 + t.pa + 1, t.q + x, reduce_op, mult_op);
                 });
-                for (int64_t q = lo + BlockStage::MOST; q < hi; ++q)
+                for (int64_t q = lo + BlockStage<T>::MOST; q < hi; ++q)
                     block_add<SEMI>(&acc[(int)Bcrd[q] - from0], a, Bval[q], pa0 + (int)threadIdx.x + 1, q, reduce_op, mult_op);
                 return turns;
             };
@@ -1953,11 +1965,11 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
             if (!ALONE && threadIdx.x == 0 && cb > 0)
                 early = __hip_atomic_fetch_max(mark, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             int turns;
-            if (cnt <= SG_T) {
+            if (cnt <= T) {
                 turns = walk(0, lo0, hi0, a0);
                 lds_barrier();
             } else {
-                // the entries of A beyond the first SG_T, SG_T at a time: a pass's entries are loaded two passes
+                // the entries of A beyond the first T, T at a time: a pass's entries are loaded two passes
                 // ahead and its slices one, so that a walk does not begin with two trips to memory
                 const auto load_more = [&](int base, int &k, double &a) {
                     k = -1;
@@ -1970,14 +1982,14 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
                 int kn;
                 double ab = a0, an;
                 int64_t lob = lo0, hib = hi0;
-                load_more(SG_T, kn, an);
+                load_more(T, kn, an);
                 turns = 0;
-                for (int base = 0; base < cnt; base += SG_T) {
+                for (int base = 0; base < cnt; base += T) {
                     int64_t lon, hin;
                     load_slice(kn, lon, hin);
                     int kf;
                     double af;
-                    load_more(base + 2 * SG_T, kf, af);
+                    load_more(base + 2 * T, kf, af);
                     turns += walk(base, lob, hib, ab);
                     lds_barrier();
                     lob = lon;
@@ -1985,7 +1997,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
                     ab = an;
                     kn = kf;
                     an = af;
-                    if (base + SG_T < cnt) {
+                    if (base + T < cnt) {
                         slice_put(st, lob, hib, ab, lane, wave);
                         lds_barrier();
                     }
@@ -2015,7 +2027,7 @@ __global__ __launch_bounds__(SG_T) void spgemm_numeric_dense_blocks_kernel(
             if (any) {
                 if (threadIdx.x == 0)
                     ahead_slot = await();          // (read behind the first barrier of the write-out)
-                block_emit<SEMI>(acc, wave_tot, lane, wave, col0, reduce_op, Ccrd, Cval,
+                block_emit<SEMI, T / 64, ROWS>(acc, wave_tot, lane, wave, col0, reduce_op, Ccrd, Cval,
                                  [&](unsigned long long v) {
                                      return SEMI ? semiring_lds_value(v, reduce_op, mult_op, as, Aval, Bval)
                                                  : __longlong_as_double((long long)v);
@@ -3971,35 +3983,46 @@ static int numeric_rows(const Csr *a, Csr *b, const Csr *m, const int64_t *Cpos,
                 patience = atoi(e);
             KernelTimer t("spgemm_numeric_dense_blocks");
             const dim3 cus((unsigned)(num_cus() > 0 ? num_cus() : 256));
-            // as many rows to a ticket as leave every CU some four of them (8 to each of 50 CUs: 78 us for a graph of 1024
-            // vertices, the others idle)
-            const int rows_each = (int)std::max<int64_t>(1, std::min<int64_t>(DB_ROWS, nd * nblk / (4 * (int64_t)cus.x)));
             if (!alone)
                 spgemm_dense_rows<<<dim3((unsigned)ceil_div(nd * nblk, 256)), dim3(256), 0, stream()>>>(
                     source, nd, nblk, (DenseRow *)g_sg.dense_rows.ptr, (int32_t *)g_sg.dense_before.ptr);
-#define LAUNCH_BLOCKS_C(S, COL, CRD, ALONE)                                                                \
-    do {                                                                                                   \
-        COMET_CHK(sg_allow_lds(spgemm_numeric_dense_blocks_kernel<S, COL, ALONE>, DB_LDS));                \
-        spgemm_numeric_dense_blocks_kernel<S, COL, ALONE><<<cus, block, DB_LDS, stream()>>>(               \
-            (const DenseRow *)g_sg.dense_rows.ptr, source, nd, a->crd, a->val, CRD, b->val, b->nnz,        \
-            b->sg_blkptr, nblk, tickets + 1, (int32_t *)g_sg.dense_before.ptr, rows_each, patience,        \
-            gave_up, Ccrd, Cval, reduce_op, mult_op);                                                      \
-    } while (0)
-#define LAUNCH_BLOCKS(S)                                                                                   \
-    do {                                                                                                   \
-        const bool narrow = b->sg_crd16 && getenv("COMET_HIP_SPGEMM_WIDE_COLUMNS") == nullptr;             \
-        if (narrow && alone)                                                                               \
-            LAUNCH_BLOCKS_C(S, uint16_t, b->sg_crd16, true);                                               \
-        else if (narrow)                                                                                   \
-            LAUNCH_BLOCKS_C(S, uint16_t, b->sg_crd16, false);                                              \
-        else if (alone)                                                                                    \
-            LAUNCH_BLOCKS_C(S, int32_t, b->crd, true);                                                     \
-        else                                                                                               \
-            LAUNCH_BLOCKS_C(S, int32_t, b->crd, false);                                                    \
-    } while (0)
-            if (semi) LAUNCH_BLOCKS(true); else LAUNCH_BLOCKS(false);
-#undef LAUNCH_BLOCKS_C
-#undef LAUNCH_BLOCKS
+            const auto launch = [&](auto kernel, const auto *crd, int lanes, size_t lds, unsigned a_cu) -> int {
+                // as many rows to a ticket as leave every workgroup some four of them (8 to each of 50 CUs: 78 us for a
+                // graph of 1024 vertices, the others idle)
+                const dim3 grid(a_cu * cus.x);
+                const int rows_each = (int)std::max<int64_t>(1, std::min<int64_t>(DB_ROWS, nd * nblk / (4 * (int64_t)grid.x)));
+                COMET_CHK(sg_allow_lds(kernel, lds));
+                kernel<<<grid, dim3(lanes), lds, stream()>>>(
+                    (const DenseRow *)g_sg.dense_rows.ptr, source, nd, a->crd, a->val, crd, b->val, b->nnz, b->sg_blkptr, nblk,
+                    tickets + 1, (int32_t *)g_sg.dense_before.ptr, rows_each, patience, gave_up, Ccrd, Cval, reduce_op, mult_op);
+                return COMET_HIP_OK;
+            };
+            const auto by_shape = [&](auto semiring) -> int {
+                constexpr bool S = decltype(semiring)::value;
+                if (!b->sg_crd16 || getenv("COMET_HIP_SPGEMM_WIDE_COLUMNS") != nullptr)
+                    return alone ? launch(spgemm_numeric_dense_blocks_kernel<S, int32_t, true, SG_T, 16>, b->crd, SG_T, DB_LDS<SG_T, 16>, 1)
+                                 : launch(spgemm_numeric_dense_blocks_kernel<S, int32_t, false, SG_T, 16>, b->crd, SG_T, DB_LDS<SG_T, 16>, 1);
+                if (!alone)
+                    return launch(spgemm_numeric_dense_blocks_kernel<S, uint16_t, false, SG_T, 16>, b->sg_crd16, SG_T, DB_LDS<SG_T, 16>, 1);
+#define LAUNCH_ALONE(T, ROWS, A_CU)                                                                                     \
+    return launch(spgemm_numeric_dense_blocks_kernel<S, uint16_t, true, T, ROWS>, b->sg_crd16, T, DB_LDS<T, ROWS>, A_CU)
+                if (b->ncols <= SG_NARROW && nd >= DB_TWO_ROWS * (int64_t)cus.x / 2) {
+                    if (b->ncols <= 512 * 4)
+                        LAUNCH_ALONE(512, 4, 2);
+                    if (b->ncols <= 512 * 8)
+                        LAUNCH_ALONE(512, 8, 2);
+                    LAUNCH_ALONE(512, 16, 2);
+                }
+                if (b->ncols <= SG_T * 2)
+                    LAUNCH_ALONE(SG_T, 2, 1);
+                if (b->ncols <= SG_T * 4)
+                    LAUNCH_ALONE(SG_T, 4, 1);
+                if (b->ncols <= SG_T * 8)
+                    LAUNCH_ALONE(SG_T, 8, 1);
+                LAUNCH_ALONE(SG_T, 16, 1);
+#undef LAUNCH_ALONE
+            };
+            COMET_CHK(semi ? by_shape(std::true_type()) : by_shape(std::false_type()));
             COMET_HIPCHK(hipGetLastError());
         }
     }

@@ -297,6 +297,30 @@ def test_masked_product_by_stretches_of_its_lists(semiring):
         assert np.array_equal(v, want[2]) if semiring else np.all(np.abs(v - want[2]) <= 1e-12 * np.abs(want[2]))
 
 
+@pytest.mark.parametrize("semiring", [None, ("min", "plus")])
+@pytest.mark.parametrize("rows", [40, 1152 * 3])
+@pytest.mark.parametrize("n", [600, 2048, 2049, 4096, 4097, 8192, 8193])
+def test_rows_of_many_products_of_a_matrix_within_a_block(n, rows, semiring):
+    # the columns of a wavefront by those there are, two workgroups a CU from 4.5 such rows a CU on; rows of A of fewer and
+    # of more entries than either has lanes, the first and the last column taken
+    rng = np.random.default_rng(n)
+    long_rows, short_rows = 10, 1100
+    crd = [np.unique(np.r_[0, rng.permutation(n)[:548], n - 1]) for _ in range(long_rows)]
+    crd += [np.sort(rng.permutation(n)[:4]) for _ in range(short_rows)]
+    k = len(crd)
+    b = (np.concatenate([[0], np.cumsum([len(c) for c in crd])]).astype(np.int64), np.concatenate(crd).astype(np.int32),
+         rng.integers(1, 9, sum(len(c) for c in crd)).astype(np.float64))
+    kinds = [np.array([0, 2, 3, 5, 7]), np.arange(k), np.arange(long_rows, long_rows + 513), np.arange(3)]
+    picked = [kinds[i % 40 if i % 40 < 4 else 0] for i in range(rows)]
+    a = (np.concatenate([[0], np.cumsum([len(r) for r in picked])]).astype(np.int64), np.concatenate(picked).astype(np.int32), None)
+    a = a[:2] + (rng.integers(1, 9, len(a[1])).astype(np.float64),)
+    want = orc.spgemm(*a, *b, n, **({"semiring": semiring} if semiring else {}))
+    A, B = rt.CsrMatrix.from_arrays((rows, k), *a), rt.CsrMatrix.from_arrays((k, n), *b)
+    for _ in range(2):
+        for g, w in zip(rt.spgemm(A, B, semiring=semiring).to_arrays(), want):
+            assert np.array_equal(g, w)
+
+
 @pytest.mark.parametrize("counted", [True, False])
 @pytest.mark.parametrize("rows,long_row,b_entries", [(60, 120, 900), (10_240, 120, 900), (10_242, 120, 900), (60, 2, 900),
                                                      (9000, 2, 900), (60, 120, 3), (7, 0, 900)])
