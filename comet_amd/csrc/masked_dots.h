@@ -604,9 +604,10 @@ static int pair_dot_values(Csr *a, Csr *b, Csr *m, int64_t rb, int64_t re, doubl
     const bool beside = nheavy > 0 && nlight > 0 && plan->side[0].pairs + plan->side[1].pairs >= PAIR_BESIDE;
     if (beside)
         COMET_CHK(aux_fork());
-    unsigned long long *tickets = nullptr;
+    unsigned long long *kept = nullptr, *tickets = nullptr;
     if (nheavy > 0) {
-        COMET_CHK(pair_tickets(&tickets));
+        COMET_CHK(pair_tickets(&kept));
+        tickets = kept;
         const bool big = dot_table_big(a->ncols);
         const int words = dot_table_words(a->ncols);
         const int before_at = (int)ceil_div(a->ncols, 256) * 8;
@@ -653,8 +654,7 @@ static int pair_dot_values(Csr *a, Csr *b, Csr *m, int64_t rb, int64_t re, doubl
     }
     if (beside)
         COMET_CHK(aux_join());
-    COMET_HIPCHK(hipGetLastError());
-    return COMET_HIP_OK;
+    return pair_launched(kept);
 }
 
 // ---------------------------------------------------------------------------

@@ -1067,11 +1067,12 @@ static int pair_tickets(unsigned long long **tickets)
     return COMET_HIP_OK;
 }
 
-// After the launches of a sum of hits: one that failed leaves the others' hits behind.
+// After the launches of a call: one that failed leaves the tickets that the others drew, or their hits, behind (null: it has
+// drawn none).
 static int pair_launched(unsigned long long *tickets)
 {
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess)
+    if (e != hipSuccess && tickets)
         (void)hipMemsetAsync(tickets, 0, PAIR_WORDS * sizeof *tickets, stream());
     COMET_HIPCHK(e);
     return COMET_HIP_OK;

@@ -1,6 +1,6 @@
 // A stand-in for the HIP runtime, for checks of what the library does on the host: two devices that exist in name only,
 // memory that is counted, streams and events that know their device, and one kernel, the one that moves a group of a
-// transfer.  Its functions take the place of the real ones because the program that is asked for a symbol first is the
+// transfer (a scenario that asks for them has the others too, which do what `pretend` says).  Its functions take the place of the real ones because the program that is asked for a symbol first is the
 // executable.  Each scenario of main() prints what went wrong and returns non-zero.
 #include <dlfcn.h>
 #include <errno.h>
@@ -62,6 +62,7 @@ bool on_device(const char *p, size_t bytes, int device)
 }  // namespace
 
 static int threads_left = 1 << 20;          // how many more the system has
+static bool (*pretend)(const std::string &kernel, void **args) = nullptr;          // false: the launch is refused
 
 extern "C" {
 
@@ -104,6 +105,8 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *p, int)
 }
 hipError_t hipGetSymbolAddress(void **p, const void *) { static char room[16 << 20]; *p = room; return hipSuccess; }
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+int hipGetStreamDeviceId(hipStream_t s) { return stream_of(s)->device; }
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size_t) { *n = 1; return hipSuccess; }
 const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "fake error"; }
 hipError_t hipGetLastError(void) { const hipError_t e = last; last = hipSuccess; return e; }
 
@@ -196,6 +199,8 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
     const std::string &name = kernels()[f];
     if (!stream_of(s)->live || stream_of(s)->device != current)
         return fail(hipErrorInvalidHandle, "launch on a stream of another device, or one that was destroyed");
+    if (name.find("move_segments") == std::string::npos && pretend)
+        return pretend(name, args) ? hipSuccess : fail(hipErrorOutOfMemory, "a launch is refused");
     if (name.find("move_segments") == std::string::npos)
         return fail(hipErrorInvalidValue, ("no such kernel here: " + name).c_str());
     struct Segments { char *dev[12]; uint32_t at[12], bytes[12]; int n; };
@@ -391,6 +396,59 @@ static int few_threads(int n)
     return 0;
 }
 
+// a masked product of which one row is a workgroup's, drawn by ticket, and one a wavefront's, whose launch is refused: the
+// tickets are as they were for the next product
+static unsigned long long *tickets_drawn = nullptr;
+static bool refuse_light = false;
+static bool masked_product_kernels(const std::string &kernel, void **args)
+{
+    const auto is = [&](const char *name) { return kernel.find(name) != std::string::npos; };
+    const auto at = [&](int i) { return *static_cast<int64_t **>(args[i]); };
+    if (is("coo_flag"))
+        std::fill_n(at(4), *static_cast<int64_t *>(args[0]), 1);
+    if (is("scan_one")) {
+        int64_t sum = 0;
+        for (int i = 0; i < *static_cast<int *>(args[1]); ++i) {
+            at(2)[i] = sum;
+            sum += at(0)[i];
+        }
+        at(2)[*static_cast<int *>(args[1])] = sum;
+    }
+    if (is("pair_parts")) {
+        at(10)[0] = 1;
+        at(10)[1] = 1ll << 32;
+    }
+    if (is("pair_dot_heavy")) {
+        tickets_drawn = *static_cast<unsigned long long **>(args[6]);
+        tickets_drawn[0] += 2;
+    }
+    if (is("pair_dot_light")) {
+        unsigned long long *cleared = *static_cast<unsigned long long **>(args[2]);
+        if (cleared && !refuse_light)
+            cleared[0] = 0;
+        return !refuse_light;
+    }
+    return true;
+}
+static int refused_launch()
+{
+    REQUIRE(comet_hip_init(0) == 0);
+    pretend = masked_product_kernels;
+    const int64_t pos[] = {0, 3, 6, 9}, crd[] = {0, 1, 2, 0, 1, 2, 0, 1, 2};
+    const double val[] = {1, 2, 3, 4, 5, 6, 7, 8, 9};
+    const int64_t a = comet_hip_csr_upload_i64(3, 3, pos, crd, val);
+    REQUIRE(a != 0);
+    for (bool refused : {false, true, false}) {
+        refuse_light = refused;
+        tickets_drawn = nullptr;
+        const int64_t c = comet_hip_spgemm_csr(a, a, a);
+        REQUIRE(tickets_drawn && (c == 0) == refused);
+        REQUIRE(tickets_drawn[0] == 0);
+        REQUIRE(refused || comet_hip_csr_destroy(c) == 0);
+    }
+    return 0;
+}
+
 int main(int, char **argv)
 {
     const std::string what = argv[1];
@@ -410,6 +468,8 @@ int main(int, char **argv)
         return few_threads(0);
     if (what == "two_threads")
         return few_threads(2);
+    if (what == "refused_launch")
+        return refused_launch();
     fprintf(stderr, "no scenario %s\n", argv[1]);
     return 2;
 }

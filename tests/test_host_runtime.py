@@ -24,7 +24,7 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("scenario", ["another_device", "whole_device", "given_back", "block_of_another_device",
-                                      "memory_while_another_waits", "waiting_is_cheap", "no_threads", "two_threads"])
+                                      "memory_while_another_waits", "waiting_is_cheap", "no_threads", "two_threads", "refused_launch"])
 def test_host_side(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
