@@ -1327,7 +1327,7 @@ static int spmm_long_rows(Csr *a)
 static bool spmm_by_columns(Csr *a, int64_t K, SpmmShape *h)
 {
     const int64_t bytes = a->ncols * K * 8, most = K < 16 ? INT64_MAX : (K > 32 ? 56 : 80) << 20;
-    if (bytes < SPMM_ORDER_B || bytes > most || a->rowmap || getenv("COMET_HIP_SPMM_GROUPS") || getenv("COMET_HIP_SPMM_MEDIUM"))
+    if (a->nnz == 0 || bytes < SPMM_ORDER_B || bytes > most || a->rowmap || getenv("COMET_HIP_SPMM_GROUPS") || getenv("COMET_HIP_SPMM_MEDIUM"))
         return false;           // the two switches shape the sweep, and ask for it
     SpmmShape cut = *h;
     if (cut.len == SPMM_CH && bytes > (K > 16 ? 28 << 20 : 48 << 20)) {

@@ -480,6 +480,20 @@ def test_spmm_chunks_by_columns(nlong, ncols, K, accumulate, monkeypatch):
     assert sorted_at == [False, True, False]
 
 
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("K", [8, 33])
+def test_spmm_of_a_matrix_without_entries_again_and_again(K, accumulate, monkeypatch):
+    # with a B of the size for which chunks go by columns: there are none, and no call leaves an error behind
+    monkeypatch.delenv("COMET_HIP_PLAN_AT_ONCE")
+    nrows, ncols = 70, 40_000
+    A = rt.CsrMatrix.from_arrays((nrows, ncols), np.zeros(nrows + 1, np.int64), np.zeros(0, np.int64), np.zeros(0))
+    C0, dB = np.random.default_rng(K).uniform(-1, 1, (nrows, K)), rt.DeviceArray((ncols, K), zero=True)
+    for _ in range(3):
+        dC = rt.DeviceArray.from_numpy(C0)
+        rt.spmm(A, dB, dC, accumulate=accumulate)
+        assert np.array_equal(dC.to_numpy(), C0 if accumulate else np.zeros((nrows, K)))
+
+
 @pytest.mark.parametrize("K", [1, 2, 3, 5, 16, 17, 31, 32, 33, 63, 64, 65, 66, 130])
 @pytest.mark.parametrize("nnz", [1, 15, 17, 63, 65, 4097])
 def test_sddmm_of_every_tile_and_width(nnz, K):
