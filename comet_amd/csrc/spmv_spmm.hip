@@ -797,7 +797,6 @@ constexpr int spmm_hrows(int g) { return g * (SPMM_HW - 1) * SPMM_HR; }    // lo
 constexpr int SPMM_MED_MIN_LEN = COMET_SPMM_MED_MIN;   // such a row has at least this many nonzeros
 constexpr int SPMM_MSLOTS = 287;                        // sums a workgroup keeps in LDS, beside the entries of its lists (SWEEP_LDS)
 constexpr int SPMM_HEAVY_MIN_LEN = COMET_SPMM_HEAVY_MIN;              // a long row has at least this many nonzeros
-constexpr int64_t SPMM_SWEEP_NNZ = 1 << 19;             // a matrix of fewer nonzeros is not swept
 constexpr int64_t SPMM_UNEVEN_SWEEP = 24 << 20;         // bytes of B from which on rows of any alignment are swept
 constexpr int SPMM_HCB = 32;                         // column blocks a wavefront's list is cut into
 
@@ -1327,8 +1326,9 @@ static int spmm_long_rows(Csr *a)
 static bool spmm_by_columns(Csr *a, int64_t K, SpmmShape *h)
 {
     const int64_t bytes = a->ncols * K * 8, most = K < 16 ? INT64_MAX : (K > 32 ? 56 : 80) << 20;
-    if (a->nnz == 0 || bytes < SPMM_ORDER_B || bytes > most || a->rowmap || getenv("COMET_HIP_SPMM_GROUPS") || getenv("COMET_HIP_SPMM_MEDIUM"))
-        return false;           // the two switches shape the sweep, and ask for it
+    if (a->nnz == 0 || bytes < SPMM_ORDER_B || bytes > most || a->rowmap || getenv("COMET_HIP_SPMM_NO_COLUMNS") ||
+        getenv("COMET_HIP_SPMM_GROUPS") || getenv("COMET_HIP_SPMM_MEDIUM"))
+        return false;           // the last two shape the sweep, and ask for it
     SpmmShape cut = *h;
     if (cut.len == SPMM_CH && bytes > (K > 16 ? 28 << 20 : 48 << 20)) {
         cut.len = SPMM_CH / 2;
@@ -1630,7 +1630,7 @@ static int spmm_heavy_plan(Csr *a, bool even, int64_t K)
     if (a->heavy_state != 0)
         return COMET_HIP_OK;
     a->heavy_state = 1;
-    if (a->nnz < SPMM_SWEEP_NNZ || a->nnz >= (1ll << 32) || ceil_div(a->ncols, 8) >= (1ll << SPMM_HCOLB))
+    if (a->nnz < (1 << 19) || a->nnz >= (1ll << 32) || ceil_div(a->ncols, 8) >= (1ll << SPMM_HCOLB))
         return COMET_HIP_OK;        // a list entry has SPMM_HCOLB bits for the column inside an XCD's eighth
     const int64_t n = a->nrows;
     // The long rows may hold too little for the sweep: looked at before the row pointers are fetched and gone through here
@@ -1926,7 +1926,7 @@ static int spmm_heavy_plan(Csr *a, bool even, int64_t K)
 using namespace comet;
 
 static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate, const SpmmShape &h,
-                       bool ordered = false, const char *name = "spmm_csr_nnzsplit", hipStream_t on = nullptr);
+                       bool ordered = false, hipStream_t on = nullptr);
 static int spmv_run(Csr *a, int64_t x_dptr, int64_t y_dptr, int accumulate);
 static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dptr, int64_t ldc, int accumulate);
 
@@ -2064,11 +2064,8 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
     const bool plan_now = a->spmm_uses > 0 || plan_at_once();
     a->spmm_uses = a->spmm_uses < 2 ? a->spmm_uses + 1 : 2;
     SpmmShape h = spmm_shape(a, K);
-    if (plan_now && spmm_by_columns(a, K, &h)) {
-        // what would be swept with the sums in registers is a sweep in this form too, and listed as one by the profile
-        const bool sweep = sweep_fits && a->nnz >= SPMM_SWEEP_NNZ && a->long_nnz[0] * 4 >= a->nnz && (even || sweep_uneven(a, K));
-        return spmm_chunks(a, K, B, ldb, C, ldc, accumulate, h, true, sweep ? "spmm_heavy_sweep" : "spmm_csr_nnzsplit");
-    }
+    if (plan_now && spmm_by_columns(a, K, &h))
+        return spmm_chunks(a, K, B, ldb, C, ldc, accumulate, h, true);
     if (sweep_fits && plan_now && a->heavy_state == 0)
         (void)plan_made([&] { return spmm_heavy_plan(a, even, K); });          // or the chunk kernel goes on taking all rows
     if (a->heavy_state != 2 || !sweep_fits)
@@ -2117,7 +2114,7 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
             COMET_CHK(accumulate ? launch(spmm_heavy_sweep<false, true>) : launch(spmm_heavy_sweep<false, false>));
     }
     if (overlap) {      // the rows in between, on the CUs the sweep leaves free
-        COMET_CHK(spmm_chunks(a->light, K, B, ldb, C, ldc, accumulate, light, false, "spmm_csr_nnzsplit", aux_stream()));
+        COMET_CHK(spmm_chunks(a->light, K, B, ldb, C, ldc, accumulate, light, false, aux_stream()));
         COMET_CHK(aux_join());
     }
     {
@@ -2138,15 +2135,15 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
 
 // The chunk kernel: the row of every grain'th nonzero in chunk_row, chunks of h.len nonzeros (a multiple of grain), two
 // slots for each of them and column tile in carry and a zero in arrived; order: the chunks in the order they are taken in, or
-// null.  name: what events are recorded under (null: none, where the stream is being captured).
+// null.  timed: events may be recorded (not where the stream is being captured).
 static void spmm_chunk_launch(const Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate,
                               const int32_t *chunk_row, int grain, const SpmmShape &h, const uint32_t *order, double *carry,
-                              unsigned *arrived, hipStream_t on, const char *name)
+                              unsigned *arrived, hipStream_t on, bool timed)
 {
     const int64_t wide = order ? 8 * ceil_div(ceil_div(h.chunks, 8), SPMM_WAVES) : ceil_div(h.chunks, SPMM_WAVES);
     const dim3 grid((unsigned)wide, (unsigned)h.tiles), block(SPMM_WAVES * 64);
     const auto split = [&](auto kernel) {
-        std::unique_ptr<KernelTimer> t(name ? new KernelTimer(name, on) : nullptr);
+        std::unique_ptr<KernelTimer> t(timed ? new KernelTimer("spmm_csr_nnzsplit", on) : nullptr);
         kernel<<<grid, block, 0, on>>>(a->pos, a->crd, a->val, a->nnz, a->nrows, chunk_row, grain, h.len, h.chunks, order, B, ldb, C,
                                        ldc, K, h.cols, carry, arrived, a->rowmap);
     };
@@ -2161,7 +2158,7 @@ static void spmm_chunk_launch(const Csr *a, int64_t K, const double *B, int64_t 
 
 // ordered: h is how spmm_by_columns cut the product
 static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *C, int64_t ldc, int accumulate, const SpmmShape &h,
-                       bool ordered, const char *name, hipStream_t on)
+                       bool ordered, hipStream_t on)
 {
     if (!on)
         on = stream();
@@ -2178,7 +2175,7 @@ static int spmm_chunks(Csr *a, int64_t K, const double *B, int64_t ldb, double *
     COMET_CHK(spmm_chunk_scratch(h));
     spmm_chunk_launch(a, K, B, ldb, C, ldc, accumulate, a->spmm_chunk_row, SPMM_GRAIN, h,
                       ordered ? a->spmm_order[h.len / SPMM_GRAIN / 2] : nullptr, (double *)g_spmm_carry.ptr,
-                      (unsigned *)g_spmm_arrived.ptr, on, name);
+                      (unsigned *)g_spmm_arrived.ptr, on, true);
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
 }
@@ -2317,7 +2314,7 @@ extern "C" int comet_hip_spmm_csr_f64_noalloc(int64_t csr, int64_t K, int64_t b_
     unsigned *arrived = reinterpret_cast<unsigned *>(scratch + SPMM_STATIC_TABLE_BYTES + SPMM_STATIC_CARRY_BYTES);
     spmm_chunk_rows<<<dim3((unsigned)ceil_div(h.chunks, 256)), dim3(256), 0, on>>>(a->pos, a->nrows, h.chunks, h.len, chunk_row, arrived,
                                                                                    h.tiles * h.chunks);
-    spmm_chunk_launch(a, K, (const double *)b_dptr, ldb, C, ldc, accumulate, chunk_row, h.len, h, nullptr, carry, arrived, on, nullptr);
+    spmm_chunk_launch(a, K, (const double *)b_dptr, ldb, C, ldc, accumulate, chunk_row, h.len, h, nullptr, carry, arrived, on, false);
     COMET_HIPCHK(hipGetLastError());
     return COMET_HIP_OK;
 }

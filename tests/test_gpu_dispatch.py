@@ -480,6 +480,29 @@ def test_spmm_chunks_by_columns(nlong, ncols, K, accumulate, monkeypatch):
     assert sorted_at == [False, True, False]
 
 
+def test_spmm_launches_are_listed_by_the_kernel_that_runs(monkeypatch):
+    # a first product and chunks by columns: the chunk kernel; a B beyond those, or the switch that turns them off: the sweep
+    monkeypatch.delenv("COMET_HIP_PLAN_AT_ONCE")
+    n = 120_000
+    pos, crd, val = gen.zipf_csr(n=n, mean=16.0, cap=4096, seed=7)
+    A, B = rt.CsrMatrix.from_arrays((n, n), pos, crd, val), np.random.default_rng(3).uniform(-1, 1, (n, 64))
+    for K, columns, swept in [(32, True, False), (32, True, False), (64, True, True), (32, True, False), (32, False, True)]:
+        if not columns:
+            monkeypatch.setenv("COMET_HIP_SPMM_NO_COLUMNS", "1")
+        b = np.ascontiguousarray(B[:, :K])
+        dB, dC = rt.DeviceArray.from_numpy(b), rt.DeviceArray((n, K))
+        rt.profile_reset()
+        rt.profile_enable(True)
+        rt.spmm(A, dB, dC, accumulate=False)
+        rt.sync()
+        rep = rt.profile_report()
+        rt.profile_enable(False)
+        assert ("spmm_heavy_sweep" in rep) == ("spmm_heavy_combine" in rep) == swept, (K, columns, sorted(rep))
+        assert swept or "spmm_csr_nnzsplit" in rep, (K, columns, sorted(rep))
+        bound = orc.spmm(pos, crd, np.abs(val), np.abs(b))
+        assert np.all(np.abs(dC.to_numpy() - orc.spmm(pos, crd, val, b)) <= 1e-12 * bound)
+
+
 @pytest.mark.parametrize("accumulate", [False, True])
 @pytest.mark.parametrize("K", [8, 33])
 def test_spmm_of_a_matrix_without_entries_again_and_again(K, accumulate, monkeypatch):
@@ -817,6 +840,7 @@ def test_spgemm_of_one_entry_and_a_row_with_repeated_columns(semiring, monkeypat
 def test_spmm_sweep_of_rows_that_are_no_multiple_of_16_bytes(K, ldb, ldc, shift, accumulate, medium, monkeypatch):
     # odd widths, odd leading dimensions and addresses 8 bytes off, where B is large enough for the sweep; the last column
     # is a lane's own and its neighbour's; nothing outside C's columns is written, B's last row is the end of its array
+    monkeypatch.setenv("COMET_HIP_SPMM_NO_COLUMNS", "1")
     if medium:
         monkeypatch.setenv("COMET_HIP_SPMM_MEDIUM", "1")
     n = 60_000
@@ -850,8 +874,9 @@ def test_spmm_sweep_of_rows_that_are_no_multiple_of_16_bytes(K, ldb, ldc, shift,
 
 @pytest.mark.parametrize("mean,widths", [(4.0, {17: False, 33: False, 63: False, 64: True}), (8.0, {17: False, 33: True, 63: True, 64: True}),
                                          (16.0, {17: True, 63: True, 64: True})])
-def test_spmm_sweeps_odd_widths_where_long_rows_hold_the_matrix(mean, widths):
+def test_spmm_sweeps_odd_widths_where_long_rows_hold_the_matrix(mean, widths, monkeypatch):
     # the plan of a matrix is made by the first call it is right for, whatever calls came before
+    monkeypatch.setenv("COMET_HIP_SPMM_NO_COLUMNS", "1")
     n = 200_000
     pos, crd, val = gen.zipf_csr(n=n, mean=mean, cap=4096, seed=7)
     A = rt.CsrMatrix.from_arrays((n, n), pos, crd, val)
@@ -1026,10 +1051,13 @@ def test_a_refused_request_fails_its_own_call_only():
     assert rt.spgemm(A, A).nnz == rt.spgemm(B, A).nnz > 0
 
 
-@pytest.mark.parametrize("op,K", [("spmm", 64), ("spmm", 81), ("spmv", 1), ("sddmm", 40)])
+@pytest.mark.parametrize("op,K", [("spmm", 64), ("spmm", 81), ("sweep", 64), ("sweep", 81), ("spmv", 1), ("sddmm", 40)])
 def test_a_plan_without_memory_is_done_without(op, K, monkeypatch):
     # the second call on a handle makes its plan; where that finds no memory the call goes the way of the first
     monkeypatch.delenv("COMET_HIP_PLAN_AT_ONCE")
+    if op == "sweep":                     # the long rows' lists in place of the chunks by columns
+        monkeypatch.setenv("COMET_HIP_SPMM_NO_COLUMNS", "1")
+        op = "spmm"
     n = 700_001 if op == "spmv" else 40_001
     pos, crd, val = (gen.poisson_csr(n=n, mean=3.0, seed=5) if op == "spmv" else gen.zipf_csr(n=n, mean=16.0, cap=4096, seed=7))
     rng = np.random.default_rng(2)
@@ -1064,8 +1092,9 @@ def test_a_plan_without_memory_is_done_without(op, K, monkeypatch):
         assert np.all(np.abs(call(A) - want) <= 1e-12 * bound), k
 
 
-def test_a_sweep_without_room_for_its_sums_is_done_without():
+def test_a_sweep_without_room_for_its_sums_is_done_without(monkeypatch):
     # a planned matrix meets a wider B than any before: scratch for the sums, and for the chunk kernel, is refused in turn
+    monkeypatch.setenv("COMET_HIP_SPMM_NO_COLUMNS", "1")          # the first product plans the sweep
     n = 40_001
     pos, crd, val = gen.zipf_csr(n=n, mean=16.0, cap=4096, seed=7)
     A = rt.CsrMatrix.from_arrays((n, n), pos, crd, val)

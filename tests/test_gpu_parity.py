@@ -1409,6 +1409,7 @@ def _sweep_check(pos, crd, val, B, C0=None, ld_pad=0):
 @pytest.mark.parametrize("K,acc,pad", [(64, False, 0), (64, True, 0), (20, False, 4), (100, True, 6), (64, False, 3),
                                         (33, True, 0)])
 def test_spmm_long_rows_sweep(K, acc, pad, medium, monkeypatch):
+    monkeypatch.setenv("COMET_HIP_SPMM_NO_COLUMNS", "1")          # a B of this size would go through the chunks by columns
     if medium:      # rows of 32..127 nonzeros ride on the sweep too, their sums in LDS
         monkeypatch.setenv("COMET_HIP_SPMM_MEDIUM", "1")
     pos, crd, val = gen.zipf_csr(n=40_000, mean=16.0, cap=4096, seed=7)
@@ -1423,6 +1424,7 @@ def test_spmm_plan_waits_for_the_second_product(monkeypatch):
     # The plan of a matrix costs some forty products, so a matrix multiplied once (what a .ta program does) goes
     # through the chunk kernel whole; the plan is made when the same handle is multiplied again, and kept.
     monkeypatch.delenv("COMET_HIP_PLAN_AT_ONCE")
+    monkeypatch.setenv("COMET_HIP_SPMM_NO_COLUMNS", "1")
     pos, crd, val = gen.zipf_csr(n=40_000, mean=16.0, cap=4096, seed=7)
     assert len(crd) >= 1 << 19
     B = gen.dense((40_000, 64), seed=8)
@@ -1625,9 +1627,12 @@ def test_wrapped_device_arrays_are_checked():
     assert L.comet_hip_csr_destroy(h) == 0
 
 
-def test_wrapped_arrays_changed_in_place_need_invalidate():
+@pytest.mark.parametrize("swept", [False, True])
+def test_wrapped_arrays_changed_in_place_need_invalidate(swept, monkeypatch):
     """A handle over caller-owned device arrays caches re-ordered copies; after the caller rewrites the values
     comet_hip_csr_invalidate makes every kernel see them."""
+    if swept:
+        monkeypatch.setenv("COMET_HIP_SPMM_NO_COLUMNS", "1")
     pos, crd, val = gen.zipf_csr(n=40_000, mean=16.0, cap=4096, seed=11)      # large enough for every plan
     n, nnz = 40_000, len(crd)
     dpos = rt.DeviceArray.from_numpy(pos.astype(np.int64))
@@ -1638,7 +1643,10 @@ def test_wrapped_arrays_changed_in_place_need_invalidate():
     B = gen.dense((n, 32), seed=12)
     x = gen.dense(n, seed=13)
     dB, dx = rt.DeviceArray.from_numpy(B), rt.DeviceArray.from_numpy(x)
-    first = rt.spmm(A, dB).to_numpy()
+    out = []
+    rep = _kernels_of(lambda: out.append(rt.spmm(A, dB).to_numpy()))
+    assert ("spmm_heavy_sweep" in rep) == swept, sorted(rep)
+    first = out[0]
     y1 = rt.spmv(A, dx).to_numpy()
     z1 = rt.vecmat(dx, A).to_numpy()
     val2 = -2.0 * val
