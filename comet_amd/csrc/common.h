@@ -167,6 +167,7 @@ struct Csr {
     uint32_t *spmm_order[3] = {};            // the chunks by columns, for chunks of 64, 128 and 256
     // entries of the rows of 128, 256, 512 and 1024 entries and more; -1: not looked at
     int64_t long_nnz[SPMM_LONG_KINDS] = {-1, -1, -1, -1};
+    int crowded_columns = -1;                // whether few columns hold much of the matrix; -1: not looked at
     // SpMV plan: the matrix re-stored as `spmv_nb` column blocks (block-major copy of crd/val, one row
     // pointer array per block) so that the slice of x a pass gathers from stays inside one L2.
     // spmv_nb == 0: not decided yet; 1: run on the original arrays.

@@ -444,6 +444,7 @@ static void csr_drop_plans(Csr *c)
     c->sddmm_tile_state = 0;
     c->heavy_nnz = -1;
     c->long_nnz[0] = -1;
+    c->crowded_columns = -1;
     c->heavy_rows = 0;
     (void)dev_free(c->spmm_chunk_row);
     c->spmm_chunk_row = nullptr;

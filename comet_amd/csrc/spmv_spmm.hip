@@ -1228,10 +1228,10 @@ static int spmm_chunk_scratch(const SpmmShape &h)
 // somewhere else.  So, from a matrix's second product on, the chunks are taken in
 // the order of their columns, an eighth of them by every XCD: an L2 then sees an
 // eighth of B, ascending, in place of all of it (workgroup w runs on XCD w % 8).
-// The sums do not change: pieces of rows are added in the order of the chunks'
-// numbers.  It pays where rows of four chunks and more hold half of the matrix;
-// graphs whose columns are as uneven as their rows (R-MAT scale 13 to 18: 7 to 48 %
-// in such rows) have the rows of B that count in every L2 as it is, and lose up to 15 %.
+// Pieces of rows are added in the order of the chunks' numbers, so the sums are what they are as stored, unless the chunks are
+// shorter (below): a long row is cut in more places then, and its rounding may differ from that of the first product.
+// It pays where rows of four chunks and more hold half of the matrix and few columns do not (SPMM_CROWDED): graphs
+// whose columns are as uneven as their rows have the rows of B that count in every L2 as it is.
 // us, zipf, 16 nonzeros a row, as stored / by columns: 30000 rows K = 64 51 / 38, 60001 rows K = 33 61 / 45, 250000 rows
 // K = 15 146 / 99, 500000 rows K = 3 153 / 121, K = 15 298 / 182, 1000000 rows K = 8 343 / 249.
 // Chunks of half the length keep a window of a larger B in the L2: 120000 rows K = 33 83 / 75, 250000 rows K = 32 131 / 105;
@@ -1322,9 +1322,70 @@ static int spmm_long_rows(Csr *a)
     return COMET_HIP_OK;
 }
 
-// Whether a product of a matrix that has been multiplied before goes through its chunks by columns (*h: cut as it is then).
-static bool spmm_by_columns(Csr *a, int64_t K, SpmmShape *h)
+// Columns that hold four times what they would if all held the same.  Where such columns hold this share of the entries, chunks
+// stay as they are stored.  Share, and us as stored / by columns: columns n * u^p of a random u, rows as zipf, 60000 rows K = 33
+// p = 2 (0.10) 54.8 / 44.7, p = 4 (0.30) 44.0 / 39.5, p = 6 (0.38) 37.9 / 37.2, the same columns at random places 38.9 / 35.1,
+// 250000 rows K = 21 p = 6 (0.42) 113.9 / 91.2; R-MAT scale 13, 32 edges a vertex (0.50) K = 17 22.8 / 24.5, K = 32 24.8 / 27.1,
+// 18 and 16 (0.73) K = 17 235 / 253, K = 31 276 / 283, 17 and 32 (0.75) K = 31 184 / 219, K = 48 248 / 276, its vertices at random
+// places K = 33 188 / 202.  The sweep is no way out for these either: 18 and 16 K = 24 238 / 526 swept, 17 and 32 K = 32 176 / 459.
+constexpr double SPMM_CROWDED = 0.46;
+constexpr int64_t SPMM_COLUMN_SAMPLE = 1 << 19;           // entries that are looked at, about
+
+// count[j] += samples in column j: one at a random place of every `every` entries (at the same place of each it might be of
+// every row the first)
+__global__ __launch_bounds__(256) void spmm_column_counts(int64_t samples, int64_t every, int64_t nnz, const int32_t *__restrict__ crd,
+                                                          uint32_t *__restrict__ count)
 {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= samples)
+        return;
+    const int64_t p = i * every + (int64_t)((uint32_t)i * 0x9E3779B1u >> 8) % every;
+    atomicAdd(&count[crd[p < nnz ? p : nnz - 1]], 1u);
+}
+
+// *held += samples in columns of `least` and more
+__global__ __launch_bounds__(256) void spmm_column_share(int64_t ncols, const uint32_t *__restrict__ count, uint32_t least,
+                                                         unsigned long long *__restrict__ held)
+{
+    int mine = 0;          // all samples fit
+    for (int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x; j < ncols; j += (int64_t)gridDim.x * 256)
+        mine += count[j] >= least ? (int)count[j] : 0;
+    for (int d = 32; d > 0; d >>= 1)
+        mine += __shfl_down(mine, d, 64);
+    if ((threadIdx.x & 63) == 0 && mine > 0)
+        atomicAdd(held, (unsigned long long)mine);
+}
+
+// a->crowded_columns: asked of the device once
+static int spmm_crowded(Csr *a)
+{
+    if (a->crowded_columns >= 0)
+        return COMET_HIP_OK;
+    const int64_t every = ceil_div(a->nnz, SPMM_COLUMN_SAMPLE), samples = ceil_div(a->nnz, every);
+    unsigned long long *word = nullptr;
+    COMET_CHK(mailbox((void **)&word));
+    const size_t bytes = sizeof *word + sizeof(uint32_t) * (size_t)a->ncols;
+    COMET_CHK(g_long_entries.ensure(bytes, false));
+    unsigned long long *held = (unsigned long long *)g_long_entries.ptr;
+    uint32_t *count = (uint32_t *)(held + 1);
+    COMET_HIPCHK(hipMemsetAsync(held, 0, bytes, stream()));
+    spmm_column_counts<<<dim3((unsigned)ceil_div(samples, 256)), dim3(256), 0, stream()>>>(samples, every, a->nnz, a->crd, count);
+    // (a column that happens to be seen a few times is not a crowded one)
+    const uint32_t least = (uint32_t)std::max<int64_t>(8, ceil_div(4 * samples, a->ncols));
+    spmm_column_share<<<dim3((unsigned)std::min<int64_t>(ceil_div(a->ncols, 256), 2 * (int64_t)num_cus())), dim3(256), 0, stream()>>>(
+        a->ncols, count, least, held);
+    COMET_HIPCHK(hipGetLastError());
+    COMET_HIPCHK(hipMemcpyAsync(word, held, sizeof *word, hipMemcpyDeviceToHost, stream()));
+    COMET_CHK(stream_wait());
+    a->crowded_columns = (double)*(volatile unsigned long long *)word > SPMM_CROWDED * (double)samples;
+    return COMET_HIP_OK;
+}
+
+// Whether a product of a matrix that has been multiplied before goes through its chunks by columns, *h as it is cut then.
+// *stored: it does not, because of its columns, and is not to be swept.
+static bool spmm_by_columns(Csr *a, int64_t K, SpmmShape *h, bool *stored)
+{
+    *stored = false;
     const int64_t bytes = a->ncols * K * 8, most = K < 16 ? INT64_MAX : (K > 32 ? 56 : 80) << 20;
     if (a->nnz == 0 || bytes < SPMM_ORDER_B || bytes > most || a->rowmap || getenv("COMET_HIP_SPMM_NO_COLUMNS") ||
         getenv("COMET_HIP_SPMM_GROUPS") || getenv("COMET_HIP_SPMM_MEDIUM"))
@@ -1336,7 +1397,10 @@ static bool spmm_by_columns(Csr *a, int64_t K, SpmmShape *h)
     }
     if (cut.chunks >= 1ll << 31 || (a->long_nnz[0] < 0 && !plan_made([&] { return spmm_long_rows(a); })))
         return false;
-    if (a->long_nnz[1 + cut.len / SPMM_GRAIN / 2] * 2 < a->nnz || !plan_made([&] { return spmm_order(a, cut); }))
+    if (a->long_nnz[1 + cut.len / SPMM_GRAIN / 2] * 2 < a->nnz || (a->crowded_columns < 0 && !plan_made([&] { return spmm_crowded(a); })))
+        return false;
+    *stored = a->crowded_columns == 1;
+    if (*stored || !plan_made([&] { return spmm_order(a, cut); }))
         return false;
     *h = cut;
     return true;
@@ -2064,8 +2128,10 @@ static int spmm_run(Csr *a, int64_t K, int64_t b_dptr, int64_t ldb, int64_t c_dp
     const bool plan_now = a->spmm_uses > 0 || plan_at_once();
     a->spmm_uses = a->spmm_uses < 2 ? a->spmm_uses + 1 : 2;
     SpmmShape h = spmm_shape(a, K);
-    if (plan_now && spmm_by_columns(a, K, &h))
-        return spmm_chunks(a, K, B, ldb, C, ldc, accumulate, h, true);
+    bool stored = false;
+    const bool by_columns = plan_now && spmm_by_columns(a, K, &h, &stored);
+    if (by_columns || stored)
+        return spmm_chunks(a, K, B, ldb, C, ldc, accumulate, h, by_columns);
     if (sweep_fits && plan_now && a->heavy_state == 0)
         (void)plan_made([&] { return spmm_heavy_plan(a, even, K); });          // or the chunk kernel goes on taking all rows
     if (a->heavy_state != 2 || !sweep_fits)

@@ -480,6 +480,48 @@ def test_spmm_chunks_by_columns(nlong, ncols, K, accumulate, monkeypatch):
     assert sorted_at == [False, True, False]
 
 
+@pytest.mark.parametrize("columns,K,ordered", [("graph", 17, False), ("graph", 32, False), ("graph at random places", 17, False),
+                                               ("uniform", 17, True), ("uneven", 32, True), ("one", 32, False), ("far apart", 14, True)])
+def test_spmm_chunks_go_by_columns_unless_few_hold_much_of_the_matrix(columns, K, ordered, monkeypatch):
+    # rows of four chunks hold half of each of these; where the columns are as uneven, the chunks stay as stored
+    monkeypatch.delenv("COMET_HIP_PLAN_AT_ONCE")
+    rng = np.random.default_rng(8)
+    if columns.startswith("graph"):
+        n = 1 << 13
+        pos, crd, val = gen.rmat_symmetric_csr(scale=13, edge_factor=32, seed=2)
+        if columns != "graph":
+            place = rng.permutation(n)
+            rows, cols = place[np.repeat(np.arange(n), np.diff(pos))], place[crd]
+            order = np.lexsort((cols, rows))
+            crd, pos = cols[order], np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))])
+        ncols = n
+    else:
+        n, ncols = 3000, 500_000 if columns == "far apart" else 20_000
+        lens = np.where(np.arange(n) % 3 == 0, 1200, 9)
+        u = rng.random(lens.sum()) ** (4 if columns == "uneven" else 1)
+        rows, cols = np.repeat(np.arange(n), lens), (u * ncols).astype(np.int64)
+        if columns == "one":              # half of the entries in columns that are in every row
+            cols[::2] = np.arange(len(cols[::2])) % 700
+        key = np.unique(rows * ncols + cols)
+        crd, pos = key % ncols, np.concatenate([[0], np.cumsum(np.bincount(key // ncols, minlength=n))])
+        val = rng.uniform(-1, 1, len(crd))
+    lens, four_chunks = np.diff(pos), {"graph": 256, "uneven": 512}.get(columns.split()[0], 1024)
+    assert lens[lens >= four_chunks].sum() * 2 >= len(crd)
+    A, B = rt.CsrMatrix.from_arrays((n, ncols), pos.astype(np.int64), crd.astype(np.int64), val), rng.uniform(-1, 1, (ncols, K))
+    dB, dC = rt.DeviceArray.from_numpy(B), rt.DeviceArray((n, K))
+    bound = orc.spmm(pos, crd, np.abs(val), np.abs(B))
+    for call in range(3):
+        rt.profile_reset()
+        rt.profile_enable(True)
+        rt.spmm(A, dB, dC, accumulate=False)
+        rt.sync()
+        rep = rt.profile_report()
+        rt.profile_enable(False)
+        assert "spmm_csr_nnzsplit" in rep and "spmm_heavy_sweep" not in rep, sorted(rep)
+        assert ("radix_sort_pairs" in rep) == (ordered and call == 1), call
+        assert np.all(np.abs(dC.to_numpy() - orc.spmm(pos, crd, val, B)) <= 1e-12 * bound)
+
+
 def test_spmm_launches_are_listed_by_the_kernel_that_runs(monkeypatch):
     # a first product and chunks by columns: the chunk kernel; a B beyond those, or the switch that turns them off: the sweep
     monkeypatch.delenv("COMET_HIP_PLAN_AT_ONCE")
