@@ -1359,24 +1359,26 @@ __global__ __launch_bounds__(256) void spmm_column_share(int64_t ncols, const ui
 // a->crowded_columns: asked of the device once
 static int spmm_crowded(Csr *a)
 {
-    if (a->crowded_columns >= 0)
-        return COMET_HIP_OK;
     const int64_t every = ceil_div(a->nnz, SPMM_COLUMN_SAMPLE), samples = ceil_div(a->nnz, every);
-    unsigned long long *word = nullptr;
+    const size_t bytes = sizeof(unsigned long long) + sizeof(uint32_t) * (size_t)a->ncols;
+    unsigned long long *word = nullptr, *held = nullptr;
     COMET_CHK(mailbox((void **)&word));
-    const size_t bytes = sizeof *word + sizeof(uint32_t) * (size_t)a->ncols;
-    COMET_CHK(g_long_entries.ensure(bytes, false));
-    unsigned long long *held = (unsigned long long *)g_long_entries.ptr;
-    uint32_t *count = (uint32_t *)(held + 1);
-    COMET_HIPCHK(hipMemsetAsync(held, 0, bytes, stream()));
-    spmm_column_counts<<<dim3((unsigned)ceil_div(samples, 256)), dim3(256), 0, stream()>>>(samples, every, a->nnz, a->crd, count);
-    // (a column that happens to be seen a few times is not a crowded one)
-    const uint32_t least = (uint32_t)std::max<int64_t>(8, ceil_div(4 * samples, a->ncols));
-    spmm_column_share<<<dim3((unsigned)std::min<int64_t>(ceil_div(a->ncols, 256), 2 * (int64_t)num_cus())), dim3(256), 0, stream()>>>(
-        a->ncols, count, least, held);
-    COMET_HIPCHK(hipGetLastError());
-    COMET_HIPCHK(hipMemcpyAsync(word, held, sizeof *word, hipMemcpyDeviceToHost, stream()));
-    COMET_CHK(stream_wait());
+    COMET_HIPCHK(dev_malloc((void **)&held, bytes));          // given back: 4 bytes a column may be much
+    const auto run = [&]() -> int {
+        uint32_t *count = (uint32_t *)(held + 1);
+        COMET_HIPCHK(hipMemsetAsync(held, 0, bytes, stream()));
+        spmm_column_counts<<<dim3((unsigned)ceil_div(samples, 256)), dim3(256), 0, stream()>>>(samples, every, a->nnz, a->crd, count);
+        // (a column that happens to be seen a few times is not a crowded one)
+        const uint32_t least = (uint32_t)std::max<int64_t>(8, ceil_div(4 * samples, a->ncols));
+        spmm_column_share<<<dim3((unsigned)std::min<int64_t>(ceil_div(a->ncols, 256), 2 * (int64_t)num_cus())), dim3(256), 0, stream()>>>(
+            a->ncols, count, least, held);
+        COMET_HIPCHK(hipGetLastError());
+        COMET_HIPCHK(hipMemcpyAsync(word, held, sizeof *word, hipMemcpyDeviceToHost, stream()));
+        return stream_wait();
+    };
+    const int rc = run();
+    (void)dev_free(held);
+    COMET_CHK(rc);
     a->crowded_columns = (double)*(volatile unsigned long long *)word > SPMM_CROWDED * (double)samples;
     return COMET_HIP_OK;
 }
