@@ -996,18 +996,26 @@ static int pair_side_plan(const Csr *T, const Csr *P, const Csr *L, int64_t firs
     COMET_HIPCHK(dev_malloc((void **)&plan->heavy, sizeof(uint2) * (size_t)(plan->nheavy > 0 ? plan->nheavy : 1)));
     COMET_HIPCHK(dev_malloc((void **)&plan->light, sizeof(int32_t) * (size_t)(plan->nlight > 0 ? plan->nlight : 1)));
     pair_items<<<rows, block, 0, stream()>>>(first, n, parts, wpos, (uint2 *)plan->heavy, plan->light, plan->counts);
-    if (ranged && plan->nheavy > 0) {
-        const size_t items = (size_t)plan->nheavy;
-        COMET_HIPCHK(dev_malloc((void **)&plan->ranged, sizeof(uint4) * items));
-        COMET_CHK(g_pair_range.ensure((sizeof(uint4) + 2 * sizeof(uint64_t) + 2 * sizeof(uint32_t)) * items, false));
-        uint4 *list = (uint4 *)g_pair_range.ptr;
-        uint64_t *keys = (uint64_t *)(list + items);
-        uint32_t *idx = (uint32_t *)(keys + 2 * items);
-        pair_ranges<<<rows, block, 0, stream()>>>(first, n, parts, wpos, plan->kpos, (const PairEnt *)plan->ent, (uint32_t)L->nnz, list,
-                                                  keys, idx);
-        COMET_CHK(sort_pairs_u64_u32(keys, keys + items, idx, idx + items, plan->nheavy, 20));
-        pair_ranges_sorted<<<dim3((unsigned)ceil_div(plan->nheavy, 256)), block, 0, stream()>>>(plan->nheavy, list, idx + items,
-                                                                                               (uint4 *)plan->ranged);
+    COMET_HIPCHK(hipGetLastError());
+    if (ranged && plan->nheavy > 0) {          // without memory for them the parts stay as pair_items has them
+        const auto ranges = [&]() -> int {
+            const size_t items = (size_t)plan->nheavy;
+            COMET_CHK(g_pair_range.ensure((sizeof(uint4) + 2 * sizeof(uint64_t) + 2 * sizeof(uint32_t)) * items, false));
+            COMET_HIPCHK(dev_malloc((void **)&plan->ranged, sizeof(uint4) * items));
+            uint4 *list = (uint4 *)g_pair_range.ptr;
+            uint64_t *keys = (uint64_t *)(list + items);
+            uint32_t *idx = (uint32_t *)(keys + 2 * items);
+            pair_ranges<<<rows, block, 0, stream()>>>(first, n, parts, wpos, plan->kpos, (const PairEnt *)plan->ent, (uint32_t)L->nnz,
+                                                      list, keys, idx);
+            COMET_CHK(sort_pairs_u64_u32(keys, keys + items, idx, idx + items, plan->nheavy, 20));
+            pair_ranges_sorted<<<dim3((unsigned)ceil_div(plan->nheavy, 256)), block, 0, stream()>>>(
+                plan->nheavy, list, idx + items, (uint4 *)plan->ranged);
+            return COMET_HIP_OK;
+        };
+        if (!plan_made(ranges)) {
+            (void)dev_free(plan->ranged);
+            plan->ranged = nullptr;
+        }
     }
     if (L->nnz < 4) {          // a lane reads four columns at a time
         constexpr size_t room = 4 * (sizeof(double) + sizeof(int32_t));

@@ -1184,6 +1184,31 @@ def test_a_plan_without_memory_is_done_without_triangle_count():
         assert _refusing(k, lambda: [rt.triangle_count(L) for _ in range(3)]) == [want] * 3, k
 
 
+def test_parts_by_stretches_are_done_without_where_they_find_no_memory():
+    # of what the plan of a masked product asks for, the parts by stretches (lists of more than 14 MiB) are no condition of it
+    n = 4000
+    rng = np.random.default_rng(5)
+    crd = np.sort(rng.random((n, n)).argsort(1)[:, :330], axis=1).astype(np.int32).ravel()
+    pos, val = np.arange(n + 1, dtype=np.int64) * 330, rng.integers(1, 9, n * 330).astype(float)
+    assert len(crd) * 12 > 14 << 20
+    new = lambda: rt.CsrMatrix.from_arrays((n, n), pos, crd, val)
+    mask = np.arange(0, n + 1, dtype=np.int64) * 40, np.tile(np.arange(0, n, 100, dtype=np.int32), n), np.ones(40 * n)
+    M = rt.CsrMatrix.from_arrays((n, n), *mask)
+    want = orc.spgemm(pos, crd, val, pos, crd, val, n, mask=mask[:2])
+    rt.spgemm(new(), new(), M)          # what the library keeps for all matrices is there
+    served = []
+    for k in range(40):
+        A, B = new(), new()
+        try:
+            got = _refusing(k, lambda: rt.spgemm(A, B, M)).to_arrays()
+            served.append(True)
+            assert all(np.array_equal(g, w) for g, w in zip(got, want)), k
+        except rt.CometHipError:
+            served.append(False)
+    last = max(k for k in range(40) if not served[k])
+    assert last < 39 and 1 <= sum(served[:last]) <= 2, served          # one for each side of the plan that has such parts
+
+
 @pytest.mark.parametrize("long_rows", [0, 3])
 def test_what_a_structure_keeps_is_for_rows_that_are_long(long_rows):
     # bitmaps of rows with a 64th of the columns: for as many as there are, and nothing for a matrix without
