@@ -315,6 +315,15 @@ __device__ __forceinline__ GettPlace gett_place(uint32_t tiles_m, uint32_t tiles
     return p;
 }
 
+// Of how many turns the offsets of irregular k are worked out at a time: sixteen, but one where sixteen would take the fourth
+// workgroup its LDS (3844 sums of 3844 products 37.4 us, with one 33.8); and the LDS of a workgroup.
+constexpr int gett_kt(int bn) { return bn == 16 ? 1 : 16; }
+constexpr size_t gett_lds(int bm, int bn, bool reg)
+{
+    return sizeof(double) * 2 * GM_BK * (size_t)(bm + bn + 2 * GM_PAD) + (sizeof(uint32_t) + sizeof(int64_t)) * (size_t)(bm + bn) +
+           (reg ? 0 : sizeof(uint32_t) * 4 * GM_BK * (size_t)gett_kt(bn));
+}
+
 template <int BM, int BN, int WM, int OCC, bool A_M, bool B_N, bool REG, bool RUN>
 __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const double *__restrict__ A,
                                                              const double *__restrict__ B, double *__restrict__ C,
@@ -326,11 +335,12 @@ __global__ __launch_bounds__(256, OCC) void gett_mfma_kernel(GettArgs g, const d
     constexpr int KSA = 256 / BM, KSB = 256 / BN;
     __shared__ double As[2][GM_BK][LDA];
     __shared__ double Bs[2][GM_BK][LDB];
-    // offsets in bytes of the rows (A), the columns (B) and, unless they are regular, of the k of KT turns, twice: sixteen,
-    // but one where sixteen would take the fourth workgroup its LDS (3844 sums of 3844 products 37.4 us, with one 33.8)
-    constexpr int KT = BN == 16 ? 1 : 16, KN = REG ? 1 : KT * GM_BK;
+    // offsets in bytes of the rows (A), the columns (B) and, unless they are regular, of the k of KT turns, twice
+    constexpr int KT = gett_kt(BN), KN = REG ? 1 : KT * GM_BK;
     __shared__ uint32_t rowA[BM], colB[BN], kA[REG ? 1 : 2][KN], kB[REG ? 1 : 2][KN];
     __shared__ int64_t rowC[BM], colC[BN];
+    static_assert(sizeof As + sizeof Bs + sizeof rowA + sizeof colB + sizeof rowC + sizeof colC + (REG ? 0 : sizeof kA + sizeof kB) ==
+                      gett_lds(BM, BN, REG), "what a CU holds is reckoned with it");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WN, wn = wave % WN;
     const GettPlace place = gett_place((g.M + BM - 1) / BM, (g.N + BN - 1) / BN);
@@ -609,7 +619,7 @@ struct GettShape {
     int bm, bn, resident;
     double turn_us, alone_us;
 };
-constexpr GettShape GETT_SHAPES[] = {{128, 128, 2, 1.86, 2.65}, {64, 64, 4, 0.52, 1.2}, {64, 32, 6, 0.30, 0.71}, {128, 16, 4, 0.38, 0.83}};
+constexpr GettShape GETT_SHAPES[] = {{128, 128, 2, 1.86, 2.65}, {64, 64, 4, 0.52, 1.2}, {64, 32, 5, 0.30, 0.71}, {128, 16, 4, 0.38, 0.83}};
 // What adding the shares up costs besides reading them, a launch: 10 x 60 x 12 x 40 over 120 products take 13.7 us in eight
 // shares, 10.9 in one.
 constexpr double GETT_REDUCE_US = 5.0;
@@ -753,6 +763,7 @@ static int gett_run(GettIndex m, GettIndex n, GettIndex k, int64_t M, int64_t N,
         const auto launch = [&](auto kernel_shape, auto wave_rows, auto occ) {
             constexpr GettShape S = GETT_SHAPES[decltype(kernel_shape)::value];
             constexpr int WM = decltype(wave_rows)::value, OCC = decltype(occ)::value;
+            static_assert(S.resident * gett_lds(S.bm, S.bn, false) <= 160 * 1024, "a CU has room for them");
             if constexpr (S.bn >= 64)
                 if (unbroken)
                     return gett_launch<S.bm, S.bn, WM, OCC, true, true>(a_m, b_n, grid, g, A, B, C, partial, use_c);
