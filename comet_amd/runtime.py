@@ -606,14 +606,19 @@ def dgemm(A, B, Cm=None, beta=0.0):
     return Cm
 
 
-def label_ids(a, b, c):
-    """Label numbering by first appearance in A, B, C (frontends/comet_dsl/mlir/MLIRGen.cpp:2236-2276)."""
+def _label_numbers(a, b, c):
+    """Labels are numbered by first appearance in A, B, C (frontends/comet_dsl/mlir/MLIRGen.cpp:2236-2276)."""
     ids = {}
     for s in (a, b, c):
         for ch in s:
             ids.setdefault(ch, len(ids))
-    conv = lambda s: np.array([ids[ch] for ch in s], dtype=np.int32)
-    return ids, conv(a), conv(b), conv(c)
+    return ids, [ids[ch] for ch in a], [ids[ch] for ch in b], [ids[ch] for ch in c]
+
+
+def label_ids(a, b, c):
+    """The numbers of the labels, and those of each operand as an array."""
+    ids, *operands = _label_numbers(a, b, c)
+    return (ids, *(np.array(x, dtype=np.int32) for x in operands))
 
 
 def _ints(code, values):
@@ -625,13 +630,8 @@ def _ints(code, values):
 
 
 def ttgt_plan(a, b, c, extent, which=-1):
-    ids = {}
-    for s in (a, b, c):
-        for ch in s:
-            ids.setdefault(ch, len(ids))
-    al, al_at = _ints("i", [ids[ch] for ch in a])
-    bl, bl_at = _ints("i", [ids[ch] for ch in b])
-    cl, cl_at = _ints("i", [ids[ch] for ch in c])
+    ids, in_a, in_b, in_c = _label_numbers(a, b, c)
+    (al, al_at), (bl, bl_at), (cl, cl_at) = _ints("i", in_a), _ints("i", in_b), _ints("i", in_c)
     ext, ext_at = _ints("q", [int(extent[ch]) for ch in ids])
     plan = TtgtPlan()
     _check(lib().comet_hip_ttgt_plan(len(a), al_at, len(b), bl_at, len(c), cl_at, ext_at, which, C.byref(plan)),
