@@ -372,6 +372,10 @@ static int spmv_plan(Csr *a)
 // from group to group.  Until that was so, one group went through a row of up to
 // 255 nonzeros by itself, 22 of the 24 us that a matrix of 2000 rows took (zipf, 12
 // nonzeros a row; 14 now); 20000 rows and K = 8 30 -> 20, 500000 and K = 3 175 -> 152.
+// Empty rows are cleared by all wavefronts, an equal share of the matrix's rows to each, whichever chunk they lie in: the
+// last rows of a graph are nearly all empty, and one wavefront's chunk had a thousand of them (us, R-MAT scale 16, 8 edges a
+// vertex K = 3 66 -> 29, K = 33 80 -> 45, scale 18 and 16 K = 8 180 -> 110, scale 19 and 16 K = 33 614 -> 499; 300000 rows, nine
+// of ten empty, K = 3 56 -> 13; the loads for it cost 100000 rows of 9 in a band 0.3 of 14).
 // Bound by the latency of that where the matrix is small, by the gathers' way from
 // the memory-side cache where B is larger than an L2.
 // ============================================================================
@@ -425,7 +429,7 @@ template <bool ACC, int W, bool SMALL>
 __global__ __launch_bounds__(SPMM_WAVES * 64, ACC ? 4 : 6) void spmm_csr_nnzsplit(
     const int64_t *__restrict__ pos, const int32_t *__restrict__ crd, const double *__restrict__ val,
     int64_t nnz, int64_t nrows, const int32_t *__restrict__ chunk_row, int grain, int chunk_len, int64_t nchunks, const uint32_t *__restrict__ order,
-    const double *__restrict__ B, int64_t ldb, double *__restrict__ C, int64_t ldc, int64_t K, int tile_cols,
+    const double *__restrict__ B, int64_t ldb, double *__restrict__ C, int64_t ldc, int K, int tile_cols, int rows_each,
     double *__restrict__ carry, unsigned *__restrict__ arrived, const int32_t *__restrict__ rowmap)
 {
     __shared__ __align__(16) SpmmChunkLds all[SPMM_WAVES];
@@ -449,6 +453,11 @@ __global__ __launch_bounds__(SPMM_WAVES * 64, ACC ? 4 : 6) void spmm_csr_nnzspli
     // the last lane of an odd tile has one column, and reads the one before it as well
     const bool half = W == 2 && sub == L - 1 && (kt & 1);
     const int64_t col = tile + W * sub, from = col - (half ? 1 : 0);
+    // rows of which the empty ones are this wavefront's to clear: where the first of them begin is loaded here
+    const int64_t z0 = chunk * rows_each, z1 = z0 + rows_each < nrows ? z0 + rows_each : nrows;
+    int64_t zp = 0;
+    if (!ACC && z0 + lane <= z1)
+        zp = pos[z0 + lane];
     // ---- the nonzeros [s, e) of the chunk, moved to the ends of rows that are not to be cut, and the rows they are of
     const int64_t s_cut = chunk * chunk_len, e_cut = s_cut + chunk_len < nnz ? s_cut + chunk_len : nnz;
     const int64_t block = s_cut / SPMM_CH * SPMM_CH;
@@ -475,14 +484,27 @@ __global__ __launch_bounds__(SPMM_WAVES * 64, ACC ? 4 : 6) void spmm_csr_nnzspli
     }
     for (int t = lane; t < n; t += 64)
         sh.row[t] = 0;
-    auto clear = [&](int64_t r) {
-        if (lane < kt)
-            C[crow(r) * ldc + tile + lane] = 0.0;
-    };
-    // rows in front of the first stored nonzero are empty: chunk 0 clears them
-    if (!ACC && chunk == 0)
-        for (int64_t z = 0; z < r0; ++z)
-            clear(z);
+    if constexpr (!ACC)          // accumulating leaves empty rows untouched
+        for (int64_t base = z0; base < z1; base += 63) {
+            if (base > z0 && base + lane <= z1)
+                zp = pos[base + lane];
+            const int64_t zq = __shfl_down(zp, 1, 64);
+            unsigned long long empty = __ballot(lane < 63 && base + lane < z1 && zp == zq);
+            while (empty) {          // as many next to each other as there are groups
+                const int first = __builtin_ctzll(empty), r = first + g;
+                if (g < G && r < 64 && (empty >> r & 1)) {
+                    double *to = C + crow(base + r) * ldc + col;
+                    if (W == 2 && !half) {
+                        spmm_pair v;
+                        v.x = v.y = 0.0;
+                        *reinterpret_cast<spmm_pair *>(to) = v;
+                    } else {
+                        *to = 0.0;
+                    }
+                }
+                empty = first + G < 64 ? empty >> (first + G) << (first + G) : 0;
+            }
+        }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
     for (int64_t base = r0 + 1; base <= rn && base < nrows; base += 64) {
         const int64_t r = base + lane;
@@ -494,13 +516,6 @@ __global__ __launch_bounds__(SPMM_WAVES * 64, ACC ? 4 : 6) void spmm_csr_nnzspli
         }
         if (in && p < q && p < e)
             sh.row[p - s] = (int32_t)(r - r0);
-        if constexpr (!ACC) {            // accumulating leaves empty rows untouched
-            unsigned long long empty = __ballot(in && p == q);
-            while (empty) {
-                clear(base + __builtin_ctzll(empty));
-                empty &= empty - 1;
-            }
-        }
     }
     if (n == 0)
         return;
@@ -2213,7 +2228,7 @@ static void spmm_chunk_launch(const Csr *a, int64_t K, const double *B, int64_t 
     const auto split = [&](auto kernel) {
         std::unique_ptr<KernelTimer> t(timed ? new KernelTimer("spmm_csr_nnzsplit", on) : nullptr);
         kernel<<<grid, block, 0, on>>>(a->pos, a->crd, a->val, a->nnz, a->nrows, chunk_row, grain, h.len, h.chunks, order, B, ldb, C,
-                                       ldc, K, h.cols, carry, arrived, a->rowmap);
+                                       ldc, (int)K, h.cols, (int)ceil_div(a->nrows, h.chunks), carry, arrived, a->rowmap);
     };
     const bool small_b = K > 1 && a->ncols * ldb * 8 < (1ll << 32);
     if (K == 1)

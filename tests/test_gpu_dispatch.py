@@ -445,6 +445,25 @@ def test_spmm_rows_that_are_not_cut(nrows, K, accumulate):
     assert np.array_equal(dC.to_numpy(), orc.spmm(pos, crd, val, B, C0 if accumulate else None))
 
 
+@pytest.mark.parametrize("K", [1, 3, 33, 64, 130])
+@pytest.mark.parametrize("nrows,filled", [(70, 1), (20_000, 3), (20_000, 300), (4_000, 3_900), (100, 100)])
+def test_spmm_empty_rows_belong_to_one_chunk_each(nrows, filled, K):
+    # in front, between and behind, few and thousands of them to a chunk, fewer rows than chunks; C's padding is not touched
+    rng = np.random.default_rng(nrows + filled)
+    lens = np.zeros(nrows, np.int64)
+    lens[rng.choice(np.arange(nrows // 3, nrows) if 2 * filled < nrows else nrows, filled, replace=False)] = 1
+    lens[np.flatnonzero(lens)[::3]] = 90 if nrows < 200 else 7
+    pos = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    crd = np.concatenate([np.sort(rng.choice(500, l, replace=False)) for l in lens]).astype(np.int32)
+    val, B, ldc = rng.uniform(-1, 1, pos[-1]), rng.uniform(-1, 1, (500, K)), K + 3
+    A, dB, dC = rt.CsrMatrix.from_arrays((nrows, 500), pos, crd, val), rt.DeviceArray.from_numpy(B), rt.DeviceArray((nrows, ldc))
+    for _ in range(2):
+        rt._check(rt.lib().comet_hip_memcpy(dC.ptr, rt._vptr(np.full((nrows, ldc), 7.0)), dC.nbytes, 0), "upload")
+        rt._check(rt.lib().comet_hip_spmm_csr_f64(A.handle, K, dB.ptr, K, dC.ptr, ldc, 0), "spmm")
+        got = dC.to_numpy()
+        assert np.array_equal(got[:, :K], orc.spmm(pos, crd, val, B)) and np.all(got[:, K:] == 7.0)
+
+
 @pytest.mark.parametrize("accumulate", [False, True])
 @pytest.mark.parametrize("nlong,ncols,K", [(40, 20_000, 7), (40, 9_000, 16), (300, 9_000, 21), (300, 4_100, 64), (700, 9_000, 33),
                                            (700, 120_000, 32), (700, 120_001, 31)])
