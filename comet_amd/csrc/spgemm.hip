@@ -1807,7 +1807,7 @@ __device__ __forceinline__ void block_add(double *slot, double a, double b, int 
 }
 
 // Writes out what the accumulators of a block hold, in order of the columns, and leaves them empty; place(total) as in
-// dense_emit_block.  A wavefront has 1024 columns to itself: it takes them into registers, and its part of acc becomes
+// dense_emit_block.  A wavefront has 64 * ROWS columns to itself: it takes them into registers, and its part of acc becomes
 // the list, half of the columns at a time, from which every lane writes the entry at its own place.
 template <bool SEMI, int WAVES, int ROWS, typename VALUE, typename PLACE>
 __device__ __forceinline__ void block_emit(double *acc, int *wave_tot, int lane, int wave, int col0, int reduce_op,

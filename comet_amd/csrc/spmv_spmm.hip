@@ -1340,9 +1340,9 @@ static int spmm_long_rows(Csr *a)
 // Columns that hold four times what they would if all held the same.  Where such columns hold this share of the entries, chunks
 // stay as they are stored.  Share, and us as stored / by columns: columns n * u^p of a random u, rows as zipf, 60000 rows K = 33
 // p = 2 (0.10) 54.8 / 44.7, p = 4 (0.30) 44.0 / 39.5, p = 6 (0.38) 37.9 / 37.2, the same columns at random places 38.9 / 35.1,
-// 250000 rows K = 21 p = 6 (0.42) 113.9 / 91.2; R-MAT scale 13, 32 edges a vertex (0.50) K = 17 22.8 / 24.5, K = 32 24.8 / 27.1,
-// 18 and 16 (0.73) K = 17 235 / 253, K = 31 276 / 283, 17 and 32 (0.75) K = 31 184 / 219, K = 48 248 / 276, its vertices at random
-// places K = 33 188 / 202.  The sweep is no way out for these either: 18 and 16 K = 24 238 / 526 swept, 17 and 32 K = 32 176 / 459.
+// 250000 rows K = 21 p = 6 (0.42) 113.9 / 91.2; R-MAT scale 13, 32 edges a vertex (0.50) K = 17 21.6 / 22.1, K = 32 23.6 / 23.9,
+// 18 and 16 (0.73) K = 17 156 / 196, K = 31 194 / 223, 17 and 32 (0.75) K = 31 162 / 196, K = 48 201 / 232, its vertices at random
+// places K = 33 185 / 200.  The sweep is no way out for these either: 18 and 16 K = 24 156 / 518 swept, 17 and 32 K = 32 145 / 457.
 constexpr double SPMM_CROWDED = 0.46;
 constexpr int64_t SPMM_COLUMN_SAMPLE = 1 << 19;           // entries that are looked at, about
 
@@ -1698,7 +1698,7 @@ static int sweep_launch(Kern kernel, dim3 grid, dim3 block, size_t lds, Args... 
 // row of B in several of them.  us, chunks as stored / sweep at K = 17, 33, 63, and of the entries the share in long rows and how many
 // of them there are a column: zipf, 200000 rows of 4 (0.69, 2.7) 62 / 124, 77 / 131, 113 / 113, of 8 (0.81, 6.5) 87 / 100, 115 /
 // 107, 177 / 106, 100000 of 16 (0.86, 14) K = 33 101 / 78, 63 159 / 83; R-MAT scale 17, 4 edges a vertex (0.37, 2.8) K = 33
-// 105 / 145, 16 (0.54, 15) 144 / 332.
+// 50 / 145, 16 (0.54, 15) 115 / 332.
 static bool sweep_uneven(const Csr *a, int64_t K)
 {
     return a->heavy_nnz * 4 >= a->nnz * 3 && a->heavy_nnz >= (K < 32 ? 8 : 4) * a->ncols;
