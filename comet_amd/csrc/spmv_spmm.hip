@@ -2911,8 +2911,9 @@ static int sddmm_order(Csr *b, const int32_t *rows)
 // ascending k in a register.  D is read once, and neither turned over nor gathered;
 // no product goes through LDS.  What is left is the lines of C: one for every run
 // of entries of one row in a tile, looked up eight times, since a lane takes
-// sixteen bytes of it - two thirds of the time of the CUs' address units, and the
-// reason why runs have to be long (sddmm_tiles).  Rows of C staged in LDS, loaded
+// sixteen bytes of it - the reason why runs have to be long (sddmm_tiles).  250000
+// rows K = 64: the CUs' path for what loads return is busy in 91 % of the cycles,
+// their address units in 73 (gathering D 83 and 73, in 237 us with D's transposition against 210).  Rows of C staged in LDS, loaded
 // a line at a time, were slower (250000 rows K = 64 279 us against 234).
 // ---------------------------------------------------------------------------
 constexpr int SDDMM_TILE_T = 1024, SDDMM_TILE_COLS = 512, SDDMM_TILE_K = 16, SDDMM_TILE_BATCHES = 10;
